@@ -18,8 +18,9 @@ struct nncase_hip_weights {
     int fold = 0;
     // igemm: packed for the wide-tile kernels (qconv_wide.hpp): 1 = long reductions over many pixels and channels
     // (blocks of 256 or 128 pixels, waves of 64), 2 = reductions of five k-steps and more over fewer pixels (blocks of
-    // 128 pixels x 64 channels or 64 x 32, waves of 32 pixels)
+    // `small_shape`, waves of 32 pixels)
     int wide = 0;
+    int small_shape = 0;
     long long dw_const_bound = 0; // depthwise: max over channels of |bias| + 255 |sum(w - zw)|
     long long bias_absmax = 0;    // largest |bias|
     int64_t pixels_hint = 0; // output pixels per call the tiling was planned for (0 = unknown)
@@ -42,6 +43,9 @@ struct nncase_hip_weights {
 };
 
 namespace nnhip {
+
+// Blocks of the wide kernel's small form, pixels x channels (nncase_hip_weights::small_shape).
+enum SmallShape { kBlock128x64 = 0, kBlock64x128 = 1, kBlock64x32 = 2, kBlock32x64 = 3 };
 
 // Output forms of the conv / matmul epilogue.
 enum OutMode { kOutU8 = 0, kOutI32 = 1, kOutF32 = 2 };

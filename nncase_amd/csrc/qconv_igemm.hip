@@ -53,14 +53,15 @@ int prepack_igemm(nncase_hip_ctx *ctx, nncase_hip_weights *w, const uint8_t *w_o
     w->ksteps = ceil_div(w->k, 64);
     const int max_tiles = (w->g_ic % 4 == 0) ? 16 : 4;
     plan_igemm(w->g_oc, w->ksteps, max_tiles, w->pixels_hint, ctx->compute_units, &w->tiles, &w->nchunks, &w->kc_steps);
-    // Long reductions over many pixels and at least 64 channels are bound by the matrix cores: they take the
+    // Long reductions over many pixels and more than 64 channels are bound by the matrix cores: they take the
     // wide-tile kernels (a wave owns 64 pixels x 64 or 128 channels) when the launch has a 256-pixel block for every
-    // compute unit; smaller launches keep the small tiles, whose larger wave count fills the device better.
+    // compute unit; smaller launches keep the small tiles, whose larger wave count fills the device better.  (Up to 64
+    // channels the 128 x 64 blocks below are quicker at any size: 200 704 pixels 64 -> 64 3x3 20.6 us against 25.6.)
     {
         const long long ptiles = ceil_div((int)std::min<int64_t>(std::max<int64_t>(w->pixels_hint, 0), 1 << 30), 256);
         // 256-channel chunks (two waves side by side share the block's activations) where that still fills the device
-        const int wide_tiles = w->g_oc <= 64 ? 4 : (w->g_oc > 128 && ptiles * ceil_div(w->g_oc, 256) >= ctx->compute_units ? 16 : 8);
-        w->wide = w->g_ic % 16 == 0 && w->ksteps >= kWideMinKsteps && w->g_oc >= 64 &&
+        const int wide_tiles = (w->g_oc > 128 && ptiles * ceil_div(w->g_oc, 256) >= ctx->compute_units ? 16 : 8);
+        w->wide = w->g_ic % 16 == 0 && w->ksteps >= kWideMinKsteps && w->g_oc > 64 &&
                   ptiles * ceil_div(w->g_oc, wide_tiles * 16) >= ctx->compute_units;
         if (w->wide) {
             w->tiles = wide_tiles;
@@ -68,16 +69,22 @@ int prepack_igemm(nncase_hip_ctx *ctx, nncase_hip_weights *w, const uint8_t *w_o
             w->kc_steps = std::min(w->ksteps, kLdsFrags / w->tiles);
         }
     }
-    // Reductions of kSmallWideMinKsteps k-steps and more over fewer pixels take the same kernel with 128 x 64 blocks
-    // (four waves of 32 pixels) or 64 x 32 ones: against the small tiles' per-lane loads of 16 pixels' slices, the
-    // row-order fetch through LDS needs a quarter of the requests to the vector L1, which is what such launches
-    // are bound by.
+    // Reductions of kSmallWideMinKsteps k-steps and more over fewer pixels take the same kernel with blocks of 8192 or 2048
+    // outputs: against the small tiles' per-lane loads of 16 pixels' slices, the row-order fetch through LDS needs a
+    // quarter of the requests to the vector L1, which is what such launches are bound by.
     if (!w->wide && w->g_ic % 16 == 0 && w->ksteps >= kSmallWideMinKsteps) {
         w->wide = 2;
-        // (64 x 32 blocks of two waves while the larger ones would leave more than half of the compute units without a
-        // block: the 512 x 1024 x 1024 product takes 7.0 us with them, 9.2 us with 64 blocks of 128 x 64)
-        const long long blocks128 = (long long)ceil_div((int)std::min<int64_t>(std::max<int64_t>(w->pixels_hint, 1), 1 << 30), 128) * ceil_div(w->g_oc, 64);
-        w->tiles = (w->g_oc <= 32 || (w->pixels_hint > 0 && 2 * blocks128 < ctx->compute_units)) ? 2 : 4;
+        // (2048 outputs per block while the larger ones would leave more than half of the compute units without a block:
+        // the 512 x 1024 x 1024 product takes 7.0 us with them, 9.2 us with 64 blocks of 8192)
+        const long long blocks = (long long)ceil_div((int)std::min<int64_t>(std::max<int64_t>(w->pixels_hint, 1), 1 << 30), 128) * ceil_div(w->g_oc, 64);
+        const bool small = w->g_oc <= 32 || (w->pixels_hint > 0 && 2 * blocks < ctx->compute_units);
+        // A block that is wide in channels stages and re-biases half the activations per product (6400 pixels 256 -> 256 3x3:
+        // 17.4 -> 16.1 us; 400 pixels: 14.5 -> 12.3 us), unless that rounds the channel count up by more than an eighth.
+        auto rounded = [&](int chunk) { return ceil_div(w->g_oc, chunk) * chunk; };
+        const int narrow = small ? 32 : 64;
+        const bool flat = w->g_oc > narrow && 8 * rounded(2 * narrow) <= 9 * rounded(narrow);
+        w->small_shape = small ? (flat ? kBlock32x64 : kBlock64x32) : (flat ? kBlock64x128 : kBlock128x64);
+        w->tiles = (flat ? 2 * narrow : narrow) / 16;
         w->nchunks = ceil_div(w->g_oc, w->tiles * 16);
         w->kc_steps = std::min(w->ksteps, kLdsFrags / w->tiles);
     }
@@ -200,7 +207,7 @@ int launch_qconv_igemm(nncase_hip_ctx *ctx, const uint8_t *x, const nncase_hip_w
         a.r_coff = g * w->g_oc;
         int rc;
         if (w->wide == 2) {
-            rc = mode == kRows16 ? launch_wide_small_rows16(ctx, a, w->tiles, w->nchunks) : launch_wide_small_vec16(ctx, a, w->tiles, w->nchunks);
+            rc = mode == kRows16 ? launch_wide_small_rows16(ctx, a, w->small_shape, w->nchunks) : launch_wide_small_vec16(ctx, a, w->small_shape, w->nchunks);
             if (rc) return rc;
             continue;
         }

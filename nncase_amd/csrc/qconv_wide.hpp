@@ -64,9 +64,17 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t wide_rsrc(const void *base, ui
 // banks, so pixels p and p + 2 (128 bytes apart) must not present the same piece (measured: 241 bytes per clock and
 // compute unit with this rotation, 128 with a rotation by (p >> 2) or none); the row-order writes cover whole
 // 128-byte runs whatever the rotation.
-template <int T, int RG, int WM, int WN, int LM>
-__global__ __launch_bounds__(WM * WN * 64, 2) void qconv_wide_kernel(const IgemmArgs a, int nchunks) {
-    constexpr int THREADS = WM * WN * 64;
+//
+// KG > 1: the reduction is split inside the block.  KG groups of WM x WN waves each run this loop over every KG-th
+// k-step with a ring of their own and meet only in the epilogue, where pixel group rg of every wave is summed by the
+// group rg (LDS) and finished there.  A wave alone on its SIMD issues an instruction every eight to nine cycles, and a
+// k-step is about a hundred of them (880 cycles for 128 cycles of matrix work), so a launch with one block per compute
+// unit is bound by that; KG waves per SIMD take turns issuing.
+template <int T, int RG, int WM, int WN, int LM, int KG = 1>
+__global__ __launch_bounds__(WM * WN * KG * 64, WM * WN * KG > 8 ? 4 : 2) void qconv_wide_kernel(const IgemmArgs a, int nchunks) {
+    static_assert(KG == 1 || RG <= KG, "every pixel group of a wave has a group of its own to finish it");
+    constexpr int THREADS = WM * WN * 64;               // of a group: the threads that move a k-step's operands
+    constexpr int BLOCK = THREADS * KG;
     constexpr int PIX = WM * RG * 16;                   // pixels per block
     constexpr int TB = T * WN;                          // channel tiles per block
     constexpr int AV = PIX * 4, WV = TB * 64;           // 16-byte vectors of activations / weights per k-step
@@ -80,7 +88,7 @@ __global__ __launch_bounds__(WM * WN * 64, 2) void qconv_wide_kernel(const Igemm
     int32_t *cterm = reinterpret_cast<int32_t *>(smem);              // [TB * 16]
     uint8_t *lutl = smem + TB * 16 * sizeof(int32_t);                // [256]
     int32_t *rowsums = reinterpret_cast<int32_t *>(lutl + 256);      // [PIX]
-    uint8_t *ring = lutl + 256 + PIX * sizeof(int32_t);              // [kWideSlots][SLOT]
+    uint8_t *const rings = lutl + 256 + PIX * sizeof(int32_t);       // [KG][kWideSlots][SLOT]
 
     // channel chunks of a pixel tile are consecutive on one XCD (blocks go to the 8 XCDs round-robin)
     // ... and every XCD takes a contiguous eighth of the pixel tiles, in the order of the tensor: the tiles that share
@@ -92,20 +100,24 @@ __global__ __launch_bounds__(WM * WN * 64, 2) void qconv_wide_kernel(const Igemm
     if (seq / nchunks >= per || mt >= a.num_mtiles) return;
 
     const int lane = threadIdx.x & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int bwave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int kg = KG == 1 ? 0 : bwave / (WM * WN), wave = bwave - kg * (WM * WN);
+    const int tid = threadIdx.x - kg * THREADS;          // thread of the group
+    uint8_t *const ring = rings + kg * (kWideSlots * SLOT);
     const int wm = wave % WM, wn = wave / WM;
     const int j = lane & 15, gq = lane >> 4; // matrix operand order: pixel j of a group, 16-byte piece gq of the k-step
     const int ch_base = chunk * (TB * 16);
     const int KS = a.ksteps;
+    const int KL = KG == 1 ? KS : (KS - kg + KG - 1) / KG; // k-steps of this group: kg, kg + KG, ... (the loop counts them from 0)
     const __amdgpu_buffer_rsrc_t wres = wide_rsrc(a.wpk + (size_t)chunk * KS * TB * 1024, (uint32_t)KS * TB * 1024);
     const __amdgpu_buffer_rsrc_t xres = wide_rsrc(a.x, (uint32_t)a.x_bytes);
 
     // per-channel constant of the zero-point identity and the byte table: requested now, needed by the epilogue
-    constexpr int NC = (TB * 16 + THREADS - 1) / THREADS;
+    constexpr int NC = (TB * 16 + BLOCK - 1) / BLOCK;
     int32_t c_bias[NC], c_wsum[NC];
 #pragma unroll
     for (int i = 0; i < NC; i++) {
-        const int c = i * THREADS + threadIdx.x;
+        const int c = i * BLOCK + threadIdx.x;
         const bool real = c < TB * 16 && ch_base + c < a.n;
         c_bias[i] = real ? a.bias[ch_base + c] : 0;
         c_wsum[i] = real ? a.wsum[ch_base + c] : 0;
@@ -113,15 +125,17 @@ __global__ __launch_bounds__(WM * WN * 64, 2) void qconv_wide_kernel(const Igemm
     uint32_t lut_word = 0;
     const bool lut_mine = a.lut && threadIdx.x < 64;
     if (lut_mine) lut_word = a.lut[threadIdx.x];
+    if (KG > 1) // (the groups add their shares of a pixel's sum of x' up; the first barrier is in front of the first addition)
+        for (int i = threadIdx.x; i < PIX; i += BLOCK) rowsums[i] = 0;
 
     // ---- weights: thread t moves vectors t + i * THREADS of every k-step ----
-    const uint32_t w_voff = threadIdx.x * 16;
-    auto load_w = [&](wide_u32x4 (&dst)[NW], int ks) {
-        const int ksc = min(ks, KS - 1); // a k-step past the end re-reads the last one (its data is never multiplied)
+    const uint32_t w_voff = tid * 16;
+    auto load_w = [&](wide_u32x4 (&dst)[NW], int sl) {
+        const int ksc = min(sl * KG + kg, KS - 1); // a k-step past the end re-reads the last one (its data is never multiplied)
 #pragma unroll
         for (int i = 0; i < NW; i++) dst[i] = __builtin_amdgcn_raw_buffer_load_b128(wres, w_voff, (ksc * WV + i * THREADS) * 16, 0);
     };
-    uint8_t *const w_dst = ring + AV * 16 + threadIdx.x * 16;
+    uint8_t *const w_dst = ring + AV * 16 + tid * 16;
     auto store_w = [&](const wide_u32x4 (&src)[NW], int slot /* byte offset of the ring slot */) {
 #pragma unroll
         for (int i = 0; i < NW; i++) *reinterpret_cast<wide_u32x4 *>(w_dst + slot + i * THREADS * 16) = src[i];
@@ -129,7 +143,7 @@ __global__ __launch_bounds__(WM * WN * 64, 2) void qconv_wide_kernel(const Igemm
 
     // ---- activations: the NA pieces this thread fetches per k-step (row order: the four threads of a quad read the
     // 64 bytes of one pixel's k-step): piece lq of pixel lp + i * (THREADS / 4) of the block ----
-    const int lp = threadIdx.x >> 2, lq = threadIdx.x & 3;
+    const int lp = tid >> 2, lq = tid & 3;
     int32_t p_off[NA];          // byte offset of the pixel's first piece (windows: of the window origin, may be negative)
     int32_t p_iy0[NA], p_ix0[NA];
 #pragma unroll
@@ -150,8 +164,8 @@ __global__ __launch_bounds__(WM * WN * 64, 2) void qconv_wide_kernel(const Igemm
         uint32_t fill;    // what a piece that is not taken holds: the zero point (padding tap) or x' = 0 (past the reduction)
         bool take[NA];
     };
-    auto load_acts = [&](Acts &f, int ks) {
-        const int ksc = min(ks, KS - 1); // as for the weights
+    auto load_acts = [&](Acts &f, int sl) {
+        const int ksc = min(sl * KG + kg, KS - 1); // as for the weights
         if (LM == kWideRowsFull) {
 #pragma unroll
             for (int i = 0; i < NA; i++) {
@@ -206,9 +220,9 @@ __global__ __launch_bounds__(WM * WN * 64, 2) void qconv_wide_kernel(const Igemm
     for (int i = 0; i < NA; i++) rsum[i] = 0;
     // Padding and re-biasing happen on the way into the ring: x' = (piece taken ? x : fill) ^ 0x80; the sums of x are
     // taken from the same registers (every staged k-step adds 64 bytes per pixel, positions past the reduction as 128:
-    // the sum of x' is the sum of x less 128 * 64 * k-steps).  A k-step past the end of the reduction is not staged (ks < KS is uniform).
-    auto store_acts = [&](const Acts &f, int slot, int ks) {
-        if (ks >= KS) return;
+    // the sum of x' is the sum of x less 128 * 64 * k-steps).  A k-step past the end of the reduction is not staged (sl < KL is uniform).
+    auto store_acts = [&](const Acts &f, int slot, int sl) {
+        if (sl >= KL) return;
 #pragma unroll
         for (int i = 0; i < NA; i++) {
             wide_u32x4 r;
@@ -293,16 +307,17 @@ __global__ __launch_bounds__(WM * WN * 64, 2) void qconv_wide_kernel(const Igemm
     };
     int s = 0;
 #pragma clang loop unroll(disable)
-    for (; s + 1 < KS; s += 2) {
+    for (; s + 1 < KL; s += 2) {
         kstep(s, std::integral_constant<int, 0>());
         kstep(s + 1, std::integral_constant<int, 1>());
     }
-    if (s < KS) kstep(s, std::integral_constant<int, 0>()); // an odd number of k-steps
+    if (s < KL) kstep(s, std::integral_constant<int, 0>()); // an odd number of k-steps
+    if (KG > 1 && KL < (KS + KG - 1) / KG) __syncthreads();  // a group with one k-step less still meets the others' barriers
 
     // ---- epilogue ----
 #pragma unroll
     for (int i = 0; i < NC; i++) {
-        const int c = i * THREADS + threadIdx.x;
+        const int c = i * BLOCK + threadIdx.x;
         if (c < TB * 16) cterm[c] = ch_base + c < a.n ? c_bias[i] - a.zxp * c_wsum[i] + a.k * a.zxp * a.zwp : 0;
     }
     if (lut_mine) reinterpret_cast<uint32_t *>(lutl)[threadIdx.x] = lut_word;
@@ -312,17 +327,43 @@ __global__ __launch_bounds__(WM * WN * 64, 2) void qconv_wide_kernel(const Igemm
         int32_t r = (int32_t)rsum[i];
         r += __shfl_xor(r, 1);
         r += __shfl_xor(r, 2);
-        if (lq == 0) rowsums[lp + i * (THREADS / 4)] = r - 128 * 64 * KS;
+        if (KG == 1) {
+            if (lq == 0) rowsums[lp + i * (THREADS / 4)] = r - 128 * 64 * KS;
+        } else {
+            if (lq == 0) atomicAdd(&rowsums[lp + i * (THREADS / 4)], r - 128 * 64 * KL);
+        }
+    }
+    // the rings are free: partial sums on their way to the group that finishes them, [rg][other group][wave][tile][lane]
+    constexpr int PART = KG == 1 ? 0 : RG * (KG - 1) * WM * WN * T * 1024;
+    auto part = [&](int rg, int from, int nt) {
+        return reinterpret_cast<v4i *>(rings + (((rg * (KG - 1) + from) * (WM * WN) + wave) * T + nt) * 1024 + lane * 16);
+    };
+    if constexpr (KG > 1) {
+        static_for<0, RG>([&](auto rg_c) __attribute__((always_inline)) {
+            constexpr int rg = decltype(rg_c)::value;
+            if (kg == rg) return;
+#pragma unroll
+            for (int nt = 0; nt < T; nt++) *part(rg, kg - (kg > rg ? 1 : 0), nt) = acc[rg][nt];
+        });
     }
     __syncthreads();
-    // dword outputs are written through a staging area per wave (store_dword_rows): the ring is free now
-    static_assert(!staged_store_built(T) || WM * WN * staged_store_bytes() <= kWideSlots * SLOT, "the staging areas fit the ring");
-    uint8_t *const stage = staged_store_built(T) ? ring + wave * staged_store_bytes() : nullptr;
+    // dword outputs are written through a staging area per wave (store_dword_rows) behind the partial sums
+    constexpr int FIN = KG == 1 ? WM * WN : RG * WM * WN; // waves that finish pixels
+    static_assert(PART + (staged_store_built(T) ? FIN * staged_store_bytes() : 0) <= KG * kWideSlots * SLOT, "the staging areas fit the rings");
+    if (KG > 1 && kg >= RG) return;
+    uint8_t *const stage = staged_store_built(T) ? rings + PART + bwave * staged_store_bytes() : nullptr;
     // lane (j, gq) of wave (wm, wn) holds channels ch_base + gq * 4 TB + wn * 4 T + [0, 4 T) of its pixels
     const int ch0 = ch_base + gq * (4 * TB) + wn * (4 * T);
     const int32_t *ct = cterm + gq * (4 * TB) + wn * (4 * T) - gq * (4 * T); // igemm_store_tile adds gq * 4 T
     static_for<0, RG>([&](auto rg_c) __attribute__((always_inline)) {
         constexpr int rg = decltype(rg_c)::value;
+        if (KG > 1 && kg != rg) return;
+        if constexpr (KG > 1) {
+#pragma unroll
+            for (int from = 0; from < KG - 1; from++)
+#pragma unroll
+                for (int nt = 0; nt < T; nt++) acc[rg][nt] += *part(rg, from, nt);
+        }
         const int pl = (wm * RG + rg) * 16 + j;
         igemm_store_tile<T, kOwesAll, false, staged_store_built(T)>(a, acc[rg], rowsums[pl], mt * PIX + pl, ch0, gq, ct, lutl, stage, 4 * TB);
     });
@@ -970,21 +1011,21 @@ template <int T, int RG, int WM, int WN, int LM> int launch_wide_dma_t(nncase_hi
     return 0;
 }
 
-template <int T, int RG, int WM, int WN, int LM> int launch_wide_t(nncase_hip_ctx *ctx, const IgemmArgs &a, int nchunks) {
+template <int T, int RG, int WM, int WN, int LM, int KG = 1> int launch_wide_t(nncase_hip_ctx *ctx, const IgemmArgs &a, int nchunks) {
     IgemmArgs args = a;
     constexpr int PIX = WM * RG * 16, TB = T * WN;
     args.num_mtiles = ceil_div(a.m, PIX);
     const int blocks = ceil_div(args.num_mtiles, 8) * 8 * nchunks;
-    const size_t lds = (size_t)TB * 16 * sizeof(int32_t) + 256 + PIX * sizeof(int32_t) + (size_t)kWideSlots * (PIX * 64 + TB * 1024);
+    const size_t lds = (size_t)TB * 16 * sizeof(int32_t) + 256 + PIX * sizeof(int32_t) + (size_t)KG * kWideSlots * (PIX * 64 + TB * 1024);
     if (lds > 65536) { // more than 64 KiB of dynamic LDS has to be asked for once per kernel and device
         static std::once_flag raised[16];
         hipError_t attr = hipSuccess;
         std::call_once(raised[ctx->device & 15], [&] {
-            attr = hipFuncSetAttribute(reinterpret_cast<const void *>(&qconv_wide_kernel<T, RG, WM, WN, LM>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+            attr = hipFuncSetAttribute(reinterpret_cast<const void *>(&qconv_wide_kernel<T, RG, WM, WN, LM, KG>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
         });
         NNHIP_HIP(ctx, attr);
     }
-    hipLaunchKernelGGL((qconv_wide_kernel<T, RG, WM, WN, LM>), dim3(blocks), dim3(WM * WN * 64), lds, ctx->stream, args, nchunks);
+    hipLaunchKernelGGL((qconv_wide_kernel<T, RG, WM, WN, LM, KG>), dim3(blocks), dim3(WM * WN * KG * 64), lds, ctx->stream, args, nchunks);
     NNHIP_LAUNCH_CHECK(ctx, "qconv_wide_kernel");
     return 0;
 }
@@ -994,8 +1035,26 @@ inline int wide_waves(const nncase_hip_ctx *ctx, int m, int nchunks) {
     return (long long)ceil_div(m, 256) * nchunks >= (long long)ctx->compute_units ? 4 : 2;
 }
 
-// Block shapes: tiles = 16 -> 256 pixels x 256 channels (4 x 2 waves); tiles = 8 -> 256 or 128 pixels x 128 channels;
-// tiles = 4 -> 256 or 128 pixels x 64 channels.
+// Groups of waves that share a block's reduction (KG), by the waves per compute unit the launch has without a split and
+// the k-steps there are to share.  A split costs a start-up and an exchange of sums, so a longer reduction is asked for
+// the more waves there already are.  Measured, us with 1 / 2 / 4 groups: 6400 pixels 256 -> 256 3x3 (3.1 waves, 36 k-steps)
+// 16.1 / 12.5 / 12.0; 25 600 pixels 128 -> 128 3x3 (6.2, 18) 13.0 / 11.9 / 16.3; 6400 pixels 512 -> 512 1x1 (6.2, 8) 7.7 / 8.1 / 12.1;
+// 1600 pixels 128 -> 128 3x3 (0.8, 18) 7.9 / 6.2 / 5.6; 400 pixels 512 -> 512 1x1 (0.8, 8) 4.7 / 4.3 / 4.4.
+inline int small_wide_groups(const nncase_hip_ctx *ctx, int m, int ksteps, int pix, int waves, int nchunks) {
+    const double per_cu = (double)ceil_div(m, pix) * nchunks * waves / ctx->compute_units;
+    if ((per_cu <= 4 && ksteps >= 32) || (per_cu <= 1.6 && ksteps >= 16)) return 4;
+    return per_cu <= 4 || (per_cu <= 8 && ksteps >= 16) ? 2 : 1;
+}
+
+template <int T, int WM, int WN, int LM> int launch_wide_small_t(nncase_hip_ctx *ctx, const IgemmArgs &a, int nchunks) {
+    switch (small_wide_groups(ctx, a.m, a.ksteps, WM * 32, WM * WN, nchunks)) {
+    case 4: return launch_wide_t<T, 2, WM, WN, LM, 4>(ctx, a, nchunks);
+    case 2: return launch_wide_t<T, 2, WM, WN, LM, 2>(ctx, a, nchunks);
+    default: return launch_wide_t<T, 2, WM, WN, LM>(ctx, a, nchunks);
+    }
+}
+
+// Block shapes: tiles = 16 -> 256 pixels x 256 channels (4 x 2 waves); tiles = 8 -> 256 or 128 pixels x 128 channels.
 template <int LM> int launch_wide_lm(nncase_hip_ctx *ctx, const IgemmArgs &a, int tiles, int nchunks) {
     if (tiles == 16) {
         if constexpr (LM == kWideRowsFull || LM == kWideRows) {
@@ -1005,17 +1064,20 @@ template <int LM> int launch_wide_lm(nncase_hip_ctx *ctx, const IgemmArgs &a, in
     }
     const int wmv = wide_waves(ctx, a.m, nchunks);
     if (tiles == 8) return wmv == 4 ? launch_wide_t<8, 4, 4, 1, LM>(ctx, a, nchunks) : launch_wide_t<8, 4, 2, 1, LM>(ctx, a, nchunks);
-    if (tiles == 4) return wmv == 4 ? launch_wide_t<4, 4, 4, 1, LM>(ctx, a, nchunks) : launch_wide_t<4, 4, 2, 1, LM>(ctx, a, nchunks);
     return fail(ctx, -EINVAL, "qconv2d: no wide kernel for %d channel tiles", tiles);
 }
 
-template <int LM> int launch_wide_small_lm(nncase_hip_ctx *ctx, const IgemmArgs &a, int tiles, int nchunks) {
-    if (tiles == 4) return launch_wide_t<4, 2, 4, 1, LM>(ctx, a, nchunks);
-    if (tiles == 2) return launch_wide_t<2, 2, 2, 1, LM>(ctx, a, nchunks);
-    return fail(ctx, -EINVAL, "qconv2d: no small wide kernel for %d channel tiles", tiles);
+template <int LM> int launch_wide_small_lm(nncase_hip_ctx *ctx, const IgemmArgs &a, int shape, int nchunks) {
+    switch (shape) {
+    case kBlock64x128: return launch_wide_small_t<4, 2, 2, LM>(ctx, a, nchunks);
+    case kBlock128x64: return launch_wide_small_t<4, 4, 1, LM>(ctx, a, nchunks);
+    case kBlock32x64: return launch_wide_small_t<2, 1, 2, LM>(ctx, a, nchunks);
+    case kBlock64x32: return launch_wide_small_t<2, 2, 1, LM>(ctx, a, nchunks);
+    }
+    return fail(ctx, -EINVAL, "qconv2d: no small wide kernel of shape %d", shape);
 }
-int launch_wide_small_rows16(nncase_hip_ctx *ctx, const IgemmArgs &a, int variant, int nchunks);
-int launch_wide_small_vec16(nncase_hip_ctx *ctx, const IgemmArgs &a, int variant, int nchunks);
+int launch_wide_small_rows16(nncase_hip_ctx *ctx, const IgemmArgs &a, int shape, int nchunks);
+int launch_wide_small_vec16(nncase_hip_ctx *ctx, const IgemmArgs &a, int shape, int nchunks);
 int launch_wide_rows16(nncase_hip_ctx *ctx, const IgemmArgs &a, int tiles, int nchunks);
 int launch_wide_vec16(nncase_hip_ctx *ctx, const IgemmArgs &a, int tiles, int nchunks);
 

@@ -282,6 +282,20 @@ def test_extreme_values_and_zero_points(hip_ctx):
             assert np.array_equal(got, want)
 
 
+@pytest.mark.parametrize("n,c,h,w,oc,k", [
+    (4, 240, 40, 41, 130, 3),     # 128 x 64 blocks, four groups, 34 k-steps: two groups have one more than the others
+    (3, 128, 41, 40, 250, 3),     # 64 x 128 blocks, two groups, one tap per k-step
+    (1, 272, 15, 20, 190, 3),     # 32 x 64 blocks, four groups, 39 k-steps
+    (1, 272, 15, 20, 200, 3),     # 64 x 32 blocks
+    (2, 112, 16, 16, 64, 2),      # two groups, seven k-steps
+    (1, 1056, 7, 11, 48, 1),      # contiguous rows, 17 k-steps of which the last is half full, a block that is mostly past the end
+    (5, 320, 1, 1, 33, 1)])
+def test_reductions_shared_by_groups_of_waves(hip_ctx, n, c, h, w, oc, k):
+    """Launches with few blocks split a block's k-steps between groups of waves and add the groups' sums up at the end."""
+    pad = ((k // 2, k // 2), (k // 2, k // 2))
+    run_case(hip_ctx, n, c, h, w, oc, k, k, (1, 1), pad, (1, 1), 1, seed=c + oc + k)
+
+
 @pytest.mark.parametrize("zw", [0, 1, 2, 127, 128, 129, 254, 255])
 @pytest.mark.parametrize("cin,k,pad", [(16, 1, 0), (24, 1, 0), (32, 1, 0), (3, 3, 1), (8, 2, 0), (33, 1, 0), (48, 1, 0)])
 def test_short_reductions_for_every_weight_zero_point(hip_ctx, zw, cin, k, pad):
