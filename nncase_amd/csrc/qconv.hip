@@ -29,7 +29,7 @@ void nnhip::describe_conv_kernel(const nncase_hip_ctx *ctx, const nncase_hip_wei
         snprintf(buf, cap, "qconv_smallc<C=%d>", w->in_channels);
         return;
     }
-    static const char *modes[] = {"rows16", "vec16", "vec8", "vec4", "bytes", "rows8"};
+    static const char *modes[] = {"rows16", "vec16", "vec8", "rows8"};
     const int out_h = windowed_output_size(a->in_h, w->kernel_h, a->stride_h, a->dilation_h, a->pad_h_before, a->pad_h_after);
     const int out_w = windowed_output_size(a->in_w, w->kernel_w, a->stride_w, a->dilation_w, a->pad_w_before, a->pad_w_after);
     if (rows_path_taken(w, a, out_h, out_w)) {
@@ -42,7 +42,7 @@ void nnhip::describe_conv_kernel(const nncase_hip_ctx *ctx, const nncase_hip_wei
     if (w->wide) {
         snprintf(buf, cap, "qconv_wide%s%s%s<T=%d,%s%s>", w->d_post_lut ? "+lut" : "", a->residual_dev ? "+add" : "",
                  a->dequantize_output ? "+dequantize" : "", w->tiles,
-                 w->wide == 2 ? "RG=2," : "", modes[mode]);
+                 w->wide == 2 ? "RG=2," : "", w->ragged ? "ragged" : modes[mode]);
         return;
     }
     snprintf(buf, cap, "qconv_igemm%s%s%s<T=%d,RG=%d,%s>", w->d_post_lut ? "+lut" : "", a->residual_dev ? "+add" : "",

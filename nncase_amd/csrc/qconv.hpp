@@ -8,7 +8,9 @@ struct nncase_hip_weights {
     int kind = kIgemm;
     int in_channels = 0, out_channels = 0, kernel_h = 0, kernel_w = 0, groups = 1;
     int g_ic = 0, g_oc = 0; // channels per group
-    int k = 0;              // reduction length per group: kernel_h * kernel_w * g_ic
+    int tap_ic = 0;         // igemm: channels per tap in the packed reduction: g_ic, or the next multiple of 16 (`ragged`)
+    bool ragged = false;    // ... the surplus channels carrying the weight zero point (qconv_wide.hpp, kWideRagRows)
+    int k = 0;              // reduction length per group: kernel_h * kernel_w * tap_ic
     int ksteps = 0;         // ceil(k / 64)
     int tiles = 0;          // 16-channel MFMA tiles per channel chunk (T)
     int nchunks = 0;        // channel chunks per group

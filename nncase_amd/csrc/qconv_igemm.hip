@@ -20,8 +20,7 @@ static int round_tiles(int t) {
 // activation fragment for more output channels; narrow ones give more blocks.  With a
 // pixel-count hint the widest chunk that still yields about two blocks per compute unit
 // (at the smallest pixel tile) is taken; without one, the widest that fits the LDS budget.
-// max_tiles bounds T (the byte-gather loader is only built for T <= 4).
-static void plan_igemm(int g_oc, int ksteps, int max_tiles, int64_t pixels_hint, int compute_units, int *tiles, int *nchunks,
+static void plan_igemm(int g_oc, int ksteps, int64_t pixels_hint, int compute_units, int *tiles, int *nchunks,
                        int *kc_steps) {
     const int tt = ceil_div(g_oc, 16);
     const long long target = 2LL * compute_units;
@@ -29,7 +28,6 @@ static void plan_igemm(int g_oc, int ksteps, int max_tiles, int64_t pixels_hint,
     for (int nc = 1; nc <= tt; nc++) {
         if (ceil_div(tt, nc) > 16) continue; // more tiles than the widest kernel
         const int t = round_tiles(ceil_div(tt, nc));
-        if (t > max_tiles) continue;
         int kc;
         if (ksteps * t <= kLdsFrags) kc = ksteps;              // whole reduction resident
         else if (ksteps > 12 && t <= 4) kc = kLdsFrags / t;     // long reduction: staged in pieces
@@ -44,15 +42,25 @@ static void plan_igemm(int g_oc, int ksteps, int max_tiles, int64_t pixels_hint,
     *kc_steps = best_kc;
 }
 
+// Whether a layer whose channels per group are no multiple of 16 is packed with its taps rounded up to 16 channels, for the
+// ragged loader of the wide kernels.  Multiples of 8 with a short reduction stay with the small tiles (8-byte pieces; us, ragged
+// against those: 25 088 pixels 24 -> 64 1x1 4.8 / 4.4, 8 -> 16 3x3 stride 2 5.8 / 4.5; from five k-steps on 24 -> 64 3x3 6.9 / 7.9,
+// 72 -> 64 3x3 9.3 / 13.4).  For anything else the small tiles gathered dwords or bytes (8893 pixels 90 -> 203 3x3 stride 2 61 us,
+// now 13.8; 3001 x 1000 product of one row 139, 9.5; of 5000 rows with 2100 columns 876, 82).
+static bool ragged_pays(int g_ic, int taps) {
+    return g_ic % 8 != 0 || ceil_div(taps * ceil_div(g_ic, 16) * 16, 64) >= kSmallWideMinKsteps;
+}
+
 int prepack_igemm(nncase_hip_ctx *ctx, nncase_hip_weights *w, const uint8_t *w_oihw, const int32_t *bias) {
     const int taps = w->kernel_h * w->kernel_w;
     NNHIP_REQUIRE(ctx, (int64_t)taps * w->g_ic < 65536, -EINVAL,
                   "qconv2d_prepack: reduction length %lld would overflow the int32 accumulator",
                   (long long)taps * w->g_ic);
-    w->k = taps * w->g_ic;
+    w->tap_ic = w->g_ic;
+    if (w->g_ic % 16 != 0 && ragged_pays(w->g_ic, taps)) w->ragged = true, w->tap_ic = ceil_div(w->g_ic, 16) * 16;
+    w->k = taps * w->tap_ic;
     w->ksteps = ceil_div(w->k, 64);
-    const int max_tiles = (w->g_ic % 4 == 0) ? 16 : 4;
-    plan_igemm(w->g_oc, w->ksteps, max_tiles, w->pixels_hint, ctx->compute_units, &w->tiles, &w->nchunks, &w->kc_steps);
+    plan_igemm(w->g_oc, w->ksteps, w->pixels_hint, ctx->compute_units, &w->tiles, &w->nchunks, &w->kc_steps);
     // Long reductions over many pixels and more than 64 channels are bound by the matrix cores: they take the
     // wide-tile kernels (a wave owns 64 pixels x 64 or 128 channels) when the launch has a 256-pixel block for every
     // compute unit; smaller launches keep the small tiles, whose larger wave count fills the device better.  (Up to 64
@@ -60,8 +68,8 @@ int prepack_igemm(nncase_hip_ctx *ctx, nncase_hip_weights *w, const uint8_t *w_o
     {
         const long long ptiles = ceil_div((int)std::min<int64_t>(std::max<int64_t>(w->pixels_hint, 0), 1 << 30), 256);
         // 256-channel chunks (two waves side by side share the block's activations) where that still fills the device
-        const int wide_tiles = (w->g_oc > 128 && ptiles * ceil_div(w->g_oc, 256) >= ctx->compute_units ? 16 : 8);
-        w->wide = w->g_ic % 16 == 0 && w->ksteps >= kWideMinKsteps && w->g_oc > 64 &&
+        const int wide_tiles = (w->g_oc > 128 && ptiles * ceil_div(w->g_oc, 256) >= ctx->compute_units && !w->ragged ? 16 : 8);
+        w->wide = w->tap_ic % 16 == 0 && w->ksteps >= kWideMinKsteps && w->g_oc > 64 &&
                   ptiles * ceil_div(w->g_oc, wide_tiles * 16) >= ctx->compute_units;
         if (w->wide) {
             w->tiles = wide_tiles;
@@ -72,7 +80,7 @@ int prepack_igemm(nncase_hip_ctx *ctx, nncase_hip_weights *w, const uint8_t *w_o
     // Reductions of kSmallWideMinKsteps k-steps and more over fewer pixels take the same kernel with blocks of 8192 or 2048
     // outputs: against the small tiles' per-lane loads of 16 pixels' slices, the row-order fetch through LDS needs a
     // quarter of the requests to the vector L1, which is what such launches are bound by.
-    if (!w->wide && w->g_ic % 16 == 0 && w->ksteps >= kSmallWideMinKsteps) {
+    if (!w->wide && (w->ragged || (w->g_ic % 16 == 0 && w->ksteps >= kSmallWideMinKsteps))) {
         w->wide = 2;
         // (2048 outputs per block while the larger ones would leave more than half of the compute units without a block:
         // the 512 x 1024 x 1024 product takes 7.0 us with them, 9.2 us with 64 blocks of 8192)
@@ -89,18 +97,19 @@ int prepack_igemm(nncase_hip_ctx *ctx, nncase_hip_weights *w, const uint8_t *w_o
         w->kc_steps = std::min(w->ksteps, kLdsFrags / w->tiles);
     }
     // -(zw - 128) has to be an s8 value
-    w->fold = w->ksteps == 1 && w->k <= 32 && w->zw >= 1;
+    w->fold = !w->ragged && w->ksteps == 1 && w->k <= 32 && w->zw >= 1;
     const size_t group_bytes = (size_t)w->nchunks * w->ksteps * w->tiles * 1024;
     w->packed_bytes = group_bytes * w->groups;
     std::vector<uint8_t> packed(w->packed_bytes);
     std::vector<int32_t> wsum(w->out_channels), hb(w->out_channels, 0);
     if (bias) std::copy(bias, bias + w->out_channels, hb.begin());
     for (int32_t b : hb) w->bias_absmax = std::max<long long>(w->bias_absmax, std::llabs((long long)b));
-    const int g_ic = w->g_ic, kh = w->kernel_h, kw = w->kernel_w;
+    const int g_ic = w->g_ic, tap_ic = w->tap_ic, kh = w->kernel_h, kw = w->kernel_w;
     for (int g = 0; g < w->groups; g++) {
         const uint8_t *wg = w_oihw + (size_t)g * w->g_oc * g_ic * kh * kw;
         auto w_at = [&](int oc, int kk) -> uint8_t {
-            const int tap = kk / g_ic, ic = kk % g_ic;
+            const int tap = kk / tap_ic, ic = kk % tap_ic;
+            if (ic >= g_ic) return (uint8_t)w->zw;
             return wg[((size_t)oc * g_ic + ic) * kh * kw + tap]; // OIHW: tap = ky * kw + kx
         };
         pack_group(packed.data() + g * group_bytes, wsum.data() + (size_t)g * w->g_oc, w->g_oc, w->k, w->ksteps, w->tiles,
@@ -119,14 +128,16 @@ int igemm_pixel_groups(const nncase_hip_ctx *ctx, const nncase_hip_weights *w, i
     return choose_rg(ctx, w->tiles, w->nchunks, m);
 }
 
+static bool igemm_is_pointwise(const nncase_hip_weights *w, const nncase_hip_conv2d_args_t *c, int out_h, int out_w) {
+    return w->kernel_h == 1 && w->kernel_w == 1 && c->stride_h == 1 && c->stride_w == 1 && c->pad_h_before == 0 && c->pad_w_before == 0 &&
+           out_h == c->in_h && out_w == c->in_w;
+}
+
 int igemm_load_mode(const nncase_hip_weights *w, const nncase_hip_conv2d_args_t *c, int out_h, int out_w) {
-    const bool pointwise = w->kernel_h == 1 && w->kernel_w == 1 && c->stride_h == 1 && c->stride_w == 1 &&
-                           c->pad_h_before == 0 && c->pad_w_before == 0 && out_h == c->in_h && out_w == c->in_w;
+    const bool pointwise = igemm_is_pointwise(w, c, out_h, out_w);
     if (w->g_ic % 16 == 0) return pointwise ? kRows16 : kVec16;
     // (the row loader reads 16 bytes at a time: the tensor has to hold that many)
-    if (w->g_ic % 8 == 0) return pointwise && (int64_t)c->batch * c->in_h * c->in_w * w->in_channels >= 16 ? kRows8 : kVec8;
-    if (w->g_ic % 4 == 0) return kVec4;
-    return kBytes;
+    return pointwise && (int64_t)c->batch * c->in_h * c->in_w * w->in_channels >= 16 ? kRows8 : kVec8; // (anything else is ragged)
 }
 
 int launch_qconv_igemm(nncase_hip_ctx *ctx, const uint8_t *x, const nncase_hip_weights *w, void *y,
@@ -160,9 +171,10 @@ int launch_qconv_igemm(nncase_hip_ctx *ctx, const uint8_t *x, const nncase_hip_w
                   -EINVAL, "qconv2d: %d output channels at offset %d do not fit a pixel stride of %d", w->out_channels, c->out_channel_offset,
                   c->out_channel_stride);
     NNHIP_REQUIRE(ctx, m64 * a.ldy * out_es < ((int64_t)1 << 40), -EINVAL, "qconv2d: output too large");
-    a.g_ic = w->g_ic;
+    a.g_ic = w->tap_ic;
     a.in_h = c->in_h;
     a.in_w = c->in_w;
+    a.kh = w->kernel_h;
     a.kw = w->kernel_w;
     a.stride_h = c->stride_h;
     a.stride_w = c->stride_w;
@@ -173,7 +185,7 @@ int launch_qconv_igemm(nncase_hip_ctx *ctx, const uint8_t *x, const nncase_hip_w
     a.d_ohow = make_fastdiv((uint32_t)(out_h * out_w));
     a.d_ow = make_fastdiv((uint32_t)out_w);
     a.d_kw = make_fastdiv((uint32_t)w->kernel_w);
-    a.d_gic = make_fastdiv((uint32_t)w->g_ic);
+    a.d_gic = make_fastdiv((uint32_t)w->tap_ic);
     a.zxp = c->x_qp.zero_point - 128;
     a.zwp = w->zw - 128;
     a.zwp_rows = w->fold ? 0 : a.zwp;
@@ -206,6 +218,12 @@ int launch_qconv_igemm(nncase_hip_ctx *ctx, const uint8_t *x, const nncase_hip_w
         a.y_coff = g * w->g_oc + c->out_channel_offset;
         a.r_coff = g * w->g_oc;
         int rc;
+        if (w->ragged) {
+            const bool rows = igemm_is_pointwise(w, c, out_h, out_w);
+            rc = w->wide == 2 ? launch_wide_small_ragged(ctx, a, rows, w->small_shape, w->nchunks) : launch_wide_ragged(ctx, a, rows, w->tiles, w->nchunks);
+            if (rc) return rc;
+            continue;
+        }
         if (w->wide == 2) {
             rc = mode == kRows16 ? launch_wide_small_rows16(ctx, a, w->small_shape, w->nchunks) : launch_wide_small_vec16(ctx, a, w->small_shape, w->nchunks);
             if (rc) return rc;
@@ -221,9 +239,7 @@ int launch_qconv_igemm(nncase_hip_ctx *ctx, const uint8_t *x, const nncase_hip_w
         case kRows16: rc = launch_igemm_rows16(ctx, a, w->tiles, w->nchunks, rg); break;
         case kVec16: rc = launch_igemm_vec16(ctx, a, w->tiles, w->nchunks, rg); break;
         case kVec8: rc = launch_igemm_vec8(ctx, a, w->tiles, w->nchunks, rg); break;
-        case kRows8: rc = launch_igemm_rows8(ctx, a, w->tiles, w->nchunks, rg); break;
-        case kVec4: rc = launch_igemm_vec4(ctx, a, w->tiles, w->nchunks, rg); break;
-        default: rc = launch_igemm_bytes(ctx, a, w->tiles, w->nchunks, rg); break;
+        default: rc = launch_igemm_rows8(ctx, a, w->tiles, w->nchunks, rg); break;
         }
         if (rc) return rc;
     }

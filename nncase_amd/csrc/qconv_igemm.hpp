@@ -28,9 +28,9 @@
 //   kRows16  1x1 / stride 1 / no padding, channels % 16 == 0: a pixel's
 //            reduction row is contiguous, one 16-byte load per lane and k-step
 //   kRows8   the same for channels % 8 == 0: the last load of a row is half used
-//   kVec16/8/4  any window; channels % VW == 0, so a VW-byte piece of the
+//   kVec16/8 any window; channels % VW == 0, so a VW-byte piece of the
 //            reduction never straddles two taps
-//   kBytes   anything else (e.g. 3 input channels): byte gathers
+// (other channel counts: the ragged loader of qconv_wide.hpp)
 #pragma once
 
 #include <mutex>
@@ -49,7 +49,7 @@ constexpr int kThreads = 256;
 constexpr int kWaves = 4;
 constexpr int kLdsFrags = 48; // weight fragments (1 KiB each) resident in LDS per block
 
-enum LoadMode { kRows16 = 0, kVec16 = 1, kVec8 = 2, kVec4 = 3, kBytes = 4, kRows8 = 5 };
+enum LoadMode { kRows16 = 0, kVec16 = 1, kVec8 = 2, kRows8 = 3 };
 constexpr bool loads_rows(int mode) { return mode == kRows16 || mode == kRows8; }
 
 struct IgemmArgs {
@@ -66,9 +66,9 @@ struct IgemmArgs {
     size_t x_bytes;        // size of the input tensor
     int ldy, y_coff;       // output pixel stride / channel offset (elements)
     int ldr, r_coff;       // the same for the (dense) residual tensor
-    int g_ic;
+    int g_ic;              // channels per tap in the packed reduction
     int in_h, in_w;
-    int kw, stride_h, stride_w, dil_h, dil_w, pad_h, pad_w;
+    int kh, kw, stride_h, stride_w, dil_h, dil_w, pad_h, pad_w;
     FastDiv d_ohow, d_ow, d_kw, d_gic;
     int zxp, zwp;          // zx - 128, zw - 128
     int zwp_rows;          // zwp where the kernel still owes -zwp * (sum of x') per pixel, 0 where the weights carry it
@@ -200,6 +200,7 @@ __device__ __forceinline__ v4i finish_act(const ActFrag &f) {
 }
 
 template <int MODE> __device__ __forceinline__ ActFrag load_act(const IgemmArgs &a, const PixInfo &pi, int kc) {
+    static_assert(MODE == kRows8 || MODE == kVec8, "8-byte pieces");
     const u32x4 zero_s8 = {0x80808080u, 0x80808080u, 0x80808080u, 0x80808080u}; // x' = 0
     ActFrag f;
     f.take = 0;
@@ -208,66 +209,30 @@ template <int MODE> __device__ __forceinline__ ActFrag load_act(const IgemmArgs 
     const bool pix_ok = pi.base >= 0;
     PixInfo sp = pi; // any valid pixel for the address
     if (!pix_ok) sp.base = 0, sp.iy0 = 0, sp.ix0 = 0;
-    if (loads_rows(MODE)) {
+    if (MODE == kRows8) {
         const bool in_k = kc * 16 < a.k;
         const int kcc = in_k ? kc : 0;
         const uint32_t off = (uint32_t)sp.base * (uint32_t)a.ldx + a.x_coff + kcc * 16;
-        if (MODE == kRows16) {
-            f.raw = *reinterpret_cast<const u32x4 *>(a.x + (size_t)off);
-            f.take = (pix_ok && in_k) ? 0xfu : 0u;
-        } else {
-            // The last slice of a pixel ends 8 bytes past its channels,
-            // in the next pixel (those two dwords are replaced) or, for the tensor's last pixel, past the tensor:
-            // that one slice is read 8 bytes lower and moved up, so that nothing outside the tensor is touched.
-            const bool over = (size_t)off + 16 > a.x_bytes;
-            const u32x4 v = *reinterpret_cast<const u32x4 *>(a.x + (size_t)(over ? off - 8 : off));
-            f.raw = u32x4{over ? v[2] : v[0], over ? v[3] : v[1], v[2], v[3]};
-            f.take = (pix_ok && in_k) ? (a.k - kcc * 16 >= 16 ? 0xfu : 0x3u) : 0u;
-        }
-    } else if (MODE == kBytes) {
-        // byte gathers: assembled immediately (this loader does not overlap with the multiply)
-        uint32_t w0 = 0x80808080u, w1 = 0x80808080u, w2 = 0x80808080u, w3 = 0x80808080u;
-        if (pix_ok) {
-#pragma unroll
-            for (int b = 0; b < 16; b++) {
-                const int kk = kc * 16 + b;
-                if (kk < a.k) {
-                    bool inside;
-                    const uint32_t off = tap_offset(a, pi, kk, &inside);
-                    const uint32_t byte = inside ? (uint32_t)a.x[(size_t)off] : (a.zx_splat & 0xffu);
-                    const uint32_t clr = ~(0xffu << (8 * (b & 3))), ins = byte << (8 * (b & 3));
-                    if ((b >> 2) == 0) w0 = (w0 & clr) | ins;
-                    if ((b >> 2) == 1) w1 = (w1 & clr) | ins;
-                    if ((b >> 2) == 2) w2 = (w2 & clr) | ins;
-                    if ((b >> 2) == 3) w3 = (w3 & clr) | ins;
-                }
-            }
-        }
-        f.fill = u32x4{w0, w1, w2, w3};
+        // The last slice of a pixel ends 8 bytes past its channels,
+        // in the next pixel (those two dwords are replaced) or, for the tensor's last pixel, past the tensor:
+        // that one slice is read 8 bytes lower and moved up, so that nothing outside the tensor is touched.
+        const bool over = (size_t)off + 16 > a.x_bytes;
+        const u32x4 v = *reinterpret_cast<const u32x4 *>(a.x + (size_t)(over ? off - 8 : off));
+        f.raw = u32x4{over ? v[2] : v[0], over ? v[3] : v[1], v[2], v[3]};
+        f.take = (pix_ok && in_k) ? (a.k - kcc * 16 >= 16 ? 0xfu : 0x3u) : 0u;
     } else {
-        constexpr int VW = MODE == kVec16 ? 16 : (MODE == kVec8 ? 8 : 4);
 #pragma unroll
-        for (int piece = 0; piece < 16 / VW; piece++) {
-            const int kk = kc * 16 + piece * VW;
+        for (int piece = 0; piece < 2; piece++) {
+            const int kk = kc * 16 + piece * 8;
             const bool in_k = kk < a.k;
             bool inside;
             const uint32_t off = tap_offset(a, sp, in_k ? kk : 0, &inside);
             const bool ok = pix_ok && in_k && inside;
             const uint32_t fill = (pix_ok && in_k) ? a.zx_splat : 0x80808080u; // padding tap : outside the problem
-            if (VW == 16) {
-                f.raw = *reinterpret_cast<const u32x4 *>(a.x + (size_t)off);
-                f.fill = u32x4{fill, fill, fill, fill};
-                f.take = ok ? 0xfu : 0u;
-            } else if (VW == 8) {
-                const u32x2 v = *reinterpret_cast<const u32x2 *>(a.x + (size_t)off);
-                f.raw[piece * 2] = v[0], f.raw[piece * 2 + 1] = v[1];
-                f.fill[piece * 2] = fill, f.fill[piece * 2 + 1] = fill;
-                f.take |= ok ? (3u << (piece * 2)) : 0u;
-            } else {
-                f.raw[piece] = *reinterpret_cast<const uint32_t *>(a.x + (size_t)off);
-                f.fill[piece] = fill;
-                f.take |= ok ? (1u << piece) : 0u;
-            }
+            const u32x2 v = *reinterpret_cast<const u32x2 *>(a.x + (size_t)off);
+            f.raw[piece * 2] = v[0], f.raw[piece * 2 + 1] = v[1];
+            f.fill[piece * 2] = fill, f.fill[piece * 2 + 1] = fill;
+            f.take |= ok ? (3u << (piece * 2)) : 0u;
         }
     }
     return f;
@@ -1161,19 +1126,14 @@ template <int MODE> int launch_mode(nncase_hip_ctx *ctx, const IgemmArgs &a, int
     case 2: return launch_t<2, MODE>(ctx, a, nchunks, rg);
     case 3: return launch_t<3, MODE>(ctx, a, nchunks, rg);
     case 4: return launch_t<4, MODE>(ctx, a, nchunks, rg);
+    case 5: return launch_t<5, MODE>(ctx, a, nchunks, rg);
+    case 6: return launch_t<6, MODE>(ctx, a, nchunks, rg);
+    case 8: return launch_t<8, MODE>(ctx, a, nchunks, rg);
+    case 9: return launch_t<9, MODE>(ctx, a, nchunks, rg);
+    case 10: return launch_t<10, MODE>(ctx, a, nchunks, rg);
+    case 12: return launch_t<12, MODE>(ctx, a, nchunks, rg);
+    case 16: return launch_t<16, MODE>(ctx, a, nchunks, rg);
     default: break;
-    }
-    if constexpr (MODE != kBytes) {
-        switch (tiles) {
-        case 5: return launch_t<5, MODE>(ctx, a, nchunks, rg);
-        case 6: return launch_t<6, MODE>(ctx, a, nchunks, rg);
-        case 8: return launch_t<8, MODE>(ctx, a, nchunks, rg);
-        case 9: return launch_t<9, MODE>(ctx, a, nchunks, rg);
-        case 10: return launch_t<10, MODE>(ctx, a, nchunks, rg);
-        case 12: return launch_t<12, MODE>(ctx, a, nchunks, rg);
-        case 16: return launch_t<16, MODE>(ctx, a, nchunks, rg);
-        default: break;
-        }
     }
     return fail(ctx, -EINVAL, "igemm: no kernel for %d tiles (load mode %d)", tiles, MODE);
 }
@@ -1182,7 +1142,5 @@ int launch_igemm_rows16(nncase_hip_ctx *ctx, const IgemmArgs &a, int tiles, int 
 int launch_igemm_vec16(nncase_hip_ctx *ctx, const IgemmArgs &a, int tiles, int nchunks, int rg);
 int launch_igemm_vec8(nncase_hip_ctx *ctx, const IgemmArgs &a, int tiles, int nchunks, int rg);
 int launch_igemm_rows8(nncase_hip_ctx *ctx, const IgemmArgs &a, int tiles, int nchunks, int rg);
-int launch_igemm_vec4(nncase_hip_ctx *ctx, const IgemmArgs &a, int tiles, int nchunks, int rg);
-int launch_igemm_bytes(nncase_hip_ctx *ctx, const IgemmArgs &a, int tiles, int nchunks, int rg);
 
 } // namespace nnhip

@@ -24,6 +24,7 @@ struct SmallCArgs {
     void *y;
     const int32_t *wpk;  // [oc_pad][KDP] packed s8 weights (dwords)
     const int32_t *wsum; // [oc]
+    int32_t wsum_surplus; // what the sums contain for the channels the packed taps were rounded up by
     const int32_t *bias; // [oc]
     int m, oc, oc_pad;
     int in_h, in_w, out_w;
@@ -50,7 +51,7 @@ template <int C, int KW, int KH> __global__ __launch_bounds__(kScThreads) void q
     int32_t *cterm = sc_lds + a.oc_pad * KDP; // [oc_pad]
     for (int i = threadIdx.x; i < a.oc_pad * KDP; i += kScThreads) wl[i] = a.wpk[i];
     for (int i = threadIdx.x; i < a.oc_pad; i += kScThreads)
-        cterm[i] = i < a.oc ? a.bias[i] - a.zxp * a.wsum[i] + a.k * a.zxp * a.zwp : 0;
+        cterm[i] = i < a.oc ? a.bias[i] - a.zxp * (a.wsum[i] - a.wsum_surplus) + a.k * a.zxp * a.zwp : 0;
     __syncthreads();
 
     const int p = blockIdx.x * kScThreads + threadIdx.x;
@@ -191,6 +192,7 @@ int launch_qconv_smallc(nncase_hip_ctx *ctx, const uint8_t *x, const nncase_hip_
     a.y = y;
     a.wpk = reinterpret_cast<const int32_t *>(w->d_smallc);
     a.wsum = w->d_wsum;
+    a.wsum_surplus = w->kernel_h * w->kernel_w * (w->tap_ic - w->g_ic) * (w->zw - 128);
     a.bias = w->d_bias;
     a.m = (int)m64;
     a.oc = w->out_channels;
@@ -205,7 +207,7 @@ int launch_qconv_smallc(nncase_hip_ctx *ctx, const uint8_t *x, const nncase_hip_
     a.in_bytes = (long long)c->batch * c->in_h * c->in_w * w->in_channels;
     a.d_ohow = make_fastdiv((uint32_t)(out_h * out_w));
     a.d_ow = make_fastdiv((uint32_t)out_w);
-    a.k = w->k;
+    a.k = w->kernel_h * w->kernel_w * w->g_ic;
     a.zxp = c->x_qp.zero_point - 128;
     a.zwp = w->zw - 128;
     a.zx_splat = (uint32_t)(c->x_qp.zero_point & 0xff) * 0x01010101u;

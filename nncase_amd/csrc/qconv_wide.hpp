@@ -47,13 +47,35 @@ constexpr int kWideSlots = 3;
 //   kWideRows      contiguous reduction rows, any multiple of 16
 //   kWideTap       windows; channels per group a multiple of 64, so a k-step lies within one tap (scalar tap geometry)
 //   kWideWindow    windows; channels per group a multiple of 16
-enum WideLoad { kWideRowsFull = 0, kWideRows = 1, kWideTap = 2, kWideWindow = 3 };
+//   kWideRagRows, kWideRagWindow   the same two for any other channel count: the reduction is packed as if every tap had the
+//                  next multiple of 16 channels (IgemmArgs::g_ic), the surplus weights equal to the weight zero point,
+//                  so that a piece may run over into whatever follows the tap's channels -- (x - zx)(zw - zw) is 0 for
+//                  any x -- and is fetched from the byte address where it starts, aligned or not
+enum WideLoad { kWideRowsFull = 0, kWideRows = 1, kWideTap = 2, kWideWindow = 3, kWideRagRows = 4, kWideRagWindow = 5 };
 
 typedef uint32_t wide_u32x4 __attribute__((ext_vector_type(4)));
 
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t wide_rsrc(const void *base, uint32_t bytes) {
     // raw buffer (stride 0): offsets are range-checked against `bytes`, reads outside return 0
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(base), 0, (int)bytes, 0x00020000);
+}
+
+struct __attribute__((packed, aligned(1))) wide_unaligned16 {
+    wide_u32x4 v;
+};
+
+// 16 bytes of the tensor x (bytes `bytes`, 16-byte aligned) from any byte offset; what lies outside it is undefined.
+// near_end (wave-uniform) says that a lane's piece may reach past the last byte: it is then put together from aligned
+// dwords, range-checked one by one (the last dword that holds a byte of the tensor never crosses into another page).
+__device__ __forceinline__ wide_u32x4 load_ragged(const uint8_t *x, const __amdgpu_buffer_rsrc_t &dwords, int bytes, int off, bool near_end) {
+    if (!near_end) return reinterpret_cast<const wide_unaligned16 *>(x + (uint32_t)min(max(off, 0), bytes - 16))->v;
+    uint32_t d[5];
+#pragma unroll
+    for (int i = 0; i < 5; i++) d[i] = __builtin_amdgcn_raw_buffer_load_b32(dwords, (off & ~3) + i * 4, 0, 0);
+    wide_u32x4 r;
+#pragma unroll
+    for (int i = 0; i < 4; i++) r[i] = __builtin_amdgcn_alignbyte(d[i + 1], d[i], off & 3);
+    return r;
 }
 
 // T: 16-channel tiles per wave; RG: 16-pixel groups per wave; a block is WM x WN waves: WM * RG * 16 pixels by
@@ -83,7 +105,8 @@ __global__ __launch_bounds__(WM * WN * KG * 64, WM * WN * KG > 8 ? 4 : 2) void q
     static_assert(T % 2 == 0, "channel tiles are multiplied in pairs");
     constexpr int G = T / 2;
     constexpr int SLOT = AV * 16 + WV * 16;             // bytes of a ring slot
-    constexpr bool kRows = LM == kWideRowsFull || LM == kWideRows;
+    constexpr bool kRows = LM == kWideRowsFull || LM == kWideRows || LM == kWideRagRows;
+    constexpr bool kRagged = LM == kWideRagRows || LM == kWideRagWindow;
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
     int32_t *cterm = reinterpret_cast<int32_t *>(smem);              // [TB * 16]
     uint8_t *lutl = smem + TB * 16 * sizeof(int32_t);                // [256]
@@ -110,7 +133,7 @@ __global__ __launch_bounds__(WM * WN * KG * 64, WM * WN * KG > 8 ? 4 : 2) void q
     const int KS = a.ksteps;
     const int KL = KG == 1 ? KS : (KS - kg + KG - 1) / KG; // k-steps of this group: kg, kg + KG, ... (the loop counts them from 0)
     const __amdgpu_buffer_rsrc_t wres = wide_rsrc(a.wpk + (size_t)chunk * KS * TB * 1024, (uint32_t)KS * TB * 1024);
-    const __amdgpu_buffer_rsrc_t xres = wide_rsrc(a.x, (uint32_t)a.x_bytes);
+    const __amdgpu_buffer_rsrc_t xres = wide_rsrc(a.x, kRagged ? ((uint32_t)a.x_bytes + 3) & ~3u : (uint32_t)a.x_bytes);
 
     // per-channel constant of the zero-point identity and the byte table: requested now, needed by the epilogue
     constexpr int NC = (TB * 16 + BLOCK - 1) / BLOCK;
@@ -159,6 +182,17 @@ __global__ __launch_bounds__(WM * WN * KG * 64, WM * WN * KG > 8 ? 4 : 2) void q
             p_off[i] = ((ok ? pi.base : 0) + p_iy0[i] * a.in_w + p_ix0[i]) * a.ldx + a.x_coff + (LM == kWideTap ? lq * 16 : 0);
         }
     }
+    bool near_end = kRagged && a.x_bytes < 16; // (ragged: some lane's last piece may reach past the tensor)
+    if (kRagged) {
+        const int last = kRows ? a.k - 16 - lq * 16 : (((a.kh - 1) * a.dil_h * a.in_w + (a.kw - 1) * a.dil_w) * a.ldx + a.g_ic - 16);
+#pragma unroll
+        for (int i = 0; i < NA; i++) near_end = near_end || (int64_t)p_off[i] + last + 16 > (int64_t)a.x_bytes;
+        near_end = __any(near_end);
+    }
+    auto fetch = [&](int off) __attribute__((always_inline)) {
+        if constexpr (kRagged) return load_ragged(a.x, xres, (int)a.x_bytes, off, near_end);
+        else return __builtin_amdgcn_raw_buffer_load_b128(xres, off, 0, 0);
+    };
     struct Acts {
         wide_u32x4 raw[NA];
         uint32_t fill;    // what a piece that is not taken holds: the zero point (padding tap) or x' = 0 (past the reduction)
@@ -173,12 +207,12 @@ __global__ __launch_bounds__(WM * WN * KG * 64, WM * WN * KG > 8 ? 4 : 2) void q
                 f.take[i] = true;
             }
             f.fill = 0;
-        } else if (LM == kWideRows) {
+        } else if (LM == kWideRows || LM == kWideRagRows) {
             // the last k-step may end inside the row: the piece's offset goes through the range-checked operand
             const bool in_k = ksc * 64 + lq * 16 < a.k;
 #pragma unroll
             for (int i = 0; i < NA; i++) {
-                f.raw[i] = __builtin_amdgcn_raw_buffer_load_b128(xres, p_off[i] + ksc * 64, 0, 0);
+                f.raw[i] = fetch(p_off[i] + ksc * 64);
                 f.take[i] = in_k;
             }
             f.fill = 0x80808080u;
@@ -207,7 +241,7 @@ __global__ __launch_bounds__(WM * WN * KG * 64, WM * WN * KG > 8 ? 4 : 2) void q
             const int shift = (dy * a.in_w + dx) * a.ldx + c;
 #pragma unroll
             for (int i = 0; i < NA; i++) {
-                f.raw[i] = __builtin_amdgcn_raw_buffer_load_b128(xres, p_off[i] + shift, 0, 0);
+                f.raw[i] = fetch(p_off[i] + shift);
                 f.take[i] = in_k && (unsigned)(p_iy0[i] + dy) < (unsigned)a.in_h && (unsigned)(p_ix0[i] + dx) < (unsigned)a.in_w;
             }
             f.fill = in_k ? a.zx_splat : 0x80808080u;
@@ -1056,7 +1090,9 @@ template <int T, int WM, int WN, int LM> int launch_wide_small_t(nncase_hip_ctx 
 
 // Block shapes: tiles = 16 -> 256 pixels x 256 channels (4 x 2 waves); tiles = 8 -> 256 or 128 pixels x 128 channels.
 template <int LM> int launch_wide_lm(nncase_hip_ctx *ctx, const IgemmArgs &a, int tiles, int nchunks) {
-    if (tiles == 16) {
+    if constexpr (LM == kWideRagRows || LM == kWideRagWindow) {
+        if (tiles == 16) return fail(ctx, -EINVAL, "qconv2d: no 256-channel blocks for ragged rows");
+    } else if (tiles == 16) {
         if constexpr (LM == kWideRowsFull || LM == kWideRows) {
             if (a.x_bytes < ((size_t)1 << 31)) return launch_wide_dma_t<8, 4, 4, 2, LM>(ctx, a, nchunks);
         }
@@ -1080,5 +1116,7 @@ int launch_wide_small_rows16(nncase_hip_ctx *ctx, const IgemmArgs &a, int shape,
 int launch_wide_small_vec16(nncase_hip_ctx *ctx, const IgemmArgs &a, int shape, int nchunks);
 int launch_wide_rows16(nncase_hip_ctx *ctx, const IgemmArgs &a, int tiles, int nchunks);
 int launch_wide_vec16(nncase_hip_ctx *ctx, const IgemmArgs &a, int tiles, int nchunks);
+int launch_wide_ragged(nncase_hip_ctx *ctx, const IgemmArgs &a, bool rows, int tiles, int nchunks);
+int launch_wide_small_ragged(nncase_hip_ctx *ctx, const IgemmArgs &a, bool rows, int shape, int nchunks);
 
 } // namespace nnhip
