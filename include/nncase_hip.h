@@ -110,6 +110,11 @@ NNCASE_HIP_API int nncase_hip_malloc(nncase_hip_ctx_t *ctx, size_t bytes, void *
 NNCASE_HIP_API int nncase_hip_free(nncase_hip_ctx_t *ctx, void *dptr);
 NNCASE_HIP_API int nncase_hip_memcpy_h2d(nncase_hip_ctx_t *ctx, void *dst_dev, const void *src_host, size_t bytes);
 NNCASE_HIP_API int nncase_hip_memcpy_d2h(nncase_hip_ctx_t *ctx, void *dst_host, const void *src_dev, size_t bytes);
+/* Pinned host memory for results: a device-to-host copy into it runs at the speed of the bus.  Blocks are kept for the next
+ * request, at most 256 MiB in all (-ENOMEM beyond: take ordinary memory) and none after the last context; a block stays
+ * valid until it is freed, its context's end included.  Any thread may free. */
+NNCASE_HIP_API int nncase_hip_host_malloc(nncase_hip_ctx_t *ctx, size_t bytes, void **ptr);
+NNCASE_HIP_API int nncase_hip_host_free(void *ptr);
 NNCASE_HIP_API int nncase_hip_memset(nncase_hip_ctx_t *ctx, void *dptr, int byte, size_t bytes);
 NNCASE_HIP_API int nncase_hip_stream_sync(nncase_hip_ctx_t *ctx);
 
@@ -375,6 +380,17 @@ typedef struct nncase_hip_matmul_args {
 
 NNCASE_HIP_API int nncase_hip_qmatmul(nncase_hip_ctx_t *ctx, const uint8_t *a_dev, const nncase_hip_weights_t *weights,
                                       void *y_dev, const nncase_hip_matmul_args_t *args);
+
+/* The same operators on HOST tensors, as the reference's kernels take them: one call brings activations, weights and bias
+ * to the device, packs, multiplies and brings the result back (it is complete when the call returns).  Activations and
+ * result are NCHW, weights OIHW; dense and grouped convolutions without fused residual or table.  desc.expected_pixels is
+ * ignored. */
+NNCASE_HIP_API int nncase_hip_qconv2d_host(nncase_hip_ctx_t *ctx, const nncase_hip_conv2d_desc_t *desc, const uint8_t *x_nchw_host,
+                                           const uint8_t *weights_oihw_host, const int32_t *bias_host, void *y_nchw_host,
+                                           const nncase_hip_conv2d_args_t *args);
+NNCASE_HIP_API int nncase_hip_qmatmul_host(nncase_hip_ctx_t *ctx, const uint8_t *a_host, const uint8_t *b_host, int32_t k, int32_t n,
+                                           nncase_hip_quant_param_t b_qp, const int32_t *bias_host, void *y_host,
+                                           const nncase_hip_matmul_args_t *args);
 
 /* ---- u8 glue that keeps a quantized graph resident --------------------- */
 

@@ -31,6 +31,12 @@ struct nncase_hip_ctx {
     // this GPU's copy of the static scratch of nncase_hip_paged_attention_decode_noalloc (its device address, taken
     // when the context is created so that the entry point itself makes no runtime call but launches)
     void *attn_static = nullptr;
+    // hostcall.hip: pinned host memory through which small operands travel (in flight until a host call has drained the
+    // stream), and device scratch of calls on host tensors; both made on first use, bounded, kept with the context
+    uint8_t *stage = nullptr;
+    size_t stage_used = 0;
+    void *arena = nullptr;
+    size_t arena_bytes = 0;
     char last_error[512] = {0};
 };
 
@@ -39,6 +45,12 @@ namespace nnhip {
 // Device address of the static scratch array of the attention entry point that allocates nothing, on `device`
 // (which must be current).  attn.hip, where the array lives.
 hipError_t attn_static_scratch_address(void **ptr);
+
+// hostcall.hip: device scratch of at least `bytes`, valid until the next call (`*temporary`: larger than what a context
+// keeps, the caller gives it back with hipFree when the stream has drained); what a context holds for host calls.
+int scratch_reserve(nncase_hip_ctx *ctx, size_t bytes, void **ptr, bool *temporary);
+void hostcall_attach();
+void hostcall_release(nncase_hip_ctx *ctx);
 
 inline int fail(nncase_hip_ctx *ctx, int code, const char *fmt, ...) {
     if (ctx) {

@@ -38,6 +38,7 @@ extern "C" int nncase_hip_ctx_create(int device, nncase_hip_ctx_t **out) {
         delete ctx;
         return e != hipSuccess ? -(NNCASE_HIP_ERR_HIP_BASE + (int)e) : -ENOMEM;
     }
+    hostcall_attach();
     *out = ctx;
     return 0;
 }
@@ -95,6 +96,7 @@ extern "C" int nncase_hip_ctx_destroy(nncase_hip_ctx_t *ctx) {
     if (ctx->stream) (void)hipStreamSynchronize(ctx->stream);
     if (ctx->attn_ws) (void)hipFree(ctx->attn_ws);
     if (ctx->attn_done) (void)hipFree(ctx->attn_done);
+    hostcall_release(ctx);
     if (ctx->owns_stream && ctx->stream) (void)hipStreamDestroy(ctx->stream);
     delete ctx;
     return 0;

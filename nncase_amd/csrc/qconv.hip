@@ -11,7 +11,6 @@
 #include <vector>
 
 namespace nnhip {
-int prepack_igemm(nncase_hip_ctx *ctx, nncase_hip_weights *w, const uint8_t *w_oihw, const int32_t *bias);
 int prepack_depthwise(nncase_hip_ctx *ctx, nncase_hip_weights *w, const uint8_t *w_oihw, const int32_t *bias);
 } // namespace nnhip
 
@@ -273,8 +272,10 @@ int nnhip::make_residual_epilogue(nncase_hip_ctx *ctx, ResidualEpilogue *rep, co
 static void free_weights(nncase_hip_weights *w) {
     if (!w) return;
     if (w->d_packed) (void)hipFree(w->d_packed);
-    if (w->d_wsum) (void)hipFree(w->d_wsum);
-    if (w->d_bias) (void)hipFree(w->d_bias);
+    if (w->kind == nncase_hip_weights::kDepthwise) { // (dense layers: inside d_packed's block)
+        if (w->d_wsum) (void)hipFree(w->d_wsum);
+        if (w->d_bias) (void)hipFree(w->d_bias);
+    }
     if (w->d_smallc) (void)hipFree(w->d_smallc);
     if (w->d_post_lut) (void)hipFree(w->d_post_lut);
     rows_free(w);
@@ -321,22 +322,15 @@ extern "C" int nncase_hip_requant_host_magic(float sx, float sw, nncase_hip_quan
     return 1;
 }
 
-extern "C" int nncase_hip_qconv2d_prepack(nncase_hip_ctx_t *ctx, const nncase_hip_conv2d_desc_t *desc,
-                                          const uint8_t *weights_oihw_host, const int32_t *bias_host,
-                                          nncase_hip_weights_t **weights) {
-    NNHIP_CHECK_CTX(ctx);
-    NNHIP_REQUIRE(ctx, desc && weights_oihw_host && weights, -EINVAL, "qconv2d_prepack: null argument");
-    *weights = nullptr;
+int nnhip::describe_weights(nncase_hip_ctx *ctx, nncase_hip_weights *w, const nncase_hip_conv2d_desc_t *desc, const char *who) {
     NNHIP_REQUIRE(ctx, desc->in_channels > 0 && desc->out_channels > 0 && desc->kernel_h > 0 && desc->kernel_w > 0,
-                  -EINVAL, "qconv2d_prepack: non-positive dimension");
+                  -EINVAL, "%s: non-positive dimension", who);
     NNHIP_REQUIRE(ctx, desc->groups > 0 && desc->in_channels % desc->groups == 0 &&
                            desc->out_channels % desc->groups == 0,
-                  -NNCASE_HIP_ERR_SHAPE_MISMATCH, "qconv2d_prepack: groups=%d does not divide channels %d/%d",
+                  -NNCASE_HIP_ERR_SHAPE_MISMATCH, "%s: groups=%d does not divide channels %d/%d", who,
                   desc->groups, desc->in_channels, desc->out_channels);
     NNHIP_REQUIRE(ctx, desc->w_qp.zero_point >= 0 && desc->w_qp.zero_point <= 255, -EINVAL,
-                  "qconv2d_prepack: weight zero point %d outside u8", desc->w_qp.zero_point);
-    nncase_hip_weights *w = new (std::nothrow) nncase_hip_weights();
-    NNHIP_REQUIRE(ctx, w, -ENOMEM, "qconv2d_prepack: out of host memory");
+                  "%s: weight zero point %d outside u8", who, desc->w_qp.zero_point);
     w->in_channels = desc->in_channels;
     w->out_channels = desc->out_channels;
     w->kernel_h = desc->kernel_h;
@@ -349,17 +343,78 @@ extern "C" int nncase_hip_qconv2d_prepack(nncase_hip_ctx_t *ctx, const nncase_hi
     w->pixels_hint = desc->expected_pixels > 0 ? desc->expected_pixels : 0;
     const bool depthwise = desc->groups > 1 && w->g_ic == 1 && w->g_oc == 1;
     w->kind = depthwise ? nncase_hip_weights::kDepthwise : nncase_hip_weights::kIgemm;
-    NNHIP_HIP(ctx, hipSetDevice(ctx->device));
-    int rc = depthwise ? prepack_depthwise(ctx, w, weights_oihw_host, bias_host)
-                       : prepack_igemm(ctx, w, weights_oihw_host, bias_host);
-    if (rc == 0 && !depthwise && smallc_supported(w)) rc = prepack_smallc(ctx, w, weights_oihw_host);
-    if (rc == 0 && !depthwise) rc = rows_prepack(ctx, w, weights_oihw_host);
+    return 0;
+}
+
+// Packs a dense layer: the bytes go up as they are and are brought into operand order on the device.
+static int prepack_igemm(nncase_hip_ctx *ctx, nncase_hip_weights *w, const RawWeights &raw_host, const int32_t *bias) {
+    int rc = igemm_plan(ctx, w, bias);
+    if (rc) return rc;
+    void *block = nullptr, *raw = nullptr;
+    bool temporary = false;
+    NNHIP_HIP(ctx, hipMalloc(&block, igemm_const_bytes(w)));
+    igemm_place(w, block);
+    const size_t bytes = (size_t)w->out_channels * w->g_ic * w->kernel_h * w->kernel_w;
+    rc = scratch_reserve(ctx, bytes, &raw, &temporary);
+    if (rc) return rc;
+    RawWeights dev = raw_host;
+    dev.ptr = reinterpret_cast<const uint8_t *>(raw);
+    hipError_t e = hipMemcpyAsync(raw, raw_host.ptr, bytes, hipMemcpyHostToDevice, ctx->stream);
+    if (e == hipSuccess) rc = igemm_pack(ctx, w, dev);
+    if (e == hipSuccess && !rc)
+        e = bias ? hipMemcpyAsync(w->d_bias, bias, sizeof(int32_t) * w->out_channels, hipMemcpyHostToDevice, ctx->stream)
+                 : hipMemsetAsync(w->d_bias, 0, sizeof(int32_t) * w->out_channels, ctx->stream);
+    const hipError_t done = hipStreamSynchronize(ctx->stream); // the host's arrays are free, the weights good on any stream
+    if (temporary) (void)hipFree(raw);
+    if (rc) return rc;
+    NNHIP_HIP(ctx, e);
+    NNHIP_HIP(ctx, done);
+    return 0;
+}
+
+// kn: `weights` is a [in_channels, out_channels] matrix instead of OIHW
+static int prepack(nncase_hip_ctx *ctx, const nncase_hip_conv2d_desc_t *desc, const uint8_t *weights_host, bool kn, const int32_t *bias_host,
+                   nncase_hip_weights_t **weights) {
+    nncase_hip_weights *w = new (std::nothrow) nncase_hip_weights();
+    NNHIP_REQUIRE(ctx, w, -ENOMEM, "qconv2d_prepack: out of host memory");
+    int rc = describe_weights(ctx, w, desc, "qconv2d_prepack");
+    const bool depthwise = w->kind == nncase_hip_weights::kDepthwise;
+    if (rc == 0) {
+        const hipError_t e = hipSetDevice(ctx->device);
+        if (e != hipSuccess) rc = hip_fail(ctx, e, "hipSetDevice");
+    }
+    if (rc == 0) {
+        const int64_t taps = (int64_t)w->kernel_h * w->kernel_w;
+        const RawWeights raw = kn ? RawWeights{weights_host, 1, w->out_channels, 0}
+                                  : RawWeights{weights_host, w->g_ic * taps, taps, (size_t)(w->g_oc * w->g_ic * taps)};
+        rc = depthwise ? prepack_depthwise(ctx, w, weights_host, bias_host) : prepack_igemm(ctx, w, raw, bias_host);
+    }
+    if (rc == 0 && !depthwise && smallc_supported(w)) rc = prepack_smallc(ctx, w, weights_host);
+    if (rc == 0 && !depthwise && rows_wanted(w)) {
+        std::vector<uint8_t> transposed;
+        if (kn) { // B[K,N] row-major is a 1x1 convolution's OIHW weight [N,K,1,1] transposed
+            const int k = w->in_channels, n = w->out_channels;
+            transposed.resize((size_t)k * n);
+            for (int kk = 0; kk < k; kk++)
+                for (int j = 0; j < n; j++) transposed[(size_t)j * k + kk] = weights_host[(size_t)kk * n + j];
+        }
+        rc = rows_prepack(ctx, w, kn ? transposed.data() : weights_host, bias_host);
+    }
     if (rc) {
         free_weights(w);
         return rc;
     }
     *weights = w;
     return 0;
+}
+
+extern "C" int nncase_hip_qconv2d_prepack(nncase_hip_ctx_t *ctx, const nncase_hip_conv2d_desc_t *desc,
+                                          const uint8_t *weights_oihw_host, const int32_t *bias_host,
+                                          nncase_hip_weights_t **weights) {
+    NNHIP_CHECK_CTX(ctx);
+    NNHIP_REQUIRE(ctx, desc && weights_oihw_host && weights, -EINVAL, "qconv2d_prepack: null argument");
+    *weights = nullptr;
+    return prepack(ctx, desc, weights_oihw_host, false, bias_host, weights);
 }
 
 extern "C" int nncase_hip_weights_destroy(nncase_hip_ctx_t *ctx, nncase_hip_weights_t *weights) {
@@ -455,10 +510,7 @@ extern "C" int nncase_hip_qmatmul_prepack(nncase_hip_ctx_t *ctx, const uint8_t *
     NNHIP_CHECK_CTX(ctx);
     NNHIP_REQUIRE(ctx, b_host && weights, -EINVAL, "qmatmul_prepack: null argument");
     NNHIP_REQUIRE(ctx, k > 0 && n > 0, -EINVAL, "qmatmul_prepack: non-positive dimension");
-    // B[K,N] row-major is a 1x1 convolution's OIHW weight [N,K,1,1] transposed.
-    std::vector<uint8_t> bt((size_t)k * n);
-    for (int kk = 0; kk < k; kk++)
-        for (int j = 0; j < n; j++) bt[(size_t)j * k + kk] = b_host[(size_t)kk * n + j];
+    *weights = nullptr;
     nncase_hip_conv2d_desc_t d;
     d.in_channels = k;
     d.out_channels = n;
@@ -466,7 +518,7 @@ extern "C" int nncase_hip_qmatmul_prepack(nncase_hip_ctx_t *ctx, const uint8_t *
     d.groups = 1;
     d.w_qp = b_qp;
     d.expected_pixels = expected_rows;
-    return nncase_hip_qconv2d_prepack(ctx, &d, bt.data(), bias_host, weights);
+    return prepack(ctx, &d, b_host, true, bias_host, weights);
 }
 
 extern "C" int nncase_hip_qmatmul(nncase_hip_ctx_t *ctx, const uint8_t *a_dev, const nncase_hip_weights_t *w, void *y_dev,

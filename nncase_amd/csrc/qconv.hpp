@@ -33,6 +33,7 @@ struct nncase_hip_weights {
     void *d_packed = nullptr;
     uint32_t *d_post_lut = nullptr; // optional fused unary operator: 256-entry byte table (dense kernels)
     nncase_hip_quant_param_t post_lut_qp{0, 1.f};
+    // igemm: d_wsum and d_bias lie behind the fragments in the same allocation
     int32_t *d_wsum = nullptr; // igemm: sum_k (w ^ 0x80 as s8) per out channel; depthwise: sum_t (w - zw)
     int32_t *d_bias = nullptr; // [out_channels]
     size_t packed_bytes = 0;
@@ -107,6 +108,22 @@ int make_epilogue(nncase_hip_ctx *ctx, Epilogue *ep, float sx, float sw, nncase_
 // comparing exact residuals of the neighbouring floats).
 float reciprocal_rn(float b);
 
+// Weight bytes as the host hands them over: element (oc, ic, tap) of a group at oc * oc_stride + ic * ic_stride + tap.
+struct RawWeights {
+    const uint8_t *ptr;
+    int64_t oc_stride, ic_stride;
+    size_t group_bytes; // bytes between the groups
+};
+// qconv_igemm.hip: fills the plan of a dense layer (tiling, packed size) from its shape; bias on the host, or null.
+int igemm_plan(nncase_hip_ctx *ctx, nncase_hip_weights *w, const int32_t *bias_host);
+// Packs raw weights (on the device) into w->d_packed and w->d_wsum on the context's stream.
+int igemm_pack(nncase_hip_ctx *ctx, nncase_hip_weights *w, const RawWeights &raw_dev);
+// Layout of the constants of a dense layer in one block: [packed | sums | bias].
+size_t igemm_const_bytes(const nncase_hip_weights *w);
+void igemm_place(nncase_hip_weights *w, void *block);
+// qconv.hip: shape fields of w from a descriptor, and the checks that go with them.
+int describe_weights(nncase_hip_ctx *ctx, nncase_hip_weights *w, const nncase_hip_conv2d_desc_t *desc, const char *who);
+
 int launch_qconv_igemm(nncase_hip_ctx *ctx, const uint8_t *x, const nncase_hip_weights *w, void *y,
                        const nncase_hip_conv2d_args_t *a, int out_h, int out_w);
 int launch_qconv_smallc(nncase_hip_ctx *ctx, const uint8_t *x, const nncase_hip_weights *w, void *y,
@@ -124,7 +141,8 @@ struct PoolFront {
 };
 bool rows_shapes_ok(int in_channels, int out_channels, int64_t pixels);   // what rows_prepack packs and rows_path_taken takes
 bool pool_front_pays(int rows, int hw, int channels);
-int rows_prepack(nncase_hip_ctx *ctx, nncase_hip_weights *w, const uint8_t *w_oihw);
+bool rows_wanted(const nncase_hip_weights *w);
+int rows_prepack(nncase_hip_ctx *ctx, nncase_hip_weights *w, const uint8_t *w_oihw, const int32_t *bias_host);
 void rows_free(nncase_hip_weights *w);
 bool rows_path_taken(const nncase_hip_weights *w, const nncase_hip_conv2d_args_t *c, int out_h, int out_w);
 int launch_qconv_rows(nncase_hip_ctx *ctx, const uint8_t *x, const nncase_hip_weights *w, void *y, const nncase_hip_conv2d_args_t *c,

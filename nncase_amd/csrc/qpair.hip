@@ -466,8 +466,9 @@ bool rows_shapes_ok(int in_channels, int out_channels, int64_t pixels) {
 // per workgroup the separate pool kernel, which spreads over the device, is the faster one.
 bool pool_front_pays(int rows, int hw, int channels) { return (int64_t)std::min(rows, 16) * hw * channels <= (128 << 10); }
 
-int rows_prepack(nncase_hip_ctx *ctx, nncase_hip_weights *w, const uint8_t *w_oihw) {
-    if (!(pointwise_weights(w) && rows_shapes_ok(w->in_channels, w->out_channels, w->pixels_hint))) return 0; // not a call this path is for
+bool rows_wanted(const nncase_hip_weights *w) { return pointwise_weights(w) && rows_shapes_ok(w->in_channels, w->out_channels, w->pixels_hint); }
+
+int rows_prepack(nncase_hip_ctx *ctx, nncase_hip_weights *w, const uint8_t *w_oihw, const int32_t *bias_host) {
     nncase_hip_qpair *pr = new (std::nothrow) nncase_hip_qpair();
     NNHIP_REQUIRE(ctx, pr, -ENOMEM, "qconv2d_prepack: out of host memory");
     pr->second = w;
@@ -476,9 +477,8 @@ int rows_prepack(nncase_hip_ctx *ctx, nncase_hip_weights *w, const uint8_t *w_oi
     std::vector<uint8_t> packed;
     std::vector<int32_t> wsum, bias((size_t)pr->t2 * 16, 0);
     pack_pair_weights(packed, wsum, w_oihw, pr->n2, pr->n1, pr->t2, pr->ks2);
-    const hipError_t got = hipMemcpy(bias.data(), w->d_bias, sizeof(int32_t) * pr->n2, hipMemcpyDeviceToHost);
-    int rc = got == hipSuccess ? 0 : hip_fail(ctx, got, "hipMemcpy(bias)");
-    if (!rc) rc = upload(ctx, (void **)&pr->d_wb, packed.data(), packed.size());
+    if (bias_host) std::copy(bias_host, bias_host + pr->n2, bias.begin());
+    int rc = upload(ctx, (void **)&pr->d_wb, packed.data(), packed.size());
     if (!rc) rc = upload(ctx, (void **)&pr->d_wsum_b, wsum.data(), wsum.size() * sizeof(int32_t));
     if (!rc) rc = upload(ctx, (void **)&pr->d_bias_b, bias.data(), bias.size() * sizeof(int32_t));
     if (rc) { // (the failing call has left its message)

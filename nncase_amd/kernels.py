@@ -124,16 +124,22 @@ def conv2d(input: np.ndarray, weights: np.ndarray, bias: Optional[np.ndarray], s
     (ph0, ph1), (pw0, pw1) = padding
     oh = rt.windowed_output_size(h, kh, stride[0], dilation[0], ph0, ph1)
     ow = rt.windowed_output_size(wd, kw, stride[1], dilation[1], pw0, pw1)
+    out_dtype = np.dtype(out_dtype)
+    es = out_dtype.itemsize
+    args = rt.Conv2dArgs(n, h, wd, stride[0], stride[1], dilation[0], dilation[1], ph0, ph1, pw0, pw1, input_qp,
+                         output_qp or qp(0, 1.0), fused_clamp[0], fused_clamp[1], _out_dt(out_dtype))
+    if post_lut is None and residual is None and not (groups > 1 and gic == 1 and oc == groups) and n * oh * ow > 0:
+        b = None if bias is None else np.ascontiguousarray(bias, np.int32)
+        assert b is None or b.shape == (oc,)
+        y = c.host_array((n, oc, oh, ow), out_dtype)
+        c.qconv2d_host(x, w, b, weights_qp, groups, y, args)
+        return y
     wts = c.prepack_conv2d(w, bias, weights_qp, groups, expected_pixels=n * oh * ow)
     x_nchw = c.to_device(x)
     x_nhwc = c.alloc(x.size)
     c.nchw_to_nhwc(x_nchw, x_nhwc, 1, n, ch, h, wd)
-    out_dtype = np.dtype(out_dtype)
-    es = out_dtype.itemsize
     y_nhwc = c.alloc(max(1, n * oh * ow * oc * es))
     y_nchw = c.alloc(max(1, n * oh * ow * oc * es))
-    args = rt.Conv2dArgs(n, h, wd, stride[0], stride[1], dilation[0], dilation[1], ph0, ph1, pw0, pw1, input_qp,
-                         output_qp or qp(0, 1.0), fused_clamp[0], fused_clamp[1], _out_dt(out_dtype))
     if post_lut is not None:  # fused Quantize(unary(Dequantize(conv))) as a byte table attached to the weights
         wts.set_post_lut(post_lut, post_lut_qp)
     if residual is not None:  # fused Quantize(Dequantize(conv) + Dequantize(residual)), residual given as NCHW u8
@@ -157,8 +163,8 @@ def mat_mul(lhs: np.ndarray, rhs: np.ndarray, lhs_qp: QuantParam, rhs_qp: QuantP
     """kernels::stackvm::mat_mul(lhs, rhs) on u8 operands with the reference's operand forms
     (reference/matmul.cpp:28-48): rank-1 operands are a row / a column, both operands may carry up to two batch
     dimensions (rank <= 4) which broadcast against each other where one of them is 1.  lhs [..., M, K] against a
-    plain [K, N] matrix is one launch (the batch is stacked into rows); otherwise every distinct rhs matrix is
-    pre-packed once and serves all the lhs matrices it is paired with."""
+    plain [K, N] matrix is one product (the batch is stacked into rows); otherwise every distinct rhs matrix is
+    packed once and serves all the lhs matrices it is paired with."""
     c = _ctx(ctx)
     a = np.ascontiguousarray(lhs, np.uint8)
     b = np.ascontiguousarray(rhs, np.uint8)
@@ -174,19 +180,20 @@ def mat_mul(lhs: np.ndarray, rhs: np.ndarray, lhs_qp: QuantParam, rhs_qp: QuantP
     out_dtype = np.dtype(out_dtype)
     k, n = b.shape[-2:]
 
-    def run(a2d, wts):
+    bi32 = None if bias is None else np.ascontiguousarray(bias, np.int32)
+    assert bi32 is None or bi32.shape == (n,)
+
+    def run(a2d, b2d):
         m = a2d.shape[0]
-        dy = c.alloc(max(1, m * n * out_dtype.itemsize))
+        y = c.host_array((m, n), out_dtype)
         args = rt.MatmulArgs(m, lhs_qp, output_qp or qp(0, 1.0), fused_clamp[0], fused_clamp[1], _out_dt(out_dtype))
-        c.qmatmul(c.to_device(a2d), wts, dy, args)
-        return dy.download((m, n), out_dtype)
+        c.qmatmul_host(a2d, b2d, bi32, rhs_qp, y, args)
+        return y
 
     if b.ndim == 2:                                   # one constant matrix: every lhs row in one launch
         lead = a.shape[:-1]
         m = int(np.prod(lead)) if lead else 1
-        wts = c.prepack_matmul(b, bias, rhs_qp, expected_rows=m)
-        out = run(a.reshape(m, k), wts).reshape(tuple(lead) + (n,))
-        wts.destroy()
+        out = run(a.reshape(m, k), b).reshape(tuple(lead) + (n,))
     else:
         ab, bb = a.shape[:-2], b.shape[:-2]
         try:
@@ -198,11 +205,9 @@ def mat_mul(lhs: np.ndarray, rhs: np.ndarray, lhs_qp: QuantParam, rhs_qp: QuantP
         bi = np.broadcast_to(np.arange(int(np.prod(bb))).reshape(bb), batch).ravel()
         amats, bmats = a.reshape(-1, m, k), b.reshape(-1, k, n)
         out = np.empty((len(bi), m, n), out_dtype)
-        for j in np.unique(bi):                       # one pre-pack per distinct rhs matrix
+        for j in np.unique(bi):                       # one call per distinct rhs matrix
             sel = np.nonzero(bi == j)[0]
-            wts = c.prepack_matmul(np.ascontiguousarray(bmats[j]), bias, rhs_qp, expected_rows=m * len(sel))
-            out[sel] = run(np.ascontiguousarray(amats[ai[sel]]).reshape(-1, k), wts).reshape(len(sel), m, n)
-            wts.destroy()
+            out[sel] = run(np.ascontiguousarray(amats[ai[sel]]).reshape(-1, k), np.ascontiguousarray(bmats[j])).reshape(len(sel), m, n)
         out = out.reshape(tuple(batch) + (m, n))
     if a1:
         out = out.squeeze(-2)

@@ -97,6 +97,8 @@ SYMBOLS = {
     "nncase_hip_free": (_I, [_VP, _VP]),
     "nncase_hip_memcpy_h2d": (_I, [_VP, _VP, _VP, _SZ]),
     "nncase_hip_memcpy_d2h": (_I, [_VP, _VP, _VP, _SZ]),
+    "nncase_hip_host_malloc": (_I, [_VP, _SZ, C.POINTER(_VP)]),
+    "nncase_hip_host_free": (_I, [_VP]),
     "nncase_hip_memset": (_I, [_VP, _VP, _I, _SZ]),
     "nncase_hip_stream_sync": (_I, [_VP]),
     "nncase_hip_quantize": (_I, [_VP, _VP, _I, _VP, _I, _SZ, QuantParam]),
@@ -129,6 +131,8 @@ SYMBOLS = {
                                                            C.POINTER(Conv2dArgs)]),
     "nncase_hip_qmatmul_prepack": (_I, [_VP, _VP, C.c_int32, C.c_int32, QuantParam, _VP, C.c_int64, C.POINTER(_VP)]),
     "nncase_hip_qmatmul": (_I, [_VP, _VP, _VP, _VP, C.POINTER(MatmulArgs)]),
+    "nncase_hip_qconv2d_host": (_I, [_VP, C.POINTER(Conv2dDesc), _VP, _VP, _VP, _VP, C.POINTER(Conv2dArgs)]),
+    "nncase_hip_qmatmul_host": (_I, [_VP, _VP, _VP, C.c_int32, C.c_int32, QuantParam, _VP, _VP, C.POINTER(MatmulArgs)]),
     "nncase_hip_qadd": (_I, [_VP, _VP, QuantParam, _VP, QuantParam, _VP, QuantParam, C.c_float, C.c_float, _SZ]),
     "nncase_hip_qglobal_avgpool": (_I, [_VP, _VP, _VP, C.c_int32, C.c_int32, C.c_int32, C.c_int32, QuantParam,
                                         QuantParam]),
@@ -305,6 +309,21 @@ def _concat_args(inputs, channels, in_qps):
     return n, ptrs, ch, qps
 
 
+class _HostBlock:
+    """A block of pinned host memory that numpy arrays lie in; it goes back when the last of them is gone."""
+    __slots__ = ("ptr", "__array_interface__")
+
+    def __init__(self, ptr: int, nbytes: int):
+        self.ptr = ptr
+        self.__array_interface__ = {"shape": (nbytes,), "typestr": "|u1", "data": (ptr, False), "version": 3}
+
+    def __del__(self):
+        try:
+            _lib.nncase_hip_host_free(self.ptr)
+        except Exception:
+            pass
+
+
 class DeviceBuffer:
     """An HBM allocation owned through the context (nncase_hip_malloc / _free)."""
 
@@ -321,7 +340,7 @@ class DeviceBuffer:
         return self
 
     def download(self, shape, dtype) -> np.ndarray:
-        out = np.empty(shape, dtype)
+        out = self.ctx.host_array(shape, dtype)
         assert out.nbytes <= self.nbytes
         self.ctx._check(self.ctx.lib.nncase_hip_memcpy_d2h(self.ctx.handle, out.ctypes.data, self.ptr, out.nbytes), "d2h")
         return out
@@ -494,6 +513,18 @@ class Context:
         arr = np.ascontiguousarray(arr)
         return DeviceBuffer(self, arr.nbytes).upload(arr)
 
+    HOST_ARRAY_MIN = 256 << 10   # below it the runtime's own copy into pageable memory takes no longer
+
+    def host_array(self, shape, dtype) -> np.ndarray:
+        """An uninitialised host array for a result, in pinned memory where that is large enough to pay and to be had."""
+        dtype = np.dtype(dtype)
+        n = int(np.prod(shape, dtype=np.int64)) * dtype.itemsize
+        if n >= self.HOST_ARRAY_MIN:
+            p = C.c_void_p()
+            if self.lib.nncase_hip_host_malloc(self.handle, n, C.byref(p)) == 0:
+                return np.asarray(_HostBlock(p.value, n)).view(dtype).reshape(shape)
+        return np.empty(shape, dtype)
+
     # -- operators (raw device pointers) ----------------------------------------------
     def quantize(self, src: DeviceBuffer, in_dtype: int, dst: DeviceBuffer, out_dtype: int, count: int, q: QuantParam):
         self._check(self.lib.nncase_hip_quantize(self.handle, src.ptr, in_dtype, dst.ptr, out_dtype, count, q), "quantize")
@@ -596,6 +627,20 @@ class Context:
 
     def qmatmul(self, a: DeviceBuffer, w: Weights, y: DeviceBuffer, args: MatmulArgs):
         self._check(self.lib.nncase_hip_qmatmul(self.handle, a.ptr, w.handle, y.ptr, C.byref(args)), "qmatmul")
+
+    def qconv2d_host(self, x_nchw: np.ndarray, weights_oihw: np.ndarray, bias: Optional[np.ndarray], w_qp: QuantParam, groups: int,
+                     y_nchw: np.ndarray, args: Conv2dArgs):
+        """One dense or grouped convolution on host arrays (C-contiguous u8 / int32; y_nchw is written)."""
+        oc, gic, kh, kw = weights_oihw.shape
+        desc = Conv2dDesc(gic * groups, oc, kh, kw, groups, w_qp, 0)
+        self._check(self.lib.nncase_hip_qconv2d_host(self.handle, C.byref(desc), x_nchw.ctypes.data, weights_oihw.ctypes.data,
+                                                     None if bias is None else bias.ctypes.data, y_nchw.ctypes.data, C.byref(args)), "qconv2d_host")
+
+    def qmatmul_host(self, a_mk: np.ndarray, b_kn: np.ndarray, bias: Optional[np.ndarray], b_qp: QuantParam, y_mn: np.ndarray, args: MatmulArgs):
+        """One product on host arrays (C-contiguous; y_mn is written)."""
+        k, n = b_kn.shape
+        self._check(self.lib.nncase_hip_qmatmul_host(self.handle, a_mk.ctypes.data, b_kn.ctypes.data, k, n, b_qp,
+                                                     None if bias is None else bias.ctypes.data, y_mn.ctypes.data, C.byref(args)), "qmatmul_host")
 
     def qadd(self, a: DeviceBuffer, a_qp, b: DeviceBuffer, b_qp, out: DeviceBuffer, y_qp, count: int,
              clamp=(-FLT_MAX, FLT_MAX)):

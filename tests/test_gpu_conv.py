@@ -700,3 +700,31 @@ def test_fused_table_equals_conv_then_table(hip_ctx, cin, cout, hw, k, with_resi
     got = K.conv2d(x, w, bias, stride, pad, (1, 1), 1, FULL, qp(zx, sx), qp(zw, sw), qp(zy, sy), np.uint8, ctx=hip_ctx,
                    post_lut=rt.make_unary_lut(rt.LUT_SWISH, qp(zy, sy), qp(lz, ls)), post_lut_qp=qp(lz, ls), **kw)
     assert np.array_equal(got, want), f"{(got != want).sum()} of {want.size} bytes differ"
+
+
+@pytest.mark.parametrize("m,k,n", [(1, 1, 1), (3, 17, 5), (700, 1024, 513), (2048, 300, 256)])
+def test_matmul_on_host_arrays_of_every_transfer_size(hip_ctx, m, k, n):
+    """Operands and results below and above what travels through a context's pinned memory, call after call (its memory is
+    reused), results in pinned blocks that outlive the next call."""
+    rng = np.random.default_rng(m + k + n)
+    bias = rng.integers(-3000, 3000, n).astype(np.int32)
+    kept = []
+    for i in range(3):
+        a, b = rng.integers(0, 256, (m, k), dtype=np.uint8), rng.integers(0, 256, (k, n), dtype=np.uint8)
+        got = K.mat_mul(a, b, qp(7, 0.02), qp(131, 0.004), None, np.int32, bias, ctx=hip_ctx)
+        kept.append((got, (a.astype(np.int64) - 7) @ (b.astype(np.int64) - 131) + bias))
+    for got, want in kept:
+        assert np.array_equal(got, want)
+
+
+def test_host_results_return_their_pinned_memory(hip_ctx):
+    """More large results than the pinned pool holds are still right, and dropped ones make room again."""
+    src = np.arange(48 << 18, dtype=np.int32)                        # 48 MiB
+    buf = hip_ctx.to_device(src)
+    held = [buf.download(src.shape, np.int32) for _ in range(7)]     # more than 256 MiB
+    assert all(np.array_equal(h, src) for h in held)
+    held[0][:] = 5                                                   # an array of its own
+    assert np.array_equal(held[1], src)
+    del held
+    again = buf.download(src.shape, np.int32)
+    assert again.base is not None and np.array_equal(again, src)
