@@ -769,6 +769,12 @@ NNCASE_HIP_API int nncase_hip_kmodel_function(nncase_hip_kmodel_t *kmodel, nncas
 NNCASE_HIP_API int nncase_hip_kmodel_tensor(nncase_hip_kmodel_t *kmodel, int32_t which, void **dev_ptr, int32_t *dtype,
                                             int32_t *dims4);
 
+/* Input from host memory, the function, outputs 0 .. n_outputs - 1 to host memory, complete on return (the counterpart of
+ * interpreter::run between set_input_tensor and get_output_tensor).  An output whose memory comes from
+ * nncase_hip_host_malloc leaves as soon as it is complete, beside the operators that are still to run. */
+NNCASE_HIP_API int nncase_hip_kmodel_run(nncase_hip_kmodel_t *model, const void *input_host, size_t input_bytes, int32_t n_outputs,
+                                         void *const *outputs_host, const size_t *output_bytes);
+
 #ifdef __cplusplus
 }
 #endif

@@ -37,6 +37,9 @@ struct nncase_hip_ctx {
     size_t stage_used = 0;
     void *arena = nullptr;
     size_t arena_bytes = 0;
+    hipStream_t copy_stream = nullptr; // results on their way to the host beside the context's stream
+    static constexpr int kCopySlots = 8;
+    hipEvent_t copy_events[kCopySlots] = {nullptr};
     char last_error[512] = {0};
 };
 
@@ -49,8 +52,20 @@ hipError_t attn_static_scratch_address(void **ptr);
 // hostcall.hip: device scratch of at least `bytes`, valid until the next call (`*temporary`: larger than what a context
 // keeps, the caller gives it back with hipFree when the stream has drained); what a context holds for host calls.
 int scratch_reserve(nncase_hip_ctx *ctx, size_t bytes, void **ptr, bool *temporary);
+// Copies on the context's stream.  The one to the device may still be under way when it returns, but src may then be changed
+// only once the stream has drained (small ones: at once); the other returns when dst holds the data.
+int copy_to_device(nncase_hip_ctx *ctx, void *dst_dev, const void *src_host, size_t bytes);
+int copy_to_host(nncase_hip_ctx *ctx, void *dst_host, const void *src_dev, size_t bytes);
+int mark_result(nncase_hip_ctx *ctx, int slot);
+int fetch_result(nncase_hip_ctx *ctx, int slot, void *dst_pinned, const void *src_dev, size_t bytes); // under way when it returns, on ctx->copy_stream
+int drain_host_calls(nncase_hip_ctx *ctx); // waits for the context's stream
+bool host_is_pinned(const void *ptr);      // a block of nncase_hip_host_malloc
 void hostcall_attach();
 void hostcall_release(nncase_hip_ctx *ctx);
+
+// function.hip: a loaded model's list prepared for, and run with, results that go to host memory (complete on return).
+void function_hoist_outputs(nncase_hip_function_t *fn, void *const *outputs_dev, int n);
+int function_run_to_host(nncase_hip_function_t *fn, int n, void *const *outputs_dev, void *const *outputs_host, const size_t *bytes);
 
 inline int fail(nncase_hip_ctx *ctx, int code, const char *fmt, ...) {
     if (ctx) {

@@ -2,6 +2,7 @@
 // replayable eagerly or as one HIP graph.
 #include "qconv.hpp"
 
+#include <algorithm>
 #include <new>
 #include <vector>
 
@@ -530,6 +531,77 @@ extern "C" int nncase_hip_function_invoke_one(nncase_hip_function_t *fn, int32_t
     NNHIP_REQUIRE(fn->ctx, index >= 0 && (size_t)index < fn->ops.size(), -EINVAL, "function_invoke_one: index %d of %zu",
                   index, fn->ops.size());
     return run_op(fn, fn->ops[index]);
+}
+
+// Moves every operator that writes one of `outputs` (device addresses) up to just behind the last operator that writes what
+// it reads.  The list computes every tensor once and reads it afterwards, so nothing else depends on the operator's place;
+// its result can then travel to the host while the operators behind it run (a detection network's largest head needs
+// three quarters of the list).
+void nnhip::function_hoist_outputs(nncase_hip_function_t *fn, void *const *outputs, int n) {
+    std::vector<Op> &ops = fn->ops;
+    for (size_t k = 1; k < ops.size(); k++) {
+        const Op op = ops[k];
+        if (op.kind != Op::kConv && op.kind != Op::kDequantize) continue;
+        if (std::find(outputs, outputs + n, op.out) == outputs + n) continue;
+        const void *const reads[2] = {op.in0, op.kind == Op::kConv ? op.conv.residual_dev : nullptr};
+        size_t at = k;
+        while (at > 0) {
+            const Op &before = ops[at - 1];
+            bool writes = std::find(outputs, outputs + n, before.out) != outputs + n && before.out == op.out;
+            for (const void *r : reads) writes = writes || (r && (before.out == r || before.out2 == r || before.out3 == r));
+            if (writes) break;
+            at--;
+        }
+        if (at < k) {
+            std::move_backward(ops.begin() + at, ops.begin() + k, ops.begin() + k + 1);
+            ops[at] = op;
+        }
+    }
+    drop_graph(fn);
+}
+
+int nnhip::function_run_to_host(nncase_hip_function_t *fn, int n, void *const *outputs_dev, void *const *outputs_host, const size_t *bytes) {
+    nncase_hip_ctx *ctx = fn->ctx;
+    if (fn->exec) {
+        if (int rc = nncase_hip_function_invoke(fn)) return rc;
+    }
+    // results that lie in pinned memory leave on a stream of their own as soon as they are complete, in the order they are
+    struct Early {
+        int output, slot;
+    };
+    std::vector<Early> early;
+    auto enqueue = [&]() -> int {
+        const std::vector<Op> &ops = fn->ops;
+        for (size_t k = 0; !fn->exec && k < ops.size(); k++) {
+            if (int rc = run_op(fn, ops[k])) return rc;
+            if (k + 1 == ops.size()) break; // (the last operator's result is fetched in order)
+            for (int i = 0; i < n; i++) {
+                auto writes = [&](const Op &op) { return op.out == outputs_dev[i] || op.out2 == outputs_dev[i]; };
+                if (!writes(ops[k]) || std::any_of(ops.begin() + k + 1, ops.end(), writes)) continue;
+                if (early.size() == nncase_hip_ctx::kCopySlots || !host_is_pinned(outputs_host[i])) continue;
+                const int slot = (int)early.size();
+                if (int rc = mark_result(ctx, slot)) return rc;
+                early.push_back(Early{i, slot});
+            }
+        }
+        return 0;
+    };
+    int rc = enqueue();
+    std::vector<char> sent(n, 0);
+    bool sending = false;
+    for (const Early &e : early) {
+        if (rc) break;
+        rc = fetch_result(ctx, e.slot, outputs_host[e.output], outputs_dev[e.output], bytes[e.output]);
+        sent[e.output] = 1, sending = true;
+    }
+    for (int i = 0; i < n && !rc; i++)
+        if (!sent[i]) rc = copy_to_host(ctx, outputs_host[i], outputs_dev[i], bytes[i]);
+    if (sending) { // (also after a failure: nothing writes to the caller's memory once this returns)
+        const hipError_t e = hipStreamSynchronize(ctx->copy_stream);
+        if (!rc && e != hipSuccess) rc = hip_fail(ctx, e, "hipStreamSynchronize(copies)");
+    }
+    const int drained = drain_host_calls(ctx);
+    return rc ? rc : drained;
 }
 
 extern "C" int nncase_hip_function_invoke(nncase_hip_function_t *fn) {

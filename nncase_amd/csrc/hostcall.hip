@@ -37,7 +37,7 @@ static bool capturing(nncase_hip_ctx *ctx) {
     return hipStreamIsCapturing(ctx->stream, &st) != hipSuccess || st != hipStreamCaptureStatusNone;
 }
 
-static int drain(nncase_hip_ctx *ctx) {
+int drain_host_calls(nncase_hip_ctx *ctx) {
     NNHIP_HIP(ctx, hipStreamSynchronize(ctx->stream));
     ctx->stage_used = 0;
     return 0;
@@ -53,15 +53,13 @@ static uint8_t *stage_take(nncase_hip_ctx *ctx, size_t bytes) {
         (void)hipGetLastError();
         return nullptr;
     }
-    if (ctx->stage_used + need > kStageBytes && drain(ctx)) return nullptr;
+    if (ctx->stage_used + need > kStageBytes && drain_host_calls(ctx)) return nullptr;
     uint8_t *p = ctx->stage + ctx->stage_used;
     ctx->stage_used += need;
     return p;
 }
 
-// Copies of a host call.  The one to the device may still be under way when it returns, but src may be changed; the other
-// returns when dst holds the data.
-static int copy_to_device(nncase_hip_ctx *ctx, void *dst, const void *src, size_t bytes) {
+int copy_to_device(nncase_hip_ctx *ctx, void *dst, const void *src, size_t bytes) {
     if (bytes <= kStageMost) {
         if (uint8_t *s = stage_take(ctx, bytes)) {
             memcpy(s, src, bytes);
@@ -69,20 +67,20 @@ static int copy_to_device(nncase_hip_ctx *ctx, void *dst, const void *src, size_
         }
     }
     NNHIP_HIP(ctx, hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, ctx->stream));
-    return drain(ctx);
+    return 0;
 }
 
-static int copy_to_host(nncase_hip_ctx *ctx, void *dst, const void *src, size_t bytes) {
+int copy_to_host(nncase_hip_ctx *ctx, void *dst, const void *src, size_t bytes) {
     if (bytes <= kStageMost) {
         if (uint8_t *s = stage_take(ctx, bytes)) {
             int rc = launch_bus_copy(ctx, s, src, bytes);
-            if (!rc) rc = drain(ctx);
+            if (!rc) rc = drain_host_calls(ctx);
             if (!rc) memcpy(dst, s, bytes);
             return rc;
         }
     }
     NNHIP_HIP(ctx, hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, ctx->stream));
-    return drain(ctx);
+    return drain_host_calls(ctx);
 }
 
 int scratch_reserve(nncase_hip_ctx *ctx, size_t bytes, void **ptr, bool *temporary) {
@@ -95,7 +93,7 @@ int scratch_reserve(nncase_hip_ctx *ctx, size_t bytes, void **ptr, bool *tempora
     }
     if (bytes > ctx->arena_bytes) {
         if (ctx->arena) {
-            const int rc = drain(ctx);
+            const int rc = drain_host_calls(ctx);
             if (rc) return rc;
             NNHIP_HIP(ctx, hipFree(ctx->arena));
         }
@@ -144,6 +142,28 @@ HostPool &host_pool() {
 }
 } // namespace
 
+// A result complete on the context's stream, marked where it is enqueued and fetched while later work runs.  The wait is the
+// host's: it has nothing else to do by then, and making one stream wait for another on the device costs 25 us a time.
+int mark_result(nncase_hip_ctx *ctx, int slot) {
+    if (!ctx->copy_stream) NNHIP_HIP(ctx, hipStreamCreateWithFlags(&ctx->copy_stream, hipStreamNonBlocking));
+    if (!ctx->copy_events[slot]) NNHIP_HIP(ctx, hipEventCreateWithFlags(&ctx->copy_events[slot], hipEventDisableTiming));
+    NNHIP_HIP(ctx, hipEventRecord(ctx->copy_events[slot], ctx->stream));
+    return 0;
+}
+
+int fetch_result(nncase_hip_ctx *ctx, int slot, void *dst_pinned, const void *src, size_t bytes) {
+    NNHIP_HIP(ctx, hipEventSynchronize(ctx->copy_events[slot]));
+    NNHIP_HIP(ctx, hipMemcpyAsync(dst_pinned, src, bytes, hipMemcpyDeviceToHost, ctx->copy_stream));
+    return 0;
+}
+
+bool host_is_pinned(const void *ptr) {
+    std::lock_guard<std::mutex> guard(host_pool().mu);
+    for (const HostBlock &b : host_pool().blocks)
+        if (b.ptr == ptr && b.used) return true;
+    return false;
+}
+
 void hostcall_attach() {
     std::lock_guard<std::mutex> guard(host_pool().mu);
     host_pool().contexts++;
@@ -154,6 +174,12 @@ void hostcall_release(nncase_hip_ctx *ctx) {
         std::lock_guard<std::mutex> guard(host_pool().mu);
         if (--host_pool().contexts == 0) host_pool().trim(0);
     }
+    for (hipEvent_t &e : ctx->copy_events) {
+        if (e) (void)hipEventDestroy(e);
+        e = nullptr;
+    }
+    if (ctx->copy_stream) (void)hipStreamDestroy(ctx->copy_stream);
+    ctx->copy_stream = nullptr;
     if (ctx->stage) (void)hipHostFree(ctx->stage);
     if (ctx->arena) (void)hipFree(ctx->arena);
     ctx->stage = nullptr, ctx->arena = nullptr;
@@ -220,7 +246,7 @@ int dense_host_call(nncase_hip_ctx *ctx, nncase_hip_weights *w, const uint8_t *x
             uint8_t *const s = y_bytes <= kStageMost ? stage_take(ctx, y_bytes) : nullptr;
             if (int r = nncase_hip_nhwc_to_nchw(ctx, d + o_yn, s ? s : d + o_y, es, a->batch, w->out_channels, out_h, out_w)) return r;
             if (s) {
-                if (int r = drain(ctx)) return r;
+                if (int r = drain_host_calls(ctx)) return r;
                 memcpy(y_host, s, y_bytes);
                 return 0;
             }

@@ -922,6 +922,7 @@ static int build_function(nncase_hip_ctx_t *ctx, Span text_span, Span rdata, nnc
         }
         if (rc) return rc;
     }
+    if (m->n_outputs > 1) nnhip::function_hoist_outputs(m->fn, m->buffers.data() + m->output_tensor, (int)m->n_outputs);
     *out = m.release();
     return 0;
 }
@@ -945,4 +946,26 @@ extern "C" int nncase_hip_kmodel_tensor(nncase_hip_kmodel_t *m, int32_t which, v
     if (dims4)
         for (int i = 0; i < 4; i++) dims4[i] = (int32_t)m->tensors[t].dims[i];
     return 0;
+}
+
+extern "C" int nncase_hip_kmodel_run(nncase_hip_kmodel_t *m, const void *input_host, size_t input_bytes, int32_t n_outputs, void *const *outputs_host,
+                                     const size_t *output_bytes) {
+    if (!m) return -EINVAL;
+    nncase_hip_ctx *ctx = m->ctx;
+    NNHIP_REQUIRE(ctx, input_host && outputs_host && output_bytes && n_outputs > 0 && (uint32_t)n_outputs <= m->n_outputs, -EINVAL,
+                  "kmodel_run: null argument or %d outputs of %u", n_outputs, m->n_outputs);
+    auto bytes = [&](uint32_t t) {
+        size_t n = dtype_size(m->tensors[t].dtype);
+        for (int i = 0; i < 4; i++) n *= m->tensors[t].dims[i];
+        return n;
+    };
+    NNHIP_REQUIRE(ctx, input_bytes == bytes(m->input_tensor), -NNCASE_HIP_ERR_SHAPE_MISMATCH, "kmodel_run: input of %zu bytes, the model reads %zu",
+                  input_bytes, bytes(m->input_tensor));
+    for (int i = 0; i < n_outputs; i++)
+        NNHIP_REQUIRE(ctx, outputs_host[i] && output_bytes[i] == bytes(m->output_tensor + i), -NNCASE_HIP_ERR_SHAPE_MISMATCH,
+                      "kmodel_run: output %d of %zu bytes, the model writes %zu", i, output_bytes[i], bytes(m->output_tensor + i));
+    int rc = nnhip::copy_to_device(ctx, m->buffers[m->input_tensor], input_host, input_bytes);
+    if (!rc) rc = nnhip::function_run_to_host(m->fn, n_outputs, m->buffers.data() + m->output_tensor, outputs_host, output_bytes);
+    else (void)nnhip::drain_host_calls(ctx);
+    return rc;
 }

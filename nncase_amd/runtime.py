@@ -175,6 +175,7 @@ SYMBOLS = {
     "nncase_hip_kmodel_destroy": (_I, [_VP]),
     "nncase_hip_kmodel_function": (_I, [_VP, C.POINTER(_VP)]),
     "nncase_hip_kmodel_tensor": (_I, [_VP, C.c_int32, C.POINTER(_VP), _I32P, _I32P]),
+    "nncase_hip_kmodel_run": (_I, [_VP, _VP, _SZ, C.c_int32, C.POINTER(_VP), C.POINTER(_SZ)]),
     "nncase_hip_fill_queue_pool": (_I, [C.c_int]),
     "nncase_hip_release_queue_pool": (_I, [C.c_int]),
     "nncase_hip_pack": (_I, [_VP, _VP, _VP, C.c_int32, C.c_int32, _I32P, C.c_int32, _I32P, _I32P]),
@@ -1039,10 +1040,10 @@ class LoadedKModel:
         x = np.ascontiguousarray(x, self.input_dtype)
         if x.shape != self.input_shape:
             raise HipError(-ERR_SHAPE_MISMATCH, "kmodel run", f"input {x.shape}, model expects {self.input_shape}")
-        self.input.upload(x)
-        self.fn.invoke()
-        self.ctx.sync()
-        ys = [b.download(shape, dt) for b, shape, dt in self.outputs]
+        ys = [self.ctx.host_array(shape, dt) for _, shape, dt in self.outputs]
+        n = len(ys)
+        self.ctx._check(self.ctx.lib.nncase_hip_kmodel_run(self.handle, x.ctypes.data, x.nbytes, n, (_VP * n)(*[y.ctypes.data for y in ys]),
+                                                           (_SZ * n)(*[y.nbytes for y in ys])), "kmodel_run")
         return ys[0] if len(ys) == 1 else ys
 
     def destroy(self):

@@ -283,3 +283,29 @@ def test_a_function_with_nchw_ends_as_the_code_generator_writes_it(hip_ctx):
     want_mean = O.qglobal_avgpool(want_cat, qcat[0], qcat[1], qm[0], qm[1])
     assert np.array_equal(cat.reshape(N, 2 * OC, H, W), want_cat)
     assert np.array_equal(mean.reshape(N, 2 * OC), want_mean)
+
+
+@pytest.mark.parametrize("graph", ["yolov5s", "mobilenet_v2"])
+def test_run_to_host_equals_the_function_invoked_and_downloaded(hip_ctx, graph):
+    """Results that leave beside the operators still running (several outputs, pinned and ordinary memory, a captured graph,
+    run after run with other inputs) are the bytes that an invocation leaves on the device."""
+    hw = 160 if graph == "yolov5s" else 64
+    rng = np.random.default_rng(hw)
+    qg = nb.quantize_graph(getattr(nb, graph)(input_hw=hw), rng.random((1, hw, hw, 3), dtype=np.float32), calib_batch=1)
+    model = rt.LoadedKModel(hip_ctx, km.compile_quant_graph(qg, 2))
+    for captured in (False, True):
+        if captured:
+            model.fn.capture()
+        for limit in (rt.Context.HOST_ARRAY_MIN, 1, 1 << 40):         # (every result pinned / none)
+            hip_ctx.HOST_ARRAY_MIN = limit
+            try:
+                x = rng.random(model.input_shape, dtype=np.float32)
+                got = model.run(x)
+                got = got if isinstance(got, list) else [got]
+                model.input.upload(x)
+                model.fn.invoke()
+                hip_ctx.sync()
+                for y, (buf, shape, dt) in zip(got, model.outputs):
+                    assert np.array_equal(y.view(np.uint8), buf.download(shape, dt).view(np.uint8))
+            finally:
+                del hip_ctx.HOST_ARRAY_MIN
