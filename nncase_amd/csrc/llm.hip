@@ -127,29 +127,44 @@ __device__ __forceinline__ float rms_rstd_scalar(const __half *xr, int hidden, f
 // One rotate-half pair of the new token of sequence b: elements i and i + d/2 of head h (q heads, then k heads, then
 // v heads), given as the fp16 values the projection stores.  q goes rotated to the query buffer, k rotated and v as it
 // is to position ctx_lens[b] of the paged cache.  The one definition of that arithmetic: the rope kernel and the
-// projection that rotates in its own epilogue both call it.
-__device__ __forceinline__ void rope_store_pair(const RopeArgs &a, int b, int h, int i, float x0, float x1) {
+// projection that rotates in its own epilogue both use it.
+//
+// In two halves: where the pair goes and its angle (two dependent loads, a power, a sine and a cosine) do not depend on
+// the values, so a projection has them ready before its products are.
+struct RopePair {
+    int h, i, pos, in_block;
+    int pb; // the physical block, not used before the pair is stored: its load may still be under way
+    bool fits;
+    float c, s;
+};
+__device__ __forceinline__ RopePair rope_pair(const RopeArgs &a, int b, int h, int i, int pos /* ctx_lens[b] */) {
+    RopePair r;
+    r.h = h, r.i = i, r.pos = pos;
+    const int lb = pos / a.block_size;
+    r.in_block = pos - lb * a.block_size;
+    r.fits = pos >= 0 && lb < a.max_blocks; // a negative length appends nothing (it would index before the block)
+    r.pb = a.block_table[(size_t)b * a.max_blocks + (r.fits ? lb : 0)];
+    const float inv = powf(a.theta, -2.0f * (float)i / (float)a.d);
+    const float ang = (float)pos * inv;
+    r.c = cosf(ang), r.s = sinf(ang);
+    return r;
+}
+__device__ __forceinline__ void rope_store(const RopeArgs &a, int b, const RopePair &r, float x0, float x1) {
     const int half = a.d / 2;
-    const int pos = a.ctx_lens[b];
-    const int lb = pos / a.block_size, in_block = pos - lb * a.block_size;
-    const bool fits = pos >= 0 && lb < a.max_blocks; // a negative length appends nothing (it would index before the block)
-    const int pb = fits ? min(max(a.block_table[(size_t)b * a.max_blocks + lb], 0), a.num_blocks - 1) : 0;
-    if (h < a.hq + a.hkv) {
-        const float inv = powf(a.theta, -2.0f * (float)i / (float)a.d);
-        const float ang = (float)pos * inv;
-        const float c = cosf(ang), s = sinf(ang);
-        const __half y0 = __float2half_rn(x0 * c - x1 * s), y1 = __float2half_rn(x1 * c + x0 * s);
-        if (h < a.hq) {
-            __half *dst = a.q_out + ((size_t)b * a.hq + h) * a.d;
-            dst[i] = y0, dst[i + half] = y1;
-        } else if (fits) {
-            __half *dst = a.k_cache + ((((size_t)pb * a.hkv + (h - a.hq)) * a.block_size) + in_block) * a.d;
-            dst[i] = y0, dst[i + half] = y1;
+    const int pb = min(max(r.pb, 0), a.num_blocks - 1);
+    if (r.h < a.hq + a.hkv) {
+        const __half y0 = __float2half_rn(x0 * r.c - x1 * r.s), y1 = __float2half_rn(x1 * r.c + x0 * r.s);
+        if (r.h < a.hq) {
+            __half *dst = a.q_out + ((size_t)b * a.hq + r.h) * a.d;
+            dst[r.i] = y0, dst[r.i + half] = y1;
+        } else if (r.fits) {
+            __half *dst = a.k_cache + ((((size_t)pb * a.hkv + (r.h - a.hq)) * a.block_size) + r.in_block) * a.d;
+            dst[r.i] = y0, dst[r.i + half] = y1;
         }
-    } else if (fits) {
-        __half *dst = a.v_cache + ((size_t)pb * a.hkv + (h - a.hq - a.hkv)) * a.d * a.block_size + in_block;
-        dst[(size_t)i * a.block_size] = __float2half_rn(x0);
-        dst[(size_t)(i + half) * a.block_size] = __float2half_rn(x1);
+    } else if (r.fits) {
+        __half *dst = a.v_cache + ((size_t)pb * a.hkv + (r.h - a.hq - a.hkv)) * a.d * a.block_size + r.in_block;
+        dst[(size_t)r.i * a.block_size] = __float2half_rn(x0);
+        dst[(size_t)(r.i + half) * a.block_size] = __float2half_rn(x1);
     }
 }
 
@@ -376,7 +391,7 @@ inline int rows_in_lds_pitch(int k) { return k * 2 + 16; } // bytes per token ro
 // ROPE (with SPLIT and G = 2): a q / k / v projection whose block owns the two tiles that hold the halves of eight
 // rotate-half pairs -- tile j of a head and tile j + up_tile_offset (= head_dim / 32) -- so that a lane ends up with
 // both elements of its four pairs; the epilogue rounds them to fp16 as the projection's output would be stored and
-// hands them to rope_store_pair.
+// rotates and stores them (rope_pair, rope_store).
 template <int MT, int G, int WAVES, bool SPLIT = false, int KB = kRowsBatch, int PIECES = kRowsPieces, bool ROPE = false>
 __global__ __launch_bounds__(WAVES * 64) void w8a16_gemm_rows_in_lds_kernel(const GemmArgs a) {
     static_assert(!ROPE || (SPLIT && G == 2), "the rotating epilogue pairs two tiles of one block");
@@ -407,7 +422,13 @@ __global__ __launch_bounds__(WAVES * 64) void w8a16_gemm_rows_in_lds_kernel(cons
             for (int g = 0; g < G; g++) wv[u][g] = a.w[((size_t)tile[g] * a.ksteps + ks) * 64 + lane];
         }
     };
+    // ROPE: the pair this thread will finish is channel wave % 4 of the lane's four, of token tile wave / 4
+    const int rope_m = min((wave >> 2) * 16 + i16, a.m - 1);
+    int rope_pos = 0;
+    if constexpr (ROPE) rope_pos = a.rope.ctx_lens[rope_m]; // (loads return in order: asked for first, it is there first)
+    __builtin_amdgcn_sched_barrier(0);
     request_first();
+    RopePair rope;
     {
         constexpr int R = MT * 16 / WAVES; // rows per wave
         // The wave's rows stay in registers from the load to the one LDS write: their sums of squares, the butterflies
@@ -426,7 +447,17 @@ __global__ __launch_bounds__(WAVES * 64) void w8a16_gemm_rows_in_lds_kernel(cons
                 if (r < a.m && e0 < a.k) v[i][p] = *reinterpret_cast<const lu32x4 *>(a.a + (size_t)r * a.k + e0);
             }
         }
-            if (a.ln_w) {
+        // The angle is computed while the rows and weights travel: its few hundred instructions and the two loads in front
+        // of it were the last microseconds of the launch when they followed the products.
+        if constexpr (ROPE) {
+            __builtin_amdgcn_sched_barrier(0);
+            if (wave < MT * 4) { // (the other waves finish nothing)
+                const int c = out_tile * 16 + kg * 4 + (wave & 3);
+                rope = rope_pair(a.rope, rope_m, c / a.rope.d, c % a.rope.d, rope_pos);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        if (a.ln_w) {
             float ss[R];
 #pragma unroll
             for (int i = 0; i < R; i++) ss[i] = 0.f;
@@ -559,8 +590,7 @@ __global__ __launch_bounds__(WAVES * 64) void w8a16_gemm_rows_in_lds_kernel(cons
                 v2[g] = s;
             }
             // (rounded to fp16 as the projection's output would be stored; the partner is d / 2 channels further)
-            const int c = out_tile * 16 + kg * 4 + r;
-            rope_store_pair(a.rope, m, c / a.rope.d, c % a.rope.d, __half2float(__float2half_rn(v2[0])), __half2float(__float2half_rn(v2[1])));
+            rope_store(a.rope, m, rope, __half2float(__float2half_rn(v2[0])), __half2float(__float2half_rn(v2[1])));
             return;
         }
         if (wave >= MT) return; // wave w finishes token tile w
@@ -630,7 +660,7 @@ __global__ __launch_bounds__(kLlmThreads) void rope_append_kernel(const RopeArgs
     if (gid >= a.batch * heads * half) return;
     const int i = gid % half, h = (gid / half) % heads, b = gid / (half * heads);
     const __half *src = a.qkv + ((size_t)b * heads + h) * a.d;
-    rope_store_pair(a, b, h, i, __half2float(src[i]), __half2float(src[i + half]));
+    rope_store(a, b, rope_pair(a, b, h, i, a.ctx_lens[b]), __half2float(src[i]), __half2float(src[i + half]));
 }
 
 // Index of the largest element of every row (the lowest index among equals); one block of 1024
