@@ -6,9 +6,9 @@
 //   grid = (sequences x kv heads, splits).  A block owns one kv head of one
 //   sequence and a contiguous range of cached tokens, and serves ALL query
 //   heads that share the kv head, so K and V cross the memory system once
-//   however many query heads there are (GQA).  Each of its eight waves owns a
+//   however many query heads there are (GQA).  Each of its waves owns a
 //   contiguous run of 16-token tiles and issues the loads of ALL its K and V
-//   tiles before any arithmetic (8 KiB of K + 8 KiB of V in flight per wave).
+//   tiles before any arithmetic (up to 16 KiB of K + 16 KiB of V in flight per wave).
 //
 //   Logits: S^T[token, head] = K[token, :] . Q^T[:, head] with K rows as the
 //   MFMA A operand (one 16-byte load per lane straight from the cache) and the
@@ -27,6 +27,8 @@
 #include "common.hpp"
 
 #include <hip/hip_fp16.h>
+
+#include <algorithm>
 
 namespace nnhip {
 
@@ -61,8 +63,76 @@ __device__ __forceinline__ float coherent_load(const float *p) {
     return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
+// two neighbouring floats at an 8-byte aligned address
+__device__ __forceinline__ uint64_t coherent_load2(const float *p) {
+    return __hip_atomic_load(reinterpret_cast<const uint64_t *>(p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+// outputs i and i + 1 (i even)
+__device__ __forceinline__ void store_pair(const AttnArgs &a, size_t i, float v0, float v1) {
+    if (a.out_f16) *reinterpret_cast<__half2 *>(reinterpret_cast<__half *>(a.out) + i) = __halves2half2(__float2half_rn(v0), __float2half_rn(v1));
+    else *reinterpret_cast<float2 *>(reinterpret_cast<float *>(a.out) + i) = float2{v0, v1};
+}
+
 // bytes of dynamic LDS of a block of W waves: the waves' unnormalised outputs, maxima and sums
 constexpr size_t attn_lds_bytes(int d, int waves) { return (size_t)waves * kAttnHeads * (d + 2) * sizeof(float); }
+
+// Merges ns partials of G query heads (rows row0 + head * splits) into outputs out0 ...; every thread of the block calls it.
+// A thread merges two neighbouring outputs over every GR-th run of U splits: their (max, sum) and (value, value) pairs are
+// requested together, one memory round trip per GR * U splits (a trip per eight splits was 8 of the 12 us of one sequence of
+// 16 000 tokens); runs combine under a running maximum, the GR partial results through LDS.
+template <int D, int U>
+__device__ __forceinline__ void merge_splits(const AttnArgs &a, int ns, int G, size_t row0, size_t out0, float *part, int threads) {
+    const int pairs = G * D / 2;
+    int GR = 1, gr = 0;
+    if (U == 8) {
+        while (GR < 4 && (GR + 1) * pairs <= threads && GR * U < ns) GR++;
+        for (int q = 1; q < GR; q++) gr += (int)threadIdx.x >= q * pairs;
+        if ((int)threadIdx.x >= GR * pairs && GR > 1) gr = GR;
+    }
+    for (int p0 = gr < GR ? (int)threadIdx.x - gr * pairs : pairs; p0 < pairs; p0 += threads) { // (more than one turn only with GR = 1)
+        const int h = p0 * 2 / D, e = p0 * 2 % D;
+        const size_t rowh = row0 + (size_t)h * a.splits;
+        float m = -INFINITY, den = 0.f, n0 = 0.f, n1 = 0.f;
+        for (int sp0 = gr * U; sp0 < ns; sp0 += GR * U) {
+            float pm[U], pl[U];
+            uint64_t vv[U];
+#pragma unroll
+            for (int k = 0; k < U; k++) {
+                const size_t row = rowh + min(sp0 + k, ns - 1);
+                pm[k] = coherent_load(a.part_ml + row * 2), pl[k] = coherent_load(a.part_ml + row * 2 + 1);
+                vv[k] = coherent_load2(a.part_o + row * D + e);
+            }
+            float mc = m;
+#pragma unroll
+            for (int k = 0; k < U; k++) mc = fmaxf(mc, pm[k]); // a repeated last split does not change the max
+            const float f = __builtin_amdgcn_exp2f(m - mc);      // 0 on the first run (m = -inf)
+            n0 *= f, n1 *= f, den *= f;
+#pragma unroll
+            for (int k = 0; k < U; k++) {
+                const float w = sp0 + k < ns ? __builtin_amdgcn_exp2f(pm[k] - mc) : 0.f;
+                n0 += w * __uint_as_float((uint32_t)vv[k]);
+                n1 += w * __uint_as_float((uint32_t)(vv[k] >> 32));
+                den += w * pl[k];
+            }
+            m = mc;
+        }
+        if (GR > 1) *reinterpret_cast<f32x4 *>(part + ((size_t)gr * pairs + p0) * 4) = f32x4{m, den, n0, n1};
+        else store_pair(a, out0 + (size_t)h * D + e, n0 / den, n1 / den);
+    }
+    if (GR == 1) return;
+    __syncthreads();
+    for (int p0 = threadIdx.x; p0 < pairs; p0 += threads) {
+        float m = part[(size_t)p0 * 4];
+        for (int q = 1; q < GR; q++) m = fmaxf(m, part[((size_t)q * pairs + p0) * 4]);
+        float den = 0.f, n0 = 0.f, n1 = 0.f;
+        for (int q = 0; q < GR; q++) {
+            const f32x4 t = *reinterpret_cast<const f32x4 *>(part + ((size_t)q * pairs + p0) * 4);
+            const float w = __builtin_amdgcn_exp2f(t[0] - m);
+            den += w * t[1], n0 += w * t[2], n1 += w * t[3];
+        }
+        store_pair(a, out0 + (size_t)p0 * 2, n0 / den, n1 / den);
+    }
+}
 
 // NT = 16-token tiles per wave (even); W = waves per block (a block owns W * NT * 16 tokens).
 template <int D, int NT, int W> __global__ __launch_bounds__(W * 64, W <= 8 ? 2 : 1) void paged_attn_kernel(const AttnArgs a) {
@@ -272,42 +342,10 @@ template <int D, int NT, int W> __global__ __launch_bounds__(W * 64, W <= 8 ? 2 
         s_last = __hip_atomic_fetch_add(done, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == (uint32_t)(ns - 1);
     __syncthreads();
     if (!s_last) return;
-    // Each thread merges one output element: the (max, sum, value) triples of eight splits are
-    // requested together (one memory round trip per eight splits), and groups of eight are
-    // combined with a running maximum.
-    for (int idx = threadIdx.x; idx < G * D; idx += kAttnThreads) {
-        const int h = idx / D, e = idx % D;
-        const size_t row0 = ((size_t)b * a.hq + kvh * G + h) * a.splits;
-        float m = -INFINITY, num = 0.f, den = 0.f;
-        for (int sp0 = 0; sp0 < ns; sp0 += 8) {
-            float pm[8], pl[8], pv[8];
-#pragma unroll
-            for (int k = 0; k < 8; k++) {
-                const size_t row = row0 + min(sp0 + k, ns - 1);
-                pm[k] = coherent_load(a.part_ml + row * 2);
-                pl[k] = coherent_load(a.part_ml + row * 2 + 1);
-                pv[k] = coherent_load(a.part_o + row * D + e);
-            }
-            float mc = m;
-#pragma unroll
-            for (int k = 0; k < 8; k++) mc = fmaxf(mc, pm[k]); // a repeated last split does not change the max
-            const float f = __builtin_amdgcn_exp2f(m - mc);      // 0 on the first group (m = -inf)
-            num *= f;
-            den *= f;
-#pragma unroll
-            for (int k = 0; k < 8; k++)
-                if (sp0 + k < ns) {
-                    const float w = __builtin_amdgcn_exp2f(pm[k] - mc);
-                    num += w * pv[k];
-                    den += w * pl[k];
-                }
-            m = mc;
-        }
-        const float r = num / den;
-        const size_t oi = ((size_t)b * a.hq + kvh * G + h) * D + e;
-        if (a.out_f16) reinterpret_cast<__half *>(a.out)[oi] = __float2half_rn(r);
-        else reinterpret_cast<float *>(a.out)[oi] = r;
-    }
+    const size_t row0 = ((size_t)b * a.hq + kvh * G) * a.splits, out0 = ((size_t)b * a.hq + kvh * G) * D;
+    float *const part = attn_smem; // (the waves' outputs have been read)
+    if (ns <= 4) merge_splits<D, 4>(a, ns, G, row0, out0, part, kAttnThreads);
+    else merge_splits<D, 8>(a, ns, G, row0, out0, part, kAttnThreads);
     if (threadIdx.x == 0) // ready for the next call on this stream
         __hip_atomic_store(done, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
@@ -337,7 +375,7 @@ struct AttnPlan {
     size_t partial_bytes = 0, counter_bytes = 0;
 };
 
-static int attn_plan(nncase_hip_ctx *ctx, const nncase_hip_paged_attn_args_t *p, AttnPlan *plan) {
+static int attn_plan(nncase_hip_ctx *ctx, const nncase_hip_paged_attn_args_t *p, AttnPlan *plan, size_t most_partial_bytes = SIZE_MAX) {
     NNHIP_REQUIRE(ctx, p->batch > 0 && p->num_q_heads > 0 && p->num_kv_heads > 0 && p->max_blocks_per_seq > 0 &&
                            p->num_blocks > 0,
                   -EINVAL, "paged_attention_decode: non-positive dimension");
@@ -366,30 +404,39 @@ static int attn_plan(nncase_hip_ctx *ctx, const nncase_hip_paged_attn_args_t *p,
     a.num_blocks = p->num_blocks;
     a.len_offset = p->ctx_len_offset;
     const int64_t max_tokens = (int64_t)p->max_blocks_per_seq * p->block_size;
-    // Eight waves per block, and tiles per wave: the largest run that still leaves about two blocks per compute unit
-    // when every sequence is at full length (the kernel cannot know the real lengths on the host).  Measured at batch
-    // 32, 2 kv heads, contexts of 512-4096 tokens, microseconds for 2 / 4 / 8 tiles per wave: four waves 17.7 / 14.2 /
-    // 13.2, eight waves 13.3 / 12.2 / 12.9, sixteen waves 13.7 / 13.6 / 22.3 -- the same tokens per block are quicker as
-    // more waves with shorter runs (more loads in flight per block, a shorter chain per wave), up to the point where a
-    // block's merge through LDS outweighs it.  The rule picks 4 tiles there and 2 for the 16 sequences of a decode lane.
-    const int nt_max = 512 / p->head_dim; // 8 KiB of K per wave
-    const int waves = 8;
-    auto splits_at = [&](int tiles) { return (max_tokens + waves * tiles * 16 - 1) / (waves * tiles * 16); };
-    int nt = 2;
-    while (nt < nt_max && (splits_at(nt) > kAttnMaxSplits ||
-                           (int64_t)p->batch * p->num_kv_heads * splits_at(nt * 2) >= (int64_t)2 * ctx->compute_units))
-        nt *= 2;
+    // Tokens per block, as W waves of NT tiles, from the capacity and the launch's blocks (the kernel cannot know the real
+    // lengths on the host).  Four waves where they serve: a block of eight holds twice the registers and, at head_dim 128,
+    // half the compute unit's LDS, and its phases (requests, products, merge) then have one other block to overlap with.
+    // Measured, us as 128 / 256 / 512 tokens per block (2 / 4 tiles in four waves, 4 in eight): 48 sequences of 6000 tokens, 8 kv
+    // heads of 128: 152 / 141 / 155; 64 of 1000: 29.3 / 31.0 / 36.6; one of 1000: 7.7 / 9.2 / 12.0; one of 700, 2 kv heads of 64:
+    // 6.1 / 6.5 / 8.1.  Short blocks mean many splits to merge: up to eight (1024 tokens) they are one memory round trip,
+    // past that 256 tokens are better (16 sequences of 2048: 9.0 / 7.9 / 8.8), and 512 for the longest contexts while the
+    // launch has few blocks (one of 16 000: 18 / 12.6 / 10.9; 32 of 4096: 15.9 / 13.3 / 12.5).  A context of one block needs no
+    // merge at all (100 tokens: 4.1 us), so capacities of 129 to 256 take 256.
+    int nt = 4, waves = 4;
+    auto blocks_of = [&](int64_t tokens) { return (int64_t)p->batch * p->num_kv_heads * ((max_tokens + tokens - 1) / tokens); };
+    if (max_tokens <= 128 || (max_tokens > 256 && max_tokens <= 1024)) nt = 2;
+    else if ((max_tokens >= 8192 || (max_tokens >= 4096 && 4 * blocks_of(512) >= ctx->compute_units)) &&
+             blocks_of(512) * p->head_dim <= (int64_t)128 * ctx->compute_units)
+        waves = 8;
+    for (;;) { // (longer runs where there would be too many splits, for the merge or for the scratch there is)
+        a.split_tokens = waves * nt * 16;
+        a.splits = (int)std::min<int64_t>((max_tokens + a.split_tokens - 1) / a.split_tokens, INT32_MAX);
+        plan->partial_bytes = (size_t)a.batch * a.hq * a.splits * (a.d + 2) * sizeof(float);
+        if (a.splits <= kAttnMaxSplits && plan->partial_bytes <= most_partial_bytes) break;
+        if (nt == 2) nt = 4;
+        else if (waves == 4) waves = 8;
+        else if (p->head_dim == 64 && nt == 4) nt = 8;
+        else break;
+    }
     plan->nt = nt;
     plan->waves = waves;
-    a.split_tokens = waves * nt * 16;
-    a.splits = (int)((max_tokens + a.split_tokens - 1) / a.split_tokens);
     NNHIP_REQUIRE(ctx, a.splits <= kAttnMaxSplits, -EINVAL,
                   "paged_attention_decode: context capacity of %lld tokens exceeds %d (head_dim %d)", (long long)max_tokens,
                   kAttnMaxSplits * a.split_tokens, p->head_dim);
     a.d_block = make_fastdiv((uint32_t)p->block_size);
     a.scale_log2e = p->scale * kLog2e;
     a.out_f16 = p->out_dtype == NNCASE_HIP_DT_F16;
-    plan->partial_bytes = (size_t)a.batch * a.hq * a.splits * (a.d + 2) * sizeof(float);
     plan->counter_bytes = (size_t)a.batch * a.hkv * sizeof(uint32_t);
     return 0;
 }
@@ -420,8 +467,8 @@ static int attn_launch(nncase_hip_ctx *ctx, AttnPlan &plan, const void *q_dev, c
     };
 #define NNHIP_ATTN_CASE(DV, NTV, WV) \
     if (!launched && a.d == DV && nt == NTV && waves == WV) go(paged_attn_kernel<DV, NTV, WV>);
-    NNHIP_ATTN_CASE(64, 8, 8) NNHIP_ATTN_CASE(64, 4, 8) NNHIP_ATTN_CASE(64, 2, 8)
-    NNHIP_ATTN_CASE(128, 4, 8) NNHIP_ATTN_CASE(128, 2, 8)
+    NNHIP_ATTN_CASE(64, 2, 4) NNHIP_ATTN_CASE(64, 4, 4) NNHIP_ATTN_CASE(64, 4, 8) NNHIP_ATTN_CASE(64, 8, 8)
+    NNHIP_ATTN_CASE(128, 2, 4) NNHIP_ATTN_CASE(128, 4, 4) NNHIP_ATTN_CASE(128, 4, 8)
 #undef NNHIP_ATTN_CASE
     NNHIP_REQUIRE(ctx, launched, -EINVAL, "paged_attention_decode: no kernel for head_dim %d, %d tiles per wave, %d waves", a.d, nt, waves);
     NNHIP_LAUNCH_CHECK(ctx, "paged_attn_kernel");
@@ -432,11 +479,26 @@ static int attn_launch(nncase_hip_ctx *ctx, AttnPlan &plan, const void *q_dev, c
 // old areas, so it is refused while a captured graph holds their addresses (-EBUSY) and while the
 // context's stream is capturing (an allocation and a synchronisation would invalidate the capture):
 // resident functions reserve when the operator is recorded, before any capture.
+static bool attn_fits(const nncase_hip_ctx *ctx, const AttnPlan &plan) {
+    return ctx->attn_ws_bytes >= plan.partial_bytes && ctx->attn_done_bytes >= plan.counter_bytes;
+}
+// The plan for a call on the context's workspace: where that cannot grow and longer runs per block (fewer splits) make
+// the call fit, those are taken.
+static int attn_plan_on_context(nncase_hip_ctx *ctx, const nncase_hip_paged_attn_args_t *p, AttnPlan *plan) {
+    int rc = attn_plan(ctx, p, plan);
+    if (rc || attn_fits(ctx, *plan)) return rc;
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    if (ctx->attn_pins == 0 && hipStreamIsCapturing(ctx->stream, &cs) == hipSuccess && cs == hipStreamCaptureStatusNone) return 0;
+    AttnPlan small;
+    if (attn_plan(ctx, p, &small, ctx->attn_ws_bytes) == 0 && attn_fits(ctx, small)) *plan = small;
+    return 0;
+}
+
 int attn_reserve(nncase_hip_ctx *ctx, const nncase_hip_paged_attn_args_t *p) {
     AttnPlan plan;
-    const int rc = attn_plan(ctx, p, &plan);
+    const int rc = attn_plan_on_context(ctx, p, &plan);
     if (rc) return rc;
-    if (ctx->attn_ws_bytes >= plan.partial_bytes && ctx->attn_done_bytes >= plan.counter_bytes) return 0;
+    if (attn_fits(ctx, plan)) return 0;
     NNHIP_REQUIRE(ctx, ctx->attn_pins == 0, -EBUSY,
                   "paged_attention_decode: the split workspace would have to grow (%zu -> %zu bytes) while %d captured "
                   "function(s) refer to it; record the larger operator before capturing",
@@ -500,9 +562,9 @@ extern "C" int nncase_hip_paged_attention_decode(nncase_hip_ctx_t *ctx, const vo
     NNHIP_REQUIRE(ctx, q_dev && k_cache_dev && v_cache_dev && block_table_dev && ctx_lens_dev && out_dev && p, -EINVAL,
                   "paged_attention_decode: null argument");
     AttnPlan plan;
-    int rc = attn_plan(ctx, p, &plan);
+    int rc = attn_plan_on_context(ctx, p, &plan);
     if (rc) return rc;
-    if (ctx->attn_ws_bytes < plan.partial_bytes || ctx->attn_done_bytes < plan.counter_bytes) {
+    if (!attn_fits(ctx, plan)) {
         rc = attn_reserve(ctx, p);
         if (rc) return rc;
     }
@@ -518,7 +580,7 @@ extern "C" int nncase_hip_paged_attention_decode_noalloc(nncase_hip_ctx_t *ctx, 
     NNHIP_REQUIRE(ctx, q_dev && k_cache_dev && v_cache_dev && block_table_dev && ctx_lens_dev && out_dev && p, -EINVAL,
                   "paged_attention_decode_noalloc: null argument");
     AttnPlan plan;
-    const int rc = attn_plan(ctx, p, &plan);
+    const int rc = attn_plan(ctx, p, &plan, kScratchPartialBytes);
     if (rc) return rc;
     NNHIP_REQUIRE(ctx, plan.partial_bytes <= kScratchPartialBytes && plan.counter_bytes <= kScratchCounterBytes, -ENOSPC,
                   "paged_attention_decode_noalloc: needs %zu bytes of split partials and %zu of counters; the static "

@@ -5,6 +5,7 @@ import numpy as np
 import pytest
 
 from nncase_amd import kernels as K
+from nncase_amd import runtime as rt
 from oracle import oracle as O
 
 pytestmark = pytest.mark.gpu
@@ -194,5 +195,45 @@ def test_capture_without_a_warm_up_and_pinned_workspace(hip_ctx):
         want2 = O.paged_attention_decode(q2.view(np.uint16), kc2.view(np.uint16), d2 and K.v_cache_from_token_major(vc2).view(np.uint16), bt2, cl2, 0.125)
         got2 = dout2.download(q2.shape, np.float32)
         assert (np.abs(got2 - want2) <= RTOL * np.abs(want2).max(axis=-1, keepdims=True) + 1e-6).all()
+    finally:
+        ctx.close()
+
+
+@pytest.mark.parametrize("hq,hkv,d", [(14, 2, 64), (4, 1, 128), (16, 1, 128)])
+@pytest.mark.parametrize("capacity", [128, 144, 256, 272, 1024, 1040, 2064, 4096, 8208])
+def test_every_split_of_the_capacity(hip_ctx, hq, hkv, d, capacity):
+    """Both sides of every capacity at which the tokens per block change, contexts that end inside the first, a middle and the
+    last block, more splits than one run of the merge takes."""
+    rng = np.random.default_rng(capacity + d)
+    lens = [1, capacity // 3 + 1, capacity]
+    case = make_case(rng, len(lens), hq, hkv, d, 16, capacity, lens)
+    check(hip_ctx, *case, 1.0 / np.sqrt(d))
+
+
+def test_a_workspace_that_cannot_grow_takes_longer_runs(hip_ctx):
+    """While a captured graph holds the workspace, a call whose usual split needs more of it runs with fewer splits instead."""
+    rng = np.random.default_rng(3)
+    ctx = rt.Context(0)
+    try:
+        def device(case, out):
+            q, kc, vc, bt, cl = case
+            bufs = [ctx.to_device(t) for t in (q, kc, K.v_cache_from_token_major(vc), bt, cl)]
+            args = rt.PagedAttnArgs(q.shape[0], q.shape[1], kc.shape[1], q.shape[2], 16, bt.shape[1], kc.shape[0], 0.125, rt.DT_F32)
+            return bufs, ctx.alloc(q.size * 4), args
+        first = make_case(rng, 32, 14, 2, 64, 16, 512, [500] * 32)       # four splits
+        fn = rt.Function(ctx)
+        bufs, out, args = device(first, np.float32)
+        fn.add_paged_attention_decode(*bufs, out, args)
+        fn.capture()
+        second = make_case(rng, 32, 14, 2, 64, 16, 1024, [1000] * 32)    # eight
+        bufs2, out2, args2 = device(second, np.float32)
+        ctx.paged_attention_decode(*bufs2, out2, args2)
+        got = out2.download((32, 14, 64), np.float32)
+        q, kc, vc, bt, cl = second
+        vt = K.v_cache_from_token_major(vc)
+        want = O.paged_attention_decode(q.view(np.uint16), kc.view(np.uint16), vt.view(np.uint16), bt, cl, 0.125)
+        assert np.abs(got - want).max() <= RTOL * np.abs(want).max()
+        fn.invoke()
+        ctx.sync()
     finally:
         ctx.close()
