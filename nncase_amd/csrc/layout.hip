@@ -196,9 +196,40 @@ struct TileDesc {
     uint32_t exact;                   // 1: the destination has no padding: lanes past the plain extent of A are not stored (transposes)
     uint32_t pitch;                   // dwords per LDS row
     FastDiv d_cols, d_rowq;           // dwords per row of the tile; rows / E
-    uint32_t wide;                    // packing: every row of the source tile is whole 16-byte pieces at 16-byte addresses
+    uint32_t wide;                    // the source tile is read in 16-byte pieces: whole ones at 16-byte addresses, or (packing) ragged rows
     FastDiv d_cols4;                  // ... of which a row has this many
+    uint32_t ragged;                  // rows start at any element and end inside a dword
+    uint64_t in_bytes;                // ... size of the source tensor (at least 4)
 };
+
+struct __attribute__((packed, aligned(1))) layout_unaligned4 {
+    uint32_t v;
+};
+struct __attribute__((packed, aligned(1))) layout_unaligned16 {
+    uint32_t v[4];
+};
+// the first n < 4 bytes of a dword
+__device__ __forceinline__ uint32_t keep_bytes(uint32_t v, uint32_t n) { return n >= 4 ? v : v & ((1u << (8 * n)) - 1); }
+// A dword of a ragged tensor from any byte offset, of which `valid` bytes count and the rest read as zero; a dword that would
+// reach past the tensor is read lower and moved down.
+__device__ __forceinline__ uint32_t load_bytes4(const uint8_t *in, uint64_t off, uint64_t total, uint32_t valid) {
+    const uint64_t at = off + 4 > total ? total - 4 : off;
+    const uint32_t v = reinterpret_cast<const layout_unaligned4 *>(in + at)->v >> (8 * (uint32_t)(off - at));
+    return keep_bytes(v, valid);
+}
+// The first `valid` (up to 4) bytes of v, in whole elements of ES bytes, to any byte offset.
+template <int ES> __device__ __forceinline__ void store_bytes4(uint8_t *out, uint64_t off, uint32_t v, uint32_t valid) {
+    if (valid >= 4) {
+        reinterpret_cast<layout_unaligned4 *>(out + off)->v = v;
+    } else {
+#pragma unroll
+        for (int k = 0; k * ES < 4; k++)
+            if (k * ES < (int)valid) {
+                if (ES == 1) out[off + k] = (uint8_t)(v >> (8 * k));
+                else *reinterpret_cast<uint16_t *>(out + off + 2 * k) = (uint16_t)(v >> (16 * k));
+            }
+    }
+}
 
 template <int E> __device__ __forceinline__ void transpose_dwords(const uint32_t (&d)[E], uint32_t (&o)[E]) {
     if constexpr (E == 1) {
@@ -217,8 +248,11 @@ template <int E> __device__ __forceinline__ void transpose_dwords(const uint32_t
 }
 
 // E = elements per dword.  PACK: plain -> packed (LDS rows = lanes of A, columns = X); else packed -> plain (rows = X,
-// columns = lanes of A).  in / out are byte pointers, 4-byte aligned like every row the host admits.
-template <int E, bool PACK> __global__ __launch_bounds__(kLayoutThreads) void pack_tile_kernel(const uint8_t *in, uint8_t *out, const TileDesc d) {
+// columns = lanes of A).  in / out are byte pointers, 4-byte aligned like every row the host admits -- unless RAGGED: extents
+// that are no whole dwords, so that rows begin at any element.  Their dwords (and 16-byte pieces) are read and written where
+// they lie, the last of a row in part.  us, with a thread per element and so: NCHW -> NC/32 HW 32 of 7 x 255 x 99 x 99 u8 123.8 /
+// 11.9 (floor 6.7), its unpack by 16 52.9 / 9.3.
+template <int E, bool PACK, bool RAGGED = false> __global__ __launch_bounds__(kLayoutThreads) void pack_tile_kernel(const uint8_t *in, uint8_t *out, const TileDesc d) {
     extern __shared__ uint32_t tile[];
     constexpr int ES = 4 / E;
     // ---- which tile ----
@@ -254,8 +288,41 @@ template <int E, bool PACK> __global__ __launch_bounds__(kLayoutThreads) void pa
                 const uint32_t r = fastdiv(idx, d.d_cols4), c = (idx - r * cols4) * 4;
                 at[u] = r * d.pitch + c;
                 v[u] = uint4{0u, 0u, 0u, 0u};
-                if (has_source && r < vlim && x0 + c * E < d.x_extent)
-                    v[u] = *reinterpret_cast<const uint4 *>(in + (plain + (uint64_t)r * d.a_plain_stride) * ES + c * 4);
+                if (has_source && r < vlim && x0 + c * E < d.x_extent) {
+                    const uint64_t off = (plain + (uint64_t)r * d.a_plain_stride) * ES + c * 4;
+                    if constexpr (RAGGED) {
+                        const uint32_t left = (d.x_extent - x0 - c * E) * ES;
+                        if (off + 16 <= d.in_bytes) {
+                            const layout_unaligned16 q = *reinterpret_cast<const layout_unaligned16 *>(in + off);
+                            v[u] = uint4{keep_bytes(q.v[0], left), left > 4 ? keep_bytes(q.v[1], left - 4) : 0u, left > 8 ? keep_bytes(q.v[2], left - 8) : 0u,
+                                         left > 12 ? keep_bytes(q.v[3], left - 12) : 0u};
+                        } else {
+                            uint32_t q[4] = {0u, 0u, 0u, 0u};
+#pragma unroll
+                            for (int k = 0; k < 4; k++)
+                                if ((uint32_t)k * 4 < left) q[k] = load_bytes4(in, off + k * 4, d.in_bytes, left - k * 4);
+                            v[u] = uint4{q[0], q[1], q[2], q[3]};
+                        }
+                    } else {
+                        v[u] = *reinterpret_cast<const uint4 *>(in + off);
+                    }
+                }
+            }
+#pragma unroll
+            for (int u = 0; u < UW; u++) tile[at[u]] = v[u].x, tile[at[u] + 1] = v[u].y, tile[at[u] + 2] = v[u].z, tile[at[u] + 3] = v[u].w;
+        }
+    } else if (!PACK && d.wide) {
+        const uint32_t cols4 = d.d_cols4.div;
+        for (uint32_t base = threadIdx.x; base < rows * cols4; base += UW * kLayoutThreads) {
+            uint4 v[UW];
+            uint32_t at[UW];
+#pragma unroll
+            for (int u = 0; u < UW; u++) {
+                const uint32_t idx = min(base + u * kLayoutThreads, rows * cols4 - 1);
+                const uint32_t r = fastdiv(idx, d.d_cols4), c = (idx - r * cols4) * 4;
+                at[u] = r * d.pitch + c;
+                v[u] = uint4{0u, 0u, 0u, 0u};
+                if (x0 + r < d.x_extent) v[u] = *reinterpret_cast<const uint4 *>(in + (packed + two_term(d.x_packed, x0 + r)) * ES + c * 4);
             }
 #pragma unroll
             for (int u = 0; u < UW; u++) tile[at[u]] = v[u].x, tile[at[u] + 1] = v[u].y, tile[at[u] + 2] = v[u].z, tile[at[u] + 3] = v[u].w;
@@ -270,11 +337,17 @@ template <int E, bool PACK> __global__ __launch_bounds__(kLayoutThreads) void pa
             at[u] = r * d.pitch + c;
             v[u] = 0;
             if (PACK) { // row r = lane l, column c = E coordinates of X from x0 + c * E
-                if (has_source && r < vlim && x0 + c * E < d.x_extent)
-                    v[u] = *reinterpret_cast<const uint32_t *>(in + (plain + (uint64_t)r * d.a_plain_stride) * ES + c * 4);
+                if (has_source && r < vlim && x0 + c * E < d.x_extent) {
+                    const uint64_t off = (plain + (uint64_t)r * d.a_plain_stride) * ES + c * 4;
+                    if constexpr (RAGGED) v[u] = load_bytes4(in, off, d.in_bytes, (d.x_extent - x0 - c * E) * ES);
+                    else v[u] = *reinterpret_cast<const uint32_t *>(in + off);
+                }
             } else { // row r = coordinate x0 + r of X, column c = E lanes
-                if (x0 + r < d.x_extent && c * E < vlim)
-                    v[u] = *reinterpret_cast<const uint32_t *>(in + (packed + two_term(d.x_packed, x0 + r)) * ES + c * 4);
+                if (x0 + r < d.x_extent && c * E < vlim) {
+                    const uint64_t off = (packed + two_term(d.x_packed, x0 + r)) * ES + c * 4;
+                    if constexpr (RAGGED) v[u] = load_bytes4(in, off, d.in_bytes, 4);
+                    else v[u] = *reinterpret_cast<const uint32_t *>(in + off);
+                }
             }
         }
 #pragma unroll
@@ -295,12 +368,18 @@ template <int E, bool PACK> __global__ __launch_bounds__(kLayoutThreads) void pa
         for (int j = 0; j < E; j++) {
             if (PACK) { // o[j]: lanes rq * E .. of coordinate x0 + c * E + j
                 const uint32_t x = x0 + c * E + j;
-                if (x < d.x_padded && (!d.exact || rq * E < vlim))
-                    *reinterpret_cast<uint32_t *>(out + (packed + two_term(d.x_packed, x)) * ES + rq * 4) = o[j];
+                if (x < d.x_padded && (!d.exact || rq * E < vlim)) {
+                    const uint64_t off = (packed + two_term(d.x_packed, x)) * ES + rq * 4;
+                    if constexpr (RAGGED) store_bytes4<ES>(out, off, o[j], d.exact ? (vlim - rq * E) * ES : 4);
+                    else *reinterpret_cast<uint32_t *>(out + off) = o[j];
+                }
             } else { // o[j]: coordinates x0 + rq * E .. of lane c * E + j
                 const uint32_t l = c * E + j;
-                if (l < vlim && x0 + rq * E < d.x_extent)
-                    *reinterpret_cast<uint32_t *>(out + (plain + (uint64_t)l * d.a_plain_stride) * ES + rq * 4) = o[j];
+                if (l < vlim && x0 + rq * E < d.x_extent) {
+                    const uint64_t off = (plain + (uint64_t)l * d.a_plain_stride) * ES + rq * 4;
+                    if constexpr (RAGGED) store_bytes4<ES>(out, off, o[j], (d.x_extent - x0 - rq * E) * ES);
+                    else *reinterpret_cast<uint32_t *>(out + off) = o[j];
+                }
             }
         }
     }
@@ -355,9 +434,14 @@ static bool make_tile_desc(TileDesc &d, int es, int rank, const int32_t *shape, 
         d.x_padded = O[xs] * L[xs];
         d.x_packed = TwoTerm{L[xs], sqo[xs], sql[jpos[xs]]};
     }
-    if (a >= xs || ((uint64_t)d.x_extent * es) % 4 != 0) return false;
+    if (a >= xs) return false;
+    // (the packed tensor's runs are whole dwords, la being a multiple of e: only the plain tensor's rows can be ragged)
+    d.ragged = ((uint64_t)d.x_extent * es) % (pack ? 16 : 4) != 0; // (packing reads them in 16-byte pieces, unpacking writes them in dwords)
+    d.in_bytes = (pack ? sp[0] * (uint64_t)shape[0] : st) * es;
+    if (d.in_bytes < 4) return false;
     if (!pack) d.x_padded = d.x_extent;
-    d.wide = pack && ((uint64_t)d.x_extent * es) % 16 == 0 && (reinterpret_cast<uintptr_t>(in) & 15u) == 0;
+    if (pack) d.wide = d.ragged ? (uint64_t)d.x_extent * es >= 64 : ((uint64_t)d.x_extent * es) % 16 == 0 && (reinterpret_cast<uintptr_t>(in) & 15u) == 0;
+    else d.wide = (la * es) % 16 == 0 && (lp_all * es) % 16 == 0 && (reinterpret_cast<uintptr_t>(in) & 15u) == 0;
     d.tx = tile_stretch(la, es, d.x_padded, d.wide);
     d.x_tiles = (d.x_padded + d.tx - 1) / d.tx;
     d.la = la, d.a_extent = (uint32_t)shape[a], d.a_groups = O[a];
@@ -385,6 +469,13 @@ static bool make_tile_desc(TileDesc &d, int es, int rank, const int32_t *shape, 
 template <bool PACK> static int launch_pack_tile(nncase_hip_ctx *ctx, const void *in, void *out, int es, const TileDesc &d, uint64_t blocks, size_t lds) {
     const dim3 grid((unsigned)blocks), block(kLayoutThreads);
     if (lds > 48 * 1024) return 1; // (not asked for: the tiles are sized to stay below)
+    if (d.ragged) {
+        if (es == 4) hipLaunchKernelGGL((pack_tile_kernel<1, PACK, true>), grid, block, lds, ctx->stream, (const uint8_t *)in, (uint8_t *)out, d);
+        else if (es == 1) hipLaunchKernelGGL((pack_tile_kernel<4, PACK, true>), grid, block, lds, ctx->stream, (const uint8_t *)in, (uint8_t *)out, d);
+        else hipLaunchKernelGGL((pack_tile_kernel<2, PACK, true>), grid, block, lds, ctx->stream, (const uint8_t *)in, (uint8_t *)out, d);
+        NNHIP_LAUNCH_CHECK(ctx, "pack_tile_kernel");
+        return 0;
+    }
     switch (es) {
     case 1: hipLaunchKernelGGL((pack_tile_kernel<4, PACK>), grid, block, lds, ctx->stream, (const uint8_t *)in, (uint8_t *)out, d); break;
     case 2: hipLaunchKernelGGL((pack_tile_kernel<2, PACK>), grid, block, lds, ctx->stream, (const uint8_t *)in, (uint8_t *)out, d); break;
@@ -428,16 +519,23 @@ static bool make_transpose_desc(TileDesc &d, int es, int batch, int rows, int co
                                 uint64_t &blocks, size_t &lds) {
     if (es != 1 && es != 2 && es != 4) return false;
     const int e = 4 / es;
-    if (((reinterpret_cast<uintptr_t>(in) | reinterpret_cast<uintptr_t>(out)) & 3u) != 0 || rows % e != 0 || cols % e != 0) return false;
+    if (((reinterpret_cast<uintptr_t>(in) | reinterpret_cast<uintptr_t>(out)) & 3u) != 0) return false;
+    const bool ragged = rows % e != 0 || cols % e != 0;
+    const uint64_t bytes = (uint64_t)batch * rows * cols * es;
+    // Few ragged tiles do not fill the device with blocks this heavy, the 32 x 32 ones are then quicker (155 channels of one
+    // 51 x 51 image of u8 4.9 against 6.0 us, of float16 4.7 / 6.9; of two 201 x 201 images 18.3 / 11.8 and 21.4 / 19.4).
+    if (ragged && bytes < ((uint64_t)es << 20)) return false;
     memset(&d, 0, sizeof(d));
+    d.ragged = ragged;
+    d.in_bytes = bytes;
     const int na = packing ? rows : cols, nx = packing ? cols : rows; // extents of A and X
-    const uint32_t la = (uint32_t)std::min(na, 128 / e * e);
+    const uint32_t la = (uint32_t)std::min((na + e - 1) / e * e, 128 / e * e); // (ragged: the last group's lanes past the extent hold nothing)
     d.la = la, d.a_extent = (uint32_t)na, d.a_groups = ((uint32_t)na + la - 1) / la;
     d.a_plain_stride = (uint64_t)nx, d.a_packed_group = la;
     d.x_extent = d.x_padded = (uint32_t)nx;
     d.x_packed = TwoTerm{1, (uint64_t)na, 0};
     d.exact = 1;
-    d.wide = packing && ((uint64_t)nx * es) % 16 == 0 && (reinterpret_cast<uintptr_t>(in) & 15u) == 0;
+    d.wide = packing && (d.ragged ? (uint64_t)nx * es >= 64 : ((uint64_t)nx * es) % 16 == 0 && (reinterpret_cast<uintptr_t>(in) & 15u) == 0);
     d.tx = tile_stretch(la, es, d.x_padded, d.wide);
     d.x_tiles = (d.x_padded + d.tx - 1) / d.tx;
     d.nrest = 1;

@@ -99,3 +99,27 @@ def test_nchw_nhwc(hip_ctx, shape, dtype):
     y = K.transpose_nchw_to_nhwc(x, ctx=hip_ctx)
     assert np.array_equal(y, x.transpose(0, 2, 3, 1))
     assert np.array_equal(K.transpose_nhwc_to_nchw(y, ctx=hip_ctx), x)
+
+
+@pytest.mark.parametrize("dtype", [np.uint8, np.float16, np.float32])
+@pytest.mark.parametrize("shape,lanes", [((1, 1, 1, 5), 4), ((1, 3, 1, 1), 4), ((2, 5, 3, 7), 4), ((3, 33, 9, 11), 32), ((1, 17, 37, 41), 16),
+                                         ((2, 40, 1, 2049), 32), ((1, 8, 64, 33), 8), ((5, 7, 31, 1), 4)])
+def test_pack_and_unpack_of_rows_that_end_inside_a_piece(hip_ctx, shape, lanes, dtype):
+    """Rows of the plain tensor begin at any element: pieces are read from unaligned addresses, the last of a row in part, and
+    the tensor's last bytes are not read past."""
+    rng = np.random.default_rng(shape[1] + lanes)
+    x = rng.integers(0, 200, shape).astype(dtype)
+    got = K.pack(x, [1], [lanes], ctx=hip_ctx)
+    assert np.array_equal(got, O.pack(x, [1], [lanes]))
+    assert np.array_equal(K.unpack(got, [1], [lanes], shape, ctx=hip_ctx), x)
+
+
+@pytest.mark.parametrize("dtype", [np.uint8, np.float16])
+@pytest.mark.parametrize("shape", [(1, 155, 201, 73), (9, 3, 223, 181), (2, 66, 101, 163), (1, 1031, 33, 65)])
+def test_relayout_of_odd_extents(hip_ctx, shape, dtype):
+    """NCHW <-> NHWC of tensors large enough for the tile kernel whose rows are no whole dwords on either side."""
+    rng = np.random.default_rng(shape[1])
+    x = rng.integers(0, 200, shape).astype(dtype)
+    y = K.transpose_nchw_to_nhwc(x, ctx=hip_ctx)
+    assert np.array_equal(y, x.transpose(0, 2, 3, 1))
+    assert np.array_equal(K.transpose_nhwc_to_nchw(y, ctx=hip_ctx), x)
