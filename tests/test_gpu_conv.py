@@ -728,3 +728,11 @@ def test_host_results_return_their_pinned_memory(hip_ctx):
     del held
     again = buf.download(src.shape, np.int32)
     assert again.base is not None and np.array_equal(again, src)
+@pytest.mark.parametrize("m,k,n", [(16400, 80, 516), (16500, 192, 510), (333, 128, 255), (4100, 112, 514), (70, 256, 66)])
+def test_matmul_of_two_to_four_k_steps(hip_ctx, m, k, n):
+    """Both sides of the rules that give short reductions the small wide blocks: many outputs, channel counts that are no
+    multiple of 4, four k-steps; whole and partial last k-steps and blocks."""
+    rng = np.random.default_rng(m + k + n)
+    a, b = rng.integers(0, 256, (m, k), dtype=np.uint8), rng.integers(0, 256, (k, n), dtype=np.uint8)
+    want = ((a.astype(np.float64) - 7) @ (b.astype(np.float64) - 131)).astype(np.int32)     # exact: below 2^53
+    assert np.array_equal(K.mat_mul(a, b, qp(7, 0.02), qp(131, 0.004), None, np.int32, None, ctx=hip_ctx), want)
