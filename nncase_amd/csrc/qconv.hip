@@ -38,6 +38,10 @@ void nnhip::describe_conv_kernel(const nncase_hip_ctx *ctx, const nncase_hip_wei
     const long long m = (long long)a->batch * out_h * out_w;
     const int mode = igemm_load_mode(w, a, out_h, out_w);
     const int mi = (int)std::min<long long>(m, 1 << 30);
+    if (const char *block = tile_kernel_block(ctx, w, a, out_h, out_w)) {
+        snprintf(buf, cap, "qconv_tile%s%s<%s>", w->d_post_lut ? "+lut" : "", a->residual_dev ? "+add" : "", block);
+        return;
+    }
     if (w->wide) {
         snprintf(buf, cap, "qconv_wide%s%s%s<T=%d,%s%s>", w->d_post_lut ? "+lut" : "", a->residual_dev ? "+add" : "",
                  a->dequantize_output ? "+dequantize" : "", w->tiles,

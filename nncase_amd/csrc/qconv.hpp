@@ -19,7 +19,7 @@ struct nncase_hip_weights {
     // of the activations, which makes the weight zero point's share of the product part of the multiplication
     int fold = 0;
     // igemm: packed for the wide-tile kernels (qconv_wide.hpp): 1 = long reductions over many pixels and channels
-    // (blocks of 256 or 128 pixels, waves of 64), 2 = reductions of five k-steps and more over fewer pixels (blocks of
+    // (blocks of 256 or 128 pixels, waves of 64), 2 = shorter reductions and fewer pixels (blocks of
     // `small_shape`, waves of 32 pixels)
     int wide = 0;
     int small_shape = 0;
@@ -151,6 +151,8 @@ int launch_qconv_rows(nncase_hip_ctx *ctx, const uint8_t *x, const nncase_hip_we
 // Writes the name of the kernel a conv with these weights / arguments launches.
 void describe_conv_kernel(const nncase_hip_ctx *ctx, const nncase_hip_weights *w, const nncase_hip_conv2d_args_t *a, char *buf,
                           size_t cap);
+// The block ("pixels x channels") of the tile kernel that takes such a call (qconv_tile.hip), or null.
+const char *tile_kernel_block(const nncase_hip_ctx *ctx, const nncase_hip_weights *w, const nncase_hip_conv2d_args_t *c, int out_h, int out_w);
 int igemm_pixel_groups(const nncase_hip_ctx *ctx, const nncase_hip_weights *w, int m);
 int igemm_load_mode(const nncase_hip_weights *w, const nncase_hip_conv2d_args_t *c, int out_h, int out_w);
 } // namespace nnhip

@@ -284,6 +284,12 @@ int launch_qconv_igemm(nncase_hip_ctx *ctx, const uint8_t *x, const nncase_hip_w
         a.y_coff = g * w->g_oc + c->out_channel_offset;
         a.r_coff = g * w->g_oc;
         int rc;
+        if (!w->ragged) {
+            bool taken;
+            rc = launch_qconv_tile(ctx, a, w->tiles, w->nchunks, &taken);
+            if (rc) return rc;
+            if (taken) continue;
+        }
         if (w->ragged) {
             const bool rows = igemm_is_pointwise(w, c, out_h, out_w);
             rc = w->wide == 2 ? launch_wide_small_ragged(ctx, a, rows, w->small_shape, w->nchunks) : launch_wide_ragged(ctx, a, rows, w->tiles, w->nchunks);

@@ -1,0 +1,474 @@
+// u8/u8 convolution over a window, with the input of a two-dimensional tile of output pixels in LDS.
+//
+// The implicit-GEMM kernels fetch, re-bias and sum an activation once per tap of the window: nine times for 3x3, a hundred
+// instructions of a wave per k-step against eight products, and an instruction of a wave that is alone on its SIMD takes eight
+// to nine cycles.  Here a block brings the input under its tile of output pixels into LDS once (re-biased, the padding filled
+// with the zero point) and every tap is an LDS read at another offset; the sum of x over a window, which the weight zero
+// point multiplies, is the sum of per-pixel channel sums taken on the way in.  What is left of a k-step is RG + 1 LDS reads
+// (operands and where the next tap lies), T loads of packed weights straight into registers, four k-steps ahead, and the
+// products: no barrier, no staging.  A wave owns RG * 16 pixels x T * 16 channels; a block is WM x WN waves.
+//   * weights come from L2 through the vector L1 (64 bytes per clock): with 64 x 32 outputs per wave a k-step of four waves
+//     takes 8 KiB of them for 128 clocks of matrix work, so waves share pixels rather than channels where they can;
+//   * blocks start the reduction at different k-steps (integer sums do not care): otherwise all of them wait for the same
+//     weights to come from memory at the same time, step after step;
+//   * results leave through LDS as whole pixel rows.
+// Arithmetic, weight packing and the bytes of the result are those of qconv_igemm.hpp.
+#include "qconv_wide.hpp"
+
+namespace nnhip {
+
+struct TileArgs {
+    int th, tw;                    // output tile
+    int hr, hc;                    // input rows / columns under it
+    int half;                      // input columns per column phase (stride 2: column c lies at (c & 1) * half + c / 2, so that
+                                   // neighbouring output pixels read neighbouring LDS pixels)
+    int pitch, row_pitch;          // bytes of an LDS pixel (an odd number of 16-byte pieces: eight lanes, eight banks) / row
+    int pieces;                    // 16-byte pieces per pixel
+    int dq, dc, dr;                // a block's threads as a step in (piece, column, row)
+    int row_bytes;                 // of the tensor
+    int tile_off;
+    FastDiv d_pieces, d_hc, d_tw, d_tx, d_txy, d_nchunks, d_rest;
+};
+
+// FAST: the requantisation is the one-instruction form without a clamp of its own (Epilogue::fast and ::full).
+
+template <int T, int RG, int WM, int WN, bool FAST>
+__global__ __launch_bounds__(WM * WN * 64, 4) void qconv_tile_kernel(const IgemmArgs a, const TileArgs t) {
+    constexpr int THREADS = WM * WN * 64, PIX = WM * RG * 16, TB = T * WN;
+    constexpr int D = 4;                                             // k-steps of weights in flight
+    extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
+    int32_t *cterm = reinterpret_cast<int32_t *>(smem);              // [TB * 16]
+    int32_t *sums = cterm + TB * 16;                                 // [PIX] sum of x' over a pixel's window
+    uint8_t *lutl = reinterpret_cast<uint8_t *>(sums + PIX);         // [256]
+    int32_t *taps = reinterpret_cast<int32_t *>(lutl + 256);         // [KS + 2][4] LDS offset of a piece of the reduction
+    uint8_t *tile = smem + t.tile_off;
+
+    // as in qconv_wide_kernel: channel chunks of a tile back to back, a contiguous eighth of the tiles per XCD
+    const int xcd = blockIdx.x & 7, seq = blockIdx.x >> 3;
+    const int turn = (int)fastdiv((uint32_t)seq, t.d_nchunks), chunk = seq - turn * (int)t.d_nchunks.div;
+    const int per = (a.num_mtiles + 7) >> 3;
+    const int mt = xcd * per + turn;
+    if (turn >= per || mt >= a.num_mtiles) return;
+
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wm = wave % WM, wn = wave / WM;
+    const int j = lane & 15, gq = lane >> 4;
+    const int KS = a.ksteps;
+    const int ch_base = chunk * (TB * 16);
+    const bool two = a.stride_w == 2;
+
+    // ---- the input tile: requested in batches of U pieces per thread, the next before one is stored ----
+    const uint32_t img = fastdiv((uint32_t)mt, t.d_txy);
+    const uint32_t in_img = (uint32_t)mt - img * t.d_txy.div;
+    const uint32_t tyi = fastdiv(in_img, t.d_tx);
+    const int oy0 = (int)tyi * t.th, ox0 = (int)(in_img - tyi * t.d_tx.div) * t.tw;
+    const int iy0 = oy0 * a.stride_h - a.pad_h, ix0 = ox0 * a.stride_w - a.pad_w;
+    const int base = ((int)img * a.in_h + iy0) * t.row_bytes + ix0 * a.ldx + a.x_coff; // (may be negative at a border)
+    const __amdgpu_buffer_rsrc_t xres = wide_rsrc(a.x, (uint32_t)a.x_bytes);
+    constexpr int U = 4;
+    struct Batch {
+        wide_u32x4 v[U];
+        int dst[U];        // where the piece goes in LDS; its bit 0: the pixel lies in the padding
+    };
+    const int n = t.hr * t.hc * t.pieces;
+    const bool inside = iy0 >= 0 && ix0 >= 0 && iy0 + t.hr <= a.in_h && ix0 + t.hc <= a.in_w; // no padding under this tile
+    int q, r, c; // piece, row and column of this thread's next piece
+    {
+        const uint32_t p0 = fastdiv((uint32_t)tid, t.d_pieces);
+        q = tid - (int)p0 * t.pieces;
+        r = (int)fastdiv(p0, t.d_hc);
+        c = (int)p0 - r * t.hc;
+    }
+    // (a thread past the tile's last piece reads what follows it in the tensor, or 0 past its end, and drops it)
+    auto request = [&](Batch &f, int i0) __attribute__((always_inline)) {
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            if (i0 + u * THREADS >= n) break;
+            const int goff = __mul24(r, t.row_bytes) + __mul24(c, a.ldx) + q * 16;
+            const int pos = two ? (c & 1) * t.half + (c >> 1) : c;
+            f.dst[u] = __mul24(r, t.row_pitch) + __mul24(pos, t.pitch) + q * 16;
+            if (inside) {
+                f.v[u] = __builtin_amdgcn_raw_buffer_load_b128(xres, goff, base, 0);
+            } else {
+                const bool in = (unsigned)(iy0 + r) < (unsigned)a.in_h && (unsigned)(ix0 + c) < (unsigned)a.in_w;
+                f.v[u] = __builtin_amdgcn_raw_buffer_load_b128(xres, in ? (uint32_t)(base + goff) : 0xffffffffu, 0, 0);
+                f.dst[u] |= in ? 0 : 1;
+            }
+            q += t.dq;
+            const bool cq = q >= t.pieces;
+            q -= cq ? t.pieces : 0;
+            c += t.dc + (cq ? 1 : 0);
+            const bool cc = c >= t.hc;
+            c -= cc ? t.hc : 0;
+            r += t.dr + (cc ? 1 : 0);
+        }
+    };
+    auto keep = [&](const Batch &f, int i0) __attribute__((always_inline)) {
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            if (i0 + u * THREADS >= n) break;
+            if (i0 + u * THREADS + tid < n) {
+                const uint32_t fill = (f.dst[u] & 1) ? a.zx_splat : 0u;
+                wide_u32x4 w;
+#pragma unroll
+                for (int d = 0; d < 4; d++) w[d] = (inside ? f.v[u][d] : f.v[u][d] | fill) ^ 0x80808080u;
+                *reinterpret_cast<wide_u32x4 *>(tile + (f.dst[u] & ~1)) = w;
+            }
+        }
+    };
+    Batch fa;
+    request(fa, 0);
+
+    // ---- weights: D k-steps ahead.  The last k-step, which may end past the reduction, comes first, the others follow from
+    // where this block starts ----
+    const __amdgpu_buffer_rsrc_t wres = wide_rsrc(a.wpk + (size_t)chunk * KS * TB * 1024, (uint32_t)KS * TB * 1024);
+    const int rest = KS - 1;
+    const int ks0 = rest == 0 ? 0 : seq - (int)fastdiv((uint32_t)seq, t.d_rest) * rest;
+    const int w_end = rest * TB * 1024, w_lane = wn * T * 1024 + lane * 16;
+    int w_off = rest * TB * 1024; // of the next k-step to request
+    auto load_w = [&](v4i (&dst)[T]) __attribute__((always_inline)) {
+#pragma unroll
+        for (int nt = 0; nt < T; nt++) dst[nt] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(wres, w_lane + nt * 1024, w_off, 0));
+    };
+    v4i wf[D][T];
+    load_w(wf[0]);
+    w_off = ks0 * TB * 1024;
+    auto load_next = [&](v4i (&dst)[T]) __attribute__((always_inline)) {
+        load_w(dst);
+        w_off += TB * 1024;
+        w_off = w_off == w_end ? 0 : w_off;
+    };
+#pragma unroll
+    for (int d = 1; d < D; d++) load_next(wf[d]);
+
+    // ---- tables ----
+    for (int e = tid; e < (KS + 2) * 4; e += THREADS) { // in the order of this block's k-steps
+        const int s = e >> 2;
+        int ks = s == 0 ? rest : ks0 + s - 1;
+        ks -= s > 0 && ks >= rest ? rest : 0;
+        const int kk = ks * 64 + (e & 3) * 16;
+        int off = 0; // (past the reduction: any place, its weights are 0)
+        if (kk < a.k && s < KS) {
+            const uint32_t tap = fastdiv((uint32_t)kk, a.d_gic);
+            const uint32_t ky = fastdiv(tap, a.d_kw);
+            const int dx = ((int)tap - (int)ky * a.kw) * a.dil_w;
+            off = (int)ky * a.dil_h * t.row_pitch + (two ? (dx & 1) * t.half + (dx >> 1) : dx) * t.pitch + kk - (int)tap * a.g_ic;
+        }
+        taps[e] = off;
+    }
+    for (int i = tid; i < TB * 16; i += THREADS) {
+        const bool real = ch_base + i < a.n;
+        cterm[i] = real ? a.bias[ch_base + i] - a.zxp * a.wsum[ch_base + i] + a.k * a.zxp * a.zwp : 0;
+    }
+    if (a.lut && tid < 64) reinterpret_cast<uint32_t *>(lutl)[tid] = a.lut[tid];
+    // this lane's pixels: pixel (wm RG + rg) * 16 + j of the tile, in rows of tw
+    auto lds_of = [&](int group) __attribute__((always_inline)) {
+        const uint32_t p = (wm * RG + group) * 16 + j;
+        int ty = (int)fastdiv(p, t.d_tw);
+        int tx = (int)p - ty * t.tw;
+        if (ty >= t.th) ty = tx = 0; // (surplus of the block: not stored)
+        return __mul24(ty, a.stride_h * t.row_pitch) + __mul24(tx, t.pitch);
+    };
+    // the sum of x' of a pixel group comes from a product with ones; waves that share the pixels share that work
+    constexpr int SG = (RG + WN - 1) / WN; // groups per wave
+    int xbase[RG], xsum[SG];
+#pragma unroll
+    for (int rg = 0; rg < RG; rg++) xbase[rg] = lds_of(rg);
+#pragma unroll
+    for (int i = 0; i < SG; i++) xsum[i] = WN == 1 ? xbase[i] : lds_of(min(wn * SG + i, RG - 1));
+    {
+        int i0 = 0;
+        for (; i0 + U * THREADS < n; i0 += U * THREADS) {
+            Batch fb;
+            request(fb, i0 + U * THREADS);
+            keep(fa, i0);
+            fa = fb;
+        }
+        keep(fa, i0);
+    }
+    __syncthreads();
+
+    // ---- the reduction ----
+    const int ch0 = gq * (4 * TB) + wn * (4 * T);
+    v4i acc[RG][T], rs[SG];
+    v4i xf[2][RG], xs[2][SG]; // (a wave reads the operand it sums by itself: which of xf that is depends on the wave)
+    const int32_t *tap = taps + gq; // of the k-step whose operands are read next
+    int toff = tap[0];
+    auto operands = [&](v4i (&dst)[RG], v4i (&dsts)[SG], int ahead) __attribute__((always_inline)) {
+#pragma unroll
+        for (int rg = 0; rg < RG; rg++) dst[rg] = *reinterpret_cast<const v4i *>(tile + xbase[rg] + toff);
+#pragma unroll
+        for (int i = 0; i < SG; i++) dsts[i] = WN == 1 ? dst[i] : *reinterpret_cast<const v4i *>(tile + xsum[i] + toff);
+        toff = tap[ahead * 4];
+    };
+    operands(xf[0], xs[0], 1);
+    operands(xf[1], xs[1], 2);
+    tap += 2 * 4;
+    const v4i ones = {0x01010101, 0x01010101, 0x01010101, 0x01010101};
+    {
+        const int one = rest * 64 + gq * 16 < a.k ? 0x01010101 : 0; // (pieces past the reduction)
+        const v4i ones_last = {one, one, one, one}, zero = {0, 0, 0, 0};
+#pragma unroll
+        for (int nt = 0; nt < T; nt++) {
+            const v4i ct = *reinterpret_cast<const v4i *>(cterm + ch0 + nt * 4);
+#pragma unroll
+            for (int rg = 0; rg < RG; rg++) acc[rg][nt] = __builtin_amdgcn_mfma_i32_16x16x64_i8(wf[0][nt], xf[0][rg], ct, 0, 0, 0);
+        }
+#pragma unroll
+        for (int i = 0; i < SG; i++) rs[i] = __builtin_amdgcn_mfma_i32_16x16x64_i8(ones_last, xs[0][i], zero, 0, 0, 0);
+    }
+    load_next(wf[0]);
+    // (whole groups of D k-steps without a branch between them: behind one, a wait for one k-step's weights waits for all)
+    auto kstep = [&](auto u_c) __attribute__((always_inline)) {
+        constexpr int u = decltype(u_c)::value, b = u % D;
+        operands(xf[(u + 1) & 1], xs[(u + 1) & 1], u);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int nt = 0; nt < T; nt++)
+#pragma unroll
+            for (int rg = 0; rg < RG; rg++) acc[rg][nt] = __builtin_amdgcn_mfma_i32_16x16x64_i8(wf[b][nt], xf[u & 1][rg], acc[rg][nt], 0, 0, 0);
+#pragma unroll
+        for (int i = 0; i < SG; i++) rs[i] = __builtin_amdgcn_mfma_i32_16x16x64_i8(ones, xs[u & 1][i], rs[i], 0, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+        load_next(wf[b]);
+    };
+    int left = rest;
+#pragma clang loop unroll(disable)
+    for (; left >= D; left -= D) {
+        static_for<1, D + 1>(kstep);
+        tap += D * 4;
+    }
+    static_for<1, D>([&](auto u_c) __attribute__((always_inline)) {
+        if (decltype(u_c)::value <= left) kstep(u_c);
+    });
+
+    // ---- epilogue ----
+    if (gq == 0) {
+#pragma unroll
+        for (int i = 0; i < SG; i++)
+            if (wn * SG + i < RG) sums[(wm * RG + wn * SG + i) * 16 + j] = rs[i][0];
+    }
+    __syncthreads(); // the sums are there, and every wave is through with the tile: its place takes the result
+    int32_t owed[RG];
+#pragma unroll
+    for (int rg = 0; rg < RG; rg++) owed[rg] = -a.zwp * sums[(wm * RG + rg) * 16 + j];
+    const int oh_img = (int)a.d_ohow.div, ow = (int)a.d_ow.div;
+    // pixel index of the tensor of pixel p of the block, a.m where there is none
+    auto pixel_of = [&](uint32_t p) __attribute__((always_inline)) {
+        const int ty = (int)fastdiv(p, t.d_tw);
+        const int oy = oy0 + ty, ox = ox0 + (int)p - ty * t.tw;
+        const int at = __mul24(oy, ow) + ox;
+        return ty < t.th && ox < ow && at < oh_img ? (int)img * oh_img + at : a.m;
+    };
+    constexpr int kOutPitch = TB * 16 + 16;
+    uint32_t packed[RG][T];
+#pragma unroll
+    for (int rg = 0; rg < RG; rg++)
+#pragma unroll
+        for (int nt = 0; nt < T; nt++) {
+            int32_t v[4];
+#pragma unroll
+            for (int r = 0; r < 4; r++) v[r] = acc[rg][nt][r] + owed[rg];
+            packed[rg][nt] = FAST ? requant4_u8_packed_direct(v, a.ep) : requant4_u8_packed(v, a.ep);
+        }
+    if (a.lut) { // (every byte is asked for before the first is used)
+        uint32_t b[RG][T][4];
+#pragma unroll
+        for (int rg = 0; rg < RG; rg++)
+#pragma unroll
+            for (int nt = 0; nt < T; nt++)
+#pragma unroll
+                for (int r = 0; r < 4; r++) b[rg][nt][r] = lutl[(packed[rg][nt] >> (8 * r)) & 0xffu];
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int rg = 0; rg < RG; rg++)
+#pragma unroll
+            for (int nt = 0; nt < T; nt++) packed[rg][nt] = b[rg][nt][0] | (b[rg][nt][1] << 8) | (b[rg][nt][2] << 16) | (b[rg][nt][3] << 24);
+    }
+#pragma unroll
+    for (int rg = 0; rg < RG; rg++) {
+        uint32_t *o = reinterpret_cast<uint32_t *>(tile + ((wm * RG + rg) * 16 + j) * kOutPitch + ch0);
+#pragma unroll
+        for (int nt = 0; nt < T; nt++) o[nt] = packed[rg][nt];
+    }
+    __syncthreads();
+    // whole pixel rows: TB threads per pixel, 16 channels each
+    const bool wide_y = ((a.ldy | a.y_coff) & 3) == 0, wide_r = ((a.ldr | a.r_coff) & 3) == 0;
+    constexpr int PPT = THREADS / TB; // pixels of a pass
+    static_assert(PIX % PPT == 0, "whole passes");
+    const int cb = (tid % TB) * 16, ch = ch_base + cb;
+    if (ch >= a.n) return;
+    const bool whole = ch + 16 <= a.n;
+#pragma unroll
+    for (int it = 0; it < PIX / PPT; it++) {
+        const int p = it * PPT + tid / TB;
+        const int px = pixel_of(p);
+        if (px >= a.m) continue;
+        u32x4 v = *reinterpret_cast<const u32x4 *>(tile + p * kOutPitch + cb);
+        if (a.rep.res) {
+            const uint8_t *ro = a.rep.res + (size_t)px * a.ldr + a.r_coff + ch;
+            u32x4 rv = {0, 0, 0, 0};
+            if (whole && wide_r) {
+                const u32x4_a4 r4 = *reinterpret_cast<const u32x4_a4 *>(ro);
+                rv = u32x4{r4[0], r4[1], r4[2], r4[3]};
+            } else {
+#pragma unroll
+                for (int b = 0; b < 16; b++)
+                    if (ch + b < a.n) rv[b / 4] |= (uint32_t)ro[b] << (8 * (b & 3));
+            }
+#pragma unroll
+            for (int d = 0; d < 4; d++) v[d] = residual4_packed(v[d], rv[d], a.rep);
+        }
+        uint8_t *yo = reinterpret_cast<uint8_t *>(a.y) + (size_t)px * a.ldy + a.y_coff + ch;
+        if (whole && wide_y) {
+            *reinterpret_cast<u32x4_a4 *>(yo) = u32x4_a4{v[0], v[1], v[2], v[3]};
+        } else if (whole) {
+#pragma unroll
+            for (int d = 0; d < 4; d++) reinterpret_cast<U32Unaligned *>(yo + d * 4)->v = v[d];
+        } else {
+#pragma unroll
+            for (int b = 0; b < 16; b++)
+                if (ch + b < a.n) yo[b] = (uint8_t)(v[b / 4] >> (8 * (b & 3)));
+        }
+    }
+}
+
+namespace {
+struct TilePlan {
+    TileArgs t;
+    int tiles; // of the whole batch
+    size_t lds;
+};
+
+// The output tile of at most `pix` pixels: the fewest blocks, then the smallest input.
+TilePlan plan_tile(const IgemmArgs &a, int pix, int tb, int threads, int nchunks) {
+    const int ow = (int)a.d_ow.div, oh = (int)a.d_ohow.div / ow, batch = a.m / (int)a.d_ohow.div;
+    TilePlan best;
+    long long best_blocks = -1, best_area = 0;
+    for (int nx = ceil_div(ow, std::min(pix, 32)); nx <= ow; nx++) {
+        const int tw = ceil_div(ow, nx);
+        if (nx > 1 && tw == ceil_div(ow, nx - 1)) continue;
+        const int rows = std::min(pix / tw, oh), th = ceil_div(oh, ceil_div(oh, rows)); // rows spread evenly over the tiles
+        const int tx = ceil_div(ow, tw), ty = ceil_div(oh, th);
+        const int hr = (th - 1) * a.stride_h + (a.kh - 1) * a.dil_h + 1, hc = (tw - 1) * a.stride_w + (a.kw - 1) * a.dil_w + 1;
+        const long long blocks = (long long)tx * ty, area = (long long)hr * hc;
+        if (best_blocks >= 0 && (blocks > best_blocks || (blocks == best_blocks && area >= best_area))) {
+            if (tw < 4) break;
+            continue;
+        }
+        best_blocks = blocks, best_area = area;
+        TileArgs &t = best.t;
+        t.th = th, t.tw = tw, t.hr = hr, t.hc = hc;
+        t.half = ceil_div(hc, a.stride_w);
+        t.pieces = a.g_ic / 16;
+        t.pitch = (t.pieces | 1) * 16;
+        t.row_pitch = a.stride_w * t.half * t.pitch;
+        t.row_bytes = a.in_w * a.ldx;
+        t.d_pieces = make_fastdiv((uint32_t)t.pieces), t.d_hc = make_fastdiv((uint32_t)hc), t.d_tw = make_fastdiv((uint32_t)tw);
+        t.d_tx = make_fastdiv((uint32_t)tx), t.d_txy = make_fastdiv((uint32_t)(tx * ty));
+        best.tiles = batch * tx * ty;
+    }
+    TileArgs &t = best.t;
+    t.d_nchunks = make_fastdiv((uint32_t)nchunks), t.d_rest = make_fastdiv((uint32_t)std::max(1, a.ksteps - 1));
+    t.tile_off = (tb * 16 + pix + (a.ksteps + 2) * 4) * 4 + 256;
+    t.dq = threads % t.pieces, t.dc = threads / t.pieces % t.hc, t.dr = threads / t.pieces / t.hc;
+    best.lds = t.tile_off + std::max((size_t)t.hr * t.row_pitch, (size_t)pix * (tb * 16 + 16));
+    return best;
+}
+
+template <int T, int RG, int WM, int WN, bool FAST> int launch_tile_f(nncase_hip_ctx *ctx, const IgemmArgs &args, const TilePlan &plan, int nchunks) {
+    if (plan.lds > 65536) {
+        static std::once_flag raised[16];
+        hipError_t attr = hipSuccess;
+        std::call_once(raised[ctx->device & 15], [&] {
+            attr = hipFuncSetAttribute(reinterpret_cast<const void *>(&qconv_tile_kernel<T, RG, WM, WN, FAST>), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+        });
+        NNHIP_HIP(ctx, attr);
+    }
+    hipLaunchKernelGGL((qconv_tile_kernel<T, RG, WM, WN, FAST>), dim3(ceil_div(args.num_mtiles, 8) * 8 * nchunks), dim3(WM * WN * 64), plan.lds, ctx->stream, args,
+                       plan.t);
+    NNHIP_LAUNCH_CHECK(ctx, "qconv_tile_kernel");
+    return 0;
+}
+template <int T, int RG, int WM, int WN> int launch_tile_t(nncase_hip_ctx *ctx, const IgemmArgs &a, const TilePlan &plan, int nchunks) {
+    IgemmArgs args = a;
+    args.num_mtiles = plan.tiles;
+    return a.ep.fast && a.ep.full ? launch_tile_f<T, RG, WM, WN, true>(ctx, args, plan, nchunks) : launch_tile_f<T, RG, WM, WN, false>(ctx, args, plan, nchunks);
+}
+} // namespace
+
+namespace {
+enum TileShape { kTile128x32, kTile64x32, kTile32x64, kTile128x128, kTile64x128, kTileNone };
+
+template <int T, int RG, int WM, int WN> TilePlan plan_shape(const IgemmArgs &a, int nchunks) {
+    return plan_tile(a, WM * RG * 16, T * WN, WM * WN * 64, nchunks);
+}
+
+// Which block, if any, by the packed chunk (`tiles` of 16 channels) and the waves the launch has (byte results, windows,
+// strides of 1 and 2).  Measured us, implicit GEMM / here, byte table behind the convolution:
+//   * eight waves share the staging of a 128-channel chunk: 25 600 pixels 128 -> 128 3x3 11.7 / 9.7 with 128 pixels per block
+//     (10.4 with 64), 6400 pixels 256 -> 256 11.8 / 9.2 with 64 (11.4 with 128: fewer blocks than compute units);
+//   * one wave row of 32 pixels for 64 channels: 102 400 pixels 64 -> 64 12.7 / 11.5 (13.9 with 128 pixels, 12.3 with 64);
+//   * 32 channels: 409 600 pixels 32 -> 32 21.9 / 15.6, 1 638 400 pixels 16 -> 32 41.4 / 36.7; two k-steps and fewer are the
+//     epilogue's work alone and stay (802 816 pixels 16 -> 32 2x2 14.9 / 18.6);
+//   * stride 2 brings in four times the input: from 16 k-steps on (25 600 pixels 128 -> 256 18.5 / 15.9, 6400 pixels 256 -> 512
+//     18.0 / 15.5, but 409 600 pixels 32 -> 64, five k-steps, 28.2 / 30.3);
+//   * tiles that images do not fill by half stay (their surplus pixels are multiplied and dropped);
+//   * with fewer than three waves per two compute units (stride 2: four per unit) the k-steps split over groups of waves win
+//     (400 pixels 256 -> 256 7.1 / 7.5; 1600 pixels 128 -> 256 stride 2 5.8 / 6.8).
+TileShape choose_tile(const nncase_hip_ctx *ctx, const IgemmArgs &a, int tiles, int nchunks, TilePlan *plan) {
+    if (a.kh * a.kw == 1 || a.g_ic % 16 != 0 || a.kc_mask != -1 || a.stride_w > 2 || (int64_t)a.in_w * a.ldx >= (1 << 23)) return kTileNone;
+    if (a.ksteps < (a.stride_w == 2 ? 16 : 3)) return kTileNone;
+    TileShape shape = kTileNone;
+    int waves = 2, pix = 64;
+    // (the smaller tile too where the larger one is not half full of an image's pixels)
+    auto enough = [&](int blocks) { return (long long)plan->tiles * nchunks >= blocks && 2ll * a.m >= (long long)plan->tiles * 128; };
+    switch (tiles) {
+    case 2:
+        *plan = plan_shape<2, 4, 2, 1>(a, nchunks), shape = kTile128x32, pix = 128;
+        if (!enough(3 * ctx->compute_units)) *plan = plan_shape<2, 2, 2, 1>(a, nchunks), shape = kTile64x32, pix = 64;
+        break;
+    case 4: *plan = plan_shape<2, 2, 1, 2>(a, nchunks), shape = kTile32x64, pix = 32; break;
+    case 8:
+        *plan = plan_shape<2, 4, 2, 4>(a, nchunks), shape = kTile128x128, waves = 8, pix = 128;
+        if (!enough(3 * ctx->compute_units / 4)) *plan = plan_shape<2, 2, 2, 4>(a, nchunks), shape = kTile64x128, pix = 64;
+        break;
+    default: return kTileNone;
+    }
+    if (2ll * a.m < (long long)plan->tiles * pix) return kTileNone;
+    const long long launched = (long long)plan->tiles * nchunks * waves;
+    if (2 * launched < (a.stride_w == 2 ? 8 : 3) * (long long)ctx->compute_units) return kTileNone;
+    return plan->lds <= 160 * 1024 ? shape : kTileNone;
+}
+} // namespace
+
+const char *tile_kernel_block(const nncase_hip_ctx *ctx, const nncase_hip_weights *w, const nncase_hip_conv2d_args_t *c, int out_h, int out_w) {
+    static const char *const names[] = {"128x32", "64x32", "32x64", "128x128", "64x128", nullptr};
+    if (w->ragged || c->out_dtype != NNCASE_HIP_DT_U8 || c->dequantize_output) return nullptr;
+    IgemmArgs a;
+    memset(&a, 0, sizeof(a));
+    a.m = (int)std::min<int64_t>((int64_t)c->batch * out_h * out_w, 1 << 30);
+    a.d_ohow = make_fastdiv((uint32_t)(out_h * out_w)), a.d_ow = make_fastdiv((uint32_t)out_w);
+    a.kh = w->kernel_h, a.kw = w->kernel_w, a.stride_h = c->stride_h, a.stride_w = c->stride_w, a.dil_h = c->dilation_h, a.dil_w = c->dilation_w;
+    a.g_ic = w->tap_ic, a.in_w = c->in_w, a.ldx = w->in_channels, a.ksteps = w->ksteps, a.kc_mask = w->fold ? 1 : -1;
+    TilePlan plan;
+    return names[choose_tile(ctx, a, w->tiles, w->nchunks, &plan)];
+}
+
+int launch_qconv_tile(nncase_hip_ctx *ctx, const IgemmArgs &a, int tiles, int nchunks, bool *taken) {
+    TilePlan plan;
+    const TileShape shape = a.ep.out_mode == kOutU8 && !a.deq ? choose_tile(ctx, a, tiles, nchunks, &plan) : kTileNone;
+    *taken = shape != kTileNone;
+    switch (shape) {
+    case kTile128x32: return launch_tile_t<2, 4, 2, 1>(ctx, a, plan, nchunks);
+    case kTile64x32: return launch_tile_t<2, 2, 2, 1>(ctx, a, plan, nchunks);
+    case kTile32x64: return launch_tile_t<2, 2, 1, 2>(ctx, a, plan, nchunks);
+    case kTile128x128: return launch_tile_t<2, 4, 2, 4>(ctx, a, plan, nchunks);
+    case kTile64x128: return launch_tile_t<2, 2, 2, 4>(ctx, a, plan, nchunks);
+    case kTileNone: break;
+    }
+    return 0;
+}
+
+} // namespace nnhip

@@ -736,3 +736,65 @@ def test_matmul_of_two_to_four_k_steps(hip_ctx, m, k, n):
     a, b = rng.integers(0, 256, (m, k), dtype=np.uint8), rng.integers(0, 256, (k, n), dtype=np.uint8)
     want = ((a.astype(np.float64) - 7) @ (b.astype(np.float64) - 131)).astype(np.int32)     # exact: below 2^53
     assert np.array_equal(K.mat_mul(a, b, qp(7, 0.02), qp(131, 0.004), None, np.int32, None, ctx=hip_ctx), want)
+
+
+@pytest.mark.parametrize("n,cin,cout,hw,k,stride,dil,pad,block,extra", [
+    (2, 16, 32, (150, 131), (3, 3), (1, 1), (1, 1), ((1, 1), (1, 1)), "64x32", ""),           # 144 of 192 reduction positions
+    (6, 32, 30, (131, 150), (3, 3), (1, 1), (1, 1), ((0, 2), (2, 0)), "128x32", "lut"),       # channels that end inside a dword
+    (2, 48, 17, (97, 129), (1, 7), (2, 1), (1, 1), ((0, 0), (3, 3)), "64x32", "add"),
+    (2, 32, 64, (80, 81), (5, 3), (1, 1), (2, 3), ((4, 4), (3, 3)), "32x64", "lut+add"),      # dilated both ways
+    (3, 64, 60, (64, 67), (3, 3), (1, 1), (1, 1), ((1, 1), (1, 1)), "32x64", "slice"),
+    (8, 128, 128, (40, 41), (3, 3), (1, 1), (1, 1), ((1, 1), (1, 1)), "64x128", "clamp"),
+    (14, 96, 100, (40, 48), (3, 3), (1, 1), (1, 1), ((1, 1), (1, 1)), "128x128", "add"),
+    (12, 128, 130, (56, 64), (3, 3), (2, 2), (1, 1), ((1, 1), (1, 1)), "32x64", "lut"),       # three chunks, the last of 2 channels
+    (16, 128, 128, (64, 96), (3, 3), (1, 2), (1, 1), ((1, 1), (1, 1)), "128x128", ""),
+    (24, 256, 128, (41, 39), (3, 3), (2, 2), (1, 2), ((0, 1), (1, 2)), "64x128", ""),         # both column phases, dilated
+    (600, 32, 128, (7, 5), (3, 3), (1, 1), (1, 1), ((1, 1), (1, 1)), "64x128", "")])          # an image inside one tile
+def test_convolution_over_an_input_tile_in_lds(hip_ctx, n, cin, cout, hw, k, stride, dil, pad, block, extra):
+    """Windows over a tile of the input in LDS: partial tiles, borders, both strides and column phases, dilation, reductions that
+    end inside a k-step, channel tails, and what may sit in the epilogue."""
+    rng = np.random.default_rng(cin * 7 + cout + n)
+    x = rng.integers(0, 256, (n, cin) + hw, dtype=np.uint8)
+    w = rng.integers(0, 256, (cout, cin) + k, dtype=np.uint8)
+    bias = rng.integers(-3000, 3000, cout).astype(np.int32)
+    zx, sx, zw, sw = 203, f32(0.0235), 135, f32(0.0041)
+    geometry = dict(stride=stride, dilation=dil, padding=pad)
+    acc = O.qconv2d(x, w, bias, zx, sx, zw, sw, out_mode=O.OUT_I32, **geometry)
+    real = acc.astype(np.float64) * float(sx * sw)
+    sy, zy = f32((real.max() - real.min()) * 0.6 / 255), 120
+    clamp = tuple(float(v) for v in np.percentile(real, [5, 80]).astype(f32)) if "clamp" in extra else FULL
+    want = O.requant_u8(acc, sx, sw, sy, zy, clamp)
+    oh, ow = want.shape[2:]
+    wt = hip_ctx.prepack_conv2d(w, bias, qp(zw, sw), 1, expected_pixels=n * oh * ow)
+    a = rt.Conv2dArgs(n, hw[0], hw[1], *stride, *dil, *pad[0], *pad[1], qp(zx, sx), qp(zy, sy), *clamp, rt.DT_U8)
+    last = (zy, sy)
+    if "lut" in extra:
+        lz, ls = 18, f32(sy * 0.9)
+        want = O.unary_lut(O.LUT_SWISH, zy, sy, lz, ls)[want]
+        wt.set_post_lut(rt.make_unary_lut(rt.LUT_SWISH, qp(zy, sy), qp(lz, ls)), qp(lz, ls))
+        last = (lz, ls)
+    if "add" in extra:
+        res = rng.integers(0, 256, want.shape, dtype=np.uint8)
+        want = O.qadd(want, res, last[0], last[1], 77, 0.02, 40, float(last[1]) * 1.3)
+        res_dev = hip_ctx.to_device(np.ascontiguousarray(res.transpose(0, 2, 3, 1)))
+        a.residual_dev, a.residual_qp, a.sum_qp = res_dev.ptr, qp(77, 0.02), qp(40, float(last[1]) * 1.3)
+        a.sum_clamp_min, a.sum_clamp_max = FULL
+    want = np.ascontiguousarray(want.transpose(0, 2, 3, 1))
+    if "slice" in extra:
+        a.out_channel_stride, a.out_channel_offset = cout + 11, 7
+        whole = rng.integers(0, 256, want.shape[:3] + (cout + 11,), dtype=np.uint8)
+        y = hip_ctx.to_device(whole)
+        whole[..., 7:7 + cout] = want
+        want = whole
+    else:
+        y = hip_ctx.alloc(want.size)
+    xd = hip_ctx.to_device(np.ascontiguousarray(x.transpose(0, 2, 3, 1)))
+    fn = rt.Function(hip_ctx)
+    fn.add_qconv2d(xd, wt, y, a)
+    name = fn.op_kernel(0)
+    fn.invoke()
+    hip_ctx.sync()
+    fn.destroy()
+    got = y.download(want.shape, np.uint8)
+    assert np.array_equal(got, want), f"{name}: {(got != want).sum()} of {want.size} bytes differ"
+    assert name.startswith("qconv_tile") and name.endswith(f"<{block}>"), name
