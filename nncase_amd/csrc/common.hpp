@@ -184,4 +184,14 @@ int attn_decode_on(nncase_hip_ctx *ctx, const void *q_dev, const void *k_cache_d
                    const int32_t *ctx_lens_dev, void *out_dev, const nncase_hip_paged_attn_args_t *geometry, void *partials,
                    size_t partial_bytes, void *counters, size_t counter_bytes);
 
+// glue.hip: a max pool of stride 1 over its own result, `levels` times, and the channel concat of the tensor and all levels.
+struct MaxPoolChain {
+    const uint8_t *in;
+    uint8_t *level[NNCASE_HIP_MAX_CONCAT - 1], *cat;
+    int levels, batch, h, w, channels, kernel;
+    nncase_hip_quant_param_t qp[NNCASE_HIP_MAX_CONCAT], cat_qp; // of the tensor and of every level
+};
+bool maxpool_chain_supported(const MaxPoolChain &c);
+int launch_maxpool_chain(nncase_hip_ctx *ctx, const MaxPoolChain &c);
+
 } // namespace nnhip

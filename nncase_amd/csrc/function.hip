@@ -134,6 +134,48 @@ static int run_op(nncase_hip_function *fn, const Op &op) {
     return -EINVAL;
 }
 
+// Max pools of stride 1, each over the last one's result, and the concat of their input and all of them, recorded one behind
+// the other from operator `at` on: one launch for them all (launch_maxpool_chain).  Returns how many operators that is, 0 if none.
+static size_t find_pool_chain(const std::vector<Op> &ops, size_t at, MaxPoolChain *c) {
+    auto same = [](nncase_hip_quant_param_t a, nncase_hip_quant_param_t b) { return a.zero_point == b.zero_point && a.scale == b.scale; };
+    const Op &head = ops[at];
+    if (head.kind != Op::kMaxPool) return 0;
+    const int k = head.pool[0];
+    c->in = (const uint8_t *)head.in0, c->batch = head.batch, c->h = head.h, c->w = head.w, c->channels = head.channels, c->kernel = k;
+    c->qp[0] = head.qp0, c->levels = 0;
+    const void *x = head.in0;
+    size_t i = at;
+    for (; i < ops.size() && ops[i].kind == Op::kMaxPool && c->levels < NNCASE_HIP_MAX_CONCAT - 1; i++) {
+        const Op &op = ops[i];
+        const int32_t window[8] = {k, k, 1, 1, k / 2, k / 2, k / 2, k / 2};
+        if (op.in0 != x || op.lane != head.lane || op.batch != c->batch || op.h != c->h || op.w != c->w || op.channels != c->channels ||
+            memcmp(op.pool, window, sizeof(window)) != 0 || !same(op.qp0, c->qp[c->levels]))
+            break;
+        if (op.out == c->in || std::find(c->level, c->level + c->levels, op.out) != c->level + c->levels) break;
+        c->level[c->levels++] = (uint8_t *)op.out;
+        c->qp[c->levels] = op.qp1;
+        x = op.out;
+    }
+    if (i == ops.size()) return 0;
+    const Op &cat = ops[i];
+    if (cat.kind != Op::kConcat || cat.lane != head.lane || cat.n_inputs != c->levels + 1 || cat.pixels != (int64_t)c->batch * c->h * c->w) return 0;
+    for (int l = 0; l <= c->levels; l++)
+        if (cat.cat_in[l] != (l == 0 ? c->in : c->level[l - 1]) || cat.cat_channels[l] != c->channels || !same(cat.cat_qp[l], c->qp[l])) return 0;
+    c->cat = (uint8_t *)cat.out, c->cat_qp = cat.qp0;
+    return maxpool_chain_supported(*c) ? i + 1 - at : 0;
+}
+
+// Runs the operators from `at` on that run as one launch; *next is the first behind them.
+static int run_ops(nncase_hip_function *fn, size_t at, size_t *next) {
+    MaxPoolChain chain;
+    if (const size_t n = find_pool_chain(fn->ops, at, &chain)) {
+        *next = at + n;
+        return launch_maxpool_chain(fn->ctx, chain);
+    }
+    *next = at + 1;
+    return run_op(fn, fn->ops[at]);
+}
+
 static void drop_graph(nncase_hip_function *fn) {
     if (fn->exec) (void)hipGraphExecDestroy(fn->exec);
     if (fn->graph) (void)hipGraphDestroy(fn->graph);
@@ -572,12 +614,14 @@ int nnhip::function_run_to_host(nncase_hip_function_t *fn, int n, void *const *o
     std::vector<Early> early;
     auto enqueue = [&]() -> int {
         const std::vector<Op> &ops = fn->ops;
-        for (size_t k = 0; !fn->exec && k < ops.size(); k++) {
-            if (int rc = run_op(fn, ops[k])) return rc;
-            if (k + 1 == ops.size()) break; // (the last operator's result is fetched in order)
+        for (size_t k = 0, next = 0; !fn->exec && next < ops.size();) {
+            const size_t first = next;
+            if (int rc = run_ops(fn, first, &next)) return rc;
+            k = next - 1;
+            if (next == ops.size()) break; // (the last operator's result is fetched in order)
             for (int i = 0; i < n; i++) {
                 auto writes = [&](const Op &op) { return op.out == outputs_dev[i] || op.out2 == outputs_dev[i]; };
-                if (!writes(ops[k]) || std::any_of(ops.begin() + k + 1, ops.end(), writes)) continue;
+                if (std::none_of(ops.begin() + first, ops.begin() + next, writes) || std::any_of(ops.begin() + k + 1, ops.end(), writes)) continue;
                 if (early.size() == nncase_hip_ctx::kCopySlots || !host_is_pinned(outputs_host[i])) continue;
                 const int slot = (int)early.size();
                 if (int rc = mark_result(ctx, slot)) return rc;
@@ -610,10 +654,8 @@ extern "C" int nncase_hip_function_invoke(nncase_hip_function_t *fn) {
         NNHIP_HIP(fn->ctx, hipGraphLaunch(fn->exec, fn->ctx->stream));
         return 0;
     }
-    for (const Op &op : fn->ops) {
-        const int rc = run_op(fn, op);
-        if (rc) return rc;
-    }
+    for (size_t k = 0; k < fn->ops.size();)
+        if (int rc = run_ops(fn, k, &k)) return rc;
     return 0;
 }
 
@@ -660,10 +702,14 @@ extern "C" int nncase_hip_function_capture(nncase_hip_function_t *fn) {
         for (int l = 1; l < fn->nlanes && se == hipSuccess; l++) se = hipStreamWaitEvent(side[l], fork, 0);
     }
     if (se == hipSuccess) {
-        for (const Op &op : fn->ops) {
-            if (op.lane == NNCASE_HIP_LANE_JOINED) continue;
-            ctx->stream = op.lane == 0 ? main_stream : side[op.lane];
-            rc = run_op(fn, op);
+        for (size_t k = 0; k < fn->ops.size();) {
+            const int lane = fn->ops[k].lane;
+            if (lane == NNCASE_HIP_LANE_JOINED) {
+                k++;
+                continue;
+            }
+            ctx->stream = lane == 0 ? main_stream : side[lane];
+            rc = run_ops(fn, k, &k);
             if (rc) break;
         }
         ctx->stream = main_stream;
@@ -672,9 +718,9 @@ extern "C" int nncase_hip_function_capture(nncase_hip_function_t *fn) {
             if (se == hipSuccess) se = hipStreamWaitEvent(main_stream, join[l], 0);
         }
         // what was recorded behind the join: on the context's stream, after every lane
-        for (const Op &op : fn->ops) {
-            if (rc || se != hipSuccess) break;
-            if (op.lane == NNCASE_HIP_LANE_JOINED) rc = run_op(fn, op);
+        for (size_t k = 0; k < fn->ops.size() && !rc && se == hipSuccess;) {
+            if (fn->ops[k].lane == NNCASE_HIP_LANE_JOINED) rc = run_ops(fn, k, &k);
+            else k++;
         }
     }
     hipGraph_t graph = nullptr;
@@ -717,7 +763,12 @@ extern "C" int nncase_hip_function_op_kernel(nncase_hip_function_t *fn, int32_t 
     case Op::kConcat: snprintf(name, capacity, "qconcat<%d>", op.n_inputs); break;
     case Op::kResize: snprintf(name, capacity, "resize_nearest"); break;
     case Op::kLayout: snprintf(name, capacity, op.mode ? "nhwc_to_nchw" : "nchw_to_nhwc"); break;
-    case Op::kMaxPool: snprintf(name, capacity, "qmaxpool<%dx%d>", op.pool[0], op.pool[1]); break;
+    case Op::kMaxPool: {
+        MaxPoolChain chain;
+        if (find_pool_chain(fn->ops, (size_t)index, &chain)) snprintf(name, capacity, "qmaxpool_chain<%dx%d,%d>", chain.kernel, chain.kernel, chain.levels);
+        else snprintf(name, capacity, "qmaxpool<%dx%d>", op.pool[0], op.pool[1]);
+        break;
+    }
     case Op::kPack: snprintf(name, capacity, "pack"); break;
     case Op::kQuantPack: snprintf(name, capacity, "quantize+pack"); break;
     case Op::kGemm:
@@ -743,11 +794,12 @@ extern "C" int nncase_hip_function_profile(nncase_hip_function_t *fn, int32_t it
     NNHIP_HIP(ctx, hipEventCreate(&e0));
     NNHIP_HIP(ctx, hipEventCreate(&e1));
     int rc = 0;
-    for (size_t i = 0; i < fn->ops.size() && rc == 0; i++) {
-        rc = run_op(fn, fn->ops[i]); // warm
+    std::fill(avg_ms, avg_ms + fn->ops.size(), 0.f);
+    for (size_t i = 0, next = 0; i < fn->ops.size() && rc == 0; i = next) { // (operators that run as one launch: the first has its time)
+        rc = run_ops(fn, i, &next); // warm
         if (rc) break;
         hipError_t e = hipEventRecord(e0, ctx->stream);
-        for (int it = 0; it < iterations && rc == 0; it++) rc = run_op(fn, fn->ops[i]);
+        for (int it = 0; it < iterations && rc == 0; it++) rc = run_ops(fn, i, &next);
         if (e == hipSuccess) e = hipEventRecord(e1, ctx->stream);
         if (e == hipSuccess) e = hipEventSynchronize(e1);
         float ms = 0.f;

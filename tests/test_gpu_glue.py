@@ -10,6 +10,8 @@ from nncase_amd import runtime as rt
 from nncase_amd.runtime import qp
 from oracle import oracle as O
 
+f32 = np.float32
+
 pytestmark = pytest.mark.gpu
 
 
@@ -147,3 +149,42 @@ def test_maxpool_sppf_shape(hip_ctx):
     xp = np.pad(np.maximum(x, 0), ((0, 0), (0, 0), (2, 2), (2, 2)), constant_values=zx)   # 0.0 is the code zx
     win = np.lib.stride_tricks.sliding_window_view(xp, (5, 5), axis=(2, 3)).max(axis=(-1, -2))
     assert np.array_equal(got, win)
+
+
+@pytest.mark.parametrize("n,h,w,c,k,levels,fused", [
+    (16, 20, 20, 256, 5, 3, True),      # 16 channels per block
+    (1, 7, 11, 32, 3, 1, True),         # 4 channels per block, one level
+    (2, 43, 44, 16, 5, 3, True),        # planes that nearly fill the LDS, several pixels per thread
+    (3, 2, 3, 48, 13, 7, True),         # windows wider than the image; as many levels as a concat takes
+    (1, 45, 45, 16, 5, 2, False),       # planes that do not fit
+    (1, 9, 9, 20, 5, 2, False)])        # channels that are no multiple of 16
+def test_max_pool_chain_behind_a_concat_runs_as_one_launch(hip_ctx, n, h, w, c, k, levels, fused):
+    """Pools of each other's results and the concat of all of them, recorded in a function: every tensor and the concat equal the
+    operators one by one, with equal quant params and with a requantisation at every step, eagerly and as a graph."""
+    rng = np.random.default_rng(h * w + c)
+    x = rng.integers(0, 256, (n, h, w, c), dtype=np.uint8)
+    for qps, qcat in (([(90, 0.05)] * (levels + 1), (90, 0.05)),
+                      ([(int(rng.integers(0, 256)), f32(0.03 + 0.004 * i)) for i in range(levels + 1)], (60, f32(0.05)))):
+        parts = [np.ascontiguousarray(x.transpose(0, 3, 1, 2))]
+        for a, b in zip(qps, qps[1:]):
+            parts.append(O.qmaxpool(parts[-1], (k, k), (1, 1), ((k // 2, k // 2), (k // 2, k // 2)), a[0], a[1], b[0], b[1]))
+        want = O.qconcat(parts, qps, qcat).transpose(0, 2, 3, 1)
+        bufs = [hip_ctx.to_device(x)] + [hip_ctx.alloc(x.size) for _ in range(levels)]
+        out = hip_ctx.alloc(want.size)
+        fn = rt.Function(hip_ctx)
+        for i in range(levels):
+            fn.add_qmaxpool2d(bufs[i], bufs[i + 1], n, h, w, c, (k, k), (1, 1), ((k // 2, k // 2), (k // 2, k // 2)), qp(*qps[i]), qp(*qps[i + 1]))
+        fn.add_qconcat_channels(bufs, [c] * (levels + 1), [qp(*q) for q in qps], out, qp(*qcat), n * h * w)
+        assert fn.op_kernel(0).startswith("qmaxpool_chain") == fused
+        for capture in (False, True):
+            if capture:
+                fn.capture()
+            for b in bufs[1:] + [out]:
+                b.fill(0)
+            fn.invoke()
+            hip_ctx.sync()
+            for b, part in zip(bufs, parts):
+                assert np.array_equal(b.download(x.shape, np.uint8), part.transpose(0, 2, 3, 1))
+            assert np.array_equal(out.download(want.shape, np.uint8), want)
+        assert len(fn.profile(1)) == levels + 1
+        fn.destroy()
