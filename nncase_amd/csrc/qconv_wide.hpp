@@ -1090,8 +1090,13 @@ template <int T, int WM, int WN, int LM> int launch_wide_small_t(nncase_hip_ctx 
 
 // Block shapes: tiles = 16 -> 256 pixels x 256 channels (4 x 2 waves); tiles = 8 -> 256 or 128 pixels x 128 channels.
 template <int LM> int launch_wide_lm(nncase_hip_ctx *ctx, const IgemmArgs &a, int tiles, int nchunks) {
-    if constexpr (LM == kWideRagRows || LM == kWideRagWindow) {
-        if (tiles == 16) return fail(ctx, -EINVAL, "qconv2d: no 256-channel blocks for ragged rows");
+    if constexpr (LM == kWideRagRows) {
+        // (planned for rows of whole dwords: a piece then starts at a dword, wherever its 16 bytes lie; what runs over the end of a
+        // row meets surplus weights and is in the sums of x as well)
+        if (tiles == 16)
+            return a.k % 64 == 0 ? launch_wide_dma_t<8, 4, 4, 2, kWideRowsFull>(ctx, a, nchunks) : launch_wide_dma_t<8, 4, 4, 2, kWideRows>(ctx, a, nchunks);
+    } else if constexpr (LM == kWideRagWindow) {
+        if (tiles == 16) return launch_wide_t<8, 4, 4, 2, LM>(ctx, a, nchunks);
     } else if (tiles == 16) {
         if constexpr (LM == kWideRowsFull || LM == kWideRows) {
             if (a.x_bytes < ((size_t)1 << 31)) return launch_wide_dma_t<8, 4, 4, 2, LM>(ctx, a, nchunks);

@@ -798,3 +798,19 @@ def test_convolution_over_an_input_tile_in_lds(hip_ctx, n, cin, cout, hw, k, str
     got = y.download(want.shape, np.uint8)
     assert np.array_equal(got, want), f"{name}: {(got != want).sum()} of {want.size} bytes differ"
     assert name.startswith("qconv_tile") and name.endswith(f"<{block}>"), name
+
+
+@pytest.mark.parametrize("m,k,n", [(16500, 516, 300), (16641, 1020, 258), (33000, 532, 257)])
+def test_matmul_of_rows_of_whole_dwords_in_256_channel_blocks(hip_ctx, m, k, n):
+    """Rows that are no multiple of 16 bytes, moved straight to LDS in 256 x 256 blocks: last k-steps that end inside a piece, partial
+    blocks both ways, the last row at the end of the tensor; and the same weights behind a strided window."""
+    rng = np.random.default_rng(m + k + n)
+    a, b = rng.integers(0, 256, (m, k), dtype=np.uint8), rng.integers(0, 256, (k, n), dtype=np.uint8)
+    want = ((a.astype(np.float64) - 7) @ (b.astype(np.float64) - 131)).astype(np.int32)     # exact: below 2^53
+    assert np.array_equal(K.mat_mul(a, b, qp(7, 0.02), qp(131, 0.004), None, np.int32, None, ctx=hip_ctx), want)
+    if m == 16641:
+        x = np.zeros((1, k, 257, 257), np.uint8)
+        x[0, :, ::2, ::2] = a.T.reshape(k, 129, 129)
+        got = K.conv2d(x, np.ascontiguousarray(b.T)[:, :, None, None], None, (2, 2), ((0, 0), (0, 0)), (1, 1), 1, FULL, qp(7, 0.02), qp(131, 0.004),
+                       None, np.int32, ctx=hip_ctx)
+        assert np.array_equal(got[0].reshape(n, m).T, want)
