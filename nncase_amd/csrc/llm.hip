@@ -17,6 +17,7 @@
 
 #include <cmath>
 #include <mutex>
+#include <type_traits>
 #include <new>
 #include <vector>
 
@@ -85,10 +86,27 @@ __device__ __forceinline__ void add_squares8(const lu32x4 &v, float &ss) {
         ss += f * f;
     }
 }
+// The sum over the wave's lanes, in every lane, bit for bit the butterfly `for (o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o)`
+// (a sum of two does not mind their order) on row swaps and DPP moves: a shuffle goes through the LDS crossbar and back, six of
+// them in a row a quarter of a microsecond in front of every product that normalises its rows.
+template <int CTRL> __device__ __forceinline__ float dpp_move(float v) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xf, 0xf, true));
+}
+__device__ __forceinline__ float wave_sum(float v) {
+    // (the builtin of the swaps takes two equal operands for two equal results; the wait states are those it would insert)
+    float other = v;
+    asm("s_nop 1\n\tv_permlane32_swap_b32 %0, %1" : "+v"(v), "+v"(other)); // lanes 0..31 twice, lanes 32..63 twice
+    v += other;
+    other = v;
+    asm("s_nop 1\n\tv_permlane16_swap_b32 %0, %1" : "+v"(v), "+v"(other)); // the even rows of 16 twice, the odd ones twice
+    v += other;
+    v += dpp_move<0x128>(v); // row_ror:8
+    v += dpp_move<0x124>(v); // row_ror:4 (the lanes of a row repeat with period 8 by now)
+    v += dpp_move<0x4e>(v);  // quad_perm 2 3 0 1
+    return v + dpp_move<0xb1>(v); // quad_perm 1 0 3 2
+}
 __device__ __forceinline__ float rstd_from_sum(float ss, int hidden, float eps) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) ss += __shfl_xor(ss, o);
-    return 1.0f / sqrtf(ss / (float)hidden + eps);
+    return 1.0f / sqrtf(wave_sum(ss) / (float)hidden + eps);
 }
 // R rows at once (row r0 + i * stride for i < R, those below `rows`): the loads of one piece of all of them are in
 // flight together.  hidden is a multiple of 8 and the rows are 16-byte aligned.
@@ -392,7 +410,9 @@ inline int rows_in_lds_pitch(int k) { return k * 2 + 16; } // bytes per token ro
 // rotate-half pairs -- tile j of a head and tile j + up_tile_offset (= head_dim / 32) -- so that a lane ends up with
 // both elements of its four pairs; the epilogue rounds them to fp16 as the projection's output would be stored and
 // rotates and stores them (rope_pair, rope_store).
-template <int MT, int G, int WAVES, bool SPLIT = false, int KB = kRowsBatch, int PIECES = kRowsPieces, bool ROPE = false>
+// FEW: no more rows than waves.  A wave then has one row at most, and none where it lies past m: what LDS holds in their place
+// meets no row that is stored.  (One row, 24 layers: q / k / v 5.9 -> 4.9 us, gate / up 7.8 -> 5.8.)
+template <int MT, int G, int WAVES, bool SPLIT = false, int KB = kRowsBatch, int PIECES = kRowsPieces, bool ROPE = false, bool FEW = false>
 __global__ __launch_bounds__(WAVES * 64) void w8a16_gemm_rows_in_lds_kernel(const GemmArgs a) {
     static_assert(!ROPE || (SPLIT && G == 2), "the rotating epilogue pairs two tiles of one block");
     extern __shared__ __attribute__((aligned(16))) uint8_t xs[]; // [MT * 16][k halves + padding]
@@ -430,7 +450,7 @@ __global__ __launch_bounds__(WAVES * 64) void w8a16_gemm_rows_in_lds_kernel(cons
     request_first();
     RopePair rope;
     {
-        constexpr int R = MT * 16 / WAVES; // rows per wave
+        constexpr int R = FEW ? 1 : MT * 16 / WAVES; // rows per wave
         // The wave's rows stay in registers from the load to the one LDS write: their sums of squares, the butterflies
         // and the normalisation run for all R rows side by side (independent chains), element by element in the order
         // rms_rstd_rows and rmsnorm_f16_kernel use.
@@ -457,7 +477,7 @@ __global__ __launch_bounds__(WAVES * 64) void w8a16_gemm_rows_in_lds_kernel(cons
             }
             __builtin_amdgcn_sched_barrier(0);
         }
-        if (a.ln_w) {
+        if (a.ln_w && (!FEW || wave < a.m)) {
             float ss[R];
 #pragma unroll
             for (int i = 0; i < R; i++) ss[i] = 0.f;
@@ -466,9 +486,7 @@ __global__ __launch_bounds__(WAVES * 64) void w8a16_gemm_rows_in_lds_kernel(cons
 #pragma unroll
                 for (int i = 0; i < R; i++) add_squares8(v[i][p], ss[i]); // (pieces past the row are zeros: +0 leaves a sum as it is)
 #pragma unroll
-            for (int o = 32; o > 0; o >>= 1)
-#pragma unroll
-                for (int i = 0; i < R; i++) ss[i] += __shfl_xor(ss[i], o);
+            for (int i = 0; i < R; i++) ss[i] = wave_sum(ss[i]);
             float rr[R];
 #pragma unroll
             for (int i = 0; i < R; i++) rr[i] = 1.0f / sqrtf(ss[i] / (float)a.k + a.ln_eps); // rstd_from_sum's formula
@@ -495,7 +513,7 @@ __global__ __launch_bounds__(WAVES * 64) void w8a16_gemm_rows_in_lds_kernel(cons
 #pragma unroll
         for (int p = 0; p < PIECES; p++) {
             const int e0 = lane * 8 + p * 512;
-            if (e0 < a.k) {
+            if (e0 < a.k && (!FEW || wave < a.m)) {
 #pragma unroll
                 for (int i = 0; i < R; i++) *reinterpret_cast<lu32x4 *>(xs + (size_t)(wave + i * WAVES) * pitch + e0 * 2) = v[i][p];
             }
@@ -849,16 +867,18 @@ static int launch_w8a16_gemm(nncase_hip_ctx_t *ctx, const void *a_dev, const nnc
         a.up_tile_offset = rope->d / 32;
         const dim3 pgrid(w->ntiles / 2), pblock(kGemmThreads);
         const bool two_pieces = w->k <= 1024;
-#define NNHIP_ROPE_LAUNCH(MTV, PV)                                                                                             \
+#define NNHIP_ROPE_LAUNCH(MTV, PV, FEWV)                                                                                             \
     do {                                                                                                                       \
-        NNHIP_HIP(ctx, raise_dynamic_lds(w8a16_gemm_rows_in_lds_kernel<MTV, 2, kGemmWaves, true, 2, PV, true>, ctx->device,   \
+        NNHIP_HIP(ctx, raise_dynamic_lds(w8a16_gemm_rows_in_lds_kernel<MTV, 2, kGemmWaves, true, 2, PV, true, FEWV>, ctx->device,   \
                                          rows_lds + MTV * 16 * 1024, 96 * 1024));                                              \
-        hipLaunchKernelGGL((w8a16_gemm_rows_in_lds_kernel<MTV, 2, kGemmWaves, true, 2, PV, true>), pgrid, pblock, rows_lds, ctx->stream, a); \
+        hipLaunchKernelGGL((w8a16_gemm_rows_in_lds_kernel<MTV, 2, kGemmWaves, true, 2, PV, true, FEWV>), pgrid, pblock, rows_lds, ctx->stream, a); \
     } while (0)
-        if (mt_built == 1 && two_pieces) NNHIP_ROPE_LAUNCH(1, 2);
-        else if (mt_built == 1) NNHIP_ROPE_LAUNCH(1, kRowsPieces);
-        else if (two_pieces) NNHIP_ROPE_LAUNCH(2, 2);
-        else NNHIP_ROPE_LAUNCH(2, kRowsPieces);
+        if (m <= kGemmWaves && two_pieces) NNHIP_ROPE_LAUNCH(1, 2, true);
+        else if (m <= kGemmWaves) NNHIP_ROPE_LAUNCH(1, kRowsPieces, true);
+        else if (mt_built == 1 && two_pieces) NNHIP_ROPE_LAUNCH(1, 2, false);
+        else if (mt_built == 1) NNHIP_ROPE_LAUNCH(1, kRowsPieces, false);
+        else if (two_pieces) NNHIP_ROPE_LAUNCH(2, 2, false);
+        else NNHIP_ROPE_LAUNCH(2, kRowsPieces, false);
 #undef NNHIP_ROPE_LAUNCH
         NNHIP_LAUNCH_CHECK(ctx, "w8a16_gemm_rows_in_lds_kernel");
         return 0;
@@ -870,18 +890,21 @@ static int launch_w8a16_gemm(nncase_hip_ctx_t *ctx, const void *a_dev, const nnc
         // pair, its waves splitting the reduction, so that every compute unit takes part.  Four waves for 32 rows (eight
         // took 12.8 against 10.7 us); eight for 16 rows, where a wave then brings in and normalises two rows instead of
         // four (the decode step of two lanes: 1.097 against 1.114 ms)
-#define NNHIP_GLU_SPLIT_LAUNCH(MTV, PV, GWV, KBV)                                                                              \
+#define NNHIP_GLU_SPLIT_LAUNCH(MTV, PV, GWV, KBV, FEWV)                                                                              \
     do {                                                                                                                       \
-        NNHIP_HIP(ctx, raise_dynamic_lds(w8a16_gemm_rows_in_lds_kernel<MTV, 2, GWV, true, KBV, PV>, ctx->device,              \
+        NNHIP_HIP(ctx, raise_dynamic_lds(w8a16_gemm_rows_in_lds_kernel<MTV, 2, GWV, true, KBV, PV, false, FEWV>, ctx->device,              \
                                          rows_lds + GWV * 2 * MTV * 1024, 96 * 1024));                                         \
-        hipLaunchKernelGGL((w8a16_gemm_rows_in_lds_kernel<MTV, 2, GWV, true, KBV, PV>), grid, dim3(GWV * 64), rows_lds, ctx->stream, a); \
+        hipLaunchKernelGGL((w8a16_gemm_rows_in_lds_kernel<MTV, 2, GWV, true, KBV, PV, false, FEWV>), grid, dim3(GWV * 64), rows_lds, ctx->stream, a); \
     } while (0)
         const bool two_steps = (w->ksteps + 7) / 8 <= 2; // a wave's share of the reduction with eight waves
-        if (mt_built == 1 && short_rows && two_steps) NNHIP_GLU_SPLIT_LAUNCH(1, 2, 8, 2);
-        else if (mt_built == 1 && short_rows) NNHIP_GLU_SPLIT_LAUNCH(1, 2, 8, 4);
-        else if (mt_built == 1) NNHIP_GLU_SPLIT_LAUNCH(1, kRowsPieces, 8, 4);
-        else if (short_rows) NNHIP_GLU_SPLIT_LAUNCH(2, 2, kGluSplitWaves, 4);
-        else NNHIP_GLU_SPLIT_LAUNCH(2, kRowsPieces, kGluSplitWaves, 4);
+        if (m <= 8 && short_rows && two_steps) NNHIP_GLU_SPLIT_LAUNCH(1, 2, 8, 2, true);
+        else if (m <= 8 && short_rows) NNHIP_GLU_SPLIT_LAUNCH(1, 2, 8, 4, true);
+        else if (m <= 8) NNHIP_GLU_SPLIT_LAUNCH(1, kRowsPieces, 8, 4, true);
+        else if (mt_built == 1 && short_rows && two_steps) NNHIP_GLU_SPLIT_LAUNCH(1, 2, 8, 2, false);
+        else if (mt_built == 1 && short_rows) NNHIP_GLU_SPLIT_LAUNCH(1, 2, 8, 4, false);
+        else if (mt_built == 1) NNHIP_GLU_SPLIT_LAUNCH(1, kRowsPieces, 8, 4, false);
+        else if (short_rows) NNHIP_GLU_SPLIT_LAUNCH(2, 2, kGluSplitWaves, 4, false);
+        else NNHIP_GLU_SPLIT_LAUNCH(2, kRowsPieces, kGluSplitWaves, 4, false);
 #undef NNHIP_GLU_SPLIT_LAUNCH
         NNHIP_LAUNCH_CHECK(ctx, "w8a16_gemm_rows_in_lds_kernel");
         return 0;
@@ -892,16 +915,18 @@ static int launch_w8a16_gemm(nncase_hip_ctx_t *ctx, const void *a_dev, const nnc
         // (the kernel's static reduction area comes on top of the rows: past 48 KiB in all, the limit is raised like below)
         // (a wave's share of the reduction is requested at once where it is at most two k-steps, the decode step's case)
         const bool short_share = (w->ksteps + kGemmWaves - 1) / kGemmWaves <= 2;
-#define NNHIP_SPLIT_ROWS_LAUNCH_P(MTV, KBV, PV)                                                                                \
+#define NNHIP_SPLIT_ROWS_LAUNCH_P(MTV, KBV, PV, FEWV)                                                                                \
     do {                                                                                                                       \
-        NNHIP_HIP(ctx, raise_dynamic_lds(w8a16_gemm_rows_in_lds_kernel<MTV, 1, kGemmWaves, true, KBV, PV>, ctx->device,       \
+        NNHIP_HIP(ctx, raise_dynamic_lds(w8a16_gemm_rows_in_lds_kernel<MTV, 1, kGemmWaves, true, KBV, PV, false, FEWV>, ctx->device,       \
                                          rows_lds + MTV * 8 * 1024, 64 * 1024));                                               \
-        hipLaunchKernelGGL((w8a16_gemm_rows_in_lds_kernel<MTV, 1, kGemmWaves, true, KBV, PV>), grid, block, rows_lds, ctx->stream, a); \
+        hipLaunchKernelGGL((w8a16_gemm_rows_in_lds_kernel<MTV, 1, kGemmWaves, true, KBV, PV, false, FEWV>), grid, block, rows_lds, ctx->stream, a); \
     } while (0)
 #define NNHIP_SPLIT_ROWS_LAUNCH(MTV, KBV)                                                                                      \
     do {                                                                                                                       \
-        if (short_rows) NNHIP_SPLIT_ROWS_LAUNCH_P(MTV, KBV, 2);                                                                \
-        else NNHIP_SPLIT_ROWS_LAUNCH_P(MTV, KBV, kRowsPieces);                                                                 \
+        if (m <= kGemmWaves && short_rows) NNHIP_SPLIT_ROWS_LAUNCH_P(1, KBV, 2, true);                                        \
+        else if (m <= kGemmWaves) NNHIP_SPLIT_ROWS_LAUNCH_P(1, KBV, kRowsPieces, true);                                       \
+        else if (short_rows) NNHIP_SPLIT_ROWS_LAUNCH_P(MTV, KBV, 2, false);                                                   \
+        else NNHIP_SPLIT_ROWS_LAUNCH_P(MTV, KBV, kRowsPieces, false);                                                                 \
     } while (0)
         if (mt_built == 1) {
             if (short_share) NNHIP_SPLIT_ROWS_LAUNCH(1, 2);

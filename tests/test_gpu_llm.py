@@ -351,3 +351,15 @@ def test_decode_step_at_the_benchmark_shape(hip_ctx, lanes):
             bound = max(1e-3 * max(1.0, float(np.abs(ref).max())) + 4e-3, 1.5 * float(np.abs(other - ref).max()))
             print(f"layer {li} {name} cache: largest difference {d.max():.2e}, float32-sum evaluation {np.abs(other - ref).max():.2e}, bound {bound:.2e}")
             assert d.max() <= bound, f"layer {li} {name} cache differs by {d.max():.3e} (bound {bound:.3e})"
+
+
+@pytest.mark.parametrize("m,k,n,mode", [(1, 896, 9728, "swiglu"), (8, 896, 9728, "swiglu"), (9, 896, 9728, "swiglu"), (8, 1024, 1152, "plain"),
+                                        (3, 2048, 1152, "plain"), (5, 1536, 4096, "swiglu"), (8, 960, 4096, "residual")])
+def test_few_rows_one_per_wave(hip_ctx, m, k, n, mode):
+    """Up to eight rows a wave normalises one at most (nine: two, as before): one and two request batches, two and four row pieces."""
+    test_rmsnorm_fused_into_gemm_equals_the_two_operators(hip_ctx, m, k, n, mode)
+
+
+@pytest.mark.parametrize("B,k,norm", [(1, 896, True), (8, 896, True), (9, 896, True), (8, 1024, False)])
+def test_few_rows_one_per_wave_that_rotate(hip_ctx, B, k, norm):
+    test_projection_that_rotates_and_appends_equals_the_two_operators(hip_ctx, B, k, norm)
