@@ -354,7 +354,8 @@ __device__ __forceinline__ void store_dword_group(const IgemmArgs &a, const uint
 // STAGED: the kernel has a staging area per wave for the dword outputs (store_dword_group); the lane-by-lane dword
 // stores are then not built.
 // MAGIC (with PLAIN): the accumulators were started from kMagicBias and are requantised as floats (Epilogue::magic).
-template <int T, int OWED = kOwesAll, bool PLAIN = false, bool STAGED = false, bool MAGIC = false>
+// TABLE (with PLAIN): there is a byte table, at lutl.
+template <int T, int OWED = kOwesAll, bool PLAIN = false, bool STAGED = false, bool MAGIC = false, bool TABLE = false>
 __device__ __forceinline__ void igemm_store_tile(const IgemmArgs &a, const v4i (&acc)[T], int32_t rowsum, int p, int ch0, int gq,
                                                  const int32_t *cterm, const uint8_t *lutl, uint8_t *stage = nullptr,
                                                  int quarter_stride = 4 * T) {
@@ -378,6 +379,15 @@ __device__ __forceinline__ void igemm_store_tile(const IgemmArgs &a, const v4i (
             for (int r = 0; r < 4; r++)
                 v[r] = OWED == kOwesAll ? add3(acc[nt][r], ct[r], nrsz) : (OWED == kOwesRows ? acc[nt][r] + nrsz : acc[nt][r]);
             packed[nt] = MAGIC ? requant4_u8_packed_magic(v, a.ep) : requant4_u8_packed_direct(v, a.ep);
+        }
+        if constexpr (TABLE) { // (every byte is asked for before the first is used)
+            uint32_t b[T][4];
+#pragma unroll
+            for (int nt = 0; nt < T; nt++)
+#pragma unroll
+                for (int r = 0; r < 4; r++) b[nt][r] = lutl[(packed[nt] >> (8 * r)) & 0xffu];
+#pragma unroll
+            for (int nt = 0; nt < T; nt++) packed[nt] = b[nt][0] | (b[nt][1] << 8) | (b[nt][2] << 16) | (b[nt][3] << 24);
         }
 #pragma unroll
         for (int nt = 0; nt + 4 <= T; nt += 4)
@@ -727,10 +737,13 @@ __global__ void __launch_bounds__(kThreads, (STAGED && T >= 12) ? 2 : (((RG == 1
 // of the products.  ROWS: the epilogue still owes -zw' * (sum of x'); false where the weights carry that term
 // (reductions of at most 32: the lanes of the upper half of the only k-step then re-read the pixel's bytes).
 // MAGIC: the sums start from kMagicBias on top of the channel constants and the epilogue reads them as floats.
-template <int T, int RG, bool ROWS, bool MAGIC> __global__ void __launch_bounds__(kThreads, 4) qconv_rows_kernel(const IgemmArgs a) {
+// TABLE: a byte table behind the requantisation.  (Such layers went through qconv_igemm_kernel, 10.8 vector instructions per
+// output: 409 600 pixels 64 -> 64 14.6 -> 13.4 us, 64 -> 32 10.9 -> 9.1, 25 600 pixels 128 -> 128 5.6 -> 4.7.)
+template <int T, int RG, bool ROWS, bool MAGIC, bool TABLE = false> __global__ void __launch_bounds__(kThreads, 4) qconv_rows_kernel(const IgemmArgs a) {
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
     int32_t *cterm = reinterpret_cast<int32_t *>(smem); // [T * 16]
-    uint8_t *wlds = smem + T * 16 * sizeof(int32_t);    // [ksteps][T][1024]
+    uint8_t *lutl = smem + T * 16 * sizeof(int32_t);    // [256] (TABLE)
+    uint8_t *wlds = lutl + (TABLE ? 256 : 0);           // [ksteps][T][1024]
 
     const int lane = threadIdx.x & 63;
     const int wave = threadIdx.x >> 6;
@@ -740,6 +753,7 @@ template <int T, int RG, bool ROWS, bool MAGIC> __global__ void __launch_bounds_
     const int KS = a.ksteps;
     const __amdgpu_buffer_rsrc_t xres = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t *>(a.x), 0, (int)a.x_bytes, 0x00020000);
 
+    if (TABLE && threadIdx.x < 64) reinterpret_cast<uint32_t *>(lutl)[threadIdx.x] = a.lut[threadIdx.x];
     // constants and the chunk's weights -> LDS
     static_assert(T * 16 <= kThreads, "one constant per thread");
     if ((int)threadIdx.x < T * 16) {
@@ -845,8 +859,8 @@ template <int T, int RG, bool ROWS, bool MAGIC> __global__ void __launch_bounds_
         }
 #pragma unroll
         for (int rg = 0; rg < RG; rg++)
-            igemm_store_tile<T, ROWS ? kOwesRows : kOwesNothing, true, false, MAGIC>(a, acc[rg], ROWS ? rs[rg][0] : 0,
-                                                                        mt * pix_per_block + (wave * RG + rg) * 16 + j, ch0, gq, cterm, nullptr);
+            igemm_store_tile<T, ROWS ? kOwesRows : kOwesNothing, true, false, MAGIC, TABLE>(a, acc[rg], ROWS ? rs[rg][0] : 0,
+                                                                        mt * pix_per_block + (wave * RG + rg) * 16 + j, ch0, gq, cterm, lutl);
 #pragma unroll
         for (int rg = 0; rg < RG; rg++) poff[rg] = poff_next[rg];
     }
@@ -1059,7 +1073,19 @@ template <int T, int RG, int MODE> int launch_trg(nncase_hip_ctx *ctx, const Ige
     // the 1x1 row loaders are also built without the epilogue's options (see igemm_store_tile)
     bool plain = false;
     if constexpr (loads_rows(MODE) || MODE == kVec16)
-        plain = a.ep.out_mode == kOutU8 && !a.deq && a.ep.fast && a.ep.full && !a.lut && !a.rep.res && a.n % (4 * T) == 0 && ((a.ldy | a.y_coff) & 3) == 0;
+        plain = a.ep.out_mode == kOutU8 && !a.deq && a.ep.fast && a.ep.full && !a.rep.res && a.n % (4 * T) == 0 && ((a.ldy | a.y_coff) & 3) == 0;
+    if (plain && a.lut) {
+        plain = false;
+        if constexpr (MODE == kRows16 && T <= 8) {
+            if (a.kc_steps >= a.ksteps) {
+                const size_t lds_rows = (size_t)T * 16 * sizeof(int32_t) + 256 + (size_t)a.ksteps * T * 1024;
+                if (a.magic_ok) hipLaunchKernelGGL((qconv_rows_kernel<T, RG, true, true, true>), dim3(gx, nchunks, 1), dim3(kThreads), lds_rows, ctx->stream, args);
+                else hipLaunchKernelGGL((qconv_rows_kernel<T, RG, true, false, true>), dim3(gx, nchunks, 1), dim3(kThreads), lds_rows, ctx->stream, args);
+                NNHIP_LAUNCH_CHECK(ctx, "qconv_rows_kernel");
+                return 0;
+            }
+        }
+    }
     if constexpr (MODE == kVec16 && T <= 6) {
         // the whole chunk's weights resident and no folded reduction: the kernel with the tap table
         const size_t lds_win = (size_t)T * 16 * sizeof(int32_t) + 256 + (size_t)a.ksteps * 4 * sizeof(v4i) + (size_t)a.ksteps * T * 1024;

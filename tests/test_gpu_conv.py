@@ -814,3 +814,9 @@ def test_matmul_of_rows_of_whole_dwords_in_256_channel_blocks(hip_ctx, m, k, n):
         got = K.conv2d(x, np.ascontiguousarray(b.T)[:, :, None, None], None, (2, 2), ((0, 0), (0, 0)), (1, 1), 1, FULL, qp(7, 0.02), qp(131, 0.004),
                        None, np.int32, ctx=hip_ctx)
         assert np.array_equal(got[0].reshape(n, m).T, want)
+
+
+@pytest.mark.parametrize("cin,cout,hw", [(64, 64, 130), (32, 32, 41), (16, 48, 23), (128, 128, 60), (48, 16, 17), (192, 128, 20)])
+def test_pointwise_layers_with_a_table_on_the_lean_kernel(hip_ctx, cin, cout, hw):
+    """Whole chunks of channels behind a byte table: folded and unfolded reductions, partial pixel tiles, one to eight channel tiles."""
+    test_fused_table_equals_conv_then_table(hip_ctx, cin, cout, hw, 1, False)
