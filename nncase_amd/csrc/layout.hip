@@ -8,6 +8,7 @@
 // 4-byte group of elements where the two innermost dimensions coincide -- so
 // that writes are coalesced; 4-byte transposes go through a 32 x 33 LDS tile.
 #include "common.hpp"
+#include "layout_rules.hpp"
 
 #include <algorithm>
 #include <type_traits>
@@ -387,19 +388,31 @@ template <int E, bool PACK, bool RAGGED = false> __global__ __launch_bounds__(kL
 
 // Elements of X per tile: about 16 KiB per tile, rows of the plain tensor of 64 bytes to 2 KiB.
 // The extent is then split evenly over its tiles (3136 = 7 x 448 rather than 6 x 512 + 64).
-static uint32_t tile_stretch(uint32_t la, int es, uint32_t x_extent, bool wide) {
+static uint32_t tile_stretch(uint32_t la, int es, uint32_t x_extent, bool wide, uint32_t tile_bytes = 16384) {
     const uint32_t e = (wide ? 16 : 4) / es; // tiles begin at whole dwords (16-byte pieces) of a row
-    uint32_t tx = 16384 / (la * es);
+    uint32_t tx = tile_bytes / (la * es);
     tx = std::min<uint32_t>(std::max<uint32_t>(tx, 64 / es), 2048 / es) / e * e;
     const uint32_t tiles = (x_extent + tx - 1) / tx;
     return ((x_extent + tiles - 1) / tiles + e - 1) / e * e;
+}
+// The same for ragged rows, `others` tiles side by side in the other dimensions: a block takes a load, a barrier and a store in
+// turn and has nothing to hide them behind but its neighbours, so the tiles shrink to 8 and 4 KiB while the launch has fewer than
+// two blocks per compute unit (u8 NCHW -> NC/32 HW 32, tiles of 16 / 8 / 4 KiB: 155 x 75 x 75 5.8 / 4.8 / 4.3 us, 8 x 3 x 151 x 151
+// 6.1 / 5.5 / 6.3, 16 x 3 x 201 x 201 10.3 / 11.1 / 14.0).
+static uint32_t ragged_stretch(uint32_t la, int es, uint32_t x_extent, bool wide, uint64_t others, int compute_units) {
+    uint32_t tx = 0;
+    for (uint32_t bytes = 16384; bytes >= 4096; bytes /= 2) {
+        tx = tile_stretch(la, es, x_extent, wide, bytes);
+        if ((uint64_t)((x_extent + tx - 1) / tx) * others >= 2ull * compute_units) break;
+    }
+    return tx;
 }
 // Dwords per LDS row: odd, so that the E rows a lane reads and the rows of neighbouring lanes spread over the banks.
 static uint32_t tile_pitch(uint32_t cols) { return cols | 1u; }
 // Fills the tile description for pack (plain -> packed) or unpack of `shape` by (axes, lanes); false when the layout is
 // not one the tile kernel moves (then the element-wise kernels do).
 static bool make_tile_desc(TileDesc &d, int es, int rank, const int32_t *shape, int n_axes, const int *nax, const int32_t *lanes, bool pack,
-                           const void *in, const void *out, uint64_t &blocks, size_t &lds) {
+                           const void *in, const void *out, int compute_units, uint64_t &blocks, size_t &lds) {
     if (n_axes < 1 || (es != 1 && es != 2 && es != 4)) return false;
     const int e = 4 / es;
     if (((reinterpret_cast<uintptr_t>(in) | reinterpret_cast<uintptr_t>(out)) & 3u) != 0) return false;
@@ -436,17 +449,21 @@ static bool make_tile_desc(TileDesc &d, int es, int rank, const int32_t *shape, 
     }
     if (a >= xs) return false;
     // (the packed tensor's runs are whole dwords, la being a multiple of e: only the plain tensor's rows can be ragged)
-    d.ragged = ((uint64_t)d.x_extent * es) % (pack ? 16 : 4) != 0; // (packing reads them in 16-byte pieces, unpacking writes them in dwords)
-    d.in_bytes = (pack ? sp[0] * (uint64_t)shape[0] : st) * es;
+    const uint64_t row_bytes = (uint64_t)d.x_extent * es, plain_bytes = sp[0] * (uint64_t)shape[0] * es;
+    if (row_bytes % 4 != 0) {
+        d.ragged = 1;
+        if (!ragged_tile_pays(es, la, plain_bytes / es, st, pack, compute_units)) return false;
+    } else {
+        d.ragged = pack && row_bytes % 16 != 0 && unaligned_pieces_pay(la, row_bytes, plain_bytes);
+    }
+    d.in_bytes = pack ? plain_bytes : st * es;
     if (d.in_bytes < 4) return false;
     if (!pack) d.x_padded = d.x_extent;
     if (pack) d.wide = d.ragged ? (uint64_t)d.x_extent * es >= 64 : ((uint64_t)d.x_extent * es) % 16 == 0 && (reinterpret_cast<uintptr_t>(in) & 15u) == 0;
     else d.wide = (la * es) % 16 == 0 && (lp_all * es) % 16 == 0 && (reinterpret_cast<uintptr_t>(in) & 15u) == 0;
-    d.tx = tile_stretch(la, es, d.x_padded, d.wide);
-    d.x_tiles = (d.x_padded + d.tx - 1) / d.tx;
     d.la = la, d.a_extent = (uint32_t)shape[a], d.a_groups = O[a];
     d.a_plain_stride = sp[a], d.a_packed_group = sqo[a];
-    blocks = (uint64_t)d.x_tiles * d.a_groups;
+    blocks = d.a_groups;
     for (int i = 0; i < xs; i++) {
         if (i == a) continue;
         const int k = d.nrest++;
@@ -456,6 +473,9 @@ static bool make_tile_desc(TileDesc &d, int es, int rank, const int32_t *shape, 
         d.r_packed[k] = L[i] == 1 ? TwoTerm{1, sqo[i], 0} : TwoTerm{L[i], sqo[i], sql[jpos[i]]};
         blocks *= d.r_extent[k];
     }
+    d.tx = d.ragged ? ragged_stretch(la, es, d.x_padded, d.wide, blocks, compute_units) : tile_stretch(la, es, d.x_padded, d.wide);
+    d.x_tiles = (d.x_padded + d.tx - 1) / d.tx;
+    blocks *= d.x_tiles;
     if (blocks == 0 || blocks >= ((uint64_t)1 << 31)) return false;
     const uint32_t rows = pack ? la : d.tx, cols = (pack ? d.tx : la) / e;
     d.pitch = tile_pitch(cols);
@@ -516,15 +536,13 @@ template <typename T> static int launch_transpose(nncase_hip_ctx *ctx, const voi
 // (A = rows in groups of up to 128 lanes, X = cols), the destination the "packed" one, whose runs along A have no
 // padding.  Unpacking (short source rows): the destination is the plain tensor (A = cols, X = rows).
 static bool make_transpose_desc(TileDesc &d, int es, int batch, int rows, int cols, bool packing, const void *in, const void *out,
-                                uint64_t &blocks, size_t &lds) {
+                                int compute_units, uint64_t &blocks, size_t &lds) {
     if (es != 1 && es != 2 && es != 4) return false;
     const int e = 4 / es;
     if (((reinterpret_cast<uintptr_t>(in) | reinterpret_cast<uintptr_t>(out)) & 3u) != 0) return false;
     const bool ragged = rows % e != 0 || cols % e != 0;
     const uint64_t bytes = (uint64_t)batch * rows * cols * es;
-    // Few ragged tiles do not fill the device with blocks this heavy, the 32 x 32 ones are then quicker (155 channels of one
-    // 51 x 51 image of u8 4.9 against 6.0 us, of float16 4.7 / 6.9; of two 201 x 201 images 18.3 / 11.8 and 21.4 / 19.4).
-    if (ragged && bytes < ((uint64_t)es << 20)) return false;
+    if (ragged && !ragged_transpose_pays(es, batch, rows, cols, compute_units)) return false;
     memset(&d, 0, sizeof(d));
     d.ragged = ragged;
     d.in_bytes = bytes;
@@ -536,7 +554,7 @@ static bool make_transpose_desc(TileDesc &d, int es, int batch, int rows, int co
     d.x_packed = TwoTerm{1, (uint64_t)na, 0};
     d.exact = 1;
     d.wide = packing && (d.ragged ? (uint64_t)nx * es >= 64 : ((uint64_t)nx * es) % 16 == 0 && (reinterpret_cast<uintptr_t>(in) & 15u) == 0);
-    d.tx = tile_stretch(la, es, d.x_padded, d.wide);
+    d.tx = d.ragged ? ragged_stretch(la, es, d.x_padded, d.wide, (uint64_t)d.a_groups * batch, compute_units) : tile_stretch(la, es, d.x_padded, d.wide);
     d.x_tiles = (d.x_padded + d.tx - 1) / d.tx;
     d.nrest = 1;
     d.r_extent[0] = d.r_valid[0] = (uint32_t)batch;
@@ -563,7 +581,7 @@ static int transpose(nncase_hip_ctx *ctx, const void *in, void *out, int es, int
         uint64_t blocks = 0;
         size_t lds = 0;
         const bool packing = (size_t)cols * es >= 128; // source rows long enough to be read as rows
-        if (make_transpose_desc(t, es, batch, rows, cols, packing, in, out, blocks, lds)) {
+        if (make_transpose_desc(t, es, batch, rows, cols, packing, in, out, ctx->compute_units, blocks, lds)) {
             const int rc = packing ? launch_pack_tile<true>(ctx, in, out, es, t, blocks, lds) : launch_pack_tile<false>(ctx, in, out, es, t, blocks, lds);
             if (rc <= 0) return rc;
         }
@@ -664,7 +682,7 @@ extern "C" int nncase_hip_pack(nncase_hip_ctx_t *ctx, const void *in_dev, void *
         TileDesc t;
         uint64_t blocks = 0;
         size_t lds = 0;
-        if (make_tile_desc(t, elem_size, rank, shape, n_axes, nax, lanes, true, in_dev, out_dev, blocks, lds)) {
+        if (make_tile_desc(t, elem_size, rank, shape, n_axes, nax, lanes, true, in_dev, out_dev, ctx->compute_units, blocks, lds)) {
             rc = launch_pack_tile<true>(ctx, in_dev, out_dev, elem_size, t, blocks, lds);
             if (rc <= 0) return rc;
         }
@@ -747,7 +765,7 @@ extern "C" int nncase_hip_unpack(nncase_hip_ctx_t *ctx, const void *in_dev, void
         TileDesc t;
         uint64_t blocks = 0;
         size_t lds = 0;
-        if (make_tile_desc(t, elem_size, rank, unpacked_shape, n_axes, nax, lanes, false, in_dev, out_dev, blocks, lds)) {
+        if (make_tile_desc(t, elem_size, rank, unpacked_shape, n_axes, nax, lanes, false, in_dev, out_dev, ctx->compute_units, blocks, lds)) {
             rc = launch_pack_tile<false>(ctx, in_dev, out_dev, elem_size, t, blocks, lds);
             if (rc <= 0) return rc;
         }

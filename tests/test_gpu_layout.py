@@ -117,7 +117,31 @@ def test_pack_and_unpack_of_rows_that_end_inside_a_piece(hip_ctx, shape, lanes, 
 @pytest.mark.parametrize("dtype", [np.uint8, np.float16])
 @pytest.mark.parametrize("shape", [(1, 155, 201, 73), (9, 3, 223, 181), (2, 66, 101, 163), (1, 1031, 33, 65)])
 def test_relayout_of_odd_extents(hip_ctx, shape, dtype):
-    """NCHW <-> NHWC of tensors large enough for the tile kernel whose rows are no whole dwords on either side."""
+    """NCHW <-> NHWC of tensors whose rows are no whole dwords on either side, on both sides of where the tile kernel takes over."""
+    rng = np.random.default_rng(shape[1])
+    x = rng.integers(0, 200, shape).astype(dtype)
+    y = K.transpose_nchw_to_nhwc(x, ctx=hip_ctx)
+    assert np.array_equal(y, x.transpose(0, 2, 3, 1))
+    assert np.array_equal(K.transpose_nhwc_to_nchw(y, ctx=hip_ctx), x)
+
+
+@pytest.mark.parametrize("dtype", [np.uint8, np.float16, np.float32])
+@pytest.mark.parametrize("shape,lanes", [((1, 75, 75, 75), 32), ((1, 155, 75, 75), 4), ((8, 3, 151, 151), 32), ((16, 3, 201, 201), 16),
+                                         ((1, 61, 103, 151), 64), ((1, 75, 38, 38), 32), ((1, 33, 42, 42), 16), ((1, 40, 14, 14), 4)])
+def test_pack_and_unpack_of_ragged_rows_by_tiles(hip_ctx, shape, lanes, dtype):
+    """Tensors past the sizes from which ragged rows go through LDS tiles (of 4, 8 and 16 KiB by the launch), and rows of whole
+    dwords that are read dword by dword or in unaligned pieces."""
+    rng = np.random.default_rng(shape[1] + lanes)
+    x = rng.integers(0, 200, shape).astype(dtype)
+    got = K.pack(x, [1], [lanes], ctx=hip_ctx)
+    assert np.array_equal(got, O.pack(x, [1], [lanes]))
+    assert np.array_equal(K.unpack(got, [1], [lanes], shape, ctx=hip_ctx), x)
+
+
+@pytest.mark.parametrize("dtype", [np.uint8, np.float16])
+@pytest.mark.parametrize("shape", [(2, 155, 151, 149), (9, 3, 151, 151), (2, 1031, 71, 67), (4, 17, 251, 253)])
+def test_relayout_of_odd_extents_by_tiles(hip_ctx, shape, dtype):
+    """NCHW <-> NHWC of enough 32 x 32 tiles that the kernel with larger ones takes over."""
     rng = np.random.default_rng(shape[1])
     x = rng.integers(0, 200, shape).astype(dtype)
     y = K.transpose_nchw_to_nhwc(x, ctx=hip_ctx)
