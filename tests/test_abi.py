@@ -329,3 +329,11 @@ def test_shim_calls_declared_entry_points_with_the_right_arity():
             assert call_args(code, m.end() - 1) == arity[name], f"{fname}: {name}"
             calls += 1
     assert calls >= 8
+
+
+def test_the_environment_decides_nothing_but_the_hardware_queue_count():
+    """No variable of the caller's environment changes which kernel runs: the library reads the runtime's own
+    GPU_MAX_HW_QUEUES and nothing else."""
+    csrc = os.path.join(ROOT, "nncase_amd", "csrc")
+    text = "\n".join(open(os.path.join(csrc, f)).read() for f in sorted(os.listdir(csrc)))
+    assert re.findall(r"getenv\s*\(([^)]*)\)", text) == ['"GPU_MAX_HW_QUEUES"']
