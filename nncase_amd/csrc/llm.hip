@@ -809,12 +809,21 @@ template <typename KernelT> static hipError_t raise_dynamic_lds(KernelT kernel, 
     return e;
 }
 
+// Whether a plain product of m rows (up to two token tiles that fit half of LDS) is computed with a tile's reduction split over a
+// block's waves.  The sum's order depends on it, so it is asked for the rows' count and the matrix alone: the product, the one
+// that normalises its rows and the one that rotates them agree bit for bit.  A block per tile repeats the rows' trip (and their
+// normalisation), a tile per wave leaves the device to few blocks: us, split / not, k = 896, 4096 / 8192 / 16368 columns: one row
+// 2.9 3.4 5.0 / 4.4 4.6 5.7, 16 rows 3.2 4.0 5.8 / 4.5 5.0 6.0, 32 rows 3.9 5.0 8.7 / 5.7 6.2 7.2 (10 240 columns 7.0 / 6.6).
+static bool rows_take_split(const nncase_hip_ctx_t *ctx, const nncase_hip_w8a16_t *w, int m) {
+    const int mt_built = m <= 16 ? 1 : 2;
+    return m <= 32 && w->k <= kRowsMaxK && (size_t)mt_built * 16 * rows_in_lds_pitch(w->k) <= 64 * 1024 &&
+           2 * w->ntiles < (m <= kGemmWaves ? 8 : 5) * ctx->compute_units;
+}
+
 // Whether the q / k / v projection of this geometry can rotate and append in its own epilogue (else the caller runs
 // the projection and the rope kernel one after the other).
-static bool rope_epilogue_fits(const nncase_hip_w8a16_t *w, int m, const RopeArgs &r) {
-    const int mt_built = m <= 16 ? 1 : 2;
-    return m <= 32 && r.d % 32 == 0 && w->n == (r.hq + 2 * r.hkv) * r.d && w->k <= kRowsMaxK &&
-           (size_t)mt_built * 16 * rows_in_lds_pitch(w->k) <= 64 * 1024 && (w->ksteps + kGemmWaves - 1) / kGemmWaves <= 2;
+static bool rope_epilogue_fits(const nncase_hip_ctx_t *ctx, const nncase_hip_w8a16_t *w, int m, const RopeArgs &r) {
+    return rows_take_split(ctx, w, m) && r.d % 32 == 0 && w->n == (r.hq + 2 * r.hkv) * r.d && (w->ksteps + kGemmWaves - 1) / kGemmWaves <= 2;
 }
 
 static int launch_w8a16_gemm(nncase_hip_ctx_t *ctx, const void *a_dev, const nncase_hip_w8a16_t *w, void *out_dev, int32_t m,
@@ -909,9 +918,10 @@ static int launch_w8a16_gemm(nncase_hip_ctx_t *ctx, const void *a_dev, const nnc
         NNHIP_LAUNCH_CHECK(ctx, "w8a16_gemm_rows_in_lds_kernel");
         return 0;
     }
-    if (split && !glu && ln_weight_dev && w->k <= kRowsMaxK && rows_lds <= 64 * 1024 && mt_built <= 2) {
-        // few tiles and rows to normalise (the q / k / v projection): the reduction split over the block's waves, the
-        // rows parked and normalised in LDS in one trip to memory
+    if (!glu && rows_take_split(ctx, w, m) && (ln_weight_dev || out_tiles >= ctx->compute_units)) {
+        // few tiles (the q / k / v projection): the reduction split over the block's waves, the rows parked and normalised
+        // in LDS in one trip to memory; fewer tiles than compute units and nothing to normalise: the kernel below that
+        // reads the rows where they lie (the same order)
         // (the kernel's static reduction area comes on top of the rows: past 48 KiB in all, the limit is raised like below)
         // (a wave's share of the reduction is requested at once where it is at most two k-steps, the decode step's case)
         const bool short_share = (w->ksteps + kGemmWaves - 1) / kGemmWaves <= 2;
@@ -1055,7 +1065,7 @@ extern "C" int nncase_hip_w8a16_gemm_rope_kv_append(nncase_hip_ctx_t *ctx, const
     if (rc) return rc;
     NNHIP_REQUIRE(ctx, w->n == (r.hq + 2 * r.hkv) * r.d, -NNCASE_HIP_ERR_SHAPE_MISMATCH,
                   "w8a16_gemm_rope_kv_append: the matrix has %d output channels, the heads need %d", w->n, (r.hq + 2 * r.hkv) * r.d);
-    if (rope_epilogue_fits(w, r.batch, r))
+    if (rope_epilogue_fits(ctx, w, r.batch, r))
         return launch_w8a16_gemm(ctx, x_dev, w, qkv_dev, r.batch, NNCASE_HIP_GEMM_PLAIN, nullptr, NNCASE_HIP_DT_F16, ln_weight_dev, eps, &r);
     // other geometries: the projection into qkv_dev, then the rope kernel (the same values: the epilogue above rounds to
     // fp16 where this path stores fp16)

@@ -163,12 +163,12 @@ def test_rope_and_kv_append(hip_ctx):
 
 
 @pytest.mark.parametrize("B,k,norm", [(32, 896, True), (16, 896, True), (5, 256, False), (32, 1024, True), (7, 1536, True), (40, 896, True)])
-def test_projection_that_rotates_and_appends_equals_the_two_operators(hip_ctx, B, k, norm):
+def test_projection_that_rotates_and_appends_equals_the_two_operators(hip_ctx, B, k, norm, hq=14, hkv=2):
     """nncase_hip_w8a16_gemm_rope_kv_append against the projection into fp16 followed by nncase_hip_rope_kv_append: the same
     bytes in the query buffer and in both caches (the last two cases take the two-launch form inside the entry point: a
     reduction too long for the rows to be normalised in one block, more than 32 rows)."""
     rng = np.random.default_rng(B + k)
-    hq, hkv, d, blk, max_blocks = 14, 2, 64, 16, 8
+    d, blk, max_blocks = 64, 16, 8
     n = (hq + 2 * hkv) * d
     nb = B * max_blocks + 2
     lens = rng.integers(0, max_blocks * blk, B).astype(np.int32)
@@ -363,3 +363,19 @@ def test_few_rows_one_per_wave(hip_ctx, m, k, n, mode):
 @pytest.mark.parametrize("B,k,norm", [(1, 896, True), (8, 896, True), (9, 896, True), (8, 1024, False)])
 def test_few_rows_one_per_wave_that_rotate(hip_ctx, B, k, norm):
     test_projection_that_rotates_and_appends_equals_the_two_operators(hip_ctx, B, k, norm)
+
+
+@pytest.mark.parametrize("m,k,n,mode", [(8, 960, 4096, "residual"), (1, 896, 6144, "plain"), (9, 1984, 4096, "plain"), (16, 512, 8192, "f32"),
+                                        (17, 960, 16368, "f32"), (32, 1024, 4096, "plain"), (5, 64, 4096, "plain"), (33, 960, 4096, "plain"),
+                                        (8, 2048, 4112, "plain"), (32, 576, 4096, "residual"), (8, 256, 16384, "plain"), (9, 256, 10224, "plain"),
+                                        (9, 256, 10240, "plain")])
+def test_rmsnorm_fused_into_gemm_of_one_to_four_tiles_per_compute_unit(hip_ctx, m, k, n, mode):
+    """Sizes at which a tile's reduction is split over a block's waves or not, by rows and tiles: one order for both forms."""
+    test_rmsnorm_fused_into_gemm_equals_the_two_operators(hip_ctx, m, k, n, mode)
+
+
+@pytest.mark.parametrize("B,k,norm,hq,hkv", [(8, 896, False, 48, 8), (32, 960, False, 64, 16), (32, 1024, True, 48, 8), (1, 448, False, 200, 24),
+                                             (4, 128, False, 224, 16), (4, 896, True, 224, 16)])
+def test_projection_of_many_heads_that_rotates_and_appends(hip_ctx, B, k, norm, hq, hkv):
+    """One to four output tiles per compute unit, and more (two launches): the projection's own order of adding."""
+    test_projection_that_rotates_and_appends_equals_the_two_operators(hip_ctx, B, k, norm, hq, hkv)
