@@ -1,5 +1,6 @@
 // Host side of the implicit-GEMM convolution: weight pre-packing into MFMA
 // operand order, the tiling plan, and the launch dispatch.
+#include "qconv_rules.hpp"
 #include "qconv_wide.hpp"
 
 #include <algorithm>
@@ -42,15 +43,6 @@ static void plan_igemm(int g_oc, int ksteps, int64_t pixels_hint, int compute_un
     *kc_steps = best_kc;
 }
 
-// Whether a layer whose channels per group are no multiple of 16 is packed with its taps rounded up to 16 channels, for the
-// ragged loader of the wide kernels.  Multiples of 8 with a short reduction stay with the small tiles (8-byte pieces; us, ragged
-// against those: 25 088 pixels 24 -> 64 1x1 4.8 / 4.4, 8 -> 16 3x3 stride 2 5.8 / 4.5; from five k-steps on 24 -> 64 3x3 6.9 / 7.9,
-// 72 -> 64 3x3 9.3 / 13.4).  For anything else the small tiles gathered dwords or bytes (8893 pixels 90 -> 203 3x3 stride 2 61 us,
-// now 13.8; 3001 x 1000 product of one row 139, 9.5; of 5000 rows with 2100 columns 876, 82).
-static bool ragged_pays(int g_ic, int taps) {
-    return g_ic % 8 != 0 || ceil_div(taps * ceil_div(g_ic, 16) * 16, 64) >= 5;
-}
-
 // From how many k-steps of 64 a layer of whole 16-channel slices takes the small wide blocks.  Four, since their fetch of whole
 // rows beats the small tiles' slices by then (25 600 pixels 256 -> 256 1x1 10.1 -> 9.4 us) but not before (102 400 pixels
 // 128 -> 128 11.4 / 12.8, 200 704 pixels 144 -> 24 8.9 / 10.3).  Two where the outputs are what the launch is made of: channel
@@ -68,7 +60,7 @@ int igemm_plan(nncase_hip_ctx *ctx, nncase_hip_weights *w, const int32_t *bias) 
                   "qconv2d_prepack: reduction length %lld would overflow the int32 accumulator",
                   (long long)taps * w->g_ic);
     w->tap_ic = w->g_ic;
-    if (w->g_ic % 16 != 0 && ragged_pays(w->g_ic, taps)) w->ragged = true, w->tap_ic = ceil_div(w->g_ic, 16) * 16;
+    if (w->g_ic % 16 != 0 && ragged_pays(w->g_ic, taps, w->g_oc, w->pixels_hint)) w->ragged = true, w->tap_ic = ceil_div(w->g_ic, 16) * 16;
     w->k = taps * w->tap_ic;
     w->ksteps = ceil_div(w->k, 64);
     plan_igemm(w->g_oc, w->ksteps, w->pixels_hint, ctx->compute_units, &w->tiles, &w->nchunks, &w->kc_steps);
@@ -207,6 +199,7 @@ static bool igemm_is_pointwise(const nncase_hip_weights *w, const nncase_hip_con
 int igemm_load_mode(const nncase_hip_weights *w, const nncase_hip_conv2d_args_t *c, int out_h, int out_w) {
     const bool pointwise = igemm_is_pointwise(w, c, out_h, out_w);
     if (w->g_ic % 16 == 0) return pointwise ? kRows16 : kVec16;
+    if (w->g_ic % 8 != 0) return kVec4;
     // (the row loader reads 16 bytes at a time: the tensor has to hold that many)
     return pointwise && (int64_t)c->batch * c->in_h * c->in_w * w->in_channels >= 16 ? kRows8 : kVec8; // (anything else is ragged)
 }
@@ -315,6 +308,7 @@ int launch_qconv_igemm(nncase_hip_ctx *ctx, const uint8_t *x, const nncase_hip_w
         switch (mode) {
         case kRows16: rc = launch_igemm_rows16(ctx, a, w->tiles, w->nchunks, rg); break;
         case kVec16: rc = launch_igemm_vec16(ctx, a, w->tiles, w->nchunks, rg); break;
+        case kVec4: rc = launch_igemm_vec4(ctx, a, w->tiles, w->nchunks, rg); break;
         case kVec8: rc = launch_igemm_vec8(ctx, a, w->tiles, w->nchunks, rg); break;
         default: rc = launch_igemm_rows8(ctx, a, w->tiles, w->nchunks, rg); break;
         }

@@ -28,9 +28,10 @@
 //   kRows16  1x1 / stride 1 / no padding, channels % 16 == 0: a pixel's
 //            reduction row is contiguous, one 16-byte load per lane and k-step
 //   kRows8   the same for channels % 8 == 0: the last load of a row is half used
-//   kVec16/8 any window; channels % VW == 0, so a VW-byte piece of the
+//   kVec16/8/4 any window; channels % VW == 0, so a VW-byte piece of the
 //            reduction never straddles two taps
-// (other channel counts: the ragged loader of qconv_wide.hpp)
+// (which of the last two a layer takes, or the ragged loader of
+// qconv_wide.hpp: qconv_rules.hpp)
 #pragma once
 
 #include <mutex>
@@ -49,7 +50,7 @@ constexpr int kThreads = 256;
 constexpr int kWaves = 4;
 constexpr int kLdsFrags = 48; // weight fragments (1 KiB each) resident in LDS per block
 
-enum LoadMode { kRows16 = 0, kVec16 = 1, kVec8 = 2, kRows8 = 3 };
+enum LoadMode { kRows16 = 0, kVec16 = 1, kVec8 = 2, kRows8 = 3, kVec4 = 4 };
 constexpr bool loads_rows(int mode) { return mode == kRows16 || mode == kRows8; }
 
 struct IgemmArgs {
@@ -200,7 +201,7 @@ __device__ __forceinline__ v4i finish_act(const ActFrag &f) {
 }
 
 template <int MODE> __device__ __forceinline__ ActFrag load_act(const IgemmArgs &a, const PixInfo &pi, int kc) {
-    static_assert(MODE == kRows8 || MODE == kVec8, "8-byte pieces");
+    static_assert(MODE == kRows8 || MODE == kVec8 || MODE == kVec4, "rows or pieces below 16 bytes");
     const u32x4 zero_s8 = {0x80808080u, 0x80808080u, 0x80808080u, 0x80808080u}; // x' = 0
     ActFrag f;
     f.take = 0;
@@ -221,18 +222,25 @@ template <int MODE> __device__ __forceinline__ ActFrag load_act(const IgemmArgs 
         f.raw = u32x4{over ? v[2] : v[0], over ? v[3] : v[1], v[2], v[3]};
         f.take = (pix_ok && in_k) ? (a.k - kcc * 16 >= 16 ? 0xfu : 0x3u) : 0u;
     } else {
+        constexpr int VW = MODE == kVec8 ? 8 : 4;
 #pragma unroll
-        for (int piece = 0; piece < 2; piece++) {
-            const int kk = kc * 16 + piece * 8;
+        for (int piece = 0; piece < 16 / VW; piece++) {
+            const int kk = kc * 16 + piece * VW;
             const bool in_k = kk < a.k;
             bool inside;
             const uint32_t off = tap_offset(a, sp, in_k ? kk : 0, &inside);
             const bool ok = pix_ok && in_k && inside;
             const uint32_t fill = (pix_ok && in_k) ? a.zx_splat : 0x80808080u; // padding tap : outside the problem
-            const u32x2 v = *reinterpret_cast<const u32x2 *>(a.x + (size_t)off);
-            f.raw[piece * 2] = v[0], f.raw[piece * 2 + 1] = v[1];
-            f.fill[piece * 2] = fill, f.fill[piece * 2 + 1] = fill;
-            f.take |= ok ? (3u << (piece * 2)) : 0u;
+            if (VW == 8) {
+                const u32x2 v = *reinterpret_cast<const u32x2 *>(a.x + (size_t)off);
+                f.raw[piece * 2] = v[0], f.raw[piece * 2 + 1] = v[1];
+                f.fill[piece * 2] = fill, f.fill[piece * 2 + 1] = fill;
+                f.take |= ok ? (3u << (piece * 2)) : 0u;
+            } else {
+                f.raw[piece] = *reinterpret_cast<const uint32_t *>(a.x + (size_t)off);
+                f.fill[piece] = fill;
+                f.take |= ok ? (1u << piece) : 0u;
+            }
         }
     }
     return f;
@@ -1168,5 +1176,6 @@ int launch_igemm_rows16(nncase_hip_ctx *ctx, const IgemmArgs &a, int tiles, int 
 int launch_igemm_vec16(nncase_hip_ctx *ctx, const IgemmArgs &a, int tiles, int nchunks, int rg);
 int launch_igemm_vec8(nncase_hip_ctx *ctx, const IgemmArgs &a, int tiles, int nchunks, int rg);
 int launch_igemm_rows8(nncase_hip_ctx *ctx, const IgemmArgs &a, int tiles, int nchunks, int rg);
+int launch_igemm_vec4(nncase_hip_ctx *ctx, const IgemmArgs &a, int tiles, int nchunks, int rg);
 
 } // namespace nnhip

@@ -316,6 +316,20 @@ def test_channel_counts_that_fill_no_piece(hip_ctx, n, c, h, w, oc, k, s, groups
     run_case(hip_ctx, n, c, h, w, oc, k, k, (s, s), pad, (1, 1), groups, seed=c + oc + k + zx, zx=zx, zw=zw, modes=("u8", "i32") if big else ("u8", "i32", "f32"))
 
 
+# channels per group that are no multiple of 16, on both sides of where their taps are rounded up to 16: pieces of 4 and 8 channels
+# (4 -> 9 2x2 carries the zero-point term in its weights), and the ragged loader of the same channel counts
+PIECES = [(2, 4, 9, 11, 9, 2, 1, 1), (1, 4, 15, 13, 6, 7, 2, 1), (1, 4, 96, 97, 68, 3, 1, 1), (3, 16, 7, 9, 12, 3, 1, 4), (1, 4, 5, 3, 66, 1, 1, 1),
+          (1, 12, 28, 27, 20, 3, 2, 1), (1, 12, 80, 81, 33, 3, 1, 1), (2, 20, 9, 9, 22, 3, 1, 1), (1, 44, 17, 15, 5, 5, 1, 1),
+          (2, 8, 41, 43, 10, 5, 1, 1), (1, 24, 28, 29, 32, 3, 2, 1), (1, 40, 65, 67, 64, 3, 1, 1), (2, 48, 9, 7, 12, 7, 1, 2), (1, 52, 7, 7, 3, 3, 1, 1)]
+
+
+@pytest.mark.parametrize("n,c,h,w,oc,k,s,groups", PIECES)
+@pytest.mark.parametrize("zx,zw", [(7, 131), (255, 1)])
+def test_pieces_of_four_and_eight_channels(hip_ctx, n, c, h, w, oc, k, s, groups, zx, zw):
+    run_case(hip_ctx, n, c, h, w, oc, k, k, (s, s), ((k // 2, k // 2), (k // 2, (k - 1) // 2)), (1, 1), groups, seed=n * 31 + c + oc + k, zx=zx, zw=zw,
+             clamp=None)
+
+
 @pytest.mark.parametrize("zw", [0, 1, 2, 127, 128, 129, 254, 255])
 @pytest.mark.parametrize("cin,k,pad", [(16, 1, 0), (24, 1, 0), (32, 1, 0), (3, 3, 1), (8, 2, 0), (33, 1, 0), (48, 1, 0)])
 def test_short_reductions_for_every_weight_zero_point(hip_ctx, zw, cin, k, pad):
