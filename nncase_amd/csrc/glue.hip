@@ -5,6 +5,7 @@
 // (256 evaluations with the same fp32 operations the CPU kernels use), so the device only
 // moves bytes and the result is bit-exact by construction.
 #include "common.hpp"
+#include "glue_rules.hpp"
 
 #include <cmath>
 #include <type_traits>
@@ -200,7 +201,8 @@ struct MaxBytes16 {
 // window that overlaps the border yields max(values, 0): here max(table[m], Q(0)).
 // Bound by the re-reads of the windows (L2 when the rows of a window meet in one): 5x5 over 6400 pixels by 256 channels
 // 11.3 us with a load at a time, bytes compared one by one and rows dealt to all XCDs, now 4.8.
-template <int VEC> __global__ __launch_bounds__(kGlueThreads) void maxpool_u8_kernel(const PoolArgs a, const ByteTable lut) {
+// U: loads of a window row in flight (VEC = 16 only; loads_per_turn).
+template <int VEC, int U> __global__ __launch_bounds__(kGlueThreads) void maxpool_u8_kernel(const PoolArgs a, const ByteTable lut) {
     __shared__ __align__(16) uint8_t t[256];
     stage_table(t, lut);
     // a contiguous eighth of the blocks per XCD (they are dealt round-robin): windows share rows through one L2
@@ -221,13 +223,13 @@ template <int VEC> __global__ __launch_bounds__(kGlueThreads) void maxpool_u8_ke
     if (VEC == 16) { // 16 channels per thread: a quarter of the loads for the same bytes
         MaxBytes16 m;
         for (int y = y0; y < y1; y++)
-            for (int x = x0; x < x1; x += 5) { // five loads in flight; past the end the last one again
-                uint4 d[5];
+            for (int x = x0; x < x1; x += U) { // past the end the last one again
+                uint4 d[U];
 #pragma unroll
-                for (int e = 0; e < 5; e++)
+                for (int e = 0; e < U; e++)
                     d[e] = reinterpret_cast<const uint4 *>(a.in)[(((size_t)n * a.in_h + y) * a.in_w + min(x + e, x1 - 1)) * a.cvecs + v];
 #pragma unroll
-                for (int e = 0; e < 5; e++) m.take(d[e]);
+                for (int e = 0; e < U; e++) m.take(d[e]);
             }
         const uint4 m4 = m.get();
         uint4 o = uint4{lut4(t, m4.x), lut4(t, m4.y), lut4(t, m4.z), lut4(t, m4.w)};
@@ -272,7 +274,8 @@ struct ChainArgs {
     ByteTable pool[kChainLevels];     // requantisation level by level
     ByteTable slice[kChainLevels + 1]; // ... and to the concat's parameters (slice 0: the tensor itself)
 };
-template <int V> __global__ __launch_bounds__(kChainThreads) void maxpool_chain_kernel(const ChainArgs a) {
+// V: dwords of channels per block; U: loads_per_turn of the window.
+template <int V, int U> __global__ __launch_bounds__(kChainThreads) void maxpool_chain_kernel(const ChainArgs a) {
     typedef typename std::conditional<V == 4, uint4, uint32_t>::type Vec;
     typedef typename std::conditional<V == 4, MaxBytes16, MaxBytes>::type Max;
     __shared__ __align__(16) uint8_t tables[2 * kChainLevels + 1][256]; // [pool 0 .. | slice 0 ..]
@@ -291,15 +294,15 @@ template <int V> __global__ __launch_bounds__(kChainThreads) void maxpool_chain_
         if constexpr (V == 4) return uint4{lut4(tables[t], v.x), lut4(tables[t], v.y), lut4(tables[t], v.z), lut4(tables[t], v.w)};
         else return lut4(tables[t], v);
     };
-    // maximum of `at` over [from, to], five values in flight; past the end the last one again
+    // maximum of `at` over [from, to], U values in flight; past the end the last one again
     auto window = [&](int from, int to, auto at) {
         Max m;
-        for (int i = from; i <= to; i += 5) {
-            Vec v[5];
+        for (int i = from; i <= to; i += U) {
+            Vec v[U];
 #pragma unroll
-            for (int e = 0; e < 5; e++) v[e] = at(min(i + e, to));
+            for (int e = 0; e < U; e++) v[e] = at(min(i + e, to));
 #pragma unroll
-            for (int e = 0; e < 5; e++) m.take(v[e]);
+            for (int e = 0; e < U; e++) m.take(v[e]);
         }
         return m.get();
     };
@@ -533,8 +536,12 @@ int nnhip::launch_maxpool_chain(nncase_hip_ctx *ctx, const MaxPoolChain &c) {
     const size_t lds = (size_t)2 * c.h * c.w * (narrow ? 4 : 16);
     a.blocks = c.batch * (c.channels / (narrow ? 4 : 16));
     const dim3 grid((unsigned)((a.blocks + 7) / 8 * 8));
-    if (narrow) hipLaunchKernelGGL(maxpool_chain_kernel<1>, grid, dim3(kChainThreads), lds, ctx->stream, a);
-    else hipLaunchKernelGGL(maxpool_chain_kernel<4>, grid, dim3(kChainThreads), lds, ctx->stream, a);
+    auto launch = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, dim3(kChainThreads), lds, ctx->stream, a); };
+    switch (loads_per_turn(c.kernel)) {
+    case 5: launch(narrow ? maxpool_chain_kernel<1, 5> : maxpool_chain_kernel<4, 5>); break;
+    case 4: launch(narrow ? maxpool_chain_kernel<1, 4> : maxpool_chain_kernel<4, 4>); break;
+    default: launch(narrow ? maxpool_chain_kernel<1, 3> : maxpool_chain_kernel<4, 3>); break; // (3 x 3, and the window of one value)
+    }
     NNHIP_LAUNCH_CHECK(ctx, "maxpool_chain_kernel");
     return 0;
 }
@@ -570,9 +577,20 @@ extern "C" int nncase_hip_qmaxpool2d(nncase_hip_ctx_t *ctx, const uint8_t *x_dev
     a.d_cvecs = make_fastdiv(a.cvecs), a.d_ow = make_fastdiv((uint32_t)out_w), a.d_oh = make_fastdiv((uint32_t)out_h);
     a.zero_code = zero_code4(y_qp);
     const dim3 grid((unsigned)((total + kGlueThreads * 8 - 1) / (kGlueThreads * 8) * 8));
-    if (vec16) hipLaunchKernelGGL(maxpool_u8_kernel<16>, grid, dim3(kGlueThreads), 0, ctx->stream, a, pack_table(lut));
-    else if (vec) hipLaunchKernelGGL(maxpool_u8_kernel<4>, grid, dim3(kGlueThreads), 0, ctx->stream, a, pack_table(lut));
-    else hipLaunchKernelGGL(maxpool_u8_kernel<1>, grid, dim3(kGlueThreads), 0, ctx->stream, a, pack_table(lut));
+    auto launch = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, dim3(kGlueThreads), 0, ctx->stream, a, pack_table(lut)); };
+    if (vec16) {
+        switch (loads_per_turn(kernel_w)) {
+        case 1: launch(maxpool_u8_kernel<16, 1>); break;
+        case 2: launch(maxpool_u8_kernel<16, 2>); break;
+        case 3: launch(maxpool_u8_kernel<16, 3>); break;
+        case 4: launch(maxpool_u8_kernel<16, 4>); break;
+        default: launch(maxpool_u8_kernel<16, kMostLoadsPerTurn>); break;
+        }
+    } else if (vec) {
+        launch(maxpool_u8_kernel<4, 1>);
+    } else {
+        launch(maxpool_u8_kernel<1, 1>);
+    }
     NNHIP_LAUNCH_CHECK(ctx, "maxpool_u8_kernel");
     return 0;
 }

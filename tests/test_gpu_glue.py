@@ -188,3 +188,19 @@ def test_max_pool_chain_behind_a_concat_runs_as_one_launch(hip_ctx, n, h, w, c, 
             assert np.array_equal(out.download(want.shape, np.uint8), want)
         assert len(fn.profile(1)) == levels + 1
         fn.destroy()
+
+
+@pytest.mark.parametrize("kh,kw,s,pad", [(1, 1, 1, ((0, 0), (0, 0))), (3, 1, 2, ((1, 1), (0, 0))), (1, 4, 1, ((0, 0), (2, 1))), (2, 6, 2, ((1, 0), (3, 2))),
+                                         (7, 7, 1, ((3, 3), (3, 3))), (4, 11, 3, ((0, 3), (5, 5))), (6, 5, 1, ((2, 3), (4, 0)))])
+def test_maxpool_windows_in_turns(hip_ctx, kh, kw, s, pad):
+    """Windows whose rows are taken in one, two and three turns of one to five values, border windows shorter than a turn."""
+    x = np.random.default_rng(kh * 16 + kw).integers(0, 256, (2, 32, 19, 15), dtype=np.uint8)
+    for zx, sx, zy, sy in ((90, 0.05, 90, 0.05), (120, 0.04, 7, 0.031)):
+        got = K.max_pool2d(x, (kh, kw), (s, s), pad, qp(zx, sx), qp(zy, sy), ctx=hip_ctx)
+        assert np.array_equal(got, O.qmaxpool(x, (kh, kw), (s, s), pad, zx, sx, zy, sy))
+
+
+@pytest.mark.parametrize("n,h,w,c,k,levels,fused", [(2, 9, 11, 32, 1, 2, True), (2, 9, 11, 32, 7, 2, True), (16, 13, 12, 256, 7, 3, True), (16, 13, 12, 256, 3, 3, True),
+                                                    (1, 12, 12, 48, 11, 2, True)])
+def test_max_pool_chain_windows_in_turns(hip_ctx, n, h, w, c, k, levels, fused):
+    test_max_pool_chain_behind_a_concat_runs_as_one_launch(hip_ctx, n, h, w, c, k, levels, fused)
