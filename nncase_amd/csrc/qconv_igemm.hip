@@ -1,7 +1,7 @@
 // Host side of the implicit-GEMM convolution: weight pre-packing into MFMA
 // operand order, the tiling plan, and the launch dispatch.
 #include "qconv_rules.hpp"
-#include "qconv_wide.hpp"
+#include "qconv_tile.hpp"
 
 #include <algorithm>
 #include <vector>
@@ -273,6 +273,7 @@ int launch_qconv_igemm(nncase_hip_ctx *ctx, const uint8_t *x, const nncase_hip_w
     }
     const int mode = igemm_load_mode(w, c, out_h, out_w);
 
+    const TilePlan tile = w->ragged ? TilePlan{} : plan_qconv_tile(ctx, a, w->tiles, w->nchunks);
     const size_t group_bytes = (size_t)w->nchunks * w->ksteps * w->tiles * 1024;
     for (int g = 0; g < w->groups; g++) {
         a.wpk = reinterpret_cast<const uint8_t *>(w->d_packed) + g * group_bytes;
@@ -282,11 +283,10 @@ int launch_qconv_igemm(nncase_hip_ctx *ctx, const uint8_t *x, const nncase_hip_w
         a.y_coff = g * w->g_oc + c->out_channel_offset;
         a.r_coff = g * w->g_oc;
         int rc;
-        if (!w->ragged) {
-            bool taken;
-            rc = launch_qconv_tile(ctx, a, w->tiles, w->nchunks, &taken);
+        if (tile.shape != kTileNone) {
+            rc = launch_qconv_tile(ctx, a, tile, w->nchunks);
             if (rc) return rc;
-            if (taken) continue;
+            continue;
         }
         if (w->ragged) {
             const bool rows = igemm_is_pointwise(w, c, out_h, out_w);

@@ -13,22 +13,10 @@
 //     weights to come from memory at the same time, step after step;
 //   * results leave through LDS as whole pixel rows.
 // Arithmetic, weight packing and the bytes of the result are those of qconv_igemm.hpp.
-#include "qconv_wide.hpp"
+#include "qconv_rules.hpp"
+#include "qconv_tile.hpp"
 
 namespace nnhip {
-
-struct TileArgs {
-    int th, tw;                    // output tile
-    int hr, hc;                    // input rows / columns under it
-    int half;                      // input columns per column phase (stride 2: column c lies at (c & 1) * half + c / 2, so that
-                                   // neighbouring output pixels read neighbouring LDS pixels)
-    int pitch, row_pitch;          // bytes of an LDS pixel (an odd number of 16-byte pieces: eight lanes, eight banks) / row
-    int pieces;                    // 16-byte pieces per pixel
-    int dq, dc, dr;                // a block's threads as a step in (piece, column, row)
-    int row_bytes;                 // of the tensor
-    int tile_off;
-    FastDiv d_pieces, d_hc, d_tw, d_tx, d_txy, d_nchunks, d_rest;
-};
 
 // FAST: the requantisation is the one-instruction form without a clamp of its own (Epilogue::fast and ::full).
 
@@ -335,46 +323,26 @@ __global__ __launch_bounds__(WM * WN * 64, 4) void qconv_tile_kernel(const Igemm
 }
 
 namespace {
-struct TilePlan {
-    TileArgs t;
-    int tiles; // of the whole batch
-    size_t lds;
-};
-
-// The output tile of at most `pix` pixels: the fewest blocks, then the smallest input.
+// The plan of a kernel with `pix` pixels and `tb` 16-channel tiles per block.
 TilePlan plan_tile(const IgemmArgs &a, int pix, int tb, int threads, int nchunks) {
     const int ow = (int)a.d_ow.div, oh = (int)a.d_ohow.div / ow, batch = a.m / (int)a.d_ohow.div;
-    TilePlan best;
-    long long best_blocks = -1, best_area = 0;
-    for (int nx = ceil_div(ow, std::min(pix, 32)); nx <= ow; nx++) {
-        const int tw = ceil_div(ow, nx);
-        if (nx > 1 && tw == ceil_div(ow, nx - 1)) continue;
-        const int rows = std::min(pix / tw, oh), th = ceil_div(oh, ceil_div(oh, rows)); // rows spread evenly over the tiles
-        const int tx = ceil_div(ow, tw), ty = ceil_div(oh, th);
-        const int hr = (th - 1) * a.stride_h + (a.kh - 1) * a.dil_h + 1, hc = (tw - 1) * a.stride_w + (a.kw - 1) * a.dil_w + 1;
-        const long long blocks = (long long)tx * ty, area = (long long)hr * hc;
-        if (best_blocks >= 0 && (blocks > best_blocks || (blocks == best_blocks && area >= best_area))) {
-            if (tw < 4) break;
-            continue;
-        }
-        best_blocks = blocks, best_area = area;
-        TileArgs &t = best.t;
-        t.th = th, t.tw = tw, t.hr = hr, t.hc = hc;
-        t.half = ceil_div(hc, a.stride_w);
-        t.pieces = a.g_ic / 16;
-        t.pitch = (t.pieces | 1) * 16;
-        t.row_pitch = a.stride_w * t.half * t.pitch;
-        t.row_bytes = a.in_w * a.ldx;
-        t.d_pieces = make_fastdiv((uint32_t)t.pieces), t.d_hc = make_fastdiv((uint32_t)hc), t.d_tw = make_fastdiv((uint32_t)tw);
-        t.d_tx = make_fastdiv((uint32_t)tx), t.d_txy = make_fastdiv((uint32_t)(tx * ty));
-        best.tiles = batch * tx * ty;
-    }
-    TileArgs &t = best.t;
+    const OutputTile o = choose_output_tile(oh, ow, pix, a.stride_h, a.stride_w, (a.kh - 1) * a.dil_h + 1, (a.kw - 1) * a.dil_w + 1);
+    TilePlan p;
+    p.tiles = batch * o.across * o.down;
+    TileArgs &t = p.t;
+    t.th = o.th, t.tw = o.tw, t.hr = o.in_rows, t.hc = o.in_cols;
+    t.half = ceil_div(t.hc, a.stride_w);
+    t.pieces = a.g_ic / 16;
+    t.pitch = (t.pieces | 1) * 16;
+    t.row_pitch = a.stride_w * t.half * t.pitch;
+    t.row_bytes = a.in_w * a.ldx;
+    t.d_pieces = make_fastdiv((uint32_t)t.pieces), t.d_hc = make_fastdiv((uint32_t)t.hc), t.d_tw = make_fastdiv((uint32_t)t.tw);
+    t.d_tx = make_fastdiv((uint32_t)o.across), t.d_txy = make_fastdiv((uint32_t)(o.across * o.down));
     t.d_nchunks = make_fastdiv((uint32_t)nchunks), t.d_rest = make_fastdiv((uint32_t)std::max(1, a.ksteps - 1));
     t.tile_off = (tb * 16 + pix + (a.ksteps + 2) * 4) * 4 + 256;
     t.dq = threads % t.pieces, t.dc = threads / t.pieces % t.hc, t.dr = threads / t.pieces / t.hc;
-    best.lds = t.tile_off + std::max((size_t)t.hr * t.row_pitch, (size_t)pix * (tb * 16 + 16));
-    return best;
+    p.lds = t.tile_off + std::max((size_t)t.hr * t.row_pitch, (size_t)pix * (tb * 16 + 16));
+    return p;
 }
 
 template <int T, int RG, int WM, int WN, bool FAST> int launch_tile_f(nncase_hip_ctx *ctx, const IgemmArgs &args, const TilePlan &plan, int nchunks) {
@@ -399,8 +367,6 @@ template <int T, int RG, int WM, int WN> int launch_tile_t(nncase_hip_ctx *ctx, 
 } // namespace
 
 namespace {
-enum TileShape { kTile128x32, kTile64x32, kTile32x64, kTile128x128, kTile64x128, kTileNone };
-
 template <int T, int RG, int WM, int WN> TilePlan plan_shape(const IgemmArgs &a, int nchunks) {
     return plan_tile(a, WM * RG * 16, T * WN, WM * WN * 64, nchunks);
 }
@@ -456,11 +422,15 @@ const char *tile_kernel_block(const nncase_hip_ctx *ctx, const nncase_hip_weight
     return names[choose_tile(ctx, a, w->tiles, w->nchunks, &plan)];
 }
 
-int launch_qconv_tile(nncase_hip_ctx *ctx, const IgemmArgs &a, int tiles, int nchunks, bool *taken) {
+TilePlan plan_qconv_tile(const nncase_hip_ctx *ctx, const IgemmArgs &a, int tiles, int nchunks) {
     TilePlan plan;
     const TileShape shape = a.ep.out_mode == kOutU8 && !a.deq ? choose_tile(ctx, a, tiles, nchunks, &plan) : kTileNone;
-    *taken = shape != kTileNone;
-    switch (shape) {
+    plan.shape = shape;
+    return plan;
+}
+
+int launch_qconv_tile(nncase_hip_ctx *ctx, const IgemmArgs &a, const TilePlan &plan, int nchunks) {
+    switch (plan.shape) {
     case kTile128x32: return launch_tile_t<2, 4, 2, 1>(ctx, a, plan, nchunks);
     case kTile64x32: return launch_tile_t<2, 2, 2, 1>(ctx, a, plan, nchunks);
     case kTile32x64: return launch_tile_t<2, 2, 1, 2>(ctx, a, plan, nchunks);
@@ -468,7 +438,7 @@ int launch_qconv_tile(nncase_hip_ctx *ctx, const IgemmArgs &a, int tiles, int nc
     case kTile64x128: return launch_tile_t<2, 2, 2, 4>(ctx, a, plan, nchunks);
     case kTileNone: break;
     }
-    return 0;
+    return fail(ctx, -EINVAL, "qconv2d: not a layer of the tile kernel");
 }
 
 } // namespace nnhip

@@ -1,0 +1,34 @@
+// The window kernel that keeps a tile's input in LDS (qconv_tile.hip): what a launch of it is planned as.
+#pragma once
+
+#include "qconv_wide.hpp"
+
+namespace nnhip {
+
+struct TileArgs {
+    int th, tw;                    // output tile
+    int hr, hc;                    // input rows / columns under it
+    int half;                      // input columns per column phase (stride 2: column c lies at (c & 1) * half + c / 2, so that
+                                   // neighbouring output pixels read neighbouring LDS pixels)
+    int pitch, row_pitch;          // bytes of an LDS pixel (an odd number of 16-byte pieces: eight lanes, eight banks) / row
+    int pieces;                    // 16-byte pieces per pixel
+    int dq, dc, dr;                // a block's threads as a step in (piece, column, row)
+    int row_bytes;                 // of the tensor
+    int tile_off;
+    FastDiv d_pieces, d_hc, d_tw, d_tx, d_txy, d_nchunks, d_rest;
+};
+
+enum TileShape { kTile128x32, kTile64x32, kTile32x64, kTile128x128, kTile64x128, kTileNone };
+
+struct TilePlan {
+    TileShape shape = kTileNone;
+    TileArgs t;
+    int tiles; // of the whole batch
+    size_t lds;
+};
+
+// The plan of a call (the same for every group of a grouped layer); shape kTileNone: not a layer of this kernel.
+TilePlan plan_qconv_tile(const nncase_hip_ctx *ctx, const IgemmArgs &a, int tiles, int nchunks);
+int launch_qconv_tile(nncase_hip_ctx *ctx, const IgemmArgs &a, const TilePlan &plan, int nchunks);
+
+} // namespace nnhip

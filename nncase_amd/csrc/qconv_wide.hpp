@@ -1117,8 +1117,6 @@ template <int LM> int launch_wide_small_lm(nncase_hip_ctx *ctx, const IgemmArgs 
     }
     return fail(ctx, -EINVAL, "qconv2d: no small wide kernel of shape %d", shape);
 }
-// qconv_tile.hip: takes the launch where it pays (*taken)
-int launch_qconv_tile(nncase_hip_ctx *ctx, const IgemmArgs &a, int tiles, int nchunks, bool *taken);
 int launch_wide_small_rows16(nncase_hip_ctx *ctx, const IgemmArgs &a, int shape, int nchunks);
 int launch_wide_small_vec16(nncase_hip_ctx *ctx, const IgemmArgs &a, int shape, int nchunks);
 int launch_wide_rows16(nncase_hip_ctx *ctx, const IgemmArgs &a, int tiles, int nchunks);

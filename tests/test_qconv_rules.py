@@ -1,6 +1,6 @@
 """How a dense layer of narrow or odd channel counts is packed, held against measured times (us on the device, u8 and float32
-outputs): the choice is no more than a fifth slower than the other.  The rule is host arithmetic (csrc/qconv_rules.hpp),
-compiled here for the CPU."""
+outputs): the choice is no more than a fifth slower than the other.  And the output tile of the window kernel against its
+definition.  The rules are host arithmetic (csrc/qconv_rules.hpp), compiled here for the CPU."""
 import ctypes as C
 import os
 import subprocess
@@ -11,13 +11,24 @@ CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))),
 
 
 @pytest.fixture(scope="module")
-def ragged_pays(tmp_path_factory):
+def rules(tmp_path_factory):
     d = tmp_path_factory.mktemp("rules")
-    (d / "r.cpp").write_text('#include "qconv_rules.hpp"\nextern "C" int pays(int ic, int taps, int oc, long px) { return nnhip::ragged_pays(ic, taps, oc, px); }\n')
-    subprocess.check_call(["g++", "-std=c++17", "-shared", "-fPIC", "-I", CSRC, str(d / "r.cpp"), "-o", str(d / "r.so")])
+    (d / "r.cpp").write_text("""#include "qconv_rules.hpp"
+extern "C" int pays(int ic, int taps, int oc, long px) { return nnhip::ragged_pays(ic, taps, oc, px); }
+extern "C" void tile(int h, int w, int pix, int sh, int sw, int kh, int kw, int *out) {
+    const nnhip::OutputTile t = nnhip::choose_output_tile(h, w, pix, sh, sw, kh, kw);
+    out[0] = t.th, out[1] = t.tw, out[2] = t.across, out[3] = t.down, out[4] = t.in_rows, out[5] = t.in_cols;
+}
+""")
+    subprocess.check_call(["g++", "-std=c++17", "-O2", "-shared", "-fPIC", "-I", CSRC, str(d / "r.cpp"), "-o", str(d / "r.so")])
     lib = C.CDLL(str(d / "r.so"))
     lib.pays.argtypes = [C.c_int, C.c_int, C.c_int, C.c_long]
-    return lib.pays
+    return lib
+
+
+@pytest.fixture(scope="module")
+def ragged_pays(rules):
+    return rules.pays
 
 
 # (channels and outputs of a group, window side, output pixels, us by the small tiles, us rounded up to 16 channels per tap)
@@ -86,3 +97,26 @@ def test_channel_counts_without_a_choice(ragged_pays):
     for ic in (1, 2, 3, 5, 6, 7, 9, 30, 90, 3001):
         for taps in (1, 9, 49):
             assert ragged_pays(ic, taps, 1, 1) and ragged_pays(ic, taps, 512, 1 << 20)
+
+
+@pytest.mark.parametrize("pix", [32, 64, 128])
+@pytest.mark.parametrize("stride,span", [(1, 3), (2, 3), (1, 7), (2, 5), (1, 2)])
+def test_output_tile_is_the_best_of_all_numbers_of_tiles(rules, pix, stride, span):
+    """Fewest blocks, then the smallest input, then the widest tile, over every number of tiles side by side; below four columns
+    the first that does no better ends the search."""
+    up = lambda a, b: -(-a // b)
+    got = (C.c_int * 6)()
+    for h in (1, 2, 5, 7, 20, 33, 80):
+        for w in list(range(1, 70)) + [80, 111, 160, 320, 321, 1000]:
+            best = None
+            for nx in range(up(w, min(pix, 32)), w + 1):
+                tw = up(w, nx)
+                rows = min(pix // tw, h)
+                th = up(h, up(h, rows))
+                across, down, ih, iw = up(w, tw), up(h, th), (th - 1) * stride + span, (tw - 1) * stride + span
+                if best is None or (across * down, ih * iw) < best[0]:
+                    best = (across * down, ih * iw), [th, tw, across, down, ih, iw]
+                elif tw < 4 and tw != best[1][1]:
+                    break
+            rules.tile(h, w, pix, stride, stride, span, span, got)
+            assert list(got) == best[1], (h, w)
