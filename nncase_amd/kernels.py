@@ -5,7 +5,8 @@ target owns: same names, argument order and meaning as `kernels::stackvm::*`
 host tensors.  Every call stages its operands into HBM, runs the HIP kernel through the
 C ABI and copies the result back -- what the native `hip` runtime module does at an
 EXTCALL boundary.  Tensors are NCHW / OIHW here, as in the reference; the library works on
-NHWC internally and the relayout runs on the device.
+NHWC internally and the relayout runs on the device.  Results of 256 KiB and more are views of
+pinned memory that returns to a pool with their last view (`runtime.Context.host_array`).
 
 Quantised operators take the quantisation parameters the reference's importer attaches as
 Dequantize / Quantize nodes around the float op (QLinearConv.cs:61-75).

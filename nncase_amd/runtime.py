@@ -8,6 +8,7 @@ from __future__ import annotations
 
 import ctypes as C
 import errno
+import math
 import weakref
 import os
 from typing import Optional, Sequence, Tuple
@@ -341,6 +342,7 @@ class DeviceBuffer:
         return self
 
     def download(self, shape, dtype) -> np.ndarray:
+        """The buffer's first bytes as a new array (from 256 KiB on a view of pinned memory, see Context.host_array)."""
         out = self.ctx.host_array(shape, dtype)
         assert out.nbytes <= self.nbytes
         self.ctx._check(self.ctx.lib.nncase_hip_memcpy_d2h(self.ctx.handle, out.ctypes.data, self.ptr, out.nbytes), "d2h")
@@ -517,9 +519,12 @@ class Context:
     HOST_ARRAY_MIN = 256 << 10   # below it the runtime's own copy into pageable memory takes no longer
 
     def host_array(self, shape, dtype) -> np.ndarray:
-        """An uninitialised host array for a result, in pinned memory where that is large enough to pay and to be had."""
+        """An uninitialised host array for a result, in pinned memory where that is large enough to pay and to be had.  Such an
+        array is a view of a block from the process's pool (256 MiB at most, nncase_hip_host_malloc): it does not own its memory
+        (`flags.owndata` is False), the block goes back to the pool when the last array that views it is gone, and the array may
+        outlive the context."""
         dtype = np.dtype(dtype)
-        n = int(np.prod(shape, dtype=np.int64)) * dtype.itemsize
+        n = (math.prod(map(int, shape)) if isinstance(shape, (tuple, list)) else int(np.prod(shape, dtype=np.int64))) * dtype.itemsize
         if n >= self.HOST_ARRAY_MIN:
             p = C.c_void_p()
             if self.lib.nncase_hip_host_malloc(self.handle, n, C.byref(p)) == 0:

@@ -214,3 +214,22 @@ def test_strided_argument_checks(hip_ctx):
         hip_ctx.dequantize_strided(src, rt.DT_F32, dst, rt.DT_U8, (4, 2), (4, 1), (2, 2), qp(0, 1.0))
     assert e.value.code == -rt.ERR_DATATYPE_MISMATCH
     hip_ctx.quantize_strided(src, rt.DT_F32, dst, rt.DT_U8, (0, 4), (4, 1), (4, 1), qp(0, 1.0))   # empty: nothing to do
+
+
+def test_large_results_are_views_that_outlive_their_context():
+    """A result in pinned memory does not own it; it stays as it is, also written to, while anything views it: after the next
+    download of the same size, after its context is gone, and behind a slice of it."""
+    from nncase_amd.runtime import Context
+    ctx = Context(0)
+    n = ctx.HOST_ARRAY_MIN
+    small, large = ctx.alloc(64).fill(3), ctx.alloc(n).fill(5)
+    assert small.download((np.int64(4), 16), np.uint8).flags.owndata
+    a = large.download((n,), np.uint8)
+    assert not a.flags.owndata and a.flags.writeable
+    tail = a[-8:]
+    b = large.fill(9).download(n // 4, np.uint32)
+    a[0] = 1
+    ctx.close()
+    assert a[0] == 1 and (a[1:] == 5).all() and (b == 0x09090909).all()
+    del a, b
+    assert (tail == 5).all()
