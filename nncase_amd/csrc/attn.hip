@@ -24,6 +24,7 @@
 //   that finishes last for a (sequence, kv head) - found with one atomic
 //   counter per pair, which it resets for the next call - merges the splits
 //   and writes the output, so there is a single launch per call.
+#include "attn_rules.hpp"
 #include "common.hpp"
 
 #include <hip/hip_fp16.h>
@@ -404,21 +405,8 @@ static int attn_plan(nncase_hip_ctx *ctx, const nncase_hip_paged_attn_args_t *p,
     a.num_blocks = p->num_blocks;
     a.len_offset = p->ctx_len_offset;
     const int64_t max_tokens = (int64_t)p->max_blocks_per_seq * p->block_size;
-    // Tokens per block, as W waves of NT tiles, from the capacity and the launch's blocks (the kernel cannot know the real
-    // lengths on the host).  Four waves where they serve: a block of eight holds twice the registers and, at head_dim 128,
-    // half the compute unit's LDS, and its phases (requests, products, merge) then have one other block to overlap with.
-    // Measured, us as 128 / 256 / 512 tokens per block (2 / 4 tiles in four waves, 4 in eight): 48 sequences of 6000 tokens, 8 kv
-    // heads of 128: 152 / 141 / 155; 64 of 1000: 29.3 / 31.0 / 36.6; one of 1000: 7.7 / 9.2 / 12.0; one of 700, 2 kv heads of 64:
-    // 6.1 / 6.5 / 8.1.  Short blocks mean many splits to merge: up to eight (1024 tokens) they are one memory round trip,
-    // past that 256 tokens are better (16 sequences of 2048: 9.0 / 7.9 / 8.8), and 512 for the longest contexts while the
-    // launch has few blocks (one of 16 000: 18 / 12.6 / 10.9; 32 of 4096: 15.9 / 13.3 / 12.5).  A context of one block needs no
-    // merge at all (100 tokens: 4.1 us), so capacities of 129 to 256 take 256.
-    int nt = 4, waves = 4;
-    auto blocks_of = [&](int64_t tokens) { return (int64_t)p->batch * p->num_kv_heads * ((max_tokens + tokens - 1) / tokens); };
-    if (max_tokens <= 128 || (max_tokens > 256 && max_tokens <= 1024)) nt = 2;
-    else if ((max_tokens >= 8192 || (max_tokens >= 4096 && 4 * blocks_of(512) >= ctx->compute_units)) &&
-             blocks_of(512) * p->head_dim <= (int64_t)128 * ctx->compute_units)
-        waves = 8;
+    const AttnBlock block = choose_attn_block(p->head_dim, (int64_t)p->batch * p->num_kv_heads, max_tokens, ctx->compute_units);
+    int nt = block.tiles, waves = block.waves;
     for (;;) { // (longer runs where there would be too many splits, for the merge or for the scratch there is)
         a.split_tokens = waves * nt * 16;
         a.splits = (int)std::min<int64_t>((max_tokens + a.split_tokens - 1) / a.split_tokens, INT32_MAX);
@@ -467,8 +455,8 @@ static int attn_launch(nncase_hip_ctx *ctx, AttnPlan &plan, const void *q_dev, c
     };
 #define NNHIP_ATTN_CASE(DV, NTV, WV) \
     if (!launched && a.d == DV && nt == NTV && waves == WV) go(paged_attn_kernel<DV, NTV, WV>);
-    NNHIP_ATTN_CASE(64, 2, 4) NNHIP_ATTN_CASE(64, 4, 4) NNHIP_ATTN_CASE(64, 4, 8) NNHIP_ATTN_CASE(64, 8, 8)
-    NNHIP_ATTN_CASE(128, 2, 4) NNHIP_ATTN_CASE(128, 4, 4) NNHIP_ATTN_CASE(128, 4, 8)
+    NNHIP_ATTN_CASE(64, 2, 4) NNHIP_ATTN_CASE(64, 4, 4) NNHIP_ATTN_CASE(64, 2, 8) NNHIP_ATTN_CASE(64, 4, 8) NNHIP_ATTN_CASE(64, 8, 8)
+    NNHIP_ATTN_CASE(128, 2, 4) NNHIP_ATTN_CASE(128, 4, 4) NNHIP_ATTN_CASE(128, 2, 8) NNHIP_ATTN_CASE(128, 4, 8)
 #undef NNHIP_ATTN_CASE
     NNHIP_REQUIRE(ctx, launched, -EINVAL, "paged_attention_decode: no kernel for head_dim %d, %d tiles per wave, %d waves", a.d, nt, waves);
     NNHIP_LAUNCH_CHECK(ctx, "paged_attn_kernel");

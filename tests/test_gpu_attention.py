@@ -210,6 +210,15 @@ def test_every_split_of_the_capacity(hip_ctx, hq, hkv, d, capacity):
     check(hip_ctx, *case, 1.0 / np.sqrt(d))
 
 
+@pytest.mark.parametrize("b,hq,hkv,d,capacity", [(33, 14, 2, 64, 3216), (20, 16, 16, 64, 208), (2, 12, 12, 64, 6512), (4, 32, 8, 128, 2064), (1, 16, 8, 128, 10016),
+                                                 (33, 32, 8, 128, 160), (64, 16, 4, 128, 1040)])
+def test_block_shapes_by_the_launch(hip_ctx, b, hq, hkv, d, capacity):
+    """Capacities at which the number of sequences and kv heads decides the tokens per block, on both sides."""
+    rng = np.random.default_rng(capacity + d)
+    lens = ([1, capacity // 3 + 1, capacity, capacity - 15] * b)[-b:]
+    check(hip_ctx, *make_case(rng, b, hq, hkv, d, 16, capacity, lens), 1.0 / np.sqrt(d))
+
+
 def test_a_workspace_that_cannot_grow_takes_longer_runs(hip_ctx):
     """While a captured graph holds the workspace, a call whose usual split needs more of it runs with fewer splits instead."""
     rng = np.random.default_rng(3)
