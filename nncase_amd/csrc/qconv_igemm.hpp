@@ -1104,8 +1104,8 @@ template <int T, int RG, int MODE> int launch_trg(nncase_hip_ctx *ctx, const Ige
             NNHIP_LAUNCH_CHECK(ctx, "qconv_window_kernel");
             return 0;
         }
-        plain = false;
     }
+    if constexpr (!loads_rows(MODE)) plain = false; // (qconv_igemm_kernel has no such form for windows)
     if (plain) {
         if constexpr (MODE == kRows16) {
             // the whole chunk's weights resident, rows of at least 16 bytes: the lean kernel

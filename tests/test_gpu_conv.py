@@ -316,6 +316,33 @@ def test_channel_counts_that_fill_no_piece(hip_ctx, n, c, h, w, oc, k, s, groups
     run_case(hip_ctx, n, c, h, w, oc, k, k, (s, s), pad, (1, 1), groups, seed=c + oc + k + zx, zx=zx, zw=zw, modes=("u8", "i32") if big else ("u8", "i32", "f32"))
 
 
+# short reductions that are no rows of the input (a stride, a window), chunks of more than 96 output channels, whole groups of them
+SHORT_WINDOWS = [(2, 64, 15, 15, 128, 1, 2), (1, 16, 21, 20, 512, 1, 2), (2, 32, 13, 14, 128, 2, 1), (1, 112, 19, 19, 160, 1, 2), (1, 16, 17, 18, 448, 3, 2),
+                 (1, 48, 9, 9, 144, 1, 2), (1, 96, 31, 31, 192, 1, 2), (2, 16, 8, 9, 96, 3, 1)]
+
+
+@pytest.mark.parametrize("n,c,h,w,oc,k,s", SHORT_WINDOWS)
+@pytest.mark.parametrize("hint", [0, 1 << 20])
+def test_short_reductions_over_windows_into_many_channels(hip_ctx, n, c, h, w, oc, k, s, hint):
+    """The result is written whatever the plan: into a buffer that held something else, with the one-instruction requantisation
+    (full range, scales at which it exists) and without."""
+    rng = np.random.default_rng(c + oc + k)
+    x, wt = rng.integers(0, 256, (n, c, h, w), dtype=np.uint8), rng.integers(0, 256, (oc, c, k, k), dtype=np.uint8)
+    bias = rng.integers(-3000, 3000, oc).astype(np.int32)
+    pad = ((k // 2, (k - 1) // 2), (k // 2, (k - 1) // 2))
+    weights = hip_ctx.prepack_conv2d(wt, bias, qp(131, 0.0041), 1, expected_pixels=hint)
+    dx = hip_ctx.to_device(np.ascontiguousarray(x.transpose(0, 2, 3, 1)))
+    forms = set()
+    for sy in (f32(0.0041 * c * k * k / 16), f32(0.021), f32(0.3), f32(1.7)):
+        forms.add(rt.requant_plan(0.0235, 0.0041, qp(118, sy))[0])
+        want = O.qconv2d(x, wt, bias, 7, f32(0.0235), 131, f32(0.0041), 118, sy, fused_clamp=FULL, out_mode=O.OUT_U8, stride=(s, s), padding=pad, dilation=(1, 1), groups=1)
+        dy = hip_ctx.to_device((want ^ 0x55).transpose(0, 2, 3, 1))
+        args = rt.Conv2dArgs(n, h, w, s, s, 1, 1, *pad[0], *pad[1], qp(7, 0.0235), qp(118, sy), *FULL, rt.DT_U8)
+        hip_ctx.qconv2d(dx, weights, dy, args)
+        assert np.array_equal(dy.download((n,) + want.shape[2:] + (oc,), np.uint8).transpose(0, 3, 1, 2), want)
+    assert True in forms
+
+
 # channels per group that are no multiple of 16, on both sides of where their taps are rounded up to 16: pieces of 4 and 8 channels
 # (4 -> 9 2x2 carries the zero-point term in its weights), and the ragged loader of the same channel counts
 PIECES = [(2, 4, 9, 11, 9, 2, 1, 1), (1, 4, 15, 13, 6, 7, 2, 1), (1, 4, 96, 97, 68, 3, 1, 1), (3, 16, 7, 9, 12, 3, 1, 4), (1, 4, 5, 3, 66, 1, 1, 1),
