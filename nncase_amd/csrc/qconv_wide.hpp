@@ -430,6 +430,7 @@ __global__ __launch_bounds__(WM * WN * 64, 2) void qconv_wide4_kernel(const Igem
     static_assert((2 * AV) % THREADS == 0 && WV % THREADS == 0 && PSTEP % 8 == 0, "every thread moves the same number of vectors");
     static_assert(T % 4 == 0, "at least two pairs of channel tiles per k-step");
     constexpr int G = T / 2;
+    static_assert(NA2 <= G, "the pieces of a pair are staged one after the other");
     constexpr int SLOT = AV * 16 + WV * 16;
     constexpr bool kRows = LM == kWideRowsFull || LM == kWideRows;
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
@@ -530,7 +531,9 @@ __global__ __launch_bounds__(WM * WN * 64, 2) void qconv_wide4_kernel(const Igem
         constexpr int i = decltype(i_c)::value;
         f.raw[i] = __builtin_amdgcn_raw_buffer_load_b128(xres, g.phantom ? (int)0xfffffff0u : p_off[i] + g.shift, 0, 0);
         f.take[i] = g.phantom || (kRows ? g.in_k : (g.in_k && (unsigned)(p_iy0[i] + g.dy) < (unsigned)a.in_h && (unsigned)(p_ix0[i] + g.dx) < (unsigned)a.in_w));
-        if (i == 0) f.fill = kRows ? 0x80808080u : (g.in_k ? a.zx_splat : 0x80808080u);
+        // (One value for all pieces of a pair.  The main loop stages them in turn and requests the next pair's right behind each, so it
+        // changes with the last: until then it is still the value of the pieces that are staged.)
+        if (i == NA2 - 1) f.fill = kRows ? 0x80808080u : (g.in_k ? a.zx_splat : 0x80808080u);
     };
     auto load_acts = [&](Acts &f, int pair) {
         const Geom g = geometry(pair);

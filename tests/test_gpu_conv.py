@@ -343,6 +343,27 @@ def test_short_reductions_over_windows_into_many_channels(hip_ctx, n, c, h, w, o
     assert True in forms
 
 
+# chunks of 256 output channels (weights packed for many pixels) over windows whose reduction is no multiple of 64: the last k-steps
+# hold padding taps and positions past the reduction next to each other
+WIDE_WINDOWS = [(3, 80, 5, 18, 192, 3, 2, 1, 1), (1, 80, 5, 18, 200, 3, 3, 1, 1), (1, 96, 20, 18, 192, 3, 3, 1, 1), (1, 80, 20, 18, 320, 5, 5, 1, 1),
+                (2, 48, 17, 15, 256, 5, 5, 2, 1), (1, 16, 20, 18, 192, 7, 7, 1, 1), (1, 144, 9, 7, 130, 3, 3, 1, 2), (1, 112, 11, 13, 512, 2, 3, 2, 1)]
+
+
+@pytest.mark.parametrize("n,c,h,w,oc,kh,kw,s,d", WIDE_WINDOWS)
+@pytest.mark.parametrize("zx,zw", [(0, 1), (255, 131)])
+def test_padding_in_the_last_steps_of_a_window(hip_ctx, n, c, h, w, oc, kh, kw, s, d, zx, zw):
+    rng = np.random.default_rng(c + oc + kh)
+    x, wt = rng.integers(0, 256, (n, c, h, w), dtype=np.uint8), rng.integers(0, 256, (oc, c, kh, kw), dtype=np.uint8)
+    bias, pad = rng.integers(-3000, 3000, oc).astype(np.int32), ((kh - 2, kh - 1), (kw - 1, kw - 2))
+    weights = hip_ctx.prepack_conv2d(wt, bias, qp(zw, 0.0041), 1, expected_pixels=1 << 20)
+    dx = hip_ctx.to_device(np.ascontiguousarray(x.transpose(0, 2, 3, 1)))
+    want = O.qconv2d(x, wt, bias, zx, f32(0.0235), zw, f32(0.0041), out_mode=O.OUT_I32, stride=(s, s), padding=pad, dilation=(d, d), groups=1)
+    dy = hip_ctx.to_device((want ^ 0x55).transpose(0, 2, 3, 1))
+    hip_ctx.qconv2d(dx, weights, dy, rt.Conv2dArgs(n, h, w, s, s, d, d, *pad[0], *pad[1], qp(zx, 0.0235), qp(0, 1.0), *FULL, rt.DT_I32))
+    got = dy.download((n,) + want.shape[2:] + (oc,), np.int32).transpose(0, 3, 1, 2)
+    assert np.array_equal(got, want), f"int32 accumulators differ in {(got != want).sum()} of {got.size}"
+
+
 # channels per group that are no multiple of 16, on both sides of where their taps are rounded up to 16: pieces of 4 and 8 channels
 # (4 -> 9 2x2 carries the zero-point term in its weights), and the ragged loader of the same channel counts
 PIECES = [(2, 4, 9, 11, 9, 2, 1, 1), (1, 4, 15, 13, 6, 7, 2, 1), (1, 4, 96, 97, 68, 3, 1, 1), (3, 16, 7, 9, 12, 3, 1, 4), (1, 4, 5, 3, 66, 1, 1, 1),
