@@ -37,8 +37,9 @@ inline bool ragged_pays(int g_ic, int taps, int g_oc, int64_t pixels) {
 
 // The tile of at most `pix` output pixels (32 at most side by side) that covers an out_h x out_w image in the fewest blocks, rows
 // and columns spread evenly over them; among equals the one with the smallest input, among those the widest (below four columns
-// the first that does no better ends the search).  span: what a window reads, its dilation included.  (Asked for on every launch, so it goes through tile widths, 32 at most, and not through all
-// numbers of tiles side by side: 0.7 -> 0.3 us for rows of 320 pixels, 2.1 -> 0.35 for 1280.)
+// the first that does no better ends the search).  span: what a window reads, its dilation included.  (Asked for on every launch,
+// so it goes through tile widths, 32 at most, and not through all numbers of tiles side by side: 0.7 -> 0.3 us for rows of 320
+// pixels, 2.1 -> 0.35 for 1280.)
 struct OutputTile {
     int th, tw;         // output pixels
     int across, down;   // tiles per image
@@ -62,6 +63,38 @@ inline OutputTile choose_output_tile(int out_h, int out_w, int pix, int stride_h
         best = OutputTile{th, tw, across, down, in_rows, in_cols};
     }
     return best;
+}
+
+// Whether a launch of the window kernel as planned is quicker than the implicit GEMM of the same layer (byte results, strides of 1
+// and 2, three k-steps and more, stride 2 sixteen).  us, implicit GEMM / window kernel:
+//   * tiles that images do not fill by half stay, their surplus pixels are multiplied and dropped; with fewer than three waves per
+//     compute unit a sixth is too much (3388 pixels 256 -> 170 in two groups, 63 % full, 12.1 / 14.4)
+//   * with fewer than three waves per two compute units (stride 2: four per unit) the k-steps split over groups of waves win
+//     (400 pixels 256 -> 256 7.1 / 7.5; 1600 pixels 128 -> 256 stride 2 5.8 / 6.8)
+//   * blocks of two waves have to leave room in LDS for four of a compute unit, with stride 2, whose staging is four times as long,
+//     for five: 560 -> 32 3x3 of 40 344 pixels 27.4 / 34.2, stride 2 400 -> 320 of 11 664 33.8 / 55.4, 128 -> 32 of 147 456
+//     28.7 / 57.1; blocks of 128 pixels at stride 1 win with what fits (80 -> 32 5x5 of 149 187 37.9 / 19.0), blocks of eight
+//     waves with one per compute unit (128 -> 128 7x7 stride 2 of 56 448 78.5 / 55.7)
+//   * 32 pixels per block are too few where a short reduction meets a launch many times what the device holds: 16 -> 64 3x3, three
+//     k-steps, of 143 648 pixels 11.9 / 17.3 a group, 64 -> 64 of 421 362 39.0 / 46.2 (but of 102 400 12.7 / 11.5)
+// (Of 750 windows over 1000 to 700 000 pixels, 349 of them planned here, the choice is 1.4 % off the quicker one in the mean and
+// loses more than 5 % to the implicit GEMM on 24, a quarter at most but for two groups of 16 -> 128, 8.4 / 10.8.)
+struct TileLaunch {
+    int stride_w, ksteps;
+    int pix, waves; // per block
+    size_t lds;
+    long long tiles, chunks, pixels;
+};
+inline bool tile_kernel_pays(const TileLaunch &l, int compute_units) {
+    const long long launched = l.tiles * l.chunks * l.waves, room = l.tiles * l.pix;
+    if (l.lds > 160 * 1024 || 2 * l.pixels < room) return false;
+    if (2 * launched < (l.stride_w == 2 ? 8 : 3) * (long long)compute_units) return false;
+    if (launched < 3 * (long long)compute_units && 20 * l.pixels < 17 * room) return false;
+    if (l.waves > 2) return true;
+    const size_t resident = 160 * 1024 / l.lds;
+    if (l.stride_w == 2 && resident < 5) return false;
+    if (l.pix < 128 && resident < 4) return false;
+    return l.pix > 32 || launched <= 9ll * l.ksteps * compute_units;
 }
 
 } // namespace nnhip

@@ -374,15 +374,14 @@ template <int T, int RG, int WM, int WN> TilePlan plan_shape(const IgemmArgs &a,
 // Which block, if any, by the packed chunk (`tiles` of 16 channels) and the waves the launch has (byte results, windows,
 // strides of 1 and 2).  Measured us, implicit GEMM / here, byte table behind the convolution:
 //   * eight waves share the staging of a 128-channel chunk: 25 600 pixels 128 -> 128 3x3 11.7 / 9.7 with 128 pixels per block
-//     (10.4 with 64), 6400 pixels 256 -> 256 11.8 / 9.2 with 64 (11.4 with 128: fewer blocks than compute units);
+//     (10.4 with 64), 6400 pixels 256 -> 256 11.8 / 9.2 with 64 (11.4 with 128: fewer blocks than compute units); three blocks of
+//     128 pixels for four compute units are enough (asked for twice as many, 750 windows lose 7 % where it makes a difference);
 //   * one wave row of 32 pixels for 64 channels: 102 400 pixels 64 -> 64 12.7 / 11.5 (13.9 with 128 pixels, 12.3 with 64);
 //   * 32 channels: 409 600 pixels 32 -> 32 21.9 / 15.6, 1 638 400 pixels 16 -> 32 41.4 / 36.7; two k-steps and fewer are the
 //     epilogue's work alone and stay (802 816 pixels 16 -> 32 2x2 14.9 / 18.6);
 //   * stride 2 brings in four times the input: from 16 k-steps on (25 600 pixels 128 -> 256 18.5 / 15.9, 6400 pixels 256 -> 512
 //     18.0 / 15.5, but 409 600 pixels 32 -> 64, five k-steps, 28.2 / 30.3);
-//   * tiles that images do not fill by half stay (their surplus pixels are multiplied and dropped);
-//   * with fewer than three waves per two compute units (stride 2: four per unit) the k-steps split over groups of waves win
-//     (400 pixels 256 -> 256 7.1 / 7.5; 1600 pixels 128 -> 256 stride 2 5.8 / 6.8).
+//   * and what tile_kernel_pays asks of the launch.
 TileShape choose_tile(const nncase_hip_ctx *ctx, const IgemmArgs &a, int tiles, int nchunks, TilePlan *plan) {
     if (a.kh * a.kw == 1 || a.g_ic % 16 != 0 || a.kc_mask != -1 || a.stride_w > 2 || (int64_t)a.in_w * a.ldx >= (1 << 23)) return kTileNone;
     if (a.ksteps < (a.stride_w == 2 ? 16 : 3)) return kTileNone;
@@ -402,10 +401,7 @@ TileShape choose_tile(const nncase_hip_ctx *ctx, const IgemmArgs &a, int tiles, 
         break;
     default: return kTileNone;
     }
-    if (2ll * a.m < (long long)plan->tiles * pix) return kTileNone;
-    const long long launched = (long long)plan->tiles * nchunks * waves;
-    if (2 * launched < (a.stride_w == 2 ? 8 : 3) * (long long)ctx->compute_units) return kTileNone;
-    return plan->lds <= 160 * 1024 ? shape : kTileNone;
+    return tile_kernel_pays(TileLaunch{a.stride_w, a.ksteps, pix, waves, plan->lds, plan->tiles, nchunks, a.m}, ctx->compute_units) ? shape : kTileNone;
 }
 } // namespace
 

@@ -1,6 +1,6 @@
 """How a dense layer of narrow or odd channel counts is packed, held against measured times (us on the device, u8 and float32
 outputs): the choice is no more than a fifth slower than the other.  And the output tile of the window kernel against its
-definition.  The rules are host arithmetic (csrc/qconv_rules.hpp), compiled here for the CPU."""
+definition, and where that kernel is launched.  The rules are host arithmetic (csrc/qconv_rules.hpp), compiled here for the CPU."""
 import ctypes as C
 import os
 import subprocess
@@ -18,6 +18,9 @@ extern "C" int pays(int ic, int taps, int oc, long px) { return nnhip::ragged_pa
 extern "C" void tile(int h, int w, int pix, int sh, int sw, int kh, int kw, int *out) {
     const nnhip::OutputTile t = nnhip::choose_output_tile(h, w, pix, sh, sw, kh, kw);
     out[0] = t.th, out[1] = t.tw, out[2] = t.across, out[3] = t.down, out[4] = t.in_rows, out[5] = t.in_cols;
+}
+extern "C" int window(int stride, int ksteps, int pix, int waves, long lds, long tiles, long chunks, long pixels) {
+    return nnhip::tile_kernel_pays({stride, ksteps, pix, waves, (size_t)lds, tiles, chunks, pixels}, 256);
 }
 """)
     subprocess.check_call(["g++", "-std=c++17", "-O2", "-shared", "-fPIC", "-I", CSRC, str(d / "r.cpp"), "-o", str(d / "r.so")])
@@ -120,3 +123,73 @@ def test_output_tile_is_the_best_of_all_numbers_of_tiles(rules, pix, stride, spa
                     break
             rules.tile(h, w, pix, stride, stride, span, span, got)
             assert list(got) == best[1], (h, w)
+
+
+# windows of a group's channels -> outputs, window side, stride; k-steps; pixels and waves per block, LDS, tiles, chunks, output pixels;
+# us by the implicit GEMM, us by the window kernel (all groups)
+WINDOWS = [
+    (336, 448, 3, 1, 48, 128, 8, 62560, 150, 4, 19200, 60.3, 39.9),
+    (384, 224, 5, 1, 150, 128, 8, 99712, 96, 2, 11907, 57.0, 37.9),
+    (80, 128, 3, 1, 12, 128, 8, 19936, 512, 1, 59168, 16.1, 12.1),
+    (64, 128, 5, 1, 25, 128, 8, 21072, 490, 1, 60025, 25.1, 20.9),
+    (80, 32, 5, 1, 32, 128, 2, 20640, 1176, 1, 149187, 37.9, 19.0),
+    (112, 32, 5, 1, 44, 128, 2, 29632, 4920, 1, 605160, 163.4, 84.0),
+    (96, 32, 3, 1, 14, 128, 2, 24000, 4620, 1, 570288, 62.2, 37.9),
+    (16, 18, 5, 1, 7, 128, 2, 7184, 2210, 1, 271445, 39.9, 28.4),
+    (16, 64, 3, 1, 3, 32, 2, 3280, 9248, 1, 287296, 23.8, 34.5),
+    (16, 64, 3, 1, 3, 32, 2, 3280, 5082, 1, 155232, 15.9, 21.3),
+    (528, 320, 3, 1, 75, 32, 2, 33552, 56, 5, 1444, 11.8, 14.5),
+    (240, 46, 5, 1, 94, 32, 2, 23296, 270, 1, 6615, 13.6, 16.4),
+    (64, 64, 3, 1, 9, 32, 2, 8736, 13770, 1, 421362, 39.0, 46.2),
+    (16, 149, 3, 1, 3, 32, 2, 3280, 1386, 3, 36982, 20.0, 23.7),
+    (128, 64, 3, 1, 18, 32, 2, 9600, 1058, 1, 33856, 12.0, 8.6),
+    (80, 64, 3, 1, 12, 32, 2, 6624, 2310, 1, 71148, 13.4, 9.7),
+    (32, 320, 3, 1, 5, 32, 2, 3440, 168, 5, 4356, 6.0, 4.8),
+    (16, 48, 7, 1, 13, 32, 2, 3440, 322, 1, 9522, 6.1, 5.2),
+    (32, 240, 7, 1, 25, 64, 8, 12256, 84, 2, 4332, 9.5, 7.0),
+    (96, 255, 7, 1, 74, 64, 8, 28448, 119, 2, 6800, 21.2, 16.4),
+    (192, 128, 3, 1, 27, 64, 8, 22288, 180, 1, 9680, 10.4, 8.7),
+    (80, 208, 3, 1, 12, 64, 8, 10464, 84, 2, 4375, 7.1, 6.2),
+    (528, 96, 2, 1, 33, 64, 2, 35520, 90, 3, 4320, 7.9, 11.5),
+    (304, 16, 3, 1, 43, 64, 2, 28112, 264, 1, 14256, 8.9, 11.8),
+    (560, 32, 3, 1, 79, 64, 2, 66336, 672, 1, 40344, 27.4, 34.2),
+    (128, 85, 3, 1, 18, 64, 2, 12192, 84, 3, 3388, 12.1, 14.4),
+    (528, 16, 2, 1, 33, 64, 2, 43440, 360, 1, 18750, 10.6, 12.4),
+    (512, 32, 3, 1, 72, 64, 2, 52512, 225, 1, 12615, 12.3, 14.4),
+    (80, 22, 5, 1, 32, 64, 2, 13984, 945, 1, 56307, 33.9, 21.5),
+    (16, 15, 7, 1, 13, 64, 2, 4768, 880, 1, 53138, 9.6, 6.5),
+    (32, 32, 3, 1, 5, 64, 2, 5504, 663, 1, 39675, 5.9, 4.9),
+    (96, 32, 5, 1, 38, 64, 2, 17408, 363, 1, 21675, 11.4, 10.1),
+    (48, 272, 7, 2, 37, 128, 8, 38192, 208, 3, 21866, 49.9, 32.5),
+    (64, 256, 7, 2, 49, 128, 8, 65936, 108, 2, 13254, 24.0, 16.9),
+    (64, 128, 7, 2, 49, 128, 8, 67376, 672, 1, 84672, 59.1, 44.7),
+    (192, 512, 3, 2, 27, 128, 8, 121968, 48, 4, 6144, 15.8, 13.2),
+    (128, 32, 3, 2, 18, 128, 2, 84448, 1152, 1, 147456, 28.7, 57.0),
+    (400, 320, 3, 2, 57, 32, 2, 66384, 405, 5, 11664, 33.8, 55.4),
+    (432, 48, 3, 2, 61, 32, 2, 71632, 612, 1, 17956, 19.2, 29.1),
+    (288, 48, 3, 2, 41, 32, 2, 48144, 1071, 1, 29988, 16.3, 24.6),
+    (192, 184, 3, 2, 27, 32, 2, 33136, 1071, 3, 29988, 25.0, 34.1),
+    (368, 128, 2, 2, 23, 32, 2, 45200, 266, 2, 6859, 8.7, 11.9),
+    (288, 64, 5, 2, 113, 32, 2, 69360, 720, 1, 23040, 29.4, 39.4),
+    (32, 448, 7, 2, 25, 32, 2, 14800, 198, 7, 5808, 15.8, 12.1),
+    (48, 448, 5, 2, 19, 32, 2, 10480, 108, 7, 2601, 9.4, 7.5),
+    (160, 64, 3, 2, 23, 32, 2, 30960, 1950, 1, 60840, 18.6, 20.9),
+    (224, 480, 3, 2, 32, 64, 8, 63968, 60, 4, 3240, 12.2, 10.0),
+    (368, 128, 5, 2, 144, 64, 8, 143200, 196, 1, 11881, 33.1, 27.5),
+    (128, 96, 3, 2, 18, 64, 8, 45696, 224, 1, 13778, 8.5, 7.5),
+    (240, 208, 5, 2, 94, 64, 2, 75616, 92, 7, 3887, 22.8, 38.0),
+    (288, 32, 2, 2, 18, 64, 2, 78784, 833, 1, 51425, 15.5, 24.9),
+    (192, 32, 7, 2, 147, 64, 2, 105776, 1380, 1, 82810, 101.9, 131.3),
+    (112, 16, 3, 2, 16, 64, 2, 32960, 540, 1, 32400, 7.7, 8.7),
+]
+
+
+@pytest.mark.parametrize("row", WINDOWS, ids=lambda r: "%d-%d-%dx%d-s%d-%d" % (r[0], r[1], r[2], r[2], r[3], r[10]))
+def test_windows_take_the_quicker_kernel(rules, row):
+    ic, oc, k, stride, ksteps, pix, waves, lds, tiles, chunks, pixels, gemm, window = row
+    assert (window if rules.window(stride, ksteps, pix, waves, C.c_long(lds), C.c_long(tiles), C.c_long(chunks), C.c_long(pixels)) else gemm) <= 1.2 * min(gemm, window)
+
+
+def test_window_kernel_is_not_launched_beyond_the_lds(rules):
+    args = lambda lds: (1, 40, 128, 8, C.c_long(lds), C.c_long(4000), C.c_long(1), C.c_long(500000))
+    assert rules.window(*args(160 * 1024)) and not rules.window(*args(160 * 1024 + 16))
