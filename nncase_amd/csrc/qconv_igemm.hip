@@ -43,17 +43,6 @@ static void plan_igemm(int g_oc, int ksteps, int64_t pixels_hint, int compute_un
     *kc_steps = best_kc;
 }
 
-// From how many k-steps of 64 a layer of whole 16-channel slices takes the small wide blocks.  Four, since their fetch of whole
-// rows beats the small tiles' slices by then (25 600 pixels 256 -> 256 1x1 10.1 -> 9.4 us) but not before (102 400 pixels
-// 128 -> 128 11.4 / 12.8, 200 704 pixels 144 -> 24 8.9 / 10.3).  Two where the outputs are what the launch is made of: channel
-// counts that are no multiple of 4, whose rows only the wide kernel's whole-row stores keep together (102 400 pixels 128 -> 255
-// 44.4 -> 28.8 us, to floats 41.2 -> 29.3), and many outputs over more than 128 channels, where the small tiles would read the
-// activations once per chunk (32 768 rows 192 -> 1000 34.7 -> 26.8; but 4096 rows 128 -> 512 4.6 / 5.0).
-static int small_wide_min_ksteps(int g_oc, int64_t pixels) {
-    const bool store_bound = g_oc % 4 != 0 || (g_oc > 128 && pixels * g_oc >= (int64_t)8 << 20);
-    return g_oc > 64 && store_bound ? 2 : kSmallWideMinKsteps;
-}
-
 int igemm_plan(nncase_hip_ctx *ctx, nncase_hip_weights *w, const int32_t *bias) {
     const int taps = w->kernel_h * w->kernel_w;
     NNHIP_REQUIRE(ctx, (int64_t)taps * w->g_ic < 65536, -EINVAL,
@@ -85,10 +74,10 @@ int igemm_plan(nncase_hip_ctx *ctx, nncase_hip_weights *w, const int32_t *bias) 
             w->kc_steps = std::min(w->ksteps, kLdsFrags / w->tiles);
         }
     }
-    // Reductions of kSmallWideMinKsteps k-steps and more over fewer pixels take the same kernel with blocks of 8192 or 2048
-    // outputs: against the small tiles' per-lane loads of 16 pixels' slices, the row-order fetch through LDS needs a
+    // Reductions of five k-steps and more over fewer pixels, and some shorter ones, take the same kernel with blocks of 8192 or
+    // 2048 outputs: against the small tiles' per-lane loads of 16 pixels' slices, the row-order fetch through LDS needs a
     // quarter of the requests to the vector L1, which is what such launches are bound by.
-    if (!w->wide && (w->ragged || (w->g_ic % 16 == 0 && w->ksteps >= small_wide_min_ksteps(w->g_oc, w->pixels_hint)))) {
+    if (!w->wide && (w->ragged || (w->g_ic % 16 == 0 && small_wide_pays(w->g_oc, w->ksteps, w->tiles, w->pixels_hint)))) {
         w->wide = 2;
         // (2048 outputs per block while the larger ones would leave more than half of the compute units without a block:
         // the 512 x 1024 x 1024 product takes 7.0 us with them, 9.2 us with 64 blocks of 8192)

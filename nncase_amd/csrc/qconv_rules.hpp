@@ -35,6 +35,26 @@ inline bool ragged_pays(int g_ic, int taps, int g_oc, int64_t pixels) {
     return g_ic > 48 || taps == 1 || outputs >= 70000 || pixels >= 6000;
 }
 
+// Whether a reduction of two to four k-steps (of 64) whose channels are whole 16-channel slices takes the small wide blocks and not
+// the small tiles; longer ones always do, one k-step never.  `tiles`: the 16-channel tiles per chunk that the small tiles would be
+// packed with; `pixels`: of the launches to come, 0 = unknown.  The small tiles hold a chunk's accumulators and its weights per
+// block: up to seven tiles they are the lighter ones (a tenth quicker in the mean: 53 621 pixels 48 -> 16 2x2 4.1 / 4.6, 86 528 of
+// 160 -> 96 1x1 6.8 / 10.5), from eight on they are bound by how few of them are resident.  us, small tiles / wide blocks:
+//   * 54 450 pixels 192 -> 224 1x1 24.9 / 12.1, 47 628 of 80 -> 224 17.9 / 10.2, 32 768 rows 192 -> 1000 34.7 / 26.8, to floats
+//     38 025 of 128 -> 160 14.1 / 11.5
+//   * but many pixels for their outputs fill the device with small tiles too: 205 209 pixels 128 -> 128 1x1 13.4 / 19.1, 187 272 of
+//     48 -> 192 2x2 27.1 / 35.2 (to floats the wide blocks still win there, 217 800 of 16 -> 160 3x3 50.8 / 45.5; which of the two a
+//     layer will write is not known when its weights are packed)
+//   * unless the channel count is no multiple of 4, whose rows only the wide blocks' whole-row stores keep together (102 400 pixels
+//     128 -> 255 44.4 / 28.8, to floats 41.2 / 29.3)
+// (Of 777 such layers the choice is 1.5 % off the quicker one in the mean and loses more than 5 % to the small tiles on 15, 28 % at
+// most, 13 456 pixels 128 -> 320 4.7 / 6.0.)
+inline bool small_wide_pays(int g_oc, int ksteps, int tiles, int64_t pixels) {
+    if (ksteps >= 5) return true;
+    if (ksteps < 2 || tiles < 8) return false;
+    return pixels < 300ll * g_oc || (g_oc % 4 != 0 && g_oc > 128);
+}
+
 // The tile of at most `pix` output pixels (32 at most side by side) that covers an out_h x out_w image in the fewest blocks, rows
 // and columns spread evenly over them; among equals the one with the smallest input, among those the widest (below four columns
 // the first that does no better ends the search).  span: what a window reads, its dilation included.  (Asked for on every launch,

@@ -39,7 +39,6 @@ namespace nnhip {
 // block per compute unit; below that a launch has too few 64-pixel wave tiles to fill the device and the small tiles'
 // larger wave count wins.
 constexpr int kWideMinKsteps = 8;
-constexpr int kSmallWideMinKsteps = 4; // (igemm_plan decides between the small tiles and the small wide blocks)
 constexpr int kWideSlots = 3;
 
 // How a thread finds its 16-byte pieces of a k-step:

@@ -19,6 +19,7 @@ extern "C" void tile(int h, int w, int pix, int sh, int sw, int kh, int kw, int 
     const nnhip::OutputTile t = nnhip::choose_output_tile(h, w, pix, sh, sw, kh, kw);
     out[0] = t.th, out[1] = t.tw, out[2] = t.across, out[3] = t.down, out[4] = t.in_rows, out[5] = t.in_cols;
 }
+extern "C" int wide(int oc, int ksteps, int tiles, long px) { return nnhip::small_wide_pays(oc, ksteps, tiles, px); }
 extern "C" int window(int stride, int ksteps, int pix, int waves, long lds, long tiles, long chunks, long pixels) {
     return nnhip::tile_kernel_pays({stride, ksteps, pix, waves, (size_t)lds, tiles, chunks, pixels}, 256);
 }
@@ -193,3 +194,73 @@ def test_windows_take_the_quicker_kernel(rules, row):
 def test_window_kernel_is_not_launched_beyond_the_lds(rules):
     args = lambda lds: (1, 40, 128, 8, C.c_long(lds), C.c_long(4000), C.c_long(1), C.c_long(500000))
     assert rules.window(*args(160 * 1024)) and not rules.window(*args(160 * 1024 + 16))
+
+
+# a group's channels -> outputs, window side, k-steps, the small tiles' 16-channel tiles per chunk, output pixels; us by the small tiles,
+# us by the small wide blocks (all groups)
+SHORT = [
+    (32, 160, 2, 2, 5, 21780, 4.7, 6.7),
+    (112, 224, 1, 2, 2, 4840, 3.3, 4.7),
+    (112, 256, 1, 2, 4, 10000, 3.8, 5.2),
+    (128, 64, 1, 2, 4, 50784, 4.3, 5.4),
+    (32, 22, 2, 2, 2, 137917, 7.4, 8.9),
+    (112, 224, 1, 2, 1, 2704, 3.8, 4.4),
+    (128, 128, 1, 2, 8, 205209, 13.4, 19.1),
+    (96, 256, 1, 2, 16, 191646, 25.0, 31.4),
+    (80, 224, 1, 2, 16, 47628, 17.9, 10.2),
+    (128, 432, 1, 2, 16, 58800, 32.5, 19.1),
+    (80, 208, 1, 2, 16, 34810, 26.7, 17.8),
+    (112, 512, 1, 2, 12, 15123, 10.2, 7.2),
+    (112, 336, 1, 2, 8, 12996, 8.3, 6.6),
+    (128, 384, 1, 2, 12, 25047, 7.9, 9.4),
+    (160, 96, 1, 3, 6, 86528, 6.8, 10.5),
+    (192, 160, 1, 3, 4, 11236, 3.8, 5.4),
+    (144, 128, 1, 3, 4, 20181, 4.0, 5.6),
+    (16, 32, 3, 3, 1, 5488, 6.5, 8.2),
+    (144, 9, 1, 3, 1, 325, 5.9, 7.0),
+    (192, 124, 1, 3, 1, 3600, 6.4, 7.3),
+    (192, 128, 1, 3, 8, 223093, 17.9, 24.5),
+    (144, 128, 1, 3, 8, 257193, 18.8, 25.2),
+    (48, 192, 2, 3, 12, 187272, 27.1, 35.2),
+    (16, 160, 3, 3, 10, 217800, 50.8, 45.5),
+    (16, 160, 3, 3, 10, 134064, 34.8, 31.2),
+    (192, 224, 1, 3, 16, 54450, 24.9, 12.1),
+    (16, 241, 3, 3, 16, 39605, 21.9, 12.7),
+    (16, 512, 3, 3, 12, 15606, 18.8, 12.4),
+    (16, 624, 3, 3, 16, 52900, 52.0, 38.4),
+    (192, 375, 1, 3, 12, 27378, 15.9, 12.8),
+    (192, 150, 1, 3, 10, 84270, 27.1, 23.8),
+    (256, 160, 1, 4, 5, 24548, 5.7, 8.4),
+    (208, 32, 1, 4, 2, 91875, 7.0, 9.8),
+    (240, 96, 1, 4, 3, 24304, 4.6, 6.4),
+    (240, 160, 1, 4, 1, 252, 3.1, 3.8),
+    (256, 64, 1, 4, 4, 126350, 13.8, 16.2),
+    (256, 256, 1, 4, 1, 882, 3.3, 3.8),
+    (256, 144, 1, 4, 9, 84050, 11.9, 17.0),
+    (208, 288, 1, 4, 9, 159048, 35.0, 44.3),
+    (256, 192, 1, 4, 12, 154568, 23.5, 29.7),
+    (208, 128, 1, 4, 8, 41616, 6.0, 7.4),
+    (240, 128, 1, 4, 8, 40804, 12.4, 10.6),
+    (64, 192, 2, 4, 12, 231125, 37.4, 42.3),
+    (256, 512, 1, 4, 12, 21952, 17.7, 12.3),
+    (64, 512, 2, 4, 12, 15129, 14.4, 10.2),
+    (256, 496, 1, 4, 12, 32400, 23.4, 16.7),
+    (64, 448, 2, 4, 10, 97468, 70.6, 53.6),
+    (256, 512, 1, 4, 12, 42237, 28.8, 22.6),
+    (64, 205, 2, 4, 8, 136107, 53.3, 45.6),
+    (128, 255, 1, 2, 16, 102400, 44.4, 28.8),
+    (192, 1000, 1, 3, 16, 32768, 34.7, 26.8),
+    (144, 24, 1, 3, 2, 200704, 8.9, 10.3),
+]
+
+
+@pytest.mark.parametrize("row", SHORT, ids=lambda r: "%d-%d-%dx%d-%d" % (r[0], r[1], r[2], r[2], r[5]))
+def test_short_reductions_take_the_quicker_kernel(rules, row):
+    ic, oc, k, ksteps, tiles, pixels, small, wide = row
+    assert (wide if rules.wide(oc, ksteps, tiles, C.c_long(pixels)) else small) <= 1.2 * min(small, wide)
+
+
+def test_reductions_without_a_choice_of_blocks(rules):
+    for oc in (1, 64, 255, 1000):
+        for px in (0, 1, 1 << 22):
+            assert rules.wide(oc, 5, 1, C.c_long(px)) and not rules.wide(oc, 1, 16, C.c_long(px))
