@@ -129,6 +129,8 @@ def test_output_tile_is_the_best_of_all_numbers_of_tiles(rules, pix, stride, spa
 # windows of a group's channels -> outputs, window side, stride; k-steps; pixels and waves per block, LDS, tiles, chunks, output pixels;
 # us by the implicit GEMM, us by the window kernel (all groups)
 WINDOWS = [
+    (16, 128, 3, 1, 3, 32, 2, 3280, 765, 2, 22445, 8.4, 10.8),
+    (32, 316, 3, 1, 5, 32, 2, 5600, 3366, 5, 104907, 36.6, 40.1),
     (336, 448, 3, 1, 48, 128, 8, 62560, 150, 4, 19200, 60.3, 39.9),
     (384, 224, 5, 1, 150, 128, 8, 99712, 96, 2, 11907, 57.0, 37.9),
     (80, 128, 3, 1, 12, 128, 8, 19936, 512, 1, 59168, 16.1, 12.1),
