@@ -77,7 +77,7 @@ int igemm_plan(nncase_hip_ctx *ctx, nncase_hip_weights *w, const int32_t *bias) 
     // Reductions of five k-steps and more over fewer pixels, and some shorter ones, take the same kernel with blocks of 8192 or
     // 2048 outputs: against the small tiles' per-lane loads of 16 pixels' slices, the row-order fetch through LDS needs a
     // quarter of the requests to the vector L1, which is what such launches are bound by.
-    if (!w->wide && (w->ragged || (w->g_ic % 16 == 0 && small_wide_pays(w->g_oc, w->ksteps, w->tiles, w->pixels_hint)))) {
+    if (!w->wide && (w->ragged || (w->g_ic % 16 == 0 && small_wide_pays(w->g_oc, w->ksteps, w->tiles)))) {
         w->wide = 2;
         // (2048 outputs per block while the larger ones would leave more than half of the compute units without a block:
         // the 512 x 1024 x 1024 product takes 7.0 us with them, 9.2 us with 64 blocks of 8192)

@@ -37,22 +37,19 @@ inline bool ragged_pays(int g_ic, int taps, int g_oc, int64_t pixels) {
 
 // Whether a reduction of two to four k-steps (of 64) whose channels are whole 16-channel slices takes the small wide blocks and not
 // the small tiles; longer ones always do, one k-step never.  `tiles`: the 16-channel tiles per chunk that the small tiles would be
-// packed with; `pixels`: of the launches to come, 0 = unknown.  The small tiles hold a chunk's accumulators and its weights per
-// block: up to seven tiles they are the lighter ones (a tenth quicker in the mean: 53 621 pixels 48 -> 16 2x2 4.1 / 4.6, 86 528 of
-// 160 -> 96 1x1 6.8 / 10.5), from eight on they are bound by how few of them are resident.  us, small tiles / wide blocks:
-//   * 54 450 pixels 192 -> 224 1x1 24.9 / 12.1, 47 628 of 80 -> 224 17.9 / 10.2, 32 768 rows 192 -> 1000 34.7 / 26.8, to floats
-//     38 025 of 128 -> 160 14.1 / 11.5
-//   * but many pixels for their outputs fill the device with small tiles too: 205 209 pixels 128 -> 128 1x1 13.4 / 19.1, 187 272 of
-//     48 -> 192 2x2 27.1 / 35.2 (to floats the wide blocks still win there, 217 800 of 16 -> 160 3x3 50.8 / 45.5; which of the two a
-//     layer will write is not known when its weights are packed)
-//   * unless the channel count is no multiple of 4, whose rows only the wide blocks' whole-row stores keep together (102 400 pixels
-//     128 -> 255 44.4 / 28.8, to floats 41.2 / 29.3)
-// (Of 777 such layers the choice is 1.5 % off the quicker one in the mean and loses more than 5 % to the small tiles on 15, 28 % at
-// most, 13 456 pixels 128 -> 320 4.7 / 6.0.)
-inline bool small_wide_pays(int g_oc, int ksteps, int tiles, int64_t pixels) {
-    if (ksteps >= 5) return true;
-    if (ksteps < 2 || tiles < 8) return false;
-    return pixels < 300ll * g_oc || (g_oc % 4 != 0 && g_oc > 128);
+// packed with.  Those write a chunk whose lanes (a quarter of it each) all hold real channels with their short epilogue, and then are
+// the quicker ones whatever the size (205 209 pixels 128 -> 128 1x1 13.4 us, wide blocks 19.1; 154 568 of 256 -> 192 23.5 / 29.7;
+// 12 544 of 96 -> 576 6.4 / 7.1); with other channel counts their stores are piecemeal, where the wide blocks write whole rows: us,
+// small tiles / wide blocks, by tiles
+//   * 4 and fewer: a tenth quicker on the small tiles in the mean, 357 309 pixels 80 -> 45 1x1 20.0 / 27.4
+//   * 5 and 6: a tenth slower, 9464 pixels 112 -> 321 to floats 10.2 / 8.1
+//   * 8 and more: a quarter slower, 54 450 pixels 192 -> 224 1x1 24.9 / 12.1, 32 768 rows 192 -> 1000 34.7 / 26.8, 102 400 pixels
+//     128 -> 255 44.4 / 28.8
+// (Float32 results, of which a layer's weights know nothing when they are packed, would take the wide blocks in whole chunks too:
+// 40 095 pixels 128 -> 320 23.1 / 16.9.  Of 1350 such layers, a quarter of them to floats, the choice is 1.3 % off the quicker one in the
+// mean and loses more than 5 % to the small tiles on 13, 16 % at most.)
+inline bool small_wide_pays(int g_oc, int ksteps, int tiles) {
+    return ksteps >= 5 || (ksteps >= 2 && tiles >= 5 && g_oc % (4 * tiles) != 0);
 }
 
 // The tile of at most `pix` output pixels (32 at most side by side) that covers an out_h x out_w image in the fewest blocks, rows
