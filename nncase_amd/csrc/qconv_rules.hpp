@@ -88,18 +88,20 @@ inline OutputTile choose_output_tile(int out_h, int out_w, int pix, int stride_h
 //     compute unit a sixth is too much (3388 pixels 256 -> 170 in two groups, 63 % full, 12.1 / 14.4)
 //   * with fewer than three waves per two compute units (stride 2: four per unit) the k-steps split over groups of waves win
 //     (400 pixels 256 -> 256 7.1 / 7.5; 1600 pixels 128 -> 256 stride 2 5.8 / 6.8)
-//   * blocks of two waves have to leave room in LDS for four of a compute unit, with stride 2, whose staging is four times as long,
-//     for five: 560 -> 32 3x3 of 40 344 pixels 27.4 / 34.2, stride 2 400 -> 320 of 11 664 33.8 / 55.4, 128 -> 32 of 147 456
-//     28.7 / 57.1; blocks of 128 pixels at stride 1 win with what fits (80 -> 32 5x5 of 149 187 37.9 / 19.0), blocks of eight
-//     waves with one per compute unit (128 -> 128 7x7 stride 2 of 56 448 78.5 / 55.7)
+//   * blocks of two waves have to leave room in LDS for four of a compute unit from 400 channels on (560 -> 32 3x3 of 40 344 pixels
+//     27.4 / 34.2, 512 -> 48 5x5 of 18 150 41.9 / 49.0; up to there three are enough: 256 -> 32 5x5 of 85 264 61.4 / 43.6), and for
+//     five with stride 2, whose staging is four times as long (400 -> 320 of 11 664 33.8 / 55.4, 128 -> 32 of 147 456 28.7 / 57.1);
+//     blocks of 128 pixels at stride 1 win with what fits (80 -> 32 5x5 of 149 187 37.9 / 19.0), blocks of eight waves with one
+//     per compute unit (128 -> 128 7x7 stride 2 of 56 448 78.5 / 55.7)
 //   * 32 pixels per block do not pay for the staging of less than five k-steps (22 445 pixels 16 -> 128 3x3 in two groups 8.4 / 10.8,
 //     64 -> 64 2x2 of 35 301 4.6 / 5.9, 16 -> 64 3x3 of 287 296 11.9 / 17.3), and are too few where a short reduction meets a launch
 //     many times what the device holds: 64 -> 64 of 421 362 39.0 / 46.2, 32 -> 316 of 104 907 36.6 / 40.1 (but 64 -> 64 of 102 400
 //     12.7 / 11.5)
-// (Of 750 windows over 1000 to 700 000 pixels, 380 of them planned here, the choice is 1.3 % off the quicker one in the mean and
-// loses more than 5 % to the implicit GEMM on 23, a quarter at most.)
+// (Of 660 launches planned here, of windows over 1000 to 700 000 pixels, the choice is 1.1 % off the quicker one in the mean and
+// loses more than 5 % to the implicit GEMM on 44, 30 % at most.)
 struct TileLaunch {
     int stride_w, ksteps;
+    int channels;   // of a group's input
     int pix, waves; // per block
     size_t lds;
     long long tiles, chunks, pixels;
@@ -112,7 +114,7 @@ inline bool tile_kernel_pays(const TileLaunch &l, int compute_units) {
     if (l.waves > 2) return true;
     const size_t resident = 160 * 1024 / l.lds;
     if (l.stride_w == 2 && resident < 5) return false;
-    if (l.pix < 128 && resident < 4) return false;
+    if (l.pix < 128 && l.channels > 400 && resident < 4) return false;
     return l.pix > 32 || (l.ksteps >= 5 && launched <= 9ll * l.ksteps * compute_units);
 }
 

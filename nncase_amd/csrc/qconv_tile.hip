@@ -401,7 +401,7 @@ TileShape choose_tile(const nncase_hip_ctx *ctx, const IgemmArgs &a, int tiles, 
         break;
     default: return kTileNone;
     }
-    return tile_kernel_pays(TileLaunch{a.stride_w, a.ksteps, pix, waves, plan->lds, plan->tiles, nchunks, a.m}, ctx->compute_units) ? shape : kTileNone;
+    return tile_kernel_pays(TileLaunch{a.stride_w, a.ksteps, a.g_ic, pix, waves, plan->lds, plan->tiles, nchunks, a.m}, ctx->compute_units) ? shape : kTileNone;
 }
 } // namespace
 
