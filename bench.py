@@ -45,51 +45,54 @@ MEASURED_TRAFFIC_SOURCE = {"unfused": "profiles/mobilenetv2_b64_kernels_counters
                            "fused": "profiles/mobilenetv2_b64_fused_blocks_kernels_counters.txt"}
 MEASURED_TRAFFIC_B64 = {
     "unfused": {
-        "dw3x3<S=1>": 19011936,
-        "dw3x3<S=2>": 41883762,
-        "qconv_igemm+add<T=2,RG=1,rows16>": 13054633,
-        "qconv_igemm+add<T=2,RG=2,rows16>": 40563268,
-        "qconv_igemm<T=1,RG=1,rows16>": 3359320,
-        "qconv_igemm<T=1,RG=4,rows16>": 38602230,
+        "dw3x3<S=1>": 19019002,
+        "dw3x3<S=2>": 41946024,
+        "qconv_igemm+add<T=2,RG=1,rows16>": 13050524,
+        "qconv_igemm+add<T=2,RG=2,rows16>": 39707981,
+        "qconv_igemm<T=1,RG=1,rows16>": 3359321,
+        "qconv_igemm<T=1,RG=4,rows16>": 38602078,
         "qconv_igemm<T=12,RG=1,rows16>": 10267976,
-        "qconv_igemm<T=2,RG=1,rows16>": 8930024,
-        "qconv_igemm<T=2,RG=2,rows16>": 24171978,
-        "qconv_igemm<T=2,RG=2,vec16>": 38626465,
-        "qconv_igemm<T=5,RG=1,rows16>": 5099510,
-        "qconv_igemm<T=6,RG=2,rows16>": 90023774,
-        "qconv_igemm<T=8,RG=1,rows16>": 5904294,
-        "qconv_igemm<T=9,RG=1,rows8>": 34301598,
-        "qconv_wide+add<T=2,RG=2,rows16>": 6175918,
-        "qconv_wide+add<T=4,RG=2,rows16>": 10530291,
-        "qconv_wide+dequantize<T=2,RG=2,rows16>": 1710972,
-        "qconv_wide<T=2,RG=2,rows16>": 4725052,
-        "qconv_wide<T=4,RG=2,rows16>": 7450706,
-        "qglobal_avgpool": 4238843,
-        "quantize+pack": 51434794,
+        "qconv_igemm<T=2,RG=1,rows16>": 8930245,
+        "qconv_igemm<T=2,RG=2,rows16>": 24173738,
+        "qconv_igemm<T=2,RG=2,vec16>": 38626640,
+        "qconv_igemm<T=5,RG=1,rows16>": 5105644,
+        "qconv_igemm<T=6,RG=2,rows16>": 90037963,
+        "qconv_igemm<T=8,RG=1,rows16>": 5904417,
+        "qconv_igemm<T=9,RG=1,rows8>": 34301187,
+        "qconv_wide+add<T=2,RG=2,rows16>": 5254254,
+        "qconv_wide+add<T=4,RG=2,rows16>": 6800189,
+        "qconv_wide+add<T=8,RG=2,rows16>": 10557941,
+        "qconv_wide+dequantize<T=4,RG=2,rows16>": 3046450,
+        "qconv_wide<T=2,RG=2,rows16>": 3118543,
+        "qconv_wide<T=4,RG=2,rows16>": 6669399,
+        "qconv_wide<T=8,RG=2,rows16>": 7448863,
+        "qglobal_avgpool": 4240549,
+        "quantize+pack": 51436394,
     },
     "fused": {
-        "dw3x3<S=1>": 27882249,
-        "dw3x3<S=2>": 51731083,
-        "qblock+add<S=1,P=2>": 4954955,
-        "qblock+add<S=1,P=4>": 2669235,
-        "qblock+add<S=1,P=6>": 4553259,
-        "qblock<S=1,P=6>": 3246740,
-        "qblock<S=2,P=4>": 3355417,
-        "qconv_igemm+add<T=2,RG=2,rows16>": 39841988,
-        "qconv_igemm<T=1,RG=4,rows16>": 38602966,
-        "qconv_igemm<T=12,RG=1,rows16>": 9114287,
-        "qconv_igemm<T=2,RG=1,rows16>": 8914666,
-        "qconv_igemm<T=2,RG=2,rows16>": 24176233,
-        "qconv_igemm<T=2,RG=2,vec16>": 38614243,
-        "qconv_igemm<T=5,RG=1,rows16>": 5104363,
-        "qconv_igemm<T=6,RG=2,rows16>": 90039131,
-        "qconv_igemm<T=9,RG=1,rows8>": 34300750,
-        "qconv_wide+add<T=2,RG=2,rows16>": 5250994,
-        "qconv_wide+dequantize<T=2,RG=2,rows16>": 1710205,
-        "qconv_wide<T=2,RG=2,rows16>": 4714430,
-        "qconv_wide<T=4,RG=2,rows16>": 8201110,
-        "qglobal_avgpool": 4238971,
-        "quantize+pack": 51434890,
+        "dw3x3<S=1>": 27926481,
+        "dw3x3<S=2>": 51820711,
+        "qblock+add<S=1,P=2>": 4954137,
+        "qblock+add<S=1,P=4>": 2661070,
+        "qblock+add<S=1,P=6>": 4560536,
+        "qblock<S=1,P=6>": 3253935,
+        "qblock<S=2,P=4>": 3354545,
+        "qconv_igemm+add<T=2,RG=2,rows16>": 39743849,
+        "qconv_igemm<T=1,RG=4,rows16>": 38602486,
+        "qconv_igemm<T=12,RG=1,rows16>": 9126599,
+        "qconv_igemm<T=2,RG=1,rows16>": 8930252,
+        "qconv_igemm<T=2,RG=2,rows16>": 24173373,
+        "qconv_igemm<T=2,RG=2,vec16>": 38626951,
+        "qconv_igemm<T=5,RG=1,rows16>": 5105504,
+        "qconv_igemm<T=6,RG=2,rows16>": 90037292,
+        "qconv_igemm<T=9,RG=1,rows8>": 34301982,
+        "qconv_wide+add<T=2,RG=2,rows16>": 5254258,
+        "qconv_wide+dequantize<T=4,RG=2,rows16>": 3046453,
+        "qconv_wide<T=2,RG=2,rows16>": 3119911,
+        "qconv_wide<T=4,RG=2,rows16>": 6669404,
+        "qconv_wide<T=8,RG=2,rows16>": 8173012,
+        "qglobal_avgpool": 4240297,
+        "quantize+pack": 51436601,
     },
 }
 
