@@ -19,8 +19,8 @@ inline bool ragged_tile_pays(int es, uint32_t la, uint64_t plain, uint64_t packe
 }
 // Whether packing reads rows of whole dwords, but not of whole 16-byte pieces, in unaligned pieces and the smaller tiles (true) or
 // dword by dword.  us, dwords / pieces: u8 75 x 38 x 38 by 32 5.9 / 4.1, float32 155 x 51 x 51 by 32 6.4 / 4.5; but 4 lanes of
-// float16 8 x 155 x 150 x 150 28.2 / 35.9, a lane group of less than a tile, u8 75 x 14 x 14 by 16, 3.7 / 4.0, and past 16 MB, where it is all
-// memory traffic, float32 4 x 155 x 201 x 201 by 32 49.6 / 52.9.
+// float16 8 x 155 x 150 x 150 28.2 / 35.9, a lane group of less than a tile, u8 75 x 14 x 14 by 16, 3.7 / 4.0, and past 16 MB,
+// where it is all memory traffic, float32 4 x 155 x 201 x 201 by 32 49.6 / 52.9.
 inline bool unaligned_pieces_pay(uint32_t la, uint64_t row_bytes, uint64_t plain_bytes) {
     return la >= 16 && la * row_bytes >= 12288 && plain_bytes < ((uint64_t)16 << 20);
 }

@@ -20,7 +20,7 @@
 //     registers, LDS addresses that are a per-thread constant plus the slot's scalar offset plus an
 //     immediate, tap geometry on the scalar
 //     unit when a k-step lies within one tap, and the per-pixel sum of x' (which the weight zero
-//     point multiplies) from v_dot4 on the registers being staged instead of further matrix work;
+//     point multiplies) from v_sad_u8 on the registers being staged instead of further matrix work;
 //   * blocks are numbered so that the channel chunks of one pixel tile run back to back on one
 //     XCD: the activations are fetched from HBM once and found in that XCD's L2 by the other chunks.
 // Arithmetic, weight packing and epilogue are those of qconv_igemm.hpp: the bytes are the same
