@@ -61,7 +61,7 @@ struct GemmArgs {
     const float *scale, *bias;
     const uint16_t *residual; // [m][n_out] fp16 or null
     void *out;                // [m][n_out] fp16 or fp32
-    int m, k, n_out, ksteps, mode, out_f32;
+    int m, k, n_out, ksteps, out_f32;
     int up_tile_offset; // SwiGLU: tile t of the gate pairs with tile t + up_tile_offset of the up projection
     // RMS normalisation of the token rows in front of the product (null: none): the block computes every row's
     // 1 / sqrt(mean(x^2) + eps) the way rmsnorm_f16_kernel does, and a token slice becomes
@@ -199,29 +199,27 @@ __device__ __forceinline__ h16x8 w8_to_f16(uint32_t lo, uint32_t hi) {
     return v - (_Float16)1152.0f; // 1024 + (w + 128) - 1152 = w, exact in fp16
 }
 
-// Epilogue of 4 consecutive output channels of one token: SwiGLU gate, residual, conversion, store.  `res`: the four
-// residual halves where the caller has loaded them already (have_res), else they are read here.
-template <int G> __device__ __forceinline__ void store_gemm_row(const GemmArgs &a, const float (&v)[G][4], size_t o, uint2 res = uint2{0u, 0u},
-                                                               bool have_res = false) {
+// Epilogue of 4 consecutive output channels of one token, at element o of `out`: SwiGLU gate, residual (its four halves in `res`),
+// conversion, store.
+template <int G> __device__ __forceinline__ void store_gemm_row(const float (&v)[G][4], size_t o, bool has_residual, uint2 res, void *out, int out_f32) {
     float y[4];
-    if (a.residual && !have_res) res = *reinterpret_cast<const uint2 *>(a.residual + o);
     __half rh[4];
     __builtin_memcpy(rh, &res, 8);
 #pragma unroll
     for (int r = 0; r < 4; r++) {
         if (G == 2) y[r] = v[0][r] / (1.f + __expf(-v[0][r])) * v[G - 1][r]; // silu(gate) * up
         else y[r] = v[0][r];
-        if (a.residual) y[r] += __half2float(rh[r]);
+        if (has_residual) y[r] += __half2float(rh[r]);
     }
-    if (a.out_f32) {
-        *reinterpret_cast<float4 *>(reinterpret_cast<float *>(a.out) + o) = float4{y[0], y[1], y[2], y[3]};
+    if (out_f32) {
+        *reinterpret_cast<float4 *>(reinterpret_cast<float *>(out) + o) = float4{y[0], y[1], y[2], y[3]};
     } else {
         __half h[4];
 #pragma unroll
         for (int r = 0; r < 4; r++) h[r] = __float2half_rn(y[r]);
         uint2 pk;
         __builtin_memcpy(&pk, h, 8);
-        *reinterpret_cast<uint2 *>(reinterpret_cast<__half *>(a.out) + o) = pk;
+        *reinterpret_cast<uint2 *>(reinterpret_cast<__half *>(out) + o) = pk;
     }
 }
 
@@ -231,12 +229,15 @@ template <int G> __device__ __forceinline__ void store_gemm_row(const GemmArgs &
 // whole share of a short reduction (896 / 8 waves = 2 k-steps) is a single memory round trip.
 constexpr int kGemmWaves = 8;
 constexpr int kGemmThreads = kGemmWaves * 64;
-constexpr int kGemmBatch = 4; // k-steps a wave requests before it multiplies any (5 where that halves a long share's trips to memory)
+constexpr int kGemmBatch = 4; // k-steps a wave requests before it multiplies any
 
 // SPLIT: the block's waves share one output tile and split its reduction (few tiles, long reductions);
 // otherwise every wave owns a tile of its own and the whole reduction (many tiles: the vocabulary head).
-template <int MT, int G, bool SPLIT, int B = kGemmBatch> __global__ __launch_bounds__(kGemmThreads) void w8a16_gemm_kernel(const GemmArgs a) {
-    __shared__ float red[SPLIT ? kGemmWaves : 1][G][MT][64][4];
+// PAIRED: a wave's even and odd k-steps are summed apart, as w8a16_small_tile_kernel does.
+template <int MT, int G, bool SPLIT, bool PAIRED = false> __global__ __launch_bounds__(kGemmThreads) void w8a16_gemm_kernel(const GemmArgs a) {
+    constexpr int B = kGemmBatch, P = PAIRED ? 2 : 1;
+    static_assert(B % 2 == 0, "a batch starts with an even k-step of the wave's share");
+    __shared__ float red[SPLIT ? kGemmWaves : 1][P][G][MT][64][4];
     __shared__ float rstd[MT * 16];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int i16 = lane & 15, kg = lane >> 4;
@@ -255,11 +256,13 @@ template <int MT, int G, bool SPLIT, int B = kGemmBatch> __global__ __launch_bou
     const int ks0 = SPLIT ? wave * per : 0, ks1 = min(a.ksteps, ks0 + per);
     const int out_tile = SPLIT ? (int)blockIdx.x : (int)blockIdx.x * kGemmWaves + wave;
     if (out_tile >= a.up_tile_offset) return; // SPLIT: never; otherwise the last block's spare waves (uniform per wave)
-    f32x4v acc[G][MT];
+    f32x4v acc[P][G][MT];
 #pragma unroll
-    for (int g = 0; g < G; g++)
+    for (int q = 0; q < P; q++)
 #pragma unroll
-        for (int t = 0; t < MT; t++) acc[g][t] = f32x4v{0.f, 0.f, 0.f, 0.f};
+        for (int g = 0; g < G; g++)
+#pragma unroll
+            for (int t = 0; t < MT; t++) acc[q][g][t] = f32x4v{0.f, 0.f, 0.f, 0.f};
 
     const int tile[2] = {out_tile, out_tile + a.up_tile_offset};
     // token rows of this lane (clamped: rows past m read row m - 1 and are never stored)
@@ -271,22 +274,6 @@ template <int MT, int G, bool SPLIT, int B = kGemmBatch> __global__ __launch_bou
         rrow[t] = a.ln_w ? rstd[min(t * 16 + i16, a.m - 1)] : 1.f;
     }
 
-    // The epilogue's operands (SPLIT: of the token tile this wave finishes) are asked for before the products: the
-    // launch is a chain of memory round trips, and this takes the last one out of it.
-    // (not with four token tiles: their slices leave no registers for it)
-    constexpr bool kPre = SPLIT && MT <= 2;
-    float4 sc[G], bs[G];
-    uint2 res_pre = uint2{0u, 0u};
-    if (kPre) {
-#pragma unroll
-        for (int g = 0; g < G; g++) {
-            sc[g] = *reinterpret_cast<const float4 *>(a.scale + tile[g] * 16 + kg * 4);
-            bs[g] = float4{0.f, 0.f, 0.f, 0.f};
-            if (a.bias) bs[g] = *reinterpret_cast<const float4 *>(a.bias + tile[g] * 16 + kg * 4);
-        }
-        const int m_pre = min(min(wave, MT - 1) * 16 + i16, a.m - 1);
-        if (a.residual) res_pre = *reinterpret_cast<const uint2 *>(a.residual + (size_t)m_pre * a.n_out + out_tile * 16 + kg * 4);
-    }
     for (int kb = ks0; kb < ks1; kb += B) {
         lu32x4 wv[B][G];
         lu32x4 av[B][MT][2];
@@ -338,8 +325,9 @@ template <int MT, int G, bool SPLIT, int B = kGemmBatch> __global__ __launch_bou
                         h16x8 x0, x1;
                         __builtin_memcpy(&x0, &av[u][t][0], 16);
                         __builtin_memcpy(&x1, &av[u][t][1], 16);
-                        acc[g][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(w0, x0, acc[g][t], 0, 0, 0);
-                        acc[g][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(w1, x1, acc[g][t], 0, 0, 0);
+                        f32x4v &to = acc[u % P][g][t];
+                        to = __builtin_amdgcn_mfma_f32_16x16x32_f16(w0, x0, to, 0, 0, 0);
+                        to = __builtin_amdgcn_mfma_f32_16x16x32_f16(w1, x1, to, 0, 0, 0);
                     }
                 }
             }
@@ -348,11 +336,13 @@ template <int MT, int G, bool SPLIT, int B = kGemmBatch> __global__ __launch_bou
     // ---- combine the waves' partial sums ------------------------------------------------------------
     if (SPLIT) {
 #pragma unroll
-        for (int g = 0; g < G; g++)
+        for (int q = 0; q < P; q++)
 #pragma unroll
-            for (int t = 0; t < MT; t++)
+            for (int g = 0; g < G; g++)
 #pragma unroll
-                for (int r = 0; r < 4; r++) red[wave][g][t][lane][r] = acc[g][t][r];
+                for (int t = 0; t < MT; t++)
+#pragma unroll
+                    for (int r = 0; r < 4; r++) red[wave][q][g][t][lane][r] = acc[q][g][t][r];
         __syncthreads();
         if (wave >= MT) return; // wave w finishes token tile w
     }
@@ -364,93 +354,325 @@ template <int MT, int G, bool SPLIT, int B = kGemmBatch> __global__ __launch_bou
         float v[G][4];
 #pragma unroll
         for (int g = 0; g < G; g++) {
-            const float scv[4] = {sc[g].x, sc[g].y, sc[g].z, sc[g].w}, bsv[4] = {bs[g].x, bs[g].y, bs[g].z, bs[g].w};
 #pragma unroll
             for (int r = 0; r < 4; r++) {
                 float s = 0.f;
                 if (SPLIT) {
 #pragma unroll
-                    for (int w = 0; w < kGemmWaves; w++) s += red[w][g][t][lane][r]; // fixed order: deterministic
+                    for (int w = 0; w < kGemmWaves; w++) // fixed order: deterministic
+#pragma unroll
+                        for (int q = 0; q < P; q++) s += red[w][q][g][t][lane][r];
                 } else {
-                    s = acc[g][tt][r];
+                    s = acc[0][g][tt][r];
                 }
-                if (kPre) {
-                    s *= scv[r];
-                    if (a.bias) s += bsv[r];
-                } else {
-                    const int ch = tile[g] * 16 + kg * 4 + r;
-                    s *= a.scale[ch];
-                    if (a.bias) s += a.bias[ch];
-                }
+                const int ch = tile[g] * 16 + kg * 4 + r;
+                s *= a.scale[ch];
+                if (a.bias) s += a.bias[ch];
                 v[g][r] = s;
             }
         }
         if (m >= a.m) continue;
-        store_gemm_row<G>(a, v, (size_t)m * a.n_out + out_tile * 16 + kg * 4, res_pre, kPre);
+        const size_t o = (size_t)m * a.n_out + out_tile * 16 + kg * 4;
+        const uint2 res = a.residual ? *reinterpret_cast<const uint2 *>(a.residual + o) : uint2{0u, 0u};
+        store_gemm_row<G>(v, o, a.residual != nullptr, res, a.out, a.out_f32);
     }
 }
 
-// Many output tiles and a reduction short enough for the token rows to fit in LDS (the vocabulary head, the gate / up
-// projection): a wave owns a tile (G = 2: the gate tile and its up tile) and the whole reduction, as in the kernel
-// above without SPLIT, but the block's waves share the token rows through LDS.  A wave brings in whole rows (row
-// wave, wave + WAVES, ...): it adds their squares in rms_rstd_rows' order as they arrive, parks them in LDS as loaded,
-// and, knowing 1 / sqrt(mean + eps) of its own rows without asking another wave, normalises them in place -- one trip
-// to memory and one barrier in front of the products, and every element normalised once per block instead of once per
-// wave.  A wave has the weights of KB k-steps in flight, the first KB from the start of the kernel.  The arithmetic per element and the order of the
-// multiply-adds are those of the kernel above.
-constexpr int kRowsBatch = 8;
-constexpr int kGluSplitWaves = 4;             // waves that split the reduction of one gate / up tile pair
 constexpr int kRowsPieces = 4;                 // 512-element pieces of a row: k <= 2048
 constexpr int kRowsMaxK = kRowsPieces * 512;
-inline int rows_in_lds_pitch(int k) { return k * 2 + 16; } // bytes per token row: the padding spreads the rows over the banks
+constexpr int kTileMaxK = 5120;                // ten k-steps a wave
+inline __host__ __device__ int rows_in_lds_pitch(int k) { return k * 2 + 16; } // bytes per token row: the padding spreads the rows over the banks
 
-// SPLIT: the block's waves share ONE output tile and split its reduction (few tiles: the q / k / v projection), combined
-// through LDS in the fixed order of the kernel above.
-// ROPE (with SPLIT and G = 2): a q / k / v projection whose block owns the two tiles that hold the halves of eight
-// rotate-half pairs -- tile j of a head and tile j + up_tile_offset (= head_dim / 32) -- so that a lane ends up with
-// both elements of its four pairs; the epilogue rounds them to fp16 as the projection's output would be stored and
-// rotates and stores them (rope_pair, rope_store).
-// FEW: no more rows than waves.  A wave then has one row at most, and none where it lies past m: what LDS holds in their place
-// meets no row that is stored.  (One row, 24 layers: q / k / v 5.9 -> 4.9 us, gate / up 7.8 -> 5.8.)
-template <int MT, int G, int WAVES, bool SPLIT = false, int KB = kRowsBatch, int PIECES = kRowsPieces, bool ROPE = false, bool FEW = false>
-__global__ __launch_bounds__(WAVES * 64) void w8a16_gemm_rows_in_lds_kernel(const GemmArgs a) {
-    static_assert(!ROPE || (SPLIT && G == 2), "the rotating epilogue pairs two tiles of one block");
-    extern __shared__ __attribute__((aligned(16))) uint8_t xs[]; // [MT * 16][k halves + padding]
-    __shared__ float red[SPLIT ? WAVES : 1][G][SPLIT ? MT : 1][64][4];
+// Kernel arguments that are used at different times, asked for together: a scalar load behind a branch or a wait is a wait of its own.
+template <typename A, typename B, typename C, typename D, typename E, typename F>
+__device__ __forceinline__ void request_together(const A &a, const B &b, const C &c, const D &d, const E &e, const F &f) {
+    asm volatile("" ::"s"(a), "s"(b), "s"(c), "s"(d), "s"(e), "s"(f));
+}
+
+// One tile of 16 output channels (G = 2: a gate tile and its up tile; ROPE: the two tiles that hold the halves of eight
+// rotate-half pairs, up_tile_offset = head_dim / 32 apart) times 16 token rows per block, the reduction split over the block's
+// eight waves and combined through LDS in a fixed order: the products of a decode step, a few dozen to a few hundred tiles.
+//
+// What bounds such a launch is not its bytes (a block's share of the weights is 14 to 78 KiB) but its chain of waits, so the
+// chain is as short as it can be: every argument is requested at once, then, without a branch between them, the rows, the weights
+// and the epilogue's operands, in the order in which they are needed and with addresses clamped where there is nothing to read.
+// (Loads behind branches cannot be waited for one by one: the normalisation waited for the weights' trip to memory, and the
+// products for the scales'.)  More than 16 rows are more blocks, not longer ones: those of one tile run on one die where the
+// number of tiles is a multiple of 8, and the weights come out of its L2.
+//
+// KS: k-steps of 64 a wave may have, all requested at once (k <= 512 * KS).
+// NORM: the rows are RMS-normalised on the way (see rms_rstd_rows for the order): wave w brings in rows w and, with R = 2, w + 8,
+// PIECES pieces of 512 elements each, and the products read them from LDS.  Without it they read the rows where they lie.
+template <int G, int KS, bool NORM, int R, int PIECES, bool ROPE>
+__global__ __launch_bounds__(kGemmThreads) void w8a16_tile_kernel(const GemmArgs a) {
+    static_assert(!ROPE || G == 2, "the rotating epilogue pairs two tiles of one block");
+    extern __shared__ __attribute__((aligned(16))) uint8_t xs[]; // NORM: [16][k halves + padding]
+    __shared__ float red[kGemmWaves][G][64][4];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int i16 = lane & 15, kg = lane >> 4;
-    const int pitch = a.k * 2 + 16;
+    const int k = a.k, ksteps = a.ksteps, off = a.up_tile_offset, n_out = a.n_out, out_f32 = a.out_f32;
+    const float eps = a.ln_eps;
+    const uint16_t *const x = a.a, *const ln_w = a.ln_w, *const residual = a.residual;
+    const lu32x4 *const w = a.w;
+    const float *const scale = a.scale, *const bias = a.bias ? a.bias : a.scale;
+    void *const out = a.out;
+    const bool has_bias = a.bias != nullptr;
+    request_together(eps, out, out_f32, residual, n_out, a.m);
+    const int row0 = (int)blockIdx.y * 16, rows = min(16, a.m - row0), last = row0 + rows - 1;
+    const int tile0 = ROPE ? (int)blockIdx.x / off * (2 * off) + (int)blockIdx.x % off : (int)blockIdx.x;
+    const int tile[2] = {tile0, tile0 + off};
+
+    // ---- requests ---------------------------------------------------------------------------------------
+    int rope_pos = 0;
+    if constexpr (ROPE) rope_pos = a.rope.ctx_lens[min(row0 + i16, last)]; // (loads return in order: asked for first, it is there first)
+    const int per = (ksteps + kGemmWaves - 1) / kGemmWaves, ks0 = wave * per, ks1 = min(ksteps, ks0 + per);
+    const uint16_t *xrow = x + (size_t)min(row0 + i16, last) * k + kg * 16;
+    lu32x4 v[NORM ? R : 1][NORM ? PIECES : 1], lwp[NORM ? PIECES : 1], wv[KS][G], av[NORM ? 1 : KS][2];
+    if constexpr (NORM) {
+#pragma unroll
+        for (int p = 0; p < PIECES; p++) {
+            const int e0 = min(lane * 8 + p * 512, k - 8); // (past the row: masked below)
+#pragma unroll
+            for (int i = 0; i < R; i++) v[i][p] = *reinterpret_cast<const lu32x4 *>(x + (size_t)min(row0 + wave + i * kGemmWaves, last) * k + e0);
+            lwp[p] = *reinterpret_cast<const lu32x4 *>(ln_w + e0);
+        }
+    }
+    float4 sc[G], bs[G]; // (ahead of the products' operands: behind their thirty loads a cold line of scales would arrive last)
+#pragma unroll
+    for (int g = 0; g < G; g++) {
+        sc[g] = *reinterpret_cast<const float4 *>(scale + tile[g] * 16 + kg * 4);
+        bs[g] = *reinterpret_cast<const float4 *>(bias + tile[g] * 16 + kg * 4);
+    }
+    const size_t o = (size_t)min(row0 + i16, last) * n_out + tile[0] * 16 + kg * 4; // of the lane's four outputs
+    const uint2 res = *reinterpret_cast<const uint2 *>(residual ? residual + o : x);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int u = 0; u < KS; u++) {
+        const int ks = max(min(ks0 + u, ks1 - 1), 0);
+#pragma unroll
+        for (int g = 0; g < G; g++) wv[u][g] = w[((size_t)tile[g] * ksteps + ks) * 64 + lane];
+        if constexpr (!NORM) {
+            av[u][0] = *reinterpret_cast<const lu32x4 *>(xrow + ks * 64), av[u][1] = *reinterpret_cast<const lu32x4 *>(xrow + ks * 64 + 8);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+
+    // ---- rows --------------------------------------------------------------------------------------------
+    RopePair rope;
+    if constexpr (ROPE) {
+        // The angle is computed while the rows and weights travel; wave w finishes channel w of each lane's four.
+        if (wave < 4) rope = rope_pair(a.rope, min(row0 + i16, last), (tile0 * 16 + kg * 4 + wave) / a.rope.d, (tile0 * 16 + kg * 4 + wave) % a.rope.d, rope_pos);
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    const int pitch = rows_in_lds_pitch(k);
+    if constexpr (NORM) {
+        if (wave < rows) { // (uniform; what LDS holds in the place of rows past m meets no row that is stored)
+            float ss[R];
+#pragma unroll
+            for (int i = 0; i < R; i++) ss[i] = 0.f;
+#pragma unroll
+            for (int p = 0; p < PIECES; p++)
+#pragma unroll
+                for (int i = 0; i < R; i++) {
+                    if (lane * 8 + p * 512 >= k) v[i][p] = lu32x4{0, 0, 0, 0}; // (+0 squares leave a sum as it is)
+                    add_squares8(v[i][p], ss[i]);
+                }
+#pragma unroll
+            for (int i = 0; i < R; i++) ss[i] = 1.0f / sqrtf(wave_sum(ss[i]) / (float)k + eps); // rstd_from_sum's formula
+#pragma unroll
+            for (int p = 0; p < PIECES; p++) {
+                __half wh[8], xh[R][8];
+                __builtin_memcpy(wh, &lwp[p], 16);
+#pragma unroll
+                for (int i = 0; i < R; i++) __builtin_memcpy(xh[i], &v[i][p], 16);
+#pragma unroll
+                for (int e = 0; e < 8; e++)
+#pragma unroll
+                    for (int i = 0; i < R; i++) {
+                        // the fp32 product is rounded before it is converted, as in rmsnorm_f16_kernel (see there)
+                        float pr = __half2float(xh[i][e]) * ss[i] * __half2float(wh[e]);
+                        asm volatile("" : "+v"(pr));
+                        xh[i][e] = __float2half_rn(pr);
+                    }
+                if (lane * 8 + p * 512 < k) {
+#pragma unroll
+                    for (int i = 0; i < R; i++)
+                        *reinterpret_cast<lu32x4 *>(xs + (size_t)(wave + i * kGemmWaves) * pitch + (lane * 8 + p * 512) * 2) = *reinterpret_cast<lu32x4 *>(xh[i]);
+                }
+            }
+        }
+        __syncthreads();
+    }
+
+    // ---- products ------------------------------------------------------------------------------------------
+    f32x4v acc[G];
+#pragma unroll
+    for (int g = 0; g < G; g++) acc[g] = f32x4v{0.f, 0.f, 0.f, 0.f};
+    const uint8_t *xl = xs + (size_t)i16 * pitch + kg * 32; // the lane's 16 reduction indices of a k-step
+#pragma unroll
+    for (int u = 0; u < KS; u++) {
+        if (ks0 + u < ks1) { // uniform
+            h16x8 x0, x1;
+            if constexpr (NORM) {
+                x0 = *reinterpret_cast<const h16x8 *>(xl + (ks0 + u) * 128), x1 = *reinterpret_cast<const h16x8 *>(xl + (ks0 + u) * 128 + 16);
+            } else {
+                __builtin_memcpy(&x0, &av[u][0], 16), __builtin_memcpy(&x1, &av[u][1], 16);
+            }
+#pragma unroll
+            for (int g = 0; g < G; g++) {
+                acc[g] = __builtin_amdgcn_mfma_f32_16x16x32_f16(w8_to_f16(wv[u][g][0], wv[u][g][1]), x0, acc[g], 0, 0, 0);
+                acc[g] = __builtin_amdgcn_mfma_f32_16x16x32_f16(w8_to_f16(wv[u][g][2], wv[u][g][3]), x1, acc[g], 0, 0, 0);
+            }
+        }
+    }
+#pragma unroll
+    for (int g = 0; g < G; g++) *reinterpret_cast<f32x4v *>(red[wave][g][lane]) = acc[g];
+    __syncthreads();
+    // lane (i16 = token, kg): channels tile * 16 + kg * 4 + r
+    if constexpr (ROPE) {
+        // The rotation costs a few hundred instructions per pair, so the pairs are spread over four waves.
+        if (wave >= 4 || i16 >= rows) return;
+        float v2[2];
+#pragma unroll
+        for (int g = 0; g < 2; g++) {
+            float s = 0.f;
+#pragma unroll
+            for (int q = 0; q < kGemmWaves; q++) s += red[q][g][lane][wave]; // fixed order, as below
+            const float scv[4] = {sc[g].x, sc[g].y, sc[g].z, sc[g].w}, bsv[4] = {bs[g].x, bs[g].y, bs[g].z, bs[g].w};
+            float sv = scv[0], bv = bsv[0];
+#pragma unroll
+            for (int q = 1; q < 4; q++) sv = wave == q ? scv[q] : sv, bv = wave == q ? bsv[q] : bv;
+            s *= sv;
+            if (has_bias) s += bv;
+            v2[g] = s;
+        }
+        // (rounded to fp16 as the projection's output would be stored; the partner is d / 2 channels further)
+        rope_store(a.rope, row0 + i16, rope, __half2float(__float2half_rn(v2[0])), __half2float(__float2half_rn(v2[1])));
+        return;
+    }
+    if (wave != 0) return;
+    float y[G][4];
+#pragma unroll
+    for (int g = 0; g < G; g++) {
+        const float scv[4] = {sc[g].x, sc[g].y, sc[g].z, sc[g].w}, bsv[4] = {bs[g].x, bs[g].y, bs[g].z, bs[g].w};
+        f32x4v s = f32x4v{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int q = 0; q < kGemmWaves; q++) s += *reinterpret_cast<const f32x4v *>(red[q][g][lane]); // fixed order: deterministic
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+            y[g][r] = s[r] * scv[r];
+            if (has_bias) y[g][r] += bsv[r];
+        }
+    }
+    if (i16 >= rows) return;
+    store_gemm_row<G>(y, o, residual != nullptr, res, out, out_f32);
+}
+
+// The same product for long reductions over few tiles (the down projection), where a block of the kernel above has its compute
+// unit to itself and is bound by what passes through that unit's L1: tiles of 8 channels by 8 rows.  The matrix instruction's 16
+// rows are 8 channels of two consecutive k-steps, its 16 columns the 8 token rows of the same two; the two blocks of the result
+// on the diagonal are wanted, the other two are not.  A block then reads half the weights and half the rows for a quarter of the
+// outputs, and a wave half as many fragments.  The order of the sum: a wave's even steps and its odd steps, then the waves' two
+// sums after one another (w8a16_gemm_kernel with PAIRED adds in it too).
+// Two blocks share a 16-channel tile of the packed weights; both on one die, so that its L2 keeps the halves together.
+template <int KP> __global__ __launch_bounds__(kGemmThreads) void w8a16_small_tile_kernel(const GemmArgs a) {
+    __shared__ float red[kGemmWaves][64][4];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int i8 = lane & 7, odd = lane >> 3 & 1, kg = lane >> 4;
+    const int k = a.k, ksteps = a.ksteps, n_out = a.n_out, out_f32 = a.out_f32;
+    const uint16_t *const x = a.a, *const residual = a.residual;
+    const lu32x4 *const w = a.w;
+    const float *const scale = a.scale, *const bias = a.bias ? a.bias : a.scale;
+    void *const out = a.out;
+    const bool has_bias = a.bias != nullptr;
+    request_together(k, out, out_f32, residual, n_out, a.m);
+    const int group = (int)blockIdx.x / 16 * 8, in_group = min(8, a.up_tile_offset - group), r16 = (int)blockIdx.x % 16;
+    const int half = r16 >= in_group, tile = group + r16 - half * in_group;
+    const int row0 = (int)blockIdx.y * 8, rows = min(8, a.m - row0), last = row0 + rows - 1;
+    const int per = (ksteps + kGemmWaves - 1) / kGemmWaves, ks0 = wave * per, ks1 = min(ksteps, ks0 + per);
+    // the lane of wave 0 that finishes row i8, channels tile * 16 + half * 8 + odd * 4 + 0 .. 3
+    const int ch = tile * 16 + half * 8 + odd * 4;
+    const size_t o = (size_t)min(row0 + i8, last) * n_out + ch;
+    const float4 sc = *reinterpret_cast<const float4 *>(scale + ch), bs = *reinterpret_cast<const float4 *>(bias + ch);
+    const uint2 res = *reinterpret_cast<const uint2 *>(residual ? residual + o : x);
+    const lu32x4 *wl = w + (size_t)tile * ksteps * 64 + kg * 16 + half * 8 + i8;
+    const uint16_t *xl = x + (size_t)min(row0 + i8, last) * k + kg * 16;
+    lu32x4 wv[KP], av[KP][2];
+#pragma unroll
+    for (int u = 0; u < KP; u++) {
+        const int ks = max(min(ks0 + 2 * u + odd, ks1 - 1), 0); // steps past the share: cleared below
+        wv[u] = wl[ks * 64];
+        av[u][0] = *reinterpret_cast<const lu32x4 *>(xl + ks * 64), av[u][1] = *reinterpret_cast<const lu32x4 *>(xl + ks * 64 + 8);
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    f32x4v acc = f32x4v{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int u = 0; u < KP; u++) {
+        if (ks0 + 2 * u < ks1) { // uniform
+            if (ks0 + 2 * u + 1 >= ks1 && odd) wv[u] = av[u][0] = av[u][1] = lu32x4{0, 0, 0, 0};
+            h16x8 x0, x1;
+            __builtin_memcpy(&x0, &av[u][0], 16), __builtin_memcpy(&x1, &av[u][1], 16);
+            acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(w8_to_f16(wv[u][0], wv[u][1]), x0, acc, 0, 0, 0);
+            acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(w8_to_f16(wv[u][2], wv[u][3]), x1, acc, 0, 0, 0);
+        }
+    }
+    *reinterpret_cast<f32x4v *>(red[wave][lane]) = acc;
+    __syncthreads();
+    if (wave != 0 || lane >= 16) return;
+    f32x4v s = f32x4v{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int q = 0; q < kGemmWaves; q++) { // fixed order: deterministic
+        s += *reinterpret_cast<const f32x4v *>(red[q][odd * 16 + i8]);
+        s += *reinterpret_cast<const f32x4v *>(red[q][(odd + 2) * 16 + 8 + i8]);
+    }
+    const float scv[4] = {sc.x, sc.y, sc.z, sc.w}, bsv[4] = {bs.x, bs.y, bs.z, bs.w};
+    float y[1][4];
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+        y[0][r] = s[r] * scv[r];
+        if (has_bias) y[0][r] += bsv[r];
+    }
+    if (i8 >= rows) return;
+    store_gemm_row<1>(y, o, residual != nullptr, res, out, out_f32);
+}
+
+constexpr int kRowsBatch = 8;
+// Many output tiles and a reduction short enough for the token rows to fit in LDS (the vocabulary head): a wave owns a
+// tile (G = 2: the gate tile and its up tile) and the whole reduction, as in the kernel above without SPLIT, but the
+// block's waves share the token rows through LDS.  A wave brings in whole rows (row wave, wave + 8, ...): it adds their
+// squares in rms_rstd_rows' order as they arrive and, knowing 1 / sqrt(mean + eps) of its own rows without asking another
+// wave, normalises them on the way to LDS -- one trip to memory and one barrier in front of the products, and every element
+// normalised once per block instead of once per wave.  A wave has the weights of KB k-steps in flight, the first KB from the
+// start of the kernel.  The arithmetic per element and the order of the multiply-adds are those of the kernel above.
+template <int MT, int G, int KB, int PIECES> __global__ __launch_bounds__(kGemmThreads) void w8a16_gemm_rows_in_lds_kernel(const GemmArgs a) {
+    constexpr int WAVES = kGemmWaves;
+    extern __shared__ __attribute__((aligned(16))) uint8_t xs[]; // [MT * 16][k halves + padding]
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int i16 = lane & 15, kg = lane >> 4;
+    const int pitch = rows_in_lds_pitch(a.k);
     // The weights do not depend on the rows: the first KB k-steps of this wave's share are requested before anything
     // else, so that their trip to memory runs beside the one that brings the rows in (a spare wave of the last block
     // reads the last tile's and multiplies nothing).
-    // Without SPLIT a block walks the groups of WAVES tiles blockIdx.x, blockIdx.x + gridDim.x, ...: a launch with fewer
+    // A block walks the groups of WAVES tiles blockIdx.x, blockIdx.x + gridDim.x, ...: a launch with fewer
     // blocks than groups (the vocabulary head) brings the rows in and normalises them once per block, not once per group.
     int group = (int)blockIdx.x;
-    int out_tile = ROPE    ? ((int)blockIdx.x / a.up_tile_offset) * (2 * a.up_tile_offset) + (int)blockIdx.x % a.up_tile_offset
-                   : SPLIT ? (int)blockIdx.x
-                           : group * WAVES + wave;
-    const int per = SPLIT ? (a.ksteps + WAVES - 1) / WAVES : a.ksteps;
-    const int ks0 = SPLIT ? wave * per : 0, ks1 = min(a.ksteps, ks0 + per);
-    int first = ROPE ? out_tile : min(out_tile, a.up_tile_offset - 1);
+    int out_tile = group * WAVES + wave;
+    const int ks1 = a.ksteps;
+    int first = min(out_tile, a.up_tile_offset - 1);
     int tile[2] = {first, first + a.up_tile_offset};
     lu32x4 wv[KB][G];
     auto request_first = [&]() __attribute__((always_inline)) {
 #pragma unroll
         for (int u = 0; u < KB; u++) {
-            const int ks = max(min(ks0 + u, ks1 - 1), 0); // steps past the share re-read its last one (an empty share: step 0) and are not multiplied
+            const int ks = min(u, ks1 - 1); // steps past the end re-read the last one and are not multiplied
 #pragma unroll
             for (int g = 0; g < G; g++) wv[u][g] = a.w[((size_t)tile[g] * a.ksteps + ks) * 64 + lane];
         }
     };
-    // ROPE: the pair this thread will finish is channel wave % 4 of the lane's four, of token tile wave / 4
-    const int rope_m = min((wave >> 2) * 16 + i16, a.m - 1);
-    int rope_pos = 0;
-    if constexpr (ROPE) rope_pos = a.rope.ctx_lens[rope_m]; // (loads return in order: asked for first, it is there first)
-    __builtin_amdgcn_sched_barrier(0);
     request_first();
-    RopePair rope;
     {
-        constexpr int R = FEW ? 1 : MT * 16 / WAVES; // rows per wave
+        constexpr int R = MT * 16 / WAVES; // rows per wave
         // The wave's rows stay in registers from the load to the one LDS write: their sums of squares, the butterflies
         // and the normalisation run for all R rows side by side (independent chains), element by element in the order
         // rms_rstd_rows and rmsnorm_f16_kernel use.
@@ -467,17 +689,7 @@ __global__ __launch_bounds__(WAVES * 64) void w8a16_gemm_rows_in_lds_kernel(cons
                 if (r < a.m && e0 < a.k) v[i][p] = *reinterpret_cast<const lu32x4 *>(a.a + (size_t)r * a.k + e0);
             }
         }
-        // The angle is computed while the rows and weights travel: its few hundred instructions and the two loads in front
-        // of it were the last microseconds of the launch when they followed the products.
-        if constexpr (ROPE) {
-            __builtin_amdgcn_sched_barrier(0);
-            if (wave < MT * 4) { // (the other waves finish nothing)
-                const int c = out_tile * 16 + kg * 4 + (wave & 3);
-                rope = rope_pair(a.rope, rope_m, c / a.rope.d, c % a.rope.d, rope_pos);
-            }
-            __builtin_amdgcn_sched_barrier(0);
-        }
-        if (a.ln_w && (!FEW || wave < a.m)) {
+        if (a.ln_w) {
             float ss[R];
 #pragma unroll
             for (int i = 0; i < R; i++) ss[i] = 0.f;
@@ -513,16 +725,16 @@ __global__ __launch_bounds__(WAVES * 64) void w8a16_gemm_rows_in_lds_kernel(cons
 #pragma unroll
         for (int p = 0; p < PIECES; p++) {
             const int e0 = lane * 8 + p * 512;
-            if (e0 < a.k && (!FEW || wave < a.m)) {
+            if (e0 < a.k) {
 #pragma unroll
                 for (int i = 0; i < R; i++) *reinterpret_cast<lu32x4 *>(xs + (size_t)(wave + i * WAVES) * pitch + e0 * 2) = v[i][p];
             }
         }
     }
     __syncthreads();
-    const int groups = SPLIT ? 0 : (a.up_tile_offset + WAVES - 1) / WAVES;
-    for (;;) { // (one pass with SPLIT)
-    if (!ROPE && out_tile >= a.up_tile_offset) return; // SPLIT: never; otherwise the last group's spare waves (uniform per wave; no group follows it)
+    const int groups = (a.up_tile_offset + WAVES - 1) / WAVES;
+    for (;;) {
+    if (out_tile >= a.up_tile_offset) return; // the last group's spare waves (uniform per wave; no group follows it)
     f32x4v acc[G][MT];
 #pragma unroll
     for (int g = 0; g < G; g++)
@@ -536,11 +748,8 @@ __global__ __launch_bounds__(WAVES * 64) void w8a16_gemm_rows_in_lds_kernel(cons
         bs[g] = float4{0.f, 0.f, 0.f, 0.f};
         if (a.bias) bs[g] = *reinterpret_cast<const float4 *>(a.bias + tile[g] * 16 + kg * 4);
     }
-    uint2 res_pre = uint2{0u, 0u};
-    if (SPLIT && a.residual) // (the token tile this wave finishes)
-        res_pre = *reinterpret_cast<const uint2 *>(a.residual + (size_t)min(min(wave, MT - 1) * 16 + i16, a.m - 1) * a.n_out + out_tile * 16 + kg * 4);
-    for (int kb = ks0; kb < ks1; kb += KB) {
-        if (kb != ks0) { // (the first batch is on its way since the start)
+    for (int kb = 0; kb < ks1; kb += KB) {
+        if (kb != 0) { // (the first batch is on its way since the start)
 #pragma unroll
             for (int u = 0; u < KB; u++) {
                 const int ks = min(kb + u, ks1 - 1); // steps past the end re-read the last one and are not multiplied
@@ -571,52 +780,16 @@ __global__ __launch_bounds__(WAVES * 64) void w8a16_gemm_rows_in_lds_kernel(cons
     }
     // the next group's first weights are requested as soon as this one's are multiplied: they travel under the epilogue
     group += (int)gridDim.x;
-    const bool more = !SPLIT && group < groups;
+    const bool more = group < groups;
     const int next_tile = group * WAVES + wave;
     if (more) {
         first = min(next_tile, a.up_tile_offset - 1);
         tile[0] = first, tile[1] = first + a.up_tile_offset;
         request_first();
     }
-    if (SPLIT) {
-#pragma unroll
-        for (int g = 0; g < G; g++)
-#pragma unroll
-            for (int t = 0; t < MT; t++)
-#pragma unroll
-                for (int r = 0; r < 4; r++) red[wave][g][t][lane][r] = acc[g][t][r];
-        __syncthreads();
-        if constexpr (ROPE) {
-            // The rotation costs a few hundred instructions per pair (the angle's power, sine and cosine), so the
-            // pairs are spread over all the waves: wave w takes channel w % 4 of each lane's four, token tile w / 4.
-            static_assert(WAVES == 8, "channel w % 4, token tile w / 4");
-            const int t = wave >> 2, r = wave & 3;
-            const int m = t * 16 + i16;
-            if (t >= MT || m >= a.m) return;
-            float v2[2];
-#pragma unroll
-            for (int g = 0; g < 2; g++) {
-                const float scv[4] = {sc[g].x, sc[g].y, sc[g].z, sc[g].w}, bsv[4] = {bs[g].x, bs[g].y, bs[g].z, bs[g].w};
-                float s = 0.f;
-#pragma unroll
-                for (int w = 0; w < WAVES; w++) s += red[w][g][t][lane][r]; // fixed order, as below
-                float sv = scv[0], bv = bsv[0];
-#pragma unroll
-                for (int q = 1; q < 4; q++) sv = r == q ? scv[q] : sv, bv = r == q ? bsv[q] : bv;
-                s *= sv;
-                if (a.bias) s += bv;
-                v2[g] = s;
-            }
-            // (rounded to fp16 as the projection's output would be stored; the partner is d / 2 channels further)
-            rope_store(a.rope, m, rope, __half2float(__float2half_rn(v2[0])), __half2float(__float2half_rn(v2[1])));
-            return;
-        }
-        if (wave >= MT) return; // wave w finishes token tile w
-    }
     // lane (i16 = token within the tile, kg): channels tile * 16 + kg * 4 + r
 #pragma unroll
-    for (int tt = 0; tt < (SPLIT ? 1 : MT); tt++) {
-        const int t = SPLIT ? wave : tt;
+    for (int t = 0; t < MT; t++) {
         const int m = t * 16 + i16;
         float v[G][4];
 #pragma unroll
@@ -624,20 +797,15 @@ __global__ __launch_bounds__(WAVES * 64) void w8a16_gemm_rows_in_lds_kernel(cons
             const float scv[4] = {sc[g].x, sc[g].y, sc[g].z, sc[g].w}, bsv[4] = {bs[g].x, bs[g].y, bs[g].z, bs[g].w};
 #pragma unroll
             for (int r = 0; r < 4; r++) {
-                float s = 0.f;
-                if (SPLIT) {
-#pragma unroll
-                    for (int w = 0; w < WAVES; w++) s += red[w][g][t][lane][r]; // fixed order: deterministic
-                } else {
-                    s = acc[g][tt][r];
-                }
-                s *= scv[r];
+                float s = acc[g][t][r] * scv[r];
                 if (a.bias) s += bsv[r];
                 v[g][r] = s;
             }
         }
         if (m >= a.m) continue;
-        store_gemm_row<G>(a, v, (size_t)m * a.n_out + out_tile * 16 + kg * 4, res_pre, SPLIT);
+        const size_t o = (size_t)m * a.n_out + out_tile * 16 + kg * 4;
+        const uint2 res = a.residual ? *reinterpret_cast<const uint2 *>(a.residual + o) : uint2{0u, 0u};
+        store_gemm_row<G>(v, o, a.residual != nullptr, res, a.out, a.out_f32);
     }
     if (!more) return;
     out_tile = next_tile;
@@ -809,21 +977,74 @@ template <typename KernelT> static hipError_t raise_dynamic_lds(KernelT kernel, 
     return e;
 }
 
-// Whether a plain product of m rows (up to two token tiles that fit half of LDS) is computed with a tile's reduction split over a
-// block's waves.  The sum's order depends on it, so it is asked for the rows' count and the matrix alone: the product, the one
-// that normalises its rows and the one that rotates them agree bit for bit.  A block per tile repeats the rows' trip (and their
-// normalisation), a tile per wave leaves the device to few blocks: us, split / not, k = 896, 4096 / 8192 / 16368 columns: one row
-// 2.9 3.4 5.0 / 4.4 4.6 5.7, 16 rows 3.2 4.0 5.8 / 4.5 5.0 6.0, 32 rows 3.9 5.0 8.7 / 5.7 6.2 7.2 (10 240 columns 7.0 / 6.6).
-static bool rows_take_split(const nncase_hip_ctx_t *ctx, const nncase_hip_w8a16_t *w, int m) {
-    const int mt_built = m <= 16 ? 1 : 2;
-    return m <= 32 && w->k <= kRowsMaxK && (size_t)mt_built * 16 * rows_in_lds_pitch(w->k) <= 64 * 1024 &&
-           2 * w->ntiles < (m <= kGemmWaves ? 8 : 5) * ctx->compute_units;
+// Whether a product of m rows and `tiles` tiles (pairs) over at most kRowsMaxK is computed with a tile's reduction split over a
+// block's waves.  The sum's order depends on it, so it is asked for the rows' count and the matrix alone: the product, the one that
+// normalises its rows and the one that rotates them agree bit for bit.  A block per tile repeats the rows' trip (and their
+// normalisation), a tile per wave leaves the device to few blocks.  us, split / not, k = 896: plain, 4096 / 8192 / 12 288 columns:
+// one row 3.1 4.2 4.7 / 5.7 6.8 6.4, 16 rows 4.0 5.4 6.4 / 5.9 7.0 6.6, 32 rows 5.2 7.9 10.0 / 8.0 9.3 8.8, 64 rows 7.7 13.0 17.4 /
+// 12.4 14.0 13.4; SwiGLU, 2048 / 8192 / 14 336 columns: one row 3.7 5.7 7.4 / 7.8 9.5 9.4, 16 rows 4.5 6.8 9.9 / 7.7 9.6 9.5,
+// 32 rows 4.6 10.4 15.3 / 9.9 11.5 11.3, 64 rows 6.4 17.0 27.0 / 15.0 16.7 16.7.
+static bool rows_take_split(const nncase_hip_ctx_t *ctx, const nncase_hip_w8a16_t *w, int tiles, bool glu, int m) {
+    if (w->k > kRowsMaxK || 16 * rows_in_lds_pitch(w->k) > 64 * 1024) return false;
+    const int64_t rt = (m + 15) / 16, cus = ctx->compute_units;
+    if (m <= kGemmWaves) return tiles < 4 * cus;
+    if (glu) return tiles * rt < (2 + rt) * cus;
+    return 2 * tiles < (rt == 1 ? 5 : 4) * cus;
 }
 
 // Whether the q / k / v projection of this geometry can rotate and append in its own epilogue (else the caller runs
 // the projection and the rope kernel one after the other).
 static bool rope_epilogue_fits(const nncase_hip_ctx_t *ctx, const nncase_hip_w8a16_t *w, int m, const RopeArgs &r) {
-    return rows_take_split(ctx, w, m) && r.d % 32 == 0 && w->n == (r.hq + 2 * r.hkv) * r.d && (w->ksteps + kGemmWaves - 1) / kGemmWaves <= 2;
+    return rows_take_split(ctx, w, w->ntiles, false, m) && r.d % 32 == 0 && w->n == (r.hq + 2 * r.hkv) * r.d && w->k <= 1024;
+}
+
+// Whether a long reduction over few tiles is computed in tiles of 8 by 8 (and summed in their order, whichever kernel does it).
+// They are four times the blocks of 16 by 16, each of which moves half as much: taken while all of them run at once.  us, 16 by
+// 16 / 8 by 8, k = 4864, 896 columns: one row 5.3 / 4.4, 8 rows 6.2 / 5.7, 16 rows 7.9 / 5.6, 32 rows 7.9 / 8.4.
+static bool sums_in_pairs(const nncase_hip_ctx_t *ctx, const nncase_hip_w8a16_t *w, int m) {
+    return w->k > kRowsMaxK && w->k <= kTileMaxK && m <= 16 && 2 * w->ntiles * ((m + 7) / 8) <= ctx->compute_units;
+}
+
+// Which kernel computes a product of m rows.
+enum class GemmForm {
+    kTile,      // a tile (pair) per block, its reduction split over the waves
+    kSmallTile, // 8 channels by 8 rows per block
+    kRowsInLds, // a tile (pair) per wave, rows in LDS
+    kSplit,     // as kTile (and in its order), for reductions that it has no registers or LDS for
+    kPerWave,   // a tile (pair) per wave, rows read where they lie
+};
+static GemmForm gemm_form(const nncase_hip_ctx_t *ctx, const nncase_hip_w8a16_t *w, int m, bool glu, bool normalises) {
+    const int out_tiles = glu ? w->ntiles / 2 : w->ntiles, mt = (m + 15) / 16, mt_built = mt <= 1 ? 1 : (mt == 2 ? 2 : 4);
+    // few output tiles: the block's waves split the reduction of one tile; many: a tile per wave
+    const bool split = out_tiles < 4 * ctx->compute_units;
+    // (fewer tiles than compute units and nothing to normalise: kTile too, below)
+    if (rows_take_split(ctx, w, out_tiles, glu, m) && (glu || normalises || out_tiles >= ctx->compute_units)) return GemmForm::kTile;
+    // a tile per wave with the token rows shared through LDS: where the rows fit and the launch has a tile for every
+    // compute unit
+    if (w->k <= kRowsMaxK && (size_t)mt_built * 16 * rows_in_lds_pitch(w->k) <= 128 * 1024 && out_tiles >= ctx->compute_units) return GemmForm::kRowsInLds;
+    if (!split) return GemmForm::kPerWave;
+    if (!glu && !normalises && sums_in_pairs(ctx, w, m)) return GemmForm::kSmallTile;
+    return normalises || w->k > kTileMaxK ? GemmForm::kSplit : GemmForm::kTile;
+}
+
+template <int G, int KS, bool NORM, int R = 1, int PIECES = 1, bool ROPE = false>
+static int launch_tile(nncase_hip_ctx_t *ctx, const GemmArgs &a, int tiles) {
+    const size_t lds = NORM ? (size_t)16 * rows_in_lds_pitch(a.k) : 0;
+    NNHIP_HIP(ctx, raise_dynamic_lds(w8a16_tile_kernel<G, KS, NORM, R, PIECES, ROPE>, ctx->device, lds + G * kGemmWaves * 1024, 96 * 1024));
+    hipLaunchKernelGGL((w8a16_tile_kernel<G, KS, NORM, R, PIECES, ROPE>), dim3(tiles, (a.m + 15) / 16), dim3(kGemmThreads), lds, ctx->stream, a);
+    NNHIP_LAUNCH_CHECK(ctx, "w8a16_tile_kernel");
+    return 0;
+}
+template <int G, bool ROPE = false> static int launch_tile_normalising(nncase_hip_ctx_t *ctx, const GemmArgs &a, int tiles) {
+    const bool few = a.m <= kGemmWaves; // a row per wave at most
+    if (a.k <= 1024) return few ? launch_tile<G, 2, true, 1, 2, ROPE>(ctx, a, tiles) : launch_tile<G, 2, true, 2, 2, ROPE>(ctx, a, tiles);
+    if constexpr (ROPE) return -EINVAL; // (see rope_epilogue_fits)
+    else return few ? launch_tile<G, 4, true, 1, kRowsPieces>(ctx, a, tiles) : launch_tile<G, 4, true, 2, kRowsPieces>(ctx, a, tiles);
+}
+template <int G> static int launch_tile_plain(nncase_hip_ctx_t *ctx, const GemmArgs &a, int tiles) {
+    if (a.k <= 1024) return launch_tile<G, 2, false>(ctx, a, tiles);
+    if (a.k <= 2048) return launch_tile<G, 4, false>(ctx, a, tiles);
+    return launch_tile<G, kTileMaxK / 512, false>(ctx, a, tiles);
 }
 
 static int launch_w8a16_gemm(nncase_hip_ctx_t *ctx, const void *a_dev, const nncase_hip_w8a16_t *w, void *out_dev, int32_t m,
@@ -852,105 +1073,35 @@ static int launch_w8a16_gemm(nncase_hip_ctx_t *ctx, const void *a_dev, const nnc
     a.ln_w = (const uint16_t *)ln_weight_dev;
     a.ln_eps = ln_eps;
     a.out = out_dev;
-    a.m = m, a.k = w->k, a.ksteps = w->ksteps, a.mode = mode, a.out_f32 = out_dtype == NNCASE_HIP_DT_F32;
+    a.m = m, a.k = w->k, a.ksteps = w->ksteps, a.out_f32 = out_dtype == NNCASE_HIP_DT_F32;
     const int out_tiles = mode == NNCASE_HIP_GEMM_SWIGLU ? w->ntiles / 2 : w->ntiles;
     a.up_tile_offset = out_tiles;
     a.n_out = out_tiles * 16;
-    // few output tiles: the block's waves split the reduction of one tile; many: a tile per wave
-    const bool split = out_tiles < 4 * ctx->compute_units;
-    const dim3 grid(split ? out_tiles : (out_tiles + kGemmWaves - 1) / kGemmWaves), block(kGemmThreads);
     const int mt = (m + 15) / 16;
     const bool glu = mode == NNCASE_HIP_GEMM_SWIGLU;
-    // a tile per wave with the token rows shared through LDS: where the rows fit and the launch has a tile for every
-    // compute unit (measured on the decode step: the 72- and 56-tile products are quicker with the reduction split
-    // over a block's waves, 9.7 against 11.2 us; the 304 gate / up tile pairs take 11.4 us in 38 blocks of eight waves
-    // with a pair per wave, 10.7 us in 304 blocks of four waves that split a pair's reduction, 12.8 us in blocks of
-    // eight.  What the launches cost is not the weights' trip to memory but what every block repeats: the rows' trip,
-    // 1.2 us, their normalisation, 0.3 us of vector issue per row and SIMD, and, with a pair per wave, 0.24 us of
-    // conversions and matrix instructions per k-step on a SIMD that two waves share)
-    const int mt_built = mt <= 1 ? 1 : (mt == 2 ? 2 : 4);
-    const size_t rows_lds = (size_t)mt_built * 16 * rows_in_lds_pitch(w->k);
-    if (rope) {
-        // (the caller has checked rope_epilogue_fits) a block per pair of tiles d / 2 channels apart
+    if (rope) { // (the caller has checked rope_epilogue_fits) a block per pair of tiles d / 2 channels apart
         a.rope = *rope;
         a.up_tile_offset = rope->d / 32;
-        const dim3 pgrid(w->ntiles / 2), pblock(kGemmThreads);
-        const bool two_pieces = w->k <= 1024;
-#define NNHIP_ROPE_LAUNCH(MTV, PV, FEWV)                                                                                             \
-    do {                                                                                                                       \
-        NNHIP_HIP(ctx, raise_dynamic_lds(w8a16_gemm_rows_in_lds_kernel<MTV, 2, kGemmWaves, true, 2, PV, true, FEWV>, ctx->device,   \
-                                         rows_lds + MTV * 16 * 1024, 96 * 1024));                                              \
-        hipLaunchKernelGGL((w8a16_gemm_rows_in_lds_kernel<MTV, 2, kGemmWaves, true, 2, PV, true, FEWV>), pgrid, pblock, rows_lds, ctx->stream, a); \
-    } while (0)
-        if (m <= kGemmWaves && two_pieces) NNHIP_ROPE_LAUNCH(1, 2, true);
-        else if (m <= kGemmWaves) NNHIP_ROPE_LAUNCH(1, kRowsPieces, true);
-        else if (mt_built == 1 && two_pieces) NNHIP_ROPE_LAUNCH(1, 2, false);
-        else if (mt_built == 1) NNHIP_ROPE_LAUNCH(1, kRowsPieces, false);
-        else if (two_pieces) NNHIP_ROPE_LAUNCH(2, 2, false);
-        else NNHIP_ROPE_LAUNCH(2, kRowsPieces, false);
-#undef NNHIP_ROPE_LAUNCH
-        NNHIP_LAUNCH_CHECK(ctx, "w8a16_gemm_rows_in_lds_kernel");
+        if (a.ln_w) return launch_tile_normalising<2, true>(ctx, a, w->ntiles / 2);
+        return launch_tile<2, 2, false, 1, 1, true>(ctx, a, w->ntiles / 2);
+    }
+    const GemmForm form = gemm_form(ctx, w, m, glu, a.ln_w != nullptr);
+    if (form == GemmForm::kTile) {
+        if (a.ln_w) return glu ? launch_tile_normalising<2>(ctx, a, out_tiles) : launch_tile_normalising<1>(ctx, a, out_tiles);
+        return glu ? launch_tile_plain<2>(ctx, a, out_tiles) : launch_tile_plain<1>(ctx, a, out_tiles);
+    }
+    if (form == GemmForm::kSmallTile) {
+        hipLaunchKernelGGL((w8a16_small_tile_kernel<kTileMaxK / 1024>), dim3(out_tiles * 2, (m + 7) / 8), dim3(kGemmThreads), 0, ctx->stream, a);
+        NNHIP_LAUNCH_CHECK(ctx, "w8a16_small_tile_kernel");
         return 0;
     }
-    const bool short_rows = w->k <= 1024; // rows of two 512-element pieces (a lane keeps a row's pieces in registers)
-    if (split && glu && w->k <= kRowsMaxK && rows_lds <= 64 * 1024 && mt_built <= 2 && // (with or without rows to normalise: one summation order)
-        (w->ksteps + kGluSplitWaves - 1) / kGluSplitWaves <= 4) {
-        // the gate / up projection of a decode step (a few hundred tile pairs over a short reduction): a block per tile
-        // pair, its waves splitting the reduction, so that every compute unit takes part.  Four waves for 32 rows (eight
-        // took 12.8 against 10.7 us); eight for 16 rows, where a wave then brings in and normalises two rows instead of
-        // four (the decode step of two lanes: 1.097 against 1.114 ms)
-#define NNHIP_GLU_SPLIT_LAUNCH(MTV, PV, GWV, KBV, FEWV)                                                                              \
-    do {                                                                                                                       \
-        NNHIP_HIP(ctx, raise_dynamic_lds(w8a16_gemm_rows_in_lds_kernel<MTV, 2, GWV, true, KBV, PV, false, FEWV>, ctx->device,              \
-                                         rows_lds + GWV * 2 * MTV * 1024, 96 * 1024));                                         \
-        hipLaunchKernelGGL((w8a16_gemm_rows_in_lds_kernel<MTV, 2, GWV, true, KBV, PV, false, FEWV>), grid, dim3(GWV * 64), rows_lds, ctx->stream, a); \
-    } while (0)
-        const bool two_steps = (w->ksteps + 7) / 8 <= 2; // a wave's share of the reduction with eight waves
-        if (m <= 8 && short_rows && two_steps) NNHIP_GLU_SPLIT_LAUNCH(1, 2, 8, 2, true);
-        else if (m <= 8 && short_rows) NNHIP_GLU_SPLIT_LAUNCH(1, 2, 8, 4, true);
-        else if (m <= 8) NNHIP_GLU_SPLIT_LAUNCH(1, kRowsPieces, 8, 4, true);
-        else if (mt_built == 1 && short_rows && two_steps) NNHIP_GLU_SPLIT_LAUNCH(1, 2, 8, 2, false);
-        else if (mt_built == 1 && short_rows) NNHIP_GLU_SPLIT_LAUNCH(1, 2, 8, 4, false);
-        else if (mt_built == 1) NNHIP_GLU_SPLIT_LAUNCH(1, kRowsPieces, 8, 4, false);
-        else if (short_rows) NNHIP_GLU_SPLIT_LAUNCH(2, 2, kGluSplitWaves, 4, false);
-        else NNHIP_GLU_SPLIT_LAUNCH(2, kRowsPieces, kGluSplitWaves, 4, false);
-#undef NNHIP_GLU_SPLIT_LAUNCH
-        NNHIP_LAUNCH_CHECK(ctx, "w8a16_gemm_rows_in_lds_kernel");
-        return 0;
-    }
-    if (!glu && rows_take_split(ctx, w, m) && (ln_weight_dev || out_tiles >= ctx->compute_units)) {
-        // few tiles (the q / k / v projection): the reduction split over the block's waves, the rows parked and normalised
-        // in LDS in one trip to memory; fewer tiles than compute units and nothing to normalise: the kernel below that
-        // reads the rows where they lie (the same order)
-        // (the kernel's static reduction area comes on top of the rows: past 48 KiB in all, the limit is raised like below)
-        // (a wave's share of the reduction is requested at once where it is at most two k-steps, the decode step's case)
-        const bool short_share = (w->ksteps + kGemmWaves - 1) / kGemmWaves <= 2;
-#define NNHIP_SPLIT_ROWS_LAUNCH_P(MTV, KBV, PV, FEWV)                                                                                \
-    do {                                                                                                                       \
-        NNHIP_HIP(ctx, raise_dynamic_lds(w8a16_gemm_rows_in_lds_kernel<MTV, 1, kGemmWaves, true, KBV, PV, false, FEWV>, ctx->device,       \
-                                         rows_lds + MTV * 8 * 1024, 64 * 1024));                                               \
-        hipLaunchKernelGGL((w8a16_gemm_rows_in_lds_kernel<MTV, 1, kGemmWaves, true, KBV, PV, false, FEWV>), grid, block, rows_lds, ctx->stream, a); \
-    } while (0)
-#define NNHIP_SPLIT_ROWS_LAUNCH(MTV, KBV)                                                                                      \
-    do {                                                                                                                       \
-        if (m <= kGemmWaves && short_rows) NNHIP_SPLIT_ROWS_LAUNCH_P(1, KBV, 2, true);                                        \
-        else if (m <= kGemmWaves) NNHIP_SPLIT_ROWS_LAUNCH_P(1, KBV, kRowsPieces, true);                                       \
-        else if (short_rows) NNHIP_SPLIT_ROWS_LAUNCH_P(MTV, KBV, 2, false);                                                   \
-        else NNHIP_SPLIT_ROWS_LAUNCH_P(MTV, KBV, kRowsPieces, false);                                                                 \
-    } while (0)
-        if (mt_built == 1) {
-            if (short_share) NNHIP_SPLIT_ROWS_LAUNCH(1, 2);
-            else NNHIP_SPLIT_ROWS_LAUNCH(1, kRowsBatch);
-        } else {
-            if (short_share) NNHIP_SPLIT_ROWS_LAUNCH(2, 2);
-            else NNHIP_SPLIT_ROWS_LAUNCH(2, kRowsBatch);
-        }
-#undef NNHIP_SPLIT_ROWS_LAUNCH
-#undef NNHIP_SPLIT_ROWS_LAUNCH_P
-        NNHIP_LAUNCH_CHECK(ctx, "w8a16_gemm_rows_in_lds_kernel");
-        return 0;
-    }
-    if (w->k <= kRowsMaxK && rows_lds <= 128 * 1024 && out_tiles >= ctx->compute_units) {
+    const bool split = form == GemmForm::kSplit;
+    const bool paired = split && !glu && sums_in_pairs(ctx, w, m);
+    const dim3 grid(split ? out_tiles : (out_tiles + kGemmWaves - 1) / kGemmWaves), block(kGemmThreads);
+    if (form == GemmForm::kRowsInLds) {
+        const int mt_built = mt <= 1 ? 1 : (mt == 2 ? 2 : 4);
+        const size_t rows_lds = (size_t)mt_built * 16 * rows_in_lds_pitch(w->k);
+        const bool short_rows = w->k <= 1024; // rows of two 512-element pieces (a lane keeps a row's pieces in registers)
         // (at most two blocks per compute unit, each walking several groups of eight tiles: what a block repeats -- the
         // rows' trip and their normalisation -- is then paid twice per compute unit, not once per group)
         const dim3 rgrid(std::min((out_tiles + kGemmWaves - 1) / kGemmWaves, 2 * ctx->compute_units)), rblock(kGemmThreads);
@@ -958,8 +1109,8 @@ static int launch_w8a16_gemm(nncase_hip_ctx_t *ctx, const void *a_dev, const nnc
         // vocabulary head needs for occupancy -- 50.7 against 43.9 us when it still ran as 1187 one-group blocks)
 #define NNHIP_ROWS_LAUNCH_KB(MTV, GV, KBV, PV)                                                                                 \
     do {                                                                                                                       \
-        NNHIP_HIP(ctx, raise_dynamic_lds(w8a16_gemm_rows_in_lds_kernel<MTV, GV, kGemmWaves, false, KBV, PV>, ctx->device, rows_lds + 1024, 128 * 1024)); \
-        hipLaunchKernelGGL((w8a16_gemm_rows_in_lds_kernel<MTV, GV, kGemmWaves, false, KBV, PV>), rgrid, rblock, rows_lds, ctx->stream, a); \
+        NNHIP_HIP(ctx, raise_dynamic_lds(w8a16_gemm_rows_in_lds_kernel<MTV, GV, KBV, PV>, ctx->device, rows_lds + 1024, 128 * 1024)); \
+        hipLaunchKernelGGL((w8a16_gemm_rows_in_lds_kernel<MTV, GV, KBV, PV>), rgrid, rblock, rows_lds, ctx->stream, a); \
     } while (0)
 #define NNHIP_ROWS_LAUNCH(MTV, GV)                                                                                             \
     do {                                                                                                                       \
@@ -980,19 +1131,15 @@ static int launch_w8a16_gemm(nncase_hip_ctx_t *ctx, const void *a_dev, const nnc
         NNHIP_LAUNCH_CHECK(ctx, "w8a16_gemm_rows_in_lds_kernel");
         return 0;
     }
-    // a share of 9 or 10 k-steps per wave (the 4864-deep down projection): one request of all ten for up to 16 token rows,
-    // two of five for up to 32 (whose slices of ten k-steps do not fit the registers), instead of 4 + 4 + 2
-    const int share = (w->ksteps + kGemmWaves - 1) / kGemmWaves;
-    const bool long_share = !ln_weight_dev && mt <= 2 && (share == 9 || share == 10);
 #define NNHIP_GEMM_LAUNCH(MTV)                                                                                                 \
     do {                                                                                                                       \
         if (glu && split) hipLaunchKernelGGL((w8a16_gemm_kernel<MTV, 2, true>), grid, block, 0, ctx->stream, a);              \
         else if (glu) hipLaunchKernelGGL((w8a16_gemm_kernel<MTV, 2, false>), grid, block, 0, ctx->stream, a);                 \
-        else if (split && long_share) hipLaunchKernelGGL((w8a16_gemm_kernel<(MTV <= 2 ? MTV : 2), 1, true, (MTV == 1 ? 10 : 5)>), grid, block, 0, ctx->stream, a); \
         else if (split) hipLaunchKernelGGL((w8a16_gemm_kernel<MTV, 1, true>), grid, block, 0, ctx->stream, a);                \
         else hipLaunchKernelGGL((w8a16_gemm_kernel<MTV, 1, false>), grid, block, 0, ctx->stream, a);                          \
     } while (0)
-    if (mt == 1) NNHIP_GEMM_LAUNCH(1);
+    if (paired) hipLaunchKernelGGL((w8a16_gemm_kernel<1, 1, true, true>), grid, block, 0, ctx->stream, a); // (one token tile)
+    else if (mt == 1) NNHIP_GEMM_LAUNCH(1);
     else if (mt == 2) NNHIP_GEMM_LAUNCH(2);
     else NNHIP_GEMM_LAUNCH(4);
 #undef NNHIP_GEMM_LAUNCH

@@ -379,3 +379,27 @@ def test_rmsnorm_fused_into_gemm_of_one_to_four_tiles_per_compute_unit(hip_ctx, 
 def test_projection_of_many_heads_that_rotates_and_appends(hip_ctx, B, k, norm, hq, hkv):
     """One to four output tiles per compute unit, and more (two launches): the projection's own order of adding."""
     test_projection_that_rotates_and_appends_equals_the_two_operators(hip_ctx, B, k, norm, hq, hkv)
+
+
+@pytest.mark.parametrize("m,k,n", [(1, 64, 16), (17, 448, 32), (33, 1024, 48), (64, 1088, 144), (49, 2048, 16), (16, 2112, 112), (1, 4864, 128),
+                                   (9, 4096, 2048), (8, 5120, 4096), (16, 2176, 2048), (16, 2176, 2064), (17, 2176, 2048), (3, 5184, 64)])
+def test_products_of_a_tile_per_block(hip_ctx, m, k, n):
+    """Tiles of 16 x 16 over several row tiles and of 8 x 8, at the ends of the reductions that each takes (512 k-steps of a wave's
+    registers, 5120; beyond it the general kernel), with shares that leave waves idle or with an odd step, and where the last group
+    of eight tiles is not full."""
+    for out32 in (False, True):
+        test_w8a16_gemm(hip_ctx, m, k, n, out32)
+
+
+@pytest.mark.parametrize("m,k,n,mode", [(16, 4864, 896, "residual"), (8, 2112, 2048, "plain"), (1, 5120, 1024, "f32"), (9, 2112, 48, "plain"),
+                                        (17, 2112, 2048, "plain"), (16, 5184, 128, "f32"), (64, 896, 1152, "plain"), (33, 1024, 8176, "plain"),
+                                        (33, 1024, 8192, "plain"), (64, 896, 9728, "swiglu"), (64, 512, 16384, "swiglu"), (16, 2112, 512, "swiglu")])
+def test_rmsnorm_fused_into_gemm_over_row_tiles_and_long_reductions(hip_ctx, m, k, n, mode):
+    """One order of adding whether the rows are normalised on the way or before: 8 x 8 tiles against the general kernel's, and
+    row tiles on either side of the rules for splitting a reduction."""
+    test_rmsnorm_fused_into_gemm_equals_the_two_operators(hip_ctx, m, k, n, mode)
+
+
+@pytest.mark.parametrize("B,k,norm", [(17, 896, True), (33, 1024, True), (64, 896, True), (64, 512, False)])
+def test_projection_over_row_tiles_that_rotates_and_appends(hip_ctx, B, k, norm):
+    test_projection_that_rotates_and_appends_equals_the_two_operators(hip_ctx, B, k, norm)
