@@ -55,6 +55,7 @@ struct AttnArgs {
     FastDiv d_block;
     float scale_log2e;
     int out_f16;
+    WeightFetches fetch;
 };
 
 __device__ __forceinline__ void coherent_store(float *p, float v) {
@@ -135,6 +136,26 @@ __device__ __forceinline__ void merge_splits(const AttnArgs &a, int ns, int G, s
     }
 }
 
+// What the blocks of the grid's second and further planes do: bring fragments of the weights that the next products read into the
+// L2 of the die whose blocks will ask for them; the loads' results are dropped.  While the blocks of the first plane wait for one
+// memory round trip after another, the memory would be idle: one sequence of 700 tokens, a decode layer with its 14.9 MB of
+// weights fetched 24.8 -> 22.9 us.  (Fetched by the products' own launches instead, or by them too, it takes 23.7 to 26.7.)
+// A wave has one batch of fragments, all of them under way at once.
+constexpr int kFetchBatch = 8;
+template <int W> __device__ __forceinline__ void fetch_weights(const AttnArgs &a) {
+    const uint32_t pairs = a.hkv * a.batch, block = ((uint32_t)blockIdx.z * a.splits + blockIdx.y) * pairs + blockIdx.x;
+    const uint32_t x = block % kXcds, p = (block - pairs * a.splits) / kXcds; // (every eight consecutive blocks have one on each die)
+    const uint32_t lane = threadIdx.x & 63, u0 = p * W + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), stride = (uint32_t)a.fetch.blocks * W;
+    uint32_t n = 0;
+    for (int i = 0; i < a.fetch.count; i++) n += fetch_fragments(a.fetch.f[i], x);
+    if (p >= (uint32_t)a.fetch.blocks || u0 >= n) return;
+    au32x4 v[kFetchBatch];
+#pragma unroll
+    for (int k = 0; k < kFetchBatch; k++) v[k] = reinterpret_cast<const au32x4 *>(fetch_address(a.fetch, x, min(u0 + k * stride, n - 1)))[lane];
+#pragma unroll
+    for (int k = 0; k < kFetchBatch; k++) asm volatile("" ::"v"(v[k]));
+}
+
 // NT = 16-token tiles per wave (even); W = waves per block (a block owns W * NT * 16 tokens).
 template <int D, int NT, int W> __global__ __launch_bounds__(W * 64, W <= 8 ? 2 : 1) void paged_attn_kernel(const AttnArgs a) {
     constexpr int kAttnWaves = W, kAttnThreads = W * 64;
@@ -148,6 +169,10 @@ template <int D, int NT, int W> __global__ __launch_bounds__(W * 64, W <= 8 ? 2 
     float(*ssum)[kAttnHeads] = smax + W;                                                                            // [W][heads]
     __shared__ uint32_t s_last;
 
+    if (blockIdx.z != 0) { // (a branch on an argument would put its load's trip in front of the others')
+        fetch_weights<W>(a);
+        return;
+    }
     // kv head fastest, then sequence, then split: consecutive workgroups go to different XCDs, so
     // every XCD gets the same mix of early (always present) and late (long contexts only) splits
     const int kvh = blockIdx.x % a.hkv, b = blockIdx.x / a.hkv, split = blockIdx.y;
@@ -430,7 +455,8 @@ static int attn_plan(nncase_hip_ctx *ctx, const nncase_hip_paged_attn_args_t *p,
 }
 
 static int attn_launch(nncase_hip_ctx *ctx, AttnPlan &plan, const void *q_dev, const void *k_cache_dev, const void *v_cache_dev,
-                       const int32_t *block_table_dev, const int32_t *ctx_lens_dev, void *out_dev, void *partials, void *counters) {
+                       const int32_t *block_table_dev, const int32_t *ctx_lens_dev, void *out_dev, void *partials, void *counters,
+                       const WeightFetches *fetch = nullptr) {
     AttnArgs &a = plan.a;
     a.q = (const uint16_t *)q_dev;
     a.k_cache = (const uint16_t *)k_cache_dev;
@@ -441,8 +467,19 @@ static int attn_launch(nncase_hip_ctx *ctx, AttnPlan &plan, const void *q_dev, c
     a.done = reinterpret_cast<uint32_t *>(counters);
     a.part_o = reinterpret_cast<float *>(partials);
     a.part_ml = a.part_o + (size_t)a.batch * a.hq * a.splits * a.d;
-    const dim3 grid(a.hkv * a.batch, a.splits);
     const int nt = plan.nt, waves = plan.waves;
+    dim3 grid(a.hkv * a.batch, a.splits);
+    const int64_t own = (int64_t)grid.x * grid.y;
+    // Weights are fetched beside launches that merge splits (one that does not is over before they are here: 8 sequences of 100
+    // tokens, a decode layer 25.2 -> 25.5 us) and that leave memory idle (64 sequences of 2048, 1152 blocks: 49.3 -> 49.7; 32 of
+    // them, 576 blocks: 39.8 -> 39.5; one of 700, 12 blocks: 24.8 -> 22.9).
+    if (fetch && fetch->count > 0 && a.splits > 1 && own <= 3 * ctx->compute_units) {
+        a.fetch = *fetch;
+        uint32_t fragments = 0; // of die 0, which has the most
+        for (int i = 0; i < fetch->count; i++) fragments += fetch_fragments(fetch->f[i], 0);
+        a.fetch.blocks = (int)((fragments + waves * kFetchBatch - 1) / (waves * kFetchBatch));
+        grid.z = 1 + (unsigned)(((int64_t)a.fetch.blocks * kXcds + own - 1) / own);
+    }
     const dim3 block(waves * 64);
     const size_t lds = attn_lds_bytes(a.d, waves);
     bool launched = false;
@@ -528,14 +565,28 @@ int attn_scratch_sizes(nncase_hip_ctx *ctx, const nncase_hip_paged_attn_args_t *
 
 int attn_decode_on(nncase_hip_ctx *ctx, const void *q_dev, const void *k_cache_dev, const void *v_cache_dev, const int32_t *block_table_dev,
                    const int32_t *ctx_lens_dev, void *out_dev, const nncase_hip_paged_attn_args_t *p, void *partials,
-                   size_t partial_bytes, void *counters, size_t counter_bytes) {
+                   size_t partial_bytes, void *counters, size_t counter_bytes, const WeightFetches *fetch) {
     AttnPlan plan;
     const int rc = attn_plan(ctx, p, &plan);
     if (rc) return rc;
     NNHIP_REQUIRE(ctx, partials && counters && plan.partial_bytes <= partial_bytes && plan.counter_bytes <= counter_bytes, -ENOSPC,
                   "paged_attention_decode: the scratch areas brought along hold %zu and %zu bytes, the geometry needs %zu and %zu",
                   partial_bytes, counter_bytes, plan.partial_bytes, plan.counter_bytes);
-    return attn_launch(ctx, plan, q_dev, k_cache_dev, v_cache_dev, block_table_dev, ctx_lens_dev, out_dev, partials, counters);
+    return attn_launch(ctx, plan, q_dev, k_cache_dev, v_cache_dev, block_table_dev, ctx_lens_dev, out_dev, partials, counters, fetch);
+}
+
+int attn_decode_on_context(nncase_hip_ctx *ctx, const void *q_dev, const void *k_cache_dev, const void *v_cache_dev,
+                           const int32_t *block_table_dev, const int32_t *ctx_lens_dev, void *out_dev,
+                           const nncase_hip_paged_attn_args_t *p, const WeightFetches *fetch) {
+    AttnPlan plan;
+    int rc = attn_plan_on_context(ctx, p, &plan);
+    if (rc) return rc;
+    if (!attn_fits(ctx, plan)) {
+        rc = attn_reserve(ctx, p);
+        if (rc) return rc;
+    }
+    return attn_launch(ctx, plan, q_dev, k_cache_dev, v_cache_dev, block_table_dev, ctx_lens_dev, out_dev, ctx->attn_ws,
+                       ctx->attn_done, fetch);
 }
 
 } // namespace nnhip
@@ -549,15 +600,7 @@ extern "C" int nncase_hip_paged_attention_decode(nncase_hip_ctx_t *ctx, const vo
     NNHIP_CHECK_CTX(ctx);
     NNHIP_REQUIRE(ctx, q_dev && k_cache_dev && v_cache_dev && block_table_dev && ctx_lens_dev && out_dev && p, -EINVAL,
                   "paged_attention_decode: null argument");
-    AttnPlan plan;
-    int rc = attn_plan_on_context(ctx, p, &plan);
-    if (rc) return rc;
-    if (!attn_fits(ctx, plan)) {
-        rc = attn_reserve(ctx, p);
-        if (rc) return rc;
-    }
-    return attn_launch(ctx, plan, q_dev, k_cache_dev, v_cache_dev, block_table_dev, ctx_lens_dev, out_dev, ctx->attn_ws,
-                       ctx->attn_done);
+    return attn_decode_on_context(ctx, q_dev, k_cache_dev, v_cache_dev, block_table_dev, ctx_lens_dev, out_dev, p, nullptr);
 }
 
 extern "C" int nncase_hip_paged_attention_decode_noalloc(nncase_hip_ctx_t *ctx, const void *q_dev, const void *k_cache_dev,

@@ -11,6 +11,7 @@
 #include <cstring>
 
 #include "../../include/nncase_hip.h"
+#include "weight_fetch.hpp"
 
 struct nncase_hip_ctx {
     int device = 0;
@@ -182,7 +183,15 @@ int attn_reserve(nncase_hip_ctx *ctx, const nncase_hip_paged_attn_args_t *geomet
 int attn_scratch_sizes(nncase_hip_ctx *ctx, const nncase_hip_paged_attn_args_t *geometry, size_t *partial_bytes, size_t *counter_bytes);
 int attn_decode_on(nncase_hip_ctx *ctx, const void *q_dev, const void *k_cache_dev, const void *v_cache_dev, const int32_t *block_table_dev,
                    const int32_t *ctx_lens_dev, void *out_dev, const nncase_hip_paged_attn_args_t *geometry, void *partials,
-                   size_t partial_bytes, void *counters, size_t counter_bytes);
+                   size_t partial_bytes, void *counters, size_t counter_bytes, const WeightFetches *fetch);
+// The launch on the context's own areas.  `fetch` (may be null): weights that the operators behind it will read.
+int attn_decode_on_context(nncase_hip_ctx *ctx, const void *q_dev, const void *k_cache_dev, const void *v_cache_dev,
+                           const int32_t *block_table_dev, const int32_t *ctx_lens_dev, void *out_dev,
+                           const nncase_hip_paged_attn_args_t *geometry, const WeightFetches *fetch);
+// llm.hip: which weights each block of a product of m rows reads; false where its launch is of another kind.  rope: the q / k / v
+// projection that rotates and appends.
+bool w8a16_weight_fetch(const nncase_hip_ctx *ctx, const nncase_hip_w8a16_t *w, int m, int mode, bool normalises,
+                        const nncase_hip_paged_attn_args_t *rope, WeightFetch *f);
 
 // glue.hip: a max pool of stride 1 over its own result, `levels` times, and the channel concat of the tensor and all levels.
 struct MaxPoolChain {

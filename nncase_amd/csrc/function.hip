@@ -63,6 +63,30 @@ struct nncase_hip_function {
 
 using namespace nnhip;
 
+// The weights that the operators between an attention and the next one of its lane will read.  A decode step's attention waits for
+// memory most of the time it runs and moves little, its products wait for weights that no cache has kept since the last step: the
+// one brings them into the caches for the others.
+static WeightFetches weights_behind(const nncase_hip_function *fn, const Op &attn) {
+    WeightFetches s;
+    memset(&s, 0, sizeof(s));
+    size_t bytes = 0;
+    for (size_t i = (size_t)(&attn - fn->ops.data()) + 1; i < fn->ops.size() && s.count < kMaxWeightFetches; i++) {
+        const Op &op = fn->ops[i];
+        if (op.lane != attn.lane) continue;
+        if (op.kind == Op::kAttn) break;
+        if (op.kind != Op::kGemm && op.kind != Op::kGemmRope) continue;
+        const bool rope = op.kind == Op::kGemmRope;
+        WeightFetch f;
+        if (!w8a16_weight_fetch(fn->ctx, op.w8, rope ? op.attn.batch : op.batch, op.mode, rope ? op.in1 != nullptr : op.in2 != nullptr,
+                                rope ? &op.attn : nullptr, &f))
+            continue;
+        bytes += (size_t)f.blocks * f.per_block * f.steps * 1024;
+        if (bytes > kMaxFetchBytes) break;
+        s.f[s.count++] = f;
+    }
+    return s;
+}
+
 static int run_op(nncase_hip_function *fn, const Op &op) {
     nncase_hip_ctx *ctx = fn->ctx;
     switch (op.kind) {
@@ -111,13 +135,14 @@ static int run_op(nncase_hip_function *fn, const Op &op) {
     case Op::kRope:
         return nncase_hip_rope_kv_append(ctx, op.in0, op.out, op.out2, op.out3, (const int32_t *)op.in2, (const int32_t *)op.in3,
                                          &op.attn, op.eps);
-    case Op::kAttn:
+    case Op::kAttn: {
+        const WeightFetches fetch = weights_behind(fn, op);
         if (op.lane > 0)
             return attn_decode_on(ctx, op.in0, op.in1, op.in2, (const int32_t *)op.in3, (const int32_t *)op.in4, op.out, &op.attn,
                                   fn->lane_partials[op.lane], fn->lane_partial_bytes[op.lane], fn->lane_counters[op.lane],
-                                  fn->lane_counter_bytes[op.lane]);
-        return nncase_hip_paged_attention_decode(ctx, op.in0, op.in1, op.in2, (const int32_t *)op.in3, (const int32_t *)op.in4,
-                                                 op.out, &op.attn);
+                                  fn->lane_counter_bytes[op.lane], &fetch);
+        return attn_decode_on_context(ctx, op.in0, op.in1, op.in2, (const int32_t *)op.in3, (const int32_t *)op.in4, op.out, &op.attn, &fetch);
+    }
     case Op::kArgmax:
         return nncase_hip_argmax_f32(ctx, (const float *)op.in0, (int32_t *)op.out, op.batch, op.channels);
     case Op::kEmbed:

@@ -1147,6 +1147,28 @@ static int launch_w8a16_gemm(nncase_hip_ctx_t *ctx, const void *a_dev, const nnc
     return 0;
 }
 
+bool nnhip::w8a16_weight_fetch(const nncase_hip_ctx *ctx, const nncase_hip_w8a16_t *w, int m, int mode, bool normalises,
+                               const nncase_hip_paged_attn_args_t *rope, WeightFetch *f) {
+    const bool glu = mode == NNCASE_HIP_GEMM_SWIGLU;
+    f->packed = w->d_packed;
+    f->steps = (uint32_t)w->ksteps;
+    if (rope) {
+        RopeArgs r;
+        memset(&r, 0, sizeof(r));
+        r.hq = rope->num_q_heads, r.hkv = rope->num_kv_heads, r.d = rope->head_dim;
+        if (rope_epilogue_fits(ctx, w, m, r)) {
+            f->blocks = (uint32_t)w->ntiles / 2, f->off = (uint32_t)r.d / 32, f->per_block = 2;
+            return true;
+        }
+    }
+    const GemmForm form = gemm_form(ctx, w, m, glu, normalises);
+    if (form == GemmForm::kRowsInLds || form == GemmForm::kPerWave) return false;
+    // (kSmallTile: two blocks a tile, on the die that a block per tile would be on)
+    f->blocks = f->off = (uint32_t)(glu ? w->ntiles / 2 : w->ntiles);
+    f->per_block = glu ? 2 : 1;
+    return true;
+}
+
 extern "C" int nncase_hip_w8a16_gemm(nncase_hip_ctx_t *ctx, const void *a_dev, const nncase_hip_w8a16_t *w, void *out_dev,
                                      int32_t m, int32_t mode, const void *residual_dev, int32_t out_dtype) {
     return launch_w8a16_gemm(ctx, a_dev, w, out_dev, m, mode, residual_dev, out_dtype, nullptr, 0.f);
