@@ -723,7 +723,8 @@ NNCASE_HIP_API int nncase_hip_function_size(nncase_hip_function_t *fn, int32_t *
 NNCASE_HIP_API int nncase_hip_function_invoke(nncase_hip_function_t *fn);
 /* Enqueues operator `index` alone (per-operator timing and debugging). */
 NNCASE_HIP_API int nncase_hip_function_invoke_one(nncase_hip_function_t *fn, int32_t index);
-/* Captures the operator sequence into a HIP graph used by later invokes. */
+/* Captures the operator sequence into HIP graphs used by later invokes: one per lane, lanes other than 0 replayed on streams
+ * that belong to the context, forked from its stream and joined back into it. */
 NNCASE_HIP_API int nncase_hip_function_capture(nncase_hip_function_t *fn);
 /* Per-operator device time: every operator is enqueued `iterations` times
  * back to back between two HIP events recorded on the context's stream and

@@ -9,6 +9,7 @@
 #include <cstdint>
 #include <cstdio>
 #include <cstring>
+#include <mutex>
 
 #include "../../include/nncase_hip.h"
 #include "weight_fetch.hpp"
@@ -41,6 +42,12 @@ struct nncase_hip_ctx {
     hipStream_t copy_stream = nullptr; // results on their way to the host beside the context's stream
     static constexpr int kCopySlots = 8;
     hipEvent_t copy_events[kCopySlots] = {nullptr};
+    // function.hip: lanes 1.. of captured functions run on streams of their own, forked from the context's stream and joined back
+    // into it; made when the first function with lanes is captured, kept with the context (calls on one context are ordered on its
+    // stream, so its functions can share them)
+    hipStream_t lane_streams[NNCASE_HIP_MAX_LANES] = {nullptr};
+    hipEvent_t lane_events[NNCASE_HIP_MAX_LANES] = {nullptr}; // 0: the fork, l: the end of lane l
+    std::mutex lane_lock;                                     // two threads' forks and joins do not mix
     char last_error[512] = {0};
 };
 
@@ -63,6 +70,10 @@ int drain_host_calls(nncase_hip_ctx *ctx); // waits for the context's stream
 bool host_is_pinned(const void *ptr);      // a block of nncase_hip_host_malloc
 void hostcall_attach();
 void hostcall_release(nncase_hip_ctx *ctx);
+
+// function.hip: the context's lane streams and events, up to `lanes`; given back with the context.
+int lane_streams_reserve(nncase_hip_ctx *ctx, int lanes);
+void lane_streams_release(nncase_hip_ctx *ctx);
 
 // function.hip: a loaded model's list prepared for, and run with, results that go to host memory (complete on return).
 void function_hoist_outputs(nncase_hip_function_t *fn, void *const *outputs_dev, int n);

@@ -97,6 +97,7 @@ extern "C" int nncase_hip_ctx_destroy(nncase_hip_ctx_t *ctx) {
     if (ctx->attn_ws) (void)hipFree(ctx->attn_ws);
     if (ctx->attn_done) (void)hipFree(ctx->attn_done);
     hostcall_release(ctx);
+    lane_streams_release(ctx);
     if (ctx->owns_stream && ctx->stream) (void)hipStreamDestroy(ctx->stream);
     delete ctx;
     return 0;

@@ -1,5 +1,5 @@
 // Resident functions: an ordered operator list bound to device operands,
-// replayable eagerly or as one HIP graph.
+// replayable eagerly or as HIP graphs, one per lane.
 #include "qconv.hpp"
 
 #include <algorithm>
@@ -52,8 +52,9 @@ struct nncase_hip_function {
     nncase_hip_ctx *ctx = nullptr;
     std::vector<Op> ops;
     int cur_lane = 0, nlanes = 1;
-    hipGraph_t graph = nullptr;
-    hipGraphExec_t exec = nullptr;
+    // captured: a graph per lane and one of what was recorded behind their join (see nncase_hip_function_invoke)
+    hipGraphExec_t lane_exec[NNCASE_HIP_MAX_LANES] = {nullptr}, joined_exec = nullptr;
+    bool captured = false;
     bool pins_attn = false; // the captured graph holds the addresses of the context's attention workspace
     // Paged attention on a lane other than 0 goes through split partials and counters of that lane's own (lane 0
     // uses the context's), so that lanes may run it side by side; owned by the function.
@@ -202,12 +203,32 @@ static int run_ops(nncase_hip_function *fn, size_t at, size_t *next) {
 }
 
 static void drop_graph(nncase_hip_function *fn) {
-    if (fn->exec) (void)hipGraphExecDestroy(fn->exec);
-    if (fn->graph) (void)hipGraphDestroy(fn->graph);
-    fn->exec = nullptr;
-    fn->graph = nullptr;
+    for (hipGraphExec_t &e : fn->lane_exec) {
+        if (e) (void)hipGraphExecDestroy(e);
+        e = nullptr;
+    }
+    if (fn->joined_exec) (void)hipGraphExecDestroy(fn->joined_exec);
+    fn->joined_exec = nullptr;
+    fn->captured = false;
     if (fn->pins_attn) fn->ctx->attn_pins--;
     fn->pins_attn = false;
+}
+
+int nnhip::lane_streams_reserve(nncase_hip_ctx *ctx, int lanes) {
+    std::lock_guard<std::mutex> guard(ctx->lane_lock);
+    for (int l = 0; l < lanes; l++) {
+        if (!ctx->lane_events[l]) NNHIP_HIP(ctx, hipEventCreateWithFlags(&ctx->lane_events[l], hipEventDisableTiming));
+        if (l > 0 && !ctx->lane_streams[l]) NNHIP_HIP(ctx, hipStreamCreateWithFlags(&ctx->lane_streams[l], hipStreamNonBlocking));
+    }
+    return 0;
+}
+
+void nnhip::lane_streams_release(nncase_hip_ctx *ctx) {
+    for (int l = 0; l < NNCASE_HIP_MAX_LANES; l++) {
+        if (ctx->lane_events[l]) (void)hipEventDestroy(ctx->lane_events[l]);
+        if (ctx->lane_streams[l]) (void)hipStreamDestroy(ctx->lane_streams[l]);
+        ctx->lane_events[l] = nullptr, ctx->lane_streams[l] = nullptr;
+    }
 }
 
 static int push(nncase_hip_function *fn, const Op &op) {
@@ -533,7 +554,7 @@ extern "C" int nncase_hip_function_add_paged_attention_decode(nncase_hip_functio
         const int rc = attn_scratch_sizes(fn->ctx, args, &pb, &cb);
         if (rc) return rc;
         if (pb > fn->lane_partial_bytes[lane] || cb > fn->lane_counter_bytes[lane]) {
-            NNHIP_REQUIRE(fn->ctx, !fn->exec, -EBUSY, "function_add_paged_attention_decode: the lane's scratch would grow under a captured graph");
+            NNHIP_REQUIRE(fn->ctx, !fn->captured, -EBUSY, "function_add_paged_attention_decode: the lane's scratch would grow under a captured graph");
             NNHIP_HIP(fn->ctx, hipStreamSynchronize(fn->ctx->stream)); // earlier eager invocations may still use the old areas
             if (pb > fn->lane_partial_bytes[lane]) {
                 if (fn->lane_partials[lane]) NNHIP_HIP(fn->ctx, hipFree(fn->lane_partials[lane]));
@@ -629,7 +650,7 @@ void nnhip::function_hoist_outputs(nncase_hip_function_t *fn, void *const *outpu
 
 int nnhip::function_run_to_host(nncase_hip_function_t *fn, int n, void *const *outputs_dev, void *const *outputs_host, const size_t *bytes) {
     nncase_hip_ctx *ctx = fn->ctx;
-    if (fn->exec) {
+    if (fn->captured) {
         if (int rc = nncase_hip_function_invoke(fn)) return rc;
     }
     // results that lie in pinned memory leave on a stream of their own as soon as they are complete, in the order they are
@@ -639,7 +660,7 @@ int nnhip::function_run_to_host(nncase_hip_function_t *fn, int n, void *const *o
     std::vector<Early> early;
     auto enqueue = [&]() -> int {
         const std::vector<Op> &ops = fn->ops;
-        for (size_t k = 0, next = 0; !fn->exec && next < ops.size();) {
+        for (size_t k = 0, next = 0; !fn->captured && next < ops.size();) {
             const size_t first = next;
             if (int rc = run_ops(fn, first, &next)) return rc;
             k = next - 1;
@@ -675,12 +696,59 @@ int nnhip::function_run_to_host(nncase_hip_function_t *fn, int n, void *const *o
 
 extern "C" int nncase_hip_function_invoke(nncase_hip_function_t *fn) {
     if (!fn) return -EINVAL;
-    if (fn->exec) {
-        NNHIP_HIP(fn->ctx, hipGraphLaunch(fn->exec, fn->ctx->stream));
+    nncase_hip_ctx *ctx = fn->ctx;
+    if (!fn->captured) {
+        for (size_t k = 0; k < fn->ops.size();)
+            if (int rc = run_ops(fn, k, &k)) return rc;
         return 0;
     }
-    for (size_t k = 0; k < fn->ops.size();)
-        if (int rc = run_ops(fn, k, &k)) return rc;
+    if (fn->nlanes == 1) {
+        for (hipGraphExec_t e : {fn->lane_exec[0], fn->joined_exec})
+            if (e) NNHIP_HIP(ctx, hipGraphLaunch(e, ctx->stream));
+        return 0;
+    }
+    // Lanes side by side.  A graph without branches goes to its queue as one batch of packets, 50 us of the host for 122 launches; one
+    // graph of both lanes of a decode step was launched node by node, 520 us of the host, and the device waited for it (32 sequences
+    // as two lanes, 245 launches: 1032 us a step as one graph, 962 as three).
+    std::lock_guard<std::mutex> guard(ctx->lane_lock);
+    hipError_t first = hipEventRecord(ctx->lane_events[0], ctx->stream);
+    auto note = [&](hipError_t e) {
+        if (first == hipSuccess) first = e;
+        return e == hipSuccess;
+    };
+    if (first == hipSuccess && fn->lane_exec[0]) note(hipGraphLaunch(fn->lane_exec[0], ctx->stream));
+    for (int l = 1; l < fn->nlanes && first == hipSuccess; l++)
+        if (fn->lane_exec[l] && note(hipStreamWaitEvent(ctx->lane_streams[l], ctx->lane_events[0], 0)) &&
+            note(hipGraphLaunch(fn->lane_exec[l], ctx->lane_streams[l])))
+            note(hipEventRecord(ctx->lane_events[l], ctx->lane_streams[l]));
+    for (int l = 1; l < fn->nlanes; l++) // (also after a failure: nothing of this call is left behind the context's stream)
+        if (fn->lane_exec[l]) note(hipStreamWaitEvent(ctx->stream, ctx->lane_events[l], 0));
+    if (first == hipSuccess && fn->joined_exec) note(hipGraphLaunch(fn->joined_exec, ctx->stream));
+    return first == hipSuccess ? 0 : hip_fail(ctx, first, "function_invoke: lanes");
+}
+
+// The operators of one lane as a graph without branches, captured on `stream`; *exec null where there are none.
+static int capture_lane(nncase_hip_function *fn, int lane, hipStream_t stream, hipGraphExec_t *exec) {
+    nncase_hip_ctx *ctx = fn->ctx;
+    *exec = nullptr;
+    if (std::none_of(fn->ops.begin(), fn->ops.end(), [&](const Op &op) { return op.lane == lane; })) return 0;
+    NNHIP_HIP(ctx, hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal));
+    const hipStream_t main_stream = ctx->stream;
+    ctx->stream = stream;
+    int rc = 0;
+    for (size_t k = 0; k < fn->ops.size() && !rc;) {
+        if (fn->ops[k].lane == lane) rc = run_ops(fn, k, &k);
+        else k++;
+    }
+    ctx->stream = main_stream;
+    hipGraph_t graph = nullptr;
+    const hipError_t e = hipStreamEndCapture(stream, &graph);
+    hipError_t ie = hipSuccess;
+    if (!rc && e == hipSuccess) ie = hipGraphInstantiate(exec, graph, nullptr, nullptr, 0);
+    if (graph) (void)hipGraphDestroy(graph);
+    if (rc) return rc;
+    NNHIP_HIP(ctx, e);
+    if (ie != hipSuccess) return hip_fail(ctx, ie, "hipGraphInstantiate");
     return 0;
 }
 
@@ -694,75 +762,14 @@ extern "C" int nncase_hip_function_capture(nncase_hip_function_t *fn) {
     int attn_lane = -1;
     for (const Op &op : fn->ops)
         if (op.kind == Op::kAttn && op.lane <= 0) attn_lane = 0;
-    // Operators of different lanes are recorded on streams of their own, forked from and joined back into
-    // the context's stream, so the graph holds one independent chain per lane and the device overlaps them.
-    hipStream_t main_stream = ctx->stream;
-    hipStream_t side[NNCASE_HIP_MAX_LANES] = {nullptr};
-    hipEvent_t fork = nullptr, join[NNCASE_HIP_MAX_LANES] = {nullptr};
-    int rc = 0;
-    hipError_t se = hipSuccess;
-    for (int l = 1; l < fn->nlanes && se == hipSuccess; l++) {
-        se = hipStreamCreateWithFlags(&side[l], hipStreamNonBlocking);
-        if (se == hipSuccess) se = hipEventCreateWithFlags(&join[l], hipEventDisableTiming);
-    }
-    if (se == hipSuccess && fn->nlanes > 1) se = hipEventCreateWithFlags(&fork, hipEventDisableTiming);
-    auto release = [&]() {
-        for (int l = 1; l < NNCASE_HIP_MAX_LANES; l++) {
-            if (join[l]) (void)hipEventDestroy(join[l]);
-            if (side[l]) (void)hipStreamDestroy(side[l]);
-        }
-        if (fork) (void)hipEventDestroy(fork);
-    };
-    if (se != hipSuccess) {
-        release();
-        return hip_fail(ctx, se, "function_capture: lane streams");
-    }
-    se = hipStreamBeginCapture(main_stream, hipStreamCaptureModeThreadLocal);
-    if (se != hipSuccess) {
-        release();
-        return hip_fail(ctx, se, "hipStreamBeginCapture");
-    }
-    if (fn->nlanes > 1) {
-        se = hipEventRecord(fork, main_stream);
-        for (int l = 1; l < fn->nlanes && se == hipSuccess; l++) se = hipStreamWaitEvent(side[l], fork, 0);
-    }
-    if (se == hipSuccess) {
-        for (size_t k = 0; k < fn->ops.size();) {
-            const int lane = fn->ops[k].lane;
-            if (lane == NNCASE_HIP_LANE_JOINED) {
-                k++;
-                continue;
-            }
-            ctx->stream = lane == 0 ? main_stream : side[lane];
-            rc = run_ops(fn, k, &k);
-            if (rc) break;
-        }
-        ctx->stream = main_stream;
-        for (int l = 1; l < fn->nlanes && se == hipSuccess; l++) {
-            se = hipEventRecord(join[l], side[l]);
-            if (se == hipSuccess) se = hipStreamWaitEvent(main_stream, join[l], 0);
-        }
-        // what was recorded behind the join: on the context's stream, after every lane
-        for (size_t k = 0; k < fn->ops.size() && !rc && se == hipSuccess;) {
-            if (fn->ops[k].lane == NNCASE_HIP_LANE_JOINED) rc = run_ops(fn, k, &k);
-            else k++;
-        }
-    }
-    hipGraph_t graph = nullptr;
-    const hipError_t e = hipStreamEndCapture(main_stream, &graph);
-    release();
-    if (se != hipSuccess && !rc) rc = hip_fail(ctx, se, "function_capture: fork / join");
+    int rc = fn->nlanes > 1 ? lane_streams_reserve(ctx, fn->nlanes) : 0;
+    for (int l = 0; l < fn->nlanes && !rc; l++) rc = capture_lane(fn, l, l == 0 ? ctx->stream : ctx->lane_streams[l], &fn->lane_exec[l]);
+    if (!rc) rc = capture_lane(fn, NNCASE_HIP_LANE_JOINED, ctx->stream, &fn->joined_exec);
     if (rc) {
-        if (graph) (void)hipGraphDestroy(graph);
+        drop_graph(fn);
         return rc;
     }
-    NNHIP_HIP(ctx, e);
-    fn->graph = graph;
-    const hipError_t ie = hipGraphInstantiate(&fn->exec, fn->graph, nullptr, nullptr, 0);
-    if (ie != hipSuccess) {
-        drop_graph(fn);
-        return hip_fail(ctx, ie, "hipGraphInstantiate");
-    }
+    fn->captured = true;
     if (attn_lane >= 0) {
         fn->pins_attn = true;
         ctx->attn_pins++;

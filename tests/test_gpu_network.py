@@ -393,3 +393,30 @@ def test_mobilenetv2_fused_blocks_match_separate_operators(hip_ctx):
     want = netref.run_integer(qg, x[:1])
     want = want[0] if isinstance(want, tuple) else want
     assert np.array_equal(y0[:1].view(np.uint32), np.asarray(want).view(np.uint32))
+
+
+@pytest.mark.parametrize("lanes", [(0, 1), (0, 2), (1, 2, 7), (3,)])
+def test_lanes_are_forked_and_joined_on_every_replay(hip_ctx, lanes):
+    """Each lane adds to a part of its own, what is joined to all of them, between eager operators on the same tensor: lanes that
+    have no operators, a function without lane 0, replay after replay."""
+    n = 1 << 16
+    x = hip_ctx.to_device(np.zeros(8 * n, np.int32))
+    fn = rt.Function(hip_ctx)
+    for lane in lanes:
+        fn.set_lane(lane)
+        for _ in range(20):
+            fn.add_add_i32(x.view(lane * n * 4, n * 4), n, lane + 1)
+    fn.set_lane(rt.Function.LANE_JOINED)
+    fn.add_add_i32(x, 8 * n, 1)
+    want = np.zeros((8, n), np.int32)
+    for replay in range(6):
+        if replay == 1:
+            fn.capture()
+        hip_ctx.add_i32(x, 8 * n, 3)
+        fn.invoke()
+        hip_ctx.add_i32(x, 8 * n, -1)
+        want += 3
+        for lane in lanes:
+            want[lane] += 20 * (lane + 1)
+        if replay % 2:                                    # (two replays in flight)
+            assert np.array_equal(x.download((8, n), np.int32), want)
