@@ -59,13 +59,12 @@ int igemm_plan(nncase_hip_ctx *ctx, nncase_hip_weights *w, const int32_t *bias) 
     // channels the 128 x 64 blocks below are quicker at any size: 200 704 pixels 64 -> 64 3x3 20.6 us against 25.6.)
     {
         const long long ptiles = ceil_div((int)std::min<int64_t>(std::max<int64_t>(w->pixels_hint, 0), 1 << 30), 256);
-        // 256-channel chunks (two waves side by side share the block's activations) where that still fills the device.  Rows
-        // that the 256 x 256 kernel moves itself, from dword addresses (1x1 windows): where more than half of the compute units
-        // get a block (5120 rows of 3008 to 2048 columns, 160 blocks, 47.9 us in blocks half as wide, 40.8 so; 4096 rows, 128
-        // blocks, 35.1 / 38.9)
-        const long long blocks256 = ptiles * ceil_div(w->g_oc, 256);
+        // 256-channel chunks (two waves side by side share the block's activations) where that still fills the device; rows
+        // that the DMA kernel moves itself, from dword addresses (1x1 windows): by dma_pays
         const bool dma = taps == 1 && (!w->ragged || w->g_ic % 4 == 0);
-        const int wide_tiles = w->g_oc > 128 && (dma ? 2 * blocks256 > ctx->compute_units : !w->ragged && blocks256 >= ctx->compute_units) ? 16 : 8;
+        const bool fills = dma ? dma_pays(std::max<int64_t>(w->pixels_hint, 0), w->g_oc, w->ksteps, ctx->compute_units)
+                               : !w->ragged && w->g_oc > 128 && ptiles * ceil_div(w->g_oc, 256) >= ctx->compute_units;
+        const int wide_tiles = fills ? 16 : 8;
         w->wide = w->tap_ic % 16 == 0 && w->ksteps >= kWideMinKsteps && w->g_oc > 64 &&
                   (wide_tiles == 16 || ptiles * ceil_div(w->g_oc, 128) >= ctx->compute_units);
         if (w->wide) {

@@ -52,6 +52,38 @@ inline bool small_wide_pays(int g_oc, int ksteps, int tiles) {
     return ksteps >= 5 || (ksteps >= 2 && tiles >= 5 && g_oc % (4 * tiles) != 0);
 }
 
+// Rows per block, in sixteens of a wave (a block is four waves of them high: 2, 3 or 4 stand for 128, 192 and 256 rows), of the
+// products that the kernel of 256-channel chunks fed by DMA alone computes.  A block has its compute unit to itself, so a launch is
+// rounds of the device, each a fill and an epilogue (8.5 us; 12.5 with the stores of 256 x 256 outputs) and the k-steps (0.52, 0.80
+// and 0.97 us of 64 at 128, 192 and 256 rows: more rows share a k-step's weights).  us at 128 / 192 / 256 rows: 5000 rows of 3000 to
+// 2100 columns 59.6 / 46.2 / 53.7 (360, 243 and 180 blocks), 4096 of 3008 to 2048 32.4 / 38.6 / 45.2, 32 768 of 1024 to 1024
+// 67.0 / 65.7 / 56.0, 10 000 of 640 to 2000 37.8 / 36.3 / 42.7, 16 000 of 2048 to 512 25.0 / 29.5 / 35.5.
+struct DmaRows {
+    int rg;
+    double us;
+};
+inline DmaRows choose_dma_rows(int64_t rows, int nchunks, int ksteps, int compute_units) {
+    constexpr double outside[3] = {8.5, 8.5, 12.5}, per_kstep[3] = {0.52, 0.80, 0.97};
+    DmaRows best{0, 0};
+    for (int rg = 4; rg >= 2; rg--) {
+        const int64_t blocks = (rows + rg * 64 - 1) / (rg * 64) * nchunks, rounds = (blocks + compute_units - 1) / compute_units;
+        const double us = rounds * (outside[rg - 2] + ksteps * per_kstep[rg - 2]);
+        if (!best.rg || us < best.us) best = {rg, us};
+    }
+    return best;
+}
+
+// Whether a product takes that kernel and not blocks of 128 channels and fewer: with a 256 x 256 block for more than half of the
+// compute units, or where its rounds are quicker than what the others reach (1.05 POP/s behind 4 us).  us, the others / it: 4096 rows
+// of 3008 to 2048 40.9 / 32.4, 1300 of 4096 to 4096 44.3 / 31.6, 3680 of 2156 to 1554 35.0 / 24.9; but 5996 of 2816 to 624
+// 21.3 / 25.4, 8520 of 1032 to 377 12.8 / 16.1, 1532 of 704 to 3941 12.2 / 13.2.
+inline bool dma_pays(int64_t rows, int n, int ksteps, int compute_units) {
+    if (n <= 128) return false;
+    const int nchunks = (n + 255) / 256;
+    if (2 * ((rows + 255) / 256) * nchunks > compute_units) return true;
+    return choose_dma_rows(rows, nchunks, ksteps, compute_units).us < 4 + 2.0 * (double)rows * n * ksteps * 64 / 1.05e9;
+}
+
 // The tile of at most `pix` output pixels (32 at most side by side) that covers an out_h x out_w image in the fewest blocks, rows
 // and columns spread evenly over them; among equals the one with the smallest input, among those the widest (below four columns
 // the first that does no better ends the search).  span: what a window reads, its dilation included.  (Asked for on every launch,

@@ -28,6 +28,7 @@
 #pragma once
 
 #include "qconv_igemm.hpp"
+#include "qconv_rules.hpp"
 
 #include <mutex>
 #include <type_traits>
@@ -64,10 +65,11 @@ struct __attribute__((packed, aligned(1))) wide_unaligned16 {
 };
 
 // 16 bytes of the tensor x (bytes `bytes`, 16-byte aligned) from any byte offset; what lies outside it is undefined.
-// near_end (wave-uniform) says that a lane's piece may reach past the last byte: it is then put together from aligned
-// dwords, range-checked one by one (the last dword that holds a byte of the tensor never crosses into another page).
+// near_end (wave-uniform) says that some piece of the wave may reach past the last byte; those that do are put together from
+// aligned dwords, range-checked one by one (the last dword that holds a byte of the tensor never crosses into another page).
+// (Asked again for the pieces at hand: a wave near the end that fetched all of them so took twice as long as the others.)
 __device__ __forceinline__ wide_u32x4 load_ragged(const uint8_t *x, const __amdgpu_buffer_rsrc_t &dwords, int bytes, int off, bool near_end) {
-    if (!near_end) return reinterpret_cast<const wide_unaligned16 *>(x + (uint32_t)min(max(off, 0), bytes - 16))->v;
+    if (!near_end || (bytes >= 16 && !__any(off > bytes - 16))) return reinterpret_cast<const wide_unaligned16 *>(x + (uint32_t)min(max(off, 0), bytes - 16))->v;
     uint32_t d[5];
 #pragma unroll
     for (int i = 0; i < 5; i++) d[i] = __builtin_amdgcn_raw_buffer_load_b32(dwords, (off & ~3) + i * 4, 0, 0);
@@ -75,6 +77,26 @@ __device__ __forceinline__ wide_u32x4 load_ragged(const uint8_t *x, const __amdg
 #pragma unroll
     for (int i = 0; i < 4; i++) r[i] = __builtin_amdgcn_alignbyte(d[i + 1], d[i], off & 3);
     return r;
+}
+
+// Which pixel tile and channel chunk a block computes.  Blocks go to the 8 XCDs round-robin, and every XCD takes a contiguous run of
+// the pairs of tile and chunk: the chunks of a tile, which share its activations, and the tiles that share input rows of a window
+// (vertical neighbours) run on one XCD at about the same time.  Whole tiles per XCD where that is no more rounds of its compute units
+// and next to no more blocks than an eighth of all pairs (27 tiles of 9 chunks would be four tiles on some XCDs, 36 blocks on 32
+// compute units: 21 649 rows of 640 to 653 columns, 85 tiles of 3 chunks, 41.6 us so and 26.3 dealt out evenly).
+struct WideGrid {
+    int total, per; // pairs; pairs of an XCD
+    FastDiv chunks;
+};
+inline WideGrid wide_grid(const nncase_hip_ctx *ctx, int mtiles, int nchunks) {
+    const int whole = ceil_div(mtiles, 8) * nchunks, even = ceil_div(mtiles * nchunks, 8), cus = std::max(1, ctx->compute_units / 8);
+    const bool tiles = ceil_div(whole, cus) == ceil_div(even, cus) && 16ll * whole <= 17ll * even;
+    return WideGrid{mtiles * nchunks, tiles ? whole : even, make_fastdiv((uint32_t)nchunks)};
+}
+__device__ __forceinline__ bool wide_block(const WideGrid &g, int *mt, int *chunk) {
+    const int seq = blockIdx.x >> 3, i = (blockIdx.x & 7) * g.per + seq;
+    *mt = (int)fastdiv((uint32_t)i, g.chunks), *chunk = i - *mt * (int)g.chunks.div;
+    return i < g.total;
 }
 
 // T: 16-channel tiles per wave; RG: 16-pixel groups per wave; a block is WM x WN waves: WM * RG * 16 pixels by
@@ -92,7 +114,7 @@ __device__ __forceinline__ wide_u32x4 load_ragged(const uint8_t *x, const __amdg
 // k-step is about a hundred of them (880 cycles for 128 cycles of matrix work), so a launch with one block per compute
 // unit is bound by that; KG waves per SIMD take turns issuing.
 template <int T, int RG, int WM, int WN, int LM, int KG = 1>
-__global__ __launch_bounds__(WM * WN * KG * 64, WM * WN * KG > 8 ? 4 : 2) void qconv_wide_kernel(const IgemmArgs a, int nchunks) {
+__global__ __launch_bounds__(WM * WN * KG * 64, WM * WN * KG > 8 ? 4 : 2) void qconv_wide_kernel(const IgemmArgs a, const WideGrid grid) {
     static_assert(KG == 1 || RG <= KG, "every pixel group of a wave has a group of its own to finish it");
     constexpr int THREADS = WM * WN * 64;               // of a group: the threads that move a k-step's operands
     constexpr int BLOCK = THREADS * KG;
@@ -112,14 +134,8 @@ __global__ __launch_bounds__(WM * WN * KG * 64, WM * WN * KG > 8 ? 4 : 2) void q
     int32_t *rowsums = reinterpret_cast<int32_t *>(lutl + 256);      // [PIX]
     uint8_t *const rings = lutl + 256 + PIX * sizeof(int32_t);       // [KG][kWideSlots][SLOT]
 
-    // channel chunks of a pixel tile are consecutive on one XCD (blocks go to the 8 XCDs round-robin)
-    // ... and every XCD takes a contiguous eighth of the pixel tiles, in the order of the tensor: the tiles that share
-    // input rows of a window (vertical neighbours) then run on one XCD at about the same time
-    const int xcd = blockIdx.x & 7, seq = blockIdx.x >> 3;
-    const int chunk = seq % nchunks;
-    const int per = (a.num_mtiles + 7) >> 3;
-    const int mt = xcd * per + seq / nchunks;
-    if (seq / nchunks >= per || mt >= a.num_mtiles) return;
+    int mt, chunk;
+    if (!wide_block(grid, &mt, &chunk)) return;
 
     const int lane = threadIdx.x & 63;
     const int bwave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -417,7 +433,7 @@ __global__ __launch_bounds__(WM * WN * KG * 64, WM * WN * KG > 8 ? 4 : 2) void q
 //     DMA is requested at the top of k-step s - 3 and waited for at the end of k-step s - 2;
 // The rest (operand reads ahead of the products, rotation of a pixel's pieces, sums of x', epilogue) is the kernel above.
 template <int T, int RG, int WM, int WN, int LM>
-__global__ __launch_bounds__(WM * WN * 64, 2) void qconv_wide4_kernel(const IgemmArgs a, int nchunks) {
+__global__ __launch_bounds__(WM * WN * 64, 2) void qconv_wide4_kernel(const IgemmArgs a, const WideGrid grid) {
     constexpr int NS = 4;
     constexpr int THREADS = WM * WN * 64;
     constexpr int PIX = WM * RG * 16;
@@ -438,11 +454,8 @@ __global__ __launch_bounds__(WM * WN * 64, 2) void qconv_wide4_kernel(const Igem
     int32_t *rowsums = reinterpret_cast<int32_t *>(lutl + 256);      // [PIX]
     uint8_t *ring = lutl + 256 + PIX * sizeof(int32_t);              // [NS][SLOT]
 
-    const int xcd = blockIdx.x & 7, seq = blockIdx.x >> 3;
-    const int chunk = seq % nchunks;
-    const int per = (a.num_mtiles + 7) >> 3;
-    const int mt = xcd * per + seq / nchunks;
-    if (seq / nchunks >= per || mt >= a.num_mtiles) return;
+    int mt, chunk;
+    if (!wide_block(grid, &mt, &chunk)) return;
 
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -705,7 +718,7 @@ template <int T, int RG, int WM, int WN, int LM> int launch_wide4_t(nncase_hip_c
     IgemmArgs args = a;
     constexpr int PIX = WM * RG * 16, TB = T * WN;
     args.num_mtiles = ceil_div(a.m, PIX);
-    const int blocks = ceil_div(args.num_mtiles, 8) * 8 * nchunks;
+    const WideGrid grid = wide_grid(ctx, args.num_mtiles, nchunks);
     const size_t lds = (size_t)TB * 16 * sizeof(int32_t) + 256 + PIX * sizeof(int32_t) + (size_t)4 * (PIX * 64 + TB * 1024);
     static std::once_flag raised[16]; // more than 64 KiB of dynamic LDS has to be asked for once per kernel and device
     hipError_t attr = hipSuccess;
@@ -713,7 +726,7 @@ template <int T, int RG, int WM, int WN, int LM> int launch_wide4_t(nncase_hip_c
         attr = hipFuncSetAttribute(reinterpret_cast<const void *>(&qconv_wide4_kernel<T, RG, WM, WN, LM>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     });
     NNHIP_HIP(ctx, attr);
-    hipLaunchKernelGGL((qconv_wide4_kernel<T, RG, WM, WN, LM>), dim3(blocks), dim3(WM * WN * 64), lds, ctx->stream, args, nchunks);
+    hipLaunchKernelGGL((qconv_wide4_kernel<T, RG, WM, WN, LM>), dim3(grid.per * 8), dim3(WM * WN * 64), lds, ctx->stream, args, grid);
     NNHIP_LAUNCH_CHECK(ctx, "qconv_wide4_kernel");
     return 0;
 }
@@ -781,7 +794,7 @@ __device__ __forceinline__ void wide_store_lines(const IgemmArgs &a, const v4i (
 }
 
 template <int T, int RG, int WM, int WN, int LM>
-__global__ __launch_bounds__(WM * WN * 64, WM * WN >= 8 ? 2 : 1) void qconv_wide_dma_kernel(const IgemmArgs a, int nchunks) {
+__global__ __launch_bounds__(WM * WN * 64, WM * WN >= 8 ? 2 : 1) void qconv_wide_dma_kernel(const IgemmArgs a, const WideGrid grid) {
     static_assert(LM == kWideRowsFull || LM == kWideRows, "contiguous reduction rows only");
     constexpr int NSW = 4, NSA = 3;
     constexpr int THREADS = WM * WN * 64, WAVES = WM * WN;
@@ -791,7 +804,10 @@ __global__ __launch_bounds__(WM * WN * 64, WM * WN >= 8 ? 2 : 1) void qconv_wide
     constexpr int ASTAGE = PIX * 128;                   // bytes of an activation stage (two k-steps)
     constexpr int NW = TB / WAVES;                      // weight runs (1 KiB) per wave per k-step
     constexpr int NA = PIX / 8 / WAVES;                 // activation runs per wave per pair of k-steps
-    static_assert(TB % WAVES == 0 && (PIX / 8) % WAVES == 0 && NA % 4 == 0, "every wave moves the same number of runs");
+    static_assert(TB % WAVES == 0 && (PIX / 8) % WAVES == 0, "every wave moves the same number of runs");
+    // a pair's runs are requested in quarters: those before quarter q, those of quarter q
+    constexpr auto before = [](int q) { return q * NA / 4; };
+    constexpr auto quarter = [before](int q) { return before(q + 1) - before(q); };
     static_assert(T % 4 == 0, "at least two pairs of channel tiles per k-step");
     static_assert((WSLOT & (WSLOT - 1)) == 0, "the weight ring wraps by a mask");
     constexpr int G = T / 2;
@@ -803,11 +819,8 @@ __global__ __launch_bounds__(WM * WN * 64, WM * WN >= 8 ? 2 : 1) void qconv_wide
     uint8_t *lutl = smem + TB * 16 * sizeof(int32_t);                // [256]
     uint8_t *stage_base = lutl + 256;
 
-    const int xcd = blockIdx.x & 7, seq = blockIdx.x >> 3;
-    const int chunk = seq % nchunks;
-    const int per = (a.num_mtiles + 7) >> 3;
-    const int mt = xcd * per + seq / nchunks;
-    if (seq / nchunks >= per || mt >= a.num_mtiles) return;
+    int mt, chunk;
+    if (!wide_block(grid, &mt, &chunk)) return;
 
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -865,8 +878,7 @@ __global__ __launch_bounds__(WM * WN * 64, WM * WN >= 8 ? 2 : 1) void qconv_wide
     constexpr std::integral_constant<int, NW> cNW;
     constexpr std::integral_constant<int, NA> cNA;
     constexpr std::integral_constant<int, NW / 2> cNWh;
-    constexpr std::integral_constant<int, NA / 2> cNAh;
-    static_assert(NW % 2 == 0 && NA % 2 == 0, "requests are issued in halves");
+    static_assert(NW % 2 == 0, "requests are issued in halves");
     dma_w(0, 0, c0, cNW);
     dma_w(WSLOT, 1, c0, cNW);
     __builtin_amdgcn_sched_barrier(0);
@@ -950,13 +962,13 @@ __global__ __launch_bounds__(WM * WN * 64, WM * WN >= 8 ? 2 : 1) void qconv_wide
             if (g == 0) dma_w(wnxt3, s + 3, c0, cNWh);
             if (g == 2) dma_w(wnxt3, s + 3, cNWh, cNWh);
             if (P == 1) {
-                if (g == 1) dma_a(acur, (s + 5) >> 1, c0, std::integral_constant<int, NA / 4>());
-                if (g == 3) dma_a(acur, (s + 5) >> 1, std::integral_constant<int, NA / 4>(), std::integral_constant<int, NA / 4>());
+                if (g == 1) dma_a(acur, (s + 5) >> 1, c0, std::integral_constant<int, quarter(0)>());
+                if (g == 3) dma_a(acur, (s + 5) >> 1, std::integral_constant<int, before(1)>(), std::integral_constant<int, quarter(1)>());
             } else {
                 // (an even k-step: the stage before this one's, pair (s + 4) / 2)
                 const int aprev = acur == 0 ? (NSA - 1) * ASTAGE : acur - ASTAGE;
-                if (g == 1) dma_a(aprev, (s + 4) >> 1, cNAh, std::integral_constant<int, NA / 4>());
-                if (g == 3) dma_a(aprev, (s + 4) >> 1, std::integral_constant<int, 3 * NA / 4>(), std::integral_constant<int, NA / 4>());
+                if (g == 1) dma_a(aprev, (s + 4) >> 1, std::integral_constant<int, before(2)>(), std::integral_constant<int, quarter(2)>());
+                if (g == 3) dma_a(aprev, (s + 4) >> 1, std::integral_constant<int, before(3)>(), std::integral_constant<int, quarter(3)>());
             }
             static_for<0, NM>([&](auto m_c) __attribute__((always_inline)) {
                 constexpr int m = decltype(m_c)::value, e = m / RG, rg = m % RG;
@@ -983,9 +995,9 @@ __global__ __launch_bounds__(WM * WN * 64, WM * WN >= 8 ? 2 : 1) void qconv_wide
         __builtin_amdgcn_sched_barrier(0);
         // the weights of k-step s + 2 (requested during k-step s - 1) and the activations requested two and three
         // k-steps ago have landed: behind them came the last quarter of that k-step's activation runs, this k-step's
-        // NW weight runs and its NA / 2 activation runs; of this wave's operand reads only the four of the next weights
-        // may still be out
-        __builtin_amdgcn_s_waitcnt(waitcnt_imm(NA / 4 + NW + NA / 2, 4));
+        // NW weight runs and its two quarters of activation runs; of this wave's operand reads only the four of the next
+        // weights may still be out
+        __builtin_amdgcn_s_waitcnt(waitcnt_imm(P == 0 ? quarter(1) + NW + quarter(2) + quarter(3) : quarter(3) + NW + quarter(0) + quarter(1), 4));
         __builtin_amdgcn_s_barrier();
         __builtin_amdgcn_sched_barrier(0);
     };
@@ -1034,7 +1046,7 @@ template <int T, int RG, int WM, int WN, int LM> int launch_wide_dma_t(nncase_hi
     IgemmArgs args = a;
     constexpr int PIX = WM * RG * 16, TB = T * WN;
     args.num_mtiles = ceil_div(a.m, PIX);
-    const int blocks = ceil_div(args.num_mtiles, 8) * 8 * nchunks;
+    const WideGrid grid = wide_grid(ctx, args.num_mtiles, nchunks);
     const size_t lds = (size_t)4 * TB * 1024 + (size_t)3 * PIX * 128;
     static std::once_flag raised[16]; // more than 64 KiB of dynamic LDS has to be asked for once per kernel and device
     hipError_t attr = hipSuccess;
@@ -1042,7 +1054,7 @@ template <int T, int RG, int WM, int WN, int LM> int launch_wide_dma_t(nncase_hi
         attr = hipFuncSetAttribute(reinterpret_cast<const void *>(&qconv_wide_dma_kernel<T, RG, WM, WN, LM>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     });
     NNHIP_HIP(ctx, attr);
-    hipLaunchKernelGGL((qconv_wide_dma_kernel<T, RG, WM, WN, LM>), dim3(blocks), dim3(WM * WN * 64), lds, ctx->stream, args, nchunks);
+    hipLaunchKernelGGL((qconv_wide_dma_kernel<T, RG, WM, WN, LM>), dim3(grid.per * 8), dim3(WM * WN * 64), lds, ctx->stream, args, grid);
     NNHIP_LAUNCH_CHECK(ctx, "qconv_wide_dma_kernel");
     return 0;
 }
@@ -1051,7 +1063,7 @@ template <int T, int RG, int WM, int WN, int LM, int KG = 1> int launch_wide_t(n
     IgemmArgs args = a;
     constexpr int PIX = WM * RG * 16, TB = T * WN;
     args.num_mtiles = ceil_div(a.m, PIX);
-    const int blocks = ceil_div(args.num_mtiles, 8) * 8 * nchunks;
+    const WideGrid grid = wide_grid(ctx, args.num_mtiles, nchunks);
     const size_t lds = (size_t)TB * 16 * sizeof(int32_t) + 256 + PIX * sizeof(int32_t) + (size_t)KG * kWideSlots * (PIX * 64 + TB * 1024);
     if (lds > 65536) { // more than 64 KiB of dynamic LDS has to be asked for once per kernel and device
         static std::once_flag raised[16];
@@ -1061,7 +1073,7 @@ template <int T, int RG, int WM, int WN, int LM, int KG = 1> int launch_wide_t(n
         });
         NNHIP_HIP(ctx, attr);
     }
-    hipLaunchKernelGGL((qconv_wide_kernel<T, RG, WM, WN, LM, KG>), dim3(blocks), dim3(WM * WN * KG * 64), lds, ctx->stream, args, nchunks);
+    hipLaunchKernelGGL((qconv_wide_kernel<T, RG, WM, WN, LM, KG>), dim3(grid.per * 8), dim3(WM * WN * KG * 64), lds, ctx->stream, args, grid);
     NNHIP_LAUNCH_CHECK(ctx, "qconv_wide_kernel");
     return 0;
 }
@@ -1090,18 +1102,26 @@ template <int T, int WM, int WN, int LM> int launch_wide_small_t(nncase_hip_ctx 
     }
 }
 
-// Block shapes: tiles = 16 -> 256 pixels x 256 channels (4 x 2 waves); tiles = 8 -> 256 or 128 pixels x 128 channels.
+template <int LM> int launch_wide_dma(nncase_hip_ctx *ctx, const IgemmArgs &a, int nchunks) {
+    switch (choose_dma_rows(a.m, nchunks, a.ksteps, ctx->compute_units).rg) {
+    case 2: return launch_wide_dma_t<8, 2, 4, 2, LM>(ctx, a, nchunks);
+    case 3: return launch_wide_dma_t<8, 3, 4, 2, LM>(ctx, a, nchunks);
+    default: return launch_wide_dma_t<8, 4, 4, 2, LM>(ctx, a, nchunks);
+    }
+}
+
+// Block shapes: tiles = 16 -> 256 pixels x 256 channels (4 x 2 waves; rows that arrive by DMA also 192 and 128); tiles = 8 -> 256 or 128 pixels x 128 channels.
 template <int LM> int launch_wide_lm(nncase_hip_ctx *ctx, const IgemmArgs &a, int tiles, int nchunks) {
     if constexpr (LM == kWideRagRows) {
         // (planned for rows of whole dwords: a piece then starts at a dword, wherever its 16 bytes lie; what runs over the end of a
         // row meets surplus weights and is in the sums of x as well)
         if (tiles == 16)
-            return a.k % 64 == 0 ? launch_wide_dma_t<8, 4, 4, 2, kWideRowsFull>(ctx, a, nchunks) : launch_wide_dma_t<8, 4, 4, 2, kWideRows>(ctx, a, nchunks);
+            return a.k % 64 == 0 ? launch_wide_dma<kWideRowsFull>(ctx, a, nchunks) : launch_wide_dma<kWideRows>(ctx, a, nchunks);
     } else if constexpr (LM == kWideRagWindow) {
         if (tiles == 16) return launch_wide_t<8, 4, 4, 2, LM>(ctx, a, nchunks);
     } else if (tiles == 16) {
         if constexpr (LM == kWideRowsFull || LM == kWideRows) {
-            if (a.x_bytes < ((size_t)1 << 31)) return launch_wide_dma_t<8, 4, 4, 2, LM>(ctx, a, nchunks);
+            if (a.x_bytes < ((size_t)1 << 31)) return launch_wide_dma<LM>(ctx, a, nchunks);
         }
         return launch_wide4_t<8, 4, 4, 2, LM>(ctx, a, nchunks);
     }

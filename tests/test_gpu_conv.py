@@ -882,3 +882,18 @@ def test_matmul_of_rows_of_whole_dwords_in_256_channel_blocks(hip_ctx, m, k, n):
 def test_pointwise_layers_with_a_table_on_the_lean_kernel(hip_ctx, cin, cout, hw):
     """Whole chunks of channels behind a byte table: folded and unfolded reductions, partial pixel tiles, one to eight channel tiles."""
     test_fused_table_equals_conv_then_table(hip_ctx, cin, cout, hw, 1, False)
+
+
+@pytest.mark.parametrize("m,k,n", [
+    (8100, 1036, 1000), (8192, 1088, 1023), (3000, 4100, 1025),      # 128 rows: an odd and an even number of k-steps, ragged ends
+    (5000, 1000, 2100), (5184, 1088, 2047), (5185, 1060, 2048),      # 192
+    (13000, 520, 1290), (32768, 512, 257),                           # 256
+])
+def test_matmul_in_blocks_of_128_192_and_256_rows(hip_ctx, m, k, n):
+    """Every height of the DMA kernel's blocks at ends inside a block, inside a k-step and inside a channel chunk, tiles and chunks
+    that divide over no number of dies, with zero points at the extremes."""
+    rng = np.random.default_rng(m + n)
+    x, w = rng.integers(0, 256, (m, k), dtype=np.uint8), rng.integers(0, 256, (k, n), dtype=np.uint8)
+    x[-1] = 255                                                # (the row that the last block repeats)
+    want = ((x.astype(np.float64) - 3) @ (w.astype(np.float64) - 250)).astype(np.int32)     # exact: below 2^53
+    assert np.array_equal(K.mat_mul(x, w, qp(3, 0.02), qp(250, 0.011), None, np.int32, None, ctx=hip_ctx), want)
