@@ -13,10 +13,10 @@
 //   Logits: S^T[token, head] = K[token, :] . Q^T[:, head] with K rows as the
 //   MFMA A operand (one 16-byte load per lane straight from the cache) and the
 //   query heads, padded to 16, as B.  The accumulator layout of S^T (lane =
-//   head, 4 consecutive tokens per lane) IS the A-operand layout of the 16x16x16
+//   head, 4 consecutive tokens per lane) IS the A-operand layout of the
 //   product P.V, so probabilities never move between lanes.  V is cached
-//   d-major ([block][kv head][d][token]) so that a lane's B operand (4
-//   consecutive tokens of one d) is one 8-byte load.  P is split into two fp16
+//   d-major ([block][kv head][d][token]) so that a lane's B operand
+//   (consecutive tokens of one d) is one load.  P is split into two fp16
 //   terms (p = hi + lo), which keeps the P.V product at fp32-level accuracy.
 //
 //   Every wave keeps its own (max, sum, unnormalised output); the block merges
@@ -30,6 +30,7 @@
 #include <hip/hip_fp16.h>
 
 #include <algorithm>
+#include <type_traits>
 
 namespace nnhip {
 
@@ -41,8 +42,17 @@ typedef uint32_t au32x2 __attribute__((ext_vector_type(2)));
 
 constexpr int kAttnHeads = 16; // query heads per kv head, padded to the MFMA tile
 constexpr float kLog2e = 1.4426950408889634f;
+// Probabilities enter P.V times 2^14, up to 16 384: their second fp16 term ends at 2^-24, an eighth of a millionth of a probability of
+// a half, and the small ones of a long run lost bits there.
+constexpr float kProbScale = 16384.f;
 
 constexpr int kAttnMaxSplits = 1024; // splits of one sequence (bounds the merge loop and the workspace)
+// Keys and values of this many bytes are not found in any cache when the next step comes back to them (the memory side's holds
+// 256 MiB): values are then read past the caches, 6.8 TB/s against 6.0 (48 sequences of up to 6000, 8 heads of 128: 135.2 -> 119.6
+// us; of 268 MB, half of it in use: 30.8 -> 33.1).  Not the keys, whose loads take 64 of a
+// line's 128 bytes at a time: they are read twice then (133.9).
+constexpr int64_t kStreamedBytes = 512000000;
+constexpr int kStreamWaves = 4;
 
 struct AttnArgs {
     const uint16_t *q, *k_cache, *v_cache;
@@ -55,6 +65,10 @@ struct AttnArgs {
     FastDiv d_block;
     float scale_log2e;
     int out_f16;
+};
+// A launch that fetches weights beside its own work.  (A type of its own, and with it kernels of their own: the longer arguments and
+// the branch cost a launch 1.8 %, 8.69 -> 8.85 us at 24 x 64 x 2820 tokens.)
+struct AttnFetchArgs : AttnArgs {
     WeightFetches fetch;
 };
 
@@ -108,14 +122,15 @@ __device__ __forceinline__ void merge_splits(const AttnArgs &a, int ns, int G, s
 #pragma unroll
             for (int k = 0; k < U; k++) mc = fmaxf(mc, pm[k]); // a repeated last split does not change the max
             const float f = __builtin_amdgcn_exp2f(m - mc);      // 0 on the first run (m = -inf)
-            n0 *= f, n1 *= f, den *= f;
+            float s0 = 0.f, s1 = 0.f, sd = 0.f; // (the run's own sums first: one rounding of the total a run)
 #pragma unroll
             for (int k = 0; k < U; k++) {
                 const float w = sp0 + k < ns ? __builtin_amdgcn_exp2f(pm[k] - mc) : 0.f;
-                n0 += w * __uint_as_float((uint32_t)vv[k]);
-                n1 += w * __uint_as_float((uint32_t)(vv[k] >> 32));
-                den += w * pl[k];
+                s0 += w * __uint_as_float((uint32_t)vv[k]);
+                s1 += w * __uint_as_float((uint32_t)(vv[k] >> 32));
+                sd += w * pl[k];
             }
+            n0 = n0 * f + s0, n1 = n1 * f + s1, den = den * f + sd;
             m = mc;
         }
         if (GR > 1) *reinterpret_cast<f32x4 *>(part + ((size_t)gr * pairs + p0) * 4) = f32x4{m, den, n0, n1};
@@ -142,7 +157,7 @@ __device__ __forceinline__ void merge_splits(const AttnArgs &a, int ns, int G, s
 // weights fetched 24.8 -> 22.9 us.  (Fetched by the products' own launches instead, or by them too, it takes 23.7 to 26.7.)
 // A wave has one batch of fragments, all of them under way at once.
 constexpr int kFetchBatch = 8;
-template <int W> __device__ __forceinline__ void fetch_weights(const AttnArgs &a) {
+template <int W> __device__ __forceinline__ void fetch_weights(const AttnFetchArgs &a) {
     const uint32_t pairs = a.hkv * a.batch, block = ((uint32_t)blockIdx.z * a.splits + blockIdx.y) * pairs + blockIdx.x;
     const uint32_t x = block % kXcds, p = (block - pairs * a.splits) / kXcds; // (every eight consecutive blocks have one on each die)
     const uint32_t lane = threadIdx.x & 63, u0 = p * W + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), stride = (uint32_t)a.fetch.blocks * W;
@@ -156,23 +171,97 @@ template <int W> __device__ __forceinline__ void fetch_weights(const AttnArgs &a
     for (int k = 0; k < kFetchBatch; k++) asm volatile("" ::"v"(v[k]));
 }
 
-// NT = 16-token tiles per wave (even); W = waves per block (a block owns W * NT * 16 tokens).
-template <int D, int NT, int W> __global__ __launch_bounds__(W * 64, W <= 8 ? 2 : 1) void paged_attn_kernel(const AttnArgs a) {
-    constexpr int kAttnWaves = W, kAttnThreads = W * 64;
-    constexpr int KS = D / 32; // 32-deep steps of the logit product
-    constexpr int DT = D / 16; // 16-wide column tiles of the output
-    constexpr int WAVE_TOKENS = NT * 16;
-    constexpr int SPLIT = kAttnWaves * WAVE_TOKENS;
+// The end of a block, given every wave's maximum, sum (of head j, the same in all g) and unnormalised output of the tokens that it
+// went through: the waves merge through LDS, and the last block of the (sequence, kv head) to get here merges the splits.
+template <int D, int W>
+__device__ __forceinline__ void finish_block(const AttnArgs &a, int b, int kvh, int split, int ns, int wave, int j, int g, float m_w, float l_w,
+                                             const f32x4 (&o)[D / 16]) {
+    constexpr int kAttnWaves = W, kAttnThreads = W * 64, DT = D / 16;
     extern __shared__ __align__(16) float attn_smem[];
     float(*red)[kAttnHeads][D] = reinterpret_cast<float(*)[kAttnHeads][D]>(attn_smem);                            // [W][heads][D]
     float(*smax)[kAttnHeads] = reinterpret_cast<float(*)[kAttnHeads]>(attn_smem + (size_t)W * kAttnHeads * D);    // [W][heads]
     float(*ssum)[kAttnHeads] = smax + W;                                                                            // [W][heads]
     __shared__ uint32_t s_last;
-
-    if (blockIdx.z != 0) { // (a branch on an argument would put its load's trip in front of the others')
-        fetch_weights<W>(a);
-        return;
+    const int G = a.group;
+    // ---- merge the waves ----------------------------------------------------------------
+    if (g == 0) {
+        smax[wave][j] = m_w;
+        ssum[wave][j] = l_w;
     }
+    __syncthreads();
+    // o[dt][r] belongs to head 4g + r, column dt*16 + j
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+        const int h = g * 4 + r;
+        float m = smax[0][h];
+#pragma unroll
+        for (int w = 1; w < kAttnWaves; w++) m = fmaxf(m, smax[w][h]);
+        const float f = __builtin_amdgcn_exp2f(smax[wave][h] - m); // 0 for a wave without tokens
+#pragma unroll
+        for (int dt = 0; dt < DT; dt++) red[wave][h][dt * 16 + j] = o[dt][r] * f;
+    }
+    __syncthreads();
+    for (int idx = threadIdx.x; idx < G * D; idx += kAttnThreads) {
+        const int h = idx / D, e = idx % D;
+        float v = 0.f;
+#pragma unroll
+        for (int w = 0; w < kAttnWaves; w++) v += red[w][h][e];
+        float m = smax[0][h];
+#pragma unroll
+        for (int w = 1; w < kAttnWaves; w++) m = fmaxf(m, smax[w][h]);
+        float l = 0.f;
+#pragma unroll
+        for (int w = 0; w < kAttnWaves; w++) l += ssum[w][h] * __builtin_amdgcn_exp2f(smax[w][h] - m);
+        if (ns == 1) { // the whole context was in this block
+            const float r = v / l;
+            const size_t oi = ((size_t)b * a.hq + kvh * G + h) * D + e;
+            if (a.out_f16) reinterpret_cast<__half *>(a.out)[oi] = __float2half_rn(r);
+            else reinterpret_cast<float *>(a.out)[oi] = r;
+        } else {
+            const size_t row = ((size_t)b * a.hq + kvh * G + h) * a.splits + split;
+            coherent_store(a.part_o + row * D + e, v);
+            if (e == 0) {
+                coherent_store(a.part_ml + row * 2 + 0, m);
+                coherent_store(a.part_ml + row * 2 + 1, l);
+            }
+        }
+    }
+    if (ns == 1) return;
+
+    // ---- the last block of the (sequence, kv head) to finish merges the splits -------------------
+    // The partials are written and read with device-scope accesses, which go through to the
+    // memory side instead of staying in the L2 of the XCD that issued them; waiting for this
+    // thread's stores and then for the block makes them globally visible before the count.
+    // (A device-scope fence would do the same by writing back and invalidating the whole L2,
+    // once per block - an order of magnitude slower here.)
+    uint32_t *done = a.done + (size_t)b * a.hkv + kvh;
+    __builtin_amdgcn_s_waitcnt(0);
+    __syncthreads();
+    if (threadIdx.x == 0)
+        s_last = __hip_atomic_fetch_add(done, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == (uint32_t)(ns - 1);
+    __syncthreads();
+    if (!s_last) return;
+    const size_t row0 = ((size_t)b * a.hq + kvh * G) * a.splits, out0 = ((size_t)b * a.hq + kvh * G) * D;
+    float *const part = attn_smem; // (the waves' outputs have been read)
+    if (ns <= 4) merge_splits<D, 4>(a, ns, G, row0, out0, part, kAttnThreads);
+    else merge_splits<D, 8>(a, ns, G, row0, out0, part, kAttnThreads);
+    if (threadIdx.x == 0) // ready for the next call on this stream
+        __hip_atomic_store(done, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// NT = 16-token tiles per wave (even); W = waves per block (a block owns W * NT * 16 tokens).
+template <int D, int NT, int W, class Args> __global__ __launch_bounds__(W * 64, W <= 8 ? 2 : 1) void paged_attn_kernel(const Args a) {
+    constexpr int kAttnWaves = W, kAttnThreads = W * 64;
+    constexpr int KS = D / 32; // 32-deep steps of the logit product
+    constexpr int DT = D / 16; // 16-wide column tiles of the output
+    constexpr int WAVE_TOKENS = NT * 16;
+    constexpr int SPLIT = kAttnWaves * WAVE_TOKENS;
+
+    if constexpr (std::is_same_v<Args, AttnFetchArgs>)
+        if (blockIdx.z != 0) { // (a branch on an argument would put its load's trip in front of the others')
+            fetch_weights<W>(a);
+            return;
+        }
     // kv head fastest, then sequence, then split: consecutive workgroups go to different XCDs, so
     // every XCD gets the same mix of early (always present) and late (long contexts only) splits
     const int kvh = blockIdx.x % a.hkv, b = blockIdx.x / a.hkv, split = blockIdx.y;
@@ -310,73 +399,193 @@ template <int D, int NT, int W> __global__ __launch_bounds__(W * 64, W <= 8 ? 2 
         l_w += __shfl_xor(l_w, 32);
     }
 
-    // ---- merge the waves ----------------------------------------------------------------
-    if (g == 0) {
-        smax[wave][j] = m_w;
-        ssum[wave][j] = l_w;
-    }
-    __syncthreads();
-    // o[dt][r] belongs to head 4g + r, column dt*16 + j
-#pragma unroll
-    for (int r = 0; r < 4; r++) {
-        const int h = g * 4 + r;
-        float m = smax[0][h];
-#pragma unroll
-        for (int w = 1; w < kAttnWaves; w++) m = fmaxf(m, smax[w][h]);
-        const float f = __builtin_amdgcn_exp2f(smax[wave][h] - m); // 0 for a wave without tokens
-#pragma unroll
-        for (int dt = 0; dt < DT; dt++) red[wave][h][dt * 16 + j] = o[dt][r] * f;
-    }
-    __syncthreads();
-    for (int idx = threadIdx.x; idx < G * D; idx += kAttnThreads) {
-        const int h = idx / D, e = idx % D;
-        float v = 0.f;
-#pragma unroll
-        for (int w = 0; w < kAttnWaves; w++) v += red[w][h][e];
-        float m = smax[0][h];
-#pragma unroll
-        for (int w = 1; w < kAttnWaves; w++) m = fmaxf(m, smax[w][h]);
-        float l = 0.f;
-#pragma unroll
-        for (int w = 0; w < kAttnWaves; w++) l += ssum[w][h] * __builtin_amdgcn_exp2f(smax[w][h] - m);
-        if (ns == 1) { // the whole context was in this block
-            const float r = v / l;
-            const size_t oi = ((size_t)b * a.hq + kvh * G + h) * D + e;
-            if (a.out_f16) reinterpret_cast<__half *>(a.out)[oi] = __float2half_rn(r);
-            else reinterpret_cast<float *>(a.out)[oi] = r;
-        } else {
-            const size_t row = ((size_t)b * a.hq + kvh * G + h) * a.splits + split;
-            coherent_store(a.part_o + row * D + e, v);
-            if (e == 0) {
-                coherent_store(a.part_ml + row * 2 + 0, m);
-                coherent_store(a.part_ml + row * 2 + 1, l);
-            }
-        }
-    }
-    if (ns == 1) return;
-
-    // ---- the last block of the (sequence, kv head) to finish merges the splits -------------------
-    // The partials are written and read with device-scope accesses, which go through to the
-    // memory side instead of staying in the L2 of the XCD that issued them; waiting for this
-    // thread's stores and then for the block makes them globally visible before the count.
-    // (A device-scope fence would do the same by writing back and invalidating the whole L2,
-    // once per block - an order of magnitude slower here.)
-    uint32_t *done = a.done + (size_t)b * a.hkv + kvh;
-    __builtin_amdgcn_s_waitcnt(0);
-    __syncthreads();
-    if (threadIdx.x == 0)
-        s_last = __hip_atomic_fetch_add(done, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == (uint32_t)(ns - 1);
-    __syncthreads();
-    if (!s_last) return;
-    const size_t row0 = ((size_t)b * a.hq + kvh * G) * a.splits, out0 = ((size_t)b * a.hq + kvh * G) * D;
-    float *const part = attn_smem; // (the waves' outputs have been read)
-    if (ns <= 4) merge_splits<D, 4>(a, ns, G, row0, out0, part, kAttnThreads);
-    else merge_splits<D, 8>(a, ns, G, row0, out0, part, kAttnThreads);
-    if (threadIdx.x == 0) // ready for the next call on this stream
-        __hip_atomic_store(done, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    finish_block<D, W>(a, b, kvh, split, ns, wave, j, g, m_w, l_w, o);
 }
 
+// A wave goes through its share of the split 32 tokens at a time (the block's waves in turn: a split that the context ends in is
+// shared by all of them), under a running maximum.  The next 32 keys are requested as soon as these have met the queries, the next
+// values when these have met the probabilities, so the memory is never waited for with nothing under way, and what a block does once
+// -- lengths, queries, the merge of its waves, the partials and the count -- is paid once per split instead of once per 128 to 512
+// tokens.  Bound by the memory from some 50 MB on: 48 sequences of up to 6000 tokens, 8 heads of 128, 146.7 -> 125.7 us (5.6 TB/s).
+template <int D, int W, bool NT, class Args> __global__ __launch_bounds__(W * 64, 3) void paged_attn_stream_kernel(const Args a) {
+    constexpr int KS = D / 32, DT = D / 16;
+    if constexpr (std::is_same_v<Args, AttnFetchArgs>)
+        if (blockIdx.z != 0) { // (a branch on an argument would put its load's trip in front of the others')
+            fetch_weights<W>(a);
+            return;
+        }
+    const int kvh = blockIdx.x % a.hkv, b = blockIdx.x / a.hkv, split = blockIdx.y;
+    const int tok0 = split * a.split_tokens, G = a.group;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int j = lane & 15, g = lane >> 4;
+    const int32_t *table = a.block_table + (size_t)b * a.max_blocks;
+    struct Place {
+        int pb[2], in_block[2];
+    };
+    auto look_up = [&](int tok) {
+        Place p;
+#pragma unroll
+        for (int u = 0; u < 2; u++) {
+            const uint32_t lb = fastdiv((uint32_t)(tok + u * 16), a.d_block);
+            p.in_block[u] = tok + u * 16 - (int)lb * a.block_size;
+            p.pb[u] = table[min((int)lb, a.max_blocks - 1)]; // (a tile past the context: any entry, masked below)
+        }
+        return p;
+    };
+    int tok = tok0 + wave * 32;
+    Place at = look_up(tok);
+    const int ctx = min(a.ctx_lens[b] + a.len_offset, a.max_blocks * a.block_size);
+    if (ctx <= 0) { // empty context: zeros, written by the first block of the pair
+        if (split == 0)
+            for (int idx = threadIdx.x; idx < G * D; idx += W * 64) {
+                const size_t oi = ((size_t)b * a.hq + kvh * G) * D + idx;
+                if (a.out_f16) reinterpret_cast<__half *>(a.out)[oi] = __float2half_rn(0.f);
+                else reinterpret_cast<float *>(a.out)[oi] = 0.f;
+            }
+        return;
+    }
+    if (tok0 >= ctx) return; // uniform for the block
+    const int ns = (ctx + a.split_tokens - 1) / a.split_tokens, end = min(ctx, tok0 + a.split_tokens);
 
+    // The 32 tokens are dealt to the products so that a lane's eight of P.V, (g, e), are eight neighbours, 8 g + e: one 16-byte load of
+    // values.  Row 4 g + r of the u-th logit product is token 8 g + 4 u + r, so its rows come from both tiles.
+    const uint32_t koff = (uint32_t)(((j >> 2 & 1) * 8 + (j & 3)) * D + g * 8) * 2u, voff = (uint32_t)(j * a.block_size + (g & 1) * 8) * 2u;
+    const size_t vstep = (size_t)a.block_size * 32;
+    au32x4 kf[2][KS], vf[DT];
+    auto head_base = [&](int pb) { // a block id outside the cache would fault; read block 0 instead (undefined result, no fault)
+        return ((size_t)min(max(pb, 0), a.num_blocks - 1) * a.hkv + kvh) * (size_t)a.block_size * D;
+    };
+    auto request_keys = [&](const Place &p) {
+        const size_t b0 = head_base(p.pb[0]) + (size_t)p.in_block[0] * D, b1 = head_base(p.pb[1]) + (size_t)p.in_block[1] * D;
+        const char *kb = reinterpret_cast<const char *>(a.k_cache) + (j < 8 ? b0 : b1) * 2 + koff;
+#pragma unroll
+        for (int u = 0; u < 2; u++)
+#pragma unroll
+            for (int ks = 0; ks < KS; ks++) kf[u][ks] = *reinterpret_cast<const au32x4 *>(kb + u * (4 * D * 2) + ks * 64);
+    };
+    auto request_values = [&](const Place &p) {
+        const size_t b0 = head_base(p.pb[0]) + (size_t)p.in_block[0], b1 = head_base(p.pb[1]) + (size_t)p.in_block[1];
+        const char *vb = reinterpret_cast<const char *>(a.v_cache) + (g < 2 ? b0 : b1) * 2 + voff;
+#pragma unroll
+        for (int dt = 0; dt < DT; dt++) {
+            const au32x4 *const at = reinterpret_cast<const au32x4 *>(vb + dt * vstep);
+            vf[dt] = NT ? __builtin_nontemporal_load(at) : *at;
+        }
+    };
+    float m_w = -INFINITY, l_lane = 0.f;
+    f32x4 o[DT];
+#pragma unroll
+    for (int dt = 0; dt < DT; dt++) o[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
+    if (tok < end) { // uniform for the wave
+        f16x8 qf[KS];
+        {
+            const uint16_t *qp = a.q + ((size_t)b * a.hq + kvh * G + min(j, G - 1)) * D + g * 8;
+#pragma unroll
+            for (int ks = 0; ks < KS; ks++) {
+                au32x4 raw = *reinterpret_cast<const au32x4 *>(qp + ks * 32);
+                if (j >= G) raw = au32x4{0u, 0u, 0u, 0u};
+                __builtin_memcpy(&qf[ks], &raw, 16);
+            }
+        }
+        request_keys(at);
+        __builtin_amdgcn_sched_barrier(0);
+        request_values(at);
+        __builtin_amdgcn_sched_barrier(0);
+        // One step; LAST: the context may end in it, and nothing follows it.
+        auto step = [&](auto last_c) __attribute__((always_inline)) {
+            constexpr bool LAST = decltype(last_c)::value;
+            Place next = at;
+            if (!LAST) next = look_up(tok + W * 32);
+            __builtin_amdgcn_sched_barrier(0);
+            float s[2][4], m = -INFINITY;
+#pragma unroll
+            for (int t = 0; t < 2; t++) {
+                f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int ks = 0; ks < KS; ks++) {
+                    f16x8 kk;
+                    __builtin_memcpy(&kk, &kf[t][ks], 16);
+                    acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(kk, qf[ks], acc, 0, 0, 0);
+                }
+                const int left = ctx - (tok + g * 8 + t * 4); // valid tokens among this lane's four
+#pragma unroll
+                for (int r = 0; r < 4; r++) {
+                    s[t][r] = acc[r];
+                    if (!LAST || r < left) m = fmaxf(m, acc[r] * a.scale_log2e);
+                }
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            if (!LAST) request_keys(next);
+            __builtin_amdgcn_sched_barrier(0);
+            m = fmaxf(m, __shfl_xor(m, 16));
+            m = fmaxf(m, __shfl_xor(m, 32)); // (the first of the 32 is valid for every head: -inf only where the logits are)
+            if (__any(m > m_w)) {            // (uniform; seldom after the first few steps)
+                // (from the first step's maximum on by whole numbers, where a float has room for them: the factors are powers of two
+                // and round nothing)
+                const float up = m_w + ceilf(m - m_w), to = m > m_w ? (up >= m && up - m <= 1.f ? up : m) : m_w;
+                const float f = m > m_w ? __builtin_amdgcn_exp2f(m_w - to) : 1.f; // 0 on the first step
+                m_w = to, l_lane *= f;
+#pragma unroll
+                for (int r = 0; r < 4; r++) { // o[dt][r] belongs to head 4g + r
+                    const float fr = __shfl(f, g * 4 + r);
+#pragma unroll
+                    for (int dt = 0; dt < DT; dt++) o[dt][r] *= fr;
+                }
+            }
+            const float base = m_w == -INFINITY ? 0.f : m_w; // (logits of -inf alone so far: probabilities of 0)
+            // One rounding of the exponent: two were most of a large logit's error.  Of a logit whose float has steps of whole numbers
+            // the product is rounded as it was for the maximum, which would not be its own exponent's base otherwise.
+            float scale = a.scale_log2e;
+            if (__any(fabsf(base) > 65536.f)) {
+#pragma unroll
+                for (int u = 0; u < 2; u++)
+#pragma unroll
+                    for (int r = 0; r < 4; r++) s[u][r] *= scale;
+                scale = 1.f;
+            }
+            const int left = ctx - (tok + g * 8); // valid tokens among this lane's eight
+            f16x8 ph, pl;
+            float sum[2] = {0.f, 0.f}; // (a long run's sum takes one addition a step)
+#pragma unroll
+            for (int u = 0; u < 2; u++)
+#pragma unroll
+                for (int r = 0; r < 4; r++) {
+                    float p = __builtin_amdgcn_exp2f(__builtin_fmaf(s[u][r], scale, -base));
+                    if (LAST && left <= u * 4 + r) p = 0.f;
+                    sum[u] += p;
+                    const float ps = p * kProbScale;
+                    const _Float16 hi = (_Float16)ps;
+                    ph[u * 4 + r] = hi;
+                    pl[u * 4 + r] = (_Float16)(ps - (float)hi);
+                }
+            l_lane += sum[0] + sum[1];
+            au32x4 keep; // (what lies in a cache slot past the context may be anything)
+#pragma unroll
+            for (int d = 0; d < 4; d++) keep[d] = (left > 2 * d ? 0x0000ffffu : 0u) | (left > 2 * d + 1 ? 0xffff0000u : 0u);
+#pragma unroll
+            for (int dt = 0; dt < DT; dt++) {
+                const au32x4 raw = LAST ? vf[dt] & keep : vf[dt];
+                f16x8 vv;
+                __builtin_memcpy(&vv, &raw, 16);
+                // (the step's sum first: one rounding of the run's sum a step)
+                const f32x4 lo = __builtin_amdgcn_mfma_f32_16x16x32_f16(pl, vv, f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+                o[dt] += __builtin_amdgcn_mfma_f32_16x16x32_f16(ph, vv, lo, 0, 0, 0);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            if (!LAST) request_values(next);
+            __builtin_amdgcn_sched_barrier(0);
+            at = next;
+        };
+#pragma clang loop unroll(disable)
+        for (; tok + W * 32 < end; tok += W * 32) step(std::integral_constant<bool, false>());
+        step(std::integral_constant<bool, true>());
+#pragma unroll
+        for (int dt = 0; dt < DT; dt++) o[dt] *= 1.f / kProbScale;
+    }
+    float l_w = l_lane + __shfl_xor(l_lane, 16);
+    l_w += __shfl_xor(l_w, 32);
+    finish_block<D, W>(a, b, kvh, split, ns, wave, j, g, m_w, l_w, o);
+}
 
 // Sets `count` 32-bit words to zero (counter areas are cleared with a kernel, not a memset node, so
 // the call may sit inside a captured graph).
@@ -397,7 +606,8 @@ hipError_t attn_static_scratch_address(void **ptr) { return hipGetSymbolAddress(
 // Everything a launch needs except the buffers: checked geometry, split plan, sizes of the scratch areas.
 struct AttnPlan {
     AttnArgs a;
-    int nt = 2, waves = 8;
+    int nt = 2, waves = 8;               // of the kernel that has a block's whole share under way at once, or
+    bool stream = false, stream_values = false; // the one that goes through it
     size_t partial_bytes = 0, counter_bytes = 0;
 };
 
@@ -430,7 +640,10 @@ static int attn_plan(nncase_hip_ctx *ctx, const nncase_hip_paged_attn_args_t *p,
     a.num_blocks = p->num_blocks;
     a.len_offset = p->ctx_len_offset;
     const int64_t max_tokens = (int64_t)p->max_blocks_per_seq * p->block_size;
-    const AttnBlock block = choose_attn_block(p->head_dim, (int64_t)p->batch * p->num_kv_heads, max_tokens, ctx->compute_units);
+    const int64_t pairs = (int64_t)p->batch * p->num_kv_heads;
+    const int longest = p->head_dim == 64 ? 1024 : 512; // tokens per split that a capacity is accepted for
+    const int run = choose_attn_run(p->head_dim, pairs, max_tokens, ctx->compute_units);
+    const AttnBlock block = choose_attn_block(p->head_dim, pairs, max_tokens, ctx->compute_units);
     int nt = block.tiles, waves = block.waves;
     for (;;) { // (longer runs where there would be too many splits, for the merge or for the scratch there is)
         a.split_tokens = waves * nt * 16;
@@ -444,14 +657,54 @@ static int attn_plan(nncase_hip_ctx *ctx, const nncase_hip_paged_attn_args_t *p,
     }
     plan->nt = nt;
     plan->waves = waves;
+    plan->stream = plan->stream_values = false;
     NNHIP_REQUIRE(ctx, a.splits <= kAttnMaxSplits, -EINVAL,
                   "paged_attention_decode: context capacity of %lld tokens exceeds %d (head_dim %d)", (long long)max_tokens,
                   kAttnMaxSplits * a.split_tokens, p->head_dim);
+    if (run > 0) {
+        auto bytes = [&](int64_t splits) { return (size_t)(a.batch * a.hq * splits * (a.d + 2) * (int64_t)sizeof(float)); };
+        const int64_t splits = (max_tokens + run - 1) / run;
+        // (what is refused for want of scratch does not depend on which kernel it would be)
+        const size_t needed = bytes(std::max(splits, (max_tokens + longest - 1) / longest));
+        if (splits <= kAttnMaxSplits && needed <= most_partial_bytes) {
+            a.split_tokens = run, a.splits = (int)splits, plan->partial_bytes = needed, plan->stream = true;
+            plan->stream_values = pairs * max_tokens * a.d * 4 >= kStreamedBytes;
+        }
+    }
     a.d_block = make_fastdiv((uint32_t)p->block_size);
     a.scale_log2e = p->scale * kLog2e;
     a.out_f16 = p->out_dtype == NNCASE_HIP_DT_F16;
     plan->counter_bytes = (size_t)a.batch * a.hkv * sizeof(uint32_t);
     return 0;
+}
+
+template <class Args> static bool attn_launch_kernel(nncase_hip_ctx *ctx, const AttnPlan &plan, dim3 grid, int waves, const Args &a) {
+    const dim3 block(waves * 64);
+    const size_t lds = attn_lds_bytes(a.d, waves);
+    bool launched = false;
+    auto go = [&](auto kernel) {
+        if (lds > 65536) { // more than 64 KiB of dynamic LDS has to be asked for (cheap: a field of the function's record)
+            if (hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess) return;
+        }
+        hipLaunchKernelGGL(kernel, grid, block, lds, ctx->stream, a);
+        launched = true;
+    };
+    if (plan.stream) {
+        if (a.d == 64) {
+            if constexpr (std::is_same_v<Args, AttnArgs>) go(paged_attn_stream_kernel<64, kStreamWaves, false, Args>); // (one split)
+        } else if (plan.stream_values) {
+            go(paged_attn_stream_kernel<128, kStreamWaves, true, Args>);
+        } else {
+            go(paged_attn_stream_kernel<128, kStreamWaves, false, Args>);
+        }
+        return launched;
+    }
+#define NNHIP_ATTN_CASE(DV, NTV, WV) \
+    if (!launched && a.d == DV && plan.nt == NTV && waves == WV) go(paged_attn_kernel<DV, NTV, WV, Args>);
+    NNHIP_ATTN_CASE(64, 2, 4) NNHIP_ATTN_CASE(64, 4, 4) NNHIP_ATTN_CASE(64, 2, 8) NNHIP_ATTN_CASE(64, 4, 8) NNHIP_ATTN_CASE(64, 8, 8)
+    NNHIP_ATTN_CASE(128, 2, 4) NNHIP_ATTN_CASE(128, 4, 4) NNHIP_ATTN_CASE(128, 2, 8) NNHIP_ATTN_CASE(128, 4, 8)
+#undef NNHIP_ATTN_CASE
+    return launched;
 }
 
 static int attn_launch(nncase_hip_ctx *ctx, AttnPlan &plan, const void *q_dev, const void *k_cache_dev, const void *v_cache_dev,
@@ -467,35 +720,26 @@ static int attn_launch(nncase_hip_ctx *ctx, AttnPlan &plan, const void *q_dev, c
     a.done = reinterpret_cast<uint32_t *>(counters);
     a.part_o = reinterpret_cast<float *>(partials);
     a.part_ml = a.part_o + (size_t)a.batch * a.hq * a.splits * a.d;
-    const int nt = plan.nt, waves = plan.waves;
+    const int waves = plan.stream ? kStreamWaves : plan.waves;
     dim3 grid(a.hkv * a.batch, a.splits);
     const int64_t own = (int64_t)grid.x * grid.y;
     // Weights are fetched beside launches that merge splits (one that does not is over before they are here: 8 sequences of 100
     // tokens, a decode layer 25.2 -> 25.5 us) and that leave memory idle (64 sequences of 2048, 1152 blocks: 49.3 -> 49.7; 32 of
     // them, 576 blocks: 39.8 -> 39.5; one of 700, 12 blocks: 24.8 -> 22.9).
+    bool launched;
     if (fetch && fetch->count > 0 && a.splits > 1 && own <= 3 * ctx->compute_units) {
-        a.fetch = *fetch;
+        AttnFetchArgs f;
+        static_cast<AttnArgs &>(f) = a;
+        f.fetch = *fetch;
         uint32_t fragments = 0; // of die 0, which has the most
         for (int i = 0; i < fetch->count; i++) fragments += fetch_fragments(fetch->f[i], 0);
-        a.fetch.blocks = (int)((fragments + waves * kFetchBatch - 1) / (waves * kFetchBatch));
-        grid.z = 1 + (unsigned)(((int64_t)a.fetch.blocks * kXcds + own - 1) / own);
+        f.fetch.blocks = (int)((fragments + waves * kFetchBatch - 1) / (waves * kFetchBatch));
+        grid.z = 1 + (unsigned)(((int64_t)f.fetch.blocks * kXcds + own - 1) / own);
+        launched = attn_launch_kernel(ctx, plan, grid, waves, f);
+    } else {
+        launched = attn_launch_kernel(ctx, plan, grid, waves, a);
     }
-    const dim3 block(waves * 64);
-    const size_t lds = attn_lds_bytes(a.d, waves);
-    bool launched = false;
-    auto go = [&](auto kernel) {
-        if (lds > 65536) { // more than 64 KiB of dynamic LDS has to be asked for (cheap: a field of the function's record)
-            if (hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess) return;
-        }
-        hipLaunchKernelGGL(kernel, grid, block, lds, ctx->stream, a);
-        launched = true;
-    };
-#define NNHIP_ATTN_CASE(DV, NTV, WV) \
-    if (!launched && a.d == DV && nt == NTV && waves == WV) go(paged_attn_kernel<DV, NTV, WV>);
-    NNHIP_ATTN_CASE(64, 2, 4) NNHIP_ATTN_CASE(64, 4, 4) NNHIP_ATTN_CASE(64, 2, 8) NNHIP_ATTN_CASE(64, 4, 8) NNHIP_ATTN_CASE(64, 8, 8)
-    NNHIP_ATTN_CASE(128, 2, 4) NNHIP_ATTN_CASE(128, 4, 4) NNHIP_ATTN_CASE(128, 2, 8) NNHIP_ATTN_CASE(128, 4, 8)
-#undef NNHIP_ATTN_CASE
-    NNHIP_REQUIRE(ctx, launched, -EINVAL, "paged_attention_decode: no kernel for head_dim %d, %d tiles per wave, %d waves", a.d, nt, waves);
+    NNHIP_REQUIRE(ctx, launched, -EINVAL, "paged_attention_decode: no kernel for head_dim %d, %d tiles per wave, %d waves", a.d, plan.nt, waves);
     NNHIP_LAUNCH_CHECK(ctx, "paged_attn_kernel");
     return 0;
 }

@@ -2,6 +2,7 @@
 // measured times without a device.
 #pragma once
 
+#include <algorithm>
 #include <cstdint>
 
 namespace nnhip {
@@ -36,6 +37,29 @@ inline AttnBlock choose_attn_block(int head_dim, int64_t pairs, int64_t max_toke
     if (max_tokens >= 3200 && per_ten_units >= 17 && per_ten_units <= 23) return {4, 8};
     if (max_tokens >= 6500 && 4 * blocks(512) >= compute_units && blocks(512) <= 3ll * compute_units) return {4, 8};
     return {4, 4};
+}
+
+// Tokens per split of the kernel that goes through a split 128 tokens at a time, or 0 where the one above is taken (us, that one's
+// best block / in steps):
+//   * 64-wide heads, 257 to 512 tokens, from 24 pairs: one split, no merge (24 pairs of 265 tokens 5.8 / 5.3, 60 of 459 6.6 / 6.2, 240
+//     of 384 7.8 / 5.9; 12 of 433 6.2 / 6.4).  Longer contexts come out even with that (12 pairs of 13 658 13.9 / 12.7, 84 of 4759
+//     16.4 / 17.9, 132 of 14 756 50.7 / 52.1)
+//   * 128-wide heads from 50 MB of keys and values on (48 pairs of 1851 15.2 / 13.8, 36 of 6028 22.3 / 17.9, 104 of 9746 107 / 80, 656 of
+//     4073 267 / 229; below, 64 of 1205 12.1 / 13.0 and 8 of 4387 12.3 / 14.0), which few pairs reach with long contexts only, and too
+//     many splits (8 of 12 668 18.4 / 20.0).
+// There one split up to 384 tokens, else as many as make one round of the device, a block per compute unit: fewer leave units idle, a
+// second round costs as much as the first (with runs of 256 / 512 / 1024 / 2048: 32 of 3425 12.6 11.3 15.3 23.9, 80 of 2220 19.0 18.8
+// 16.8 25.2).  Where splits of 2048 tokens would still be more than that: 512 tokens, which even the rounds out (152 of 10 998 82.7
+// 77.6 82.4 91.1), or 1024 where that is the whole context or with nine rounds and more (1600 of 1500 136 126 117 119).
+inline int choose_attn_run(int head_dim, int64_t pairs, int64_t max_tokens, int compute_units) {
+    auto even = [&](int64_t splits) { return (int)(((max_tokens + splits - 1) / splits + 127) / 128 * 128); };
+    if (head_dim == 64) return max_tokens > 256 && max_tokens <= 512 && pairs >= 24 ? even(1) : 0;
+    if (pairs < 16 || pairs * max_tokens < 98304) return 0;
+    if (max_tokens <= 384) return even(1);
+    const int64_t one_round = compute_units / pairs;
+    if (one_round >= 1 && even(one_round) <= 2048) return std::max(even(one_round), 256);
+    if (max_tokens <= 1024) return 1024;
+    return pairs * ((max_tokens + 1023) / 1024) >= 9ll * compute_units ? 1024 : 512;
 }
 
 } // namespace nnhip

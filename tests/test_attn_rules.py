@@ -81,3 +81,38 @@ def test_every_choice_is_a_kernel_that_is_built(choose):
         for pairs in (1, 3, 8, 30, 64, 200, 256, 257, 1000, 100000):
             for tokens in list(range(1, 1200, 37)) + [2048, 3200, 4096, 4112, 6500, 9999, 10000, 16384, 131072, 1 << 20]:
                 assert choose(d, pairs, tokens, 256) in SHAPES
+
+
+# head_dim, pairs, capacity in tokens, us of the block chosen above, us with the split gone through in steps
+STEPS = [
+    (64, 12, 433, 6.2, 6.4), (64, 24, 265, 5.8, 5.3), (64, 60, 459, 6.6, 6.2), (64, 240, 384, 7.8, 5.9), (64, 84, 4759, 16.4, 17.9),
+    (64, 144, 3041, 16.7, 18.2), (64, 132, 14756, 50.7, 52.1), (128, 64, 1205, 12.1, 13.0), (128, 8, 4387, 12.3, 14.0), (128, 4, 993, 8.6, 9.3),
+    (128, 36, 6028, 22.3, 17.9), (128, 104, 9746, 106.9, 79.6), (128, 256, 490, 13.0, 10.2), (128, 624, 280, 21.6, 19.0), (128, 656, 4073, 266.7, 229.1),
+    (128, 16, 15583, 32.1, 21.7), (128, 8, 12668, 18.4, 20.0),
+]
+
+
+@pytest.fixture(scope="module")
+def choose_run(tmp_path_factory):
+    d = tmp_path_factory.mktemp("run")
+    (d / "r.cpp").write_text("""#include "attn_rules.hpp"
+extern "C" int choose_run(int head_dim, long pairs, long tokens, int cus) { return nnhip::choose_attn_run(head_dim, pairs, tokens, cus); }
+""")
+    subprocess.check_call(["g++", "-std=c++17", "-shared", "-fPIC", "-I", CSRC, str(d / "r.cpp"), "-o", str(d / "r.so")])
+    fn = C.CDLL(str(d / "r.so")).choose_run
+    fn.argtypes = [C.c_int, C.c_long, C.c_long, C.c_int]
+    return fn
+
+
+@pytest.mark.parametrize("row", STEPS, ids=lambda r: "%d-%d-%d" % r[:3])
+def test_steps_are_taken_where_they_are_quicker(choose_run, row):
+    assert (choose_run(row[0], row[1], row[2], 256) > 0) == (row[4] < row[3])
+
+
+def test_runs_are_whole_steps(choose_run):
+    for d in (64, 128):
+        for pairs in (1, 16, 24, 30, 64, 200, 256, 257, 1000, 100000, 1 << 30):
+            for tokens in list(range(1, 1200, 37)) + [2048, 4112, 9999, 131072, 1 << 20, (1 << 31) - 1]:
+                run = choose_run(d, pairs, tokens, 256)
+                assert run % 128 == 0 and 0 <= run <= 2048
+                assert run == 0 or d == 128 or run >= tokens      # (64-wide heads: one split alone)

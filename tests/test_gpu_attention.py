@@ -246,3 +246,54 @@ def test_a_workspace_that_cannot_grow_takes_longer_runs(hip_ctx):
         ctx.sync()
     finally:
         ctx.close()
+
+
+@pytest.mark.parametrize("b,hq,hkv,d,blk,capacity", [
+    (2, 32, 8, 128, 16, 6144), (16, 16, 1, 128, 48, 6144), (38, 8, 8, 128, 32, 704), (26, 28, 4, 128, 64, 1024), (33, 8, 8, 128, 16, 384),
+    (9, 32, 32, 128, 16, 1040), (16, 64, 64, 128, 16, 1024), (64, 16, 16, 128, 16, 1040),
+    (12, 14, 2, 64, 16, 272), (24, 16, 1, 64, 64, 320), (3, 12, 12, 64, 48, 480), (40, 24, 24, 64, 16, 512)])
+def test_a_split_gone_through_in_steps(hip_ctx, b, hq, hkv, d, blk, capacity):
+    """Launches of the kernel that goes through a split 128 tokens at a time (few splits, one split, 512 and 1024 tokens each, values
+    past the caches): contexts that end around a wave's 32 tokens, a step and the splits.  Slots past a context hold NaN."""
+    rng = np.random.default_rng(b * 1000 + capacity)
+    edges = [1, 31, 32, 33, 127, 128, 129, 255, 257, 383, 385, 511, 513, 1023, 1025, capacity - 1, capacity]
+    lens = np.asarray([n for n in edges if n <= capacity] + [0], np.int32)
+    cl = np.resize(np.roll(lens, 1 + b % 5), b)
+    cl[0] = capacity
+    blocks, nb = capacity // blk, 40     # (entries of the table repeat: the caches stay small)
+    q = rng.standard_normal((b, hq, d)).astype(np.float16)
+    kc, vc = (rng.standard_normal((nb + b, hkv, blk, d)).astype(np.float16) for _ in range(2))
+    bt = rng.integers(0, nb, (b, blocks)).astype(np.int32)
+    for i, n in enumerate(cl):           # a sequence's last, partly filled block is its own
+        if n % blk:
+            bt[i, n // blk] = nb + i
+            kc[nb + i, :, n % blk:], vc[nb + i, :, n % blk:] = np.nan, np.nan
+    vt = K.v_cache_from_token_major(vc)
+    got = K.paged_attention_decode(q, kc, vt, bt, cl, d ** -0.5, np.float32, ctx=hip_ctx).astype(np.float64)
+    want = O.paged_attention_decode(q.view(np.uint16), np.nan_to_num(kc).view(np.uint16), np.nan_to_num(vt).view(np.uint16), bt, cl, d ** -0.5)
+    # of the exponent's rounding (at most 2^-23 of a logit of about 8 / ln 2), the float32 sums' and the final division's: 1e-5
+    assert (np.abs(got - want) <= 1e-5 * np.abs(want).max(axis=-1, keepdims=True)).all(), f"max err {np.abs(got - want).max()}"
+
+
+def test_infinite_and_very_large_logits_in_steps(hip_ctx):
+    """Whole steps of keys at -inf have no weight, whatever comes before and after them; logits whose float32 neighbours are thousands
+    apart choose one key."""
+    rng = np.random.default_rng(23)
+    b, hq, hkv, d, blk, capacity = 2, 16, 8, 128, 16, 6144
+    q = rng.uniform(0.5, 1, (b, hq, d)).astype(np.float16)
+    kc, vc = (rng.standard_normal((b * capacity // blk, hkv, blk, d)).astype(np.float16) for _ in range(2))
+    bt = np.arange(b * capacity // blk, dtype=np.int32).reshape(b, -1)
+    dead = kc.copy()
+    dead[:8], dead[24:32], dead[100:104], dead[384:400] = -np.inf, -np.inf, -np.inf, -np.inf
+    vt = K.v_cache_from_token_major(vc)
+    cl = np.asarray([capacity, 700], np.int32)
+    got = K.paged_attention_decode(q, dead, vt, bt, cl, d ** -0.5, np.float32, ctx=hip_ctx).astype(np.float64)
+    want = O.paged_attention_decode(q.view(np.uint16), np.maximum(dead, np.float16(-60000)).view(np.uint16), vt.view(np.uint16), bt, cl, d ** -0.5)
+    assert (np.abs(got - want) <= 1e-5 * np.abs(want).max(axis=-1, keepdims=True)).all()
+    big = (kc * 8000).clip(-60000, 60000).astype(np.float16)
+    got = K.paged_attention_decode((q * 60000).astype(np.float16), big, vt, bt, cl, 1.0, np.float32, ctx=hip_ctx)
+    for i in range(b):
+        for h in range(hq):
+            keys = big[bt[i], h // 2].reshape(-1, d)[: cl[i]].astype(np.float64)
+            at = np.argmax(keys @ (q[i, h] * 60000).astype(np.float16).astype(np.float64))
+            assert np.array_equal(got[i, h], vc[bt[i], h // 2].reshape(-1, d)[at].astype(np.float32))
