@@ -406,7 +406,7 @@ template <int D, int NT, int W, class Args> __global__ __launch_bounds__(W * 64,
 // shared by all of them), under a running maximum.  The next 32 keys are requested as soon as these have met the queries, the next
 // values when these have met the probabilities, so the memory is never waited for with nothing under way, and what a block does once
 // -- lengths, queries, the merge of its waves, the partials and the count -- is paid once per split instead of once per 128 to 512
-// tokens.  Bound by the memory from some 50 MB on: 48 sequences of up to 6000 tokens, 8 heads of 128, 146.7 -> 125.7 us (5.6 TB/s).
+// tokens.  Bound by the memory from some 50 MB on: 48 sequences of up to 6000 tokens, 8 heads of 128, 146.7 -> 125.7 us (5.4 TB/s).
 template <int D, int W, bool NT, class Args> __global__ __launch_bounds__(W * 64, 3) void paged_attn_stream_kernel(const Args a) {
     constexpr int KS = D / 32, DT = D / 16;
     if constexpr (std::is_same_v<Args, AttnFetchArgs>)

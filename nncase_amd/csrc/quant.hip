@@ -1,8 +1,7 @@
 // Quantize / Dequantize streaming kernels and the u8 elementwise glue
 // (residual add, global average pool).  All HBM-bound: every thread moves
-// 4 elements per step with one vector load and one vector store, the grid is
-// a few waves per SIMD deep and walks the tensor with a grid stride so the
-// loads of several steps are in flight together.
+// pieces of up to 16 bytes, all requested before the first is used, and a
+// block owns neighbouring ones.
 //
 // Arithmetic contracts (each fp32 step is a single IEEE operation; the file
 // is compiled with -ffp-contract=off):
@@ -14,64 +13,113 @@
 
 #include <algorithm>
 #include <cmath>
+#include <type_traits>
 
 namespace nnhip {
 
 constexpr int kEwThreads = 256;
-constexpr int kEwVec = 4;
 constexpr int kEwUnroll = 4;
 
-template <typename T> struct Vec4;
-template <> struct Vec4<float> { typedef float4 type; };
-template <> struct Vec4<int32_t> { typedef int4 type; };
-template <> struct Vec4<__half> { typedef uint2 type; };
-template <> struct Vec4<int16_t> { typedef uint2 type; };
-template <> struct Vec4<uint8_t> { typedef uint32_t type; };
-template <> struct Vec4<int8_t> { typedef uint32_t type; };
-
-template <typename T> __device__ __forceinline__ void load4(const T *p, T (&v)[4]) {
-    typename Vec4<T>::type raw = *reinterpret_cast<const typename Vec4<T>::type *>(p);
-    __builtin_memcpy(v, &raw, sizeof(raw));
+// V neighbouring elements at any address a T may have; PAST: through the caches without a stay there
+template <int BYTES> struct PieceWord;
+template <> struct PieceWord<1> { typedef uint8_t type; };
+template <> struct PieceWord<2> { typedef uint16_t type __attribute__((aligned(1))); };
+template <> struct PieceWord<4> { typedef uint32_t type __attribute__((aligned(1))); };
+template <> struct PieceWord<8> { typedef uint32_t type __attribute__((ext_vector_type(2), aligned(1))); };
+template <> struct PieceWord<16> { typedef uint32_t type __attribute__((ext_vector_type(4), aligned(1))); };
+template <bool PAST, int V, typename T> __device__ __forceinline__ void load_piece(const T *p, T (&v)[V]) {
+    typedef typename PieceWord<sizeof(T) * V>::type W;
+    const W raw = PAST ? __builtin_nontemporal_load(reinterpret_cast<const W *>(p)) : *reinterpret_cast<const W *>(p);
+    __builtin_memcpy(v, &raw, sizeof(v));
 }
-template <typename T> __device__ __forceinline__ void store4(T *p, const T (&v)[4]) {
-    typename Vec4<T>::type raw;
-    __builtin_memcpy(&raw, v, sizeof(raw));
-    *reinterpret_cast<typename Vec4<T>::type *>(p) = raw;
+template <bool PAST, int V, typename T> __device__ __forceinline__ void store_piece(T *p, const T (&v)[V]) {
+    typedef typename PieceWord<sizeof(T) * V>::type W;
+    W raw;
+    __builtin_memcpy(&raw, v, sizeof(v));
+    if (PAST) __builtin_nontemporal_store(raw, reinterpret_cast<W *>(p));
+    else *reinterpret_cast<W *>(p) = raw;
 }
+// Elements per load and store: up to 16 bytes of either, but no more than 4 codes of a byte read at once (u8 -> f16 by 8: 1.5 % slower).
+template <typename A, typename B> constexpr int piece_elements() { return sizeof(A) == 2 && sizeof(B) <= 2 ? 8 : 4; }
 
 template <typename T> __device__ __forceinline__ float to_f32(T v) { return (float)v; }
 template <> __device__ __forceinline__ float to_f32<__half>(__half v) { return __half2float(v); }
 
-template <typename TIn, typename TQ>
-__global__ __launch_bounds__(kEwThreads) void quantize_kernel(const TIn *__restrict__ in, TQ *__restrict__ out,
-                                                              size_t count, float scale, float bias, int vec_ok) {
-    const size_t tid = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const size_t nthreads = (size_t)gridDim.x * blockDim.x;
-    const size_t nvec = vec_ok ? count / kEwVec : 0;
-    // a block owns kEwUnroll * kEwThreads neighbouring vectors (see ew_block_grid)
-    const size_t i = (size_t)blockIdx.x * (kEwUnroll * kEwThreads) + threadIdx.x;
-    if (i + (kEwUnroll - 1) * kEwThreads < nvec) {
-        TIn v[kEwUnroll][4];
+// A block owns U * kEwThreads neighbouring pieces, each read and written where it lies; the last block's last elements, fewer than a
+// piece, take a thread each.
+template <int U, bool PAST, typename A, typename B, class F> __device__ __forceinline__ void for_pieces(const A *in, B *out, size_t count, F &&f) {
+    constexpr int V = piece_elements<A, B>();
+    const size_t first = (size_t)blockIdx.x * (U * kEwThreads * V), i = first + threadIdx.x * V;
+    if (first + U * kEwThreads * V <= count) {
+        A v[U][V];
 #pragma unroll
-        for (int u = 0; u < kEwUnroll; u++) load4(in + (i + u * kEwThreads) * kEwVec, v[u]);
+        for (int u = 0; u < U; u++) load_piece<PAST, V>(in + i + u * kEwThreads * V, v[u]);
+        __builtin_amdgcn_sched_barrier(0); // (every request before the first piece is waited for)
 #pragma unroll
-        for (int u = 0; u < kEwUnroll; u++) {
-            TQ q[4];
-#pragma unroll
-            for (int e = 0; e < 4; e++) q[e] = quantize_one<TQ>(to_f32(v[u][e]), scale, bias);
-            store4(out + (i + u * kEwThreads) * kEwVec, q);
+        for (int u = 0; u < U; u++) {
+            B w[V];
+            f(v[u], w);
+            store_piece<PAST, V>(out + i + u * kEwThreads * V, w);
         }
-    } else {
-        for (size_t k = i; k < nvec && k < i + kEwUnroll * kEwThreads; k += kEwThreads) {
-            TIn v[4];
-            TQ q[4];
-            load4(in + k * kEwVec, v);
-#pragma unroll
-            for (int e = 0; e < 4; e++) q[e] = quantize_one<TQ>(to_f32(v[e]), scale, bias);
-            store4(out + k * kEwVec, q);
-        }
+        return;
     }
-    for (size_t j = nvec * kEwVec + tid; j < count; j += nthreads) out[j] = quantize_one<TQ>(to_f32(in[j]), scale, bias);
+    for (size_t k = i; k + V <= count; k += kEwThreads * V) {
+        A v[V];
+        B w[V];
+        load_piece<PAST, V>(in + k, v);
+        f(v, w);
+        store_piece<PAST, V>(out + k, w);
+    }
+    const size_t k = count / V * V + threadIdx.x;
+    if (k < count) {
+        const A v[1] = {in[k]};
+        B w[1];
+        f(v, w);
+        out[k] = w[0];
+    }
+}
+
+// What quantize divides by.  QUICK: x / scale by the reciprocal, 3 instructions instead of some 11, which bound the kernel (25 M
+// elements f16 -> u8: 14.9 -> 12.0 us, 6.3 TB/s; 3.3 M f32 -> u8 4.5 -> 3.3).  q0 = x * r is within 1.5 ulp of the quotient and q0 + (x - scale * q0) * r, rounded once, is
+// the quotient's nearest float (held by enumeration of every pair of mantissas whose quotient lies near enough to the middle of two
+// floats).  A q0 far past every code is cut to +-2^40, so that an infinity leaves no difference of two infinities behind; a NaN stays
+// one up to the conversion, which makes the lowest code of it like the general form.
+struct Divisor {
+    float scale, reciprocal, bias;
+};
+constexpr float kReach = 0x1p40f;
+// scales from 2^-60 to 2^60: no quotient that a code depends on, nor its residual, leaves the range of normal floats
+inline bool quick_divisor(float scale) { return std::fabs(scale) >= 0x1p-60f && std::fabs(scale) <= 0x1p60f; }
+
+template <typename TQ, int V, typename TIn> __device__ __forceinline__ void quantize_quick(const TIn (&x)[V], TQ (&q)[V], const Divisor &d) {
+    float v[V];
+#pragma unroll
+    for (int e = 0; e < V; e++) {
+        const float f = to_f32(x[e]), q0 = __builtin_amdgcn_fmed3f(f * d.reciprocal, -kReach, kReach);
+        v[e] = __builtin_fmaf(__builtin_fmaf(-d.scale, q0, f), d.reciprocal, q0) + d.bias;
+    }
+    if constexpr (std::is_same_v<TQ, uint8_t> && V % 4 == 0) {
+        uint32_t w[V / 4];
+#pragma unroll
+        for (int e = 0; e < V; e++) w[e / 4] = __builtin_amdgcn_cvt_pk_u8_f32(v[e], e % 4, e % 4 ? w[e / 4] : 0u);
+        __builtin_memcpy(q, w, sizeof(q));
+    } else {
+#pragma unroll
+        for (int e = 0; e < V; e++) q[e] = (TQ)(int32_t)rintf(__builtin_amdgcn_fmed3f(v[e], QLimits<TQ>::lo, QLimits<TQ>::hi));
+    }
+}
+
+template <typename TIn, typename TQ, int U, bool PAST, bool QUICK>
+__global__ __launch_bounds__(kEwThreads) void quantize_kernel(const TIn *__restrict__ in, TQ *__restrict__ out, size_t count, const Divisor d) {
+    for_pieces<U, PAST>(in, out, count, [&](const auto &x, auto &q) {
+        constexpr int V = sizeof(x) / sizeof(TIn);
+        if constexpr (QUICK) {
+            quantize_quick<TQ, V>(x, q, d);
+        } else {
+#pragma unroll
+            for (int e = 0; e < V; e++) q[e] = quantize_one<TQ>(to_f32(x[e]), d.scale, d.bias);
+        }
+    });
 }
 
 template <typename TOut> __device__ __forceinline__ TOut from_f32(float v);
@@ -84,35 +132,12 @@ template <> __device__ __forceinline__ __half from_f32<__half>(float v) {
     return __float2half_rn(v);
 }
 
-template <typename TQ, typename TOut>
-__global__ __launch_bounds__(kEwThreads) void dequantize_kernel(const TQ *__restrict__ in, TOut *__restrict__ out,
-                                                                size_t count, float scale, float bias, int vec_ok) {
-    const size_t tid = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const size_t nthreads = (size_t)gridDim.x * blockDim.x;
-    const size_t nvec = vec_ok ? count / kEwVec : 0;
-    const size_t i = (size_t)blockIdx.x * (kEwUnroll * kEwThreads) + threadIdx.x;
-    if (i + (kEwUnroll - 1) * kEwThreads < nvec) {
-        TQ v[kEwUnroll][4];
+template <typename TQ, typename TOut, int U, bool PAST>
+__global__ __launch_bounds__(kEwThreads) void dequantize_kernel(const TQ *__restrict__ in, TOut *__restrict__ out, size_t count, float scale, float bias) {
+    for_pieces<U, PAST>(in, out, count, [&](const auto &q, auto &y) {
 #pragma unroll
-        for (int u = 0; u < kEwUnroll; u++) load4(in + (i + u * kEwThreads) * kEwVec, v[u]);
-#pragma unroll
-        for (int u = 0; u < kEwUnroll; u++) {
-            TOut y[4];
-#pragma unroll
-            for (int e = 0; e < 4; e++) y[e] = from_f32<TOut>(((float)v[u][e] - bias) * scale);
-            store4(out + (i + u * kEwThreads) * kEwVec, y);
-        }
-    } else {
-        for (size_t k = i; k < nvec && k < i + kEwUnroll * kEwThreads; k += kEwThreads) {
-            TQ v[4];
-            TOut y[4];
-            load4(in + k * kEwVec, v);
-#pragma unroll
-            for (int e = 0; e < 4; e++) y[e] = from_f32<TOut>(((float)v[e] - bias) * scale);
-            store4(out + k * kEwVec, y);
-        }
-    }
-    for (size_t j = nvec * kEwVec + tid; j < count; j += nthreads) out[j] = from_f32<TOut>(((float)in[j] - bias) * scale);
+        for (int e = 0; e < (int)(sizeof(q) / sizeof(TQ)); e++) y[e] = from_f32<TOut>(((float)q[e] - bias) * scale);
+    });
 }
 
 // Strided forms: element `index` of a tensor of `rank` dimensions is read at sum(index[d] * in_strides[d]) and
@@ -240,32 +265,46 @@ inline int ew_grid(const nncase_hip_ctx *ctx, size_t work_items) {
 
 inline bool aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
-// Quantize / dequantize: a block per kEwUnroll * kEwThreads neighbouring vectors, however many that makes.  Blocks that
+// Quantize / dequantize: a block per U * kEwThreads neighbouring pieces, however many that makes.  Blocks that
 // run at the same time then read and write neighbouring addresses (measured on 100 M elements against a capped grid that
-// strides over the tensor: quantize f32 -> u8 114 -> 96 us, dequantize i32 -> f32 202 -> 136 us).  Without vectors (an
-// unaligned buffer) the capped grid walks the elements.
-inline int ew_block_grid(const nncase_hip_ctx *ctx, size_t count, bool vec_ok) {
-    if (!vec_ok) return ew_grid(ctx, count);
-    const size_t per_block = (size_t)kEwUnroll * kEwThreads * kEwVec;
-    return (int)std::max<size_t>(1, (count + per_block - 1) / per_block);
+// strides over the tensor: quantize f32 -> u8 114 -> 96 us, dequantize i32 -> f32 202 -> 136 us).  Four pieces a thread where that leaves
+// two blocks per compute unit (one of bytes), else one (0.5 M f32 -> u8 3.3 -> 2.5 us; 1.04 M u8 -> f16 2.6 with four, 2.8 with one).
+template <typename A, typename B> inline unsigned piece_blocks(size_t count, int unroll) {
+    const size_t per_block = (size_t)unroll * kEwThreads * piece_elements<A, B>();
+    return (unsigned)((count + per_block - 1) / per_block);
+}
+// Both sides' bytes from which on next to nothing of them is in a cache when the next operator comes (the memory side's holds 256 MiB;
+// us through the caches / past them: f32 -> u8 of 275 MB 42.8 / 46.0, of 300 MB 48.7 / 48.3, of 375 MB 70.6 / 62.4, i32 -> f32 of 428 MB
+// 76.7 / 68.6)
+constexpr size_t kPastCaches = 300000000;
+// go(pieces per thread, past the caches)
+template <typename A, typename B, class F> void with_piece_form(const nncase_hip_ctx *ctx, size_t count, F &&go) {
+    const bool several = count >= (size_t)(sizeof(A) == 1 ? 1 : 2) * ctx->compute_units * (kEwUnroll * kEwThreads * piece_elements<A, B>());
+    if (!several) go(std::integral_constant<int, 1>(), std::false_type());
+    else if (count * (sizeof(A) + sizeof(B)) < kPastCaches) go(std::integral_constant<int, kEwUnroll>(), std::false_type());
+    else go(std::integral_constant<int, kEwUnroll>(), std::true_type());
 }
 
 template <typename TIn, typename TQ>
 int launch_quantize(nncase_hip_ctx *ctx, const void *in, void *out, size_t count, float scale, float bias) {
-    const int vec_ok = aligned16(in) && aligned16(out);
-    const int grid = ew_block_grid(ctx, count, vec_ok);
-    hipLaunchKernelGGL((quantize_kernel<TIn, TQ>), dim3(grid), dim3(kEwThreads), 0, ctx->stream, (const TIn *)in,
-                       (TQ *)out, count, scale, bias, vec_ok);
+    const Divisor d{scale, 1.f / scale, bias};
+    with_piece_form<TIn, TQ>(ctx, count, [&](auto u, auto past) {
+        auto go = [&](auto kernel) {
+            hipLaunchKernelGGL(kernel, dim3(piece_blocks<TIn, TQ>(count, u)), dim3(kEwThreads), 0, ctx->stream, (const TIn *)in, (TQ *)out, count, d);
+        };
+        if (quick_divisor(scale)) go(quantize_kernel<TIn, TQ, u, past, true>);
+        else go(quantize_kernel<TIn, TQ, u, past, false>);
+    });
     NNHIP_LAUNCH_CHECK(ctx, "quantize_kernel");
     return 0;
 }
 
 template <typename TQ, typename TOut>
 int launch_dequantize(nncase_hip_ctx *ctx, const void *in, void *out, size_t count, float scale, float bias) {
-    const int vec_ok = aligned16(in) && aligned16(out);
-    const int grid = ew_block_grid(ctx, count, vec_ok);
-    hipLaunchKernelGGL((dequantize_kernel<TQ, TOut>), dim3(grid), dim3(kEwThreads), 0, ctx->stream, (const TQ *)in,
-                       (TOut *)out, count, scale, bias, vec_ok);
+    with_piece_form<TQ, TOut>(ctx, count, [&](auto u, auto past) {
+        hipLaunchKernelGGL((dequantize_kernel<TQ, TOut, u, past>), dim3(piece_blocks<TQ, TOut>(count, u)), dim3(kEwThreads), 0, ctx->stream,
+                           (const TQ *)in, (TOut *)out, count, scale, bias);
+    });
     NNHIP_LAUNCH_CHECK(ctx, "dequantize_kernel");
     return 0;
 }

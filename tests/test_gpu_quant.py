@@ -125,6 +125,55 @@ def test_unaligned_pointers_take_the_scalar_path(hip_ctx):
     assert np.array_equal(got, O.quantize(x, 0.03, 128, O.U8))
 
 
+@pytest.mark.parametrize("scale", [0.045, 1.0, 0.0235, 1.9999999, 2.0 ** -60, 2.0 ** 60, 2.0 ** -61, 2.0 ** 61, -0.045, 1e-44, 3e38])
+@pytest.mark.parametrize("npdt", [np.uint8, np.int8, np.int16])
+def test_quantize_divides_exactly(hip_ctx, scale, npdt):
+    """Every float16, and float32 of any bits (NaN and infinities included) or near the middle of two codes, by scales in and out of
+    the range where the reciprocal serves: the bytes of an IEEE division, a NaN as the lowest code."""
+    rng = np.random.default_rng(31)
+    info, zp = np.iinfo(npdt), 3
+    half = np.arange(1 << 16, dtype=np.uint16).view(np.float16)
+    with np.errstate(all="ignore"):
+        near = ((rng.integers(info.min, info.max + 1, 50001) - zp + 0.5).astype(f32) * f32(scale)).view(np.int32) + rng.integers(-2, 3, 50001)
+        x = np.concatenate([rng.integers(0, 1 << 32, 300003, dtype=np.uint32), near.astype(np.int32).view(np.uint32),
+                            np.asarray([0x7f800001, 0x7fc00000, 0xff800001, 0x7f800000, 0xff800000, 0x7f7fffff, 0xff7fffff, 1, 0x80000000], np.uint32)]).view(f32)
+
+        def want(v):
+            q = v.astype(f32) / f32(scale) + f32(zp)
+            return np.rint(np.clip(np.where(np.isnan(q), info.min, q), info.min, info.max)).astype(npdt)
+        assert np.array_equal(K.quantize(half, qp(zp, scale), npdt, ctx=hip_ctx), want(half))
+        assert np.array_equal(K.quantize(x, qp(zp, scale), npdt, ctx=hip_ctx), want(x))
+
+
+@pytest.mark.parametrize("src,dst", [("f2", "u1"), ("f4", "i1"), ("f4", "i2"), ("u1", "f2"), ("i1", "f4"), ("i4", "f2")])
+def test_casts_around_a_block_at_any_address(hip_ctx, src, dst):
+    """Counts around one piece, one block and the launch that gives a thread several pieces; buffers that begin anywhere their
+    elements may; nothing written past the last element."""
+    rng = np.random.default_rng(37)
+    src, dst = np.dtype(src), np.dtype(dst)
+    code = {"f2": rt.DT_F16, "f4": rt.DT_F32, "u1": rt.DT_U8, "i1": rt.DT_I8, "i2": rt.DT_I16, "i4": rt.DT_I32}
+    piece = 8 if src.itemsize == 2 and dst.itemsize <= 2 else 4
+    several = 2 * hip_ctx.compute_units * 1024 * piece
+
+    class View:
+        def __init__(self, ptr):
+            self.ptr = ptr
+    for n in (1, piece - 1, piece + 1, 256 * piece - 1, 256 * piece, 256 * piece + 1, several - 1, several + 1, several + 5 * 1024 * piece - 3):
+        x = (rng.standard_normal(n) * 3).astype(src) if src.kind == "f" else rng.integers(0, 100, n).astype(src)
+        inside = hip_ctx.to_device(np.concatenate([np.zeros(1, src), x]))
+        out = hip_ctx.to_device(np.full(n + 2, 77, dst))
+        a, b = View(inside.ptr + src.itemsize), View(out.ptr + dst.itemsize)
+        if src.kind == "f":
+            hip_ctx.quantize(a, code[src.str[1:]], b, code[dst.str[1:]], n, qp(5, 0.0471))
+            info = np.iinfo(dst)
+            want = np.rint(np.clip(x.astype(f32) / f32(0.0471) + f32(5), info.min, info.max)).astype(dst)
+        else:
+            hip_ctx.dequantize(a, code[src.str[1:]], b, code[dst.str[1:]], n, qp(5, 0.0471))
+            want = ((x.astype(f32) - f32(5)) * f32(0.0471)).astype(dst)
+        got = out.download((n + 2,), dst)
+        assert got[0] == 77 and got[-1] == 77 and np.array_equal(got[1:-1], want), n
+
+
 def test_error_codes(hip_ctx):
     x = np.zeros(4, f32)
     with pytest.raises(rt.HipError) as e:

@@ -38,3 +38,48 @@ def test_calibration_union_and_weight_quantisation():
     q, zp, sc = quant.quantize_weights(w)
     assert (zp, sc) == O.get_quant_param(w.min(), w.max())
     assert np.array_equal(q, O.quantize(w, sc, zp, O.U8))
+
+
+def test_division_by_the_reciprocal_is_exact(tmp_path):
+    """x * r corrected once by the residual is the nearest float of x / b wherever the quotient lies so near to the middle of two floats
+    that the correction's own error (at most 1.5 * 2^-24 ulp) could matter: for a mantissa b, the a with a * 2^24 or a * 2^25 = r mod b
+    and |r| up to 6, found by the inverse of the power of two.  Every 64th b here; all of them have been held once."""
+    import subprocess
+    (tmp_path / "d.c").write_text("""
+#include <math.h>
+#include <stdint.h>
+static int64_t inverse(int64_t x, int64_t m) {
+    int64_t a = x % m, b = m, u = 1, v = 0;
+    while (b) { int64_t t = a / b, s = a - t * b; a = b; b = s; s = u - t * v; u = v; v = s; }
+    return (u % m + m) % m;
+}
+long held(int64_t first, long *tried) {
+    long bad = 0, n = 0;
+    for (int64_t b = (1 << 23) + first; b < 1 << 24; b += 64) {
+        const float fb = (float)b, y = 1.0f / fb;
+        const int t = __builtin_ctzll(b);
+        const int64_t odd = b >> t;
+        if (odd == 1 || t > 2) continue; /* (r would have to be a multiple of 8) */
+        for (int s = 24; s <= 25; s++)
+            for (int r = -6; r <= 6; r++) {
+                if (!r || (r & ((1 << t) - 1))) continue;
+                int64_t two = 1;
+                for (int i = 0; i < s - t; i++) two = two * 2 % odd;
+                for (int64_t a = (int64_t)((__int128)inverse(two, odd) * ((r >> t) + odd) % odd); a < 1 << 24; a += odd) {
+                    if (a < 1 << 23) continue;
+                    const float fa = (float)a, q0 = fa * y, q = fmaf(fmaf(-fb, q0, fa), y, q0);
+                    n++, bad += q != fa / fb;
+                }
+            }
+    }
+    *tried = n;
+    return bad;
+}
+""")
+    subprocess.check_call(["gcc", "-O2", "-mfma", "-ffp-contract=off", "-shared", "-fPIC", str(tmp_path / "d.c"), "-o", str(tmp_path / "d.so"), "-lm"])
+    import ctypes
+    fn = ctypes.CDLL(str(tmp_path / "d.so")).held
+    fn.argtypes, fn.restype = [ctypes.c_int64, ctypes.POINTER(ctypes.c_long)], ctypes.c_long
+    tried = ctypes.c_long()
+    for first in (1, 2, 63):
+        assert fn(first, ctypes.byref(tried)) == 0 and tried.value > 100000
