@@ -199,6 +199,9 @@ struct TileDesc {
     FastDiv d_cols, d_rowq;           // dwords per row of the tile; rows / E
     uint32_t wide;                    // the source tile is read in 16-byte pieces: whole ones at 16-byte addresses, or (packing) ragged rows
     FastDiv d_cols4;                  // ... of which a row has this many
+    uint32_t wide_out;                // the destination is written in 16-byte pieces
+    FastDiv d_rowp;                   // ... of which a column of the tile makes this many
+    uint32_t skew;                    // LDS row r begins (r >> skew) dwords late
     uint32_t ragged;                  // rows start at any element and end inside a dword
     uint64_t in_bytes;                // ... size of the source tensor (at least 4)
 };
@@ -287,7 +290,7 @@ template <int E, bool PACK, bool RAGGED = false> __global__ __launch_bounds__(kL
             for (int u = 0; u < UW; u++) {
                 const uint32_t idx = min(base + u * kLayoutThreads, rows * cols4 - 1);
                 const uint32_t r = fastdiv(idx, d.d_cols4), c = (idx - r * cols4) * 4;
-                at[u] = r * d.pitch + c;
+                at[u] = r * d.pitch + c + (r >> d.skew);
                 v[u] = uint4{0u, 0u, 0u, 0u};
                 if (has_source && r < vlim && x0 + c * E < d.x_extent) {
                     const uint64_t off = (plain + (uint64_t)r * d.a_plain_stride) * ES + c * 4;
@@ -321,7 +324,7 @@ template <int E, bool PACK, bool RAGGED = false> __global__ __launch_bounds__(kL
             for (int u = 0; u < UW; u++) {
                 const uint32_t idx = min(base + u * kLayoutThreads, rows * cols4 - 1);
                 const uint32_t r = fastdiv(idx, d.d_cols4), c = (idx - r * cols4) * 4;
-                at[u] = r * d.pitch + c;
+                at[u] = r * d.pitch + c + (r >> d.skew);
                 v[u] = uint4{0u, 0u, 0u, 0u};
                 if (x0 + r < d.x_extent) v[u] = *reinterpret_cast<const uint4 *>(in + (packed + two_term(d.x_packed, x0 + r)) * ES + c * 4);
             }
@@ -335,7 +338,7 @@ template <int E, bool PACK, bool RAGGED = false> __global__ __launch_bounds__(kL
         for (int u = 0; u < U; u++) {
             const uint32_t idx = min(base + u * kLayoutThreads, rows * cols - 1); // (a repeat of the last dword: the same value to the same place)
             const uint32_t r = fastdiv(idx, d.d_cols), c = idx - r * cols;
-            at[u] = r * d.pitch + c;
+            at[u] = r * d.pitch + c + (r >> d.skew);
             v[u] = 0;
             if (PACK) { // row r = lane l, column c = E coordinates of X from x0 + c * E
                 if (has_source && r < vlim && x0 + c * E < d.x_extent) {
@@ -356,8 +359,43 @@ template <int E, bool PACK, bool RAGGED = false> __global__ __launch_bounds__(kL
     }
     __syncthreads();
     // ---- out: E rows x one dword column at a time, the lanes of a wave along the destination's contiguous axis ----
-    // (packing, a lane's E dwords go to E different runs of the destination; parking the transposed tile in a second
-    // LDS area so that it leaves in address order was measured and is no quicker)
+    if (d.wide_out) {
+        constexpr int ER = 4 * E;
+        const uint32_t rowp = d.d_rowp.div;
+        for (uint32_t idx = threadIdx.x; idx < rowp * cols; idx += kLayoutThreads) {
+            const uint32_t c = fastdiv(idx, d.d_rowp), rp = idx - c * rowp;
+            uint32_t o[4][E];
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                uint32_t w[E];
+#pragma unroll
+                for (int k = 0; k < E; k++) w[k] = tile[(rp * ER + q * E + k) * d.pitch + c + ((rp * ER) >> d.skew)];
+                transpose_dwords<E>(w, o[q]);
+            }
+#pragma unroll
+            for (int j = 0; j < E; j++) {
+                uint64_t off;
+                uint32_t left; // elements of the piece that the destination has
+                if (PACK) {    // o[.][j]: lanes rp * ER .. of coordinate x0 + c * E + j
+                    const uint32_t x = x0 + c * E + j;
+                    left = x >= d.x_padded ? 0 : d.exact ? (vlim > rp * ER ? vlim - rp * ER : 0) : ER;
+                    off = (packed + two_term(d.x_packed, x)) * ES + rp * 16;
+                } else { // coordinates x0 + rp * ER .. of lane c * E + j
+                    const uint32_t l = c * E + j, x = x0 + rp * ER;
+                    left = l < vlim && x < d.x_extent ? d.x_extent - x : 0;
+                    off = (plain + (uint64_t)l * d.a_plain_stride) * ES + rp * 16;
+                }
+                if (left >= ER) {
+                    *reinterpret_cast<layout_unaligned16 *>(out + off) = layout_unaligned16{o[0][j], o[1][j], o[2][j], o[3][j]};
+                } else {
+#pragma unroll
+                    for (int q = 0; q < 4; q++)
+                        if ((uint32_t)(q * E) < left) store_bytes4<ES>(out, off + q * 4, o[q][j], (left - q * E) * ES);
+                }
+            }
+        }
+        return;
+    }
     const uint32_t rowq = d.d_rowq.div;
     for (uint32_t idx = threadIdx.x; idx < rowq * cols; idx += kLayoutThreads) {
         const uint32_t c = fastdiv(idx, d.d_rowq), rq = idx - c * rowq;
@@ -388,27 +426,40 @@ template <int E, bool PACK, bool RAGGED = false> __global__ __launch_bounds__(kL
 
 // Elements of X per tile: about 16 KiB per tile, rows of the plain tensor of 64 bytes to 2 KiB.
 // The extent is then split evenly over its tiles (3136 = 7 x 448 rather than 6 x 512 + 64).
-static uint32_t tile_stretch(uint32_t la, int es, uint32_t x_extent, bool wide, uint32_t tile_bytes = 16384) {
+static uint32_t tile_stretch(uint32_t la, int es, uint32_t x_extent, bool wide, uint32_t tile_bytes) {
     const uint32_t e = (wide ? 16 : 4) / es; // tiles begin at whole dwords (16-byte pieces) of a row
     uint32_t tx = tile_bytes / (la * es);
     tx = std::min<uint32_t>(std::max<uint32_t>(tx, 64 / es), 2048 / es) / e * e;
     const uint32_t tiles = (x_extent + tx - 1) / tx;
     return ((x_extent + tiles - 1) / tiles + e - 1) / e * e;
 }
-// The same for ragged rows, `others` tiles side by side in the other dimensions: a block takes a load, a barrier and a store in
-// turn and has nothing to hide them behind but its neighbours, so the tiles shrink to 8 and 4 KiB while the launch has fewer than
-// two blocks per compute unit (u8 NCHW -> NC/32 HW 32, tiles of 16 / 8 / 4 KiB: 155 x 75 x 75 5.8 / 4.8 / 4.3 us, 8 x 3 x 151 x 151
-// 6.1 / 5.5 / 6.3, 16 x 3 x 201 x 201 10.3 / 11.1 / 14.0).
-static uint32_t ragged_stretch(uint32_t la, int es, uint32_t x_extent, bool wide, uint64_t others, int compute_units) {
-    uint32_t tx = 0;
-    for (uint32_t bytes = 16384; bytes >= 4096; bytes /= 2) {
-        tx = tile_stretch(la, es, x_extent, wide, bytes);
-        if ((uint64_t)((x_extent + tx - 1) / tx) * others >= 2ull * compute_units) break;
-    }
+// The same with `others` tiles side by side in the other dimensions: a block takes a load, a barrier and a store in
+// turn and has nothing to hide them behind but its neighbours, so the tiles shrink to 8 and 4 KiB where the launch has few
+// blocks (tiles of 16 / 8 / 4 KiB: u8 NCHW -> NC/32 HW 32 of 155 x 75 x 75 5.8 / 4.8 / 4.3 us, f16 NCHW -> NHWC of 70 x 90 x 90 6.0 / 4.3 /
+// 4.0, f32 NHWC -> NCHW of 4 x 6 x 206 x 206, 332 blocks of 16 KiB, 5.8 / 4.6 / 5.9; bytes in whole pieces only below one block per compute unit, 6 x 36 x 160 x 160 back from 16
+// lanes, 450 blocks, 4.8 / 5.2; ragged rows gain from the third up to two blocks
+// per compute unit, u8 NCHW -> NHWC of 4 x 11 x 214 x 214 6.0 / 6.7 / 5.9).
+static uint32_t launch_stretch(uint32_t la, int es, uint32_t x_extent, bool wide, bool ragged, uint64_t others, int compute_units) {
+    auto blocks = [&](uint32_t tx) { return (x_extent + tx - 1) / tx * others; };
+    uint32_t tx = tile_stretch(la, es, x_extent, wide, 16384);
+    if (blocks(tx) < (es > 1 || ragged ? 2ull : 1ull) * compute_units) tx = tile_stretch(la, es, x_extent, wide, 8192);
+    if (blocks(tx) < (ragged ? 2ull : 1ull) * compute_units) tx = tile_stretch(la, es, x_extent, wide, 4096);
     return tx;
 }
 // Dwords per LDS row: odd, so that the E rows a lane reads and the rows of neighbouring lanes spread over the banks.
 static uint32_t tile_pitch(uint32_t cols) { return cols | 1u; }
+// Whether the tile leaves in 16-byte pieces: four times fewer stores and half the LDS reads in flight per byte are what the large
+// launches were short of (f16 NCHW -> NC/32 HW 32 of 24 x 75 x 80 x 80 13.5 -> 10.5 us, 5.0 TB/s; f32 back from NC/16 HW 16 of 124 x 201 x
+// 201 10.7 -> 8.2; f16 NHWC -> NCHW of 3 x 64 x 192 x 192 8.4 -> 6.5).  Bytes, where a thread then has sixteen rows to gather: not in
+// launches of fewer than two blocks per compute unit (3 x 6 x 155 x 155 back from 16 lanes 3.5 / 4.0), not from lanes back to rows (as quick
+// at best), and of a transpose only where its runs are whole pieces or long (9 x 93 x 165 x 165 15.7 / 17.6; 9 x 490 x 57 x 57 12.3 / 11.3).
+// Rows read at 16 * E apart would all lie in E banks: unpacking, they are skewed.
+static void set_wide_out(TileDesc &d, bool pack, uint32_t rows, int e, uint64_t blocks, int compute_units) {
+    d.wide_out = rows % (4 * e) == 0;
+    if (e == 4) d.wide_out = d.wide_out && blocks >= 2ull * compute_units && (pack ? !d.exact || d.la == 128 || d.a_extent % 16 == 0 : d.exact);
+    d.d_rowp = make_fastdiv(std::max<uint32_t>(rows / (4 * e), 1));
+    d.skew = d.wide_out && !pack && e > 1 ? (e == 4 ? 4 : 3) : 31;
+}
 // Fills the tile description for pack (plain -> packed) or unpack of `shape` by (axes, lanes); false when the layout is
 // not one the tile kernel moves (then the element-wise kernels do).
 static bool make_tile_desc(TileDesc &d, int es, int rank, const int32_t *shape, int n_axes, const int *nax, const int32_t *lanes, bool pack,
@@ -473,7 +524,7 @@ static bool make_tile_desc(TileDesc &d, int es, int rank, const int32_t *shape, 
         d.r_packed[k] = L[i] == 1 ? TwoTerm{1, sqo[i], 0} : TwoTerm{L[i], sqo[i], sql[jpos[i]]};
         blocks *= d.r_extent[k];
     }
-    d.tx = d.ragged ? ragged_stretch(la, es, d.x_padded, d.wide, blocks, compute_units) : tile_stretch(la, es, d.x_padded, d.wide);
+    d.tx = launch_stretch(la, es, d.x_padded, d.wide, d.ragged, blocks, compute_units);
     d.x_tiles = (d.x_padded + d.tx - 1) / d.tx;
     blocks *= d.x_tiles;
     if (blocks == 0 || blocks >= ((uint64_t)1 << 31)) return false;
@@ -481,8 +532,9 @@ static bool make_tile_desc(TileDesc &d, int es, int rank, const int32_t *shape, 
     d.pitch = tile_pitch(cols);
     d.d_cols = make_fastdiv(cols);
     d.d_rowq = make_fastdiv(rows / e);
+    set_wide_out(d, pack, rows, e, blocks, compute_units);
     d.d_cols4 = make_fastdiv(std::max<uint32_t>(cols / 4, 1));
-    lds = (size_t)rows * d.pitch * 4;
+    lds = (size_t)(rows * d.pitch + (rows >> d.skew)) * 4;
     return lds <= 48 * 1024;
 }
 
@@ -532,6 +584,12 @@ template <typename T> static int launch_transpose(nncase_hip_ctx *ctx, const voi
     return 0;
 }
 
+// A transpose's tiles of 128 lanes are 128 bytes of a plain row by u8, and rows that are no whole 16-byte pieces share the lines at both
+// ends with their neighbours: with twice the tile they share half as many (f16, 16 / 32 KiB: 64 x 89 x 86 x 86 to NCHW 49.5 / 35.1 us, 3 x 424
+// x 181 x 181 to NHWC 44.3 / 37.2; whole pieces 7 x 219 x 160 x 160 29.4 / 32.7).  Not of launches that it leaves some four blocks per
+// compute unit or fewer (2 x 157 x 163 x 163 11.5 / 12.1), nor of tensors that no cache holds (15 x 490 x 115 x 115, 389 MB both sides, 102.6 /
+// 116.6).
+constexpr uint64_t kTwiceTilesUpTo = 300000000; // bytes of both sides
 // [batch][rows][cols] -> [batch][cols][rows] as the tile kernel sees it.  Packing: the source is the plain tensor
 // (A = rows in groups of up to 128 lanes, X = cols), the destination the "packed" one, whose runs along A have no
 // padding.  Unpacking (short source rows): the destination is the plain tensor (A = cols, X = rows).
@@ -554,7 +612,11 @@ static bool make_transpose_desc(TileDesc &d, int es, int batch, int rows, int co
     d.x_packed = TwoTerm{1, (uint64_t)na, 0};
     d.exact = 1;
     d.wide = packing && (d.ragged ? (uint64_t)nx * es >= 64 : ((uint64_t)nx * es) % 16 == 0 && (reinterpret_cast<uintptr_t>(in) & 15u) == 0);
-    d.tx = d.ragged ? ragged_stretch(la, es, d.x_padded, d.wide, (uint64_t)d.a_groups * batch, compute_units) : tile_stretch(la, es, d.x_padded, d.wide);
+    d.tx = launch_stretch(la, es, d.x_padded, d.wide, d.ragged, (uint64_t)d.a_groups * batch, compute_units);
+    if (la == 128 && (uint64_t)nx * es % 16 != 0 && 2 * bytes < kTwiceTilesUpTo) {
+        const uint32_t twice = tile_stretch(la, es, d.x_padded, d.wide, 32768);
+        if ((uint64_t)((d.x_padded + twice - 1) / twice) * d.a_groups * batch * 10 >= 43ull * compute_units) d.tx = twice;
+    }
     d.x_tiles = (d.x_padded + d.tx - 1) / d.tx;
     d.nrest = 1;
     d.r_extent[0] = d.r_valid[0] = (uint32_t)batch;
@@ -565,8 +627,9 @@ static bool make_transpose_desc(TileDesc &d, int es, int batch, int rows, int co
     d.pitch = tile_pitch(tcols);
     d.d_cols = make_fastdiv(tcols);
     d.d_rowq = make_fastdiv(trows / e);
+    set_wide_out(d, packing, trows, e, blocks, compute_units);
     d.d_cols4 = make_fastdiv(std::max<uint32_t>(tcols / 4, 1));
-    lds = (size_t)trows * d.pitch * 4;
+    lds = (size_t)(trows * d.pitch + (trows >> d.skew)) * 4;
     return lds <= 48 * 1024;
 }
 

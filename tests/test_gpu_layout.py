@@ -147,3 +147,32 @@ def test_relayout_of_odd_extents_by_tiles(hip_ctx, shape, dtype):
     y = K.transpose_nchw_to_nhwc(x, ctx=hip_ctx)
     assert np.array_equal(y, x.transpose(0, 2, 3, 1))
     assert np.array_equal(K.transpose_nhwc_to_nchw(y, ctx=hip_ctx), x)
+
+
+@pytest.mark.parametrize("dtype", [np.uint8, np.float16, np.float32])
+@pytest.mark.parametrize("shape,lanes", [((16, 75, 80, 79), 32), ((5, 130, 81, 83), 16), ((3, 250, 118, 118), 64), ((40, 96, 44, 45), 128)])
+def test_tiles_that_leave_in_16_byte_pieces(hip_ctx, shape, lanes, dtype):
+    """Launches large enough for 16-byte stores (bytes: two blocks per compute unit) and, transposing, for tiles twice as large: last
+    lane groups, tiles and pieces that are partly filled; the surroundings of the result stay as they were."""
+    rng = np.random.default_rng(shape[1] + lanes)
+    x = rng.integers(0, 200, shape).astype(dtype)
+    src = hip_ctx.to_device(x)
+    nchw_axis = [1]
+
+    def run(call, want):
+        out = hip_ctx.to_device(np.full(want.size + 64, 77, dtype))
+
+        class Inside:
+            ptr = out.ptr + 32 * x.itemsize
+        call(Inside)
+        got = out.download((want.size + 64,), dtype)
+        assert (got[:32] == 77).all() and (got[-32:] == 77).all()
+        assert np.array_equal(got[32:-32].reshape(want.shape), want)
+    packed = O.pack(x, nchw_axis, [lanes])
+    nhwc = np.ascontiguousarray(x.transpose(0, 2, 3, 1))
+    run(lambda o: hip_ctx.pack(src, o, x.itemsize, shape, nchw_axis, [lanes]), packed)
+    run(lambda o: hip_ctx.nchw_to_nhwc(src, o, x.itemsize, *shape), nhwc)
+    src = hip_ctx.to_device(packed)
+    run(lambda o: hip_ctx.unpack(src, o, x.itemsize, shape, nchw_axis, [lanes]), x)
+    src = hip_ctx.to_device(nhwc)
+    run(lambda o: hip_ctx.nhwc_to_nchw(src, o, x.itemsize, *shape), x)
