@@ -46,6 +46,9 @@ constexpr int kRowPad = 16;       // bytes between LDS rows beyond the padded re
 // bytes of an LDS row: the reduction rounded up to whole chunks of `chunk` k-steps, and the pad
 __host__ __device__ constexpr int pair_row_bytes(int ksteps, int chunk) { return (ksteps + chunk - 1) / chunk * chunk * 64 + kRowPad; }
 
+// k-steps that an LDS row is rounded up to, of a kernel that requests kc fragments at a time
+__host__ __device__ constexpr int pair_chunk(int kc) { return kc > 8 ? 4 : kc; }
+
 struct PairArgs {
     const uint8_t *x;
     uint8_t *y1, *y2;
@@ -55,6 +58,7 @@ struct PairArgs {
     int m;                 // pixels
     int k1, n1, n2;
     int ks1, ks2, t1, t2;
+    FastDiv d_pieces;      // 16-byte pieces per LDS row of x
     int tiles_per_block;   // conv_b channel tiles per workgroup (blockIdx.y selects the range)
     int zxa, zwa, zxb, zwb; // zero points - 128
     Epilogue ep_a, ep_b;
@@ -89,11 +93,17 @@ template <int KC> struct TileLoads {
 };
 
 // Loads KC weight fragments of one tile from k-step ks0 on; past the tile's last k-step the last one is loaded again
-// (the activation tile is zero there, so what such a fragment holds does not matter, and no lane branches).
+// (the activation tile is zero there, so what such a fragment holds does not matter, and no lane branches).  Of long chunks only
+// the groups of kPairGroup that hold any of the reduction.
+constexpr int kPairGroup = 4;
 template <int KC> __device__ __forceinline__ void load_chunk(v4i (&f)[KC], const uint8_t *w, int tile, int ks0, int ksteps, int lane) {
     const v4i *src = reinterpret_cast<const v4i *>(w) + (size_t)tile * ksteps * 64 + lane;
 #pragma unroll
-    for (int c = 0; c < KC; c++) f[c] = src[min(ks0 + c, ksteps - 1) * 64];
+    for (int c0 = 0; c0 < KC; c0 += kPairGroup)
+        if (c0 == 0 || KC <= 8 || ks0 + c0 < ksteps) {
+#pragma unroll
+            for (int c = c0; c < c0 + kPairGroup && c < KC; c++) f[c] = src[min(ks0 + c, ksteps - 1) * 64];
+        }
 }
 
 template <int KC, bool FIRST>
@@ -106,71 +116,81 @@ __device__ __forceinline__ void load_tile(TileLoads<KC> &l, const PairArgs &a, i
     if (FIRST && a.rep_a.res && p < a.m && ch < a.n1) l.res = *reinterpret_cast<const uint32_t *>(a.rep_a.res + (size_t)p * a.n1 + ch);
 }
 
-// sum over k of the LDS tile's row j (every lane of pixel j gets it)
-__device__ __forceinline__ int32_t row_sum(const uint8_t *rows, int stride, int ksteps, int lane) {
-    const v4i ones = {0x01010101, 0x01010101, 0x01010101, 0x01010101};
-    const uint8_t *row = rows + (lane & 15) * stride + (lane >> 4) * 16;
-    v4i rs = {0, 0, 0, 0};
-#pragma unroll 1
-    for (int ks = 0; ks < ksteps; ks++) rs = __builtin_amdgcn_mfma_i32_16x16x64_i8(ones, *reinterpret_cast<const v4i *>(row + ks * 64), rs, 0, 0, 0);
-    return rs[0];
+// A tile's accumulators to its results: `sum` is the sum of this lane's pixel's row (the same in every lane of it).
+template <bool FIRST>
+__device__ __forceinline__ void finish_tile(const PairArgs &a, int t, const v4i &acc, int32_t sum, const v4i &bias, const v4i &ws, uint32_t rv, uint8_t *ys,
+                                            int sy, const uint8_t *lut, int lane, int p, bool store_y1) {
+    const int j = lane & 15, g = lane >> 4;
+    const int zx = FIRST ? a.zxa : a.zxb, zw = FIRST ? a.zwa : a.zwb;
+    const Epilogue &ep = FIRST ? a.ep_a : a.ep_b;
+    const int32_t kzz = (FIRST ? a.k1 : a.n1) * zx * zw;
+    const int ch = t * 16 + g * 4;
+    const int32_t nrs = -zw * sum;
+    int32_t v[4];
+#pragma unroll
+    for (int r = 0; r < 4; r++) v[r] = acc[r] + (bias[r] - zx * ws[r] + kzz) + nrs;
+    uint32_t q = requant4_u8_packed(v, ep);
+    if (lut) q = table4(lut, q);
+    if constexpr (FIRST) {
+        if (ch < a.n1) {
+            if (a.rep_a.res) q = residual4_packed(q, rv, a.rep_a);
+            *reinterpret_cast<uint32_t *>(ys + j * sy + ch) = q ^ 0x80808080u;
+            if (store_y1 && p < a.m) *reinterpret_cast<uint32_t *>(a.y1 + (size_t)p * a.n1 + ch) = q;
+        }
+    } else if (ch < a.n2 && p < a.m) {
+        if (a.deq) { // the Dequantize behind the convolution: one float per channel
+            u32x4 o;
+#pragma unroll
+            for (int r = 0; r < 4; r++) o[r] = __float_as_uint((float)((int)((q >> (8 * r)) & 0xffu) - a.deq_zero) * a.deq_scale);
+            *reinterpret_cast<u32x4 *>(reinterpret_cast<float *>(a.y2) + (size_t)p * a.n2 + ch) = o;
+        } else {
+            *reinterpret_cast<uint32_t *>(a.y2 + (size_t)p * a.n2 + ch) = q;
+        }
+    }
 }
 
 // One convolution of the pair for this wave's channel tiles first, first + step, ... below end.  `rows` is the LDS
 // activation tile ([16][stride] s8); `cur` holds the loads of the first tile already.  FIRST: results go to the LDS tile
-// `ys` as s8 (and to y1 when store_y1); else to y2.
-template <int KC, bool FIRST>
+// `ys` as s8 (and to y1 when store_y1); else to y2.  ONCE: there is one tile, and its reduction is one chunk.  The sum of a row, which
+// the weight zero point multiplies, is a second product of the same operands with ones, beside the first (by itself, before it, it
+// was 0.3 us of a launch).
+template <int KC, bool FIRST, bool ONCE>
 __device__ __forceinline__ void run_stage(const PairArgs &a, const uint8_t *rows, int stride, uint8_t *ys, int sy, const uint8_t *lut, int first,
                                           int step, int end, TileLoads<KC> &cur, int lane, int p, bool store_y1) {
     const int j = lane & 15, g = lane >> 4;
     const int ksteps = FIRST ? a.ks1 : a.ks2;
-    const int zx = FIRST ? a.zxa : a.zxb, zw = FIRST ? a.zwa : a.zwb;
-    const Epilogue &ep = FIRST ? a.ep_a : a.ep_b;
-    const int32_t nrs = -zw * row_sum(rows, stride, ksteps, lane);
-    const int32_t kzz = (FIRST ? a.k1 : a.n1) * zx * zw;
+    const v4i ones = {0x01010101, 0x01010101, 0x01010101, 0x01010101};
     const uint8_t *row = rows + j * stride + g * 16;
     v4i bias = cur.bias, ws = cur.wsum; // the constants of a tile arrive with its first chunk and are used after its last
     uint32_t rv = cur.res;
 #pragma unroll 1
-    for (int t = first; t < end; t += step) {
-        v4i acc = {0, 0, 0, 0};
+    for (int t = first; ONCE || t < end; t += step) {
+        v4i acc = {0, 0, 0, 0}, rs = {0, 0, 0, 0};
 #pragma unroll 1
-        for (int ks0 = 0; ks0 < ksteps; ks0 += KC) {
+        for (int ks0 = 0; ONCE || ks0 < ksteps; ks0 += KC) {
             // what follows this chunk (the tile's next one, else the next tile's first) travels while this one multiplies;
             // one wave-uniform branch around all of it: behind the last chunk nothing is requested, so nothing is waited for
             const bool more = ks0 + KC < ksteps;
             TileLoads<KC> nxt;
-            if (more || t + step < end) load_tile<KC, FIRST>(nxt, a, more ? t : t + step, more ? ks0 + KC : 0, lane, p);
-            if (!more) bias = cur.bias, ws = cur.wsum, rv = cur.res;
-#pragma unroll
-            for (int c = 0; c < KC; c++) {
-                const v4i xf = *reinterpret_cast<const v4i *>(row + (ks0 + c) * 64);
-                acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(cur.frag[c], xf, acc, 0, 0, 0);
+            if constexpr (!ONCE) {
+                if (more || t + step < end) load_tile<KC, FIRST>(nxt, a, more ? t : t + step, more ? ks0 + KC : 0, lane, p);
+                if (!more) bias = cur.bias, ws = cur.wsum, rv = cur.res;
             }
-            cur = nxt;
+#pragma unroll
+            for (int c0 = 0; c0 < KC; c0 += kPairGroup)
+                if (c0 == 0 || KC <= 8 || c0 < ksteps) {
+#pragma unroll
+                    for (int c = c0; c < c0 + kPairGroup && c < KC; c++) {
+                        const v4i xf = *reinterpret_cast<const v4i *>(row + (ks0 + c) * 64);
+                        acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(cur.frag[c], xf, acc, 0, 0, 0);
+                        rs = __builtin_amdgcn_mfma_i32_16x16x64_i8(ones, xf, rs, 0, 0, 0);
+                    }
+                }
+            if constexpr (ONCE) break;
+            else cur = nxt;
         }
-        const int ch = t * 16 + g * 4;
-        int32_t v[4];
-#pragma unroll
-        for (int r = 0; r < 4; r++) v[r] = acc[r] + (bias[r] - zx * ws[r] + kzz) + nrs;
-        uint32_t q = requant4_u8_packed(v, ep);
-        if (lut) q = table4(lut, q);
-        if constexpr (FIRST) {
-            if (ch < a.n1) {
-                if (a.rep_a.res) q = residual4_packed(q, rv, a.rep_a);
-                *reinterpret_cast<uint32_t *>(ys + j * sy + ch) = q ^ 0x80808080u;
-                if (store_y1 && p < a.m) *reinterpret_cast<uint32_t *>(a.y1 + (size_t)p * a.n1 + ch) = q;
-            }
-        } else if (ch < a.n2 && p < a.m) {
-            if (a.deq) { // the Dequantize behind the convolution: one float per channel
-                u32x4 o;
-#pragma unroll
-                for (int r = 0; r < 4; r++) o[r] = __float_as_uint((float)((int)((q >> (8 * r)) & 0xffu) - a.deq_zero) * a.deq_scale);
-                *reinterpret_cast<u32x4 *>(reinterpret_cast<float *>(a.y2) + (size_t)p * a.n2 + ch) = o;
-            } else {
-                *reinterpret_cast<uint32_t *>(a.y2 + (size_t)p * a.n2 + ch) = q;
-            }
-        }
+        finish_tile<FIRST>(a, t, acc, rs[0], bias, ws, rv, ys, sy, lut, lane, p, store_y1);
+        if constexpr (ONCE) break;
     }
 }
 
@@ -243,11 +263,15 @@ __device__ __forceinline__ void dw_stage(const PairArgs &a, uint8_t *xs, int sx,
 // KA / KB: weight fragments a wave requests at a time for the first / second convolution (each twice in registers).
 // MAXW: most waves a workgroup is launched with; OCC: waves per SIMD the register budget is held to.
 // DW: a 3x3 depthwise convolution produces the pixel tile (dw_stage).
-template <int KA, int KB, int MAXW, int OCC, bool DW>
+// ONCE: no wave has more than one tile of either convolution, and KA and KB hold their reductions: everything a wave will multiply is
+// requested at the start.  These launches are bound by their chain of memory round trips (us of one in a chain of them, with chunks of 8
+// k-steps and the rows' sums ahead / so: 384 -> 64 -> 384 over 14 x 14 4.64 / 4.40, 576 -> 96 -> 576 6.00 / 5.05, 960 -> 160 -> 960 over 7 x 7
+// 6.95 / 6.3; MobileNetV2 of one image 167.4 -> 159.3).
+template <int KA, int KB, int MAXW, int OCC, bool DW, bool ONCE>
 __global__ __launch_bounds__(MAXW * 64, OCC) void qpointwise_pair_kernel(const PairArgs a) {
     extern __shared__ __align__(16) uint8_t smem[];
     // rows hold whole chunks of k-steps, zero past the real reduction
-    const int sx = pair_row_bytes(a.ks1, KA), sy = pair_row_bytes(a.ks2, KB);
+    const int sx = pair_row_bytes(a.ks1, pair_chunk(KA)), sy = pair_row_bytes(a.ks2, pair_chunk(KB));
     uint8_t *xs = smem;              // [16][sx]  x - 128
     uint8_t *ys = xs + 16 * sx;      // [16][sy]  y1 - 128
     uint8_t *lut_a = ys + 16 * sy;   // 256 bytes each
@@ -273,12 +297,22 @@ __global__ __launch_bounds__(MAXW * 64, OCC) void qpointwise_pair_kernel(const P
             *reinterpret_cast<u32x4 *>(xs + r * sx + c * 16) = u32x4{0u, 0u, 0u, 0u};
         }
     } else {
+        const u32x4 none = {0x80808080u, 0x80808080u, 0x80808080u, 0x80808080u};
+        constexpr int U = KA > 4 ? 2 : 1; // (both requested before the first is waited for: 16 pixels of 960 channels are two a thread)
 #pragma unroll 1
-        for (int e = tid; e < 16 * pieces; e += threads) {
-            const int r = e / pieces, c = e - r * pieces;
-            u32x4 v = {0x80808080u, 0x80808080u, 0x80808080u, 0x80808080u};
-            if (p0 + r < a.m && c * 16 < a.k1) v = *reinterpret_cast<const u32x4 *>(a.x + (size_t)(p0 + r) * a.k1 + c * 16);
-            *reinterpret_cast<u32x4 *>(xs + r * sx + c * 16) = v ^ 0x80808080u;
+        for (int e0 = tid; e0 < 16 * pieces; e0 += U * threads) {
+            u32x4 v[U];
+            uint32_t at[U];
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                const uint32_t e = (uint32_t)(e0 + u * threads), r = fastdiv(e, a.d_pieces), c = e - r * (uint32_t)pieces;
+                at[u] = r * sx + c * 16;
+                v[u] = none;
+                if (r < 16 && p0 + (int)r < a.m && (int)c * 16 < a.k1) v[u] = *reinterpret_cast<const u32x4 *>(a.x + (size_t)(p0 + (int)r) * a.k1 + c * 16);
+            }
+#pragma unroll
+            for (int u = 0; u < U; u++)
+                if (e0 + u * threads < 16 * pieces) *reinterpret_cast<u32x4 *>(xs + at[u]) = v[u] ^ 0x80808080u;
         }
     }
     for (int e = tid; e < 4 * sy; e += threads) reinterpret_cast<uint32_t *>(ys)[e] = 0; // channels past N1 stay zero
@@ -291,10 +325,10 @@ __global__ __launch_bounds__(MAXW * 64, OCC) void qpointwise_pair_kernel(const P
     }
     __syncthreads();
     // the first convolution over the whole of its channels, into LDS (and, from the first channel range, into y1)
-    if (wave < a.t1) run_stage<KA, true>(a, xs, sx, ys, sy, a.lut_a ? lut_a : nullptr, wave, waves, a.t1, la, lane, p, blockIdx.y == 0);
+    if (wave < a.t1) run_stage<KA, true, ONCE>(a, xs, sx, ys, sy, a.lut_a ? lut_a : nullptr, wave, waves, a.t1, la, lane, p, blockIdx.y == 0);
     __syncthreads();
     // the second: this workgroup's channel tiles from the LDS tile
-    if (b_first + wave < b_end) run_stage<KB, false>(a, ys, sy, nullptr, 0, a.lut_b ? lut_b : nullptr, b_first + wave, waves, b_end, lb, lane, p, false);
+    if (b_first + wave < b_end) run_stage<KB, false, ONCE>(a, ys, sy, nullptr, 0, a.lut_b ? lut_b : nullptr, b_first + wave, waves, b_end, lb, lane, p, false);
 }
 
 // One dense 1x1 convolution over a few rows (pixels): the second stage of the pair kernel alone.  A workgroup stages 16
@@ -341,15 +375,10 @@ template <bool POOL> __global__ __launch_bounds__(kRowsWaves * 64, 3) void qpoin
     if (a.lut_b)
         for (int e = tid; e < 64; e += threads) reinterpret_cast<uint32_t *>(lut_b)[e] = a.lut_b[e];
     __syncthreads();
-    if (b_first + wave < b_end) run_stage<kRowsChunk, false>(a, ys, sy, nullptr, 0, a.lut_b ? lut_b : nullptr, b_first + wave, waves, b_end, lb, lane, p, false);
+    if (b_first + wave < b_end) run_stage<kRowsChunk, false, false>(a, ys, sy, nullptr, 0, a.lut_b ? lut_b : nullptr, b_first + wave, waves, b_end, lb, lane, p, false);
 }
 
 static bool pair_is_small(int ks1, int ks2) { return ks1 <= 4 && ks2 <= 2; }
-static size_t pair_lds_bytes(const nncase_hip_qpair *pr) {
-    const bool small = pair_is_small(pr->ks1, pr->ks2);
-    return 16 * (size_t)pair_row_bytes(pr->ks1, small ? 4 : 8) + 16 * (size_t)pair_row_bytes(pr->ks2, small ? 2 : 4) + 512;
-}
-
 // [tile][k-step][lane][16] s8 of w - 128, zero beyond the real channels / reduction
 static void pack_pair_weights(std::vector<uint8_t> &out, std::vector<int32_t> &wsum, const uint8_t *w_oihw, int n, int k, int tiles, int ksteps) {
     out.assign((size_t)tiles * ksteps * 1024, 0);
@@ -639,21 +668,24 @@ static int launch_pair(nncase_hip_ctx *ctx, const char *who, const uint8_t *x_de
     {
         // ... but no more than lets every workgroup be resident at once (a second round of workgroups doubles the
         // launch's latency chain; a wave that takes two channel tiles one after the other adds a fraction of it)
-        const int occupancy = small ? (dw ? 4 : 5) : 3; // waves per SIMD the variant is built for
+        const int occupancy = small ? 4 : 3; // waves per SIMD the variant is built for
         const int per_cu = (ptiles * ranges + ctx->compute_units - 1) / std::max(ctx->compute_units, 1);
         waves = std::max(1, std::min(waves, 4 * occupancy / std::max(per_cu, 1)));
     }
     NNHIP_HIP(ctx, hipSetDevice(ctx->device));
     const dim3 grid(ptiles, ranges), block(waves * 64);
-    const size_t lds = pair_lds_bytes(pr);
-    if (small && dw)
-        hipLaunchKernelGGL((qpointwise_pair_kernel<4, 2, 16, 4, true>), grid, block, lds, ctx->stream, a);
-    else if (small)
-        hipLaunchKernelGGL((qpointwise_pair_kernel<4, 2, 16, 5, false>), grid, block, lds, ctx->stream, a);
-    else if (dw)
-        hipLaunchKernelGGL((qpointwise_pair_kernel<8, 4, 12, 3, true>), grid, block, lds, ctx->stream, a);
-    else
-        hipLaunchKernelGGL((qpointwise_pair_kernel<8, 4, 12, 3, false>), grid, block, lds, ctx->stream, a);
+    auto go = [&](auto kernel, int ka, int kb) {
+        const int sx = pair_row_bytes(a.ks1, pair_chunk(ka)), sy = pair_row_bytes(a.ks2, pair_chunk(kb));
+        a.d_pieces = make_fastdiv((uint32_t)(sx - kRowPad) / 16);
+        hipLaunchKernelGGL(kernel, grid, block, 16 * (size_t)(sx + sy) + 512, ctx->stream, a);
+    };
+    // Everything at once where no wave has a second tile or chunk to come (with a depthwise stage only for short reductions: longer
+    // ones have that in a launch of its own).
+    const bool one_tile = a.t1 <= waves && a.tiles_per_block <= waves;
+    if (small && one_tile) dw ? go(qpointwise_pair_kernel<4, 2, 16, 4, true, true>, 4, 2) : go(qpointwise_pair_kernel<4, 2, 16, 4, false, true>, 4, 2);
+    else if (small) dw ? go(qpointwise_pair_kernel<4, 2, 16, 4, true, false>, 4, 2) : go(qpointwise_pair_kernel<4, 2, 16, 4, false, false>, 4, 2);
+    else if (one_tile && !dw && a.ks1 <= 16 && a.ks2 <= 4) go(qpointwise_pair_kernel<16, 4, 12, 3, false, true>, 16, 4);
+    else dw ? go(qpointwise_pair_kernel<8, 4, 12, 3, true, false>, 8, 4) : go(qpointwise_pair_kernel<8, 4, 12, 3, false, false>, 8, 4);
     NNHIP_LAUNCH_CHECK(ctx, "qpointwise_pair_kernel");
     return 0;
 }

@@ -144,6 +144,16 @@ def test_ragged_pairs(hip_ctx, n, k1, n1, n2, h, w, residual, lut_a, lut_b, relu
     run_pair(hip_ctx, n, k1, n1, n2, h, w, seed=n + k1 + n1 + n2 + h * w, residual=residual, lut_a=lut_a, lut_b=lut_b, relu_b=relu_b)
 
 
+ALL_AT_ONCE = [  # (in, mid, out): reductions around the groups of k-steps that a wave requests, tiles around the waves there are
+    (256, 128, 192), (272, 64, 64), (512, 68, 400), (528, 192, 192), (768, 20, 36), (784, 132, 260), (1024, 192, 64), (1024, 256, 192), (640, 196, 200),
+]
+
+
+@pytest.mark.parametrize("k1,n1,n2", ALL_AT_ONCE)
+def test_pairs_whose_weights_are_requested_at_once(hip_ctx, k1, n1, n2):
+    run_pair(hip_ctx, 1, k1, n1, n2, 5, 9, seed=k1 + n1 + n2, residual=n1 % 8 == 0, lut_b=n2 == 64)
+
+
 P1 = ((1, 1), (1, 1))
 MOBILENET_TRIPLES = [  # (channels, mid, out, in_h, in_w, depthwise stride, residual): MobileNetV2's depthwise -> projection -> expansion
     (96, 24, 144, 28, 30, 2, False), (144, 24, 144, 14, 15, 1, True), (144, 32, 192, 56, 56, 2, False), (192, 32, 192, 28, 28, 1, True),
