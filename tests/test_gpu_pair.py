@@ -309,6 +309,13 @@ def test_rows_path_of_qconv2d(hip_ctx, m, k, n, lut, deq):
     assert np.array_equal(got.view(np.uint32) if deq else got, want.reshape(m, n).view(np.uint32) if deq else want.reshape(m, n))
 
 
+@pytest.mark.parametrize("m,k,n,lut,deq", [(1, 512, 16, False, False), (1, 528, 16, True, False), (20, 1536, 20, False, True), (16, 1552, 68, False, False),
+                                           (1, 2048, 2048, False, False), (3, 448, 9200, True, False), (2, 80, 20000, False, False)])
+def test_rows_path_with_a_shared_reduction(hip_ctx, m, k, n, lut, deq):
+    """Reductions around whole chunks, one to four of them shared by waves, one to three channel tiles to a workgroup."""
+    test_rows_path_of_qconv2d(hip_ctx, m, k, n, lut, deq)
+
+
 POOLED = [  # (batch, h, w, channels, out, dequantised)
     (1, 7, 7, 1280, 1000, True), (2, 7, 7, 320, 36, False), (3, 1, 1, 64, 20, False), (1, 10, 9, 96, 132, True), (5, 3, 3, 48, 8, False),
 ]
