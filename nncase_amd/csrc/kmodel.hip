@@ -576,7 +576,7 @@ static int build_function(nncase_hip_ctx_t *ctx, Span text_span, Span rdata, nnc
             // (the conditions of nncase_hip_qglobal_avgpool_qconv2d_supported, decided here because the pooled tensor gets no buffer)
             const hipf_tensor &ty = m->tensors[ops[c].output];
             if (pointwise(ops[c]) && !skipped[c] && !block_head[c] && through[c].concat < 0 && fused_add[c] < 0 && pair_second[c] < 0 &&
-                (ty.dtype == NNCASE_HIP_DT_U8 || fused_deq[c] >= 0) && rows_shapes_ok(ops[c].p[1], ops[c].p[0], (int64_t)tp.dims[0]) &&
+                (ty.dtype == NNCASE_HIP_DT_U8 || fused_deq[c] >= 0) && pool_rows_ok(ops[c].p[1], ops[c].p[0], (int64_t)tp.dims[0]) &&
                 pool_front_pays((int)tg.dims[0], (int)(tg.dims[1] * tg.dims[2]), (int)tg.dims[3]))
                 pool_reader[k] = (int)c, pool_of[c] = (int)k;
             break;

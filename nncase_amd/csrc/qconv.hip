@@ -32,7 +32,7 @@ void nnhip::describe_conv_kernel(const nncase_hip_ctx *ctx, const nncase_hip_wei
     const int out_h = windowed_output_size(a->in_h, w->kernel_h, a->stride_h, a->dilation_h, a->pad_h_before, a->pad_h_after);
     const int out_w = windowed_output_size(a->in_w, w->kernel_w, a->stride_w, a->dilation_w, a->pad_w_before, a->pad_w_after);
     if (rows_path_taken(w, a, out_h, out_w)) {
-        snprintf(buf, cap, "qpointwise_rows%s%s", w->d_post_lut ? "+lut" : "", a->dequantize_output ? "+dequantize" : "");
+        snprintf(buf, cap, "qpointwise_rows%s%s%s", w->d_post_lut ? "+lut" : "", a->residual_dev ? "+add" : "", a->dequantize_output ? "+dequantize" : "");
         return;
     }
     const long long m = (long long)a->batch * out_h * out_w;
@@ -368,6 +368,7 @@ static int prepack_igemm(nncase_hip_ctx *ctx, nncase_hip_weights *w, const RawWe
     if (e == hipSuccess && !rc)
         e = bias ? hipMemcpyAsync(w->d_bias, bias, sizeof(int32_t) * w->out_channels, hipMemcpyHostToDevice, ctx->stream)
                  : hipMemsetAsync(w->d_bias, 0, sizeof(int32_t) * w->out_channels, ctx->stream);
+    if (e == hipSuccess && !rc && rows_wanted(w)) rc = rows_prepack(ctx, w, dev);
     const hipError_t done = hipStreamSynchronize(ctx->stream); // the host's arrays are free, the weights good on any stream
     if (temporary) (void)hipFree(raw);
     if (rc) return rc;
@@ -394,16 +395,6 @@ static int prepack(nncase_hip_ctx *ctx, const nncase_hip_conv2d_desc_t *desc, co
         rc = depthwise ? prepack_depthwise(ctx, w, weights_host, bias_host) : prepack_igemm(ctx, w, raw, bias_host);
     }
     if (rc == 0 && !depthwise && smallc_supported(w)) rc = prepack_smallc(ctx, w, weights_host);
-    if (rc == 0 && !depthwise && rows_wanted(w)) {
-        std::vector<uint8_t> transposed;
-        if (kn) { // B[K,N] row-major is a 1x1 convolution's OIHW weight [N,K,1,1] transposed
-            const int k = w->in_channels, n = w->out_channels;
-            transposed.resize((size_t)k * n);
-            for (int kk = 0; kk < k; kk++)
-                for (int j = 0; j < n; j++) transposed[(size_t)j * k + kk] = weights_host[(size_t)kk * n + j];
-        }
-        rc = rows_prepack(ctx, w, kn ? transposed.data() : weights_host, bias_host);
-    }
     if (rc) {
         free_weights(w);
         return rc;
@@ -566,7 +557,9 @@ extern "C" int nncase_hip_qglobal_avgpool_qconv2d(nncase_hip_ctx_t *ctx, const u
     }
     const int rc = check_out_dtype(ctx, a->out_dtype, a->y_qp, "qglobal_avgpool_qconv2d");
     if (rc) return rc;
-    NNHIP_REQUIRE(ctx, rows_path_taken(w, a, 1, 1), -EINVAL,
+    NNHIP_REQUIRE(ctx, !a->residual_dev && !a->out_channel_stride && !a->out_channel_offset && pool_rows_ok(w->in_channels, w->out_channels, a->batch) &&
+                           rows_path_taken(w, a, 1, 1),
+                  -EINVAL,
                   "qglobal_avgpool_qconv2d: needs a dense 1x1 convolution packed for a few pixels (expected_pixels = batch at pre-pack "
                   "time), u8 or dequantised output, no residual");
     const PoolFront pool{h * w_, x_qp};
@@ -577,5 +570,6 @@ extern "C" int nncase_hip_qglobal_avgpool_qconv2d_supported(const nncase_hip_wei
                                                             int32_t w_) {
     if (!w || !a || a->in_h != 1 || a->in_w != 1 || h <= 0 || w_ <= 0 || a->batch <= 0) return 0;
     if (!pool_front_pays(a->batch, h * w_, w->in_channels)) return 0;
+    if (a->residual_dev || a->out_channel_stride || a->out_channel_offset || !pool_rows_ok(w->in_channels, w->out_channels, a->batch)) return 0;
     return rows_path_taken(w, a, 1, 1) ? 1 : 0;
 }

@@ -140,9 +140,10 @@ struct PoolFront {
     nncase_hip_quant_param_t x_qp;
 };
 bool rows_shapes_ok(int in_channels, int out_channels, int64_t pixels);   // what rows_prepack packs and rows_path_taken takes
+bool pool_rows_ok(int in_channels, int out_channels, int64_t rows);        // ... behind a global average pool
 bool pool_front_pays(int rows, int hw, int channels);
 bool rows_wanted(const nncase_hip_weights *w);
-int rows_prepack(nncase_hip_ctx *ctx, nncase_hip_weights *w, const uint8_t *w_oihw, const int32_t *bias_host);
+int rows_prepack(nncase_hip_ctx *ctx, nncase_hip_weights *w, const RawWeights &raw_dev);
 void rows_free(nncase_hip_weights *w);
 bool rows_path_taken(const nncase_hip_weights *w, const nncase_hip_conv2d_args_t *c, int out_h, int out_w);
 int launch_qconv_rows(nncase_hip_ctx *ctx, const uint8_t *x, const nncase_hip_weights *w, void *y, const nncase_hip_conv2d_args_t *c,

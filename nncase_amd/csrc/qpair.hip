@@ -16,7 +16,7 @@
 // operand and lane (j, g) of the result holds channels 16 t + 4 g .. + 3 of pixel j: four neighbours, one dword.
 //
 // The second stage alone is the few-pixel path of nncase_hip_qconv2d (qpointwise_rows_kernel, further down): one dense
-// 1x1 convolution over at most 32 pixels, optionally behind a global average pool computed by the same launch.
+// 1x1 convolution over few pixels (rows_shapes_ok), optionally behind a global average pool computed by the same launch.
 #include "qconv.hpp"
 
 #include <new>
@@ -56,6 +56,7 @@ struct PairArgs {
     const int32_t *bias_a, *wsum_a, *bias_b, *wsum_b;
     const uint32_t *lut_a, *lut_b;
     int m;                 // pixels
+    int ldy, y_coff;       // bytes between pixels of y2, and where its channels begin (n2 and 0 but for one convolution alone)
     int k1, n1, n2;
     int ks1, ks2, t1, t2;
     FastDiv d_pieces;      // 16-byte pieces per LDS row of x
@@ -75,6 +76,7 @@ struct PairArgs {
     // float32 value of the u8 code, and its rows may be the global average of x [m][pool_hw][n1]
     int parts, part_steps; // waves that share a channel tile's reduction, and the k-steps of each (whole chunks)
     FastDiv d_tiles;       // tiles_per_block
+    ResidualEpilogue rep_b;
     int deq, deq_zero;
     float deq_scale;
     int pool_hw;
@@ -119,7 +121,8 @@ __device__ __forceinline__ void load_tile(TileLoads<KC> &l, const PairArgs &a, i
 }
 
 // A tile's accumulators to its results: `sum` is the sum of this lane's pixel's row (the same in every lane of it).
-template <bool FIRST>
+// ALONE: of one convolution by itself, which may add a residual.
+template <bool FIRST, bool ALONE = false>
 __device__ __forceinline__ void finish_tile(const PairArgs &a, int t, const v4i &acc, int32_t sum, const v4i &bias, const v4i &ws, uint32_t rv, uint8_t *ys,
                                             int sy, const uint8_t *lut, int lane, int p, bool store_y1) {
     const int j = lane & 15, g = lane >> 4;
@@ -140,13 +143,14 @@ __device__ __forceinline__ void finish_tile(const PairArgs &a, int t, const v4i 
             if (store_y1 && p < a.m) *reinterpret_cast<uint32_t *>(a.y1 + (size_t)p * a.n1 + ch) = q;
         }
     } else if (ch < a.n2 && p < a.m) {
-        if (a.deq) { // the Dequantize behind the convolution: one float per channel
+        if (ALONE && a.rep_b.res) q = residual4_packed(q, rv, a.rep_b);
+        if (ALONE && a.deq) { // the Dequantize behind the convolution: one float per channel
             u32x4 o;
 #pragma unroll
             for (int r = 0; r < 4; r++) o[r] = __float_as_uint((float)((int)((q >> (8 * r)) & 0xffu) - a.deq_zero) * a.deq_scale);
             *reinterpret_cast<u32x4 *>(reinterpret_cast<float *>(a.y2) + (size_t)p * a.n2 + ch) = o;
         } else {
-            *reinterpret_cast<uint32_t *>(a.y2 + (size_t)p * a.n2 + ch) = q;
+            *reinterpret_cast<uint32_t *>(a.y2 + (size_t)p * a.ldy + a.y_coff + ch) = q;
         }
     }
 }
@@ -355,7 +359,12 @@ template <bool POOL> __global__ __launch_bounds__(kRowsWaves * 64, 3) void qpoin
     const int first = part * a.part_steps, last = min(a.ks2, first + a.part_steps);
     const bool works = part < a.parts && tile < a.t2;
     TileLoads<kRowsChunk> cur;
-    if (works) load_tile<kRowsChunk, false>(cur, a, tile, first, lane, p);
+    uint32_t rv = 0;
+    if (works) {
+        load_tile<kRowsChunk, false>(cur, a, tile, first, lane, p);
+        const int ch = tile * 16 + (lane >> 4) * 4;
+        if (a.rep_b.res && part == 0 && p < a.m && ch < a.n2) rv = *reinterpret_cast<const uint32_t *>(a.rep_b.res + (size_t)p * a.n2 + ch);
+    }
     const int pieces = (sy - kRowPad) / 16;
     if constexpr (POOL) {
         const int quads = a.n1 >> 2;
@@ -428,7 +437,7 @@ template <bool POOL> __global__ __launch_bounds__(kRowsWaves * 64, 3) void qpoin
                 acc += accs[at], rs[0] += sums[at];
             }
     }
-    if (works && part == 0) finish_tile<false>(a, tile, acc, rs[0], bias, ws, 0u, nullptr, 0, a.lut_b ? lut_b : nullptr, lane, p, false);
+    if (works && part == 0) finish_tile<false, true>(a, tile, acc, rs[0], bias, ws, rv, nullptr, 0, a.lut_b ? lut_b : nullptr, lane, p, false);
 }
 
 static bool pair_is_small(int ks1, int ks2) { return ks1 <= 4 && ks2 <= 2; }
@@ -536,13 +545,20 @@ extern "C" int nncase_hip_qpointwise_pair_destroy(nncase_hip_ctx_t *ctx, nncase_
 namespace nnhip {
 constexpr int kRowsMaxK = 2048;                 // reduction length (an LDS row: 16 of them stay below 64 KiB)
 constexpr int64_t kRowsStreamLimit = 4 << 20;   // weight bytes all pixel tiles stream between them
-constexpr int64_t kRowsMaxPixels = 32;          // beyond two pixel tiles the tiled kernels, which share the weights of a tile
-                                                // among many pixels, are the faster ones (measured on MobileNetV2's 7x7 layers)
+constexpr int64_t kRowsMaxPixels = 32;
+// Past two pixel tiles: reductions long enough that a wave per chunk of them is a shorter chain than the tiled kernels' steps, while
+// what the tiles stream between them stays small (us, tiled / so: 49 pixels of 512 -> 512 4.1 / 3.3, 400 of them 4.2 / 3.7, 400 of 960 ->
+// 160 5.0 / 4.0, 1600 of 512 -> 128 4.2 / 3.7; shorter reductions 400 of 160 -> 960 3.8 / 3.9, 1600 of 64 -> 256 3.6 / 4.0; more to stream
+// 784 of 1024 -> 512, 26 MB, 5.0 / 5.3, 1600 of 1536 -> 256, 39 MB, 5.6 / 7.7).
+constexpr int kManyRowsMinK = 256;
+constexpr int64_t kManyRowsStreamLimit = 14000000, kManyRowsMaxPixels = 1600;
 
 bool rows_shapes_ok(int in_channels, int out_channels, int64_t pixels) {
-    return pixels > 0 && pixels <= kRowsMaxPixels && in_channels % 16 == 0 && out_channels % 4 == 0 && in_channels <= kRowsMaxK &&
-           (pixels + 15) / 16 * (int64_t)in_channels * out_channels <= kRowsStreamLimit;
+    if (pixels <= 0 || pixels > kManyRowsMaxPixels || in_channels % 16 != 0 || out_channels % 4 != 0 || in_channels > kRowsMaxK) return false;
+    const int64_t stream = (pixels + 15) / 16 * (int64_t)in_channels * out_channels;
+    return pixels <= kRowsMaxPixels ? stream <= kRowsStreamLimit : in_channels >= kManyRowsMinK && stream <= kManyRowsStreamLimit;
 }
+bool pool_rows_ok(int in_channels, int out_channels, int64_t rows) { return rows <= kRowsMaxPixels && rows_shapes_ok(in_channels, out_channels, rows); }
 
 // Every workgroup of the pooled launch pools its (up to 16) rows itself, on one compute unit: beyond this many values
 // per workgroup the separate pool kernel, which spreads over the device, is the faster one.
@@ -550,24 +566,51 @@ bool pool_front_pays(int rows, int hw, int channels) { return (int64_t)std::min(
 
 bool rows_wanted(const nncase_hip_weights *w) { return pointwise_weights(w) && rows_shapes_ok(w->in_channels, w->out_channels, w->pixels_hint); }
 
-int rows_prepack(nncase_hip_ctx *ctx, nncase_hip_weights *w, const uint8_t *w_oihw, const int32_t *bias_host) {
+// A block per channel tile: the tile's fragments as pack_pair_weights lays them out, its weight sums and its bias.
+constexpr int kRowsPackWaves = 4;
+__global__ __launch_bounds__(kRowsPackWaves * 64) void rows_pack_kernel(RawWeights raw, const int32_t *bias_in, int n, int k, int ksteps, uint8_t *dst, int32_t *wsum,
+                                                                        int32_t *bias) {
+    __shared__ int32_t sums[kRowsPackWaves][16];
+    const int t = blockIdx.x, lane = threadIdx.x & 63, wave = threadIdx.x >> 6, i = lane & 15, ch = t * 16 + i;
+    int32_t sum = 0;
+    for (int ks = wave; ks < ksteps; ks += kRowsPackWaves) {
+        const int k0 = ks * 64 + (lane >> 4) * 16;
+        u32x4 d = {0u, 0u, 0u, 0u};
+        if (ch < n && k0 < k) { // (k is whole pieces)
+#pragma unroll
+            for (int b = 0; b < 16; b++) {
+                const uint32_t v = raw.ptr[(int64_t)ch * raw.oc_stride + (int64_t)(k0 + b) * raw.ic_stride];
+                sum += (int32_t)v - 128;
+                d[b / 4] |= (v ^ 0x80u) << (8 * (b & 3));
+            }
+        }
+        *reinterpret_cast<u32x4 *>(dst + (((size_t)t * ksteps + ks) * 64 + lane) * 16) = d;
+    }
+    sum += __shfl_xor(sum, 16);
+    sum += __shfl_xor(sum, 32);
+    if (lane < 16) sums[wave][i] = sum;
+    __syncthreads();
+    if (threadIdx.x < 16) {
+        int32_t s = 0;
+        for (int w = 0; w < kRowsPackWaves; w++) s += sums[w][i];
+        wsum[ch] = s, bias[ch] = ch < n ? bias_in[ch] : 0;
+    }
+}
+
+// `raw`: the weights on the device; w->d_bias is on its way on the context's stream.
+int rows_prepack(nncase_hip_ctx *ctx, nncase_hip_weights *w, const RawWeights &raw) {
     nncase_hip_qpair *pr = new (std::nothrow) nncase_hip_qpair();
     NNHIP_REQUIRE(ctx, pr, -ENOMEM, "qconv2d_prepack: out of host memory");
     pr->second = w;
     pr->n1 = w->in_channels, pr->n2 = w->out_channels;
     pr->ks2 = (pr->n1 + 63) / 64, pr->t2 = (pr->n2 + 15) / 16;
-    std::vector<uint8_t> packed;
-    std::vector<int32_t> wsum, bias((size_t)pr->t2 * 16, 0);
-    pack_pair_weights(packed, wsum, w_oihw, pr->n2, pr->n1, pr->t2, pr->ks2);
-    if (bias_host) std::copy(bias_host, bias_host + pr->n2, bias.begin());
-    int rc = upload(ctx, (void **)&pr->d_wb, packed.data(), packed.size());
-    if (!rc) rc = upload(ctx, (void **)&pr->d_wsum_b, wsum.data(), wsum.size() * sizeof(int32_t));
-    if (!rc) rc = upload(ctx, (void **)&pr->d_bias_b, bias.data(), bias.size() * sizeof(int32_t));
-    if (rc) { // (the failing call has left its message)
-        free_pair(pr);
-        return rc;
-    }
-    w->rows_pack = pr;
+    w->rows_pack = pr; // (released with the weights, also if what follows fails)
+    NNHIP_HIP(ctx, hipMalloc((void **)&pr->d_wb, (size_t)pr->t2 * pr->ks2 * 1024));
+    NNHIP_HIP(ctx, hipMalloc((void **)&pr->d_wsum_b, (size_t)pr->t2 * 16 * sizeof(int32_t)));
+    NNHIP_HIP(ctx, hipMalloc((void **)&pr->d_bias_b, (size_t)pr->t2 * 16 * sizeof(int32_t)));
+    hipLaunchKernelGGL(rows_pack_kernel, dim3(pr->t2), dim3(kRowsPackWaves * 64), 0, ctx->stream, raw, w->d_bias, pr->n2, pr->n1, pr->ks2, pr->d_wb,
+                       pr->d_wsum_b, pr->d_bias_b);
+    NNHIP_LAUNCH_CHECK(ctx, "rows_pack_kernel");
     return 0;
 }
 
@@ -577,7 +620,11 @@ void rows_free(nncase_hip_weights *w) {
 }
 
 bool rows_path_taken(const nncase_hip_weights *w, const nncase_hip_conv2d_args_t *c, int out_h, int out_w) {
-    if (!w->rows_pack || c->residual_dev || c->out_channel_stride || c->out_channel_offset) return false;
+    if (!w->rows_pack) return false;
+    // (a pixel's channels leave as dwords: a wider tensor's have to lie at such addresses)
+    if (((c->out_channel_stride | c->out_channel_offset) & 3) != 0 || c->out_channel_offset < 0 ||
+        (c->out_channel_stride ? (int64_t)c->out_channel_offset + w->out_channels > c->out_channel_stride : c->out_channel_offset != 0))
+        return false;
     if (!(c->stride_h == 1 && c->stride_w == 1 && c->pad_h_before == 0 && c->pad_w_before == 0 && out_h == c->in_h && out_w == c->in_w)) return false;
     // (u8 codes, or their float32 values: the entry point turns the latter into a u8 call with the flag set)
     if (!(c->out_dtype == NNCASE_HIP_DT_U8 || (c->out_dtype == NNCASE_HIP_DT_F32 && c->dequantize_output != 0))) return false;
@@ -601,8 +648,12 @@ int launch_qconv_rows(nncase_hip_ctx *ctx, const uint8_t *x, const nncase_hip_we
     a.zxb = c->x_qp.zero_point - 128, a.zwb = w->zw - 128;
     const int rc = make_epilogue(ctx, &a.ep_b, c->x_qp.scale, w->sw, c->y_qp, c->clamp_min, c->clamp_max, NNCASE_HIP_DT_U8, "qconv2d");
     if (rc) return rc;
+    const int res = make_residual_epilogue(ctx, &a.rep_b, c, w);
+    if (res) return res;
+    a.ldy = c->out_channel_stride ? c->out_channel_stride : w->out_channels, a.y_coff = c->out_channel_offset;
+    NNHIP_REQUIRE(ctx, m64 * a.ldy < ((int64_t)1 << 40), -EINVAL, "qconv2d: output too large");
     if (c->dequantize_output != 0) {
-        const nncase_hip_quant_param_t last = w->d_post_lut ? w->post_lut_qp : c->y_qp;
+        const nncase_hip_quant_param_t last = c->residual_dev ? c->sum_qp : (w->d_post_lut ? w->post_lut_qp : c->y_qp);
         a.deq = 1, a.deq_zero = last.zero_point, a.deq_scale = last.scale;
     }
     if (pool) {
@@ -679,6 +730,7 @@ static int launch_pair(nncase_hip_ctx *ctx, const char *who, const uint8_t *x_de
     a.lut_a = pr->first->d_post_lut, a.lut_b = pr->second->d_post_lut;
     a.m = (int)m64;
     a.k1 = pr->k1, a.n1 = pr->n1, a.n2 = pr->n2;
+    a.ldy = a.n2;
     a.ks1 = pr->ks1, a.ks2 = pr->ks2, a.t1 = pr->t1, a.t2 = pr->t2;
     a.zxa = fa->x_qp.zero_point - 128, a.zwa = pr->first->zw - 128;
     a.zxb = sa->x_qp.zero_point - 128, a.zwb = pr->second->zw - 128;

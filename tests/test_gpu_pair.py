@@ -309,6 +309,56 @@ def test_rows_path_of_qconv2d(hip_ctx, m, k, n, lut, deq):
     assert np.array_equal(got.view(np.uint32) if deq else got, want.reshape(m, n).view(np.uint32) if deq else want.reshape(m, n))
 
 
+@pytest.mark.parametrize("n,h,w,k,c,residual,lut,deq,stride,offset", [
+    (1, 7, 7, 256, 64, True, False, False, 0, 0), (3, 3, 11, 272, 36, False, True, False, 100, 60), (1, 40, 40, 512, 128, True, True, False, 0, 0),
+    (2, 20, 20, 256, 128, False, True, False, 256, 128), (1, 5, 7, 1024, 516, True, False, True, 0, 0), (1, 17, 1, 1536, 20, True, True, False, 24, 4),
+    (8, 7, 7, 960, 160, True, False, False, 0, 0), (1, 10, 10, 2048, 256, False, False, True, 0, 0)])
+def test_rows_path_over_many_pixels(hip_ctx, n, h, w, k, c, residual, lut, deq, stride, offset):
+    """Past two pixel tiles, with what one convolution may have: a table, a residual, the Dequantize behind it, a place in the channels of
+    a wider tensor; the bytes of the oracle, and nothing around them touched."""
+    rng = np.random.default_rng(n + h + w + k + c)
+    x = rng.integers(0, 256, (n, k, h, w), dtype=np.uint8)
+    wt = rng.integers(0, 256, (c, k, 1, 1), dtype=np.uint8)
+    b = rng.integers(-3000, 3000, c).astype(np.int32)
+    zx, sx, zw, sw = 9, f32(0.0235), 131, f32(0.0041)
+    clamp, zy, sy = pick_quant(O.qconv2d(x, wt, b, zx, sx, zw, sw, out_mode=O.OUT_F32))
+    want = O.qconv2d(x, wt, b, zx, sx, zw, sw, zy, sy, fused_clamp=clamp, out_mode=O.OUT_U8)
+    zl, sl = zy, sy
+    packed = hip_ctx.prepack_conv2d(wt, b, qp(zw, sw), expected_pixels=n * h * w)
+    if lut:
+        table = rng.permutation(256).astype(np.uint8)
+        want, zl, sl = table[want], 23, f32(sy * 1.5)
+        packed.set_post_lut(table, qp(zl, sl))
+    a = conv_args(n, h, w, qp(zx, sx), qp(zy, sy), clamp)
+    keep = []
+    if residual:
+        res = rng.integers(0, 256, want.shape, dtype=np.uint8)
+        zr, sr = 101, f32(0.031)
+        _, zs, ss = pick_quant((want.astype(f32) - f32(zl)) * sl + (res.astype(f32) - f32(zr)) * sr)
+        want = O.qadd(want, res, zl, sl, zr, sr, zs, ss)
+        zl, sl = zs, ss
+        keep.append(hip_ctx.to_device(np.ascontiguousarray(res.transpose(0, 2, 3, 1))))
+        a.residual_dev, a.residual_qp, a.sum_qp = keep[0].ptr, qp(zr, sr), qp(zs, ss)
+        a.sum_clamp_min, a.sum_clamp_max = FULL
+    want = want.transpose(0, 2, 3, 1)
+    if deq:
+        a.out_dtype, a.dequantize_output = rt.DT_F32, 1
+        want = ((want.astype(np.int32) - zl).astype(f32) * sl).astype(f32)
+    a.out_channel_stride, a.out_channel_offset = stride, offset
+    ld = stride or c
+    xd = hip_ctx.to_device(np.ascontiguousarray(x.transpose(0, 2, 3, 1)))
+    yd = hip_ctx.alloc(n * h * w * ld * want.itemsize).fill(0xA5)
+    fn = rt.Function(hip_ctx)
+    fn.add_qconv2d(xd, packed, yd, a)
+    assert fn.op_kernel(0).startswith("qpointwise_rows")
+    hip_ctx.qconv2d(xd, packed, yd, a)
+    got = yd.download((n, h, w, ld), want.dtype)
+    mine = got[..., offset:offset + c]
+    assert np.array_equal(mine.view(np.uint8), np.ascontiguousarray(want).view(np.uint8).reshape(n, h, w, -1))
+    rest = np.delete(got.view(np.uint8).reshape(n, h, w, -1), np.s_[offset * want.itemsize:(offset + c) * want.itemsize], axis=3)
+    assert (rest == 0xA5).all()
+
+
 @pytest.mark.parametrize("m,k,n,lut,deq", [(1, 512, 16, False, False), (1, 528, 16, True, False), (20, 1536, 20, False, True), (16, 1552, 68, False, False),
                                            (1, 2048, 2048, False, False), (3, 448, 9200, True, False), (2, 80, 20000, False, False)])
 def test_rows_path_with_a_shared_reduction(hip_ctx, m, k, n, lut, deq):
