@@ -631,6 +631,34 @@ bool rows_path_taken(const nncase_hip_weights *w, const nncase_hip_conv2d_args_t
     return rows_shapes_ok(w->in_channels, w->out_channels, (int64_t)c->batch * out_h * out_w);
 }
 
+// Fills in how the launch is split, and launches.
+static int launch_rows(nncase_hip_ctx *ctx, PairArgs &a, bool pool) {
+    // pixel tiles x ranges of channel tiles, enough workgroups to spread the weights over the device; a wave per tile and chunk of
+    // the reduction, up to the waves there are
+    const int ptiles = (a.m + 15) / 16;
+    int ranges = (a.t2 + kRowsWaves - 1) / kRowsWaves;
+    const int want = std::max(1, 2 * ctx->compute_units / ptiles);
+    int per = std::max(1, (a.t2 + want - 1) / want); // tiles per workgroup when as many workgroups as wanted
+    if (pool) per = std::max(per, 4);                 // (every workgroup repeats the pooling)
+    per = std::min(per, kRowsWaves);
+    ranges = (a.t2 + per - 1) / per;
+    a.tiles_per_block = per;
+    const int chunks = (a.ks2 + kRowsChunk - 1) / kRowsChunk, most = std::min(chunks, kRowsWaves / per);
+    a.part_steps = (chunks + most - 1) / most * kRowsChunk;
+    a.parts = (a.ks2 + a.part_steps - 1) / a.part_steps;
+    a.d_tiles = make_fastdiv((uint32_t)per);
+    const int sy = pair_row_bytes(a.ks2, kRowsChunk);
+    a.d_pieces = make_fastdiv((uint32_t)(sy - kRowPad) / 16);
+    int waves = std::max(4, per * a.parts); // (four stage the rows in fewer trips than one)
+    if (pool) waves = kRowsWaves; // the pooling has a thread per four channels
+    const size_t lds = 16 * (size_t)sy + 256 + (size_t)(a.parts - 1) * per * kRowsShareBytes;
+    NNHIP_HIP(ctx, hipSetDevice(ctx->device));
+    if (pool) hipLaunchKernelGGL(qpointwise_rows_kernel<true>, dim3(ptiles, ranges), dim3(waves * 64), lds, ctx->stream, a);
+    else hipLaunchKernelGGL(qpointwise_rows_kernel<false>, dim3(ptiles, ranges), dim3(waves * 64), lds, ctx->stream, a);
+    NNHIP_LAUNCH_CHECK(ctx, "qpointwise_rows_kernel");
+    return 0;
+}
+
 int launch_qconv_rows(nncase_hip_ctx *ctx, const uint8_t *x, const nncase_hip_weights *w, void *y, const nncase_hip_conv2d_args_t *c,
                       const PoolFront *pool) {
     const nncase_hip_qpair *pr = w->rows_pack;
@@ -662,30 +690,7 @@ int launch_qconv_rows(nncase_hip_ctx *ctx, const uint8_t *x, const nncase_hip_we
         a.pool_zx = (float)pool->x_qp.zero_point, a.pool_sx = pool->x_qp.scale;
         a.pool_zy = (float)c->x_qp.zero_point, a.pool_sy = c->x_qp.scale;
     }
-    // pixel tiles x ranges of channel tiles, enough workgroups to spread the weights over the device; a wave per tile and chunk of
-    // the reduction, up to the waves there are
-    const int ptiles = (a.m + 15) / 16;
-    int ranges = (a.t2 + kRowsWaves - 1) / kRowsWaves;
-    const int want = std::max(1, 2 * ctx->compute_units / ptiles);
-    int per = std::max(1, (a.t2 + want - 1) / want); // tiles per workgroup when as many workgroups as wanted
-    if (pool) per = std::max(per, 4);                 // (every workgroup repeats the pooling)
-    per = std::min(per, kRowsWaves);
-    ranges = (a.t2 + per - 1) / per;
-    a.tiles_per_block = per;
-    const int chunks = (a.ks2 + kRowsChunk - 1) / kRowsChunk, most = std::min(chunks, kRowsWaves / per);
-    a.part_steps = (chunks + most - 1) / most * kRowsChunk;
-    a.parts = (a.ks2 + a.part_steps - 1) / a.part_steps;
-    a.d_tiles = make_fastdiv((uint32_t)per);
-    const int sy = pair_row_bytes(a.ks2, kRowsChunk);
-    a.d_pieces = make_fastdiv((uint32_t)(sy - kRowPad) / 16);
-    int waves = std::max(4, per * a.parts); // (four stage the rows in fewer trips than one)
-    if (pool) waves = kRowsWaves; // the pooling has a thread per four channels
-    const size_t lds = 16 * (size_t)sy + 256 + (size_t)(a.parts - 1) * per * kRowsShareBytes;
-    NNHIP_HIP(ctx, hipSetDevice(ctx->device));
-    if (pool) hipLaunchKernelGGL(qpointwise_rows_kernel<true>, dim3(ptiles, ranges), dim3(waves * 64), lds, ctx->stream, a);
-    else hipLaunchKernelGGL(qpointwise_rows_kernel<false>, dim3(ptiles, ranges), dim3(waves * 64), lds, ctx->stream, a);
-    NNHIP_LAUNCH_CHECK(ctx, "qpointwise_rows_kernel");
-    return 0;
+    return launch_rows(ctx, a, pool != nullptr);
 }
 } // namespace nnhip
 
@@ -786,6 +791,18 @@ static int launch_pair(nncase_hip_ctx *ctx, const char *who, const uint8_t *x_de
         waves = std::max(1, std::min(waves, 4 * occupancy / std::max(per_cu, 1)));
     }
     NNHIP_HIP(ctx, hipSetDevice(ctx->device));
+    // More channels between the two than a workgroup has waves: some of the waves would take two tiles of the whole reduction, and the
+    // one after the other by the kernel for one convolution is quicker (960 -> 320 -> 1280 over 7 x 7: MobileNetV2 of one image 159.1 -> 157.2
+    // us, of two at 160 x 160 156 -> 150.6).
+    if (!dw && !small && a.t1 > max_waves && a.n1 % 16 == 0) { // (whose rows are whole pieces)
+        PairArgs one = a;
+        one.ldy = a.n1, one.y2 = y1_dev, one.wb = a.wa, one.bias_b = a.bias_a, one.wsum_b = a.wsum_a, one.lut_b = a.lut_a;
+        one.n1 = a.k1, one.n2 = a.n1, one.ks2 = a.ks1, one.t2 = a.t1, one.zxb = a.zxa, one.zwb = a.zwa, one.ep_b = a.ep_a, one.rep_b = a.rep_a;
+        rc = launch_rows(ctx, one, false);
+        if (rc) return rc;
+        a.x = y1_dev;
+        return launch_rows(ctx, a, false);
+    }
     const dim3 grid(ptiles, ranges), block(waves * 64);
     auto go = [&](auto kernel, int ka, int kb) {
         const int sx = pair_row_bytes(a.ks1, pair_chunk(ka)), sy = pair_row_bytes(a.ks2, pair_chunk(kb));
