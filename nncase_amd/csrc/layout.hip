@@ -256,9 +256,10 @@ template <int E> __device__ __forceinline__ void transpose_dwords(const uint32_t
 // that are no whole dwords, so that rows begin at any element.  Their dwords (and 16-byte pieces) are read and written where
 // they lie, the last of a row in part.  us, with a thread per element and so: NCHW -> NC/32 HW 32 of 7 x 255 x 99 x 99 u8 123.8 /
 // 11.9 (floor 6.7), its unpack by 16 52.9 / 9.3.
-template <int E, bool PACK, bool RAGGED = false> __global__ __launch_bounds__(kLayoutThreads) void pack_tile_kernel(const uint8_t *in, uint8_t *out, const TileDesc d) {
+template <int E, bool PACK, bool RAGGED, bool WIDE_OUT> __global__ __launch_bounds__(kLayoutThreads) void pack_tile_kernel(const uint8_t *in, uint8_t *out, const TileDesc d) {
     extern __shared__ uint32_t tile[];
     constexpr int ES = 4 / E;
+    constexpr bool SKEWED = WIDE_OUT && !PACK && E > 1;
     // ---- which tile ----
     uint32_t b = blockIdx.x;
     const uint32_t xt = b % d.x_tiles;
@@ -290,7 +291,7 @@ template <int E, bool PACK, bool RAGGED = false> __global__ __launch_bounds__(kL
             for (int u = 0; u < UW; u++) {
                 const uint32_t idx = min(base + u * kLayoutThreads, rows * cols4 - 1);
                 const uint32_t r = fastdiv(idx, d.d_cols4), c = (idx - r * cols4) * 4;
-                at[u] = r * d.pitch + c + (r >> d.skew);
+                at[u] = r * d.pitch + c + (SKEWED ? r >> d.skew : 0);
                 v[u] = uint4{0u, 0u, 0u, 0u};
                 if (has_source && r < vlim && x0 + c * E < d.x_extent) {
                     const uint64_t off = (plain + (uint64_t)r * d.a_plain_stride) * ES + c * 4;
@@ -324,7 +325,7 @@ template <int E, bool PACK, bool RAGGED = false> __global__ __launch_bounds__(kL
             for (int u = 0; u < UW; u++) {
                 const uint32_t idx = min(base + u * kLayoutThreads, rows * cols4 - 1);
                 const uint32_t r = fastdiv(idx, d.d_cols4), c = (idx - r * cols4) * 4;
-                at[u] = r * d.pitch + c + (r >> d.skew);
+                at[u] = r * d.pitch + c + (SKEWED ? r >> d.skew : 0);
                 v[u] = uint4{0u, 0u, 0u, 0u};
                 if (x0 + r < d.x_extent) v[u] = *reinterpret_cast<const uint4 *>(in + (packed + two_term(d.x_packed, x0 + r)) * ES + c * 4);
             }
@@ -338,7 +339,7 @@ template <int E, bool PACK, bool RAGGED = false> __global__ __launch_bounds__(kL
         for (int u = 0; u < U; u++) {
             const uint32_t idx = min(base + u * kLayoutThreads, rows * cols - 1); // (a repeat of the last dword: the same value to the same place)
             const uint32_t r = fastdiv(idx, d.d_cols), c = idx - r * cols;
-            at[u] = r * d.pitch + c + (r >> d.skew);
+            at[u] = r * d.pitch + c + (SKEWED ? r >> d.skew : 0);
             v[u] = 0;
             if (PACK) { // row r = lane l, column c = E coordinates of X from x0 + c * E
                 if (has_source && r < vlim && x0 + c * E < d.x_extent) {
@@ -359,7 +360,7 @@ template <int E, bool PACK, bool RAGGED = false> __global__ __launch_bounds__(kL
     }
     __syncthreads();
     // ---- out: E rows x one dword column at a time, the lanes of a wave along the destination's contiguous axis ----
-    if (d.wide_out) {
+    if constexpr (WIDE_OUT) {
         constexpr int ER = 4 * E;
         const uint32_t rowp = d.d_rowp.div;
         for (uint32_t idx = threadIdx.x; idx < rowp * cols; idx += kLayoutThreads) {
@@ -369,7 +370,7 @@ template <int E, bool PACK, bool RAGGED = false> __global__ __launch_bounds__(kL
             for (int q = 0; q < 4; q++) {
                 uint32_t w[E];
 #pragma unroll
-                for (int k = 0; k < E; k++) w[k] = tile[(rp * ER + q * E + k) * d.pitch + c + ((rp * ER) >> d.skew)];
+                for (int k = 0; k < E; k++) w[k] = tile[(rp * ER + q * E + k) * d.pitch + c + (SKEWED ? rp : 0)];
                 transpose_dwords<E>(w, o[q]);
             }
 #pragma unroll
@@ -541,18 +542,16 @@ static bool make_tile_desc(TileDesc &d, int es, int rank, const int32_t *shape, 
 template <bool PACK> static int launch_pack_tile(nncase_hip_ctx *ctx, const void *in, void *out, int es, const TileDesc &d, uint64_t blocks, size_t lds) {
     const dim3 grid((unsigned)blocks), block(kLayoutThreads);
     if (lds > 48 * 1024) return 1; // (not asked for: the tiles are sized to stay below)
-    if (d.ragged) {
-        if (es == 4) hipLaunchKernelGGL((pack_tile_kernel<1, PACK, true>), grid, block, lds, ctx->stream, (const uint8_t *)in, (uint8_t *)out, d);
-        else if (es == 1) hipLaunchKernelGGL((pack_tile_kernel<4, PACK, true>), grid, block, lds, ctx->stream, (const uint8_t *)in, (uint8_t *)out, d);
-        else hipLaunchKernelGGL((pack_tile_kernel<2, PACK, true>), grid, block, lds, ctx->stream, (const uint8_t *)in, (uint8_t *)out, d);
-        NNHIP_LAUNCH_CHECK(ctx, "pack_tile_kernel");
-        return 0;
-    }
-    switch (es) {
-    case 1: hipLaunchKernelGGL((pack_tile_kernel<4, PACK>), grid, block, lds, ctx->stream, (const uint8_t *)in, (uint8_t *)out, d); break;
-    case 2: hipLaunchKernelGGL((pack_tile_kernel<2, PACK>), grid, block, lds, ctx->stream, (const uint8_t *)in, (uint8_t *)out, d); break;
-    default: hipLaunchKernelGGL((pack_tile_kernel<1, PACK>), grid, block, lds, ctx->stream, (const uint8_t *)in, (uint8_t *)out, d); break;
-    }
+    auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, block, lds, ctx->stream, (const uint8_t *)in, (uint8_t *)out, d); };
+    auto by_size = [&](auto ragged, auto wide) {
+        if (es == 1) go(pack_tile_kernel<4, PACK, ragged, wide>);
+        else if (es == 2) go(pack_tile_kernel<2, PACK, ragged, wide>);
+        else go(pack_tile_kernel<1, PACK, ragged, wide>);
+    };
+    const std::true_type yes;
+    const std::false_type no;
+    if (d.ragged) d.wide_out ? by_size(yes, yes) : by_size(yes, no);
+    else d.wide_out ? by_size(no, yes) : by_size(no, no);
     NNHIP_LAUNCH_CHECK(ctx, "pack_tile_kernel");
     return 0;
 }
