@@ -297,3 +297,23 @@ def test_infinite_and_very_large_logits_in_steps(hip_ctx):
             keys = big[bt[i], h // 2].reshape(-1, d)[: cl[i]].astype(np.float64)
             at = np.argmax(keys @ (q[i, h] * 60000).astype(np.float16).astype(np.float64))
             assert np.array_equal(got[i, h], vc[bt[i], h // 2].reshape(-1, d)[at].astype(np.float32))
+
+
+@pytest.mark.parametrize("b,hq,hkv,capacity,split", [(2, 16, 8, 6144, 384), (16, 64, 8, 2048, 1024)])
+def test_a_split_of_infinite_logits(hip_ctx, b, hq, hkv, capacity, split):
+    """Splits whose keys are all at -inf, the first and a later one of a context, have no weight beside the others."""
+    rng = np.random.default_rng(29)
+    d, blk = 128, 16
+    q = rng.uniform(0.5, 1, (b, hq, d)).astype(np.float16)
+    kc, vc = (rng.standard_normal((b * capacity // blk, hkv, blk, d)).astype(np.float16) for _ in range(2))
+    bt = np.arange(b * capacity // blk, dtype=np.int32).reshape(b, -1)
+    dead = kc.copy()
+    n = capacity // blk
+    dead[:split // blk] = -np.inf
+    dead[2 * n - split // blk:2 * n] = -np.inf
+    vt = K.v_cache_from_token_major(vc)
+    cl = np.full(b, capacity, np.int32)
+    got = K.paged_attention_decode(q, dead, vt, bt, cl, d ** -0.5, np.float32, ctx=hip_ctx).astype(np.float64)
+    want = O.paged_attention_decode(q.view(np.uint16), np.maximum(dead, np.float16(-60000)).view(np.uint16), vt.view(np.uint16), bt, cl, d ** -0.5)
+    # (the bound of the launches above)
+    assert (np.abs(got - want) <= 1e-5 * np.abs(want).max(axis=-1, keepdims=True)).all(), f"max err {np.abs(got - want).max()}"
