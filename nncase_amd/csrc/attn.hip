@@ -24,8 +24,9 @@
 //   that finishes last for a (sequence, kv head) - found with one atomic
 //   counter per pair, which it resets for the next call - merges the splits
 //   and writes the output, so there is a single launch per call.
-#include "attn_rules.hpp"
 #include "common.hpp"
+
+#include "attn_rules.hpp"
 
 #include <hip/hip_fp16.h>
 
@@ -46,10 +47,10 @@ constexpr float kLog2e = 1.4426950408889634f;
 // a half, and the small ones of a long run lost bits there.
 constexpr float kProbScale = 16384.f;
 
-constexpr int kAttnMaxSplits = 1024; // splits of one sequence (bounds the merge loop and the workspace)
 // Keys and values of this many bytes are not found in any cache when the next step comes back to them (the memory side's holds
 // 256 MiB): values are then read past the caches, 6.8 TB/s against 6.0 (48 sequences of up to 6000, 8 heads of 128: 135.2 -> 119.6
-// us; of 268 MB, half of it in use: 30.8 -> 33.1).  Not the keys, whose loads take 64 of a
+// us; of 268 MB, half of it in use: 30.8 -> 33.1).  By the capacity, whatever is in use of it: of 805 MB, 48 sequences of 300 / 700 /
+// 1000 / 2000 / 8192 tokens 13.3 -> 12.4, 23.4 -> 24.6, 31.2 -> 32.7, 65.3 -> 56.9, 280 -> 254.  Not the keys, whose loads take 64 of a
 // line's 128 bytes at a time: they are read twice then (133.9).
 constexpr int64_t kStreamedBytes = 512000000;
 constexpr int kStreamWaves = 4;
@@ -65,6 +66,8 @@ struct AttnArgs {
     FastDiv d_block;
     float scale_log2e;
     int out_f16;
+    AttnRunRule rule; // (this and the next of the kernel that goes through its split)
+    int rotate;       // a mask on the split: by how many pairs its blocks are moved on
 };
 // A launch that fetches weights beside its own work.  (A type of its own, and with it kernels of their own: the longer arguments and
 // the branch cost a launch 1.8 %, 8.69 -> 8.85 us at 24 x 64 x 2820 tokens.)
@@ -406,20 +409,54 @@ template <int D, int NT, int W, class Args> __global__ __launch_bounds__(W * 64,
     finish_block<D, W>(a, b, kvh, split, ns, wave, j, g, m_w, l_w, o);
 }
 
+// Tokens per split, chosen from the lengths of all sequences (at most 256): the same in every block.  `first`: the lane's sequence's.
+// (The capacity says nothing of a server's contexts, whose cache holds the longest that the model takes.  With splits by the capacity
+// 32 pairs of 1000 / 3400 tokens took 13.7 / 29.4 us in one of 16 384, and take 9.3 / 15.3; full ones 49.8 -> 50.1, 300 tokens 7.5 -> 7.7.
+// A few shapes whose lengths are spread evenly up to the capacity lost: 32 pairs of one head 34.5 -> 36.9, 48 of four 29.0 -> 31.0, where
+// the blocks without work stay a little longer and more of those with work share a compute unit.)
+__device__ __forceinline__ int run_of_launch(const AttnArgs &a, int lane, int capacity, int32_t first) {
+    uint32_t total = 0, longest = 0;
+    auto add = [&](int i, int32_t len) __attribute__((always_inline)) {
+        const uint32_t n = (uint32_t)max(min(len + a.len_offset, capacity), 0);
+        total += i < a.batch ? n : 0, longest = max(longest, n);
+    };
+    add(lane, first);
+    if (a.batch > 64) {
+        int32_t more[3];
+#pragma unroll
+        for (int k = 0; k < 3; k++) more[k] = a.ctx_lens[min(lane + 64 * (k + 1), a.batch - 1)];
+#pragma unroll
+        for (int k = 0; k < 3; k++) add(lane + 64 * (k + 1), more[k]);
+    }
+#define NNHIP_STEP(CTRL, ROWS)                                                                  \
+    total += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)total, CTRL, ROWS, 0xf, false); \
+    longest = max(longest, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)longest, CTRL, ROWS, 0xf, false));
+    NNHIP_STEP(0x111, 0xf) NNHIP_STEP(0x112, 0xf) NNHIP_STEP(0x114, 0xf) NNHIP_STEP(0x118, 0xf) // row_shr:1, 2, 4, 8
+    NNHIP_STEP(0x142, 0xa) NNHIP_STEP(0x143, 0xc)                                               // row_bcast:15, 31
+#undef NNHIP_STEP
+    return attn_run(a.rule, (uint32_t)__builtin_amdgcn_readlane((int)longest, 63), (uint32_t)__builtin_amdgcn_readlane((int)total, 63));
+}
+
 // A wave goes through its share of the split 32 tokens at a time (the block's waves in turn: a split that the context ends in is
 // shared by all of them), under a running maximum.  The next 32 keys are requested as soon as these have met the queries, the next
 // values when these have met the probabilities, so the memory is never waited for with nothing under way, and what a block does once
 // -- lengths, queries, the merge of its waves, the partials and the count -- is paid once per split instead of once per 128 to 512
 // tokens.  Bound by the memory from some 50 MB on: 48 sequences of up to 6000 tokens, 8 heads of 128, 146.7 -> 125.7 us (5.4 TB/s).
-template <int D, int W, bool NT, class Args> __global__ __launch_bounds__(W * 64, 3) void paged_attn_stream_kernel(const Args a) {
+template <int D, int W, bool NT, bool BY_LENS, class Args> __global__ __launch_bounds__(W * 64, 3) void paged_attn_stream_kernel(const Args a) {
     constexpr int KS = D / 32, DT = D / 16;
     if constexpr (std::is_same_v<Args, AttnFetchArgs>)
         if (blockIdx.z != 0) { // (a branch on an argument would put its load's trip in front of the others')
             fetch_weights<W>(a);
             return;
         }
-    const int kvh = blockIdx.x % a.hkv, b = blockIdx.x / a.hkv, split = blockIdx.y;
-    const int tok0 = split * a.split_tokens, G = a.group;
+    const int split = blockIdx.y;
+    int pair = blockIdx.x;
+    if (BY_LENS) {
+        pair += split & a.rotate;
+        if (pair >= a.batch * a.hkv) pair -= a.batch * a.hkv;
+    }
+    const int kvh = pair % a.hkv, b = pair / a.hkv;
+    const int G = a.group;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int j = lane & 15, g = lane >> 4;
     const int32_t *table = a.block_table + (size_t)b * a.max_blocks;
@@ -436,9 +473,20 @@ template <int D, int W, bool NT, class Args> __global__ __launch_bounds__(W * 64
         }
         return p;
     };
-    int tok = tok0 + wave * 32;
-    Place at = look_up(tok);
-    const int ctx = min(a.ctx_lens[b] + a.len_offset, a.max_blocks * a.block_size);
+    // Every length, the block's own and its first pages in one trip (the pages as for splits of split_tokens: right for the first
+    // split, and for all where the contexts fill the cache).
+    int32_t first_len = 0;
+    if (BY_LENS) {
+        first_len = a.ctx_lens[min(lane, a.batch - 1)];
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    int tok0 = split * a.split_tokens, run = a.split_tokens;
+    Place at = look_up(tok0 + wave * 32);
+    const int capacity = a.max_blocks * a.block_size, ctx = min(a.ctx_lens[b] + a.len_offset, capacity);
+    if (BY_LENS) {
+        __builtin_amdgcn_sched_barrier(0); // (all requested above the wait for the lengths)
+        run = run_of_launch(a, lane, capacity, first_len);
+    }
     if (ctx <= 0) { // empty context: zeros, written by the first block of the pair
         if (split == 0)
             for (int idx = threadIdx.x; idx < G * D; idx += W * 64) {
@@ -448,8 +496,13 @@ template <int D, int W, bool NT, class Args> __global__ __launch_bounds__(W * 64
             }
         return;
     }
-    if (tok0 >= ctx) return; // uniform for the block
-    const int ns = (ctx + a.split_tokens - 1) / a.split_tokens, end = min(ctx, tok0 + a.split_tokens);
+    if (split * run >= ctx) return; // uniform for the block
+    if (BY_LENS && split > 0 && run != a.split_tokens) {
+        tok0 = split * run;
+        at = look_up(tok0 + wave * 32);
+    }
+    int tok = tok0 + wave * 32;
+    const int end = min(ctx, tok0 + run);
 
     // The 32 tokens are dealt to the products so that a lane's eight of P.V, (g, e), are eight neighbours, 8 g + e: one 16-byte load of
     // values.  Row 4 g + r of the u-th logit product is token 8 g + 4 u + r, so its rows come from both tiles.
@@ -588,6 +641,7 @@ template <int D, int W, bool NT, class Args> __global__ __launch_bounds__(W * 64
     }
     float l_w = l_lane + __shfl_xor(l_lane, 16);
     l_w += __shfl_xor(l_w, 32);
+    const int ns = D == 128 ? (int)(((uint32_t)ctx + run - 1) / (uint32_t)run) : 1; // blocks of this (sequence, kv head) that get here
     finish_block<D, W>(a, b, kvh, split, ns, wave, j, g, m_w, l_w, o);
 }
 
@@ -611,7 +665,7 @@ hipError_t attn_static_scratch_address(void **ptr) { return hipGetSymbolAddress(
 struct AttnPlan {
     AttnArgs a;
     int nt = 2, waves = 8;               // of the kernel that has a block's whole share under way at once, or
-    bool stream = false, stream_values = false; // the one that goes through it
+    bool stream = false, stream_values = false, by_lens = false; // the one that goes through it
     size_t partial_bytes = 0, counter_bytes = 0;
 };
 
@@ -661,7 +715,7 @@ static int attn_plan(nncase_hip_ctx *ctx, const nncase_hip_paged_attn_args_t *p,
     }
     plan->nt = nt;
     plan->waves = waves;
-    plan->stream = plan->stream_values = false;
+    plan->stream = plan->stream_values = plan->by_lens = false;
     NNHIP_REQUIRE(ctx, a.splits <= kAttnMaxSplits, -EINVAL,
                   "paged_attention_decode: context capacity of %lld tokens exceeds %d (head_dim %d)", (long long)max_tokens,
                   kAttnMaxSplits * a.split_tokens, p->head_dim);
@@ -673,6 +727,16 @@ static int attn_plan(nncase_hip_ctx *ctx, const nncase_hip_paged_attn_args_t *p,
         if (splits <= kAttnMaxSplits && needed <= most_partial_bytes) {
             a.split_tokens = run, a.splits = (int)splits, plan->partial_bytes = needed, plan->stream = true;
             plan->stream_values = pairs * max_tokens * a.d * 4 >= kStreamedBytes;
+            // (with more pairs than compute units the capacity's run is at most 1024 tokens, and many blocks would read many lengths)
+            if (a.d == 128 && pairs <= ctx->compute_units) {
+                const int64_t room = (int64_t)std::min(most_partial_bytes / bytes(1), (size_t)kAttnMaxSplits);
+                const int64_t most = std::max(splits, std::min(attn_most_splits(pairs, max_tokens, run), room));
+                a.splits = (int)most, plan->partial_bytes = std::max(needed, bytes(most)), plan->by_lens = true;
+                a.rule = attn_run_rule(a.batch, a.hkv, ctx->compute_units, most);
+                // Splits of one sequence of few heads on all dies, where the launch's shape would put them on the same few: 32
+                // sequences of one head, one of 16 384 tokens and 31 of 400: 32.1 -> 17.7 us.
+                a.rotate = a.hkv % kXcds ? 15 : 0;
+            }
         }
     }
     a.d_block = make_fastdiv((uint32_t)p->block_size);
@@ -695,11 +759,13 @@ template <class Args> static bool attn_launch_kernel(nncase_hip_ctx *ctx, const 
     };
     if (plan.stream) {
         if (a.d == 64) {
-            if constexpr (std::is_same_v<Args, AttnArgs>) go(paged_attn_stream_kernel<64, kStreamWaves, false, Args>); // (one split)
+            if constexpr (std::is_same_v<Args, AttnArgs>) go(paged_attn_stream_kernel<64, kStreamWaves, false, false, Args>); // (one split)
         } else if (plan.stream_values) {
-            go(paged_attn_stream_kernel<128, kStreamWaves, true, Args>);
+            if (plan.by_lens) go(paged_attn_stream_kernel<128, kStreamWaves, true, true, Args>);
+            else go(paged_attn_stream_kernel<128, kStreamWaves, true, false, Args>);
         } else {
-            go(paged_attn_stream_kernel<128, kStreamWaves, false, Args>);
+            if (plan.by_lens) go(paged_attn_stream_kernel<128, kStreamWaves, false, true, Args>);
+            else go(paged_attn_stream_kernel<128, kStreamWaves, false, false, Args>);
         }
         return launched;
     }
@@ -726,12 +792,12 @@ static int attn_launch(nncase_hip_ctx *ctx, AttnPlan &plan, const void *q_dev, c
     a.part_ml = a.part_o + (size_t)a.batch * a.hq * a.splits * a.d;
     const int waves = plan.stream ? kStreamWaves : plan.waves;
     dim3 grid(a.hkv * a.batch, a.splits);
-    const int64_t own = (int64_t)grid.x * grid.y;
+    const int64_t own = (int64_t)grid.x * grid.y, busy = (int64_t)grid.x * (((int64_t)a.max_blocks * a.block_size + a.split_tokens - 1) / a.split_tokens);
     // Weights are fetched beside launches that merge splits (one that does not is over before they are here: 8 sequences of 100
     // tokens, a decode layer 25.2 -> 25.5 us) and that leave memory idle (64 sequences of 2048, 1152 blocks: 49.3 -> 49.7; 32 of
     // them, 576 blocks: 39.8 -> 39.5; one of 700, 12 blocks: 24.8 -> 22.9).
     bool launched;
-    if (fetch && fetch->count > 0 && a.splits > 1 && own <= 3 * ctx->compute_units) {
+    if (fetch && fetch->count > 0 && a.splits > 1 && busy <= 3 * ctx->compute_units) {
         AttnFetchArgs f;
         static_cast<AttnArgs &>(f) = a;
         f.fetch = *fetch;

@@ -116,3 +116,77 @@ def test_runs_are_whole_steps(choose_run):
                 run = choose_run(d, pairs, tokens, 256)
                 assert run % 128 == 0 and 0 <= run <= 2048
                 assert run == 0 or d == 128 or run >= tokens      # (64-wide heads: one split alone)
+
+
+RUNS = [256, 384, 512, 768, 1024, 1536, 2048]
+# sequences, kv heads of 128, tokens together, tokens of the longest, us with splits of RUNS tokens (evenly from 0.9 of the longest to the
+# longest, from a half of it, from an eighth, or one long one and the rest 400), in caches of two to fifty times the longest
+LENGTHS = [
+    (4, 8, 1140, 300, 8.5, 7.4, 7.4, 7.3, 7.4, 7.3, 7.4),
+    (4, 8, 3800, 1000, 9.0, 10.0, 11.0, 13.2, 13.6, 13.6, 13.6),
+    (4, 8, 12920, 3400, 16.4, 18.9, 15.1, 17.4, 19.4, 24.0, 29.3),
+    (4, 8, 30400, 8000, 30.7, 30.6, 28.7, 32.8, 26.9, 28.3, 32.7),
+    (4, 8, 49152, 16384, 50.2, 50.0, 45.7, 46.7, 43.6, 53.1, 39.3),
+    (4, 8, 65536, 16384, 57.9, 57.7, 54.4, 54.2, 51.4, 59.5, 49.7),
+    (4, 8, 36864, 16384, 44.1, 44.1, 40.0, 42.3, 38.0, 47.4, 34.0),
+    (32, 1, 30400, 1000, 8.8, 9.8, 10.7, 12.8, 13.2, 13.1, 13.2),
+    (32, 1, 103360, 3400, 17.2, 19.3, 16.0, 18.7, 20.9, 24.4, 29.3),
+    (16, 8, 15200, 1000, 17.8, 18.3, 17.0, 19.2, 19.5, 19.7, 19.7),
+    (16, 8, 30400, 2000, 29.7, 30.1, 28.5, 29.9, 27.9, 31.9, 33.5),
+    (16, 8, 65536, 4096, 56.5, 55.9, 53.6, 54.7, 52.1, 56.1, 51.4),
+    (16, 8, 10096, 4096, 18.3, 21.9, 25.4, 33.3, 30.1, 35.2, 29.2),
+    (2, 8, 1900, 1000, 8.7, 9.6, 10.5, 12.7, 13.1, 13.1, 13.1),
+    (2, 8, 6460, 3400, 12.0, 12.0, 12.2, 14.3, 16.6, 21.1, 25.9),
+    (2, 8, 15200, 8000, 20.8, 21.2, 18.7, 19.4, 22.2, 26.2, 29.9),
+    (10, 8, 9500, 1000, 13.7, 12.5, 13.9, 15.9, 16.3, 16.2, 16.2),
+    (10, 8, 19000, 2000, 21.7, 21.1, 22.8, 20.3, 21.4, 27.0, 29.7),
+    (10, 8, 6600, 3000, 14.4, 15.0, 16.4, 14.3, 16.7, 21.5, 26.5),
+    (64, 4, 60800, 1000, 25.1, 24.7, 24.8, 24.8, 22.7, 22.7, 22.7),
+    (64, 4, 121600, 2000, 51.0, 49.4, 48.0, 47.3, 47.3, 47.1, 44.5),
+    (40, 1, 76000, 2000, 14.2, 12.8, 13.8, 15.8, 17.8, 23.1, 26.0),
+]
+
+
+@pytest.fixture(scope="module")
+def run_by_lengths(tmp_path_factory):
+    d = tmp_path_factory.mktemp("lengths")
+    (d / "r.cpp").write_text("""#include "attn_rules.hpp"
+extern "C" int run_by_lengths(long batch, long kv_heads, unsigned longest, unsigned total, long most) {
+    return nnhip::attn_run(nnhip::attn_run_rule(batch, kv_heads, 256, most), longest, total);
+}
+extern "C" long most_splits(long pairs, long capacity, int run) { return nnhip::attn_most_splits(pairs, capacity, run); }
+""")
+    subprocess.check_call(["g++", "-std=c++17", "-shared", "-fPIC", "-I", CSRC, str(d / "r.cpp"), "-o", str(d / "r.so")])
+    lib = C.CDLL(str(d / "r.so"))
+    lib.run_by_lengths.argtypes = [C.c_long, C.c_long, C.c_uint, C.c_uint, C.c_long]
+    lib.most_splits.argtypes, lib.most_splits.restype = [C.c_long, C.c_long, C.c_int], C.c_long
+    return lib
+
+
+@pytest.mark.parametrize("row", LENGTHS, ids=lambda r: "%dx%d-%d-%d" % (r[0], r[1], r[3], r[2]))
+def test_splits_follow_the_lengths_not_the_capacity(run_by_lengths, row):
+    """(A run between two measured ones is held to the slower of them.)"""
+    run = run_by_lengths.run_by_lengths(row[0], row[1], row[3], row[2], 1024)
+    near = [t for r, t in zip(RUNS, row[4:]) if r == run] or [t for r, t, n in zip(RUNS, row[4:], RUNS[1:] + [0]) if r < run < n or r == min(x for x in RUNS if x > run)]
+    assert max(near) <= 1.125 * min(row[4:]), (run, near)
+
+
+def test_every_split_of_a_sequence_has_its_blocks(run_by_lengths, choose_run):
+    """Whatever the lengths: whole steps, no more splits than the launch has blocks for, and the capacity's run for full contexts."""
+    for kv_heads in (1, 2, 8, 30):
+        for batch in (1, 2, 3, 16, 33, 64, 65, 200, 256):
+            pairs = batch * kv_heads
+            if not 16 <= pairs <= 256: continue
+            for capacity in (400, 1024, 1040, 3000, 4096, 16384, 131072, 1 << 20, 1 << 21):
+                run = choose_run(128, pairs, capacity, 256)
+                if run == 0: continue
+                least = -(-capacity // run)
+                most = run_by_lengths.most_splits(pairs, capacity, run)
+                assert least <= most <= max(least, 1024)
+                assert run_by_lengths.run_by_lengths(batch, kv_heads, capacity, capacity * batch, most) == run
+                for room in {least, most}:                       # (as many as the scratch there is has room for)
+                    for longest in {1, 127, 128, 129, 383, 384, 385, 511, 513, 1023, 1025, 2047, 2049, capacity // 2 + 1, capacity - 1, capacity}:
+                        if longest > capacity: continue
+                        for total in {longest, longest + (batch - 1) * (longest // 9), longest * batch}:
+                            r = run_by_lengths.run_by_lengths(batch, kv_heads, longest, total, room)
+                            assert r > 0 and r % 128 == 0 and r * room >= longest, (batch, kv_heads, capacity, longest, total, r)

@@ -317,3 +317,49 @@ def test_a_split_of_infinite_logits(hip_ctx, b, hq, hkv, capacity, split):
     want = O.paged_attention_decode(q.view(np.uint16), np.maximum(dead, np.float16(-60000)).view(np.uint16), vt.view(np.uint16), bt, cl, d ** -0.5)
     # (the bound of the launches above)
     assert (np.abs(got - want) <= 1e-5 * np.abs(want).max(axis=-1, keepdims=True)).all(), f"max err {np.abs(got - want).max()}"
+
+
+@pytest.mark.parametrize("b,hkv,capacity,lens", [
+    (4, 8, 16384, [300]), (4, 8, 16384, [385, 1000, 0, 1]), (32, 1, 16384, [400]), (16, 8, 4096, [129, 256, 257, 0, 511]), (10, 8, 3008, [2049, 2047, 1]),
+    (70, 3, 2048, [640, 33, 0]), (256, 1, 2048, [512, 513, 64]), (130, 1, 4096, [384, 383]), (16, 3, 8192, [0]), (2, 8, 32768, [8001, 7])])
+@pytest.mark.parametrize("one_fills_it", [False, True])
+def test_contexts_shorter_than_the_cache(hip_ctx, b, hkv, capacity, lens, one_fills_it):
+    """Splits as the launch's lengths have it: short contexts in a large cache, with and without a sequence that fills it, more sequences
+    than a wave has lanes, empty ones among them and alone."""
+    rng = np.random.default_rng(b * 1000 + capacity)
+    cl = np.resize(np.asarray(lens, np.int32), b)
+    if one_fills_it: cl[b // 2] = capacity
+    d, blk, nb, hq = 128, 16, 40, hkv * 2
+    q = rng.standard_normal((b, hq, d)).astype(np.float16)
+    kc, vc = (rng.standard_normal((nb, hkv, blk, d)).astype(np.float16) for _ in range(2))
+    bt = rng.integers(0, nb, (b, capacity // blk)).astype(np.int32)
+    vt = K.v_cache_from_token_major(vc)
+    want = O.paged_attention_decode(q.view(np.uint16), kc.view(np.uint16), vt.view(np.uint16), bt, cl, d ** -0.5)
+    for _ in range(2):                                                       # (the second finds the counters as the first left them)
+        got = K.paged_attention_decode(q, kc, vt, bt, cl, d ** -0.5, np.float32, ctx=hip_ctx).astype(np.float64)
+        # (the bound of the launches above)
+        assert (np.abs(got - want) <= 1e-5 * np.abs(want).max(axis=-1, keepdims=True)).all(), f"max err {np.abs(got - want).max()}"
+
+
+@pytest.mark.parametrize("b,hkv,capacity,n", [(4, 8, 3072, 200), (16, 1, 6400, 700), (4, 8, 16384, 900)])
+def test_short_contexts_beside_a_products_weights(hip_ctx, b, hkv, capacity, n):
+    """Recorded with a product behind it (whose weights the launch brings along) and replayed as a graph: the same bits as the call alone."""
+    rng = np.random.default_rng(b + capacity)
+    d, blk, nb, hq = 128, 16, 40, hkv * 2
+    q, kc, vt = (rng.standard_normal(s).astype(np.float16) for s in ((b, hq, d), (nb, hkv, blk, d), (nb, hkv, d, blk)))
+    bt = rng.integers(0, nb, (b, capacity // blk)).astype(np.int32)
+    bufs = [hip_ctx.to_device(t) for t in (q, kc, vt, bt, np.resize(np.asarray([n, n // 2, 1], np.int32), b))]
+    out, y, alone, y_alone = (hip_ctx.alloc(x) for x in (b * hq * d * 2, b * 256 * 2, b * hq * d * 2, b * 256 * 2))
+    args = rt.PagedAttnArgs(b, hq, hkv, d, blk, capacity // blk, nb, d ** -0.5, rt.DT_F16)
+    w = hip_ctx.prepack_w8a16(rng.integers(-127, 128, (256, hq * d), dtype=np.int8), np.full(256, 1e-3, np.float32))
+    fn = rt.Function(hip_ctx)
+    fn.add_paged_attention_decode(*bufs, out, args)
+    fn.add_w8a16_gemm(out, w, y, b)
+    fn.capture()
+    hip_ctx.paged_attention_decode(*bufs, alone, args)
+    hip_ctx.w8a16_gemm(alone, w, y_alone, b)
+    want = alone.download((b, hq, d), np.uint16), y_alone.download((b, 256), np.uint16)
+    for _ in range(3):
+        fn.invoke()
+        hip_ctx.sync()
+        assert np.array_equal(out.download((b, hq, d), np.uint16), want[0]) and np.array_equal(y.download((b, 256), np.uint16), want[1])
