@@ -24,9 +24,8 @@
 //   that finishes last for a (sequence, kv head) - found with one atomic
 //   counter per pair, which it resets for the next call - merges the splits
 //   and writes the output, so there is a single launch per call.
-#include "common.hpp"
-
 #include "attn_rules.hpp"
+#include "common.hpp"
 
 #include <hip/hip_fp16.h>
 

@@ -70,6 +70,12 @@ using namespace nnhip;
 static WeightFetches weights_behind(const nncase_hip_function *fn, const Op &attn) {
     WeightFetches s;
     memset(&s, 0, sizeof(s));
+    uint32_t lanes = 0; // that have operators
+    for (const Op &op : fn->ops)
+        if (op.lane >= 0) lanes |= 1u << op.lane;
+    const nncase_hip_paged_attn_args_t &g = attn.attn;
+    const int64_t kv_bytes = (int64_t)g.batch * g.num_kv_heads * g.max_blocks_per_seq * g.block_size * g.head_dim * 4;
+    if (!fetch_beside_lanes(__builtin_popcount(lanes), g.batch, kv_bytes)) return s;
     size_t bytes = 0;
     for (size_t i = (size_t)(&attn - fn->ops.data()) + 1; i < fn->ops.size() && s.count < kMaxWeightFetches; i++) {
         const Op &op = fn->ops[i];

@@ -7,6 +7,7 @@
 #include <cstdint>
 
 #ifdef __HIPCC__
+#include <hip/hip_runtime.h>
 #define NNHIP_HOST_DEVICE __host__ __device__ __forceinline__
 #else
 #define NNHIP_HOST_DEVICE inline
@@ -52,5 +53,13 @@ NNHIP_HOST_DEVICE const char *fetch_address(const WeightFetches &s, uint32_t x, 
         u -= n;
     }
 }
+
+// Whether an attention brings weights into the caches for the products behind it where its function has lanes that run side by side:
+// another lane's products are then using the memory that the attention leaves idle, and two lanes' weights and rows do not fit the
+// caches together.  Beyond eight rows a lane it costs more than it gives, and where a lane's keys and values are some 30 MB (a decode step of 24 layers as two lanes, us a step without / with: rows a lane x context 4 x 700 753 / 731, 8 x 700
+// 793 / 790, 8 x 4096 901 / 890, 8 x 8192 963 / 998, 12 x 1500 880 / 901, 16 x 700 869 / 885, 16 x 2048 909 / 953, 16 x 4096 1037 / 1069,
+// 32 x 2048 1138 / 1180; as four lanes 8 x 700 1668 / 1643, 16 x 2048 1962 / 1992).  With one lane 1 x 700 655 / 602, 16 x 2048 817 /
+// 814, 32 x 700 895 / 886, 32 x 4096 1057 / 1068.
+inline bool fetch_beside_lanes(int lanes, int rows, int64_t kv_bytes) { return lanes <= 1 || (rows <= 8 && kv_bytes <= 25000000); }
 
 } // namespace nnhip

@@ -48,3 +48,27 @@ def test_every_fragment_once_on_its_die(lib, products):
             block = tile // (2 * off) * off + tile % off if per == 2 else tile
             assert block < blocks and block % 8 == x
     assert all(v == 1 for s in seen for v in s)
+
+
+# lanes, rows of a lane, longest context, us a decode step of 24 layers without and with the weights fetched (2 kv heads of 64)
+FETCHED = [
+    (1, 1, 700, 654.8, 602.1), (1, 1, 16000, 757.2, 726.6), (1, 8, 8192, 838.0, 827.3), (1, 16, 700, 769.9, 752.9), (1, 32, 700, 894.5, 886.2),
+    (2, 4, 700, 752.6, 730.7), (2, 4, 4096, 823.0, 806.5), (2, 6, 1500, 815.2, 806.0), (2, 8, 700, 793.0, 790.4), (2, 8, 4096, 901.4, 890.3), (2, 8, 8192, 962.8, 997.5),
+    (2, 10, 1500, 864.2, 877.3), (2, 12, 1500, 879.5, 901.2), (2, 16, 700, 869.2, 885.1), (2, 16, 2048, 909.0, 953.1), (2, 16, 4096, 1037.4, 1069.2),
+    (2, 32, 1000, 1046.8, 1066.9), (2, 32, 2048, 1138.4, 1179.8), (4, 2, 700, 1515.8, 1469.9), (4, 4, 1500, 1630.0, 1592.0), (4, 8, 700, 1667.7, 1643.2),
+    (4, 16, 2048, 1961.8, 1991.5),
+]
+
+
+@pytest.mark.parametrize("lanes,rows,tokens,without,fetched", FETCHED)
+def test_weights_are_fetched_where_that_is_the_quicker(tmp_path_factory, lanes, rows, tokens, without, fetched):
+    d = tmp_path_factory.getbasetemp() / "beside"
+    if not (d / "r.so").exists():
+        d.mkdir(exist_ok=True)
+        (d / "r.cpp").write_text("""#include "weight_fetch.hpp"
+extern "C" int beside(int lanes, int rows, long kv_bytes) { return nnhip::fetch_beside_lanes(lanes, rows, kv_bytes); }
+""")
+        subprocess.check_call(["g++", "-std=c++17", "-shared", "-fPIC", "-I", CSRC, str(d / "r.cpp"), "-o", str(d / "r.so")])
+    fn = C.CDLL(str(d / "r.so")).beside
+    fn.argtypes = [C.c_int, C.c_int, C.c_long]
+    assert bool(fn(lanes, rows, rows * 2 * tokens * 64 * 4)) == (fetched < without)
