@@ -715,7 +715,10 @@ extern "C" int nncase_hip_function_invoke(nncase_hip_function_t *fn) {
     }
     // Lanes side by side.  A graph without branches goes to its queue as one batch of packets, 50 us of the host for 122 launches; one
     // graph of both lanes of a decode step was launched node by node, 520 us of the host, and the device waited for it (32 sequences
-    // as two lanes, 245 launches: 1032 us a step as one graph, 962 as three).
+    // as two lanes, 245 launches: 1032 us a step as one graph, 962 as three).  Also where steps are enqueued one behind the other, whose
+    // host time would not show: 50 in a row as one graph / three, decode 920 / 908, MobileNetV2 at batch 64 and YOLOv5s at 16 as two lanes
+    // 432 / 435 and 739 / 743, 2 in a row 1080 / 958, 485 / 450 and 815 / 758.  (One graph where the stream is still busy, asked before
+    // each launch: 1054 for 2 in a row.)
     std::lock_guard<std::mutex> guard(ctx->lane_lock);
     hipError_t first = hipEventRecord(ctx->lane_events[0], ctx->stream);
     auto note = [&](hipError_t e) {
