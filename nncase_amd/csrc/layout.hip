@@ -455,8 +455,8 @@ static uint32_t tile_pitch(uint32_t cols) { return cols | 1u; }
 // launches of fewer than two blocks per compute unit (3 x 6 x 155 x 155 back from 16 lanes 3.5 / 4.0), not from lanes back to rows (as quick
 // at best), and of a transpose only where its runs are whole pieces or long (9 x 93 x 165 x 165 15.7 / 17.6; 9 x 490 x 57 x 57 12.3 / 11.3).
 // Rows read at 16 * E apart would all lie in E banks: unpacking, they are skewed.
-static void set_wide_out(TileDesc &d, bool pack, uint32_t rows, int e, uint64_t blocks, int compute_units) {
-    d.wide_out = rows % (4 * e) == 0;
+static void set_wide_out(TileDesc &d, bool pack, uint32_t rows, int e, uint64_t blocks, int compute_units, bool runs_pay = true) {
+    d.wide_out = runs_pay && rows % (4 * e) == 0;
     if (e == 4) d.wide_out = d.wide_out && blocks >= 2ull * compute_units && (pack ? !d.exact || d.la == 128 || d.a_extent % 16 == 0 : d.exact);
     d.d_rowp = make_fastdiv(std::max<uint32_t>(rows / (4 * e), 1));
     d.skew = d.wide_out && !pack && e > 1 ? (e == 4 ? 4 : 3) : 31;
@@ -586,9 +586,8 @@ template <typename T> static int launch_transpose(nncase_hip_ctx *ctx, const voi
 // A transpose's tiles of 128 lanes are 128 bytes of a plain row by u8, and rows that are no whole 16-byte pieces share the lines at both
 // ends with their neighbours: with twice the tile they share half as many (f16, 16 / 32 KiB: 64 x 89 x 86 x 86 to NCHW 49.5 / 35.1 us, 3 x 424
 // x 181 x 181 to NHWC 44.3 / 37.2; whole pieces 7 x 219 x 160 x 160 29.4 / 32.7).  Not of launches that it leaves some four blocks per
-// compute unit or fewer (2 x 157 x 163 x 163 11.5 / 12.1), nor of tensors that no cache holds (15 x 490 x 115 x 115, 389 MB both sides, 102.6 /
-// 116.6).
-constexpr uint64_t kTwiceTilesUpTo = 300000000; // bytes of both sides
+// compute unit or fewer (2 x 157 x 163 x 163 11.5 / 12.1), nor of tensors that no cache holds (to NHWC, u8 92 x 332 x 70 x 70, 299 MB both
+// sides, 94.4 / 107.5, f16 46 x 332 x 70 x 70 90.6 / 97.9; 130 x 382 x 51 x 51, 258 MB, 76.4 / 68.9).
 // [batch][rows][cols] -> [batch][cols][rows] as the tile kernel sees it.  Packing: the source is the plain tensor
 // (A = rows in groups of up to 128 lanes, X = cols), the destination the "packed" one, whose runs along A have no
 // padding.  Unpacking (short source rows): the destination is the plain tensor (A = cols, X = rows).
@@ -612,7 +611,7 @@ static bool make_transpose_desc(TileDesc &d, int es, int batch, int rows, int co
     d.exact = 1;
     d.wide = packing && (d.ragged ? (uint64_t)nx * es >= 64 : ((uint64_t)nx * es) % 16 == 0 && (reinterpret_cast<uintptr_t>(in) & 15u) == 0);
     d.tx = launch_stretch(la, es, d.x_padded, d.wide, d.ragged, (uint64_t)d.a_groups * batch, compute_units);
-    if (la == 128 && (uint64_t)nx * es % 16 != 0 && 2 * bytes < kTwiceTilesUpTo) {
+    if (la == 128 && (uint64_t)nx * es % 16 != 0 && 2 * bytes < kRelayoutCached) {
         const uint32_t twice = tile_stretch(la, es, d.x_padded, d.wide, 32768);
         if ((uint64_t)((d.x_padded + twice - 1) / twice) * d.a_groups * batch * 10 >= 43ull * compute_units) d.tx = twice;
     }
@@ -626,7 +625,7 @@ static bool make_transpose_desc(TileDesc &d, int es, int batch, int rows, int co
     d.pitch = tile_pitch(tcols);
     d.d_cols = make_fastdiv(tcols);
     d.d_rowq = make_fastdiv(trows / e);
-    set_wide_out(d, packing, trows, e, blocks, compute_units);
+    set_wide_out(d, packing, trows, e, blocks, compute_units, !packing || wide_runs_pay(es, (uint64_t)na, (uint64_t)nx, 2 * bytes));
     d.d_cols4 = make_fastdiv(std::max<uint32_t>(tcols / 4, 1));
     lds = (size_t)(trows * d.pitch + (trows >> d.skew)) * 4;
     return lds <= 48 * 1024;

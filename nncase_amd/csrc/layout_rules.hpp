@@ -35,4 +35,22 @@ inline bool ragged_transpose_pays(int es, int batch, int rows, int cols, int com
     return tiles32 >= (es == 1 ? 16ull : std::min(rows, cols) <= 16 ? 24ull : 32ull) * compute_units;
 }
 
+// Bytes of both sides up to which a relayout finds them in the memory side's cache of 256 MiB.
+constexpr uint64_t kRelayoutCached = 270000000;
+// Whether a relayout's runs along A (na elements, nx of them per image) leave in 16-byte pieces (true) or in dwords.  Within the cache
+// they do: float16 1 to 22 % quicker, bytes up to 47.  Past it, where the lines that neighbouring tiles share meet in the memory itself,
+// it goes either way by the shape, and the dwords' time is seldom far above the pieces', while the pieces' is up to a quarter above the
+// dwords': pieces where that was so of whole classes, us dwords / pieces, [na x nx] of 360 to 800 MB:
+//   * bytes, short rows of whole pieces: 32 x 784 195 / 172, 128 x 625 117 / 103, 256 x 3136 152 / 147; not long ones (3136 x 256 159 /
+//     169, 784 x 512 271 / 281, 256 x 12 544 143 / 146) nor ragged ones (489 x 1936 155 / 189, 253 x 2025 114 / 131, 254 x 3025 188 / 200; but
+//     397 x 6084 178 / 158 and 174 x 900 208 / 186)
+//   * float16 but for short ragged rows: 5184 x 96 267 / 246, 199 x 2500 274 / 259, 397 x 6084 1.8 % quicker; 87 x 7225 139 / 172, 111 x
+//     784 133 / 158, 254 x 3025 142 / 160.
+inline bool wide_runs_pay(int es, uint64_t na, uint64_t nx, uint64_t both_bytes) {
+    if (both_bytes < kRelayoutCached || es == 4) return true;
+    const bool whole = na * es % 16 == 0;
+    if (es == 1) return whole && na <= 576 && (na < 128 || nx < 8000);
+    return whole || na > 300;
+}
+
 } // namespace nnhip
