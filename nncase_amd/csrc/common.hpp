@@ -12,6 +12,7 @@
 #include <mutex>
 
 #include "../../include/nncase_hip.h"
+#include "once_per_kernel.hpp"
 #include "weight_fetch.hpp"
 
 struct nncase_hip_ctx {
@@ -56,6 +57,11 @@ namespace nnhip {
 // Device address of the static scratch array of the attention entry point that allocates nothing, on `device`
 // (which must be current).  attn.hip, where the array lives.
 hipError_t attn_static_scratch_address(void **ptr);
+
+// Asks for a dynamic LDS limit of `limit` bytes, always the same for one kernel (a call slow next to a launch: once per kernel and device).
+template <auto Kernel> hipError_t raise_dynamic_lds(int device, int limit) {
+    return once_per_kernel<Kernel>(device, [&] { return hipFuncSetAttribute(reinterpret_cast<const void *>(Kernel), hipFuncAttributeMaxDynamicSharedMemorySize, limit); });
+}
 
 // hostcall.hip: device scratch of at least `bytes`, valid until the next call (`*temporary`: larger than what a context
 // keeps, the caller gives it back with hipFree when the stream has drained); what a context holds for host calls.

@@ -16,7 +16,6 @@
 #include <hip/hip_fp16.h>
 
 #include <cmath>
-#include <mutex>
 #include <type_traits>
 #include <new>
 #include <vector>
@@ -967,16 +966,6 @@ extern "C" int nncase_hip_w8a16_prepack(nncase_hip_ctx_t *ctx, const int8_t *w_h
     return 0;
 }
 
-// A launch whose LDS (the dynamic part plus the kernel's own static arrays: `total`) passes 48 KiB asks, once per kernel
-// and device, for a dynamic limit of `limit` bytes.
-template <typename KernelT> static hipError_t raise_dynamic_lds(KernelT kernel, int device, size_t total, int limit) {
-    if (total <= 48 * 1024) return hipSuccess;
-    static std::once_flag raised[16];
-    hipError_t e = hipSuccess;
-    std::call_once(raised[device & 15], [&] { e = hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, limit); });
-    return e;
-}
-
 // Whether a product of m rows and `tiles` tiles (pairs) over at most kRowsMaxK is computed with a tile's reduction split over a
 // block's waves.  The sum's order depends on it, so it is asked for the rows' count and the matrix alone: the product, the one that
 // normalises its rows and the one that rotates them agree bit for bit.  A block per tile repeats the rows' trip (and their
@@ -1030,7 +1019,7 @@ static GemmForm gemm_form(const nncase_hip_ctx_t *ctx, const nncase_hip_w8a16_t 
 template <int G, int KS, bool NORM, int R = 1, int PIECES = 1, bool ROPE = false>
 static int launch_tile(nncase_hip_ctx_t *ctx, const GemmArgs &a, int tiles) {
     const size_t lds = NORM ? (size_t)16 * rows_in_lds_pitch(a.k) : 0;
-    NNHIP_HIP(ctx, raise_dynamic_lds(w8a16_tile_kernel<G, KS, NORM, R, PIECES, ROPE>, ctx->device, lds + G * kGemmWaves * 1024, 96 * 1024));
+    if (lds + G * kGemmWaves * 1024 > 48 * 1024) NNHIP_HIP(ctx, (raise_dynamic_lds<w8a16_tile_kernel<G, KS, NORM, R, PIECES, ROPE>>(ctx->device, 96 * 1024)));
     hipLaunchKernelGGL((w8a16_tile_kernel<G, KS, NORM, R, PIECES, ROPE>), dim3(tiles, (a.m + 15) / 16), dim3(kGemmThreads), lds, ctx->stream, a);
     NNHIP_LAUNCH_CHECK(ctx, "w8a16_tile_kernel");
     return 0;
@@ -1109,7 +1098,7 @@ static int launch_w8a16_gemm(nncase_hip_ctx_t *ctx, const void *a_dev, const nnc
         // vocabulary head needs for occupancy -- 50.7 against 43.9 us when it still ran as 1187 one-group blocks)
 #define NNHIP_ROWS_LAUNCH_KB(MTV, GV, KBV, PV)                                                                                 \
     do {                                                                                                                       \
-        NNHIP_HIP(ctx, raise_dynamic_lds(w8a16_gemm_rows_in_lds_kernel<MTV, GV, KBV, PV>, ctx->device, rows_lds + 1024, 128 * 1024)); \
+        if (rows_lds > 47 * 1024) NNHIP_HIP(ctx, (raise_dynamic_lds<w8a16_gemm_rows_in_lds_kernel<MTV, GV, KBV, PV>>(ctx->device, 128 * 1024))); \
         hipLaunchKernelGGL((w8a16_gemm_rows_in_lds_kernel<MTV, GV, KBV, PV>), rgrid, rblock, rows_lds, ctx->stream, a); \
     } while (0)
 #define NNHIP_ROWS_LAUNCH(MTV, GV)                                                                                             \

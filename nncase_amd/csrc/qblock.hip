@@ -384,13 +384,7 @@ __global__ __launch_bounds__(NW * 64) void qblock_kernel(const BlockArgs a) {
 }
 
 template <int S, int TPT, int NW> static int launch_block_inst(nncase_hip_ctx *ctx, const BlockArgs &a, int blocks, size_t lds) {
-    // the dynamic LDS limit of a kernel is raised once per device (the attribute call is slow next to a launch)
-    static int raised_on_device = -1;
-    if (lds > 48 * 1024 && raised_on_device != ctx->device) {
-        NNHIP_HIP(ctx, hipFuncSetAttribute(reinterpret_cast<const void *>(&qblock_kernel<S, TPT, NW>),
-                                           hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
-        raised_on_device = ctx->device;
-    }
+    if (lds > 48 * 1024) NNHIP_HIP(ctx, (raise_dynamic_lds<qblock_kernel<S, TPT, NW>>(ctx->device, 160 * 1024)));
     hipLaunchKernelGGL((qblock_kernel<S, TPT, NW>), dim3(blocks), dim3(NW * 64), lds, ctx->stream, a);
     NNHIP_LAUNCH_CHECK(ctx, "qblock_kernel");
     return 0;

@@ -346,14 +346,7 @@ TilePlan plan_tile(const IgemmArgs &a, int pix, int tb, int threads, int nchunks
 }
 
 template <int T, int RG, int WM, int WN, bool FAST> int launch_tile_f(nncase_hip_ctx *ctx, const IgemmArgs &args, const TilePlan &plan, int nchunks) {
-    if (plan.lds > 65536) {
-        static std::once_flag raised[16];
-        hipError_t attr = hipSuccess;
-        std::call_once(raised[ctx->device & 15], [&] {
-            attr = hipFuncSetAttribute(reinterpret_cast<const void *>(&qconv_tile_kernel<T, RG, WM, WN, FAST>), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
-        });
-        NNHIP_HIP(ctx, attr);
-    }
+    if (plan.lds > 65536) NNHIP_HIP(ctx, (raise_dynamic_lds<qconv_tile_kernel<T, RG, WM, WN, FAST>>(ctx->device, 160 * 1024)));
     hipLaunchKernelGGL((qconv_tile_kernel<T, RG, WM, WN, FAST>), dim3(ceil_div(args.num_mtiles, 8) * 8 * nchunks), dim3(WM * WN * 64), plan.lds, ctx->stream, args,
                        plan.t);
     NNHIP_LAUNCH_CHECK(ctx, "qconv_tile_kernel");

@@ -30,7 +30,6 @@
 #include "qconv_igemm.hpp"
 #include "qconv_rules.hpp"
 
-#include <mutex>
 #include <type_traits>
 
 namespace nnhip {
@@ -720,12 +719,8 @@ template <int T, int RG, int WM, int WN, int LM> int launch_wide4_t(nncase_hip_c
     args.num_mtiles = ceil_div(a.m, PIX);
     const WideGrid grid = wide_grid(ctx, args.num_mtiles, nchunks);
     const size_t lds = (size_t)TB * 16 * sizeof(int32_t) + 256 + PIX * sizeof(int32_t) + (size_t)4 * (PIX * 64 + TB * 1024);
-    static std::once_flag raised[16]; // more than 64 KiB of dynamic LDS has to be asked for once per kernel and device
-    hipError_t attr = hipSuccess;
-    std::call_once(raised[ctx->device & 15], [&] {
-        attr = hipFuncSetAttribute(reinterpret_cast<const void *>(&qconv_wide4_kernel<T, RG, WM, WN, LM>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-    });
-    NNHIP_HIP(ctx, attr);
+    // more than 64 KiB of dynamic LDS has to be asked for
+    NNHIP_HIP(ctx, (raise_dynamic_lds<qconv_wide4_kernel<T, RG, WM, WN, LM>>(ctx->device, (int)lds)));
     hipLaunchKernelGGL((qconv_wide4_kernel<T, RG, WM, WN, LM>), dim3(grid.per * 8), dim3(WM * WN * 64), lds, ctx->stream, args, grid);
     NNHIP_LAUNCH_CHECK(ctx, "qconv_wide4_kernel");
     return 0;
@@ -1048,12 +1043,8 @@ template <int T, int RG, int WM, int WN, int LM> int launch_wide_dma_t(nncase_hi
     args.num_mtiles = ceil_div(a.m, PIX);
     const WideGrid grid = wide_grid(ctx, args.num_mtiles, nchunks);
     const size_t lds = (size_t)4 * TB * 1024 + (size_t)3 * PIX * 128;
-    static std::once_flag raised[16]; // more than 64 KiB of dynamic LDS has to be asked for once per kernel and device
-    hipError_t attr = hipSuccess;
-    std::call_once(raised[ctx->device & 15], [&] {
-        attr = hipFuncSetAttribute(reinterpret_cast<const void *>(&qconv_wide_dma_kernel<T, RG, WM, WN, LM>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-    });
-    NNHIP_HIP(ctx, attr);
+    // more than 64 KiB of dynamic LDS has to be asked for
+    NNHIP_HIP(ctx, (raise_dynamic_lds<qconv_wide_dma_kernel<T, RG, WM, WN, LM>>(ctx->device, (int)lds)));
     hipLaunchKernelGGL((qconv_wide_dma_kernel<T, RG, WM, WN, LM>), dim3(grid.per * 8), dim3(WM * WN * 64), lds, ctx->stream, args, grid);
     NNHIP_LAUNCH_CHECK(ctx, "qconv_wide_dma_kernel");
     return 0;
@@ -1065,14 +1056,8 @@ template <int T, int RG, int WM, int WN, int LM, int KG = 1> int launch_wide_t(n
     args.num_mtiles = ceil_div(a.m, PIX);
     const WideGrid grid = wide_grid(ctx, args.num_mtiles, nchunks);
     const size_t lds = (size_t)TB * 16 * sizeof(int32_t) + 256 + PIX * sizeof(int32_t) + (size_t)KG * kWideSlots * (PIX * 64 + TB * 1024);
-    if (lds > 65536) { // more than 64 KiB of dynamic LDS has to be asked for once per kernel and device
-        static std::once_flag raised[16];
-        hipError_t attr = hipSuccess;
-        std::call_once(raised[ctx->device & 15], [&] {
-            attr = hipFuncSetAttribute(reinterpret_cast<const void *>(&qconv_wide_kernel<T, RG, WM, WN, LM, KG>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-        });
-        NNHIP_HIP(ctx, attr);
-    }
+    // more than 64 KiB of dynamic LDS has to be asked for
+    if (lds > 65536) NNHIP_HIP(ctx, (raise_dynamic_lds<qconv_wide_kernel<T, RG, WM, WN, LM, KG>>(ctx->device, (int)lds)));
     hipLaunchKernelGGL((qconv_wide_kernel<T, RG, WM, WN, LM, KG>), dim3(grid.per * 8), dim3(WM * WN * KG * 64), lds, ctx->stream, args, grid);
     NNHIP_LAUNCH_CHECK(ctx, "qconv_wide_kernel");
     return 0;
