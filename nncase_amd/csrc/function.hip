@@ -244,6 +244,7 @@ static int push(nncase_hip_function *fn, const Op &op) {
     drop_graph(fn); // a captured graph no longer matches the list
     fn->ops.push_back(op);
     fn->ops.back().lane = fn->cur_lane;
+    fn->nlanes = std::max(fn->nlanes, fn->cur_lane + 1); // (with the operator: a lane that is only chosen leaves the captured graphs as they are)
     return 0;
 }
 
@@ -252,7 +253,6 @@ extern "C" int nncase_hip_function_set_lane(nncase_hip_function_t *fn, int32_t l
     NNHIP_REQUIRE(fn->ctx, lane == NNCASE_HIP_LANE_JOINED || (lane >= 0 && lane < NNCASE_HIP_MAX_LANES), -EINVAL,
                   "function_set_lane: lane %d (0..%d, or NNCASE_HIP_LANE_JOINED)", lane, NNCASE_HIP_MAX_LANES - 1);
     fn->cur_lane = lane;
-    if (lane + 1 > fn->nlanes) fn->nlanes = lane + 1;
     return 0;
 }
 

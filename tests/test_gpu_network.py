@@ -420,3 +420,20 @@ def test_lanes_are_forked_and_joined_on_every_replay(hip_ctx, lanes):
             want[lane] += 20 * (lane + 1)
         if replay % 2:                                    # (two replays in flight)
             assert np.array_equal(x.download((8, n), np.int32), want)
+
+
+def test_a_lane_chosen_after_the_capture_leaves_it_as_it_is():
+    """A lane becomes one of the function's with its first operator: chosen by itself, behind a capture and in a context that has no
+    streams for lanes yet, it changes nothing of the replay."""
+    ctx = rt.Context(0)
+    a, b = ctx.alloc(64), ctx.alloc(64)
+    a.upload(np.arange(64, dtype=np.uint8))
+    fn = rt.Function(ctx)
+    fn.add_lut_u8(a, b, 64, ((np.arange(256) + 3) % 256).astype(np.uint8))
+    fn.capture()
+    for lane in (1, 3, rt.Function.LANE_JOINED, 0):
+        fn.set_lane(lane)
+        b.fill(0)
+        fn.invoke()
+        assert np.array_equal(b.download((64,), np.uint8), np.arange(64, dtype=np.uint8) + 3), f"lane {lane}"
+    ctx.close()
