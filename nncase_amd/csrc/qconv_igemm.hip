@@ -184,8 +184,16 @@ static bool igemm_is_pointwise(const nncase_hip_weights *w, const nncase_hip_con
            out_h == c->in_h && out_w == c->in_w;
 }
 
+// Strided 1x1 windows packed for the DMA kernel: it moves whole pixels, wherever they lie (the plan, which does not know the stride, has
+// counted on its blocks' heights).  us, with 8 tiles / by the window's taps in blocks of 256 x 256 / so: 16 000 pixels 640 -> 512 14.9 / 19.2 /
+// 12.5, 2048 of 4096 -> 4096 55.8 / 63.5 / 41.0, 15 488 of 2240 -> 364 28.7 / 41.9 / 25.0, 12 288 of 1536 -> 1024 - / 32.9 / 26.2.
+static bool igemm_rows_apart(const nncase_hip_weights *w, const nncase_hip_conv2d_args_t *c, int out_h, int out_w) {
+    return w->wide == 1 && w->tiles == 16 && w->kernel_h == 1 && w->kernel_w == 1 && !igemm_is_pointwise(w, c, out_h, out_w) && c->pad_h_before == 0 &&
+           c->pad_w_before == 0 && (int64_t)(out_h - 1) * c->stride_h < c->in_h && (int64_t)(out_w - 1) * c->stride_w < c->in_w;
+}
+
 int igemm_load_mode(const nncase_hip_weights *w, const nncase_hip_conv2d_args_t *c, int out_h, int out_w) {
-    const bool pointwise = igemm_is_pointwise(w, c, out_h, out_w);
+    const bool pointwise = igemm_is_pointwise(w, c, out_h, out_w) || igemm_rows_apart(w, c, out_h, out_w);
     if (w->g_ic % 16 == 0) return pointwise ? kRows16 : kVec16;
     if (w->g_ic % 8 != 0) return kVec4;
     // (the row loader reads 16 bytes at a time: the tensor has to hold that many)
@@ -260,6 +268,7 @@ int launch_qconv_igemm(nncase_hip_ctx *ctx, const uint8_t *x, const nncase_hip_w
         a.deq = 1, a.deq_zero = last.zero_point, a.deq_scale = last.scale;
     }
     const int mode = igemm_load_mode(w, c, out_h, out_w);
+    a.apart = igemm_rows_apart(w, c, out_h, out_w);
 
     const TilePlan tile = w->ragged ? TilePlan{} : plan_qconv_tile(ctx, a, w->tiles, w->nchunks);
     const size_t group_bytes = (size_t)w->nchunks * w->ksteps * w->tiles * 1024;
@@ -277,7 +286,7 @@ int launch_qconv_igemm(nncase_hip_ctx *ctx, const uint8_t *x, const nncase_hip_w
             continue;
         }
         if (w->ragged) {
-            const bool rows = igemm_is_pointwise(w, c, out_h, out_w);
+            const bool rows = a.apart || igemm_is_pointwise(w, c, out_h, out_w);
             rc = w->wide == 2 ? launch_wide_small_ragged(ctx, a, rows, w->small_shape, w->nchunks) : launch_wide_ragged(ctx, a, rows, w->tiles, w->nchunks);
             if (rc) return rc;
             continue;

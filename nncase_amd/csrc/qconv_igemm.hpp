@@ -69,6 +69,7 @@ struct IgemmArgs {
     int g_ic;              // channels per tap in the packed reduction
     int in_h, in_w;
     int kh, kw, stride_h, stride_w, dil_h, dil_w, pad_h, pad_w;
+    int apart;             // contiguous reduction rows that are not neighbours: the pixels of a strided 1x1 window (DMA kernel only)
     FastDiv d_ohow, d_ow, d_kw, d_gic;
     int zxp, zwp;          // zx - 128, zw - 128
     int zwp_rows;          // zwp where the kernel still owes -zwp * (sum of x') per pixel, 0 where the weights carry it

@@ -844,7 +844,12 @@ __global__ __launch_bounds__(WM * WN * 64, WM * WN >= 8 ? 2 : 1) void qconv_wide
         const int pl = (wave * NA + i) * 8 + (lane >> 3);                 // pixel of the block
         const int p = min(mt * PIX + pl, a.m - 1);                         // (a pixel past the end repeats the last one: not stored)
         const int piece = ((lane & 7) - pl) & 7;
-        a_voff[i] = (uint32_t)p * (uint32_t)a.ldx + (uint32_t)a.x_coff + piece * 16;
+        uint32_t row = (uint32_t)p;
+        if (a.apart) { // (uniform)
+            const PixInfo pi = pix_info<kVec16>(a, p);
+            row = (uint32_t)(pi.base + pi.iy0 * a.in_w + pi.ix0);
+        }
+        a_voff[i] = row * (uint32_t)a.ldx + (uint32_t)a.x_coff + piece * 16;
     }
     auto dma_a = [&](int stage /* byte offset in the activation ring */, int pair, auto first, auto count) __attribute__((always_inline)) {
         const int pc = min(pair, (KS - 1) >> 1);
@@ -1095,18 +1100,23 @@ template <int LM> int launch_wide_dma(nncase_hip_ctx *ctx, const IgemmArgs &a, i
     }
 }
 
-// Block shapes: tiles = 16 -> 256 pixels x 256 channels (4 x 2 waves; rows that arrive by DMA also 192 and 128); tiles = 8 -> 256 or 128 pixels x 128 channels.
+// Block shapes: tiles = 16 -> 256 pixels x 256 channels (4 x 2 waves; rows that arrive by DMA also 192 and 128, padded 1x1 windows 128); tiles = 8 -> 256 or 128 pixels x 128 channels.
 template <int LM> int launch_wide_lm(nncase_hip_ctx *ctx, const IgemmArgs &a, int tiles, int nchunks) {
+    // What the plan gave 16 tiles for the DMA kernel's lower blocks, and padding keeps from it (4096 pixels 4096 -> 2048 1x1: 62.7 us in
+    // blocks of 256 x 256, 51.5 so, 54.0 with 8 tiles)
+    [[maybe_unused]] const bool few = 2ll * ceil_div(a.m, 256) * nchunks <= ctx->compute_units;
     if constexpr (LM == kWideRagRows) {
         // (planned for rows of whole dwords: a piece then starts at a dword, wherever its 16 bytes lie; what runs over the end of a
         // row meets surplus weights and is in the sums of x as well)
         if (tiles == 16)
             return a.k % 64 == 0 ? launch_wide_dma<kWideRowsFull>(ctx, a, nchunks) : launch_wide_dma<kWideRows>(ctx, a, nchunks);
     } else if constexpr (LM == kWideRagWindow) {
-        if (tiles == 16) return launch_wide_t<8, 4, 4, 2, LM>(ctx, a, nchunks);
+        if (tiles == 16) return few ? launch_wide_t<8, 4, 2, 2, LM>(ctx, a, nchunks) : launch_wide_t<8, 4, 4, 2, LM>(ctx, a, nchunks);
     } else if (tiles == 16) {
         if constexpr (LM == kWideRowsFull || LM == kWideRows) {
             if (a.x_bytes < ((size_t)1 << 31)) return launch_wide_dma<LM>(ctx, a, nchunks);
+        } else if (few) {
+            return launch_wide_t<8, 4, 2, 2, LM>(ctx, a, nchunks);
         }
         return launch_wide4_t<8, 4, 4, 2, LM>(ctx, a, nchunks);
     }

@@ -897,3 +897,31 @@ def test_matmul_in_blocks_of_128_192_and_256_rows(hip_ctx, m, k, n):
     x[-1] = 255                                                # (the row that the last block repeats)
     want = ((x.astype(np.float64) - 3) @ (w.astype(np.float64) - 250)).astype(np.int32)     # exact: below 2^53
     assert np.array_equal(K.mat_mul(x, w, qp(3, 0.02), qp(250, 0.011), None, np.int32, None, ctx=hip_ctx), want)
+
+
+@pytest.mark.parametrize("n,h,w,k,oc,stride,pad,groups", [
+    (2, 63, 63, 1088, 4090, (2, 2), (0, 0), 1),    # blocks of 128 pixels, an odd number of k-steps, channels that end inside a chunk
+    (1, 143, 144, 1060, 2047, (2, 2), (0, 0), 1),  # 192, a reduction that ends inside a k-step, no multiple of 16
+    (3, 130, 127, 512, 1026, (3, 1), (0, 0), 2),   # 256, lines left out, two groups
+    (1, 127, 130, 1040, 4096, (3, 3), (0, 2), 1),  # padding behind the last pixel only, which no window reaches
+    (2, 63, 63, 1088, 4090, (2, 2), (1, 1), 1),    # padding that the windows do reach: by their taps, in blocks of 256 pixels
+    (2, 62, 62, 1088, 4090, (2, 2), (1, 1), 1),    # ... of 128
+    (2, 62, 62, 1092, 4090, (2, 2), (1, 1), 1),
+])
+def test_strided_pointwise_layers_packed_for_the_dma_kernel(hip_ctx, n, h, w, k, oc, stride, pad, groups):
+    """1x1 windows with a stride, in the layers whose plan counts on blocks fed by DMA: every pixel's row from where it lies."""
+    rng = np.random.default_rng(h + oc)
+    x, wt = rng.integers(0, 256, (n, k * groups, h, w), dtype=np.uint8), rng.integers(0, 256, (oc, k, 1, 1), dtype=np.uint8)
+    oh, ow = ((s + sum(pad) - 1) // t + 1 for s, t in zip((h, w), stride))
+    shifted = np.zeros((n, k * groups, h + sum(pad), w + sum(pad)), np.float32)   # (padding is the input's zero point)
+    shifted[:, :, pad[0]:pad[0] + h, pad[0]:pad[0] + w] = x.astype(np.float32) - 3
+    rows = shifted[:, :, ::stride[0], ::stride[1]].transpose(0, 2, 3, 1).reshape(-1, groups, k)
+    want = np.concatenate([rows[:, g].astype(np.float64) @ (wt[g * oc // groups:(g + 1) * oc // groups, :, 0, 0].astype(np.float64) - 250).T
+                           for g in range(groups)], axis=1).astype(np.int32)      # exact: below 2^53
+    got = K.conv2d(x, wt, None, stride, (pad, pad), (1, 1), groups, FULL, qp(3, 0.02), qp(250, 0.011), None, np.int32, ctx=hip_ctx)
+    assert got.shape == (n, oc, oh, ow) and np.array_equal(got.transpose(0, 2, 3, 1).reshape(-1, oc), want)
+    fn, buf = rt.Function(hip_ctx), hip_ctx.alloc(16)          # (never invoked: which kernel it would be)
+    fn.add_qconv2d(buf, hip_ctx.prepack_conv2d(wt, None, qp(250, 0.011), groups, expected_pixels=n * oh * ow), buf,
+                   rt.Conv2dArgs(n, h, w, *stride, 1, 1, *pad, *pad, qp(3, 0.02), qp(0, 1.0), *FULL, rt.DT_I32))
+    lies_in_the_image = pad[0] == 0 and (oh - 1) * stride[0] < h and (ow - 1) * stride[1] < w
+    assert "T=16" in fn.op_kernel(0) and (k % 16 != 0 or ("rows16" in fn.op_kernel(0)) == lies_in_the_image)
