@@ -797,7 +797,7 @@ extern "C" int nncase_hip_function_op_kernel(nncase_hip_function_t *fn, int32_t 
     case Op::kConv: describe_conv_kernel(fn->ctx, op.weights, &op.conv, name, capacity); break;
     case Op::kBlock: nncase_hip_qblock_describe(op.block, &op.blk, name, capacity); break;
     case Op::kPoolConv: snprintf(name, capacity, "qglobal_avgpool+qpointwise_rows%s", op.conv.dequantize_output ? "+dequantize" : ""); break;
-    case Op::kPair: snprintf(name, capacity, op.weights ? "dw3x3+qpointwise_pair_kernel" : "qpointwise_pair_kernel"); break;
+    case Op::kPair: describe_pair(fn->ctx, op.pair, &op.conv, op.weights != nullptr, name, capacity); break;
     case Op::kAdd: snprintf(name, capacity, "qadd"); break;
     case Op::kPool: snprintf(name, capacity, "qglobal_avgpool"); break;
     case Op::kLut: snprintf(name, capacity, "lut_u8"); break;

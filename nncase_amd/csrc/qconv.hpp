@@ -135,6 +135,7 @@ int launch_qconv_depthwise(nncase_hip_ctx *ctx, const uint8_t *x, const nncase_h
 
 // The few-pixel path of a dense 1x1 convolution (qpair.hip): packing at pre-pack time, whether a call takes it, the launch
 // (pool != nullptr: x is [batch, pool_hw, channels] and the convolution reads its global average, requantised to c->x_qp).
+void describe_pair(const nncase_hip_ctx *ctx, const nncase_hip_qpair *pair, const nncase_hip_conv2d_args_t *first, bool dw, char *buf, size_t cap);
 struct PoolFront {
     int hw;
     nncase_hip_quant_param_t x_qp;

@@ -84,6 +84,40 @@ inline bool dma_pays(int64_t rows, int n, int ksteps, int compute_units) {
     return choose_dma_rows(rows, nchunks, ksteps, compute_units).us < 4 + 2.0 * (double)rows * n * ksteps * 64 / 1.05e9;
 }
 
+// How a pair of dense 1x1 convolutions (k1 -> n1 -> n2 channels) is launched: a wave per channel tile of whichever convolution has more of
+// them in a workgroup (up to the variant's most), and enough workgroups to occupy the device: pixel tiles x ranges of the second
+// convolution's channel tiles.  With a depthwise stage, also enough threads that none of them walks more than four of the 16 pixels.
+struct PairSplit {
+    int ranges, tiles_per_block, waves;
+    bool small; // the variant for short reductions
+    bool apart; // not as a pair at all, but as two launches of the kernel for one convolution over few pixels
+};
+inline PairSplit split_pair(int64_t pixels, int k1, int n1, int n2, bool dw, int compute_units) {
+    auto up = [](int64_t v, int64_t d) { return (int)((v + d - 1) / d); };
+    const int ks1 = up(k1, 64), ks2 = up(n1, 64), t1 = up(n1, 16), t2 = up(n2, 16), ptiles = up(std::max<int64_t>(pixels, 1), 16);
+    PairSplit s;
+    s.small = ks1 <= 4 && ks2 <= 2;
+    const int max_waves = s.small ? 16 : 12, want = ptiles >= 512 ? 1 : 512 / ptiles;
+    s.tiles_per_block = up(t2, std::min(up(t2, max_waves), want));
+    s.ranges = up(t2, s.tiles_per_block);
+    s.waves = std::min(max_waves, std::max(t1, s.tiles_per_block));
+    if (dw) s.waves = std::min(max_waves, std::max(s.waves, up(k1, 64)));
+    // ... but no more than lets every workgroup be resident at once (a second round of workgroups doubles the
+    // launch's latency chain; a wave that takes two channel tiles one after the other adds a fraction of it)
+    const int occupancy = s.small ? 4 : 3; // waves per SIMD the variant is built for
+    s.waves = std::max(1, std::min(s.waves, 4 * occupancy / std::max(up((int64_t)ptiles * s.ranges, compute_units), 1)));
+    // With more tiles between the two than a workgroup has waves, some waves take several tiles of the whole reduction, chunk by chunk:
+    // so many trips to the weights in turn.  Apart where they are many, three tiles of few pixels, or more workgroups than units (us in a
+    // chain, pair / apart: 49 pixels 960 -> 320 -> 1280, 6 trips, 8.4 / 7.3; 50 of 960 -> 512 -> 96, 8, 10.0 / 7.0; 57 of 448 -> 480 -> 512, 3
+    // tiles, 7.6 / 6.7; 1143 of 640 -> 208 -> 640, two workgroups a unit, 14.9 / 8.7; but 60 of 512 -> 240 -> 1280, 3, 5.8 / 6.8, 85 of 384 ->
+    // 288 -> 64, 4, 5.8 / 6.9, 492 of 640 -> 240 -> 256, 5, 7.2 / 8.0, 585 of 320 -> 416 -> 24, 3 tiles, 6.5 / 7.2, 961 of 576 -> 272 -> 96, 6,
+    // 7.9 / 8.8).  Up to the pixels for which the kernel of few is measured: 3136 of 512 -> 256 -> 512 13.0 / 14.1.
+    const int tiles1 = up(t1, s.waves), tiles2 = up(s.tiles_per_block, s.waves), trips = tiles1 * up(ks1, 8) + tiles2 * up(ks2, 4);
+    s.apart = !dw && !s.small && t1 > max_waves && n1 % 16 == 0 && pixels <= 1600 && // (whose rows are whole pieces)
+              (trips >= (pixels <= 800 ? 6 : 7) || (tiles1 >= 3 && pixels <= 128) || tiles2 >= 2);
+    return s;
+}
+
 // The tile of at most `pix` output pixels (32 at most side by side) that covers an out_h x out_w image in the fewest blocks, rows
 // and columns spread evenly over them; among equals the one with the smallest input, among those the widest (below four columns
 // the first that does no better ends the search).  span: what a window reads, its dilation included.  (Asked for on every launch,

@@ -18,6 +18,7 @@
 // The second stage alone is the few-pixel path of nncase_hip_qconv2d (qpointwise_rows_kernel, further down): one dense
 // 1x1 convolution over few pixels (rows_shapes_ok), optionally behind a global average pool computed by the same launch.
 #include "qconv.hpp"
+#include "qconv_rules.hpp"
 
 #include <new>
 #include <vector>
@@ -440,7 +441,6 @@ template <bool POOL> __global__ __launch_bounds__(kRowsWaves * 64, 3) void qpoin
     if (works && part == 0) finish_tile<false, true>(a, tile, acc, rs[0], bias, ws, rv, nullptr, 0, a.lut_b ? lut_b : nullptr, lane, p, false);
 }
 
-static bool pair_is_small(int ks1, int ks2) { return ks1 <= 4 && ks2 <= 2; }
 // [tile][k-step][lane][16] s8 of w - 128, zero beyond the real channels / reduction
 static void pack_pair_weights(std::vector<uint8_t> &out, std::vector<int32_t> &wsum, const uint8_t *w_oihw, int n, int k, int tiles, int ksteps) {
     out.assign((size_t)tiles * ksteps * 1024, 0);
@@ -694,6 +694,11 @@ int launch_qconv_rows(nncase_hip_ctx *ctx, const uint8_t *x, const nncase_hip_we
 }
 } // namespace nnhip
 
+void nnhip::describe_pair(const nncase_hip_ctx *ctx, const nncase_hip_qpair *pr, const nncase_hip_conv2d_args_t *first, bool dw, char *buf, size_t cap) {
+    const bool apart = split_pair((int64_t)first->batch * first->in_h * first->in_w, pr->k1, pr->n1, pr->n2, dw, ctx->compute_units).apart;
+    snprintf(buf, cap, "%s", apart ? "qpointwise_rows+qpointwise_rows" : dw ? "dw3x3+qpointwise_pair_kernel" : "qpointwise_pair_kernel");
+}
+
 // dw / da: the depthwise convolution in front and its arguments, or null
 static int launch_pair(nncase_hip_ctx *ctx, const char *who, const uint8_t *x_dev, const nncase_hip_weights *dw,
                        const nncase_hip_conv2d_args_t *da, const nncase_hip_qpair *pr, uint8_t *y1_dev, uint8_t *y2_dev,
@@ -770,31 +775,12 @@ static int launch_pair(nncase_hip_ctx *ctx, const char *who, const uint8_t *x_de
         if (rc) return rc;
     }
 
-    // A wave per channel tile of whichever convolution has more of them in this workgroup (up to the variant's most),
-    // and enough workgroups to occupy the device: pixel tiles x ranges of the second convolution's channel tiles.  With
-    // a depthwise stage, also enough threads that none of them walks more than four of the 16 pixels.
-    const bool small = pair_is_small(a.ks1, a.ks2);
-    const int max_waves = small ? 16 : 12;
-    const int ptiles = (a.m + 15) / 16;
-    int ranges = (a.t2 + max_waves - 1) / max_waves;
-    const int want = ptiles >= 512 ? 1 : 512 / ptiles;
-    if (ranges > want) ranges = want;
-    a.tiles_per_block = (a.t2 + ranges - 1) / ranges;
-    ranges = (a.t2 + a.tiles_per_block - 1) / a.tiles_per_block;
-    int waves = std::min(max_waves, std::max(a.t1, a.tiles_per_block));
-    if (dw) waves = std::min(max_waves, std::max(waves, (a.k1 + 63) / 64));
-    {
-        // ... but no more than lets every workgroup be resident at once (a second round of workgroups doubles the
-        // launch's latency chain; a wave that takes two channel tiles one after the other adds a fraction of it)
-        const int occupancy = small ? 4 : 3; // waves per SIMD the variant is built for
-        const int per_cu = (ptiles * ranges + ctx->compute_units - 1) / std::max(ctx->compute_units, 1);
-        waves = std::max(1, std::min(waves, 4 * occupancy / std::max(per_cu, 1)));
-    }
+    const PairSplit split = split_pair(a.m, pr->k1, pr->n1, pr->n2, dw != nullptr, ctx->compute_units);
+    a.tiles_per_block = split.tiles_per_block;
+    const int waves = split.waves;
+    const bool small = split.small;
     NNHIP_HIP(ctx, hipSetDevice(ctx->device));
-    // More channels between the two than a workgroup has waves: some of the waves would take two tiles of the whole reduction, and the
-    // one after the other by the kernel for one convolution is quicker (960 -> 320 -> 1280 over 7 x 7: MobileNetV2 of one image 159.1 -> 157.2
-    // us, of two at 160 x 160 156 -> 150.6).
-    if (!dw && !small && a.t1 > max_waves && a.n1 % 16 == 0) { // (whose rows are whole pieces)
+    if (split.apart) {
         PairArgs one = a;
         one.ldy = a.n1, one.y2 = y1_dev, one.wb = a.wa, one.bias_b = a.bias_a, one.wsum_b = a.wsum_a, one.lut_b = a.lut_a;
         one.n1 = a.k1, one.n2 = a.n1, one.ks2 = a.ks1, one.t2 = a.t1, one.zxb = a.zxa, one.zwb = a.zwa, one.ep_b = a.ep_a, one.rep_b = a.rep_a;
@@ -803,7 +789,7 @@ static int launch_pair(nncase_hip_ctx *ctx, const char *who, const uint8_t *x_de
         a.x = y1_dev;
         return launch_rows(ctx, a, false);
     }
-    const dim3 grid(ptiles, ranges), block(waves * 64);
+    const dim3 grid((a.m + 15) / 16, split.ranges), block(waves * 64);
     auto go = [&](auto kernel, int ka, int kb) {
         const int sx = pair_row_bytes(a.ks1, pair_chunk(ka)), sy = pair_row_bytes(a.ks2, pair_chunk(kb));
         a.d_pieces = make_fastdiv((uint32_t)(sx - kRowPad) / 16);

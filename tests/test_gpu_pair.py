@@ -154,6 +154,22 @@ def test_pairs_whose_weights_are_requested_at_once(hip_ctx, k1, n1, n2):
     run_pair(hip_ctx, 1, k1, n1, n2, 5, 9, seed=k1 + n1 + n2, residual=n1 % 8 == 0, lut_b=n2 == 64)
 
 
+FORMS = [  # (in, mid, out, h, w, as two launches): either side of the rule's lines
+    (448, 240, 24, 3, 5, False), (384, 288, 64, 5, 17, False), (640, 240, 256, 7, 7, False),          # two tiles a wave, 3 to 5 trips
+    (1024, 272, 32, 5, 7, True), (576, 272, 96, 28, 29, False), (640, 400, 24, 1, 3, True),           # 6 trips, 6 of many pixels, 8
+    (128, 496, 1280, 4, 11, True), (96, 480, 96, 10, 13, False), (96, 480, 96, 8, 16, True),          # three tiles a wave up to 128 pixels
+    (192, 256, 960, 23, 39, True), (64, 288, 960, 40, 40, True), (64, 288, 960, 41, 40, False),       # two workgroups a unit, the most pixels
+]
+
+
+@pytest.mark.parametrize("k1,n1,n2,h,w,apart", FORMS)
+def test_pairs_as_one_launch_and_as_two(hip_ctx, k1, n1, n2, h, w, apart):
+    pair, (xd, y1d, y2d, fa_, sa_, keep) = run_pair(hip_ctx, 1, k1, n1, n2, h, w, seed=k1 + n1 + n2 + h, residual=n2 % 64 == 0, lut_a=h > 4, lut_b=n2 == 24)
+    fn = rt.Function(hip_ctx)
+    fn.add_qpointwise_pair(xd, pair, y1d, y2d, fa_, sa_)
+    assert fn.op_kernel(0) == ("qpointwise_rows+qpointwise_rows" if apart else "qpointwise_pair_kernel")
+
+
 P1 = ((1, 1), (1, 1))
 MOBILENET_TRIPLES = [  # (channels, mid, out, in_h, in_w, depthwise stride, residual): MobileNetV2's depthwise -> projection -> expansion
     (96, 24, 144, 28, 30, 2, False), (144, 24, 144, 14, 15, 1, True), (144, 32, 192, 56, 56, 2, False), (192, 32, 192, 28, 28, 1, True),

@@ -24,6 +24,7 @@ extern "C" int window(int stride, int ksteps, int channels, int pix, int waves, 
     return nnhip::tile_kernel_pays({stride, ksteps, channels, pix, waves, (size_t)lds, tiles, chunks, pixels}, 256);
 }
 extern "C" int dma_rows(long rows, int nchunks, int ksteps) { return 64 * nnhip::choose_dma_rows(rows, nchunks, ksteps, 256).rg; }
+extern "C" int pair_apart(long pixels, int k1, int n1, int n2, int dw) { return nnhip::split_pair(pixels, k1, n1, n2, dw, 256).apart; }
 extern "C" int dma(long rows, int n, int ksteps) { return nnhip::dma_pays(rows, n, ksteps, 256); }
 """)
     subprocess.check_call(["g++", "-std=c++17", "-O2", "-shared", "-fPIC", "-I", CSRC, str(d / "r.cpp"), "-o", str(d / "r.so")])
@@ -330,3 +331,24 @@ def test_large_products_take_the_quicker_blocks(rules, row):
     assert chosen <= 1.06 * min(us.values())
     if row[6] is not None:
         assert (chosen if rules.dma(rows, n, -(-k // 64)) else row[6]) <= 1.06 * min(chosen, row[6])
+
+
+# (pixels, channels in, between and out, us in a chain as one launch, as two)
+PAIRS = [
+    (1, 128, 256, 192, 5.16, 5.91), (13, 480, 208, 64, 4.78, 6.48), (60, 512, 240, 1280, 5.79, 6.75), (424, 288, 240, 640, 5.84, 7.62),
+    (834, 256, 224, 32, 5.19, 7.21), (73, 480, 288, 32, 5.65, 6.81), (138, 64, 320, 1280, 6.46, 7.11), (1253, 256, 304, 96, 6.27, 8.19),
+    (1, 512, 496, 1280, 7.18, 6.14), (57, 448, 480, 512, 7.58, 6.7), (125, 128, 512, 960, 7.62, 6.3), (198, 256, 400, 1536, 7.36, 7.59),
+    (86, 640, 240, 128, 6.99, 7.33), (492, 640, 240, 256, 7.15, 8.0), (585, 320, 416, 24, 6.52, 7.23), (892, 192, 256, 960, 11.95, 8.09),
+    (1070, 192, 496, 32, 7.05, 7.92), (1, 640, 384, 1280, 8.73, 6.29), (49, 960, 320, 1280, 8.38, 7.26), (122, 640, 384, 320, 9.4, 6.78),
+    (692, 1024, 352, 256, 9.03, 8.17), (961, 576, 272, 96, 7.9, 8.77), (819, 192, 288, 1280, 13.88, 10.2), (50, 960, 512, 96, 9.97, 7.03),
+    (1143, 640, 208, 640, 14.9, 8.7), (1407, 160, 320, 1280, 16.41, 12.94), (980, 1024, 304, 1280, 19.38, 11.81),
+    (3136, 512, 256, 512, 12.97, 14.07), (6400, 960, 320, 320, 23.24, 25.71),
+]
+
+
+@pytest.mark.parametrize("pixels,k1,n1,n2,one,two", PAIRS)
+def test_pairs_take_the_quicker_form(rules, pixels, k1, n1, n2, one, two):
+    rules.pair_apart.argtypes = [C.c_long, C.c_int, C.c_int, C.c_int, C.c_int]
+    assert (two if rules.pair_apart(pixels, k1, n1, n2, 0) else one) <= 1.02 * min(one, two)
+    assert not rules.pair_apart(pixels, k1, n1, n2, 1)                         # a depthwise stage in front: always one launch
+    assert not rules.pair_apart(pixels, k1, n1 + 4, n2, 0)                      # rows between the two that are no whole pieces
