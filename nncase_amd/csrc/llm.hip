@@ -12,6 +12,7 @@
 // of a block split the reduction and combine through LDS.  Per-output-channel scales, bias, the
 // residual add and the SwiGLU gate are applied in the epilogue.
 #include "common.hpp"
+#include "w8a16_rules.hpp"
 
 #include <hip/hip_fp16.h>
 
@@ -273,6 +274,22 @@ template <int MT, int G, bool SPLIT, bool PAIRED = false> __global__ __launch_bo
         rrow[t] = a.ln_w ? rstd[min(t * 16 + i16, a.m - 1)] : 1.f;
     }
 
+    // The epilogue's operands (SPLIT: of the token tile this wave finishes) are asked for before the products: the
+    // launch is a chain of memory round trips, and this takes the last one out of it (5 rows of 2880 to 208, normalised, 7.5 -> 7.2 us).
+    // (not with four token tiles: their slices leave no registers for it)
+    constexpr bool kPre = SPLIT && MT <= 2;
+    float4 sc[G], bs[G];
+    uint2 res_pre = uint2{0u, 0u};
+    if (kPre) {
+#pragma unroll
+        for (int g = 0; g < G; g++) {
+            sc[g] = *reinterpret_cast<const float4 *>(a.scale + tile[g] * 16 + kg * 4);
+            bs[g] = float4{0.f, 0.f, 0.f, 0.f};
+            if (a.bias) bs[g] = *reinterpret_cast<const float4 *>(a.bias + tile[g] * 16 + kg * 4);
+        }
+        const int m_pre = min(min(wave, MT - 1) * 16 + i16, a.m - 1);
+        if (a.residual) res_pre = *reinterpret_cast<const uint2 *>(a.residual + (size_t)m_pre * a.n_out + out_tile * 16 + kg * 4);
+    }
     for (int kb = ks0; kb < ks1; kb += B) {
         lu32x4 wv[B][G];
         lu32x4 av[B][MT][2];
@@ -364,23 +381,24 @@ template <int MT, int G, bool SPLIT, bool PAIRED = false> __global__ __launch_bo
                 } else {
                     s = acc[0][g][tt][r];
                 }
-                const int ch = tile[g] * 16 + kg * 4 + r;
-                s *= a.scale[ch];
-                if (a.bias) s += a.bias[ch];
+                if (kPre) {
+                    const float scv[4] = {sc[g].x, sc[g].y, sc[g].z, sc[g].w}, bsv[4] = {bs[g].x, bs[g].y, bs[g].z, bs[g].w};
+                    s *= scv[r];
+                    if (a.bias) s += bsv[r];
+                } else {
+                    const int ch = tile[g] * 16 + kg * 4 + r;
+                    s *= a.scale[ch];
+                    if (a.bias) s += a.bias[ch];
+                }
                 v[g][r] = s;
             }
         }
         if (m >= a.m) continue;
         const size_t o = (size_t)m * a.n_out + out_tile * 16 + kg * 4;
-        const uint2 res = a.residual ? *reinterpret_cast<const uint2 *>(a.residual + o) : uint2{0u, 0u};
+        const uint2 res = kPre ? res_pre : a.residual ? *reinterpret_cast<const uint2 *>(a.residual + o) : uint2{0u, 0u};
         store_gemm_row<G>(v, o, a.residual != nullptr, res, a.out, a.out_f32);
     }
 }
-
-constexpr int kRowsPieces = 4;                 // 512-element pieces of a row: k <= 2048
-constexpr int kRowsMaxK = kRowsPieces * 512;
-constexpr int kTileMaxK = 5120;                // ten k-steps a wave
-inline __host__ __device__ int rows_in_lds_pitch(int k) { return k * 2 + 16; } // bytes per token row: the padding spreads the rows over the banks
 
 // Kernel arguments that are used at different times, asked for together: a scalar load behind a branch or a wait is a wait of its own.
 template <typename A, typename B, typename C, typename D, typename E, typename F>
@@ -400,12 +418,16 @@ __device__ __forceinline__ void request_together(const A &a, const B &b, const C
 // number of tiles is a multiple of 8, and the weights come out of its L2.
 //
 // KS: k-steps of 64 a wave may have, all requested at once (k <= 512 * KS).
-// NORM: the rows are RMS-normalised on the way (see rms_rstd_rows for the order): wave w brings in rows w and, with R = 2, w + 8,
-// PIECES pieces of 512 elements each, and the products read them from LDS.  Without it they read the rows where they lie.
+// R: the products read the rows from LDS, and wave w brings in rows w and, with R = 2, w + 8, PIECES pieces of 512 elements each: whole
+// lines, where an operand read of the rows where they lie (R = 0: too long for LDS, or few) takes 32 bytes of each of 64 lines (14 rows of
+// 640 to 4768 columns 4.3 -> 3.5 us, 50 of 704 to 7760 10.8 -> 7.3).
+// NORM: the rows are RMS-normalised on the way (see rms_rstd_rows for the order).
 template <int G, int KS, bool NORM, int R, int PIECES, bool ROPE>
 __global__ __launch_bounds__(kGemmThreads) void w8a16_tile_kernel(const GemmArgs a) {
     static_assert(!ROPE || G == 2, "the rotating epilogue pairs two tiles of one block");
-    extern __shared__ __attribute__((aligned(16))) uint8_t xs[]; // NORM: [16][k halves + padding]
+    constexpr bool LDS = R > 0;
+    static_assert(LDS || !NORM, "rows are normalised on their way to LDS");
+    extern __shared__ __attribute__((aligned(16))) uint8_t xs[]; // LDS: [16][k halves + padding]
     __shared__ float red[kGemmWaves][G][64][4];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int i16 = lane & 15, kg = lane >> 4;
@@ -426,14 +448,14 @@ __global__ __launch_bounds__(kGemmThreads) void w8a16_tile_kernel(const GemmArgs
     if constexpr (ROPE) rope_pos = a.rope.ctx_lens[min(row0 + i16, last)]; // (loads return in order: asked for first, it is there first)
     const int per = (ksteps + kGemmWaves - 1) / kGemmWaves, ks0 = wave * per, ks1 = min(ksteps, ks0 + per);
     const uint16_t *xrow = x + (size_t)min(row0 + i16, last) * k + kg * 16;
-    lu32x4 v[NORM ? R : 1][NORM ? PIECES : 1], lwp[NORM ? PIECES : 1], wv[KS][G], av[NORM ? 1 : KS][2];
-    if constexpr (NORM) {
+    lu32x4 v[LDS ? R : 1][LDS ? PIECES : 1], lwp[NORM ? PIECES : 1], wv[KS][G], av[LDS ? 1 : KS][2];
+    if constexpr (LDS) {
 #pragma unroll
         for (int p = 0; p < PIECES; p++) {
             const int e0 = min(lane * 8 + p * 512, k - 8); // (past the row: masked below)
 #pragma unroll
             for (int i = 0; i < R; i++) v[i][p] = *reinterpret_cast<const lu32x4 *>(x + (size_t)min(row0 + wave + i * kGemmWaves, last) * k + e0);
-            lwp[p] = *reinterpret_cast<const lu32x4 *>(ln_w + e0);
+            if constexpr (NORM) lwp[p] = *reinterpret_cast<const lu32x4 *>(ln_w + e0);
         }
     }
     float4 sc[G], bs[G]; // (ahead of the products' operands: behind their thirty loads a cold line of scales would arrive last)
@@ -450,7 +472,7 @@ __global__ __launch_bounds__(kGemmThreads) void w8a16_tile_kernel(const GemmArgs
         const int ks = max(min(ks0 + u, ks1 - 1), 0);
 #pragma unroll
         for (int g = 0; g < G; g++) wv[u][g] = w[((size_t)tile[g] * ksteps + ks) * 64 + lane];
-        if constexpr (!NORM) {
+        if constexpr (!LDS) {
             av[u][0] = *reinterpret_cast<const lu32x4 *>(xrow + ks * 64), av[u][1] = *reinterpret_cast<const lu32x4 *>(xrow + ks * 64 + 8);
             __builtin_amdgcn_sched_barrier(0);
         }
@@ -465,41 +487,46 @@ __global__ __launch_bounds__(kGemmThreads) void w8a16_tile_kernel(const GemmArgs
         __builtin_amdgcn_sched_barrier(0);
     }
     const int pitch = rows_in_lds_pitch(k);
-    if constexpr (NORM) {
+    if constexpr (LDS) {
         if (wave < rows) { // (uniform; what LDS holds in the place of rows past m meets no row that is stored)
-            float ss[R];
+            if constexpr (NORM) {
+                float ss[R];
 #pragma unroll
-            for (int i = 0; i < R; i++) ss[i] = 0.f;
+                for (int i = 0; i < R; i++) ss[i] = 0.f;
 #pragma unroll
-            for (int p = 0; p < PIECES; p++)
-#pragma unroll
-                for (int i = 0; i < R; i++) {
-                    if (lane * 8 + p * 512 >= k) v[i][p] = lu32x4{0, 0, 0, 0}; // (+0 squares leave a sum as it is)
-                    add_squares8(v[i][p], ss[i]);
-                }
-#pragma unroll
-            for (int i = 0; i < R; i++) ss[i] = 1.0f / sqrtf(wave_sum(ss[i]) / (float)k + eps); // rstd_from_sum's formula
-#pragma unroll
-            for (int p = 0; p < PIECES; p++) {
-                __half wh[8], xh[R][8];
-                __builtin_memcpy(wh, &lwp[p], 16);
-#pragma unroll
-                for (int i = 0; i < R; i++) __builtin_memcpy(xh[i], &v[i][p], 16);
-#pragma unroll
-                for (int e = 0; e < 8; e++)
+                for (int p = 0; p < PIECES; p++)
 #pragma unroll
                     for (int i = 0; i < R; i++) {
-                        // the fp32 product is rounded before it is converted, as in rmsnorm_f16_kernel (see there)
-                        float pr = __half2float(xh[i][e]) * ss[i] * __half2float(wh[e]);
-                        asm volatile("" : "+v"(pr));
-                        xh[i][e] = __float2half_rn(pr);
+                        if (lane * 8 + p * 512 >= k) v[i][p] = lu32x4{0, 0, 0, 0}; // (+0 squares leave a sum as it is)
+                        add_squares8(v[i][p], ss[i]);
                     }
-                if (lane * 8 + p * 512 < k) {
 #pragma unroll
-                    for (int i = 0; i < R; i++)
-                        *reinterpret_cast<lu32x4 *>(xs + (size_t)(wave + i * kGemmWaves) * pitch + (lane * 8 + p * 512) * 2) = *reinterpret_cast<lu32x4 *>(xh[i]);
+                for (int i = 0; i < R; i++) ss[i] = 1.0f / sqrtf(wave_sum(ss[i]) / (float)k + eps); // rstd_from_sum's formula
+#pragma unroll
+                for (int p = 0; p < PIECES; p++) {
+                    __half wh[8], xh[R][8];
+                    __builtin_memcpy(wh, &lwp[p], 16);
+#pragma unroll
+                    for (int i = 0; i < R; i++) __builtin_memcpy(xh[i], &v[i][p], 16);
+#pragma unroll
+                    for (int e = 0; e < 8; e++)
+#pragma unroll
+                        for (int i = 0; i < R; i++) {
+                            // the fp32 product is rounded before it is converted, as in rmsnorm_f16_kernel (see there)
+                            float pr = __half2float(xh[i][e]) * ss[i] * __half2float(wh[e]);
+                            asm volatile("" : "+v"(pr));
+                            xh[i][e] = __float2half_rn(pr);
+                        }
+#pragma unroll
+                    for (int i = 0; i < R; i++) __builtin_memcpy(&v[i][p], xh[i], 16);
                 }
             }
+#pragma unroll
+            for (int p = 0; p < PIECES; p++)
+                if (lane * 8 + p * 512 < k) {
+#pragma unroll
+                    for (int i = 0; i < R; i++) *reinterpret_cast<lu32x4 *>(xs + (size_t)(wave + i * kGemmWaves) * pitch + (lane * 8 + p * 512) * 2) = v[i][p];
+                }
         }
         __syncthreads();
     }
@@ -513,7 +540,7 @@ __global__ __launch_bounds__(kGemmThreads) void w8a16_tile_kernel(const GemmArgs
     for (int u = 0; u < KS; u++) {
         if (ks0 + u < ks1) { // uniform
             h16x8 x0, x1;
-            if constexpr (NORM) {
+            if constexpr (LDS) {
                 x0 = *reinterpret_cast<const h16x8 *>(xl + (ks0 + u) * 128), x1 = *reinterpret_cast<const h16x8 *>(xl + (ks0 + u) * 128 + 16);
             } else {
                 __builtin_memcpy(&x0, &av[u][0], 16), __builtin_memcpy(&x1, &av[u][1], 16);
@@ -966,74 +993,41 @@ extern "C" int nncase_hip_w8a16_prepack(nncase_hip_ctx_t *ctx, const int8_t *w_h
     return 0;
 }
 
-// Whether a product of m rows and `tiles` tiles (pairs) over at most kRowsMaxK is computed with a tile's reduction split over a
-// block's waves.  The sum's order depends on it, so it is asked for the rows' count and the matrix alone: the product, the one that
-// normalises its rows and the one that rotates them agree bit for bit.  A block per tile repeats the rows' trip (and their
-// normalisation), a tile per wave leaves the device to few blocks.  us, split / not, k = 896: plain, 4096 / 8192 / 12 288 columns:
-// one row 3.1 4.2 4.7 / 5.7 6.8 6.4, 16 rows 4.0 5.4 6.4 / 5.9 7.0 6.6, 32 rows 5.2 7.9 10.0 / 8.0 9.3 8.8, 64 rows 7.7 13.0 17.4 /
-// 12.4 14.0 13.4; SwiGLU, 2048 / 8192 / 14 336 columns: one row 3.7 5.7 7.4 / 7.8 9.5 9.4, 16 rows 4.5 6.8 9.9 / 7.7 9.6 9.5,
-// 32 rows 4.6 10.4 15.3 / 9.9 11.5 11.3, 64 rows 6.4 17.0 27.0 / 15.0 16.7 16.7.
-static bool rows_take_split(const nncase_hip_ctx_t *ctx, const nncase_hip_w8a16_t *w, int tiles, bool glu, int m) {
-    if (w->k > kRowsMaxK || 16 * rows_in_lds_pitch(w->k) > 64 * 1024) return false;
-    const int64_t rt = (m + 15) / 16, cus = ctx->compute_units;
-    if (m <= kGemmWaves) return tiles < 4 * cus;
-    if (glu) return tiles * rt < (2 + rt) * cus;
-    return 2 * tiles < (rt == 1 ? 5 : 4) * cus;
-}
+static W8Product w8_product(const nncase_hip_w8a16_t *w, int m, bool glu) { return W8Product{m, w->k, glu ? w->ntiles / 2 : w->ntiles, glu}; }
 
 // Whether the q / k / v projection of this geometry can rotate and append in its own epilogue (else the caller runs
 // the projection and the rope kernel one after the other).
 static bool rope_epilogue_fits(const nncase_hip_ctx_t *ctx, const nncase_hip_w8a16_t *w, int m, const RopeArgs &r) {
-    return rows_take_split(ctx, w, w->ntiles, false, m) && r.d % 32 == 0 && w->n == (r.hq + 2 * r.hkv) * r.d && w->k <= 1024;
+    return rows_take_split(w8_product(w, m, false), ctx->compute_units) && r.d % 32 == 0 && w->n == (r.hq + 2 * r.hkv) * r.d && w->k <= 1024;
 }
 
-// Whether a long reduction over few tiles is computed in tiles of 8 by 8 (and summed in their order, whichever kernel does it).
-// They are four times the blocks of 16 by 16, each of which moves half as much: taken while all of them run at once.  us, 16 by
-// 16 / 8 by 8, k = 4864, 896 columns: one row 5.3 / 4.4, 8 rows 6.2 / 5.7, 16 rows 7.9 / 5.6, 32 rows 7.9 / 8.4.
-static bool sums_in_pairs(const nncase_hip_ctx_t *ctx, const nncase_hip_w8a16_t *w, int m) {
-    return w->k > kRowsMaxK && w->k <= kTileMaxK && m <= 16 && 2 * w->ntiles * ((m + 7) / 8) <= ctx->compute_units;
-}
-
-// Which kernel computes a product of m rows.
-enum class GemmForm {
-    kTile,      // a tile (pair) per block, its reduction split over the waves
-    kSmallTile, // 8 channels by 8 rows per block
-    kRowsInLds, // a tile (pair) per wave, rows in LDS
-    kSplit,     // as kTile (and in its order), for reductions that it has no registers or LDS for
-    kPerWave,   // a tile (pair) per wave, rows read where they lie
-};
-static GemmForm gemm_form(const nncase_hip_ctx_t *ctx, const nncase_hip_w8a16_t *w, int m, bool glu, bool normalises) {
-    const int out_tiles = glu ? w->ntiles / 2 : w->ntiles, mt = (m + 15) / 16, mt_built = mt <= 1 ? 1 : (mt == 2 ? 2 : 4);
-    // few output tiles: the block's waves split the reduction of one tile; many: a tile per wave
-    const bool split = out_tiles < 4 * ctx->compute_units;
-    // (fewer tiles than compute units and nothing to normalise: kTile too, below)
-    if (rows_take_split(ctx, w, out_tiles, glu, m) && (glu || normalises || out_tiles >= ctx->compute_units)) return GemmForm::kTile;
-    // a tile per wave with the token rows shared through LDS: where the rows fit and the launch has a tile for every
-    // compute unit
-    if (w->k <= kRowsMaxK && (size_t)mt_built * 16 * rows_in_lds_pitch(w->k) <= 128 * 1024 && out_tiles >= ctx->compute_units) return GemmForm::kRowsInLds;
-    if (!split) return GemmForm::kPerWave;
-    if (!glu && !normalises && sums_in_pairs(ctx, w, m)) return GemmForm::kSmallTile;
-    return normalises || w->k > kTileMaxK ? GemmForm::kSplit : GemmForm::kTile;
-}
-
-template <int G, int KS, bool NORM, int R = 1, int PIECES = 1, bool ROPE = false>
+template <int G, int KS, bool NORM, int R, int PIECES, bool ROPE>
 static int launch_tile(nncase_hip_ctx_t *ctx, const GemmArgs &a, int tiles) {
-    const size_t lds = NORM ? (size_t)16 * rows_in_lds_pitch(a.k) : 0;
+    const size_t lds = R > 0 ? (size_t)16 * rows_in_lds_pitch(a.k) : 0;
     if (lds + G * kGemmWaves * 1024 > 48 * 1024) NNHIP_HIP(ctx, (raise_dynamic_lds<w8a16_tile_kernel<G, KS, NORM, R, PIECES, ROPE>>(ctx->device, 96 * 1024)));
     hipLaunchKernelGGL((w8a16_tile_kernel<G, KS, NORM, R, PIECES, ROPE>), dim3(tiles, (a.m + 15) / 16), dim3(kGemmThreads), lds, ctx->stream, a);
     NNHIP_LAUNCH_CHECK(ctx, "w8a16_tile_kernel");
     return 0;
 }
-template <int G, bool ROPE = false> static int launch_tile_normalising(nncase_hip_ctx_t *ctx, const GemmArgs &a, int tiles) {
-    const bool few = a.m <= kGemmWaves; // a row per wave at most
-    if (a.k <= 1024) return few ? launch_tile<G, 2, true, 1, 2, ROPE>(ctx, a, tiles) : launch_tile<G, 2, true, 2, 2, ROPE>(ctx, a, tiles);
+// (kernels for the k-steps that a wave has: what is asked for past its share is read again)
+template <int G, bool NORM, bool ROPE> static int launch_tile_rows(nncase_hip_ctx_t *ctx, const GemmArgs &a, int tiles) {
+    auto by_rows = [&](auto steps) { // (a row per wave, or two)
+        constexpr int S = decltype(steps)::value;
+        return a.m <= kGemmWaves ? launch_tile<G, S, NORM, 1, S, ROPE>(ctx, a, tiles) : launch_tile<G, S, NORM, 2, S, ROPE>(ctx, a, tiles);
+    };
+    static_assert(kRowsPieces == 4, "a piece of a row is a k-step of each wave");
+    if (a.k <= 512) return by_rows(std::integral_constant<int, 1>());
+    if (a.k <= 1024) return by_rows(std::integral_constant<int, 2>());
     if constexpr (ROPE) return -EINVAL; // (see rope_epilogue_fits)
-    else return few ? launch_tile<G, 4, true, 1, kRowsPieces>(ctx, a, tiles) : launch_tile<G, 4, true, 2, kRowsPieces>(ctx, a, tiles);
+    else return a.k <= 1536 ? by_rows(std::integral_constant<int, 3>()) : by_rows(std::integral_constant<int, 4>());
 }
-template <int G> static int launch_tile_plain(nncase_hip_ctx_t *ctx, const GemmArgs &a, int tiles) {
-    if (a.k <= 1024) return launch_tile<G, 2, false>(ctx, a, tiles);
-    if (a.k <= 2048) return launch_tile<G, 4, false>(ctx, a, tiles);
-    return launch_tile<G, kTileMaxK / 512, false>(ctx, a, tiles);
+template <int G> static int launch_tile_long(nncase_hip_ctx_t *ctx, const GemmArgs &a, int tiles) {
+    const int share = (a.ksteps + kGemmWaves - 1) / kGemmWaves;
+    if (share <= 4) return launch_tile<G, 4, false, 0, 0, false>(ctx, a, tiles);
+    if (share <= 5) return launch_tile<G, 5, false, 0, 0, false>(ctx, a, tiles);
+    if (share <= 6) return launch_tile<G, 6, false, 0, 0, false>(ctx, a, tiles);
+    if (share <= 8) return launch_tile<G, 8, false, 0, 0, false>(ctx, a, tiles);
+    return launch_tile<G, kTileMaxK / 512, false, 0, 0, false>(ctx, a, tiles);
 }
 
 static int launch_w8a16_gemm(nncase_hip_ctx_t *ctx, const void *a_dev, const nncase_hip_w8a16_t *w, void *out_dev, int32_t m,
@@ -1071,23 +1065,24 @@ static int launch_w8a16_gemm(nncase_hip_ctx_t *ctx, const void *a_dev, const nnc
     if (rope) { // (the caller has checked rope_epilogue_fits) a block per pair of tiles d / 2 channels apart
         a.rope = *rope;
         a.up_tile_offset = rope->d / 32;
-        if (a.ln_w) return launch_tile_normalising<2, true>(ctx, a, w->ntiles / 2);
-        return launch_tile<2, 2, false, 1, 1, true>(ctx, a, w->ntiles / 2);
+        return a.ln_w ? launch_tile_rows<2, true, true>(ctx, a, w->ntiles / 2) : launch_tile_rows<2, false, true>(ctx, a, w->ntiles / 2);
     }
-    const GemmForm form = gemm_form(ctx, w, m, glu, a.ln_w != nullptr);
-    if (form == GemmForm::kTile) {
-        if (a.ln_w) return glu ? launch_tile_normalising<2>(ctx, a, out_tiles) : launch_tile_normalising<1>(ctx, a, out_tiles);
-        return glu ? launch_tile_plain<2>(ctx, a, out_tiles) : launch_tile_plain<1>(ctx, a, out_tiles);
+    const W8Product product = w8_product(w, m, glu);
+    const W8Form form = choose_w8_form(product, a.ln_w != nullptr, ctx->compute_units);
+    if (form == W8Form::kTileLong) return glu ? launch_tile_long<2>(ctx, a, out_tiles) : launch_tile_long<1>(ctx, a, out_tiles);
+    if (form == W8Form::kTile) {
+        if (a.ln_w) return glu ? launch_tile_rows<2, true, false>(ctx, a, out_tiles) : launch_tile_rows<1, true, false>(ctx, a, out_tiles);
+        return glu ? launch_tile_rows<2, false, false>(ctx, a, out_tiles) : launch_tile_rows<1, false, false>(ctx, a, out_tiles);
     }
-    if (form == GemmForm::kSmallTile) {
+    if (form == W8Form::kSmallTile) {
         hipLaunchKernelGGL((w8a16_small_tile_kernel<kTileMaxK / 1024>), dim3(out_tiles * 2, (m + 7) / 8), dim3(kGemmThreads), 0, ctx->stream, a);
         NNHIP_LAUNCH_CHECK(ctx, "w8a16_small_tile_kernel");
         return 0;
     }
-    const bool split = form == GemmForm::kSplit;
-    const bool paired = split && !glu && sums_in_pairs(ctx, w, m);
+    const bool split = form == W8Form::kSplit;
+    const bool paired = split && sums_in_pairs(product, ctx->compute_units);
     const dim3 grid(split ? out_tiles : (out_tiles + kGemmWaves - 1) / kGemmWaves), block(kGemmThreads);
-    if (form == GemmForm::kRowsInLds) {
+    if (form == W8Form::kRowsInLds) {
         const int mt_built = mt <= 1 ? 1 : (mt == 2 ? 2 : 4);
         const size_t rows_lds = (size_t)mt_built * 16 * rows_in_lds_pitch(w->k);
         const bool short_rows = w->k <= 1024; // rows of two 512-element pieces (a lane keeps a row's pieces in registers)
@@ -1150,8 +1145,8 @@ bool nnhip::w8a16_weight_fetch(const nncase_hip_ctx *ctx, const nncase_hip_w8a16
             return true;
         }
     }
-    const GemmForm form = gemm_form(ctx, w, m, glu, normalises);
-    if (form == GemmForm::kRowsInLds || form == GemmForm::kPerWave) return false;
+    const W8Form form = choose_w8_form(w8_product(w, m, glu), normalises, ctx->compute_units);
+    if (form == W8Form::kRowsInLds || form == W8Form::kPerWave) return false;
     // (kSmallTile: two blocks a tile, on the die that a block per tile would be on)
     f->blocks = f->off = (uint32_t)(glu ? w->ntiles / 2 : w->ntiles);
     f->per_block = glu ? 2 : 1;

@@ -384,8 +384,8 @@ def test_projection_of_many_heads_that_rotates_and_appends(hip_ctx, B, k, norm, 
 @pytest.mark.parametrize("m,k,n", [(1, 64, 16), (17, 448, 32), (33, 1024, 48), (64, 1088, 144), (49, 2048, 16), (16, 2112, 112), (1, 4864, 128),
                                    (9, 4096, 2048), (8, 5120, 4096), (16, 2176, 2048), (16, 2176, 2064), (17, 2176, 2048), (3, 5184, 64)])
 def test_products_of_a_tile_per_block(hip_ctx, m, k, n):
-    """Tiles of 16 x 16 over several row tiles and of 8 x 8, at the ends of the reductions that each takes (512 k-steps of a wave's
-    registers, 5120; beyond it the general kernel), with shares that leave waves idle or with an odd step, and where the last group
+    """Tiles of 16 x 16 over several row tiles and of 8 x 8, at the ends of the reductions that each takes (5120: ten k-steps in a
+    wave's registers; beyond it the general kernel), with shares that leave waves idle or with an odd step, and where the last group
     of eight tiles is not full."""
     for out32 in (False, True):
         test_w8a16_gemm(hip_ctx, m, k, n, out32)
@@ -403,3 +403,17 @@ def test_rmsnorm_fused_into_gemm_over_row_tiles_and_long_reductions(hip_ctx, m, 
 @pytest.mark.parametrize("B,k,norm", [(17, 896, True), (33, 1024, True), (64, 896, True), (64, 512, False)])
 def test_projection_over_row_tiles_that_rotates_and_appends(hip_ctx, B, k, norm):
     test_projection_that_rotates_and_appends_equals_the_two_operators(hip_ctx, B, k, norm)
+
+
+@pytest.mark.parametrize("m,k,n,mode", [
+    (8, 512, 256, "residual"), (9, 576, 4128, "plain"), (16, 1024, 512, "swiglu"), (17, 1088, 4096, "f32"), (5, 1536, 64, "plain"),
+    (33, 1600, 1024, "swiglu"), (64, 2048, 160, "residual"),                                    # rows through LDS: one to four pieces, one or two a wave
+    (4, 2048, 1152, "plain"), (5, 2048, 1152, "plain"), (16, 1600, 512, "swiglu"), (4, 1600, 6400, "residual"), (3, 1984, 14048, "swiglu"),  # four k-steps a wave
+    (2, 2560, 48, "plain"), (7, 2624, 4096, "residual"), (40, 3136, 1600, "f32"), (31, 4096, 784, "plain"), (16, 3648, 2048, "plain"),
+    (1, 4160, 2048, "plain"), (1, 4160, 2064, "plain"), (9, 4160, 1040, "plain"), (24, 4288, 992, "swiglu"), (20, 3776, 4896, "swiglu"),  # where they lie
+    (32, 2048, 20464, "plain"), (32, 2048, 20480, "f32"),                                       # rows that LDS does not hold, split and not
+])
+def test_every_form_of_a_product_and_its_normalised_one(hip_ctx, m, k, n, mode):
+    """At the lines between the kernels: the values, and the same bits whether the rows are normalised on the way or before."""
+    test_w8a16_gemm(hip_ctx, m, k, n, mode == "f32")
+    test_rmsnorm_fused_into_gemm_equals_the_two_operators(hip_ctx, m, k, n, mode)
