@@ -65,9 +65,10 @@ inline AttnRunRule attn_run_rule(int64_t batch, int64_t kv_heads, int compute_un
 }
 
 // Tokens per split of the kernel that goes through a split 128 tokens at a time, for sequences of `total` tokens the longest of which
-// has `longest`: one split up to 384 tokens, else as many as make one round of the device, a block per compute unit: fewer leave units
-// idle, a second round costs as much as the first (us with runs of 256 / 512 / 1024 / 2048: 32 pairs of 3425 tokens 12.6 11.3 15.3
-// 23.9, 80 of 2220 19.0 18.8 16.8 25.2).  Where splits of 2048 tokens would still be more than that: 512 tokens, which even the rounds
+// has `longest`: one split up to 512 tokens, without a merge (24 sequences of one head of up to 439 tokens 8.9 us, 10.9 as two; 13 of 4 of
+// 468 8.4 / 9.2), else as many as make one round of the device, a block per compute unit: fewer leave units idle, a second round
+// costs as much as the first (us with runs of 256 / 512 / 1024 / 2048: 32 pairs of 3425 tokens 12.6 11.3 15.3 23.9, 80 of 2220 19.0
+// 18.8 16.8 25.2).  Where splits of 2048 tokens would still be more than that: 512 tokens, which even the rounds
 // out (152 of 10 998 82.7 77.6 82.4 91.1), or 1024 where that is the whole context or with nine rounds and more (1600 of 1500 136 126
 // 117 119).
 //   * Sequences that together are less than a quarter of what they would be at the longest's length: two rounds, of 256 to 512
@@ -78,7 +79,7 @@ NNHIP_HOST_DEVICE int attn_run(const AttnRunRule &r, uint32_t longest, uint32_t 
     const uint32_t least = steps(attn_divide(longest + r.most.divisor - 1, r.most));
     const uint32_t even = steps(attn_divide(longest + r.round.divisor - 1, r.round));
     uint32_t run;
-    if (longest <= 384) run = steps(longest);
+    if (longest <= 512) run = steps(longest);
     else if (total * 4 < longest * r.batch) run = std::min(std::max(steps(attn_divide(total, r.two_rounds)), 256u), 512u);
     else if (r.has_round && even <= 2048) run = std::max(even, 256u);
     else if (longest <= 1024) run = 1024;
@@ -92,11 +93,14 @@ NNHIP_HOST_DEVICE int attn_run(const AttnRunRule &r, uint32_t longest, uint32_t 
 //     16.4 / 17.9, 132 of 14 756 50.7 / 52.1)
 //   * 128-wide heads from 50 MB of keys and values on (48 pairs of 1851 15.2 / 13.8, 36 of 6028 22.3 / 17.9, 104 of 9746 107 / 80, 656 of
 //     4073 267 / 229; below, 64 of 1205 12.1 / 13.0 and 8 of 4387 12.3 / 14.0), which few pairs reach with long contexts only, and too
-//     many splits (8 of 12 668 18.4 / 20.0).  By the capacity: short contexts in a large cache take it too, and are no slower for it
-//     (32 pairs of 300 / 1000 tokens in one of 16 384: 9.3 / 7.7 and 9.7 / 9.3).
+//     many splits (8 of 12 668 18.4 / 20.0); not in a step or less a wave (1616 of 64 8.5 / 10.4, 8192 of 16 28.9 / 38.1, 4096 of 112 17.9 /
+//     19.1; 192 of 512 level), nor where one split a pair is a block more for a few of the compute units (272 of 711 15.5 / 17.5, 260 of
+//     984 22.4 / 26.2, 288 of 670 16.1 / 18.6; 308 of 690 20.7 / 19.0, 332 of 606 19.5 / 17.2, 436 of 622 24.2 / 20.1).  By the capacity: short
+//     contexts in a large cache take it too, and are no slower for it (32 pairs of 300 / 1000 tokens in one of 16 384: 9.3 / 7.7 and 9.7 / 9.3).
 inline int choose_attn_run(int head_dim, int64_t pairs, int64_t max_tokens, int compute_units) {
     if (head_dim == 64) return max_tokens > 256 && max_tokens <= 512 && pairs >= 24 ? (int)((max_tokens + 127) / 128 * 128) : 0;
-    if (pairs < 16 || pairs * max_tokens < 98304 || max_tokens > kAttnMaxSplits * 2048) return 0;
+    if (pairs < 16 || max_tokens <= 128 || pairs * max_tokens < 98304 || max_tokens > kAttnMaxSplits * 2048) return 0;
+    if (max_tokens > 512 && max_tokens <= 1024 && pairs > compute_units && 6 * pairs <= 7ll * compute_units) return 0;
     return attn_run(attn_run_rule(1, pairs, compute_units, kAttnMaxSplits), (uint32_t)max_tokens, (uint32_t)max_tokens);
 }
 

@@ -88,7 +88,8 @@ STEPS = [
     (64, 12, 433, 6.2, 6.4), (64, 24, 265, 5.8, 5.3), (64, 60, 459, 6.6, 6.2), (64, 240, 384, 7.8, 5.9), (64, 84, 4759, 16.4, 17.9),
     (64, 144, 3041, 16.7, 18.2), (64, 132, 14756, 50.7, 52.1), (128, 64, 1205, 12.1, 13.0), (128, 8, 4387, 12.3, 14.0), (128, 4, 993, 8.6, 9.3),
     (128, 36, 6028, 22.3, 17.9), (128, 104, 9746, 106.9, 79.6), (128, 256, 490, 13.0, 10.2), (128, 624, 280, 21.6, 19.0), (128, 656, 4073, 266.7, 229.1),
-    (128, 16, 15583, 32.1, 21.7), (128, 8, 12668, 18.4, 20.0),
+    (128, 16, 15583, 32.1, 21.7), (128, 8, 12668, 18.4, 20.0), (128, 1616, 64, 8.5, 10.4), (128, 8192, 16, 28.9, 38.1), (128, 4096, 112, 17.9, 19.1),
+    (128, 260, 984, 22.4, 26.2), (128, 272, 711, 15.5, 17.5), (128, 288, 670, 16.1, 18.6), (128, 308, 690, 20.7, 19.0), (128, 332, 606, 19.5, 17.2), (128, 436, 622, 24.2, 20.1),
 ]
 
 
@@ -190,3 +191,11 @@ def test_every_split_of_a_sequence_has_its_blocks(run_by_lengths, choose_run):
                         for total in {longest, longest + (batch - 1) * (longest // 9), longest * batch}:
                             r = run_by_lengths.run_by_lengths(batch, kv_heads, longest, total, room)
                             assert r > 0 and r % 128 == 0 and r * room >= longest, (batch, kv_heads, capacity, longest, total, r)
+
+
+@pytest.mark.parametrize("batch,kv_heads,longest", [(16, 1, 300), (24, 1, 439), (13, 4, 468), (52, 2, 487), (4, 8, 512), (200, 1, 512)])
+def test_short_contexts_in_a_large_cache_are_one_split(run_by_lengths, batch, kv_heads, longest):
+    """(us with two splits / one: 24 x 1 of 439 tokens 10.9 / 8.9, 13 x 4 of 468 9.2 / 8.4, 52 x 2 of 487 9.2 / 8.5)"""
+    for total in (longest * batch, longest + (batch - 1) * (longest // 5)):
+        assert run_by_lengths.run_by_lengths(batch, kv_heads, longest, total, 64) >= longest
+    assert run_by_lengths.run_by_lengths(batch, kv_heads, 640, 640 * batch, 64) < 640 or batch * kv_heads > 128
