@@ -64,11 +64,12 @@ struct __attribute__((packed, aligned(1))) wide_unaligned16 {
 };
 
 // 16 bytes of the tensor x (bytes `bytes`, 16-byte aligned) from any byte offset; what lies outside it is undefined.
-// near_end (wave-uniform) says that some piece of the wave may reach past the last byte; those that do are put together from
-// aligned dwords, range-checked one by one (the last dword that holds a byte of the tensor never crosses into another page).
-// (Asked again for the pieces at hand: a wave near the end that fetched all of them so took twice as long as the others.)
-__device__ __forceinline__ wide_u32x4 load_ragged(const uint8_t *x, const __amdgpu_buffer_rsrc_t &dwords, int bytes, int off, bool near_end) {
-    if (!near_end || (bytes >= 16 && !__any(off > bytes - 16))) return reinterpret_cast<const wide_unaligned16 *>(x + (uint32_t)min(max(off, 0), bytes - 16))->v;
+__device__ __forceinline__ wide_u32x4 load_ragged(const uint8_t *x, int bytes, int off) {
+    return reinterpret_cast<const wide_unaligned16 *>(x + (uint32_t)min(max(off, 0), bytes - 16))->v;
+}
+// The same where it may reach past the last byte: put together from aligned dwords, range-checked one by one (the last dword that
+// holds a byte of the tensor never crosses into another page).
+__device__ __forceinline__ wide_u32x4 load_ragged_end(const __amdgpu_buffer_rsrc_t &dwords, int off) {
     uint32_t d[5];
 #pragma unroll
     for (int i = 0; i < 5; i++) d[i] = __builtin_amdgcn_raw_buffer_load_b32(dwords, (off & ~3) + i * 4, 0, 0);
@@ -203,14 +204,34 @@ __global__ __launch_bounds__(WM * WN * KG * 64, WM * WN * KG > 8 ? 4 : 2) void q
         for (int i = 0; i < NA; i++) near_end = near_end || (int64_t)p_off[i] + last + 16 > (int64_t)a.x_bytes;
         near_end = __any(near_end);
     }
-    auto fetch = [&](int off) __attribute__((always_inline)) {
-        if constexpr (kRagged) return load_ragged(a.x, xres, (int)a.x_bytes, off, near_end);
-        else return __builtin_amdgcn_raw_buffer_load_b128(xres, off, 0, 0);
-    };
     struct Acts {
         wide_u32x4 raw[NA];
         uint32_t fill;    // what a piece that is not taken holds: the zero point (padding tap) or x' = 0 (past the reduction)
         bool take[NA];
+    };
+    // the thread's pieces, at p_off + shift
+    auto fetch = [&](Acts &f, int shift) __attribute__((always_inline)) {
+        if constexpr (kRagged) {
+            // A wave near the end asks again for the pieces at hand (one that fetched all of them dword by dword took twice as long as the
+            // others), all of them at once: asked for each piece it was 2 to 12 % of a small layer (57 x 57 by 50 to 204 3x3 6.8 -> 7.6 us).
+            bool past = near_end;
+            if (near_end && a.x_bytes >= 16) {
+                past = false;
+#pragma unroll
+                for (int i = 0; i < NA; i++) past = past || p_off[i] + shift > (int)a.x_bytes - 16;
+                past = __any(past);
+            }
+            if (past) {
+#pragma unroll
+                for (int i = 0; i < NA; i++) f.raw[i] = load_ragged_end(xres, p_off[i] + shift);
+            } else {
+#pragma unroll
+                for (int i = 0; i < NA; i++) f.raw[i] = load_ragged(a.x, (int)a.x_bytes, p_off[i] + shift);
+            }
+        } else {
+#pragma unroll
+            for (int i = 0; i < NA; i++) f.raw[i] = __builtin_amdgcn_raw_buffer_load_b128(xres, p_off[i] + shift, 0, 0);
+        }
     };
     auto load_acts = [&](Acts &f, int sl) {
         const int ksc = min(sl * KG + kg, KS - 1); // as for the weights
@@ -224,11 +245,9 @@ __global__ __launch_bounds__(WM * WN * KG * 64, WM * WN * KG > 8 ? 4 : 2) void q
         } else if (LM == kWideRows || LM == kWideRagRows) {
             // the last k-step may end inside the row: the piece's offset goes through the range-checked operand
             const bool in_k = ksc * 64 + lq * 16 < a.k;
+            fetch(f, ksc * 64);
 #pragma unroll
-            for (int i = 0; i < NA; i++) {
-                f.raw[i] = fetch(p_off[i] + ksc * 64);
-                f.take[i] = in_k;
-            }
+            for (int i = 0; i < NA; i++) f.take[i] = in_k;
             f.fill = 0x80808080u;
         } else if (LM == kWideTap) {
             // one tap per k-step: its geometry is the same for the whole block (scalar unit)
@@ -253,9 +272,9 @@ __global__ __launch_bounds__(WM * WN * KG * 64, WM * WN * KG > 8 ? 4 : 2) void q
             const uint32_t ky = fastdiv(tap, a.d_kw);
             const int dy = (int)ky * a.dil_h, dx = ((int)tap - (int)ky * a.kw) * a.dil_w;
             const int shift = (dy * a.in_w + dx) * a.ldx + c;
+            fetch(f, shift);
 #pragma unroll
             for (int i = 0; i < NA; i++) {
-                f.raw[i] = fetch(p_off[i] + shift);
                 f.take[i] = in_k && (unsigned)(p_iy0[i] + dy) < (unsigned)a.in_h && (unsigned)(p_ix0[i] + dx) < (unsigned)a.in_w;
             }
             f.fill = in_k ? a.zx_splat : 0x80808080u;
