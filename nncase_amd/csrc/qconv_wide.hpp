@@ -214,14 +214,10 @@ __global__ __launch_bounds__(WM * WN * KG * 64, WM * WN * KG > 8 ? 4 : 2) void q
         if constexpr (kRagged) {
             // A wave near the end asks again for the pieces at hand (one that fetched all of them dword by dword took twice as long as the
             // others), all of them at once: asked for each piece it was 2 to 12 % of a small layer (57 x 57 by 50 to 204 3x3 6.8 -> 7.6 us).
-            bool past = near_end;
-            if (near_end && a.x_bytes >= 16) {
-                past = false;
+            int most = p_off[0];
 #pragma unroll
-                for (int i = 0; i < NA; i++) past = past || p_off[i] + shift > (int)a.x_bytes - 16;
-                past = __any(past);
-            }
-            if (past) {
+            for (int i = 1; i < NA; i++) most = max(most, p_off[i]);
+            if (near_end && (a.x_bytes < 16 || __any(most + shift > (int)a.x_bytes - 16))) {
 #pragma unroll
                 for (int i = 0; i < NA; i++) f.raw[i] = load_ragged_end(xres, p_off[i] + shift);
             } else {
