@@ -437,3 +437,23 @@ def test_a_lane_chosen_after_the_capture_leaves_it_as_it_is():
         fn.invoke()
         assert np.array_equal(b.download((64,), np.uint8), np.arange(64, dtype=np.uint8) + 3), f"lane {lane}"
     ctx.close()
+
+
+@pytest.mark.parametrize("fused", [False, True])
+def test_the_benchmark_reports_the_traffic_of_the_kernels_it_launches(hip_ctx, fused):
+    """bench.py's table of measured traffic names exactly the kernels of its batch-64 function (it reports none otherwise), and the
+    profile that it comes from holds the same figures."""
+    import importlib.util
+    import os
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    spec = importlib.util.spec_from_file_location("bench", os.path.join(root, "bench.py"))
+    bench = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(bench)
+    key = "fused" if fused else "unfused"
+    qg = nb.quantize_graph(nb.mobilenet_v2(seed=2), np.random.default_rng(3).random((32, 224, 224, 3), dtype=np.float32))
+    model = nb.HipModel(hip_ctx, qg, 64, capture_graph=False, fuse_blocks=fused)
+    table = bench.MEASURED_TRAFFIC_B64[key]
+    assert {model.fn.op_kernel(i) for i in range(len(model.fn))} == set(table)
+    with open(os.path.join(root, bench.MEASURED_TRAFFIC_SOURCE[key])) as f:
+        profile = f.read()
+    assert all(f'"{name}": {count},' in profile for name, count in table.items())
