@@ -549,7 +549,9 @@ constexpr int64_t kRowsMaxPixels = 32;
 // Past two pixel tiles: reductions long enough that a wave per chunk of them is a shorter chain than the tiled kernels' steps, while
 // what the tiles stream between them stays small (us, tiled / so: 49 pixels of 512 -> 512 4.1 / 3.3, 400 of them 4.2 / 3.7, 400 of 960 ->
 // 160 5.0 / 4.0, 1600 of 512 -> 128 4.2 / 3.7; shorter reductions 400 of 160 -> 960 3.8 / 3.9, 1600 of 64 -> 256 3.6 / 4.0; more to stream
-// 784 of 1024 -> 512, 26 MB, 5.0 / 5.3, 1600 of 1536 -> 256, 39 MB, 5.6 / 7.7).
+// 784 of 1024 -> 512, 26 MB, 5.0 / 5.3, 1600 of 1536 -> 256, 39 MB, 5.6 / 7.7).  Past 1600 pixels what streams little still gains and
+// the rest does not (2500 of 512 -> 64, 5 MB, 4.3 / 3.7, 4900 of them 4.4 / 4.0; 2500 of 960 -> 160, 24 MB, 5.4 / 5.3, 3136 of them
+// 5.5 / 7.6; 1936 of 256 -> 128, 4 MB, 3.6 / 3.7, 4900 of them 4.5 / 4.9).
 constexpr int kManyRowsMinK = 256;
 constexpr int64_t kManyRowsStreamLimit = 14000000, kManyRowsMaxPixels = 1600;
 

@@ -80,9 +80,10 @@ template <int U, bool PAST, typename A, typename B, class F> __device__ __forcei
 }
 
 // What quantize divides by.  QUICK: x / scale by the reciprocal, 3 instructions instead of some 11, which bound the kernel (25 M
-// elements f16 -> u8: 14.9 -> 12.0 us, 6.3 TB/s; 3.3 M f32 -> u8 4.5 -> 3.3).  q0 = x * r is within 1.5 ulp of the quotient and q0 + (x - scale * q0) * r, rounded once, is
-// the quotient's nearest float (held by enumeration of every pair of mantissas whose quotient lies near enough to the middle of two
-// floats).  A q0 far past every code is cut to +-2^40, so that an infinity leaves no difference of two infinities behind; a NaN stays
+// elements f16 -> u8: 14.9 -> 12.0 us, 6.3 TB/s; 3.3 M f32 -> u8 4.5 -> 3.3).  q0 = x * r is within 1.5 ulp of the quotient and
+// q0 + (x - scale * q0) * r, rounded once, is the quotient's nearest float: Markstein's theorem of the quotient corrected by a correctly
+// rounded reciprocal, which asks for a q0 within one ulp; the rest was held by enumeration of every pair of mantissas whose quotient
+// lies near enough to the middle of two floats.  A q0 far past every code is cut to +-2^40, so that an infinity leaves no difference of two infinities behind; a NaN stays
 // one up to the conversion, which makes the lowest code of it like the general form.
 struct Divisor {
     float scale, reciprocal, bias;
