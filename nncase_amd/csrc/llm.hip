@@ -6,7 +6,7 @@
 // each int8 weight byte is read from HBM exactly once and the step is bound by that stream
 // (~0.5 GB for a Qwen2-0.5B-shaped model).  The GEMM is organised around it: weights are
 // pre-packed so that a wave's load of one k-step is a contiguous 1 KiB fragment (16 bytes per
-// lane), converted int8 -> fp16 in registers (exactly: (w ^ 0x80) | 0x6400 is the fp16 1024 + w + 128)
+// lane), converted int8 -> fp16 in registers (exactly: (w + 128) | 0x6400 is the fp16 1024 + w + 128)
 // and fed to v_mfma_f32_16x16x32_f16 as the A operand (16 output channels), the token rows being
 // the B operand; a lane ends up with 4 consecutive output channels of one token.  The four waves
 // of a block split the reduction and combine through LDS.  Per-output-channel scales, bias, the
@@ -38,7 +38,7 @@ struct nncase_hip_w8a16 {
     int k = 0, n = 0;      // reduction length (multiple of 64), output channels (multiple of 16)
     int ntiles = 0, ksteps = 0;
     void *d_packed = nullptr; // [ntiles][ksteps][64 lanes][16 B]: lane (i = l % 16, kg = l / 16) holds
-                              // w[tile * 16 + i][ks * 64 + kg * 16 .. + 15]
+                              // w[tile * 16 + i][ks * 64 + kg * 16 .. + 15], each as the unsigned byte w + 128
     float *d_scale = nullptr; // [n]
     float *d_bias = nullptr;  // [n] or null
 };
@@ -77,14 +77,35 @@ struct GemmArgs {
 // 8 * lane .. 8 * lane + 7 of every 512-element piece of the row (one 16-byte load per piece); it adds their squares
 // in index order, piece after piece, and a butterfly adds the 64 lanes.  The order is part of the definition: the
 // product kernel that normalises its own rows must arrive at the same bits as rmsnorm_f16_kernel.
+//
+// Squares and scalings are one instruction per element: v_fma_mix_f32 takes halves where they lie in a dword (a conversion and a
+// multiplication or addition otherwise, each rounding where this one does: the square of a half is exact in fp32, and a sum with -0
+// is the other summand).
 __device__ __forceinline__ void add_squares8(const lu32x4 &v, float &ss) {
-    __half h[8];
-    __builtin_memcpy(h, &v, 16);
+    const h16x8 h = __builtin_bit_cast(h16x8, v);
 #pragma unroll
-    for (int e = 0; e < 8; e++) {
-        const float f = __half2float(h[e]);
-        ss += f * f;
+    for (int e = 0; e < 8; e++) ss = __builtin_fmaf((float)h[e], (float)h[e], ss);
+}
+// fp16(x * r * w) of eight elements, both products and the conversion rounding by themselves (see rmsnorm_f16_kernel): the second product
+// passes an assembly statement, or the compiler would make one rounding of it and the conversion.
+__device__ __forceinline__ lu32x4 normalise8(const lu32x4 &x, float r, const lu32x4 &w) {
+    typedef float f32x2v __attribute__((ext_vector_type(2)));
+    const h16x8 xh = __builtin_bit_cast(h16x8, x), wh = __builtin_bit_cast(h16x8, w);
+    float zero = -0.0f;
+    asm("" : "+s"(zero)); // (or the compiler would make a multiplication of it, behind a conversion)
+    lu32x4 y;
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+        f32x2v p;
+#pragma unroll
+        for (int q = 0; q < 2; q++) {
+            float v = __builtin_fmaf(__builtin_fmaf((float)xh[2 * e + q], r, zero), (float)wh[2 * e + q], zero);
+            asm("" : "+v"(v));
+            p[q] = v;
+        }
+        y[e] = __builtin_bit_cast(uint32_t, __builtin_convertvector(p, h16x2));
     }
+    return y;
 }
 // The sum over the wave's lanes, in every lane, bit for bit the butterfly `for (o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o)`
 // (a sum of two does not mind their order) on row swaps and DPP moves: a shuffle goes through the LDS crossbar and back, six of
@@ -186,14 +207,13 @@ __device__ __forceinline__ void rope_store(const RopeArgs &a, int b, const RopeP
     }
 }
 
-// 8 int8 weights (two dwords' low / high halves handled by the caller) -> 8 fp16, exact.
+// 8 packed weights -> 8 fp16, exact: the byte w + 128 under 0x64 is the half 1024 + w + 128.
 __device__ __forceinline__ h16x8 w8_to_f16(uint32_t lo, uint32_t hi) {
-    const uint32_t x0 = lo ^ 0x80808080u, x1 = hi ^ 0x80808080u;
     uint32_t h[4];
-    h[0] = __builtin_amdgcn_perm(0x64646464u, x0, 0x07010700u); // [b0, 0x64, b1, 0x64] -> halves 1024 + b0, 1024 + b1
-    h[1] = __builtin_amdgcn_perm(0x64646464u, x0, 0x07030702u);
-    h[2] = __builtin_amdgcn_perm(0x64646464u, x1, 0x07010700u);
-    h[3] = __builtin_amdgcn_perm(0x64646464u, x1, 0x07030702u);
+    h[0] = __builtin_amdgcn_perm(0x64646464u, lo, 0x07010700u); // [b0, 0x64, b1, 0x64]
+    h[1] = __builtin_amdgcn_perm(0x64646464u, lo, 0x07030702u);
+    h[2] = __builtin_amdgcn_perm(0x64646464u, hi, 0x07010700u);
+    h[3] = __builtin_amdgcn_perm(0x64646464u, hi, 0x07030702u);
     h16x8 v;
     __builtin_memcpy(&v, h, 16);
     return v - (_Float16)1152.0f; // 1024 + (w + 128) - 1152 = w, exact in fp16
@@ -223,6 +243,14 @@ template <int G> __device__ __forceinline__ void store_gemm_row(const float (&v)
     }
 }
 
+// The same for one channel.
+template <int G> __device__ __forceinline__ void store_gemm_one(const float (&v)[G], size_t o, bool has_residual, uint16_t res, void *out, int out_f32) {
+    float y = G == 2 ? v[0] / (1.f + __expf(-v[0])) * v[G - 1] : v[0];
+    if (has_residual) y += __half2float(__builtin_bit_cast(__half, res));
+    if (out_f32) reinterpret_cast<float *>(out)[o] = y;
+    else reinterpret_cast<__half *>(out)[o] = __float2half_rn(y);
+}
+
 // MT = 16-token column tiles (m <= 16 * MT); G = matrices multiplied at once (2: SwiGLU gate and up).
 // grid.x = output tiles of 16 channels.  The eight waves of a block split the reduction; a wave
 // requests the weights and token slices of four k-steps before it multiplies any of them, so a
@@ -230,6 +258,7 @@ template <int G> __device__ __forceinline__ void store_gemm_row(const float (&v)
 constexpr int kGemmWaves = 8;
 constexpr int kGemmThreads = kGemmWaves * 64;
 constexpr int kGemmBatch = 4; // k-steps a wave requests before it multiplies any
+constexpr int kRedPitch = 64 + 16; // floats
 
 // SPLIT: the block's waves share one output tile and split its reduction (few tiles, long reductions);
 // otherwise every wave owns a tile of its own and the whole reduction (many tiles: the vocabulary head).
@@ -316,19 +345,7 @@ template <int MT, int G, bool SPLIT, bool PAIRED = false> __global__ __launch_bo
 #pragma unroll
                 for (int t = 0; t < MT; t++)
 #pragma unroll
-                    for (int hlf = 0; hlf < 2; hlf++) {
-                        __half xh[8], wh[8];
-                        __builtin_memcpy(xh, &av[u][t][hlf], 16);
-                        __builtin_memcpy(wh, &lw[u][hlf], 16);
-#pragma unroll
-                        for (int e = 0; e < 8; e++) {
-                            // the fp32 product is rounded before it is converted, as in rmsnorm_f16_kernel (see there)
-                            float pr = __half2float(xh[e]) * rrow[t] * __half2float(wh[e]);
-                            asm volatile("" : "+v"(pr));
-                            xh[e] = __float2half_rn(pr);
-                        }
-                        __builtin_memcpy(&av[u][t][hlf], xh, 16);
-                    }
+                    for (int hlf = 0; hlf < 2; hlf++) av[u][t][hlf] = normalise8(av[u][t][hlf], rrow[t], lw[u][hlf]);
         }
 #pragma unroll
         for (int u = 0; u < B; u++) {
@@ -416,6 +433,11 @@ __device__ __forceinline__ void request_together(const A &a, const B &b, const C
 // (Loads behind branches cannot be waited for one by one: the normalisation waited for the weights' trip to memory, and the
 // products for the scales'.)  More than 16 rows are more blocks, not longer ones: those of one tile run on one die where the
 // number of tiles is a multiple of 8, and the weights come out of its L2.
+// Between the waits it is instructions: a wave issues one every 4 to 9 cycles, so the hundred that one wave runs while the others
+// wait for it are a quarter of a microsecond.  Hence rows scaled with v_fma_mix_f32, weights converted ahead of the barrier, an output
+// per lane on four waves behind the last one, the rotation on waves that have fewer rows to bring in (one operator over 24 layers, us,
+// before / after: 1 row gate / up 4.86 / 4.34, q / k / v 4.16 / 3.60, output 2.55 / 2.29; 16 rows 6.34 / 5.53, 5.06 / 4.72, 2.89 /
+// 2.61; 64 rows gate / up 11.6 / 9.3).
 //
 // KS: k-steps of 64 a wave may have, all requested at once (k <= 512 * KS).
 // R: the products read the rows from LDS, and wave w brings in rows w and, with R = 2, w + 8, PIECES pieces of 512 elements each: whole
@@ -428,7 +450,8 @@ __global__ __launch_bounds__(kGemmThreads) void w8a16_tile_kernel(const GemmArgs
     constexpr bool LDS = R > 0;
     static_assert(LDS || !NORM, "rows are normalised on their way to LDS");
     extern __shared__ __attribute__((aligned(16))) uint8_t xs[]; // LDS: [16][k halves + padding]
-    __shared__ float red[kGemmWaves][G][64][4];
+    // a wave's sums: [four channels][16 rows][channel of the four], the rows of the next four 16 banks on
+    __shared__ float red[kGemmWaves][G][4][kRedPitch];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int i16 = lane & 15, kg = lane >> 4;
     const int k = a.k, ksteps = a.ksteps, off = a.up_tile_offset, n_out = a.n_out, out_f32 = a.out_f32;
@@ -445,7 +468,7 @@ __global__ __launch_bounds__(kGemmThreads) void w8a16_tile_kernel(const GemmArgs
 
     // ---- requests ---------------------------------------------------------------------------------------
     int rope_pos = 0;
-    if constexpr (ROPE) rope_pos = a.rope.ctx_lens[min(row0 + i16, last)]; // (loads return in order: asked for first, it is there first)
+    if constexpr (ROPE) rope_pos = a.rope.ctx_lens[min(row0 + (wave & 3) * 4 + kg, last)]; // (loads return in order: asked for first, it is there first)
     const int per = (ksteps + kGemmWaves - 1) / kGemmWaves, ks0 = wave * per, ks1 = min(ksteps, ks0 + per);
     const uint16_t *xrow = x + (size_t)min(row0 + i16, last) * k + kg * 16;
     lu32x4 v[LDS ? R : 1][LDS ? PIECES : 1], lwp[NORM ? PIECES : 1], wv[KS][G], av[LDS ? 1 : KS][2];
@@ -458,14 +481,13 @@ __global__ __launch_bounds__(kGemmThreads) void w8a16_tile_kernel(const GemmArgs
             if constexpr (NORM) lwp[p] = *reinterpret_cast<const lu32x4 *>(ln_w + e0);
         }
     }
-    float4 sc[G], bs[G]; // (ahead of the products' operands: behind their thirty loads a cold line of scales would arrive last)
+    // The lane's output, of the four waves that finish the tile: row fw * 4 + lane / 16, channel lane % 16.
+    const int fw = ROPE ? wave - 4 : wave, frow = (fw & 3) * 4 + kg, fch = tile0 * 16 + i16;
+    float sc[G], bs[G]; // (ahead of the products' operands: behind their thirty loads a cold line of scales would arrive last)
 #pragma unroll
-    for (int g = 0; g < G; g++) {
-        sc[g] = *reinterpret_cast<const float4 *>(scale + tile[g] * 16 + kg * 4);
-        bs[g] = *reinterpret_cast<const float4 *>(bias + tile[g] * 16 + kg * 4);
-    }
-    const size_t o = (size_t)min(row0 + i16, last) * n_out + tile[0] * 16 + kg * 4; // of the lane's four outputs
-    const uint2 res = *reinterpret_cast<const uint2 *>(residual ? residual + o : x);
+    for (int g = 0; g < G; g++) sc[g] = scale[fch + g * off * 16], bs[g] = bias[fch + g * off * 16];
+    const size_t o = (size_t)min(row0 + frow, last) * n_out + fch;
+    const uint16_t res = *(residual ? residual + o : x);
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int u = 0; u < KS; u++) {
@@ -482,8 +504,9 @@ __global__ __launch_bounds__(kGemmThreads) void w8a16_tile_kernel(const GemmArgs
     // ---- rows --------------------------------------------------------------------------------------------
     RopePair rope;
     if constexpr (ROPE) {
-        // The angle is computed while the rows and weights travel; wave w finishes channel w of each lane's four.
-        if (wave < 4) rope = rope_pair(a.rope, min(row0 + i16, last), (tile0 * 16 + kg * 4 + wave) / a.rope.d, (tile0 * 16 + kg * 4 + wave) % a.rope.d, rope_pos);
+        // The angle is computed while the rows and weights travel, by the waves that finish the tile: the upper four, which have fewer
+        // rows to bring in or none.
+        if (fw >= 0 && fw * 4 < rows) rope = rope_pair(a.rope, min(row0 + frow, last), fch / a.rope.d, fch % a.rope.d, rope_pos);
         __builtin_amdgcn_sched_barrier(0);
     }
     const int pitch = rows_in_lds_pitch(k);
@@ -503,23 +526,9 @@ __global__ __launch_bounds__(kGemmThreads) void w8a16_tile_kernel(const GemmArgs
 #pragma unroll
                 for (int i = 0; i < R; i++) ss[i] = 1.0f / sqrtf(wave_sum(ss[i]) / (float)k + eps); // rstd_from_sum's formula
 #pragma unroll
-                for (int p = 0; p < PIECES; p++) {
-                    __half wh[8], xh[R][8];
-                    __builtin_memcpy(wh, &lwp[p], 16);
+                for (int p = 0; p < PIECES; p++)
 #pragma unroll
-                    for (int i = 0; i < R; i++) __builtin_memcpy(xh[i], &v[i][p], 16);
-#pragma unroll
-                    for (int e = 0; e < 8; e++)
-#pragma unroll
-                        for (int i = 0; i < R; i++) {
-                            // the fp32 product is rounded before it is converted, as in rmsnorm_f16_kernel (see there)
-                            float pr = __half2float(xh[i][e]) * ss[i] * __half2float(wh[e]);
-                            asm volatile("" : "+v"(pr));
-                            xh[i][e] = __float2half_rn(pr);
-                        }
-#pragma unroll
-                    for (int i = 0; i < R; i++) __builtin_memcpy(&v[i][p], xh[i], 16);
-                }
+                    for (int i = 0; i < R; i++) v[i][p] = normalise8(v[i][p], ss[i], lwp[p]);
             }
 #pragma unroll
             for (int p = 0; p < PIECES; p++)
@@ -528,8 +537,14 @@ __global__ __launch_bounds__(kGemmThreads) void w8a16_tile_kernel(const GemmArgs
                     for (int i = 0; i < R; i++) *reinterpret_cast<lu32x4 *>(xs + (size_t)(wave + i * kGemmWaves) * pitch + (lane * 8 + p * 512) * 2) = v[i][p];
                 }
         }
-        __syncthreads();
     }
+    // (converted ahead of the barrier: by the waves without a row while the others normalise theirs)
+    h16x8 wf[KS][G][2];
+#pragma unroll
+    for (int u = 0; u < KS; u++)
+#pragma unroll
+        for (int g = 0; g < G; g++) wf[u][g][0] = w8_to_f16(wv[u][g][0], wv[u][g][1]), wf[u][g][1] = w8_to_f16(wv[u][g][2], wv[u][g][3]);
+    if constexpr (LDS) __syncthreads();
 
     // ---- products ------------------------------------------------------------------------------------------
     f32x4v acc[G];
@@ -547,52 +562,30 @@ __global__ __launch_bounds__(kGemmThreads) void w8a16_tile_kernel(const GemmArgs
             }
 #pragma unroll
             for (int g = 0; g < G; g++) {
-                acc[g] = __builtin_amdgcn_mfma_f32_16x16x32_f16(w8_to_f16(wv[u][g][0], wv[u][g][1]), x0, acc[g], 0, 0, 0);
-                acc[g] = __builtin_amdgcn_mfma_f32_16x16x32_f16(w8_to_f16(wv[u][g][2], wv[u][g][3]), x1, acc[g], 0, 0, 0);
+                acc[g] = __builtin_amdgcn_mfma_f32_16x16x32_f16(wf[u][g][0], x0, acc[g], 0, 0, 0);
+                acc[g] = __builtin_amdgcn_mfma_f32_16x16x32_f16(wf[u][g][1], x1, acc[g], 0, 0, 0);
             }
         }
     }
 #pragma unroll
-    for (int g = 0; g < G; g++) *reinterpret_cast<f32x4v *>(red[wave][g][lane]) = acc[g];
+    for (int g = 0; g < G; g++) *reinterpret_cast<f32x4v *>(&red[wave][g][kg][i16 * 4]) = acc[g];
     __syncthreads();
-    // lane (i16 = token, kg): channels tile * 16 + kg * 4 + r
-    if constexpr (ROPE) {
-        // The rotation costs a few hundred instructions per pair, so the pairs are spread over four waves.
-        if (wave >= 4 || i16 >= rows) return;
-        float v2[2];
-#pragma unroll
-        for (int g = 0; g < 2; g++) {
-            float s = 0.f;
-#pragma unroll
-            for (int q = 0; q < kGemmWaves; q++) s += red[q][g][lane][wave]; // fixed order, as below
-            const float scv[4] = {sc[g].x, sc[g].y, sc[g].z, sc[g].w}, bsv[4] = {bs[g].x, bs[g].y, bs[g].z, bs[g].w};
-            float sv = scv[0], bv = bsv[0];
-#pragma unroll
-            for (int q = 1; q < 4; q++) sv = wave == q ? scv[q] : sv, bv = wave == q ? bsv[q] : bv;
-            s *= sv;
-            if (has_bias) s += bv;
-            v2[g] = s;
-        }
-        // (rounded to fp16 as the projection's output would be stored; the partner is d / 2 channels further)
-        rope_store(a.rope, row0 + i16, rope, __half2float(__float2half_rn(v2[0])), __half2float(__float2half_rn(v2[1])));
-        return;
-    }
-    if (wave != 0) return;
-    float y[G][4];
+    // An output per lane, by as many waves as the rows need: what follows is a chain of some hundred instructions, and with four
+    // channels a lane on one wave it was twice as long.
+    if (fw < 0 || fw * 4 >= rows) return; // (uniform)
+    float y[G];
 #pragma unroll
     for (int g = 0; g < G; g++) {
-        const float scv[4] = {sc[g].x, sc[g].y, sc[g].z, sc[g].w}, bsv[4] = {bs[g].x, bs[g].y, bs[g].z, bs[g].w};
-        f32x4v s = f32x4v{0.f, 0.f, 0.f, 0.f};
+        float s = 0.f;
 #pragma unroll
-        for (int q = 0; q < kGemmWaves; q++) s += *reinterpret_cast<const f32x4v *>(red[q][g][lane]); // fixed order: deterministic
-#pragma unroll
-        for (int r = 0; r < 4; r++) {
-            y[g][r] = s[r] * scv[r];
-            if (has_bias) y[g][r] += bsv[r];
-        }
+        for (int q = 0; q < kGemmWaves; q++) s += red[q][g][i16 >> 2][frow * 4 + (i16 & 3)]; // fixed order: deterministic
+        y[g] = s * sc[g];
+        if (has_bias) y[g] += bs[g];
     }
-    if (i16 >= rows) return;
-    store_gemm_row<G>(y, o, residual != nullptr, res, out, out_f32);
+    if (frow >= rows) return;
+    // (rounded to fp16 as the projection's output would be stored; the partner is d / 2 channels further)
+    if constexpr (ROPE) rope_store(a.rope, row0 + frow, rope, __half2float(__float2half_rn(y[0])), __half2float(__float2half_rn(y[1])));
+    else store_gemm_one<G>(y, o, residual != nullptr, res, out, out_f32);
 }
 
 // The same product for long reductions over few tiles (the down projection), where a block of the kernel above has its compute
@@ -617,11 +610,11 @@ template <int KP> __global__ __launch_bounds__(kGemmThreads) void w8a16_small_ti
     const int half = r16 >= in_group, tile = group + r16 - half * in_group;
     const int row0 = (int)blockIdx.y * 8, rows = min(8, a.m - row0), last = row0 + rows - 1;
     const int per = (ksteps + kGemmWaves - 1) / kGemmWaves, ks0 = wave * per, ks1 = min(ksteps, ks0 + per);
-    // the lane of wave 0 that finishes row i8, channels tile * 16 + half * 8 + odd * 4 + 0 .. 3
-    const int ch = tile * 16 + half * 8 + odd * 4;
-    const size_t o = (size_t)min(row0 + i8, last) * n_out + ch;
-    const float4 sc = *reinterpret_cast<const float4 *>(scale + ch), bs = *reinterpret_cast<const float4 *>(bias + ch);
-    const uint2 res = *reinterpret_cast<const uint2 *>(residual ? residual + o : x);
+    // the output of wave 0's lane: row lane / 8, channel lane % 8 of the eight
+    const int frow = lane >> 3, ch = tile * 16 + half * 8 + i8;
+    const size_t o = (size_t)min(row0 + frow, last) * n_out + ch;
+    const float sc = scale[ch], bs = bias[ch];
+    const uint16_t res = *(residual ? residual + o : x);
     const lu32x4 *wl = w + (size_t)tile * ksteps * 64 + kg * 16 + half * 8 + i8;
     const uint16_t *xl = x + (size_t)min(row0 + i8, last) * k + kg * 16;
     lu32x4 wv[KP], av[KP][2];
@@ -645,22 +638,17 @@ template <int KP> __global__ __launch_bounds__(kGemmThreads) void w8a16_small_ti
     }
     *reinterpret_cast<f32x4v *>(red[wave][lane]) = acc;
     __syncthreads();
-    if (wave != 0 || lane >= 16) return;
-    f32x4v s = f32x4v{0.f, 0.f, 0.f, 0.f};
+    if (wave != 0) return;
+    float y[1] = {0.f};
 #pragma unroll
     for (int q = 0; q < kGemmWaves; q++) { // fixed order: deterministic
-        s += *reinterpret_cast<const f32x4v *>(red[q][odd * 16 + i8]);
-        s += *reinterpret_cast<const f32x4v *>(red[q][(odd + 2) * 16 + 8 + i8]);
+        y[0] += red[q][(i8 >> 2) * 16 + frow][i8 & 3];
+        y[0] += red[q][((i8 >> 2) + 2) * 16 + 8 + frow][i8 & 3];
     }
-    const float scv[4] = {sc.x, sc.y, sc.z, sc.w}, bsv[4] = {bs.x, bs.y, bs.z, bs.w};
-    float y[1][4];
-#pragma unroll
-    for (int r = 0; r < 4; r++) {
-        y[0][r] = s[r] * scv[r];
-        if (has_bias) y[0][r] += bsv[r];
-    }
-    if (i8 >= rows) return;
-    store_gemm_row<1>(y, o, residual != nullptr, res, out, out_f32);
+    y[0] *= sc;
+    if (has_bias) y[0] += bs;
+    if (frow >= rows) return;
+    store_gemm_one<1>(y, o, residual != nullptr, res, out, out_f32);
 }
 
 constexpr int kRowsBatch = 8;
@@ -729,24 +717,9 @@ template <int MT, int G, int KB, int PIECES> __global__ __launch_bounds__(kGemmT
 #pragma unroll
             for (int i = 0; i < R; i++) rr[i] = 1.0f / sqrtf(ss[i] / (float)a.k + a.ln_eps); // rstd_from_sum's formula
 #pragma unroll
-            for (int p = 0; p < PIECES; p++) {
-                __half wh[8];
-                __builtin_memcpy(wh, &lwp[p], 16);
-                __half xh[R][8];
+            for (int p = 0; p < PIECES; p++)
 #pragma unroll
-                for (int i = 0; i < R; i++) __builtin_memcpy(xh[i], &v[i][p], 16);
-#pragma unroll
-                for (int e = 0; e < 8; e++)
-#pragma unroll
-                    for (int i = 0; i < R; i++) {
-                        // the fp32 product is rounded before it is converted, as in rmsnorm_f16_kernel (see there)
-                        float pr = __half2float(xh[i][e]) * rr[i] * __half2float(wh[e]);
-                        asm volatile("" : "+v"(pr));
-                        xh[i][e] = __float2half_rn(pr);
-                    }
-#pragma unroll
-                for (int i = 0; i < R; i++) __builtin_memcpy(&v[i][p], xh[i], 16);
-            }
+                for (int i = 0; i < R; i++) v[i][p] = normalise8(v[i][p], rr[i], lwp[p]);
         }
 #pragma unroll
         for (int p = 0; p < PIECES; p++) {
@@ -970,12 +943,14 @@ extern "C" int nncase_hip_w8a16_prepack(nncase_hip_ctx_t *ctx, const int8_t *w_h
     NNHIP_REQUIRE(ctx, w, -ENOMEM, "w8a16_prepack: out of host memory");
     w->k = k, w->n = n, w->ntiles = n / 16, w->ksteps = k / 64;
     const size_t bytes = (size_t)n * k;
-    std::vector<int8_t> packed(bytes);
+    std::vector<uint8_t> packed(bytes);
     for (int t = 0; t < w->ntiles; t++)
         for (int ks = 0; ks < w->ksteps; ks++)
             for (int l = 0; l < 64; l++) {
                 const int i = l & 15, kg = l >> 4;
-                memcpy(&packed[(((size_t)t * w->ksteps + ks) * 64 + l) * 16], w_host + (size_t)(t * 16 + i) * k + ks * 64 + kg * 16, 16);
+                const int8_t *src = w_host + (size_t)(t * 16 + i) * k + ks * 64 + kg * 16;
+                uint8_t *dst = &packed[(((size_t)t * w->ksteps + ks) * 64 + l) * 16];
+                for (int b = 0; b < 16; b++) dst[b] = (uint8_t)src[b] ^ 0x80u;
             }
     auto cleanup = [&](int rc) {
         (void)nncase_hip_w8a16_destroy(ctx, w);
@@ -1004,7 +979,7 @@ static bool rope_epilogue_fits(const nncase_hip_ctx_t *ctx, const nncase_hip_w8a
 template <int G, int KS, bool NORM, int R, int PIECES, bool ROPE>
 static int launch_tile(nncase_hip_ctx_t *ctx, const GemmArgs &a, int tiles) {
     const size_t lds = R > 0 ? (size_t)16 * rows_in_lds_pitch(a.k) : 0;
-    if (lds + G * kGemmWaves * 1024 > 48 * 1024) NNHIP_HIP(ctx, (raise_dynamic_lds<w8a16_tile_kernel<G, KS, NORM, R, PIECES, ROPE>>(ctx->device, 96 * 1024)));
+    if (lds + G * kGemmWaves * 4 * kRedPitch * sizeof(float) > 48 * 1024) NNHIP_HIP(ctx, (raise_dynamic_lds<w8a16_tile_kernel<G, KS, NORM, R, PIECES, ROPE>>(ctx->device, 96 * 1024)));
     hipLaunchKernelGGL((w8a16_tile_kernel<G, KS, NORM, R, PIECES, ROPE>), dim3(tiles, (a.m + 15) / 16), dim3(kGemmThreads), lds, ctx->stream, a);
     NNHIP_LAUNCH_CHECK(ctx, "w8a16_tile_kernel");
     return 0;

@@ -417,3 +417,48 @@ def test_every_form_of_a_product_and_its_normalised_one(hip_ctx, m, k, n, mode):
     """At the lines between the kernels: the values, and the same bits whether the rows are normalised on the way or before."""
     test_w8a16_gemm(hip_ctx, m, k, n, mode == "f32")
     test_rmsnorm_fused_into_gemm_equals_the_two_operators(hip_ctx, m, k, n, mode)
+
+
+@pytest.mark.parametrize("m", [3, 4, 5, 12, 13, 17])
+@pytest.mark.parametrize("k,n,mode", [(896, 1152, "residual"), (448, 64, "swiglu"), (4864, 112, "f32")])
+def test_waves_that_finish_a_tile(hip_ctx, m, k, n, mode):
+    """A wave finishes four rows of a 16 x 16 tile (or all eight of an 8 x 8 one): row counts around its multiples."""
+    test_w8a16_gemm(hip_ctx, m, k, n, mode == "f32")
+    test_rmsnorm_fused_into_gemm_equals_the_two_operators(hip_ctx, m, k, n, mode)
+
+
+@pytest.mark.parametrize("B,k", [(4, 896), (5, 512), (12, 1024), (13, 896)])
+def test_waves_that_finish_a_rotated_tile(hip_ctx, B, k):
+    test_projection_that_rotates_and_appends_equals_the_two_operators(hip_ctx, B, k, True)
+
+
+@pytest.mark.parametrize("hidden", [64, 896, 1528])
+def test_rmsnorm_bits(hip_ctx, hidden):
+    """The definition, in float32 and in its order (a lane's eight consecutive elements of every 512, a butterfly over the lanes): the same
+    bits, subnormal and signed-zero halves included."""
+    rng = np.random.default_rng(hidden)
+    x = (rng.standard_normal((6, hidden)) * np.array([[3], [1e-3], [6e-7], [1e-5], [200], [1]])).astype(np.float16)
+    x[5, ::3], x[5, 1::3] = 0.0, -0.0
+    w = (1 + 0.3 * rng.standard_normal(hidden)).astype(np.float16)
+    w[::7] = np.float16(6e-8)
+    pieces = -(-hidden // 512)
+    f = np.zeros((6, pieces * 512), np.float32)
+    f[:, :hidden] = x
+    f = f.reshape(6, pieces, 64, 8)
+    v = np.zeros((6, 64), np.float32)
+    for p in range(pieces):
+        for e in range(8):
+            v = v + f[:, p, :, e] * f[:, p, :, e]
+    for o in (32, 16, 8, 4, 2, 1):
+        v = v + v[:, np.arange(64) ^ o]
+    r = np.float32(1) / np.sqrt(v[:, :1] / np.float32(hidden) + np.float32(1e-12), dtype=np.float32)
+    want = (x.astype(np.float32) * r * w.astype(np.float32)).astype(np.float16)
+    out = hip_ctx.alloc(x.nbytes)
+    hip_ctx.rmsnorm_f16(hip_ctx.to_device(x), hip_ctx.to_device(w), out, 6, hidden, 1e-12)
+    assert np.array_equal(out.download(x.shape, np.float16).view(np.uint16), want.view(np.uint16))
+    # ... and through a product with the identity, which normalises on its own
+    eye = hip_ctx.prepack_w8a16(np.eye(hidden, dtype=np.int8)[: hidden // 16 * 16], np.ones(hidden // 16 * 16, np.float32)) if hidden % 64 == 0 else None
+    if eye:
+        y = hip_ctx.alloc(6 * hidden * 4)
+        hip_ctx.rmsnorm_w8a16_gemm(hip_ctx.to_device(x), hip_ctx.to_device(w), 1e-12, eye, y, 6, out_dtype=rt.DT_F32)
+        assert np.array_equal(y.download((6, hidden), np.float32), want.astype(np.float32))
