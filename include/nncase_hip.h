@@ -602,7 +602,9 @@ NNCASE_HIP_API int nncase_hip_add_i32(nncase_hip_ctx_t *ctx, int32_t *x_dev, int
  * nncase_hip_function_capture() the same sequence is replayed as one HIP
  * graph launch (the operands must stay where they were when captured).
  * Operand buffers and weights stay owned by the caller and must outlive the
- * function.
+ * function.  Operators recorded one behind the other may share a launch where
+ * that is quicker (max pools and their concat, a depthwise convolution and the
+ * 1x1 convolutions behind it); every result is stored either way.
  */
 typedef struct nncase_hip_function nncase_hip_function_t;
 
@@ -729,11 +731,12 @@ NNCASE_HIP_API int nncase_hip_function_capture(nncase_hip_function_t *fn);
 /* Per-operator device time: every operator is enqueued `iterations` times
  * back to back between two HIP events recorded on the context's stream and
  * the mean duration in milliseconds is written to avg_ms[index] (the array
- * holds nncase_hip_function_size entries).  Blocks until done.  The HIP
+ * holds nncase_hip_function_size entries; of operators that share a launch the
+ * first has its time and the others 0).  Blocks until done.  The HIP
  * counterpart of the reference's per-op profiler
  * (src/Native/include/nncase/runtime/stackvm/op_profile.h:41-76). */
 NNCASE_HIP_API int nncase_hip_function_profile(nncase_hip_function_t *fn, int32_t iterations, float *avg_ms);
-/* Name of the kernel operator `index` launches, e.g.
+/* Name of the kernel operator `index` launches by itself, e.g.
  * "qconv_igemm<T=9,RG=2,rows16>"; NUL-terminated, truncated to `capacity`. */
 NNCASE_HIP_API int nncase_hip_function_op_kernel(nncase_hip_function_t *fn, int32_t index, char *name,
                                                  size_t capacity);

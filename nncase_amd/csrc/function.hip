@@ -197,6 +197,35 @@ static size_t find_pool_chain(const std::vector<Op> &ops, size_t at, MaxPoolChai
     return maxpool_chain_supported(*c) ? i + 1 - at : 0;
 }
 
+// A depthwise convolution and the pair that reads it, two 1x1 convolutions, or all three recorded one by one, from operator `at` on, as
+// one launch; *count is how many they are, 0 where they run one after the other.
+static int run_joined_convs(nncase_hip_function *fn, size_t at, size_t *count) {
+    *count = 0;
+    const std::vector<Op> &ops = fn->ops;
+    auto conv = [&](size_t i) { return i < ops.size() && ops[i].kind == Op::kConv && ops[i].lane == ops[at].lane; };
+    auto joined = [&](const Op &op) { return JoinedConv{(const uint8_t *)op.in0, op.weights, &op.conv, (uint8_t *)op.out}; };
+    if (!conv(at) || at + 1 >= ops.size()) return 0;
+    const bool depthwise = ops[at].weights->kind == nncase_hip_weights::kDepthwise;
+    const JoinedConv head = joined(ops[at]);
+    bool taken = false;
+    int rc = 0;
+    if (!depthwise) {
+        if (conv(at + 1)) rc = launch_joined_convs(fn->ctx, nullptr, nullptr, head, joined(ops[at + 1]), &taken);
+        if (taken) *count = 2;
+        return rc;
+    }
+    const Op &next = ops[at + 1];
+    if (next.kind == Op::kPair && !next.weights && next.lane == ops[at].lane) {
+        const JoinedConv first{(const uint8_t *)next.in0, nullptr, &next.conv, (uint8_t *)next.out}, second{(const uint8_t *)next.out, nullptr, &next.conv2, (uint8_t *)next.out2};
+        rc = launch_joined_convs(fn->ctx, &head, next.pair, first, second, &taken);
+        if (taken) *count = 2;
+    } else if (conv(at + 1) && conv(at + 2)) {
+        rc = launch_joined_convs(fn->ctx, &head, nullptr, joined(ops[at + 1]), joined(ops[at + 2]), &taken);
+        if (taken) *count = 3;
+    }
+    return rc;
+}
+
 // Runs the operators from `at` on that run as one launch; *next is the first behind them.
 static int run_ops(nncase_hip_function *fn, size_t at, size_t *next) {
     MaxPoolChain chain;
@@ -204,8 +233,10 @@ static int run_ops(nncase_hip_function *fn, size_t at, size_t *next) {
         *next = at + n;
         return launch_maxpool_chain(fn->ctx, chain);
     }
-    *next = at + 1;
-    return run_op(fn, fn->ops[at]);
+    size_t joined = 0;
+    if (int rc = run_joined_convs(fn, at, &joined)) return rc;
+    *next = at + std::max<size_t>(joined, 1);
+    return joined ? 0 : run_op(fn, fn->ops[at]);
 }
 
 static void drop_graph(nncase_hip_function *fn) {

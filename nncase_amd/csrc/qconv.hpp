@@ -140,6 +140,18 @@ struct PoolFront {
     int hw;
     nncase_hip_quant_param_t x_qp;
 };
+// A convolution of a recorded list.
+struct JoinedConv {
+    const uint8_t *x;
+    const nncase_hip_weights *weights;
+    const nncase_hip_conv2d_args_t *args;
+    uint8_t *y;
+};
+// Runs operators that follow one another as one launch, where they can be and it pays (*taken; else nothing is launched): a 3x3 depthwise
+// convolution (`dw`, may be null) and the two 1x1 convolutions of a pair, recorded as a pair (`pair`) or one by one (null).  All results are
+// stored, so nothing but the number of launches tells it from the operators one after the other.  (qpair.hip)
+int launch_joined_convs(nncase_hip_ctx *ctx, const JoinedConv *dw, const nncase_hip_qpair *pair, const JoinedConv &first, const JoinedConv &second,
+                        bool *taken);
 bool rows_shapes_ok(int in_channels, int out_channels, int64_t pixels);   // what rows_prepack packs and rows_path_taken takes
 bool pool_rows_ok(int in_channels, int out_channels, int64_t rows);        // ... behind a global average pool
 bool pool_front_pays(int rows, int hw, int channels);

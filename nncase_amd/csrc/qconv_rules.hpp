@@ -86,26 +86,43 @@ inline bool dma_pays(int64_t rows, int n, int ksteps, int compute_units) {
 
 // How a pair of dense 1x1 convolutions (k1 -> n1 -> n2 channels) is launched: a wave per channel tile of whichever convolution has more of
 // them in a workgroup (up to the variant's most), and enough workgroups to occupy the device: pixel tiles x ranges of the second
-// convolution's channel tiles.  With a depthwise stage, also enough threads that none of them walks more than four of the 16 pixels.
+// convolution's channel tiles.  With a depthwise stage, also enough threads that none of them walks more than four of the 16 pixels,
+// and tiles of 8 or 4 pixels where that still leaves a compute unit to every workgroup.
 struct PairSplit {
     int ranges, tiles_per_block, waves;
+    int pixels; // of a workgroup
+    bool once;  // no wave has a second tile or chunk of its reduction to come
     bool small; // the variant for short reductions
     bool apart; // not as a pair at all, but as two launches of the kernel for one convolution over few pixels
 };
 inline PairSplit split_pair(int64_t pixels, int k1, int n1, int n2, bool dw, int compute_units) {
     auto up = [](int64_t v, int64_t d) { return (int)((v + d - 1) / d); };
-    const int ks1 = up(k1, 64), ks2 = up(n1, 64), t1 = up(n1, 16), t2 = up(n2, 16), ptiles = up(std::max<int64_t>(pixels, 1), 16);
+    const int ks1 = up(k1, 64), ks2 = up(n1, 64), t1 = up(n1, 16), t2 = up(n2, 16);
     PairSplit s;
     s.small = ks1 <= 4 && ks2 <= 2;
-    const int max_waves = s.small ? 16 : 12, want = ptiles >= 512 ? 1 : 512 / ptiles;
-    s.tiles_per_block = up(t2, std::min(up(t2, max_waves), want));
-    s.ranges = up(t2, s.tiles_per_block);
-    s.waves = std::min(max_waves, std::max(t1, s.tiles_per_block));
-    if (dw) s.waves = std::min(max_waves, std::max(s.waves, up(k1, 64)));
+    const int max_waves = s.small ? 16 : 12;
+    int ptiles = 0;
+    auto tile = [&](int pt) {
+        s.pixels = pt, ptiles = up(std::max<int64_t>(pixels, 1), pt);
+        const int want = ptiles >= 512 ? 1 : 512 / ptiles;
+        s.tiles_per_block = up(t2, std::min(up(t2, max_waves), want));
+        s.ranges = up(t2, s.tiles_per_block);
+        s.waves = std::min(max_waves, std::max(t1, s.tiles_per_block));
+        if (dw) s.waves = std::min(max_waves, std::max(s.waves, up((int64_t)k1 * pt, pt == 16 ? 1024 : 256)));
+        s.once = t1 <= s.waves && s.tiles_per_block <= s.waves && ks1 <= 16 && ks2 <= 4;
+    };
+    tile(16);
+    if (dw)
+        for (int pt = 4; pt < 16; pt *= 2) {
+            tile(pt);
+            if (s.once && (int64_t)ptiles * s.ranges <= compute_units) break;
+            tile(16);
+        }
     // ... but no more than lets every workgroup be resident at once (a second round of workgroups doubles the
     // launch's latency chain; a wave that takes two channel tiles one after the other adds a fraction of it)
     const int occupancy = s.small ? 4 : 3; // waves per SIMD the variant is built for
     s.waves = std::max(1, std::min(s.waves, 4 * occupancy / std::max(up((int64_t)ptiles * s.ranges, compute_units), 1)));
+    s.once = s.once && t1 <= s.waves && s.tiles_per_block <= s.waves;
     // With more tiles between the two than a workgroup has waves, some waves take several tiles of the whole reduction, chunk by chunk:
     // so many trips to the weights in turn.  Apart where they are many, three tiles of few pixels, or more workgroups than units (us in a
     // chain, pair / apart: 49 pixels 960 -> 320 -> 1280, 6 trips, 8.4 / 7.3; 50 of 960 -> 512 -> 96, 8, 10.0 / 7.0; 57 of 448 -> 480 -> 512, 3
@@ -182,6 +199,31 @@ inline bool tile_kernel_pays(const TileLaunch &l, int compute_units) {
     if (l.stride_w == 2 && resident < 5) return false;
     if (l.pix < 128 && l.channels > 400 && resident < 4) return false;
     return l.pix > 32 || (l.ksteps >= 5 && launched <= 9ll * l.ksteps * compute_units);
+}
+
+// Whether two dense 1x1 convolutions, the second over the first one's result, are quicker as a pair than as two launches: while every
+// workgroup has a compute unit to itself, or several share one and each requests everything at once and repeats nothing (one range), or
+// what the workgroups stream between them is little (us of the two / the pair, 20 in a chain, with their depthwise stage where there is
+// one, joined where it is: 384 -> 64 -> 384 of 196 pixels 8.9 / 4.6, 576 -> 96 -> 576 of 1200 11.4 / 8.6 and, 300 workgroups, of 1600
+// 12.1 / 14.5, 960 -> 160 -> 960 of 588 11.7 / 9.7, 384 -> 64 -> 384 of 2400 9.9 / 12.4; one range 256 -> 128 -> 128 of 6272 8.2 / 4.7, 128 ->
+// 64 -> 64 of 12 800 7.0 / 4.6; little 32 -> 16 -> 96 of 12 544 9.6 / 6.9).  Of 1274 such pairs and triples the choice is 0.7 % off the quickest
+// of the three in the mean, 43 % at most (32 -> 100 -> 300 of 6400 9.3 / 6.5).
+inline bool pair_pays(int64_t pixels, int k1, int n1, int n2, int compute_units) {
+    const PairSplit s = split_pair(pixels, k1, n1, n2, false, compute_units);
+    const int64_t ptiles = (pixels + 15) / 16, blocks = ptiles * s.ranges;
+    if (blocks <= compute_units) return true;
+    if (ptiles > 4ll * compute_units) return false;
+    return (s.once && s.ranges == 1) || (s.small && ptiles * ((int64_t)k1 * n1 + (int64_t)n1 * n2) <= (4 << 20));
+}
+
+// Whether a depthwise stage in front joins the pair's launch: while the plan for it requests everything at once and no thread has more
+// than two and a half windows of four channels (us of the two launches / joined, over 20 in a chain: 192 -> 32 -> 192 of 784 pixels
+// 6.4 / 4.2, 384 -> 64 -> 384 of 196 6.7 / 4.6, 576 -> 96 -> 576 7.7 / 5.5, 960 -> 160 -> 960 of 49 8.8 / 7.4; 2.5 windows 960 -> 88 -> 912
+// of 363 8.4 / 8.0, 2.6 496 -> 8 -> 824 of 576 6.7 / 7.4, 4.2 800 -> 72 -> 928 of 507 8.2 / 10.6; several tiles a wave 592 -> 228 -> 160 of
+// 16 10.2 / 11.1, 528 -> 32 -> 812 of 1323 13.8 / 25.6).
+inline bool front_pays(int64_t pixels, int k1, int n1, int n2, int compute_units) {
+    const PairSplit s = split_pair(pixels, k1, n1, n2, true, compute_units);
+    return s.once && 2 * (int64_t)s.pixels * (k1 / 4) <= 5 * (int64_t)s.waves * 64;
 }
 
 } // namespace nnhip

@@ -6,7 +6,7 @@
 // launch-latency-bound kernels of a few microseconds; here the few-channel tensor between them stays in LDS (it is
 // also stored: a later residual add reads it), and the second product starts as soon as the first's tile exists.
 //
-// Work split: a workgroup owns 16 pixels and a range of conv_b's channel tiles.  It computes ALL of conv_a for its
+// Work split: a workgroup owns 16 pixels (8 or 4 behind a depthwise convolution) and a range of conv_b's channel tiles.  It computes ALL of conv_a for its
 // pixels (every workgroup of a pixel tile repeats that: the reduction is the cheap side of the pair and recomputing
 // keeps enough workgroups alive on 7x7 and 14x14 maps), requantises it exactly as nncase_hip_qconv2d does, and
 // multiplies the LDS tile with its range of conv_b.  Results are bit-identical to the two nncase_hip_qconv2d calls.
@@ -42,16 +42,15 @@ typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int kPairMaxK1 = 1024;  // x channels
 constexpr int kPairMaxN1 = 512;   // y1 channels
+constexpr int kPairMaxPixelTiles = 1024; // (of 16: four to a compute unit, see pair_pays)
 constexpr int kRowPad = 16;       // bytes between LDS rows beyond the padded reduction (spreads the 16 rows over the banks)
 
 // bytes of an LDS row: the reduction rounded up to whole chunks of `chunk` k-steps, and the pad
 __host__ __device__ constexpr int pair_row_bytes(int ksteps, int chunk) { return (ksteps + chunk - 1) / chunk * chunk * 64 + kRowPad; }
 
-// k-steps that an LDS row is rounded up to, of a kernel that requests kc fragments at a time
-__host__ __device__ constexpr int pair_chunk(int kc) { return kc > 8 ? 4 : kc; }
-
 struct PairArgs {
     const uint8_t *x;
+    uint8_t *y0;           // of the depthwise convolution, where its result is stored too
     uint8_t *y1, *y2;
     const uint8_t *wa, *wb;
     const int32_t *bias_a, *wsum_a, *bias_b, *wsum_b;
@@ -71,6 +70,8 @@ struct PairArgs {
     const int32_t *dw_bias, *dw_wsum; // [k1]; sum over the taps of w - zw
     int in_h, in_w, out_w, out_hw, stride, pad_h, pad_w;
     FastDiv d_out_hw, d_out_w;
+    FastDiv d_quads;       // four channels of k1
+    int dw_groups;         // pixels that the workgroup's threads cover at a time, or 0: fewer threads than quads
     int dw_zx;
     Epilogue ep_dw;
     // the second convolution alone (qpointwise_rows_kernel): x holds ITS input rows [m][n1]; its result may leave as the
@@ -98,17 +99,11 @@ template <int KC> struct TileLoads {
 };
 
 // Loads KC weight fragments of one tile from k-step ks0 on; past the tile's last k-step the last one is loaded again
-// (the activation tile is zero there, so what such a fragment holds does not matter, and no lane branches).  Of long chunks only
-// the groups of kPairGroup that hold any of the reduction.
-constexpr int kPairGroup = 4;
+// (the activation tile is zero there, so what such a fragment holds does not matter, and no lane branches).
 template <int KC> __device__ __forceinline__ void load_chunk(v4i (&f)[KC], const uint8_t *w, int tile, int ks0, int ksteps, int lane) {
     const v4i *src = reinterpret_cast<const v4i *>(w) + (size_t)tile * ksteps * 64 + lane;
 #pragma unroll
-    for (int c0 = 0; c0 < KC; c0 += kPairGroup)
-        if (c0 == 0 || KC <= 8 || ks0 + c0 < ksteps) {
-#pragma unroll
-            for (int c = c0; c < c0 + kPairGroup && c < KC; c++) f[c] = src[min(ks0 + c, ksteps - 1) * 64];
-        }
+    for (int c = 0; c < KC; c++) f[c] = src[min(ks0 + c, ksteps - 1) * 64];
 }
 
 template <int KC, bool FIRST>
@@ -122,11 +117,12 @@ __device__ __forceinline__ void load_tile(TileLoads<KC> &l, const PairArgs &a, i
 }
 
 // A tile's accumulators to its results: `sum` is the sum of this lane's pixel's row (the same in every lane of it).
-// ALONE: of one convolution by itself, which may add a residual.
+// ALONE: of one convolution by itself, which may add a residual.  row: of the lane's pixel in `ys`; live: it is a pixel of the tensor, and
+// this lane the one to store it.
 template <bool FIRST, bool ALONE = false>
 __device__ __forceinline__ void finish_tile(const PairArgs &a, int t, const v4i &acc, int32_t sum, const v4i &bias, const v4i &ws, uint32_t rv, uint8_t *ys,
-                                            int sy, const uint8_t *lut, int lane, int p, bool store_y1) {
-    const int j = lane & 15, g = lane >> 4;
+                                            int sy, const uint8_t *lut, int lane, int row, int p, bool live, bool store_y1) {
+    const int g = lane >> 4;
     const int zx = FIRST ? a.zxa : a.zxb, zw = FIRST ? a.zwa : a.zwb;
     const Epilogue &ep = FIRST ? a.ep_a : a.ep_b;
     const int32_t kzz = (FIRST ? a.k1 : a.n1) * zx * zw;
@@ -140,10 +136,10 @@ __device__ __forceinline__ void finish_tile(const PairArgs &a, int t, const v4i 
     if constexpr (FIRST) {
         if (ch < a.n1) {
             if (a.rep_a.res) q = residual4_packed(q, rv, a.rep_a);
-            *reinterpret_cast<uint32_t *>(ys + j * sy + ch) = q ^ 0x80808080u;
-            if (store_y1 && p < a.m) *reinterpret_cast<uint32_t *>(a.y1 + (size_t)p * a.n1 + ch) = q;
+            *reinterpret_cast<uint32_t *>(ys + row * sy + ch) = q ^ 0x80808080u;
+            if (store_y1 && live) *reinterpret_cast<uint32_t *>(a.y1 + (size_t)p * a.n1 + ch) = q;
         }
-    } else if (ch < a.n2 && p < a.m) {
+    } else if (ch < a.n2 && live) {
         if (ALONE && a.rep_b.res) q = residual4_packed(q, rv, a.rep_b);
         if (ALONE && a.deq) { // the Dequantize behind the convolution: one float per channel
             u32x4 o;
@@ -158,10 +154,10 @@ __device__ __forceinline__ void finish_tile(const PairArgs &a, int t, const v4i 
 
 // One convolution of the pair for this wave's channel tiles first, first + step, ... below end.  `rows` is the LDS
 // activation tile ([16][stride] s8); `cur` holds the loads of the first tile already.  FIRST: results go to the LDS tile
-// `ys` as s8 (and to y1 when store_y1); else to y2.  ONCE: there is one tile, and its reduction is one chunk.  The sum of a row, which
+// `ys` as s8 (and to y1 when store_y1); else to y2.  The sum of a row, which
 // the weight zero point multiplies, is a second product of the same operands with ones, beside the first (by itself, before it, it
 // was 0.3 us of a launch).
-template <int KC, bool FIRST, bool ONCE>
+template <int KC, bool FIRST>
 __device__ __forceinline__ void run_stage(const PairArgs &a, const uint8_t *rows, int stride, uint8_t *ys, int sy, const uint8_t *lut, int first,
                                           int step, int end, TileLoads<KC> &cur, int lane, int p, bool store_y1) {
     const int j = lane & 15, g = lane >> 4;
@@ -171,33 +167,25 @@ __device__ __forceinline__ void run_stage(const PairArgs &a, const uint8_t *rows
     v4i bias = cur.bias, ws = cur.wsum; // the constants of a tile arrive with its first chunk and are used after its last
     uint32_t rv = cur.res;
 #pragma unroll 1
-    for (int t = first; ONCE || t < end; t += step) {
+    for (int t = first; t < end; t += step) {
         v4i acc = {0, 0, 0, 0}, rs = {0, 0, 0, 0};
 #pragma unroll 1
-        for (int ks0 = 0; ONCE || ks0 < ksteps; ks0 += KC) {
+        for (int ks0 = 0; ks0 < ksteps; ks0 += KC) {
             // what follows this chunk (the tile's next one, else the next tile's first) travels while this one multiplies;
             // one wave-uniform branch around all of it: behind the last chunk nothing is requested, so nothing is waited for
             const bool more = ks0 + KC < ksteps;
             TileLoads<KC> nxt;
-            if constexpr (!ONCE) {
-                if (more || t + step < end) load_tile<KC, FIRST>(nxt, a, more ? t : t + step, more ? ks0 + KC : 0, lane, p);
-                if (!more) bias = cur.bias, ws = cur.wsum, rv = cur.res;
+            if (more || t + step < end) load_tile<KC, FIRST>(nxt, a, more ? t : t + step, more ? ks0 + KC : 0, lane, p);
+            if (!more) bias = cur.bias, ws = cur.wsum, rv = cur.res;
+#pragma unroll
+            for (int c = 0; c < KC; c++) {
+                const v4i xf = *reinterpret_cast<const v4i *>(row + (ks0 + c) * 64);
+                acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(cur.frag[c], xf, acc, 0, 0, 0);
+                rs = __builtin_amdgcn_mfma_i32_16x16x64_i8(ones, xf, rs, 0, 0, 0);
             }
-#pragma unroll
-            for (int c0 = 0; c0 < KC; c0 += kPairGroup)
-                if (c0 == 0 || KC <= 8 || c0 < ksteps) {
-#pragma unroll
-                    for (int c = c0; c < c0 + kPairGroup && c < KC; c++) {
-                        const v4i xf = *reinterpret_cast<const v4i *>(row + (ks0 + c) * 64);
-                        acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(cur.frag[c], xf, acc, 0, 0, 0);
-                        rs = __builtin_amdgcn_mfma_i32_16x16x64_i8(ones, xf, rs, 0, 0, 0);
-                    }
-                }
-            if constexpr (ONCE) break;
-            else cur = nxt;
+            cur = nxt;
         }
-        finish_tile<FIRST>(a, t, acc, rs[0], bias, ws, rv, ys, sy, lut, lane, p, store_y1);
-        if constexpr (ONCE) break;
+        finish_tile<FIRST>(a, t, acc, rs[0], bias, ws, rv, ys, sy, lut, lane, j, p, p < a.m, store_y1);
     }
 }
 
@@ -270,15 +258,11 @@ __device__ __forceinline__ void dw_stage(const PairArgs &a, uint8_t *xs, int sx,
 // KA / KB: weight fragments a wave requests at a time for the first / second convolution (each twice in registers).
 // MAXW: most waves a workgroup is launched with; OCC: waves per SIMD the register budget is held to.
 // DW: a 3x3 depthwise convolution produces the pixel tile (dw_stage).
-// ONCE: no wave has more than one tile of either convolution, and KA and KB hold their reductions: everything a wave will multiply is
-// requested at the start.  These launches are bound by their chain of memory round trips (us of one in a chain of them, with chunks of 8
-// k-steps and the rows' sums ahead / so: 384 -> 64 -> 384 over 14 x 14 4.64 / 4.40, 576 -> 96 -> 576 6.00 / 5.05, 960 -> 160 -> 960 over 7 x 7
-// 6.95 / 6.3; MobileNetV2 of one image 167.4 -> 159.3).
-template <int KA, int KB, int MAXW, int OCC, bool DW, bool ONCE>
+template <int KA, int KB, int MAXW, int OCC, bool DW>
 __global__ __launch_bounds__(MAXW * 64, OCC) void qpointwise_pair_kernel(const PairArgs a) {
     extern __shared__ __align__(16) uint8_t smem[];
     // rows hold whole chunks of k-steps, zero past the real reduction
-    const int sx = pair_row_bytes(a.ks1, pair_chunk(KA)), sy = pair_row_bytes(a.ks2, pair_chunk(KB));
+    const int sx = pair_row_bytes(a.ks1, KA), sy = pair_row_bytes(a.ks2, KB);
     uint8_t *xs = smem;              // [16][sx]  x - 128
     uint8_t *ys = xs + 16 * sx;      // [16][sy]  y1 - 128
     uint8_t *lut_a = ys + 16 * sy;   // 256 bytes each
@@ -305,7 +289,7 @@ __global__ __launch_bounds__(MAXW * 64, OCC) void qpointwise_pair_kernel(const P
         }
     } else {
         const u32x4 none = {0x80808080u, 0x80808080u, 0x80808080u, 0x80808080u};
-        constexpr int U = KA > 4 ? 2 : 1; // (both requested before the first is waited for: 16 pixels of 960 channels are two a thread)
+        constexpr int U = KA > 4 ? 2 : 1;
 #pragma unroll 1
         for (int e0 = tid; e0 < 16 * pieces; e0 += U * threads) {
             u32x4 v[U];
@@ -332,10 +316,257 @@ __global__ __launch_bounds__(MAXW * 64, OCC) void qpointwise_pair_kernel(const P
     }
     __syncthreads();
     // the first convolution over the whole of its channels, into LDS (and, from the first channel range, into y1)
-    if (wave < a.t1) run_stage<KA, true, ONCE>(a, xs, sx, ys, sy, a.lut_a ? lut_a : nullptr, wave, waves, a.t1, la, lane, p, blockIdx.y == 0);
+    if (wave < a.t1) run_stage<KA, true>(a, xs, sx, ys, sy, a.lut_a ? lut_a : nullptr, wave, waves, a.t1, la, lane, p, blockIdx.y == 0);
     __syncthreads();
     // the second: this workgroup's channel tiles from the LDS tile
-    if (b_first + wave < b_end) run_stage<KB, false, ONCE>(a, ys, sy, nullptr, 0, a.lut_b ? lut_b : nullptr, b_first + wave, waves, b_end, lb, lane, p, false);
+    if (b_first + wave < b_end) run_stage<KB, false>(a, ys, sy, nullptr, 0, a.lut_b ? lut_b : nullptr, b_first + wave, waves, b_end, lb, lane, p, false);
+}
+
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t pair_resource(const void *base, uint32_t bytes) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(base), 0, (int)bytes, 0x00020000);
+}
+
+// The kernel's arguments that its epilogues take, loaded where this is called and all together.  With what a launch needs at its start
+// there are more than scalar registers: left to itself the compiler loads everything first and puts it in lanes of vector registers and
+// out again, eight scalar round trips in front of the first request; or, kept from that, each where a branch first uses it.
+__device__ __forceinline__ void gather(Epilogue &to, const Epilogue &ep) {
+    to.mult = ep.mult, to.sy = ep.sy, to.rsy = ep.rsy, to.zy = ep.zy, to.qlo = ep.qlo, to.qhi = ep.qhi, to.c1 = ep.c1, to.c2 = ep.c2;
+    to.fast = ep.fast, to.full = ep.full;
+}
+template <bool FRONT> __device__ __forceinline__ PairArgs gather_epilogues() {
+    auto p = (const __attribute__((address_space(4))) PairArgs *)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(p));
+    const PairArgs &a = *(const PairArgs *)p;
+    PairArgs l; // (what is not assigned here is not used)
+    if constexpr (FRONT) { // the depthwise stage's
+        gather(l.ep_dw, a.ep_dw);
+        l.dw_zx = a.dw_zx, l.y0 = a.y0;
+        asm volatile("" ::"s"(l.ep_dw.mult), "s"(l.ep_dw.sy), "s"(l.ep_dw.rsy), "s"(l.ep_dw.zy), "s"(l.ep_dw.qlo), "s"(l.ep_dw.qhi), "s"(l.ep_dw.c1),
+                     "s"(l.ep_dw.c2), "s"(l.ep_dw.fast), "s"(l.ep_dw.full), "s"(l.dw_zx), "s"(l.y0));
+    } else {
+        gather(l.ep_a, a.ep_a), gather(l.ep_b, a.ep_b), gather(l.rep_a.sum, a.rep_a.sum);
+        l.rep_a.res = a.rep_a.res, l.rep_a.zy = a.rep_a.zy, l.rep_a.sy = a.rep_a.sy, l.rep_a.zr = a.rep_a.zr, l.rep_a.sr = a.rep_a.sr;
+        l.y1 = a.y1, l.y2 = a.y2, l.k1 = a.k1, l.n1 = a.n1, l.n2 = a.n2, l.ldy = a.ldy, l.y_coff = a.y_coff;
+        l.zxa = a.zxa, l.zwa = a.zwa, l.zxb = a.zxb, l.zwb = a.zwb;
+        asm volatile("" ::"s"(l.ep_a.mult), "s"(l.ep_a.sy), "s"(l.ep_a.rsy), "s"(l.ep_a.zy), "s"(l.ep_a.qlo), "s"(l.ep_a.qhi), "s"(l.ep_a.c1), "s"(l.ep_a.c2),
+                     "s"(l.ep_a.fast), "s"(l.ep_a.full), "s"(l.rep_a.sum.sy), "s"(l.rep_a.sum.rsy), "s"(l.rep_a.sum.zy), "s"(l.rep_a.sum.qlo),
+                     "s"(l.rep_a.sum.qhi), "s"(l.rep_a.res), "s"(l.rep_a.zy), "s"(l.rep_a.sy), "s"(l.rep_a.zr), "s"(l.rep_a.sr), "s"(l.y1), "s"(l.zxa), "s"(l.zwa));
+        asm volatile("" ::"s"(l.ep_b.mult), "s"(l.ep_b.sy), "s"(l.ep_b.rsy), "s"(l.ep_b.zy), "s"(l.ep_b.qlo), "s"(l.ep_b.qhi), "s"(l.ep_b.c1), "s"(l.ep_b.c2),
+                     "s"(l.ep_b.fast), "s"(l.ep_b.full), "s"(l.y2), "s"(l.n2), "s"(l.zxb), "s"(l.zwb), "s"(l.ldy), "s"(l.y_coff));
+    }
+    return l;
+}
+
+// A window of the depthwise convolution as dw_fetch's, in two halves: the requests, and the taps outside the image.  (The input is less
+// than 2 GiB.)
+struct DwWindow {
+    uint32_t x[9];
+    bool in_y[3], in_x[3];
+};
+__device__ __forceinline__ void dw_request(DwWindow &w, const PairArgs &a, int px, int c4) {
+    px = min(px, a.m - 1);
+    const int n = (int)fastdiv((uint32_t)px, a.d_out_hw), rem = px - n * a.out_hw;
+    const int oy = (int)fastdiv((uint32_t)rem, a.d_out_w), ox = rem - oy * a.out_w;
+    const int iy0 = oy * a.stride - a.pad_h, ix0 = ox * a.stride - a.pad_w;
+    int iy[3], ix[3];
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+        iy[k] = min(max(iy0 + k, 0), a.in_h - 1), w.in_y[k] = iy[k] == iy0 + k;
+        ix[k] = min(max(ix0 + k, 0), a.in_w - 1), w.in_x[k] = ix[k] == ix0 + k;
+    }
+    const uint32_t pitch = (uint32_t)a.in_w * (uint32_t)a.k1;
+    uint32_t ro[3], co[3]; // (a clamped position is the last one's or one further: one multiplication each, which takes four times an addition)
+    ro[0] = (uint32_t)(n * a.in_h + iy[0]) * pitch, co[0] = (uint32_t)ix[0] * (uint32_t)a.k1 + (uint32_t)c4;
+#pragma unroll
+    for (int k = 1; k < 3; k++) ro[k] = ro[k - 1] + (iy[k] != iy[k - 1] ? pitch : 0u), co[k] = co[k - 1] + (ix[k] != ix[k - 1] ? (uint32_t)a.k1 : 0u);
+#pragma unroll
+    for (int t = 0; t < 9; t++) w.x[t] = *reinterpret_cast<const uint32_t *>(a.x + (size_t)(ro[t / 3] + co[t % 3]));
+}
+struct DwTaps {
+    uint32_t w01[9], w23[9];
+    v4i bias, ws;
+};
+__device__ __forceinline__ void dw_request_taps(DwTaps &d, const PairArgs &a, int c4) {
+#pragma unroll
+    for (int t = 0; t < 9; t++) {
+        const uint2 wv = *reinterpret_cast<const uint2 *>(a.dw_w + (uint32_t)(t * a.k1 + c4));
+        d.w01[t] = wv.x, d.w23[t] = wv.y;
+    }
+    d.bias = *reinterpret_cast<const v4i *>(a.dw_bias + c4), d.ws = *reinterpret_cast<const v4i *>(a.dw_wsum + c4);
+}
+__device__ __forceinline__ uint32_t dw_codes(const DwWindow &w, const DwTaps &d, const PairArgs &a) {
+    const uint32_t zx4 = (uint32_t)a.dw_zx * 0x01010101u;
+    int32_t acc[4];
+#pragma unroll
+    for (int c = 0; c < 4; c++) acc[c] = d.bias[c] - a.dw_zx * d.ws[c];
+#pragma unroll
+    for (int t = 0; t < 9; t++) {
+        const uint32_t x = w.in_y[t / 3] && w.in_x[t % 3] ? w.x[t] : zx4;
+        const uint32_t x01 = __builtin_amdgcn_perm(0, x, 0x0c010c00u), x23 = __builtin_amdgcn_perm(0, x, 0x0c030c02u);
+        acc[0] = mad16_lo(x01, d.w01[t], acc[0]);
+        acc[1] = mad16_hi(x01, d.w01[t], acc[1]);
+        acc[2] = mad16_lo(x23, d.w23[t], acc[2]);
+        acc[3] = mad16_hi(x23, d.w23[t], acc[3]);
+    }
+    return requant4_u8_packed(acc, a.ep_dw);
+}
+
+// The same where no wave has more than one tile of either convolution and KA and KB fragments hold their reductions.  Such a launch is
+// bound by its chain of waits and by the instructions between them, so a wave's requests come first, in the order in which they are
+// needed, and where a wave has none of a kind it skips them as a whole (a load past the end of a buffer resource fetches nothing, but
+// holds up the loads behind it like any other: a wave's spare fragments are few).
+//
+// PT: pixels of a workgroup, 16, 8 or 4.  The matrix instruction's 16 columns hold them 16 / PT times over; what is saved is the
+// depthwise stage, which is vector work on one compute unit, by leaving it to more of them.  us from the first wave's start to the last
+// store, in a MobileNetV2 step of one image, before / now: 192 -> 32 -> 192 of 784 pixels with the stage 4.6 / 3.3, 192 -> 64 -> 384 of 196
+// 4.5 / 3.2, without it 384 -> 64 -> 384 3.5 / 2.9; a launch of its own for 384 channels' stage, 1.4 us and a gap of 1.6, is now 0.8 us of
+// the pair's.  The step: 160.9 -> 125.7.
+template <int KA, int KB, int MAXW, int OCC, bool DW, int PT>
+__global__ __launch_bounds__(MAXW * 64, OCC) void qpointwise_pair_once_kernel(const PairArgs a) {
+    static_assert(DW || PT == 16, "smaller tiles are for the depthwise stage");
+    extern __shared__ __align__(16) uint8_t smem[];
+    const int ks1 = a.ks1, ks2 = a.ks2, k1 = a.k1, n1 = a.n1;
+    const int sx = pair_row_bytes(ks1, 1), sy = pair_row_bytes(ks2, 1);
+    uint8_t *const xs = smem;              // [PT][sx]  x - 128
+    uint8_t *const ys = xs + PT * sx;      // [PT][sy]  y1 - 128
+    uint8_t *const lut_a = ys + PT * sy;   // 256 bytes each
+    uint8_t *const lut_b = lut_a + 256;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), threads = blockDim.x, waves = threads >> 6;
+    const int g = lane >> 4, row = lane & (PT - 1);
+    const int p0 = (int)blockIdx.x * PT, p = p0 + row, pixels = min(PT, a.m - p0);
+    const bool live = (lane & 15) < PT && p < a.m;
+    const int tile_b = (int)blockIdx.y * a.tiles_per_block + wave;
+    const bool works_a = wave < a.t1, works_b = wave < a.tiles_per_block && tile_b < a.t2; // uniform
+    const bool has_lut_a = a.lut_a != nullptr, has_lut_b = a.lut_b != nullptr;
+
+    // ---- requests: a wave's weights and constants of the first convolution ---------------------------------
+    v4i fa[KA], fb[KB], bias_a, wsum_a, bias_b, wsum_b;
+    uint32_t rv = 0;
+    const int ch_a = wave * 16 + g * 4, ch_b = tile_b * 16 + g * 4;
+    auto request_a = [&]() __attribute__((always_inline)) { // (where works_a; k-steps past the reduction: past the end)
+        const auto w = pair_resource(a.wa + (size_t)wave * ks1 * 1024, (uint32_t)ks1 * 1024u);
+#pragma unroll
+        for (int c = 0; c < KA; c++) fa[c] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(w, lane * 16 + c * 1024, 0, 0));
+        bias_a = *reinterpret_cast<const v4i *>(a.bias_a + ch_a), wsum_a = *reinterpret_cast<const v4i *>(a.wsum_a + ch_a);
+        const auto residual = pair_resource(a.rep_a.res + (a.rep_a.res ? (size_t)p0 * n1 : 0), a.rep_a.res ? (uint32_t)(pixels * n1) : 0u);
+        rv = __builtin_amdgcn_raw_buffer_load_b32(residual, row * n1 + ch_a, 0, 0); // (of channels past N1: the next pixel's, unused)
+    };
+    // ... and of the second, behind the pixels: there is the first convolution's time for them
+    uint32_t ta, tb;
+    auto request_b = [&]() __attribute__((always_inline)) {
+        const auto w = pair_resource(a.wb + (size_t)(works_b ? tile_b : 0) * ks2 * 1024, works_b ? (uint32_t)ks2 * 1024u : 0u);
+#pragma unroll
+        for (int c = 0; c < KB; c++) fb[c] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(w, lane * 16 + c * 1024, 0, 0));
+        const uint32_t bytes_b = works_b ? (uint32_t)a.t2 * 64u : 0u;
+        bias_b = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(pair_resource(a.bias_b, bytes_b), ch_b * 4, 0, 0));
+        wsum_b = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(pair_resource(a.wsum_b, bytes_b), ch_b * 4, 0, 0));
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    ta = __builtin_amdgcn_raw_buffer_load_b32(pair_resource(a.lut_a, wave == 0 && has_lut_a ? 256u : 0u), lane * 4, 0, 0);
+    tb = __builtin_amdgcn_raw_buffer_load_b32(pair_resource(a.lut_b, wave == waves - 1 && has_lut_b ? 256u : 0u), lane * 4, 0, 0);
+
+    // ---- the pixel tile as s8 (x - 128); bytes past K are zero --------------------------------------------
+    if constexpr (DW) {
+        // A thread per window of four channels, in the last waves: the first ones bring the first convolution's weights in.
+        const int quads = k1 >> 2, ftid = threads - 1 - tid, fwave = waves - 1 - wave;
+        int pg = 0, quad = ftid;
+        if (a.dw_groups > 0) pg = (int)fastdiv((uint32_t)ftid, a.d_quads), quad = ftid - pg * quads;
+        bool mine = a.dw_groups > 0 ? pg < a.dw_groups : ftid < quads;
+        const bool fronts = fwave * 64 < quads * max(a.dw_groups, 1); // uniform
+        DwWindow win;
+        DwTaps taps;
+        if (fronts) {
+            const int c4 = mine ? quad * 4 : 0;
+            dw_request(win, a, p0 + pg, c4);
+            dw_request_taps(taps, a, c4);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        if (works_a) request_a();
+        const PairArgs later = gather_epilogues<true>(); // (the trip beside the others')
+        for (int q = quad, r = pg; fronts;) { // (one turn where there is a thread per window)
+            const uint32_t code = dw_codes(win, taps, later);
+            if (mine) {
+                *reinterpret_cast<uint32_t *>(xs + r * sx + q * 4) = (p0 + r < a.m ? code : 0x80808080u) ^ 0x80808080u;
+                if (later.y0 && blockIdx.y == 0 && p0 + r < a.m) *reinterpret_cast<uint32_t *>(later.y0 + (size_t)(p0 + r) * k1 + q * 4) = code;
+            }
+            r += max(a.dw_groups, 1);
+            bool more = r < PT;
+            if (a.dw_groups == 0 && !more) q += threads, r = 0, more = q < quads, mine = more;
+            if (!__any(mine && more)) break;
+            mine = mine && more;
+            const int c4 = mine ? q * 4 : 0;
+            dw_request(win, a, p0 + min(r, PT - 1), c4);
+            if (a.dw_groups == 0) dw_request_taps(taps, a, c4);
+        }
+        request_b();
+        for (int r = wave; r < PT && k1 < ks1 * 64; r += waves)
+            if (k1 + lane * 4 < ks1 * 64) *reinterpret_cast<uint32_t *>(xs + r * sx + k1 + lane * 4) = 0u;
+    } else {
+        constexpr int U = KA > 8 ? 2 : 1; // pieces of 16 bytes that a thread brings in at once
+        const int pieces = ks1 * 4;       // ... of a row, past K as well
+        const auto rows = pair_resource(a.x + (size_t)p0 * k1, (uint32_t)(pixels * k1));
+        u32x4 v[U];
+        auto request_x = [&](int e0) __attribute__((always_inline)) {
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                const uint32_t e = (uint32_t)(e0 + u * threads), r = fastdiv(e, a.d_pieces), c = e - r * (uint32_t)pieces;
+                v[u] = __builtin_amdgcn_raw_buffer_load_b128(rows, (int)(r * (uint32_t)k1 + c * 16u), 0, 0);
+            }
+        };
+        auto put_x = [&](int e0) __attribute__((always_inline)) {
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                const uint32_t e = (uint32_t)(e0 + u * threads), r = fastdiv(e, a.d_pieces), c = e - r * (uint32_t)pieces;
+                if (r < 16) *reinterpret_cast<u32x4 *>(xs + r * sx + c * 16) = (int)c * 16 < k1 ? v[u] ^ 0x80808080u : u32x4{0u, 0u, 0u, 0u};
+            }
+        };
+        request_x(tid);
+        __builtin_amdgcn_sched_barrier(0);
+        if (works_a) { // (each with the pixels' first turn: behind a join the wait for them would be one for the weights too)
+            request_a();
+            __builtin_amdgcn_sched_barrier(0);
+            put_x(tid);
+        } else {
+            put_x(tid);
+        }
+#pragma unroll 1
+        for (int e0 = tid + U * threads; e0 - tid < 16 * pieces; e0 += U * threads) request_x(e0), put_x(e0);
+        request_b();
+    }
+    const PairArgs later = gather_epilogues<false>();
+    for (int r = wave; r < PT && n1 < ks2 * 64; r += waves)
+        if (n1 + lane * 4 < ks2 * 64) *reinterpret_cast<uint32_t *>(ys + r * sy + n1 + lane * 4) = 0u;
+    if (wave == 0 && has_lut_a) reinterpret_cast<uint32_t *>(lut_a)[lane] = ta;
+    if (wave == waves - 1 && has_lut_b) reinterpret_cast<uint32_t *>(lut_b)[lane] = tb;
+    __syncthreads();
+
+    // ---- products: the first over the whole of its channels into LDS (and, from the first channel range, into y1), then the second ----
+    const v4i ones = {0x01010101, 0x01010101, 0x01010101, 0x01010101};
+    if (works_a) {
+        const uint8_t *from = xs + row * sx + g * 16;
+        v4i acc = {0, 0, 0, 0}, rs = {0, 0, 0, 0};
+#pragma unroll
+        for (int c = 0; c < KA; c++)
+            if (c < ks1) { // uniform
+                const v4i xf = *reinterpret_cast<const v4i *>(from + c * 64);
+                acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(fa[c], xf, acc, 0, 0, 0);
+                rs = __builtin_amdgcn_mfma_i32_16x16x64_i8(ones, xf, rs, 0, 0, 0);
+            }
+        finish_tile<true>(later, wave, acc, rs[0], bias_a, wsum_a, rv, ys, sy, has_lut_a ? lut_a : nullptr, lane, row, p, live, blockIdx.y == 0);
+    }
+    __syncthreads();
+    if (works_b) {
+        const uint8_t *from = ys + row * sy + g * 16;
+        v4i acc = {0, 0, 0, 0}, rs = {0, 0, 0, 0};
+#pragma unroll
+        for (int c = 0; c < KB; c++)
+            if (c < ks2) { // uniform
+                const v4i xf = *reinterpret_cast<const v4i *>(from + c * 64);
+                acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(fb[c], xf, acc, 0, 0, 0);
+                rs = __builtin_amdgcn_mfma_i32_16x16x64_i8(ones, xf, rs, 0, 0, 0);
+            }
+        finish_tile<false>(later, tile_b, acc, rs[0], bias_b, wsum_b, 0u, nullptr, 0, has_lut_b ? lut_b : nullptr, lane, row, p, live, false);
+    }
 }
 
 // One dense 1x1 convolution over a few rows (pixels): the second stage of the pair kernel alone.  A workgroup stages 16
@@ -438,7 +669,7 @@ template <bool POOL> __global__ __launch_bounds__(kRowsWaves * 64, 3) void qpoin
                 acc += accs[at], rs[0] += sums[at];
             }
     }
-    if (works && part == 0) finish_tile<false, true>(a, tile, acc, rs[0], bias, ws, rv, nullptr, 0, a.lut_b ? lut_b : nullptr, lane, p, false);
+    if (works && part == 0) finish_tile<false, true>(a, tile, acc, rs[0], bias, ws, rv, nullptr, 0, a.lut_b ? lut_b : nullptr, lane, lane & 15, p, p < a.m, false);
 }
 
 // [tile][k-step][lane][16] s8 of w - 128, zero beyond the real channels / reduction
@@ -566,7 +797,13 @@ bool pool_rows_ok(int in_channels, int out_channels, int64_t rows) { return rows
 // per workgroup the separate pool kernel, which spreads over the device, is the faster one.
 bool pool_front_pays(int rows, int hw, int channels) { return (int64_t)std::min(rows, 16) * hw * channels <= (128 << 10); }
 
-bool rows_wanted(const nncase_hip_weights *w) { return pointwise_weights(w) && rows_shapes_ok(w->in_channels, w->out_channels, w->pixels_hint); }
+// Also of what may become half of a pair with the operator recorded next to it (launch_joined_convs), up to the pixels where one pays.
+bool rows_wanted(const nncase_hip_weights *w) {
+    if (!pointwise_weights(w)) return false;
+    const bool pair_half = w->pixels_hint > 0 && w->pixels_hint <= 16 * kPairMaxPixelTiles && w->in_channels % 16 == 0 && w->out_channels % 4 == 0 &&
+                           w->in_channels <= kPairMaxK1;
+    return pair_half || rows_shapes_ok(w->in_channels, w->out_channels, w->pixels_hint);
+}
 
 // A block per channel tile: the tile's fragments as pack_pair_weights lays them out, its weight sums and its bias.
 constexpr int kRowsPackWaves = 4;
@@ -701,10 +938,10 @@ void nnhip::describe_pair(const nncase_hip_ctx *ctx, const nncase_hip_qpair *pr,
     snprintf(buf, cap, "%s", apart ? "qpointwise_rows+qpointwise_rows" : dw ? "dw3x3+qpointwise_pair_kernel" : "qpointwise_pair_kernel");
 }
 
-// dw / da: the depthwise convolution in front and its arguments, or null
+// dw / da: the depthwise convolution in front and its arguments, or null; y0_dev: where its result is stored too, or null
 static int launch_pair(nncase_hip_ctx *ctx, const char *who, const uint8_t *x_dev, const nncase_hip_weights *dw,
                        const nncase_hip_conv2d_args_t *da, const nncase_hip_qpair *pr, uint8_t *y1_dev, uint8_t *y2_dev,
-                       const nncase_hip_conv2d_args_t *fa, const nncase_hip_conv2d_args_t *sa) {
+                       const nncase_hip_conv2d_args_t *fa, const nncase_hip_conv2d_args_t *sa, uint8_t *y0_dev = nullptr) {
     NNHIP_REQUIRE(ctx, x_dev && pr && y1_dev && y2_dev && fa && sa, -EINVAL, "%s: null argument", who);
     NNHIP_REQUIRE(ctx, fa->batch > 0 && fa->in_h > 0 && fa->in_w > 0, -EINVAL, "%s: non-positive input shape", who);
     NNHIP_REQUIRE(ctx, sa->batch == fa->batch && sa->in_h == fa->in_h && sa->in_w == fa->in_w, -NNCASE_HIP_ERR_SHAPE_MISMATCH,
@@ -736,7 +973,7 @@ static int launch_pair(nncase_hip_ctx *ctx, const char *who, const uint8_t *x_de
 
     PairArgs a;
     memset(&a, 0, sizeof(a));
-    a.x = x_dev, a.y1 = y1_dev, a.y2 = y2_dev;
+    a.x = x_dev, a.y0 = y0_dev, a.y1 = y1_dev, a.y2 = y2_dev;
     a.wa = pr->d_wa, a.wb = pr->d_wb;
     a.bias_a = pr->d_bias_a, a.wsum_a = pr->d_wsum_a, a.bias_b = pr->d_bias_b, a.wsum_b = pr->d_wsum_b;
     a.lut_a = pr->first->d_post_lut, a.lut_b = pr->second->d_post_lut;
@@ -791,22 +1028,119 @@ static int launch_pair(nncase_hip_ctx *ctx, const char *who, const uint8_t *x_de
         a.x = y1_dev;
         return launch_rows(ctx, a, false);
     }
-    const dim3 grid((a.m + 15) / 16, split.ranges), block(waves * 64);
-    auto go = [&](auto kernel, int ka, int kb) {
-        const int sx = pair_row_bytes(a.ks1, pair_chunk(ka)), sy = pair_row_bytes(a.ks2, pair_chunk(kb));
+    const int pt = split.pixels;
+    const dim3 grid((a.m + pt - 1) / pt, split.ranges), block(waves * 64);
+    if (dw) {
+        a.d_quads = make_fastdiv((uint32_t)pr->k1 / 4);
+        a.dw_groups = std::min(waves * 64 / (pr->k1 / 4), pt);
+    }
+    auto go = [&](auto kernel, int ka, int kb) { // (rows of whole chunks)
+        const int sx = pair_row_bytes(a.ks1, ka), sy = pair_row_bytes(a.ks2, kb);
         a.d_pieces = make_fastdiv((uint32_t)(sx - kRowPad) / 16);
-        hipLaunchKernelGGL(kernel, grid, block, 16 * (size_t)(sx + sy) + 512, ctx->stream, a);
+        hipLaunchKernelGGL(kernel, grid, block, pt * (size_t)(sx + sy) + 512, ctx->stream, a);
     };
-    // Everything at once where no wave has a second tile or chunk to come (with a depthwise stage only for short reductions: longer
-    // ones have that in a launch of its own).
-    const bool one_tile = a.t1 <= waves && a.tiles_per_block <= waves;
-    if (small && one_tile) dw ? go(qpointwise_pair_kernel<4, 2, 16, 4, true, true>, 4, 2) : go(qpointwise_pair_kernel<4, 2, 16, 4, false, true>, 4, 2);
-    else if (small) dw ? go(qpointwise_pair_kernel<4, 2, 16, 4, true, false>, 4, 2) : go(qpointwise_pair_kernel<4, 2, 16, 4, false, false>, 4, 2);
-    else if (one_tile && !dw && a.ks1 <= 16 && a.ks2 <= 4) go(qpointwise_pair_kernel<16, 4, 12, 3, false, true>, 16, 4);
-    else dw ? go(qpointwise_pair_kernel<8, 4, 12, 3, true, false>, 8, 4) : go(qpointwise_pair_kernel<8, 4, 12, 3, false, false>, 8, 4);
+    if (split.once) {
+#define NNHIP_PAIR_CASE(KA, KB, MAXW, OCC)                                               \
+    do {                                                                                 \
+        if (!dw) go(qpointwise_pair_once_kernel<KA, KB, MAXW, OCC, false, 16>, 1, 1);    \
+        else if (pt == 16) go(qpointwise_pair_once_kernel<KA, KB, MAXW, OCC, true, 16>, 1, 1); \
+        else if (pt == 8) go(qpointwise_pair_once_kernel<KA, KB, MAXW, OCC, true, 8>, 1, 1);   \
+        else go(qpointwise_pair_once_kernel<KA, KB, MAXW, OCC, true, 4>, 1, 1);          \
+    } while (0)
+        if (small) NNHIP_PAIR_CASE(4, 2, 16, 4);
+        else if (a.ks1 <= 8 && a.ks2 <= 2) NNHIP_PAIR_CASE(8, 2, 12, 3);
+        else if (a.ks1 <= 8) NNHIP_PAIR_CASE(8, 4, 12, 3);
+        else if (a.ks1 <= 12) NNHIP_PAIR_CASE(12, 4, 12, 3);
+        else NNHIP_PAIR_CASE(16, 4, 12, 3);
+#undef NNHIP_PAIR_CASE
+    } else if (small) {
+        dw ? go(qpointwise_pair_kernel<4, 2, 16, 4, true>, 4, 2) : go(qpointwise_pair_kernel<4, 2, 16, 4, false>, 4, 2);
+    } else {
+        dw ? go(qpointwise_pair_kernel<8, 4, 12, 3, true>, 8, 4) : go(qpointwise_pair_kernel<8, 4, 12, 3, false>, 8, 4);
+    }
     NNHIP_LAUNCH_CHECK(ctx, "qpointwise_pair_kernel");
     return 0;
 }
+
+// ---- operators recorded one behind the other, as one launch ---------------------------------------------------------------
+namespace nnhip {
+struct Range {
+    const uint8_t *p;
+    size_t bytes;
+};
+static bool apart(Range a, Range b) { return !a.p || !b.p || a.p + a.bytes <= b.p || b.p + b.bytes <= a.p; }
+
+static bool plain_u8(const nncase_hip_conv2d_args_t &c) { // what launch_pair would refuse stays with the operators' own entry points
+    auto fits = [](const nncase_hip_quant_param_t &q) { return q.scale > 0.f && std::isfinite(q.scale) && q.zero_point >= 0 && q.zero_point <= 255; };
+    return c.out_dtype == NNCASE_HIP_DT_U8 && c.dequantize_output == 0 && c.out_channel_stride == 0 && c.out_channel_offset == 0 && c.batch > 0 &&
+           c.in_h > 0 && c.in_w > 0 && fits(c.x_qp) && fits(c.y_qp) && (!c.residual_dev || fits(c.sum_qp));
+}
+static int64_t pixels_of(const nncase_hip_conv2d_args_t &c) { return (int64_t)c.batch * c.in_h * c.in_w; }
+
+// Two convolutions as a pair over the fragments that each of them carries for its few-pixel kernel.
+static bool as_pair(const nncase_hip_ctx *ctx, const JoinedConv &first, const JoinedConv &second, nncase_hip_qpair *pr) {
+    for (const JoinedConv *j : {&first, &second}) {
+        const nncase_hip_conv2d_args_t &c = *j->args;
+        if (!j->weights->rows_pack || !plain_u8(c) || c.stride_h != 1 || c.stride_w != 1 || c.pad_h_before || c.pad_h_after || c.pad_w_before ||
+            c.pad_w_after)
+            return false;
+    }
+    const nncase_hip_conv2d_args_t &fa = *first.args, &sa = *second.args;
+    const int k1 = first.weights->in_channels, n1 = first.weights->out_channels, n2 = second.weights->out_channels;
+    if (second.x != first.y || second.weights->in_channels != n1 || sa.residual_dev || sa.batch != fa.batch || sa.in_h != fa.in_h || sa.in_w != fa.in_w ||
+        !nncase_hip_qpointwise_pair_supported(k1, n1, n2))
+        return false;
+    const int64_t m = pixels_of(fa);
+    if (m >= ((int64_t)1 << 30) || !pair_pays(m, k1, n1, n2, ctx->compute_units) || split_pair(m, k1, n1, n2, false, ctx->compute_units).apart) return false;
+    // (every range of the second convolution reads the pixels and the residual again, while others store)
+    const Range x{first.x, (size_t)m * k1}, res{reinterpret_cast<const uint8_t *>(fa.residual_dev), (size_t)m * n1}, y1{first.y, (size_t)m * n1},
+        y2{second.y, (size_t)m * n2};
+    if (!apart(x, y1) || !apart(x, y2) || !apart(res, y1) || !apart(res, y2) || !apart(y1, y2)) return false;
+    const nncase_hip_qpair *a = first.weights->rows_pack, *b = second.weights->rows_pack;
+    pr->first = first.weights, pr->second = second.weights;
+    pr->k1 = k1, pr->n1 = n1, pr->n2 = n2, pr->ks1 = a->ks2, pr->ks2 = b->ks2, pr->t1 = a->t2, pr->t2 = b->t2;
+    pr->d_wa = a->d_wb, pr->d_wsum_a = a->d_wsum_b, pr->d_bias_a = a->d_bias_b, pr->d_wb = b->d_wb, pr->d_wsum_b = b->d_wsum_b, pr->d_bias_b = b->d_bias_b;
+    return true;
+}
+
+// Whether the depthwise convolution joins the launch of the pair that reads its result.
+static bool front_joins(const nncase_hip_ctx *ctx, const JoinedConv &dw, const nncase_hip_qpair &pr, const JoinedConv &first, const JoinedConv &second) {
+    const nncase_hip_conv2d_args_t &da = *dw.args, &fa = *first.args;
+    const nncase_hip_weights &w = *dw.weights;
+    if (w.kind != nncase_hip_weights::kDepthwise || w.kernel_h != 3 || w.kernel_w != 3 || w.out_channels != pr.k1 || w.d_post_lut || !plain_u8(da) ||
+        da.residual_dev || da.stride_h != da.stride_w || (da.stride_h != 1 && da.stride_h != 2) || da.dilation_h != 1 || da.dilation_w != 1 ||
+        da.pad_h_before < 0 || da.pad_h_after < 0 || da.pad_w_before < 0 || da.pad_w_after < 0)
+        return false;
+    if (first.x != dw.y || !plain_u8(fa) || !plain_u8(*second.args) || da.batch != fa.batch ||
+        windowed_output_size(da.in_h, 3, da.stride_h, 1, da.pad_h_before, da.pad_h_after) != fa.in_h ||
+        windowed_output_size(da.in_w, 3, da.stride_w, 1, da.pad_w_before, da.pad_w_after) != fa.in_w ||
+        da.y_qp.zero_point != fa.x_qp.zero_point || da.y_qp.scale != fa.x_qp.scale)
+        return false;
+    const int64_t m = pixels_of(fa), in_bytes = pixels_of(da) * pr.k1;
+    if (in_bytes >= ((int64_t)1 << 31) || m >= ((int64_t)1 << 30) || (reinterpret_cast<uintptr_t>(dw.x) & 15u) != 0 ||
+        !front_pays(m, pr.k1, pr.n1, pr.n2, ctx->compute_units))
+        return false;
+    const Range x{dw.x, (size_t)in_bytes}, mid{dw.y, (size_t)m * pr.k1}, res{reinterpret_cast<const uint8_t *>(fa.residual_dev), (size_t)m * pr.n1},
+        y1{first.y, (size_t)m * pr.n1}, y2{second.y, (size_t)m * pr.n2};
+    return apart(x, mid) && apart(x, y1) && apart(x, y2) && apart(mid, res) && apart(mid, y1) && apart(mid, y2);
+}
+
+int launch_joined_convs(nncase_hip_ctx *ctx, const JoinedConv *dw, const nncase_hip_qpair *pair, const JoinedConv &first, const JoinedConv &second, bool *taken) {
+    *taken = false;
+    nncase_hip_qpair made; // (borrows what it points to)
+    if (!pair) {
+        if (!as_pair(ctx, first, second, &made)) return 0;
+        pair = &made;
+    }
+    if (dw && !front_joins(ctx, *dw, *pair, first, second)) return 0;
+    const uint8_t *const x = dw ? dw->x : first.x;
+    for (const uint8_t *p : {x, (const uint8_t *)first.y, (const uint8_t *)second.y})
+        if ((reinterpret_cast<uintptr_t>(p) & 15u) != 0) return 0;
+    *taken = true;
+    return launch_pair(ctx, dw ? "qdepthwise_pointwise_pair" : "qpointwise_pair", x, dw ? dw->weights : nullptr, dw ? dw->args : nullptr, pair, first.y,
+                       second.y, first.args, second.args, dw ? dw->y : nullptr);
+}
+} // namespace nnhip
 
 extern "C" int nncase_hip_qpointwise_pair(nncase_hip_ctx_t *ctx, const uint8_t *x_dev, const nncase_hip_qpair_t *pair, uint8_t *y1_dev,
                                           uint8_t *y2_dev, const nncase_hip_conv2d_args_t *first_args,

@@ -402,8 +402,9 @@ def pad_small_channel_convs(qg: QuantGraph) -> QuantGraph:
 # batches 1 and 2 (0.215 -> 0.184 ms per image at batch 1); beyond them the separate kernels win.
 PAIR_STREAM_LIMIT = 4 << 20
 PAIR_MAX_PIXEL_TILES = 1024
-# A depthwise convolution in front joins the pair while it has few channels: a workgroup computes its 16 pixels of it
-# alone, about 50 ns per 16 channels, against the 3.5 us of the separate launch it saves.
+# A depthwise convolution in front is recorded as part of the pair while it has few channels, and its result is then never
+# stored.  (Recorded as operators of their own, convolutions and pairs still share a launch where that is the quicker: the
+# function sees to it, and stores every result.)
 PAIR_FRONT_MAX_CHANNELS = 256
 
 

@@ -446,3 +446,105 @@ def test_random_pairs(hip_ctx, seed):
     if seed % 2:
         dw = (int(rng.integers(1, 3)), [P1, ((0, 1), (0, 1)), ((1, 0), (1, 0)), ((0, 0), (0, 0))][int(rng.integers(0, 4))])
     run_pair(hip_ctx, n, k1, n1, n2, h, w, seed=seed, dw=dw, **options)
+
+
+PIXEL_TILES = [  # (n, channels, mid, out, in_h, in_w, stride, residual): tiles of 4, 8 and 16 pixels that the tensor fills and not, windows of one and
+    # two turns of a workgroup's threads, channels that fill no quad of waves and no k-step
+    (1, 192, 32, 192, 2, 2, 1, True), (1, 192, 32, 192, 1, 3, 1, True), (1, 384, 64, 384, 13, 13, 1, True), (3, 80, 20, 36, 11, 9, 2, False),
+    (1, 960, 160, 960, 5, 1, 1, False), (1, 976, 172, 100, 7, 9, 1, True), (2, 592, 132, 320, 21, 23, 2, False), (1, 528, 68, 64, 17, 15, 1, True),
+    (1, 48, 16, 2000, 8, 8, 1, False), (1, 64, 128, 768, 9, 31, 1, True), (1, 1024, 192, 40, 1, 1, 1, False), (1, 272, 24, 384, 33, 33, 1, True),
+    (1, 400, 12, 384, 40, 39, 1, False), (4, 16, 64, 64, 31, 32, 1, True),
+]
+
+
+@pytest.mark.parametrize("n,k1,n1,n2,h,w,stride,residual", PIXEL_TILES)
+@pytest.mark.parametrize("lut", [False, True])
+def test_pixel_tiles_of_a_depthwise_pair(hip_ctx, n, k1, n1, n2, h, w, stride, residual, lut):
+    run_pair(hip_ctx, n, k1, n1, n2, h, w, seed=n + k1 + n1 + n2 + h * w, residual=residual, lut_a=lut, lut_b=lut, dw=(stride, P1))
+
+
+@pytest.mark.parametrize("n,k1,n1,n2,h,w,stride,residual", [
+    (1, 384, 64, 384, 14, 14, 1, True), (1, 960, 160, 960, 7, 7, 1, True), (2, 192, 32, 192, 9, 11, 2, False), (1, 576, 96, 560, 13, 14, 1, True),
+    (1, 80, 20, 36, 30, 31, 1, False), (1, 16, 4, 4, 1, 1, 1, True), (1, 800, 72, 928, 23, 23, 1, True), (3, 576, 160, 960, 24, 23, 1, False)])
+@pytest.mark.parametrize("form", ["pair", "convolutions", "no front"])
+@pytest.mark.parametrize("lut", [False, True])
+def test_operators_recorded_one_behind_the_other(hip_ctx, n, k1, n1, n2, h, w, stride, residual, form, lut):
+    """A depthwise convolution and a pair, and the three (or the last two) convolutions one by one, which a function may run as one launch: every
+    result is stored with the bytes of the operators' own calls, eagerly and replayed."""
+    rng = np.random.default_rng(k1 + n1 + n2 + h)
+    oh, ow = (h - 1) // stride + 1, (w - 1) // stride + 1
+    m = n * oh * ow
+    wd, wa, wb = (rng.integers(0, 256, s, dtype=np.uint8) for s in ((k1, 1, 3, 3), (n1, k1, 1, 1), (n2, n1, 1, 1)))
+    bias = [rng.integers(-3000, 3000, c).astype(np.int32) for c in (k1, n1, n2)]
+    q = [qp(11, 0.019), qp(120, 0.9), qp(117, 3.1), qp(125, 2.9)]
+    depthwise = hip_ctx.prepack_conv2d(wd, bias[0], qp(119, 0.0123), groups=k1)
+    first, second = hip_ctx.prepack_conv2d(wa, bias[1], qp(131, 0.0041), expected_pixels=m), hip_ctx.prepack_conv2d(wb, bias[2], qp(122, 0.0037), expected_pixels=m)
+    if lut:
+        first.set_post_lut(rng.permutation(256).astype(np.uint8), q[2])
+        second.set_post_lut(rng.permutation(256).astype(np.uint8), q[3])
+    x = hip_ctx.to_device(rng.integers(0, 256, n * h * w * k1, dtype=np.uint8))
+    res = hip_ctx.to_device(rng.integers(0, 256, m * n1, dtype=np.uint8))
+    sizes = [m * k1, m * n1, m * n2]
+    alone, got = ([hip_ctx.alloc(s).fill(0x5A) for s in sizes] for _ in range(2))
+    da = rt.Conv2dArgs(n, h, w, stride, stride, 1, 1, 1, 1, 1, 1, q[0], q[1], FULL[0], FULL[1], rt.DT_U8)
+    fa, sa = conv_args(n, oh, ow, q[1], q[2], FULL), conv_args(n, oh, ow, q[2], q[3], FULL)
+    if residual:
+        fa.residual_dev, fa.residual_qp, fa.sum_qp = res.ptr, qp(101, 1.7), q[2]
+        fa.sum_clamp_min, fa.sum_clamp_max = FULL
+    hip_ctx.qconv2d(x, depthwise, alone[0], da)
+    hip_ctx.qconv2d(alone[0], first, alone[1], fa)
+    hip_ctx.qconv2d(alone[1], second, alone[2], sa)
+    hip_ctx.sync()
+    want = [b.download((s,), np.uint8) for b, s in zip(alone, sizes)]
+    assert all(len(np.unique(v)) > 8 for v in want if v.size > 256)
+    fn = rt.Function(hip_ctx)
+    if form == "no front":
+        got[0].upload(want[0])
+    else:
+        fn.add_qconv2d(x, depthwise, got[0], da)
+    if form == "pair":
+        pair = hip_ctx.prepack_qpointwise_pair(first, wa, second, wb)
+        fn.add_qpointwise_pair(got[0], pair, got[1], got[2], fa, sa)
+    else:
+        fn.add_qconv2d(got[0], first, got[1], fa)
+        fn.add_qconv2d(got[1], second, got[2], sa)
+    for step in range(4):
+        if step == 2:
+            fn.capture()
+        for b in got[1 if form == "no front" else 0:]:
+            b.fill(0xA5)
+        fn.invoke()
+        hip_ctx.sync()
+        for b, v in zip(got, want):
+            assert np.array_equal(b.download(v.shape, np.uint8), v)
+
+
+def test_operators_whose_buffers_meet_stay_apart(hip_ctx):
+    """A result that lies over an earlier operator's input or residual: as one launch some workgroups would store over what others still read."""
+    rng = np.random.default_rng(2)
+    n, k1, n1, n2, h = 1, 384, 384, 384, 14
+    m = h * h
+    wd, wa, wb = (rng.integers(0, 256, s, dtype=np.uint8) for s in ((k1, 1, 3, 3), (128, k1, 1, 1), (n2, 128, 1, 1)))
+    z = lambda c: np.zeros(c, np.int32)
+    depthwise = hip_ctx.prepack_conv2d(wd, z(k1), qp(119, 0.0123), groups=k1)
+    first, second = hip_ctx.prepack_conv2d(wa, z(128), qp(131, 0.0041), expected_pixels=m), hip_ctx.prepack_conv2d(wb, z(n2), qp(122, 0.0037), expected_pixels=m)
+    q = [qp(11, 0.019), qp(120, 0.9), qp(117, 3.1), qp(125, 2.9)]
+    da = rt.Conv2dArgs(n, h, h, 1, 1, 1, 1, 1, 1, 1, 1, q[0], q[1], FULL[0], FULL[1], rt.DT_U8)
+    fa, sa = conv_args(n, h, h, q[1], q[2], FULL), conv_args(n, h, h, q[2], q[3], FULL)
+    x0 = rng.integers(0, 256, m * k1, dtype=np.uint8)
+    x, mid, y1, y2 = (hip_ctx.alloc(m * c) for c in (k1, k1, 128, n2))
+    hip_ctx.qconv2d(x.upload(x0), depthwise, mid, da)
+    hip_ctx.qconv2d(mid, first, y1, fa)
+    hip_ctx.qconv2d(y1, second, y2, sa)
+    hip_ctx.sync()
+    want = y2.download((m * n2,), np.uint8)
+    for over in ("the depthwise input", "the first input"):
+        out = x if over == "the depthwise input" else mid
+        fn = rt.Function(hip_ctx)
+        fn.add_qconv2d(x, depthwise, mid, da)
+        fn.add_qconv2d(mid, first, y1, fa)
+        fn.add_qconv2d(y1, second, out, sa)
+        x.upload(x0)
+        fn.invoke()
+        hip_ctx.sync()
+        assert np.array_equal(out.download((m * n2,), np.uint8), want)

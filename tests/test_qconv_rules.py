@@ -25,6 +25,12 @@ extern "C" int window(int stride, int ksteps, int channels, int pix, int waves, 
 }
 extern "C" int dma_rows(long rows, int nchunks, int ksteps) { return 64 * nnhip::choose_dma_rows(rows, nchunks, ksteps, 256).rg; }
 extern "C" int pair_apart(long pixels, int k1, int n1, int n2, int dw) { return nnhip::split_pair(pixels, k1, n1, n2, dw, 256).apart; }
+extern "C" int pair_pays(long pixels, int k1, int n1, int n2) { return nnhip::pair_pays(pixels, k1, n1, n2, 256); }
+extern "C" int front_pays(long pixels, int k1, int n1, int n2) { return nnhip::front_pays(pixels, k1, n1, n2, 256); }
+extern "C" void pair_plan(long pixels, int k1, int n1, int n2, int dw, int *out) {
+    const nnhip::PairSplit s = nnhip::split_pair(pixels, k1, n1, n2, dw, 256);
+    out[0] = s.pixels, out[1] = s.ranges, out[2] = s.tiles_per_block, out[3] = s.waves, out[4] = s.once, out[5] = s.small;
+}
 extern "C" int dma(long rows, int n, int ksteps) { return nnhip::dma_pays(rows, n, ksteps, 256); }
 """)
     subprocess.check_call(["g++", "-std=c++17", "-O2", "-shared", "-fPIC", "-I", CSRC, str(d / "r.cpp"), "-o", str(d / "r.so")])
@@ -352,3 +358,56 @@ def test_pairs_take_the_quicker_form(rules, pixels, k1, n1, n2, one, two):
     assert (two if rules.pair_apart(pixels, k1, n1, n2, 0) else one) <= 1.02 * min(one, two)
     assert not rules.pair_apart(pixels, k1, n1, n2, 1)                         # a depthwise stage in front: always one launch
     assert not rules.pair_apart(pixels, k1, n1 + 4, n2, 0)                      # rows between the two that are no whole pieces
+
+
+# us of the launches apart / as a pair / with the depthwise stage in the pair's launch (None: no depthwise stage), 20 in a chain
+PAIRS_TIMED = [  # (pixels, in, mid, out, ...)
+    (392, 32, 16, 96, 7.86, 5.94, 3.53), (6400, 32, 16, 96, 8.57, 6.71, 4.66), (9408, 32, 120, 428, 10.75, 12.41, None),
+    (27, 64, 32, 32, 6.06, 3.01, None), (32, 64, 32, 32, 6.13, 3.03, None), (16, 64, 64, 64, 6.46, 2.86, None),
+    (800, 64, 64, 64, 5.21, 3.1, None), (6400, 64, 184, 528, 12.14, 18.41, 17.29), (12800, 96, 24, 144, 10.91, 10.24, 9.55),
+    (25, 128, 64, 64, 6.35, 3.0, None), (4800, 128, 64, 64, 5.85, 3.55, None), (256, 128, 68, 404, 9.39, 6.66, 4.54),
+    (108, 128, 128, 256, 5.45, 4.02, None), (400, 144, 24, 144, 8.88, 6.23, 4.0), (9408, 144, 24, 144, 10.97, 11.3, 12.07),
+    (256, 144, 32, 192, 8.17, 6.34, 4.11), (400, 144, 32, 192, 8.38, 6.32, 4.09), (196, 192, 32, 192, 8.38, 6.35, 4.09),
+    (6400, 192, 32, 192, 10.12, 9.26, 8.52), (800, 192, 64, 384, 8.75, 6.51, 4.47), (1568, 192, 64, 384, 9.11, 6.74, 5.31),
+    (9408, 192, 112, 820, 13.93, 17.61, None), (25, 256, 128, 128, 6.59, 3.43, None), (1600, 256, 128, 128, 6.16, 3.68, None),
+    (4704, 304, 76, 1136, 10.2, 19.8, None), (256, 384, 64, 384, 8.69, 6.74, 4.67), (1176, 384, 64, 384, 9.6, 7.17, 6.41),
+    (147, 384, 96, 576, 9.07, 7.1, 4.89), (400, 384, 96, 576, 9.39, 7.17, 5.75), (200, 384, 168, 628, 10.0, 7.48, 5.66),
+    (100, 416, 196, 56, 6.96, 4.96, None), (200, 448, 188, 200, 7.31, 4.65, None), (200, 480, 152, 92, 6.54, 4.42, None),
+    (1200, 496, 12, 448, 6.73, 3.85, None), (392, 512, 256, 256, 7.24, 5.52, None), (4800, 512, 256, 256, 10.17, 12.88, None),
+    (588, 528, 64, 340, 6.27, 4.14, None), (100, 544, 64, 92, 9.32, 6.83, 5.12), (400, 576, 96, 576, 10.07, 7.92, 6.79),
+    (9408, 576, 96, 576, 17.8, 24.2, 36.94), (100, 576, 160, 960, 10.19, 8.39, 6.25), (4800, 576, 160, 960, 16.21, 28.3, 38.51),
+    (3136, 592, 104, 396, 8.26, 12.73, None), (400, 624, 56, 248, 10.07, 7.43, 5.55), (192, 672, 184, 340, 6.94, 5.4, None),
+    (196, 704, 160, 816, 6.79, 5.32, None), (3136, 720, 12, 960, 14.56, 19.87, 30.12), (16, 736, 40, 144, 9.34, 6.98, 5.37),
+    (300, 736, 40, 456, 6.5, 4.25, None), (49, 736, 108, 1036, 7.19, 4.77, None), (400, 768, 148, 628, 11.36, 8.57, 7.67),
+    (392, 768, 164, 832, 11.37, 8.89, 7.94), (4800, 896, 208, 696, 18.02, 28.81, 51.45), (72, 912, 164, 844, 11.18, 8.97, 7.61),
+    (18, 944, 124, 100, 10.39, 7.84, 6.82), (196, 960, 64, 332, 6.11, 4.39, None), (400, 960, 160, 960, 10.79, 9.46, 8.97),
+    (2352, 960, 160, 960, 13.97, 22.03, 43.51), (9600, 1008, 40, 936, 26.86, 30.01, 50.16), (3200, 1024, 120, 1064, 16.75, 23.29, 45.22),
+]
+
+
+@pytest.mark.parametrize("pixels,k1,n1,n2,apart,pair,joined", PAIRS_TIMED)
+def test_pairs_and_fronts_where_they_pay(rules, pixels, k1, n1, n2, apart, pair, joined):
+    """At most half more than the quickest of the three as measured (7 in 1000 in the mean of those the rule was drawn from)."""
+    for f in (rules.pair_pays, rules.front_pays):
+        f.argtypes = [C.c_long, C.c_int, C.c_int, C.c_int]
+    as_pair = joined if joined is not None and rules.front_pays(pixels, k1, n1, n2) else pair
+    taken = as_pair if rules.pair_pays(pixels, k1, n1, n2) else apart
+    assert taken <= 1.5 * min(apart, pair, joined or pair)
+
+
+def test_pair_plans_cover_the_work(rules):
+    """Every channel tile of the second convolution once, a wave per tile where all is requested at once, and small pixel tiles only then."""
+    import random
+    rng = random.Random(5)
+    rules.pair_plan.argtypes = [C.c_long, C.c_int, C.c_int, C.c_int, C.c_int, C.POINTER(C.c_int)]
+    out = (C.c_int * 6)()
+    for _ in range(20000):
+        pixels, k1, n1, n2 = rng.choice([rng.randint(1, 100), rng.randint(1, 20000)]), 16 * rng.randint(1, 64), 4 * rng.randint(1, 128), 4 * rng.randint(1, 400)
+        dw = rng.randint(0, 1)
+        rules.pair_plan(pixels, k1, n1, n2, dw, out)
+        pt, ranges, per, waves, once, small = out
+        t1, t2, ks1, ks2 = -(-n1 // 16), -(-n2 // 16), -(-k1 // 64), -(-n1 // 64)
+        assert pt in (4, 8, 16) and (pt == 16 or (dw and once)) and (ranges - 1) * per < t2 <= ranges * per
+        assert 1 <= waves <= (16 if small else 12)
+        if once:
+            assert t1 <= waves and per <= waves and ks1 <= 16 and ks2 <= 4 and (not small or (ks1 <= 4 and ks2 <= 2))
