@@ -165,6 +165,12 @@ inline OutputTile choose_output_tile(int out_h, int out_w, int pix, int stride_h
     return best;
 }
 
+// A division of what counts the window kernel's threads or pixels, two instructions: p / d = p * mul >> 20 for 0 <= p < kTileDivMost and
+// every d >= 1.  (mul is less than 1 above 2^20 / d, so the product less than p above 2^20 p / d: short of the next whole number while
+// p d < 2^20, and of the first while p < d, which covers every larger d.)
+constexpr int kTileDivMost = 512;
+inline uint32_t make_tile_div(int d) { return ((1u << 20) + (uint32_t)d - 1) / (uint32_t)d; }
+
 // Whether a launch of the window kernel as planned is quicker than the implicit GEMM of the same layer (byte results, strides of 1
 // and 2, three k-steps and more, stride 2 sixteen).  us, implicit GEMM / window kernel:
 //   * tiles that images do not fill by half stay, their surplus pixels are multiplied and dropped; with fewer than three waves per

@@ -11,25 +11,59 @@
 //     takes 8 KiB of them for 128 clocks of matrix work, so waves share pixels rather than channels where they can;
 //   * blocks start the reduction at different k-steps (integer sums do not care): otherwise all of them wait for the same
 //     weights to come from memory at the same time, step after step;
-//   * results leave through LDS as whole pixel rows.
+//   * results leave through LDS as whole pixel rows, whose bytes of a residual are asked for before the sums meet;
+//   * what a block does before its first request and after its last product counts as much as the reduction: all arguments of the
+//     requests in one trip and those of the stores in another, a thread that keeps its piece of a pixel (two multiply-adds an address,
+//     short divisions), a channel's terms asked for first.  Start to end of a block, 6400 pixels 64 -> 64 3x3 with a residual 4.6 us ->
+//     3.7 (before the first request 0.6 -> 0.4, requests 0.5 -> 0.3, results 1.1 -> 0.5), 409 600 pixels 32 -> 32 21.8 -> 19.2 a launch.
 // Arithmetic, weight packing and the bytes of the result are those of qconv_igemm.hpp.
 #include "qconv_rules.hpp"
 #include "qconv_tile.hpp"
 
 namespace nnhip {
 
-// FAST: the requantisation is the one-instruction form without a clamp of its own (Epilogue::fast and ::full).
+// What a launch's last stage takes of the arguments, in one trip: fetched ahead, the values would be spilled while the reduction runs,
+// and a request of the first stage would wait behind them.
+template <bool FAST> __device__ __forceinline__ IgemmArgs gather_store_args() {
+    auto p = (const __attribute__((address_space(4))) IgemmArgs *)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(p));
+    const IgemmArgs &a = *(const IgemmArgs *)p;
+    IgemmArgs l; // (what is not assigned here is not used)
+    l.ep.c1 = a.ep.c1, l.ep.c2 = a.ep.c2;
+    if constexpr (!FAST) {
+        l.ep.mult = a.ep.mult, l.ep.sy = a.ep.sy, l.ep.rsy = a.ep.rsy, l.ep.zy = a.ep.zy, l.ep.qlo = a.ep.qlo, l.ep.qhi = a.ep.qhi;
+        l.ep.fast = a.ep.fast, l.ep.full = a.ep.full;
+        asm volatile("" ::"s"(l.ep.mult), "s"(l.ep.sy), "s"(l.ep.rsy), "s"(l.ep.zy), "s"(l.ep.qlo), "s"(l.ep.qhi), "s"(l.ep.fast), "s"(l.ep.full));
+    }
+    l.rep.res = a.rep.res, l.rep.zy = a.rep.zy, l.rep.sy = a.rep.sy, l.rep.zr = a.rep.zr, l.rep.sr = a.rep.sr;
+    l.rep.sum.sy = a.rep.sum.sy, l.rep.sum.rsy = a.rep.sum.rsy, l.rep.sum.zy = a.rep.sum.zy, l.rep.sum.qlo = a.rep.sum.qlo, l.rep.sum.qhi = a.rep.sum.qhi;
+    l.y = a.y, l.m = a.m, l.n = a.n, l.ldy = a.ldy, l.y_coff = a.y_coff, l.ldr = a.ldr, l.r_coff = a.r_coff, l.zwp = a.zwp, l.lut = a.lut;
+    l.d_ohow.div = a.d_ohow.div, l.d_ow.div = a.d_ow.div;
+    asm volatile("" ::"s"(l.ep.c1), "s"(l.ep.c2), "s"(l.rep.res), "s"(l.rep.zy), "s"(l.rep.sy), "s"(l.rep.zr), "s"(l.rep.sr), "s"(l.rep.sum.sy), "s"(l.rep.sum.rsy),
+                 "s"(l.rep.sum.zy), "s"(l.rep.sum.qlo), "s"(l.rep.sum.qhi), "s"(l.y), "s"(l.m), "s"(l.n), "s"(l.ldy), "s"(l.y_coff), "s"(l.ldr), "s"(l.r_coff),
+                 "s"(l.zwp), "s"(l.lut), "s"(l.d_ohow.div), "s"(l.d_ow.div));
+    return l;
+}
 
+// FAST: the requantisation is the one-instruction form without a clamp of its own (Epilogue::fast and ::full).
 template <int T, int RG, int WM, int WN, bool FAST>
 __global__ __launch_bounds__(WM * WN * 64, 4) void qconv_tile_kernel(const IgemmArgs a, const TileArgs t) {
     constexpr int THREADS = WM * WN * 64, PIX = WM * RG * 16, TB = T * WN;
     constexpr int D = 4;                                             // k-steps of weights in flight
+    static_assert(TB * 16 <= THREADS && THREADS <= kTileDivMost, "a thread per channel, tile_div");
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
     int32_t *cterm = reinterpret_cast<int32_t *>(smem);              // [TB * 16]
     int32_t *sums = cterm + TB * 16;                                 // [PIX] sum of x' over a pixel's window
     uint8_t *lutl = reinterpret_cast<uint8_t *>(sums + PIX);         // [256]
     int32_t *taps = reinterpret_cast<int32_t *>(lutl + 256);         // [KS + 2][4] LDS offset of a piece of the reduction
     uint8_t *tile = smem + t.tile_off;
+
+    // (what the requests need, in one trip; see gather_store_args for the rest)
+    asm volatile("" ::"s"(a.x), "s"(a.x_bytes), "s"(a.wpk), "s"(a.bias), "s"(a.wsum), "s"(a.lut), "s"(a.ksteps), "s"(a.ldx), "s"(a.x_coff), "s"(a.in_h), "s"(a.in_w),
+                 "s"(a.stride_h), "s"(a.stride_w), "s"(a.pad_h), "s"(a.pad_w), "s"(a.num_mtiles), "s"(a.n));
+    asm volatile("" ::"s"(t.th), "s"(t.tw), "s"(t.hr), "s"(t.hc), "s"(t.half), "s"(t.pitch), "s"(t.row_pitch), "s"(t.pieces), "s"(t.apart), "s"(t.dc), "s"(t.dr),
+                 "s"(t.row_bytes), "s"(t.d_pieces), "s"(t.d_hc), "s"(t.d_txy.mul), "s"(t.d_txy.shift), "s"(t.d_txy.div), "s"(t.d_tx.mul), "s"(t.d_tx.shift),
+                 "s"(t.d_tx.div), "s"(t.d_nchunks.mul), "s"(t.d_nchunks.shift), "s"(t.d_nchunks.div));
 
     // as in qconv_wide_kernel: channel chunks of a tile back to back, a contiguous eighth of the tiles per XCD
     const int xcd = blockIdx.x & 7, seq = blockIdx.x >> 3;
@@ -46,7 +80,14 @@ __global__ __launch_bounds__(WM * WN * 64, 4) void qconv_tile_kernel(const Igemm
     const int ch_base = chunk * (TB * 16);
     const bool two = a.stride_w == 2;
 
-    // ---- the input tile: requested in batches of U pieces per thread, the next before one is stored ----
+    // ---- a channel's terms and the byte table: asked for first, needed last ----
+    int32_t bias = 0, wsum = 0;
+    uint32_t table = 0;
+    if (ch_base + tid < a.n && tid < TB * 16) bias = a.bias[ch_base + tid], wsum = a.wsum[ch_base + tid];
+    if (a.lut && tid < 64) table = a.lut[tid];
+
+    // ---- the input tile: requested in batches of U pieces per thread, the next before one is stored.  A thread keeps its piece of
+    // a pixel and goes through the pixels t.apart at a time ----
     const uint32_t img = fastdiv((uint32_t)mt, t.d_txy);
     const uint32_t in_img = (uint32_t)mt - img * t.d_txy.div;
     const uint32_t tyi = fastdiv(in_img, t.d_tx);
@@ -59,44 +100,55 @@ __global__ __launch_bounds__(WM * WN * 64, 4) void qconv_tile_kernel(const Igemm
         wide_u32x4 v[U];
         int dst[U];        // where the piece goes in LDS; its bit 0: the pixel lies in the padding
     };
-    const int n = t.hr * t.hc * t.pieces;
+    const int n = t.hr * t.hc; // pixels
     const bool inside = iy0 >= 0 && ix0 >= 0 && iy0 + t.hr <= a.in_h && ix0 + t.hc <= a.in_w; // no padding under this tile
-    int q, r, c; // piece, row and column of this thread's next piece
+    int r, c;  // row and column of this thread's next pixel
+    int owned; // its pixels are those of t.apart, 2 t.apart, ... below this
+    int q16;   // its piece
     {
-        const uint32_t p0 = fastdiv((uint32_t)tid, t.d_pieces);
-        q = tid - (int)p0 * t.pieces;
-        r = (int)fastdiv(p0, t.d_hc);
-        c = (int)p0 - r * t.hc;
+        const int p0 = tile_div(tid, t.d_pieces);
+        q16 = (tid - __mul24(p0, t.pieces)) * 16;
+        r = tile_div(p0, t.d_hc);
+        c = p0 - __mul24(r, t.hc);
+        owned = p0 < t.apart ? n - p0 : 0; // (threads past the last whole pixel: none)
     }
-    // (a thread past the tile's last piece reads what follows it in the tensor, or 0 past its end, and drops it)
+    // (a thread past the tile's last pixel reads what follows it in the tensor, or 0 past its end, and drops it)
+    auto request_piece = [&](Batch &f, int u, bool in_c) __attribute__((always_inline)) {
+        const int goff = __mul24(r, t.row_bytes) + (__mul24(c, a.ldx) + q16);
+        f.dst[u] = __mul24(r, t.row_pitch) + (__mul24(two ? (c & 1) * t.half + (c >> 1) : c, t.pitch) + q16);
+        if (in_c) {
+            f.v[u] = __builtin_amdgcn_raw_buffer_load_b128(xres, goff, base, 0);
+        } else {
+            const bool in = (unsigned)(iy0 + r) < (unsigned)a.in_h && (unsigned)(ix0 + c) < (unsigned)a.in_w;
+            f.v[u] = __builtin_amdgcn_raw_buffer_load_b128(xres, in ? (uint32_t)(base + goff) : 0xffffffffu, 0, 0);
+            f.dst[u] |= in ? 0 : 1;
+        }
+        c += t.dc;
+        const bool carry = c >= t.hc;
+        c -= carry ? t.hc : 0;
+        r += t.dr + (carry ? 1 : 0);
+    };
     auto request = [&](Batch &f, int i0) __attribute__((always_inline)) {
+        if (inside) {
 #pragma unroll
-        for (int u = 0; u < U; u++) {
-            if (i0 + u * THREADS >= n) break;
-            const int goff = __mul24(r, t.row_bytes) + __mul24(c, a.ldx) + q * 16;
-            const int pos = two ? (c & 1) * t.half + (c >> 1) : c;
-            f.dst[u] = __mul24(r, t.row_pitch) + __mul24(pos, t.pitch) + q * 16;
-            if (inside) {
-                f.v[u] = __builtin_amdgcn_raw_buffer_load_b128(xres, goff, base, 0);
-            } else {
-                const bool in = (unsigned)(iy0 + r) < (unsigned)a.in_h && (unsigned)(ix0 + c) < (unsigned)a.in_w;
-                f.v[u] = __builtin_amdgcn_raw_buffer_load_b128(xres, in ? (uint32_t)(base + goff) : 0xffffffffu, 0, 0);
-                f.dst[u] |= in ? 0 : 1;
+            for (int u = 0; u < U; u++) {
+                if (i0 + u * t.apart >= n) break;
+                request_piece(f, u, true);
             }
-            q += t.dq;
-            const bool cq = q >= t.pieces;
-            q -= cq ? t.pieces : 0;
-            c += t.dc + (cq ? 1 : 0);
-            const bool cc = c >= t.hc;
-            c -= cc ? t.hc : 0;
-            r += t.dr + (cc ? 1 : 0);
+        } else {
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                if (i0 + u * t.apart >= n) break;
+                request_piece(f, u, false);
+            }
         }
     };
     auto keep = [&](const Batch &f, int i0) __attribute__((always_inline)) {
 #pragma unroll
         for (int u = 0; u < U; u++) {
-            if (i0 + u * THREADS >= n) break;
-            if (i0 + u * THREADS + tid < n) {
+            const int i = i0 + u * t.apart;
+            if (i >= n) break;
+            if (i < owned) {
                 const uint32_t fill = (f.dst[u] & 1) ? a.zx_splat : 0u;
                 wide_u32x4 w;
 #pragma unroll
@@ -145,16 +197,11 @@ __global__ __launch_bounds__(WM * WN * 64, 4) void qconv_tile_kernel(const Igemm
         }
         taps[e] = off;
     }
-    for (int i = tid; i < TB * 16; i += THREADS) {
-        const bool real = ch_base + i < a.n;
-        cterm[i] = real ? a.bias[ch_base + i] - a.zxp * a.wsum[ch_base + i] + a.k * a.zxp * a.zwp : 0;
-    }
-    if (a.lut && tid < 64) reinterpret_cast<uint32_t *>(lutl)[tid] = a.lut[tid];
     // this lane's pixels: pixel (wm RG + rg) * 16 + j of the tile, in rows of tw
     auto lds_of = [&](int group) __attribute__((always_inline)) {
-        const uint32_t p = (wm * RG + group) * 16 + j;
-        int ty = (int)fastdiv(p, t.d_tw);
-        int tx = (int)p - ty * t.tw;
+        const int p = (wm * RG + group) * 16 + j;
+        int ty = tile_div(p, t.d_tw);
+        int tx = p - __mul24(ty, t.tw);
         if (ty >= t.th) ty = tx = 0; // (surplus of the block: not stored)
         return __mul24(ty, a.stride_h * t.row_pitch) + __mul24(tx, t.pitch);
     };
@@ -165,16 +212,19 @@ __global__ __launch_bounds__(WM * WN * 64, 4) void qconv_tile_kernel(const Igemm
     for (int rg = 0; rg < RG; rg++) xbase[rg] = lds_of(rg);
 #pragma unroll
     for (int i = 0; i < SG; i++) xsum[i] = WN == 1 ? xbase[i] : lds_of(min(wn * SG + i, RG - 1));
+    if (tid < TB * 16) cterm[tid] = bias - a.zxp * wsum + a.k * a.zxp * a.zwp;
+    if (tid < 64) reinterpret_cast<uint32_t *>(lutl)[tid] = table;
     {
         int i0 = 0;
-        for (; i0 + U * THREADS < n; i0 += U * THREADS) {
+        for (; i0 + U * t.apart < n; i0 += U * t.apart) {
             Batch fb;
-            request(fb, i0 + U * THREADS);
+            request(fb, i0 + U * t.apart);
             keep(fa, i0);
             fa = fb;
         }
         keep(fa, i0);
     }
+    const IgemmArgs late = gather_store_args<FAST>();
     __syncthreads();
 
     // ---- the reduction ----
@@ -232,6 +282,39 @@ __global__ __launch_bounds__(WM * WN * 64, 4) void qconv_tile_kernel(const Igemm
     });
 
     // ---- epilogue ----
+    // whole pixel rows: TB threads per pixel, 16 channels each.  Their bytes of the residual are asked for before the sums meet.
+    constexpr int PPT = THREADS / TB, PASSES = PIX / PPT; // pixels of a pass
+    static_assert(PIX % PPT == 0, "whole passes");
+    const int oh_img = (int)late.d_ohow.div, ow = (int)late.d_ow.div;
+    const int cb = (tid % TB) * 16, ch = ch_base + cb;
+    const bool whole = ch + 16 <= late.n, wide_y = ((late.ldy | late.y_coff) & 3) == 0;
+    int px[PASSES]; // pixel index of the tensor, late.m where there is none
+    u32x4 rv[PASSES];
+#pragma unroll
+    for (int it = 0; it < PASSES; it++) {
+        const int p = it * PPT + tid / TB;
+        const int ty = tile_div(p, t.d_tw);
+        const int oy = oy0 + ty, ox = ox0 + p - __mul24(ty, t.tw);
+        const int at = __mul24(oy, ow) + ox;
+        px[it] = ty < t.th && ox < ow && at < oh_img && ch < late.n ? (int)img * oh_img + at : late.m;
+    }
+    if (late.rep.res) {
+        const bool wide_r = ((late.ldr | late.r_coff) & 3) == 0;
+#pragma unroll
+        for (int it = 0; it < PASSES; it++) {
+            rv[it] = u32x4{0, 0, 0, 0};
+            if (px[it] >= late.m) continue;
+            const uint8_t *ro = late.rep.res + (size_t)px[it] * late.ldr + late.r_coff + ch;
+            if (whole && wide_r) {
+                const u32x4_a4 r4 = *reinterpret_cast<const u32x4_a4 *>(ro);
+                rv[it] = u32x4{r4[0], r4[1], r4[2], r4[3]};
+            } else {
+#pragma unroll
+                for (int b = 0; b < 16; b++)
+                    if (ch + b < late.n) rv[it][b / 4] |= (uint32_t)ro[b] << (8 * (b & 3));
+            }
+        }
+    }
     if (gq == 0) {
 #pragma unroll
         for (int i = 0; i < SG; i++)
@@ -240,15 +323,7 @@ __global__ __launch_bounds__(WM * WN * 64, 4) void qconv_tile_kernel(const Igemm
     __syncthreads(); // the sums are there, and every wave is through with the tile: its place takes the result
     int32_t owed[RG];
 #pragma unroll
-    for (int rg = 0; rg < RG; rg++) owed[rg] = -a.zwp * sums[(wm * RG + rg) * 16 + j];
-    const int oh_img = (int)a.d_ohow.div, ow = (int)a.d_ow.div;
-    // pixel index of the tensor of pixel p of the block, a.m where there is none
-    auto pixel_of = [&](uint32_t p) __attribute__((always_inline)) {
-        const int ty = (int)fastdiv(p, t.d_tw);
-        const int oy = oy0 + ty, ox = ox0 + (int)p - ty * t.tw;
-        const int at = __mul24(oy, ow) + ox;
-        return ty < t.th && ox < ow && at < oh_img ? (int)img * oh_img + at : a.m;
-    };
+    for (int rg = 0; rg < RG; rg++) owed[rg] = -late.zwp * sums[(wm * RG + rg) * 16 + j];
     constexpr int kOutPitch = TB * 16 + 16;
     uint32_t packed[RG][T];
 #pragma unroll
@@ -258,9 +333,9 @@ __global__ __launch_bounds__(WM * WN * 64, 4) void qconv_tile_kernel(const Igemm
             int32_t v[4];
 #pragma unroll
             for (int r = 0; r < 4; r++) v[r] = acc[rg][nt][r] + owed[rg];
-            packed[rg][nt] = FAST ? requant4_u8_packed_direct(v, a.ep) : requant4_u8_packed(v, a.ep);
+            packed[rg][nt] = FAST ? requant4_u8_packed_direct(v, late.ep) : requant4_u8_packed(v, late.ep);
         }
-    if (a.lut) { // (every byte is asked for before the first is used)
+    if (late.lut) { // (every byte is asked for before the first is used)
         uint32_t b[RG][T][4];
 #pragma unroll
         for (int rg = 0; rg < RG; rg++)
@@ -281,34 +356,15 @@ __global__ __launch_bounds__(WM * WN * 64, 4) void qconv_tile_kernel(const Igemm
         for (int nt = 0; nt < T; nt++) o[nt] = packed[rg][nt];
     }
     __syncthreads();
-    // whole pixel rows: TB threads per pixel, 16 channels each
-    const bool wide_y = ((a.ldy | a.y_coff) & 3) == 0, wide_r = ((a.ldr | a.r_coff) & 3) == 0;
-    constexpr int PPT = THREADS / TB; // pixels of a pass
-    static_assert(PIX % PPT == 0, "whole passes");
-    const int cb = (tid % TB) * 16, ch = ch_base + cb;
-    if (ch >= a.n) return;
-    const bool whole = ch + 16 <= a.n;
 #pragma unroll
-    for (int it = 0; it < PIX / PPT; it++) {
-        const int p = it * PPT + tid / TB;
-        const int px = pixel_of(p);
-        if (px >= a.m) continue;
-        u32x4 v = *reinterpret_cast<const u32x4 *>(tile + p * kOutPitch + cb);
-        if (a.rep.res) {
-            const uint8_t *ro = a.rep.res + (size_t)px * a.ldr + a.r_coff + ch;
-            u32x4 rv = {0, 0, 0, 0};
-            if (whole && wide_r) {
-                const u32x4_a4 r4 = *reinterpret_cast<const u32x4_a4 *>(ro);
-                rv = u32x4{r4[0], r4[1], r4[2], r4[3]};
-            } else {
+    for (int it = 0; it < PASSES; it++) {
+        if (px[it] >= late.m) continue;
+        u32x4 v = *reinterpret_cast<const u32x4 *>(tile + (it * PPT + tid / TB) * kOutPitch + cb);
+        if (late.rep.res) {
 #pragma unroll
-                for (int b = 0; b < 16; b++)
-                    if (ch + b < a.n) rv[b / 4] |= (uint32_t)ro[b] << (8 * (b & 3));
-            }
-#pragma unroll
-            for (int d = 0; d < 4; d++) v[d] = residual4_packed(v[d], rv[d], a.rep);
+            for (int d = 0; d < 4; d++) v[d] = residual4_packed(v[d], rv[it][d], late.rep);
         }
-        uint8_t *yo = reinterpret_cast<uint8_t *>(a.y) + (size_t)px * a.ldy + a.y_coff + ch;
+        uint8_t *yo = reinterpret_cast<uint8_t *>(late.y) + (size_t)px[it] * late.ldy + late.y_coff + ch;
         if (whole && wide_y) {
             *reinterpret_cast<u32x4_a4 *>(yo) = u32x4_a4{v[0], v[1], v[2], v[3]};
         } else if (whole) {
@@ -317,7 +373,7 @@ __global__ __launch_bounds__(WM * WN * 64, 4) void qconv_tile_kernel(const Igemm
         } else {
 #pragma unroll
             for (int b = 0; b < 16; b++)
-                if (ch + b < a.n) yo[b] = (uint8_t)(v[b / 4] >> (8 * (b & 3)));
+                if (ch + b < late.n) yo[b] = (uint8_t)(v[b / 4] >> (8 * (b & 3)));
         }
     }
 }
@@ -336,11 +392,11 @@ TilePlan plan_tile(const IgemmArgs &a, int pix, int tb, int threads, int nchunks
     t.pitch = (t.pieces | 1) * 16;
     t.row_pitch = a.stride_w * t.half * t.pitch;
     t.row_bytes = a.in_w * a.ldx;
-    t.d_pieces = make_fastdiv((uint32_t)t.pieces), t.d_hc = make_fastdiv((uint32_t)t.hc), t.d_tw = make_fastdiv((uint32_t)t.tw);
+    t.d_pieces = make_tile_div(t.pieces), t.d_hc = make_tile_div(t.hc), t.d_tw = make_tile_div(t.tw);
     t.d_tx = make_fastdiv((uint32_t)o.across), t.d_txy = make_fastdiv((uint32_t)(o.across * o.down));
     t.d_nchunks = make_fastdiv((uint32_t)nchunks), t.d_rest = make_fastdiv((uint32_t)std::max(1, a.ksteps - 1));
     t.tile_off = (tb * 16 + pix + (a.ksteps + 2) * 4) * 4 + 256;
-    t.dq = threads % t.pieces, t.dc = threads / t.pieces % t.hc, t.dr = threads / t.pieces / t.hc;
+    t.apart = threads / t.pieces, t.dc = t.apart % t.hc, t.dr = t.apart / t.hc;
     p.lds = t.tile_off + std::max((size_t)t.hr * t.row_pitch, (size_t)pix * (tb * 16 + 16));
     return p;
 }
@@ -394,7 +450,7 @@ TileShape choose_tile(const nncase_hip_ctx *ctx, const IgemmArgs &a, int tiles, 
         break;
     default: return kTileNone;
     }
-    return tile_kernel_pays(TileLaunch{a.stride_w, a.ksteps, a.g_ic, pix, waves, plan->lds, plan->tiles, nchunks, a.m}, ctx->compute_units) ? shape : kTileNone;
+    return plan->t.apart > 0 && tile_kernel_pays(TileLaunch{a.stride_w, a.ksteps, a.g_ic, pix, waves, plan->lds, plan->tiles, nchunks, a.m}, ctx->compute_units) ? shape : kTileNone;
 }
 } // namespace
 

@@ -5,6 +5,8 @@
 
 namespace nnhip {
 
+__device__ __forceinline__ int tile_div(int p, uint32_t mul) { return (int)(__umul24((uint32_t)p, mul) >> 20); } // make_tile_div
+
 struct TileArgs {
     int th, tw;                    // output tile
     int hr, hc;                    // input rows / columns under it
@@ -12,10 +14,11 @@ struct TileArgs {
                                    // neighbouring output pixels read neighbouring LDS pixels)
     int pitch, row_pitch;          // bytes of an LDS pixel (an odd number of 16-byte pieces: eight lanes, eight banks) / row
     int pieces;                    // 16-byte pieces per pixel
-    int dq, dc, dr;                // a block's threads as a step in (piece, column, row)
+    int apart, dc, dr;             // whole pixels that a block's threads cover at once, and that as a step in (column, row)
     int row_bytes;                 // of the tensor
     int tile_off;
-    FastDiv d_pieces, d_hc, d_tw, d_tx, d_txy, d_nchunks, d_rest;
+    uint32_t d_pieces, d_hc, d_tw; // of make_tile_div
+    FastDiv d_tx, d_txy, d_nchunks, d_rest;
 };
 
 enum TileShape { kTile128x32, kTile64x32, kTile32x64, kTile128x128, kTile64x128, kTileNone };

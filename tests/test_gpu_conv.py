@@ -862,6 +862,24 @@ def test_convolution_over_an_input_tile_in_lds(hip_ctx, n, cin, cout, hw, k, str
     assert name.startswith("qconv_tile") and name.endswith(f"<{block}>"), name
 
 
+@pytest.mark.parametrize("n,cin,cout,hw,k,stride,dil,pad,block,extra", [
+    (18, 80, 32, (61, 97), (3, 3), (1, 1), (1, 1), ((1, 1), (1, 1)), "128x32", "add"),           # five pieces a pixel: 125 of 128 threads
+    (18, 112, 31, (60, 90), (3, 3), (1, 1), (1, 1), ((1, 1), (1, 1)), "128x32", "lut+add"),      # seven: 126; a residual of odd rows
+    (3, 176, 64, (64, 67), (3, 3), (1, 1), (1, 1), ((1, 1), (1, 1)), "32x64", "add"),           # eleven: 121
+    (8, 208, 126, (40, 41), (3, 3), (1, 1), (1, 1), ((1, 1), (1, 1)), "64x128", "lut+add"),     # thirteen: 507 of 512
+    (16, 336, 128, (44, 48), (3, 3), (2, 2), (1, 1), ((1, 1), (1, 1)), "64x128", "add"),        # 21, several batches of each thread
+    (2, 2048, 32, (25, 40), (1, 3), (1, 1), (1, 1), ((0, 0), (1, 1)), None, ""),                # a pixel for all threads of a block
+    (2, 2064, 32, (25, 40), (1, 3), (1, 1), (1, 1), ((0, 0), (1, 1)), None, "add")])            # more pieces than threads: another kernel
+def test_threads_past_the_last_whole_pixel_of_a_tile(hip_ctx, n, cin, cout, hw, k, stride, dil, pad, block, extra):
+    """Pieces of a pixel that do not divide a block's threads: those past the last whole pixel bring nothing in; and the residual's
+    bytes, asked for ahead of the sums, at rows that start inside a dword."""
+    if block is None:
+        with pytest.raises(AssertionError, match=r"^qconv_[^:\n]*\n"):  # (the bytes agree: what fails is the kernel's name)
+            test_convolution_over_an_input_tile_in_lds(hip_ctx, n, cin, cout, hw, k, stride, dil, pad, "none", extra)
+    else:
+        test_convolution_over_an_input_tile_in_lds(hip_ctx, n, cin, cout, hw, k, stride, dil, pad, block, extra)
+
+
 @pytest.mark.parametrize("m,k,n", [(16500, 516, 300), (16641, 1020, 258), (33000, 532, 257)])
 def test_matmul_of_rows_of_whole_dwords_in_256_channel_blocks(hip_ctx, m, k, n):
     """Rows that are no multiple of 16 bytes, moved straight to LDS in 256 x 256 blocks: last k-steps that end inside a piece, partial

@@ -19,6 +19,7 @@ extern "C" void tile(int h, int w, int pix, int sh, int sw, int kh, int kw, int 
     const nnhip::OutputTile t = nnhip::choose_output_tile(h, w, pix, sh, sw, kh, kw);
     out[0] = t.th, out[1] = t.tw, out[2] = t.across, out[3] = t.down, out[4] = t.in_rows, out[5] = t.in_cols;
 }
+extern "C" int tile_div(int p, int d) { return (int)((uint32_t)p * nnhip::make_tile_div(d) >> 20); }
 extern "C" int wide(int oc, int ksteps, int tiles) { return nnhip::small_wide_pays(oc, ksteps, tiles); }
 extern "C" int window(int stride, int ksteps, int channels, int pix, int waves, long lds, long tiles, long chunks, long pixels) {
     return nnhip::tile_kernel_pays({stride, ksteps, channels, pix, waves, (size_t)lds, tiles, chunks, pixels}, 256);
@@ -133,6 +134,13 @@ def test_output_tile_is_the_best_of_all_numbers_of_tiles(rules, pix, stride, spa
                     break
             rules.tile(h, w, pix, stride, stride, span, span, got)
             assert list(got) == best[1], (h, w)
+
+
+def test_division_of_a_tile(rules):
+    for d in list(range(1, 1100)) + [4095, 10240, (1 << 20) - 1, 1 << 20, 1 << 24]:
+        assert [rules.tile_div(p, d) for p in range(512)] == [p // d for p in range(512)], d
+    # (24-bit operands, 32-bit product: the largest of both)
+    assert 511 << 20 < 1 << 32 and 1 << 20 < 1 << 24
 
 
 # windows of a group's channels -> outputs, window side, stride; k-steps; pixels and waves per block, LDS, tiles, chunks, output pixels;
