@@ -168,7 +168,7 @@ inline OutputTile choose_output_tile(int out_h, int out_w, int pix, int stride_h
 // A division of what counts the window kernel's threads or pixels, two instructions: p / d = p * mul >> 20 for 0 <= p < kTileDivMost and
 // every d >= 1.  (mul is less than 1 above 2^20 / d, so the product less than p above 2^20 p / d: short of the next whole number while
 // p d < 2^20, and of the first while p < d, which covers every larger d.)
-constexpr int kTileDivMost = 512;
+constexpr int kTileDivMost = 1024;
 inline uint32_t make_tile_div(int d) { return ((1u << 20) + (uint32_t)d - 1) / (uint32_t)d; }
 
 // Whether a launch of the window kernel as planned is quicker than the implicit GEMM of the same layer (byte results, strides of 1
@@ -205,6 +205,19 @@ inline bool tile_kernel_pays(const TileLaunch &l, int compute_units) {
     if (l.stride_w == 2 && resident < 5) return false;
     if (l.pix < 128 && l.channels > 400 && resident < 4) return false;
     return l.pix > 32 || (l.ksteps >= 5 && launched <= 9ll * l.ksteps * compute_units);
+}
+
+// Whether groups of waves that share a block's k-steps (TileLaunch::waves counts all of them) are quicker in the window kernel than
+// whatever else the layer would take: all blocks run at once, with no more than eight waves to a compute unit, of which at least four
+// come from what fits into its LDS side by side.  us, without / with: 128 -> 128 3x3 of 1600 pixels 5.3 / 4.0, 256 -> 256 of 400 6.8 / 4.7,
+// 512 -> 512 of 400 11.0 / 7.9, 64 -> 64 of 1600 4.5 / 3.8, 256 -> 24 7x7 of 1083 24.3 / 7.8, 32 -> 32 of 6400 4.2 / 3.5; past eight waves
+// 80 -> 32 of 51 200 5.6 / 6.1, 128 -> 160 of 12 288 8.2 / 8.9; too few side by side 512 -> 160 stride 2 of 1352 12.1 / 14.0.
+// (Of 338 launches of 60 to 60 000 pixels 1.37 times as quick in the mean, 1.2 % off the quickest of all shapes.)
+inline long long split_window_waves(int compute_units) { return 8ll * compute_units; }
+inline bool split_window_pays(const TileLaunch &l, int compute_units) {
+    if (l.lds > 160 * 1024) return false;
+    const long long blocks = l.tiles * l.chunks, resident = (long long)(160 * 1024 / l.lds);
+    return blocks * l.waves <= split_window_waves(compute_units) && blocks <= resident * compute_units && resident * l.waves >= 4;
 }
 
 // Whether two dense 1x1 convolutions, the second over the first one's result, are quicker as a pair than as two launches: while every

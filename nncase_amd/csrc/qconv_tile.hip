@@ -16,6 +16,9 @@
 //     requests in one trip and those of the stores in another, a thread that keeps its piece of a pixel (two multiply-adds an address,
 //     short divisions), a channel's terms asked for first.  Start to end of a block, 6400 pixels 64 -> 64 3x3 with a residual 4.6 us ->
 //     3.7 (before the first request 0.6 -> 0.4, requests 0.5 -> 0.3, results 1.1 -> 0.5), 409 600 pixels 32 -> 32 21.8 -> 19.2 a launch.
+//   * a launch of few blocks splits each one's k-steps between groups of waves, which meet once: up to four k-steps of every group are on
+//     their way when the first product starts, where the ring of qconv_wide_kernel goes through a barrier for each.  In a chain, us there /
+//     here: 128 -> 128 3x3 of 1600 pixels 5.3 / 4.0, 256 -> 256 of 400 6.8 / 4.7, 512 -> 512 of 400 11.0 / 7.9.
 // Arithmetic, weight packing and the bytes of the result are those of qconv_igemm.hpp.
 #include "qconv_rules.hpp"
 #include "qconv_tile.hpp"
@@ -46,16 +49,19 @@ template <bool FAST> __device__ __forceinline__ IgemmArgs gather_store_args() {
 }
 
 // FAST: the requantisation is the one-instruction form without a clamp of its own (Epilogue::fast and ::full).
-template <int T, int RG, int WM, int WN, bool FAST>
-__global__ __launch_bounds__(WM * WN * 64, 4) void qconv_tile_kernel(const IgemmArgs a, const TileArgs t) {
-    constexpr int THREADS = WM * WN * 64, PIX = WM * RG * 16, TB = T * WN;
+// KG > 1: KG groups of WM x WN waves share the reduction, every KG-th k-step each, and add their sums up at the end.
+template <int T, int RG, int WM, int WN, int KG, bool FAST>
+__global__ __launch_bounds__(WM * WN * KG * 64, 4) void qconv_tile_kernel(const IgemmArgs a, const TileArgs t) {
+    constexpr int THREADS = WM * WN * KG * 64, PIX = WM * RG * 16, TB = T * WN;
     constexpr int D = 4;                                             // k-steps of weights in flight
+    constexpr int UNITS = RG * T, EACH = (UNITS + KG - 1) / KG;      // results of a wave, 16 pixels x 16 channels; those that a group finishes
     static_assert(TB * 16 <= THREADS && THREADS <= kTileDivMost, "a thread per channel, tile_div");
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
     int32_t *cterm = reinterpret_cast<int32_t *>(smem);              // [TB * 16]
-    int32_t *sums = cterm + TB * 16;                                 // [PIX] sum of x' over a pixel's window
-    uint8_t *lutl = reinterpret_cast<uint8_t *>(sums + PIX);         // [256]
-    int32_t *taps = reinterpret_cast<int32_t *>(lutl + 256);         // [KS + 2][4] LDS offset of a piece of the reduction
+    int32_t *sums = cterm + TB * 16;                                 // [KG][PIX] sum of x' over a group's share of a pixel's window
+    uint8_t *lutl = reinterpret_cast<uint8_t *>(sums + KG * PIX);    // [256]
+    v4i *parts = reinterpret_cast<v4i *>(lutl + 256);                // [UNITS][KG - 1][waves of a group][64] sums on their way to the group that finishes them
+    int32_t *taps = reinterpret_cast<int32_t *>(lutl + 256 + tile_part_bytes(UNITS, WM * WN, KG)); // [KS + 2 KG][4] LDS offset of a piece of the reduction
     uint8_t *tile = smem + t.tile_off;
 
     // (what the requests need, in one trip; see gather_store_args for the rest)
@@ -73,7 +79,8 @@ __global__ __launch_bounds__(WM * WN * 64, 4) void qconv_tile_kernel(const Igemm
     if (turn >= per || mt >= a.num_mtiles) return;
 
     const int tid = threadIdx.x, lane = tid & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int bwave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int kg = KG == 1 ? 0 : bwave / (WM * WN), wave = bwave - kg * (WM * WN);
     const int wm = wave % WM, wn = wave / WM;
     const int j = lane & 15, gq = lane >> 4;
     const int KS = a.ksteps;
@@ -161,29 +168,39 @@ __global__ __launch_bounds__(WM * WN * 64, 4) void qconv_tile_kernel(const Igemm
     request(fa, 0);
 
     // ---- weights: D k-steps ahead.  The last k-step, which may end past the reduction, comes first, the others follow from
-    // where this block starts ----
+    // where this block starts; group kg takes the kg-th of that order and every KG-th from there ----
     const __amdgpu_buffer_rsrc_t wres = wide_rsrc(a.wpk + (size_t)chunk * KS * TB * 1024, (uint32_t)KS * TB * 1024);
     const int rest = KS - 1;
     const int ks0 = rest == 0 ? 0 : seq - (int)fastdiv((uint32_t)seq, t.d_rest) * rest;
     const int w_end = rest * TB * 1024, w_lane = wn * T * 1024 + lane * 16;
-    int w_off = rest * TB * 1024; // of the next k-step to request
+    int w_off = w_end; // of the next k-step to request
     auto load_w = [&](v4i (&dst)[T]) __attribute__((always_inline)) {
 #pragma unroll
         for (int nt = 0; nt < T; nt++) dst[nt] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(wres, w_lane + nt * 1024, w_off, 0));
     };
-    v4i wf[D][T];
-    load_w(wf[0]);
-    w_off = ks0 * TB * 1024;
+    auto advance = [&](int ksteps) __attribute__((always_inline)) { // (of at most `rest`: choose_tile)
+        w_off += ksteps * (TB * 1024);
+        w_off -= w_off >= w_end ? w_end : 0;
+    };
     auto load_next = [&](v4i (&dst)[T]) __attribute__((always_inline)) {
         load_w(dst);
-        w_off += TB * 1024;
-        w_off = w_off == w_end ? 0 : w_off;
+        advance(KG);
     };
+    v4i wf[D][T];
+    if (KG == 1 || kg == 0) {
+        load_w(wf[0]);
+        w_off = ks0 * TB * 1024;
+        if (KG > 1) advance(KG - 1);
+    } else {
+        w_off = ks0 * TB * 1024;
+        advance(kg - 1);
+        load_next(wf[0]);
+    }
 #pragma unroll
     for (int d = 1; d < D; d++) load_next(wf[d]);
 
     // ---- tables ----
-    for (int e = tid; e < (KS + 2) * 4; e += THREADS) { // in the order of this block's k-steps
+    for (int e = tid; e < (KS + 2 * KG) * 4; e += THREADS) { // in the order of this block's k-steps
         const int s = e >> 2;
         int ks = s == 0 ? rest : ks0 + s - 1;
         ks -= s > 0 && ks >= rest ? rest : 0;
@@ -231,25 +248,26 @@ __global__ __launch_bounds__(WM * WN * 64, 4) void qconv_tile_kernel(const Igemm
     const int ch0 = gq * (4 * TB) + wn * (4 * T);
     v4i acc[RG][T], rs[SG];
     v4i xf[2][RG], xs[2][SG]; // (a wave reads the operand it sums by itself: which of xf that is depends on the wave)
-    const int32_t *tap = taps + gq; // of the k-step whose operands are read next
+    const int32_t *tap = taps + kg * 4 + gq; // of the k-step whose operands are read next
     int toff = tap[0];
     auto operands = [&](v4i (&dst)[RG], v4i (&dsts)[SG], int ahead) __attribute__((always_inline)) {
 #pragma unroll
         for (int rg = 0; rg < RG; rg++) dst[rg] = *reinterpret_cast<const v4i *>(tile + xbase[rg] + toff);
 #pragma unroll
         for (int i = 0; i < SG; i++) dsts[i] = WN == 1 ? dst[i] : *reinterpret_cast<const v4i *>(tile + xsum[i] + toff);
-        toff = tap[ahead * 4];
+        toff = tap[ahead * (4 * KG)];
     };
     operands(xf[0], xs[0], 1);
     operands(xf[1], xs[1], 2);
-    tap += 2 * 4;
+    tap += 2 * (4 * KG);
     const v4i ones = {0x01010101, 0x01010101, 0x01010101, 0x01010101};
     {
-        const int one = rest * 64 + gq * 16 < a.k ? 0x01010101 : 0; // (pieces past the reduction)
+        const int one = kg > 0 || rest * 64 + gq * 16 < a.k ? 0x01010101 : 0; // (pieces past the reduction)
         const v4i ones_last = {one, one, one, one}, zero = {0, 0, 0, 0};
 #pragma unroll
         for (int nt = 0; nt < T; nt++) {
-            const v4i ct = *reinterpret_cast<const v4i *>(cterm + ch0 + nt * 4);
+            v4i ct = *reinterpret_cast<const v4i *>(cterm + ch0 + nt * 4);
+            if (KG > 1 && kg > 0) ct = zero;
 #pragma unroll
             for (int rg = 0; rg < RG; rg++) acc[rg][nt] = __builtin_amdgcn_mfma_i32_16x16x64_i8(wf[0][nt], xf[0][rg], ct, 0, 0, 0);
         }
@@ -271,11 +289,11 @@ __global__ __launch_bounds__(WM * WN * 64, 4) void qconv_tile_kernel(const Igemm
         __builtin_amdgcn_sched_barrier(0);
         load_next(wf[b]);
     };
-    int left = rest;
+    int left = KG == 1 ? rest : (rest - kg) / KG;
 #pragma clang loop unroll(disable)
     for (; left >= D; left -= D) {
         static_for<1, D + 1>(kstep);
-        tap += D * 4;
+        tap += D * (4 * KG);
     }
     static_for<1, D>([&](auto u_c) __attribute__((always_inline)) {
         if (decltype(u_c)::value <= left) kstep(u_c);
@@ -283,7 +301,7 @@ __global__ __launch_bounds__(WM * WN * 64, 4) void qconv_tile_kernel(const Igemm
 
     // ---- epilogue ----
     // whole pixel rows: TB threads per pixel, 16 channels each.  Their bytes of the residual are asked for before the sums meet.
-    constexpr int PPT = THREADS / TB, PASSES = PIX / PPT; // pixels of a pass
+    constexpr int PPT = THREADS / TB < PIX ? THREADS / TB : PIX, PASSES = PIX / PPT; // pixels of a pass
     static_assert(PIX % PPT == 0, "whole passes");
     const int oh_img = (int)late.d_ohow.div, ow = (int)late.d_ow.div;
     const int cb = (tid % TB) * 16, ch = ch_base + cb;
@@ -296,7 +314,7 @@ __global__ __launch_bounds__(WM * WN * 64, 4) void qconv_tile_kernel(const Igemm
         const int ty = tile_div(p, t.d_tw);
         const int oy = oy0 + ty, ox = ox0 + p - __mul24(ty, t.tw);
         const int at = __mul24(oy, ow) + ox;
-        px[it] = ty < t.th && ox < ow && at < oh_img && ch < late.n ? (int)img * oh_img + at : late.m;
+        px[it] = p < PIX && ty < t.th && ox < ow && at < oh_img && ch < late.n ? (int)img * oh_img + at : late.m;
     }
     if (late.rep.res) {
         const bool wide_r = ((late.ldr | late.r_coff) & 3) == 0;
@@ -318,42 +336,68 @@ __global__ __launch_bounds__(WM * WN * 64, 4) void qconv_tile_kernel(const Igemm
     if (gq == 0) {
 #pragma unroll
         for (int i = 0; i < SG; i++)
-            if (wn * SG + i < RG) sums[(wm * RG + wn * SG + i) * 16 + j] = rs[i][0];
+            if (wn * SG + i < RG) sums[kg * PIX + (wm * RG + wn * SG + i) * 16 + j] = rs[i][0];
+    }
+    // (unit u of a wave: pixel group u / T, channel tile u % T; group u / EACH finishes it)
+    auto part = [&](int u, int from) __attribute__((always_inline)) { return parts + ((u * (KG - 1) + from) * (WM * WN) + wave) * 64 + lane; };
+    if constexpr (KG > 1) {
+        static_for<0, UNITS>([&](auto u_c) __attribute__((always_inline)) {
+            constexpr int u = decltype(u_c)::value, by = u / EACH;
+            if (kg != by) *part(u, kg - (kg > by ? 1 : 0)) = acc[u / T][u % T];
+        });
     }
     __syncthreads(); // the sums are there, and every wave is through with the tile: its place takes the result
-    int32_t owed[RG];
-#pragma unroll
-    for (int rg = 0; rg < RG; rg++) owed[rg] = -late.zwp * sums[(wm * RG + rg) * 16 + j];
     constexpr int kOutPitch = TB * 16 + 16;
-    uint32_t packed[RG][T];
+    auto finish = [&](auto first_c) __attribute__((always_inline)) { // the EACH units from there on
+        constexpr int first = decltype(first_c)::value, count = KG == 1 ? UNITS : (UNITS - first < EACH ? UNITS - first : EACH);
+        int32_t owed[RG];
 #pragma unroll
-    for (int rg = 0; rg < RG; rg++)
+        for (int rg = first / T; rg <= (first + count - 1) / T; rg++) {
+            int32_t sum = sums[(wm * RG + rg) * 16 + j];
 #pragma unroll
-        for (int nt = 0; nt < T; nt++) {
+            for (int g = 1; g < KG; g++) sum += sums[g * PIX + (wm * RG + rg) * 16 + j];
+            owed[rg] = -late.zwp * sum;
+        }
+        uint32_t packed[count];
+        if constexpr (KG > 1) {
+            v4i others[count][KG - 1];
+#pragma unroll
+            for (int u = 0; u < count; u++)
+#pragma unroll
+                for (int from = 0; from < KG - 1; from++) others[u][from] = *part(first + u, from);
+#pragma unroll
+            for (int u = 0; u < count; u++)
+#pragma unroll
+                for (int from = 0; from < KG - 1; from++) acc[(first + u) / T][(first + u) % T] += others[u][from];
+        }
+#pragma unroll
+        for (int u = 0; u < count; u++) {
+            const int rg = (first + u) / T, nt = (first + u) % T;
             int32_t v[4];
 #pragma unroll
             for (int r = 0; r < 4; r++) v[r] = acc[rg][nt][r] + owed[rg];
-            packed[rg][nt] = FAST ? requant4_u8_packed_direct(v, late.ep) : requant4_u8_packed(v, late.ep);
+            packed[u] = FAST ? requant4_u8_packed_direct(v, late.ep) : requant4_u8_packed(v, late.ep);
         }
-    if (late.lut) { // (every byte is asked for before the first is used)
-        uint32_t b[RG][T][4];
+        if (late.lut) { // (every byte is asked for before the first is used)
+            uint32_t b[count][4];
 #pragma unroll
-        for (int rg = 0; rg < RG; rg++)
+            for (int u = 0; u < count; u++)
 #pragma unroll
-            for (int nt = 0; nt < T; nt++)
+                for (int r = 0; r < 4; r++) b[u][r] = lutl[(packed[u] >> (8 * r)) & 0xffu];
+            __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-                for (int r = 0; r < 4; r++) b[rg][nt][r] = lutl[(packed[rg][nt] >> (8 * r)) & 0xffu];
-        __builtin_amdgcn_sched_barrier(0);
+            for (int u = 0; u < count; u++) packed[u] = b[u][0] | (b[u][1] << 8) | (b[u][2] << 16) | (b[u][3] << 24);
+        }
 #pragma unroll
-        for (int rg = 0; rg < RG; rg++)
-#pragma unroll
-            for (int nt = 0; nt < T; nt++) packed[rg][nt] = b[rg][nt][0] | (b[rg][nt][1] << 8) | (b[rg][nt][2] << 16) | (b[rg][nt][3] << 24);
-    }
-#pragma unroll
-    for (int rg = 0; rg < RG; rg++) {
-        uint32_t *o = reinterpret_cast<uint32_t *>(tile + ((wm * RG + rg) * 16 + j) * kOutPitch + ch0);
-#pragma unroll
-        for (int nt = 0; nt < T; nt++) o[nt] = packed[rg][nt];
+        for (int u = 0; u < count; u++)
+            *reinterpret_cast<uint32_t *>(tile + ((wm * RG + (first + u) / T) * 16 + j) * kOutPitch + ch0 + (first + u) % T * 4) = packed[u];
+    };
+    if constexpr (KG == 1) {
+        finish(std::integral_constant<int, 0>());
+    } else {
+        static_for<0, (UNITS + EACH - 1) / EACH>([&](auto g_c) __attribute__((always_inline)) {
+            if (kg == decltype(g_c)::value) finish(std::integral_constant<int, decltype(g_c)::value * EACH>());
+        });
     }
     __syncthreads();
 #pragma unroll
@@ -379,8 +423,8 @@ __global__ __launch_bounds__(WM * WN * 64, 4) void qconv_tile_kernel(const Igemm
 }
 
 namespace {
-// The plan of a kernel with `pix` pixels and `tb` 16-channel tiles per block.
-TilePlan plan_tile(const IgemmArgs &a, int pix, int tb, int threads, int nchunks) {
+// The plan of a kernel with `pix` pixels and `tb` 16-channel tiles per block; `groups` of waves, whose sums take `parts` bytes, share its k-steps.
+TilePlan plan_tile(const IgemmArgs &a, int pix, int tb, int threads, int nchunks, int groups, int parts) {
     const int ow = (int)a.d_ow.div, oh = (int)a.d_ohow.div / ow, batch = a.m / (int)a.d_ohow.div;
     const OutputTile o = choose_output_tile(oh, ow, pix, a.stride_h, a.stride_w, (a.kh - 1) * a.dil_h + 1, (a.kw - 1) * a.dil_w + 1);
     TilePlan p;
@@ -395,29 +439,50 @@ TilePlan plan_tile(const IgemmArgs &a, int pix, int tb, int threads, int nchunks
     t.d_pieces = make_tile_div(t.pieces), t.d_hc = make_tile_div(t.hc), t.d_tw = make_tile_div(t.tw);
     t.d_tx = make_fastdiv((uint32_t)o.across), t.d_txy = make_fastdiv((uint32_t)(o.across * o.down));
     t.d_nchunks = make_fastdiv((uint32_t)nchunks), t.d_rest = make_fastdiv((uint32_t)std::max(1, a.ksteps - 1));
-    t.tile_off = (tb * 16 + pix + (a.ksteps + 2) * 4) * 4 + 256;
+    t.tile_off = (tb * 16 + groups * pix + (a.ksteps + 2 * groups) * 4) * 4 + 256 + parts;
     t.apart = threads / t.pieces, t.dc = t.apart % t.hc, t.dr = t.apart / t.hc;
     p.lds = t.tile_off + std::max((size_t)t.hr * t.row_pitch, (size_t)pix * (tb * 16 + 16));
     return p;
 }
 
-template <int T, int RG, int WM, int WN, bool FAST> int launch_tile_f(nncase_hip_ctx *ctx, const IgemmArgs &args, const TilePlan &plan, int nchunks) {
-    if (plan.lds > 65536) NNHIP_HIP(ctx, (raise_dynamic_lds<qconv_tile_kernel<T, RG, WM, WN, FAST>>(ctx->device, 160 * 1024)));
-    hipLaunchKernelGGL((qconv_tile_kernel<T, RG, WM, WN, FAST>), dim3(ceil_div(args.num_mtiles, 8) * 8 * nchunks), dim3(WM * WN * 64), plan.lds, ctx->stream, args,
+template <int T, int RG, int WM, int WN, int KG, bool FAST> int launch_tile_f(nncase_hip_ctx *ctx, const IgemmArgs &args, const TilePlan &plan, int nchunks) {
+    if (plan.lds > 65536) NNHIP_HIP(ctx, (raise_dynamic_lds<qconv_tile_kernel<T, RG, WM, WN, KG, FAST>>(ctx->device, 160 * 1024)));
+    hipLaunchKernelGGL((qconv_tile_kernel<T, RG, WM, WN, KG, FAST>), dim3(ceil_div(args.num_mtiles, 8) * 8 * nchunks), dim3(WM * WN * KG * 64), plan.lds, ctx->stream, args,
                        plan.t);
     NNHIP_LAUNCH_CHECK(ctx, "qconv_tile_kernel");
     return 0;
 }
-template <int T, int RG, int WM, int WN> int launch_tile_t(nncase_hip_ctx *ctx, const IgemmArgs &a, const TilePlan &plan, int nchunks) {
+template <int T, int RG, int WM, int WN, int KG = 1> int launch_tile_t(nncase_hip_ctx *ctx, const IgemmArgs &a, const TilePlan &plan, int nchunks) {
     IgemmArgs args = a;
     args.num_mtiles = plan.tiles;
-    return a.ep.fast && a.ep.full ? launch_tile_f<T, RG, WM, WN, true>(ctx, args, plan, nchunks) : launch_tile_f<T, RG, WM, WN, false>(ctx, args, plan, nchunks);
+    return a.ep.fast && a.ep.full ? launch_tile_f<T, RG, WM, WN, KG, true>(ctx, args, plan, nchunks) : launch_tile_f<T, RG, WM, WN, KG, false>(ctx, args, plan, nchunks);
 }
 } // namespace
 
 namespace {
-template <int T, int RG, int WM, int WN> TilePlan plan_shape(const IgemmArgs &a, int nchunks) {
-    return plan_tile(a, WM * RG * 16, T * WN, WM * WN * 64, nchunks);
+template <int T, int RG, int WM, int WN, int KG = 1> TilePlan plan_shape(const IgemmArgs &a, int nchunks) {
+    return plan_tile(a, WM * RG * 16, T * WN, WM * WN * KG * 64, nchunks, KG, tile_part_bytes(RG * T, WM * WN, KG));
+}
+
+// A launch of few blocks: the smallest tile first, four groups before two.
+template <int T, int RG, int WM, int WN, int KG> bool split_tile(const nncase_hip_ctx *ctx, const IgemmArgs &a, int nchunks, TilePlan *plan) {
+    if (a.ksteps <= KG || (long long)ceil_div(a.m, WM * RG * 16) * nchunks * WM * WN * KG > split_window_waves(ctx->compute_units)) return false;
+    *plan = plan_shape<T, RG, WM, WN, KG>(a, nchunks);
+    return plan->t.apart > 0 && split_window_pays(TileLaunch{a.stride_w, a.ksteps, a.g_ic, WM * RG * 16, WM * WN * KG, plan->lds, plan->tiles, nchunks, a.m}, ctx->compute_units);
+}
+TileShape choose_split_tile(const nncase_hip_ctx *ctx, const IgemmArgs &a, int tiles, int nchunks, TilePlan *plan) {
+    if (tiles == 4) {
+        if (a.ksteps < 7) return kTileNone; // (five or six: 32 -> 100 3x3 of 400 pixels 3.9 by the k-steps' ring, 4.1 so)
+        if (split_tile<2, 1, 1, 2, 4>(ctx, a, nchunks, plan)) return kTile16x64by4;
+        if (split_tile<2, 2, 1, 2, 4>(ctx, a, nchunks, plan)) return kTile32x64by4;
+        if (split_tile<2, 2, 1, 2, 2>(ctx, a, nchunks, plan)) return kTile32x64by2;
+    } else if (tiles == 2) {
+        if (a.ksteps < 5) return kTileNone;
+        if (split_tile<2, 1, 1, 1, 4>(ctx, a, nchunks, plan)) return kTile16x32by4;
+        if (split_tile<2, 2, 1, 1, 4>(ctx, a, nchunks, plan)) return kTile32x32by4;
+        if (split_tile<2, 2, 1, 1, 2>(ctx, a, nchunks, plan)) return kTile32x32by2;
+    }
+    return kTileNone;
 }
 
 // Which block, if any, by the packed chunk (`tiles` of 16 channels) and the waves the launch has (byte results, windows,
@@ -431,8 +496,7 @@ template <int T, int RG, int WM, int WN> TilePlan plan_shape(const IgemmArgs &a,
 //   * stride 2 brings in four times the input: from 16 k-steps on (25 600 pixels 128 -> 256 18.5 / 15.9, 6400 pixels 256 -> 512
 //     18.0 / 15.5, but 409 600 pixels 32 -> 64, five k-steps, 28.2 / 30.3);
 //   * and what tile_kernel_pays asks of the launch.
-TileShape choose_tile(const nncase_hip_ctx *ctx, const IgemmArgs &a, int tiles, int nchunks, TilePlan *plan) {
-    if (a.kh * a.kw == 1 || a.g_ic % 16 != 0 || a.kc_mask != -1 || a.stride_w > 2 || (int64_t)a.in_w * a.ldx >= (1 << 23)) return kTileNone;
+TileShape choose_whole_tile(const nncase_hip_ctx *ctx, const IgemmArgs &a, int tiles, int nchunks, TilePlan *plan) {
     if (a.ksteps < (a.stride_w == 2 ? 16 : 3)) return kTileNone;
     TileShape shape = kTileNone;
     int waves = 2, pix = 64;
@@ -452,10 +516,22 @@ TileShape choose_tile(const nncase_hip_ctx *ctx, const IgemmArgs &a, int tiles, 
     }
     return plan->t.apart > 0 && tile_kernel_pays(TileLaunch{a.stride_w, a.ksteps, a.g_ic, pix, waves, plan->lds, plan->tiles, nchunks, a.m}, ctx->compute_units) ? shape : kTileNone;
 }
+TileShape choose_tile(const nncase_hip_ctx *ctx, const IgemmArgs &a, int tiles, int nchunks, TilePlan *plan) {
+    if (a.kh * a.kw == 1 || a.g_ic % 16 != 0 || a.kc_mask != -1 || a.stride_w > 2 || (int64_t)a.in_w * a.ldx >= (1 << 23)) return kTileNone;
+    // Fewer than ten k-steps are split where one group is no choice (three waves for two compute units and more: 64 -> 64 of 6400 pixels
+    // 4.2 / 4.0, 48 -> 32 of 25 600 4.5 / 4.2, 32 -> 48 of 12 800 4.1 / 4.2).
+    if (a.ksteps >= 10) {
+        const TileShape split = choose_split_tile(ctx, a, tiles, nchunks, plan);
+        if (split != kTileNone) return split;
+    }
+    const TileShape whole = choose_whole_tile(ctx, a, tiles, nchunks, plan);
+    return whole != kTileNone || a.ksteps >= 10 ? whole : choose_split_tile(ctx, a, tiles, nchunks, plan);
+}
 } // namespace
 
 const char *tile_kernel_block(const nncase_hip_ctx *ctx, const nncase_hip_weights *w, const nncase_hip_conv2d_args_t *c, int out_h, int out_w) {
-    static const char *const names[] = {"128x32", "64x32", "32x64", "128x128", "64x128", nullptr};
+    static const char *const names[] = {"128x32", "64x32", "32x64", "128x128", "64x128", "32x32,KG=2", "32x32,KG=4", "16x32,KG=4", "32x64,KG=2",
+                                        "32x64,KG=4", "16x64,KG=4", nullptr};
     if (w->ragged || c->out_dtype != NNCASE_HIP_DT_U8 || c->dequantize_output) return nullptr;
     IgemmArgs a;
     memset(&a, 0, sizeof(a));
@@ -481,6 +557,12 @@ int launch_qconv_tile(nncase_hip_ctx *ctx, const IgemmArgs &a, const TilePlan &p
     case kTile32x64: return launch_tile_t<2, 2, 1, 2>(ctx, a, plan, nchunks);
     case kTile128x128: return launch_tile_t<2, 4, 2, 4>(ctx, a, plan, nchunks);
     case kTile64x128: return launch_tile_t<2, 2, 2, 4>(ctx, a, plan, nchunks);
+    case kTile32x32by2: return launch_tile_t<2, 2, 1, 1, 2>(ctx, a, plan, nchunks);
+    case kTile32x32by4: return launch_tile_t<2, 2, 1, 1, 4>(ctx, a, plan, nchunks);
+    case kTile16x32by4: return launch_tile_t<2, 1, 1, 1, 4>(ctx, a, plan, nchunks);
+    case kTile32x64by2: return launch_tile_t<2, 2, 1, 2, 2>(ctx, a, plan, nchunks);
+    case kTile32x64by4: return launch_tile_t<2, 2, 1, 2, 4>(ctx, a, plan, nchunks);
+    case kTile16x64by4: return launch_tile_t<2, 1, 1, 2, 4>(ctx, a, plan, nchunks);
     case kTileNone: break;
     }
     return fail(ctx, -EINVAL, "qconv2d: not a layer of the tile kernel");

@@ -7,6 +7,9 @@ namespace nnhip {
 
 __device__ __forceinline__ int tile_div(int p, uint32_t mul) { return (int)(__umul24((uint32_t)p, mul) >> 20); } // make_tile_div
 
+// LDS for the sums of `units` results of each wave that the groups of a split reduction pass on.
+constexpr int tile_part_bytes(int units, int waves, int groups) { return units * (groups - 1) * waves * 1024; }
+
 struct TileArgs {
     int th, tw;                    // output tile
     int hr, hc;                    // input rows / columns under it
@@ -21,7 +24,12 @@ struct TileArgs {
     FastDiv d_tx, d_txy, d_nchunks, d_rest;
 };
 
-enum TileShape { kTile128x32, kTile64x32, kTile32x64, kTile128x128, kTile64x128, kTileNone };
+// Pixels x channels of a block; by n: its k-steps shared by n groups of waves.
+enum TileShape {
+    kTile128x32, kTile64x32, kTile32x64, kTile128x128, kTile64x128,
+    kTile32x32by2, kTile32x32by4, kTile16x32by4, kTile32x64by2, kTile32x64by4, kTile16x64by4,
+    kTileNone
+};
 
 struct TilePlan {
     TileShape shape = kTileNone;

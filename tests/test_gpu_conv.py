@@ -865,7 +865,7 @@ def test_convolution_over_an_input_tile_in_lds(hip_ctx, n, cin, cout, hw, k, str
 @pytest.mark.parametrize("n,cin,cout,hw,k,stride,dil,pad,block,extra", [
     (18, 80, 32, (61, 97), (3, 3), (1, 1), (1, 1), ((1, 1), (1, 1)), "128x32", "add"),           # five pieces a pixel: 125 of 128 threads
     (18, 112, 31, (60, 90), (3, 3), (1, 1), (1, 1), ((1, 1), (1, 1)), "128x32", "lut+add"),      # seven: 126; a residual of odd rows
-    (3, 176, 64, (64, 67), (3, 3), (1, 1), (1, 1), ((1, 1), (1, 1)), "32x64", "add"),           # eleven: 121
+    (3, 176, 64, (64, 67), (3, 3), (1, 1), (1, 1), ((1, 1), (1, 1)), "32x64,KG=2", "add"),      # eleven: 242 of 256
     (8, 208, 126, (40, 41), (3, 3), (1, 1), (1, 1), ((1, 1), (1, 1)), "64x128", "lut+add"),     # thirteen: 507 of 512
     (16, 336, 128, (44, 48), (3, 3), (2, 2), (1, 1), ((1, 1), (1, 1)), "64x128", "add"),        # 21, several batches of each thread
     (2, 2048, 32, (25, 40), (1, 3), (1, 1), (1, 1), ((0, 0), (1, 1)), None, ""),                # a pixel for all threads of a block
@@ -878,6 +878,24 @@ def test_threads_past_the_last_whole_pixel_of_a_tile(hip_ctx, n, cin, cout, hw, 
             test_convolution_over_an_input_tile_in_lds(hip_ctx, n, cin, cout, hw, k, stride, dil, pad, "none", extra)
     else:
         test_convolution_over_an_input_tile_in_lds(hip_ctx, n, cin, cout, hw, k, stride, dil, pad, block, extra)
+
+
+@pytest.mark.parametrize("n,cin,cout,hw,k,stride,dil,pad,block,extra", [
+    (1, 64, 100, (19, 23), (3, 3), (1, 1), (1, 1), ((1, 1), (1, 1)), "16x64,KG=4", "lut+add"),    # nine k-steps: one group has one more
+    (1, 64, 60, (15, 20), (7, 1), (1, 1), (1, 1), ((3, 3), (0, 0)), "16x64,KG=4", "slice"),       # seven: one group has one less
+    (1, 272, 64, (13, 9), (3, 3), (2, 1), (2, 1), ((2, 2), (1, 1)), "16x64,KG=4", "clamp"),       # a last step that is a quarter full
+    (1, 32, 64, (3, 2), (5, 3), (1, 1), (1, 1), ((2, 2), (1, 1)), "16x64,KG=4", "add"),           # an image smaller than a tile
+    (2, 128, 126, (40, 40), (3, 3), (1, 1), (1, 1), ((1, 1), (1, 1)), "32x64,KG=4", "add"),
+    (14, 96, 64, (41, 40), (3, 3), (2, 2), (1, 1), ((0, 1), (1, 1)), "32x64,KG=4", "lut"),        # both column phases
+    (4, 128, 128, (40, 41), (3, 3), (1, 1), (1, 1), ((1, 1), (1, 1)), "32x64,KG=2", "lut+add"),
+    (1, 32, 30, (40, 40), (3, 3), (1, 1), (1, 1), ((1, 1), (1, 1)), "16x32,KG=4", "add"),         # five: one group has two
+    (2, 320, 17, (25, 24), (3, 3), (1, 1), (1, 1), ((1, 1), (1, 1)), "16x32,KG=4", "lut"),
+    (2, 128, 32, (80, 80), (3, 3), (1, 1), (1, 1), ((1, 1), (1, 1)), "32x32,KG=4", "add"),
+    (2, 128, 32, (112, 110), (3, 3), (1, 1), (1, 1), ((1, 1), (1, 1)), "32x32,KG=2", "lut+add")])
+def test_window_reductions_shared_by_groups_of_waves(hip_ctx, n, cin, cout, hw, k, stride, dil, pad, block, extra):
+    """Launches of few tiles split a block's k-steps between groups of waves: shares that differ, short last steps, surplus pixels, and
+    what may sit in the epilogue, which every group finishes a part of."""
+    test_convolution_over_an_input_tile_in_lds(hip_ctx, n, cin, cout, hw, k, stride, dil, pad, block, extra)
 
 
 @pytest.mark.parametrize("m,k,n", [(16500, 516, 300), (16641, 1020, 258), (33000, 532, 257)])

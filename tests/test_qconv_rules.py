@@ -24,6 +24,9 @@ extern "C" int wide(int oc, int ksteps, int tiles) { return nnhip::small_wide_pa
 extern "C" int window(int stride, int ksteps, int channels, int pix, int waves, long lds, long tiles, long chunks, long pixels) {
     return nnhip::tile_kernel_pays({stride, ksteps, channels, pix, waves, (size_t)lds, tiles, chunks, pixels}, 256);
 }
+extern "C" int split_window(long lds, long tiles, long chunks, int waves) {
+    return nnhip::split_window_pays({1, 18, 128, 16, waves, (size_t)lds, tiles, chunks, 16 * tiles}, 256);
+}
 extern "C" int dma_rows(long rows, int nchunks, int ksteps) { return 64 * nnhip::choose_dma_rows(rows, nchunks, ksteps, 256).rg; }
 extern "C" int pair_apart(long pixels, int k1, int n1, int n2, int dw) { return nnhip::split_pair(pixels, k1, n1, n2, dw, 256).apart; }
 extern "C" int pair_pays(long pixels, int k1, int n1, int n2) { return nnhip::pair_pays(pixels, k1, n1, n2, 256); }
@@ -138,9 +141,9 @@ def test_output_tile_is_the_best_of_all_numbers_of_tiles(rules, pix, stride, spa
 
 def test_division_of_a_tile(rules):
     for d in list(range(1, 1100)) + [4095, 10240, (1 << 20) - 1, 1 << 20, 1 << 24]:
-        assert [rules.tile_div(p, d) for p in range(512)] == [p // d for p in range(512)], d
+        assert [rules.tile_div(p, d) for p in range(1024)] == [p // d for p in range(1024)], d
     # (24-bit operands, 32-bit product: the largest of both)
-    assert 511 << 20 < 1 << 32 and 1 << 20 < 1 << 24
+    assert 1023 << 20 < 1 << 32 and 1 << 20 < 1 << 24
 
 
 # windows of a group's channels -> outputs, window side, stride; k-steps; pixels and waves per block, LDS, tiles, chunks, output pixels;
@@ -220,6 +223,28 @@ def test_windows_take_the_quicker_kernel(rules, row):
 def test_window_kernel_is_not_launched_beyond_the_lds(rules):
     args = lambda lds: (1, 40, 256, 128, 8, C.c_long(lds), C.c_long(4000), C.c_long(1), C.c_long(500000))
     assert rules.window(*args(160 * 1024)) and not rules.window(*args(160 * 1024 + 16))
+
+
+# windows whose k-steps groups of waves share: LDS of a block, tiles, chunks, waves of all groups; us without the split, with it
+SPLITS = [
+    (16000, 100, 2, 8, 5.28, 4.00),     # 128 -> 128 3x3 of 1600 pixels
+    (25000, 28, 4, 8, 6.82, 4.72),      # 256 -> 256 of 400
+    (45000, 25, 8, 8, 10.95, 7.91),     # 512 -> 512 of 400
+    (22000, 200, 2, 4, 5.79, 5.15),     # 128 -> 128 of 6400, two groups
+    (34000, 200, 2, 8, 5.79, 5.50),     # ... four
+    (36000, 288, 3, 4, 8.19, 8.86),     # 128 -> 160 of 12 288
+    (14000, 1600, 1, 2, 5.60, 6.09),    # 80 -> 32 of 51 200
+    (90000, 56, 5, 2, 12.11, 13.99),    # 512 -> 160 stride 2 of 1352: one block of two waves to a compute unit
+    (97000, 392, 1, 4, 12.44, 16.40),   # 512 -> 32 stride 2 of 12 544
+    (56000, 784, 1, 4, 12.44, 13.87),
+]
+
+
+@pytest.mark.parametrize("row", SPLITS, ids=lambda r: "-".join(map(str, r[:4])))
+def test_which_windows_share_their_k_steps(rules, row):
+    lds, tiles, chunks, waves, without, split = row
+    assert (split if rules.split_window(C.c_long(lds), C.c_long(tiles), C.c_long(chunks), waves) else without) <= 1.1 * min(without, split)
+    assert not rules.split_window(C.c_long(160 * 1024 + 1), C.c_long(1), C.c_long(1), waves)
 
 
 # a group's channels -> outputs, window side, k-steps, the small tiles' 16-channel tiles per chunk, output pixels; us by the small tiles,
