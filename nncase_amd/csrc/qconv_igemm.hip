@@ -270,7 +270,7 @@ int launch_qconv_igemm(nncase_hip_ctx *ctx, const uint8_t *x, const nncase_hip_w
     const int mode = igemm_load_mode(w, c, out_h, out_w);
     a.apart = igemm_rows_apart(w, c, out_h, out_w);
 
-    const TilePlan tile = w->ragged ? TilePlan{} : plan_qconv_tile(ctx, a, w->tiles, w->nchunks);
+    const TilePlan tile = plan_qconv_tile(ctx, a, w->ragged, w->tiles, w->nchunks);
     const size_t group_bytes = (size_t)w->nchunks * w->ksteps * w->tiles * 1024;
     for (int g = 0; g < w->groups; g++) {
         a.wpk = reinterpret_cast<const uint8_t *>(w->d_packed) + g * group_bytes;

@@ -172,7 +172,7 @@ constexpr int kTileDivMost = 1024;
 inline uint32_t make_tile_div(int d) { return ((1u << 20) + (uint32_t)d - 1) / (uint32_t)d; }
 
 // Whether a launch of the window kernel as planned is quicker than the implicit GEMM of the same layer (byte results, strides of 1
-// and 2, three k-steps and more, stride 2 sixteen).  us, implicit GEMM / window kernel:
+// and 2, whole_window_ksteps and more).  us, implicit GEMM / window kernel:
 //   * tiles that images do not fill by half stay, their surplus pixels are multiplied and dropped; with fewer than three waves per
 //     compute unit a sixth is too much (3388 pixels 256 -> 170 in two groups, 63 % full, 12.1 / 14.4)
 //   * with fewer than three waves per two compute units (stride 2: four per unit) the k-steps split over groups of waves win
@@ -205,6 +205,18 @@ inline bool tile_kernel_pays(const TileLaunch &l, int compute_units) {
     if (l.stride_w == 2 && resident < 5) return false;
     if (l.pix < 128 && l.channels > 400 && resident < 4) return false;
     return l.pix > 32 || (l.ksteps >= 5 && launched <= 9ll * l.ksteps * compute_units);
+}
+
+// The k-steps from which the window kernel's undivided blocks are worth their staging; fewer are the epilogue's work alone.  `tiles`: of 16
+// channels, packed together; eight take blocks of eight waves.  us, implicit GEMM or ring / window kernel:
+//   * stride 1: three (16 -> 32 3x3 of 1 638 400 pixels 41.4 / 36.7; two, 802 816 pixels 16 -> 32 2x2, 14.9 / 18.6)
+//   * stride 2 brings in four times the input: five (32 -> 64 3x3 of 25 600 5.6 / 4.7, 32 -> 131 of 7605 6.1 / 5.1; three, 16 -> 142 of 8192
+//     4.7 / 5.4), eight tiles seven (33 -> 67 of 14 112 7.0 / 5.7, 64 -> 128 of 25 600 8.3 / 7.1; five, 32 -> 214 of 22 472 8.5 / 9.7)
+//   * channels that are no multiple of 16, eight tiles and stride 1: nine (35 -> 106 3x3 of 64 800, seven, 14.2 / 16.1; 111 -> 319 of 25 392
+//     35.6 / 20.6)
+inline int whole_window_ksteps(int stride_w, int tiles, bool ragged) {
+    if (stride_w == 2) return tiles == 8 ? 7 : 5;
+    return ragged && tiles == 8 ? 9 : 3;
 }
 
 // Whether groups of waves that share a block's k-steps (TileLaunch::waves counts all of them) are quicker in the window kernel than

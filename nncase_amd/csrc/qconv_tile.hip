@@ -20,407 +20,9 @@
 //     their way when the first product starts, where the ring of qconv_wide_kernel goes through a barrier for each.  In a chain, us there /
 //     here: 128 -> 128 3x3 of 1600 pixels 5.3 / 4.0, 256 -> 256 of 400 6.8 / 4.7, 512 -> 512 of 400 11.0 / 7.9.
 // Arithmetic, weight packing and the bytes of the result are those of qconv_igemm.hpp.
-#include "qconv_rules.hpp"
 #include "qconv_tile.hpp"
 
 namespace nnhip {
-
-// What a launch's last stage takes of the arguments, in one trip: fetched ahead, the values would be spilled while the reduction runs,
-// and a request of the first stage would wait behind them.
-template <bool FAST> __device__ __forceinline__ IgemmArgs gather_store_args() {
-    auto p = (const __attribute__((address_space(4))) IgemmArgs *)__builtin_amdgcn_kernarg_segment_ptr();
-    asm volatile("" : "+s"(p));
-    const IgemmArgs &a = *(const IgemmArgs *)p;
-    IgemmArgs l; // (what is not assigned here is not used)
-    l.ep.c1 = a.ep.c1, l.ep.c2 = a.ep.c2;
-    if constexpr (!FAST) {
-        l.ep.mult = a.ep.mult, l.ep.sy = a.ep.sy, l.ep.rsy = a.ep.rsy, l.ep.zy = a.ep.zy, l.ep.qlo = a.ep.qlo, l.ep.qhi = a.ep.qhi;
-        l.ep.fast = a.ep.fast, l.ep.full = a.ep.full;
-        asm volatile("" ::"s"(l.ep.mult), "s"(l.ep.sy), "s"(l.ep.rsy), "s"(l.ep.zy), "s"(l.ep.qlo), "s"(l.ep.qhi), "s"(l.ep.fast), "s"(l.ep.full));
-    }
-    l.rep.res = a.rep.res, l.rep.zy = a.rep.zy, l.rep.sy = a.rep.sy, l.rep.zr = a.rep.zr, l.rep.sr = a.rep.sr;
-    l.rep.sum.sy = a.rep.sum.sy, l.rep.sum.rsy = a.rep.sum.rsy, l.rep.sum.zy = a.rep.sum.zy, l.rep.sum.qlo = a.rep.sum.qlo, l.rep.sum.qhi = a.rep.sum.qhi;
-    l.y = a.y, l.m = a.m, l.n = a.n, l.ldy = a.ldy, l.y_coff = a.y_coff, l.ldr = a.ldr, l.r_coff = a.r_coff, l.zwp = a.zwp, l.lut = a.lut;
-    l.d_ohow.div = a.d_ohow.div, l.d_ow.div = a.d_ow.div;
-    asm volatile("" ::"s"(l.ep.c1), "s"(l.ep.c2), "s"(l.rep.res), "s"(l.rep.zy), "s"(l.rep.sy), "s"(l.rep.zr), "s"(l.rep.sr), "s"(l.rep.sum.sy), "s"(l.rep.sum.rsy),
-                 "s"(l.rep.sum.zy), "s"(l.rep.sum.qlo), "s"(l.rep.sum.qhi), "s"(l.y), "s"(l.m), "s"(l.n), "s"(l.ldy), "s"(l.y_coff), "s"(l.ldr), "s"(l.r_coff),
-                 "s"(l.zwp), "s"(l.lut), "s"(l.d_ohow.div), "s"(l.d_ow.div));
-    return l;
-}
-
-// FAST: the requantisation is the one-instruction form without a clamp of its own (Epilogue::fast and ::full).
-// KG > 1: KG groups of WM x WN waves share the reduction, every KG-th k-step each, and add their sums up at the end.
-template <int T, int RG, int WM, int WN, int KG, bool FAST>
-__global__ __launch_bounds__(WM * WN * KG * 64, 4) void qconv_tile_kernel(const IgemmArgs a, const TileArgs t) {
-    constexpr int THREADS = WM * WN * KG * 64, PIX = WM * RG * 16, TB = T * WN;
-    constexpr int D = 4;                                             // k-steps of weights in flight
-    constexpr int UNITS = RG * T, EACH = (UNITS + KG - 1) / KG;      // results of a wave, 16 pixels x 16 channels; those that a group finishes
-    static_assert(TB * 16 <= THREADS && THREADS <= kTileDivMost, "a thread per channel, tile_div");
-    extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
-    int32_t *cterm = reinterpret_cast<int32_t *>(smem);              // [TB * 16]
-    int32_t *sums = cterm + TB * 16;                                 // [KG][PIX] sum of x' over a group's share of a pixel's window
-    uint8_t *lutl = reinterpret_cast<uint8_t *>(sums + KG * PIX);    // [256]
-    v4i *parts = reinterpret_cast<v4i *>(lutl + 256);                // [UNITS][KG - 1][waves of a group][64] sums on their way to the group that finishes them
-    int32_t *taps = reinterpret_cast<int32_t *>(lutl + 256 + tile_part_bytes(UNITS, WM * WN, KG)); // [KS + 2 KG][4] LDS offset of a piece of the reduction
-    uint8_t *tile = smem + t.tile_off;
-
-    // (what the requests need, in one trip; see gather_store_args for the rest)
-    asm volatile("" ::"s"(a.x), "s"(a.x_bytes), "s"(a.wpk), "s"(a.bias), "s"(a.wsum), "s"(a.lut), "s"(a.ksteps), "s"(a.ldx), "s"(a.x_coff), "s"(a.in_h), "s"(a.in_w),
-                 "s"(a.stride_h), "s"(a.stride_w), "s"(a.pad_h), "s"(a.pad_w), "s"(a.num_mtiles), "s"(a.n));
-    asm volatile("" ::"s"(t.th), "s"(t.tw), "s"(t.hr), "s"(t.hc), "s"(t.half), "s"(t.pitch), "s"(t.row_pitch), "s"(t.pieces), "s"(t.apart), "s"(t.dc), "s"(t.dr),
-                 "s"(t.row_bytes), "s"(t.d_pieces), "s"(t.d_hc), "s"(t.d_txy.mul), "s"(t.d_txy.shift), "s"(t.d_txy.div), "s"(t.d_tx.mul), "s"(t.d_tx.shift),
-                 "s"(t.d_tx.div), "s"(t.d_nchunks.mul), "s"(t.d_nchunks.shift), "s"(t.d_nchunks.div));
-
-    // as in qconv_wide_kernel: channel chunks of a tile back to back, a contiguous eighth of the tiles per XCD
-    const int xcd = blockIdx.x & 7, seq = blockIdx.x >> 3;
-    const int turn = (int)fastdiv((uint32_t)seq, t.d_nchunks), chunk = seq - turn * (int)t.d_nchunks.div;
-    const int per = (a.num_mtiles + 7) >> 3;
-    const int mt = xcd * per + turn;
-    if (turn >= per || mt >= a.num_mtiles) return;
-
-    const int tid = threadIdx.x, lane = tid & 63;
-    const int bwave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int kg = KG == 1 ? 0 : bwave / (WM * WN), wave = bwave - kg * (WM * WN);
-    const int wm = wave % WM, wn = wave / WM;
-    const int j = lane & 15, gq = lane >> 4;
-    const int KS = a.ksteps;
-    const int ch_base = chunk * (TB * 16);
-    const bool two = a.stride_w == 2;
-
-    // ---- a channel's terms and the byte table: asked for first, needed last ----
-    int32_t bias = 0, wsum = 0;
-    uint32_t table = 0;
-    if (ch_base + tid < a.n && tid < TB * 16) bias = a.bias[ch_base + tid], wsum = a.wsum[ch_base + tid];
-    if (a.lut && tid < 64) table = a.lut[tid];
-
-    // ---- the input tile: requested in batches of U pieces per thread, the next before one is stored.  A thread keeps its piece of
-    // a pixel and goes through the pixels t.apart at a time ----
-    const uint32_t img = fastdiv((uint32_t)mt, t.d_txy);
-    const uint32_t in_img = (uint32_t)mt - img * t.d_txy.div;
-    const uint32_t tyi = fastdiv(in_img, t.d_tx);
-    const int oy0 = (int)tyi * t.th, ox0 = (int)(in_img - tyi * t.d_tx.div) * t.tw;
-    const int iy0 = oy0 * a.stride_h - a.pad_h, ix0 = ox0 * a.stride_w - a.pad_w;
-    const int base = ((int)img * a.in_h + iy0) * t.row_bytes + ix0 * a.ldx + a.x_coff; // (may be negative at a border)
-    const __amdgpu_buffer_rsrc_t xres = wide_rsrc(a.x, (uint32_t)a.x_bytes);
-    constexpr int U = 4;
-    struct Batch {
-        wide_u32x4 v[U];
-        int dst[U];        // where the piece goes in LDS; its bit 0: the pixel lies in the padding
-    };
-    const int n = t.hr * t.hc; // pixels
-    const bool inside = iy0 >= 0 && ix0 >= 0 && iy0 + t.hr <= a.in_h && ix0 + t.hc <= a.in_w; // no padding under this tile
-    int r, c;  // row and column of this thread's next pixel
-    int owned; // its pixels are those of t.apart, 2 t.apart, ... below this
-    int q16;   // its piece
-    {
-        const int p0 = tile_div(tid, t.d_pieces);
-        q16 = (tid - __mul24(p0, t.pieces)) * 16;
-        r = tile_div(p0, t.d_hc);
-        c = p0 - __mul24(r, t.hc);
-        owned = p0 < t.apart ? n - p0 : 0; // (threads past the last whole pixel: none)
-    }
-    // (a thread past the tile's last pixel reads what follows it in the tensor, or 0 past its end, and drops it)
-    auto request_piece = [&](Batch &f, int u, bool in_c) __attribute__((always_inline)) {
-        const int goff = __mul24(r, t.row_bytes) + (__mul24(c, a.ldx) + q16);
-        f.dst[u] = __mul24(r, t.row_pitch) + (__mul24(two ? (c & 1) * t.half + (c >> 1) : c, t.pitch) + q16);
-        if (in_c) {
-            f.v[u] = __builtin_amdgcn_raw_buffer_load_b128(xres, goff, base, 0);
-        } else {
-            const bool in = (unsigned)(iy0 + r) < (unsigned)a.in_h && (unsigned)(ix0 + c) < (unsigned)a.in_w;
-            f.v[u] = __builtin_amdgcn_raw_buffer_load_b128(xres, in ? (uint32_t)(base + goff) : 0xffffffffu, 0, 0);
-            f.dst[u] |= in ? 0 : 1;
-        }
-        c += t.dc;
-        const bool carry = c >= t.hc;
-        c -= carry ? t.hc : 0;
-        r += t.dr + (carry ? 1 : 0);
-    };
-    auto request = [&](Batch &f, int i0) __attribute__((always_inline)) {
-        if (inside) {
-#pragma unroll
-            for (int u = 0; u < U; u++) {
-                if (i0 + u * t.apart >= n) break;
-                request_piece(f, u, true);
-            }
-        } else {
-#pragma unroll
-            for (int u = 0; u < U; u++) {
-                if (i0 + u * t.apart >= n) break;
-                request_piece(f, u, false);
-            }
-        }
-    };
-    auto keep = [&](const Batch &f, int i0) __attribute__((always_inline)) {
-#pragma unroll
-        for (int u = 0; u < U; u++) {
-            const int i = i0 + u * t.apart;
-            if (i >= n) break;
-            if (i < owned) {
-                const uint32_t fill = (f.dst[u] & 1) ? a.zx_splat : 0u;
-                wide_u32x4 w;
-#pragma unroll
-                for (int d = 0; d < 4; d++) w[d] = (inside ? f.v[u][d] : f.v[u][d] | fill) ^ 0x80808080u;
-                *reinterpret_cast<wide_u32x4 *>(tile + (f.dst[u] & ~1)) = w;
-            }
-        }
-    };
-    Batch fa;
-    request(fa, 0);
-
-    // ---- weights: D k-steps ahead.  The last k-step, which may end past the reduction, comes first, the others follow from
-    // where this block starts; group kg takes the kg-th of that order and every KG-th from there ----
-    const __amdgpu_buffer_rsrc_t wres = wide_rsrc(a.wpk + (size_t)chunk * KS * TB * 1024, (uint32_t)KS * TB * 1024);
-    const int rest = KS - 1;
-    const int ks0 = rest == 0 ? 0 : seq - (int)fastdiv((uint32_t)seq, t.d_rest) * rest;
-    const int w_end = rest * TB * 1024, w_lane = wn * T * 1024 + lane * 16;
-    int w_off = w_end; // of the next k-step to request
-    auto load_w = [&](v4i (&dst)[T]) __attribute__((always_inline)) {
-#pragma unroll
-        for (int nt = 0; nt < T; nt++) dst[nt] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(wres, w_lane + nt * 1024, w_off, 0));
-    };
-    auto advance = [&](int ksteps) __attribute__((always_inline)) { // (of at most `rest`: choose_tile)
-        w_off += ksteps * (TB * 1024);
-        w_off -= w_off >= w_end ? w_end : 0;
-    };
-    auto load_next = [&](v4i (&dst)[T]) __attribute__((always_inline)) {
-        load_w(dst);
-        advance(KG);
-    };
-    v4i wf[D][T];
-    if (KG == 1 || kg == 0) {
-        load_w(wf[0]);
-        w_off = ks0 * TB * 1024;
-        if (KG > 1) advance(KG - 1);
-    } else {
-        w_off = ks0 * TB * 1024;
-        advance(kg - 1);
-        load_next(wf[0]);
-    }
-#pragma unroll
-    for (int d = 1; d < D; d++) load_next(wf[d]);
-
-    // ---- tables ----
-    for (int e = tid; e < (KS + 2 * KG) * 4; e += THREADS) { // in the order of this block's k-steps
-        const int s = e >> 2;
-        int ks = s == 0 ? rest : ks0 + s - 1;
-        ks -= s > 0 && ks >= rest ? rest : 0;
-        const int kk = ks * 64 + (e & 3) * 16;
-        int off = 0; // (past the reduction: any place, its weights are 0)
-        if (kk < a.k && s < KS) {
-            const uint32_t tap = fastdiv((uint32_t)kk, a.d_gic);
-            const uint32_t ky = fastdiv(tap, a.d_kw);
-            const int dx = ((int)tap - (int)ky * a.kw) * a.dil_w;
-            off = (int)ky * a.dil_h * t.row_pitch + (two ? (dx & 1) * t.half + (dx >> 1) : dx) * t.pitch + kk - (int)tap * a.g_ic;
-        }
-        taps[e] = off;
-    }
-    // this lane's pixels: pixel (wm RG + rg) * 16 + j of the tile, in rows of tw
-    auto lds_of = [&](int group) __attribute__((always_inline)) {
-        const int p = (wm * RG + group) * 16 + j;
-        int ty = tile_div(p, t.d_tw);
-        int tx = p - __mul24(ty, t.tw);
-        if (ty >= t.th) ty = tx = 0; // (surplus of the block: not stored)
-        return __mul24(ty, a.stride_h * t.row_pitch) + __mul24(tx, t.pitch);
-    };
-    // the sum of x' of a pixel group comes from a product with ones; waves that share the pixels share that work
-    constexpr int SG = (RG + WN - 1) / WN; // groups per wave
-    int xbase[RG], xsum[SG];
-#pragma unroll
-    for (int rg = 0; rg < RG; rg++) xbase[rg] = lds_of(rg);
-#pragma unroll
-    for (int i = 0; i < SG; i++) xsum[i] = WN == 1 ? xbase[i] : lds_of(min(wn * SG + i, RG - 1));
-    if (tid < TB * 16) cterm[tid] = bias - a.zxp * wsum + a.k * a.zxp * a.zwp;
-    if (tid < 64) reinterpret_cast<uint32_t *>(lutl)[tid] = table;
-    {
-        int i0 = 0;
-        for (; i0 + U * t.apart < n; i0 += U * t.apart) {
-            Batch fb;
-            request(fb, i0 + U * t.apart);
-            keep(fa, i0);
-            fa = fb;
-        }
-        keep(fa, i0);
-    }
-    const IgemmArgs late = gather_store_args<FAST>();
-    __syncthreads();
-
-    // ---- the reduction ----
-    const int ch0 = gq * (4 * TB) + wn * (4 * T);
-    v4i acc[RG][T], rs[SG];
-    v4i xf[2][RG], xs[2][SG]; // (a wave reads the operand it sums by itself: which of xf that is depends on the wave)
-    const int32_t *tap = taps + kg * 4 + gq; // of the k-step whose operands are read next
-    int toff = tap[0];
-    auto operands = [&](v4i (&dst)[RG], v4i (&dsts)[SG], int ahead) __attribute__((always_inline)) {
-#pragma unroll
-        for (int rg = 0; rg < RG; rg++) dst[rg] = *reinterpret_cast<const v4i *>(tile + xbase[rg] + toff);
-#pragma unroll
-        for (int i = 0; i < SG; i++) dsts[i] = WN == 1 ? dst[i] : *reinterpret_cast<const v4i *>(tile + xsum[i] + toff);
-        toff = tap[ahead * (4 * KG)];
-    };
-    operands(xf[0], xs[0], 1);
-    operands(xf[1], xs[1], 2);
-    tap += 2 * (4 * KG);
-    const v4i ones = {0x01010101, 0x01010101, 0x01010101, 0x01010101};
-    {
-        const int one = kg > 0 || rest * 64 + gq * 16 < a.k ? 0x01010101 : 0; // (pieces past the reduction)
-        const v4i ones_last = {one, one, one, one}, zero = {0, 0, 0, 0};
-#pragma unroll
-        for (int nt = 0; nt < T; nt++) {
-            v4i ct = *reinterpret_cast<const v4i *>(cterm + ch0 + nt * 4);
-            if (KG > 1 && kg > 0) ct = zero;
-#pragma unroll
-            for (int rg = 0; rg < RG; rg++) acc[rg][nt] = __builtin_amdgcn_mfma_i32_16x16x64_i8(wf[0][nt], xf[0][rg], ct, 0, 0, 0);
-        }
-#pragma unroll
-        for (int i = 0; i < SG; i++) rs[i] = __builtin_amdgcn_mfma_i32_16x16x64_i8(ones_last, xs[0][i], zero, 0, 0, 0);
-    }
-    load_next(wf[0]);
-    // (whole groups of D k-steps without a branch between them: behind one, a wait for one k-step's weights waits for all)
-    auto kstep = [&](auto u_c) __attribute__((always_inline)) {
-        constexpr int u = decltype(u_c)::value, b = u % D;
-        operands(xf[(u + 1) & 1], xs[(u + 1) & 1], u);
-        __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int nt = 0; nt < T; nt++)
-#pragma unroll
-            for (int rg = 0; rg < RG; rg++) acc[rg][nt] = __builtin_amdgcn_mfma_i32_16x16x64_i8(wf[b][nt], xf[u & 1][rg], acc[rg][nt], 0, 0, 0);
-#pragma unroll
-        for (int i = 0; i < SG; i++) rs[i] = __builtin_amdgcn_mfma_i32_16x16x64_i8(ones, xs[u & 1][i], rs[i], 0, 0, 0);
-        __builtin_amdgcn_sched_barrier(0);
-        load_next(wf[b]);
-    };
-    int left = KG == 1 ? rest : (rest - kg) / KG;
-#pragma clang loop unroll(disable)
-    for (; left >= D; left -= D) {
-        static_for<1, D + 1>(kstep);
-        tap += D * (4 * KG);
-    }
-    static_for<1, D>([&](auto u_c) __attribute__((always_inline)) {
-        if (decltype(u_c)::value <= left) kstep(u_c);
-    });
-
-    // ---- epilogue ----
-    // whole pixel rows: TB threads per pixel, 16 channels each.  Their bytes of the residual are asked for before the sums meet.
-    constexpr int PPT = THREADS / TB < PIX ? THREADS / TB : PIX, PASSES = PIX / PPT; // pixels of a pass
-    static_assert(PIX % PPT == 0, "whole passes");
-    const int oh_img = (int)late.d_ohow.div, ow = (int)late.d_ow.div;
-    const int cb = (tid % TB) * 16, ch = ch_base + cb;
-    const bool whole = ch + 16 <= late.n, wide_y = ((late.ldy | late.y_coff) & 3) == 0;
-    int px[PASSES]; // pixel index of the tensor, late.m where there is none
-    u32x4 rv[PASSES];
-#pragma unroll
-    for (int it = 0; it < PASSES; it++) {
-        const int p = it * PPT + tid / TB;
-        const int ty = tile_div(p, t.d_tw);
-        const int oy = oy0 + ty, ox = ox0 + p - __mul24(ty, t.tw);
-        const int at = __mul24(oy, ow) + ox;
-        px[it] = p < PIX && ty < t.th && ox < ow && at < oh_img && ch < late.n ? (int)img * oh_img + at : late.m;
-    }
-    if (late.rep.res) {
-        const bool wide_r = ((late.ldr | late.r_coff) & 3) == 0;
-#pragma unroll
-        for (int it = 0; it < PASSES; it++) {
-            rv[it] = u32x4{0, 0, 0, 0};
-            if (px[it] >= late.m) continue;
-            const uint8_t *ro = late.rep.res + (size_t)px[it] * late.ldr + late.r_coff + ch;
-            if (whole && wide_r) {
-                const u32x4_a4 r4 = *reinterpret_cast<const u32x4_a4 *>(ro);
-                rv[it] = u32x4{r4[0], r4[1], r4[2], r4[3]};
-            } else {
-#pragma unroll
-                for (int b = 0; b < 16; b++)
-                    if (ch + b < late.n) rv[it][b / 4] |= (uint32_t)ro[b] << (8 * (b & 3));
-            }
-        }
-    }
-    if (gq == 0) {
-#pragma unroll
-        for (int i = 0; i < SG; i++)
-            if (wn * SG + i < RG) sums[kg * PIX + (wm * RG + wn * SG + i) * 16 + j] = rs[i][0];
-    }
-    // (unit u of a wave: pixel group u / T, channel tile u % T; group u / EACH finishes it)
-    auto part = [&](int u, int from) __attribute__((always_inline)) { return parts + ((u * (KG - 1) + from) * (WM * WN) + wave) * 64 + lane; };
-    if constexpr (KG > 1) {
-        static_for<0, UNITS>([&](auto u_c) __attribute__((always_inline)) {
-            constexpr int u = decltype(u_c)::value, by = u / EACH;
-            if (kg != by) *part(u, kg - (kg > by ? 1 : 0)) = acc[u / T][u % T];
-        });
-    }
-    __syncthreads(); // the sums are there, and every wave is through with the tile: its place takes the result
-    constexpr int kOutPitch = TB * 16 + 16;
-    auto finish = [&](auto first_c) __attribute__((always_inline)) { // the EACH units from there on
-        constexpr int first = decltype(first_c)::value, count = KG == 1 ? UNITS : (UNITS - first < EACH ? UNITS - first : EACH);
-        int32_t owed[RG];
-#pragma unroll
-        for (int rg = first / T; rg <= (first + count - 1) / T; rg++) {
-            int32_t sum = sums[(wm * RG + rg) * 16 + j];
-#pragma unroll
-            for (int g = 1; g < KG; g++) sum += sums[g * PIX + (wm * RG + rg) * 16 + j];
-            owed[rg] = -late.zwp * sum;
-        }
-        uint32_t packed[count];
-        if constexpr (KG > 1) {
-            v4i others[count][KG - 1];
-#pragma unroll
-            for (int u = 0; u < count; u++)
-#pragma unroll
-                for (int from = 0; from < KG - 1; from++) others[u][from] = *part(first + u, from);
-#pragma unroll
-            for (int u = 0; u < count; u++)
-#pragma unroll
-                for (int from = 0; from < KG - 1; from++) acc[(first + u) / T][(first + u) % T] += others[u][from];
-        }
-#pragma unroll
-        for (int u = 0; u < count; u++) {
-            const int rg = (first + u) / T, nt = (first + u) % T;
-            int32_t v[4];
-#pragma unroll
-            for (int r = 0; r < 4; r++) v[r] = acc[rg][nt][r] + owed[rg];
-            packed[u] = FAST ? requant4_u8_packed_direct(v, late.ep) : requant4_u8_packed(v, late.ep);
-        }
-        if (late.lut) { // (every byte is asked for before the first is used)
-            uint32_t b[count][4];
-#pragma unroll
-            for (int u = 0; u < count; u++)
-#pragma unroll
-                for (int r = 0; r < 4; r++) b[u][r] = lutl[(packed[u] >> (8 * r)) & 0xffu];
-            __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-            for (int u = 0; u < count; u++) packed[u] = b[u][0] | (b[u][1] << 8) | (b[u][2] << 16) | (b[u][3] << 24);
-        }
-#pragma unroll
-        for (int u = 0; u < count; u++)
-            *reinterpret_cast<uint32_t *>(tile + ((wm * RG + (first + u) / T) * 16 + j) * kOutPitch + ch0 + (first + u) % T * 4) = packed[u];
-    };
-    if constexpr (KG == 1) {
-        finish(std::integral_constant<int, 0>());
-    } else {
-        static_for<0, (UNITS + EACH - 1) / EACH>([&](auto g_c) __attribute__((always_inline)) {
-            if (kg == decltype(g_c)::value) finish(std::integral_constant<int, decltype(g_c)::value * EACH>());
-        });
-    }
-    __syncthreads();
-#pragma unroll
-    for (int it = 0; it < PASSES; it++) {
-        if (px[it] >= late.m) continue;
-        u32x4 v = *reinterpret_cast<const u32x4 *>(tile + (it * PPT + tid / TB) * kOutPitch + cb);
-        if (late.rep.res) {
-#pragma unroll
-            for (int d = 0; d < 4; d++) v[d] = residual4_packed(v[d], rv[it][d], late.rep);
-        }
-        uint8_t *yo = reinterpret_cast<uint8_t *>(late.y) + (size_t)px[it] * late.ldy + late.y_coff + ch;
-        if (whole && wide_y) {
-            *reinterpret_cast<u32x4_a4 *>(yo) = u32x4_a4{v[0], v[1], v[2], v[3]};
-        } else if (whole) {
-#pragma unroll
-            for (int d = 0; d < 4; d++) reinterpret_cast<U32Unaligned *>(yo + d * 4)->v = v[d];
-        } else {
-#pragma unroll
-            for (int b = 0; b < 16; b++)
-                if (ch + b < late.n) yo[b] = (uint8_t)(v[b / 4] >> (8 * (b & 3)));
-        }
-    }
-}
 
 namespace {
 // The plan of a kernel with `pix` pixels and `tb` 16-channel tiles per block; `groups` of waves, whose sums take `parts` bytes, share its k-steps.
@@ -445,21 +47,6 @@ TilePlan plan_tile(const IgemmArgs &a, int pix, int tb, int threads, int nchunks
     return p;
 }
 
-template <int T, int RG, int WM, int WN, int KG, bool FAST> int launch_tile_f(nncase_hip_ctx *ctx, const IgemmArgs &args, const TilePlan &plan, int nchunks) {
-    if (plan.lds > 65536) NNHIP_HIP(ctx, (raise_dynamic_lds<qconv_tile_kernel<T, RG, WM, WN, KG, FAST>>(ctx->device, 160 * 1024)));
-    hipLaunchKernelGGL((qconv_tile_kernel<T, RG, WM, WN, KG, FAST>), dim3(ceil_div(args.num_mtiles, 8) * 8 * nchunks), dim3(WM * WN * KG * 64), plan.lds, ctx->stream, args,
-                       plan.t);
-    NNHIP_LAUNCH_CHECK(ctx, "qconv_tile_kernel");
-    return 0;
-}
-template <int T, int RG, int WM, int WN, int KG = 1> int launch_tile_t(nncase_hip_ctx *ctx, const IgemmArgs &a, const TilePlan &plan, int nchunks) {
-    IgemmArgs args = a;
-    args.num_mtiles = plan.tiles;
-    return a.ep.fast && a.ep.full ? launch_tile_f<T, RG, WM, WN, KG, true>(ctx, args, plan, nchunks) : launch_tile_f<T, RG, WM, WN, KG, false>(ctx, args, plan, nchunks);
-}
-} // namespace
-
-namespace {
 template <int T, int RG, int WM, int WN, int KG = 1> TilePlan plan_shape(const IgemmArgs &a, int nchunks) {
     return plan_tile(a, WM * RG * 16, T * WN, WM * WN * KG * 64, nchunks, KG, tile_part_bytes(RG * T, WM * WN, KG));
 }
@@ -493,11 +80,10 @@ TileShape choose_split_tile(const nncase_hip_ctx *ctx, const IgemmArgs &a, int t
 //   * one wave row of 32 pixels for 64 channels: 102 400 pixels 64 -> 64 12.7 / 11.5 (13.9 with 128 pixels, 12.3 with 64);
 //   * 32 channels: 409 600 pixels 32 -> 32 21.9 / 15.6, 1 638 400 pixels 16 -> 32 41.4 / 36.7; two k-steps and fewer are the
 //     epilogue's work alone and stay (802 816 pixels 16 -> 32 2x2 14.9 / 18.6);
-//   * stride 2 brings in four times the input: from 16 k-steps on (25 600 pixels 128 -> 256 18.5 / 15.9, 6400 pixels 256 -> 512
-//     18.0 / 15.5, but 409 600 pixels 32 -> 64, five k-steps, 28.2 / 30.3);
+//   * the k-steps it takes: whole_window_ksteps;
 //   * and what tile_kernel_pays asks of the launch.
-TileShape choose_whole_tile(const nncase_hip_ctx *ctx, const IgemmArgs &a, int tiles, int nchunks, TilePlan *plan) {
-    if (a.ksteps < (a.stride_w == 2 ? 16 : 3)) return kTileNone;
+TileShape choose_whole_tile(const nncase_hip_ctx *ctx, const IgemmArgs &a, bool ragged, int tiles, int nchunks, TilePlan *plan) {
+    if (a.ksteps < whole_window_ksteps(a.stride_w, tiles, ragged)) return kTileNone;
     TileShape shape = kTileNone;
     int waves = 2, pix = 64;
     // (the smaller tile too where the larger one is not half full of an image's pixels)
@@ -511,20 +97,22 @@ TileShape choose_whole_tile(const nncase_hip_ctx *ctx, const IgemmArgs &a, int t
     case 8:
         *plan = plan_shape<2, 4, 2, 4>(a, nchunks), shape = kTile128x128, waves = 8, pix = 128;
         if (!enough(3 * ctx->compute_units / 4)) *plan = plan_shape<2, 2, 2, 4>(a, nchunks), shape = kTile64x128, pix = 64;
+        // (a sixth of surplus pixels: 334 -> 360 3x3 of 47 images of 14 x 14 24.6 by the ring, 27.0 so)
+        if (ragged && 20ll * a.m < 17ll * plan->tiles * pix) return kTileNone;
         break;
     default: return kTileNone;
     }
     return plan->t.apart > 0 && tile_kernel_pays(TileLaunch{a.stride_w, a.ksteps, a.g_ic, pix, waves, plan->lds, plan->tiles, nchunks, a.m}, ctx->compute_units) ? shape : kTileNone;
 }
-TileShape choose_tile(const nncase_hip_ctx *ctx, const IgemmArgs &a, int tiles, int nchunks, TilePlan *plan) {
-    if (a.kh * a.kw == 1 || a.g_ic % 16 != 0 || a.kc_mask != -1 || a.stride_w > 2 || (int64_t)a.in_w * a.ldx >= (1 << 23)) return kTileNone;
+TileShape choose_tile(const nncase_hip_ctx *ctx, const IgemmArgs &a, bool ragged, int tiles, int nchunks, TilePlan *plan) {
+    if (a.kh * a.kw == 1 || a.g_ic % 16 != 0 || a.x_bytes < 16 || a.kc_mask != -1 || a.stride_w > 2 || (int64_t)a.in_w * a.ldx >= (1 << 23)) return kTileNone;
     // Fewer than ten k-steps are split where one group is no choice (three waves for two compute units and more: 64 -> 64 of 6400 pixels
     // 4.2 / 4.0, 48 -> 32 of 25 600 4.5 / 4.2, 32 -> 48 of 12 800 4.1 / 4.2).
     if (a.ksteps >= 10) {
         const TileShape split = choose_split_tile(ctx, a, tiles, nchunks, plan);
         if (split != kTileNone) return split;
     }
-    const TileShape whole = choose_whole_tile(ctx, a, tiles, nchunks, plan);
+    const TileShape whole = choose_whole_tile(ctx, a, ragged, tiles, nchunks, plan);
     return whole != kTileNone || a.ksteps >= 10 ? whole : choose_split_tile(ctx, a, tiles, nchunks, plan);
 }
 } // namespace
@@ -532,40 +120,27 @@ TileShape choose_tile(const nncase_hip_ctx *ctx, const IgemmArgs &a, int tiles, 
 const char *tile_kernel_block(const nncase_hip_ctx *ctx, const nncase_hip_weights *w, const nncase_hip_conv2d_args_t *c, int out_h, int out_w) {
     static const char *const names[] = {"128x32", "64x32", "32x64", "128x128", "64x128", "32x32,KG=2", "32x32,KG=4", "16x32,KG=4", "32x64,KG=2",
                                         "32x64,KG=4", "16x64,KG=4", nullptr};
-    if (w->ragged || c->out_dtype != NNCASE_HIP_DT_U8 || c->dequantize_output) return nullptr;
+    if (c->out_dtype != NNCASE_HIP_DT_U8 || c->dequantize_output) return nullptr;
     IgemmArgs a;
     memset(&a, 0, sizeof(a));
     a.m = (int)std::min<int64_t>((int64_t)c->batch * out_h * out_w, 1 << 30);
     a.d_ohow = make_fastdiv((uint32_t)(out_h * out_w)), a.d_ow = make_fastdiv((uint32_t)out_w);
     a.kh = w->kernel_h, a.kw = w->kernel_w, a.stride_h = c->stride_h, a.stride_w = c->stride_w, a.dil_h = c->dilation_h, a.dil_w = c->dilation_w;
-    a.g_ic = w->tap_ic, a.in_w = c->in_w, a.ldx = w->in_channels, a.ksteps = w->ksteps, a.kc_mask = w->fold ? 1 : -1;
+    a.g_ic = w->tap_ic, a.in_w = c->in_w, a.ldx = w->in_channels, a.x_bytes = (size_t)c->batch * c->in_h * c->in_w * w->in_channels, a.ksteps = w->ksteps, a.kc_mask = w->fold ? 1 : -1;
     TilePlan plan;
-    return names[choose_tile(ctx, a, w->tiles, w->nchunks, &plan)];
+    return names[choose_tile(ctx, a, w->ragged, w->tiles, w->nchunks, &plan)];
 }
 
-TilePlan plan_qconv_tile(const nncase_hip_ctx *ctx, const IgemmArgs &a, int tiles, int nchunks) {
+TilePlan plan_qconv_tile(const nncase_hip_ctx *ctx, const IgemmArgs &a, bool ragged, int tiles, int nchunks) {
     TilePlan plan;
-    const TileShape shape = a.ep.out_mode == kOutU8 && !a.deq ? choose_tile(ctx, a, tiles, nchunks, &plan) : kTileNone;
+    const TileShape shape = a.ep.out_mode == kOutU8 && !a.deq ? choose_tile(ctx, a, ragged, tiles, nchunks, &plan) : kTileNone;
     plan.shape = shape;
+    plan.t.ragged = ragged;
     return plan;
 }
 
 int launch_qconv_tile(nncase_hip_ctx *ctx, const IgemmArgs &a, const TilePlan &plan, int nchunks) {
-    switch (plan.shape) {
-    case kTile128x32: return launch_tile_t<2, 4, 2, 1>(ctx, a, plan, nchunks);
-    case kTile64x32: return launch_tile_t<2, 2, 2, 1>(ctx, a, plan, nchunks);
-    case kTile32x64: return launch_tile_t<2, 2, 1, 2>(ctx, a, plan, nchunks);
-    case kTile128x128: return launch_tile_t<2, 4, 2, 4>(ctx, a, plan, nchunks);
-    case kTile64x128: return launch_tile_t<2, 2, 2, 4>(ctx, a, plan, nchunks);
-    case kTile32x32by2: return launch_tile_t<2, 2, 1, 1, 2>(ctx, a, plan, nchunks);
-    case kTile32x32by4: return launch_tile_t<2, 2, 1, 1, 4>(ctx, a, plan, nchunks);
-    case kTile16x32by4: return launch_tile_t<2, 1, 1, 1, 4>(ctx, a, plan, nchunks);
-    case kTile32x64by2: return launch_tile_t<2, 2, 1, 2, 2>(ctx, a, plan, nchunks);
-    case kTile32x64by4: return launch_tile_t<2, 2, 1, 2, 4>(ctx, a, plan, nchunks);
-    case kTile16x64by4: return launch_tile_t<2, 1, 1, 2, 4>(ctx, a, plan, nchunks);
-    case kTileNone: break;
-    }
-    return fail(ctx, -EINVAL, "qconv2d: not a layer of the tile kernel");
+    return plan.t.ragged ? launch_tile_ragged(ctx, a, plan, nchunks) : launch_tile_shape<false>(ctx, a, plan, nchunks);
 }
 
 } // namespace nnhip

@@ -898,6 +898,28 @@ def test_window_reductions_shared_by_groups_of_waves(hip_ctx, n, cin, cout, hw, 
     test_convolution_over_an_input_tile_in_lds(hip_ctx, n, cin, cout, hw, k, stride, dil, pad, block, extra)
 
 
+@pytest.mark.parametrize("n,cin,cout,hw,k,stride,dil,pad,block,extra", [
+    (1, 5, 40, (9, 7), (5, 5), (1, 1), (1, 1), ((2, 2), (2, 2)), "16x64,KG=4", "lut+add"),         # the tensor ends inside its last pixel's piece
+    (1, 17, 24, (6, 5), (3, 3), (1, 1), (1, 1), ((0, 0), (0, 0)), "16x32,KG=4", ""),               # ... of an image without padding
+    (3, 90, 203, (77, 75), (3, 3), (2, 2), (1, 1), ((1, 1), (1, 1)), "64x128", "clamp"),
+    (3, 97, 60, (41, 40), (3, 3), (1, 1), (1, 1), ((1, 1), (1, 1)), "32x64,KG=4", "add"),
+    (9, 63, 42, (61, 62), (3, 3), (1, 1), (1, 1), ((1, 1), (1, 1)), "32x64", "slice"),
+    (2, 241, 20, (139, 131), (3, 3), (1, 1), (1, 1), ((2, 0), (0, 2)), "64x32", "lut"),
+    (13, 51, 18, (94, 93), (3, 3), (1, 1), (1, 1), ((1, 1), (1, 1)), "128x32", "add"),
+    (3, 111, 126, (92, 91), (3, 3), (1, 1), (1, 1), ((1, 1), (1, 1)), "128x128", "lut+add"),
+    (4, 70, 30, (50, 47), (1, 7), (2, 1), (1, 2), ((0, 0), (6, 6)), "16x32,KG=4", "")])
+def test_input_tiles_of_odd_channel_counts(hip_ctx, n, cin, cout, hw, k, stride, dil, pad, block, extra):
+    """Pieces of 16 channels that start at any byte and end in the next pixel, in the padding or past the tensor."""
+    test_convolution_over_an_input_tile_in_lds(hip_ctx, n, cin, cout, hw, k, stride, dil, pad, block, extra)
+
+
+@pytest.mark.parametrize("n,c,h,w,oc,k,s,groups", [(2, 66, 23, 21, 60, 3, 1, 2), (1, 105, 15, 17, 93, 3, 2, 3), (1, 11, 4, 3, 32, 3, 1, 1), (2, 130, 20, 19, 128, 5, 1, 2)])
+@pytest.mark.parametrize("zx,zw", [(0, 255), (255, 0), (128, 128)])
+def test_input_tiles_of_odd_groups_and_extreme_zero_points(hip_ctx, n, c, h, w, oc, k, s, groups, zx, zw):
+    """What a piece holds beyond its group's channels adds nothing, whatever the zero points."""
+    run_case(hip_ctx, n, c, h, w, oc, k, k, (s, s), ((k // 2, k // 2), (k // 2, k // 2)), (1, 1), groups, seed=c + oc, zx=zx, zw=zw, modes=("u8",))
+
+
 @pytest.mark.parametrize("m,k,n", [(16500, 516, 300), (16641, 1020, 258), (33000, 532, 257)])
 def test_matmul_of_rows_of_whole_dwords_in_256_channel_blocks(hip_ctx, m, k, n):
     """Rows that are no multiple of 16 bytes, moved straight to LDS in 256 x 256 blocks: last k-steps that end inside a piece, partial
