@@ -155,3 +155,16 @@ def test_block_argument_checks(hip_ctx):
     b.stride = 2                                   # a residual needs the input's shape
     with pytest.raises(rt.HipError):
         hip_ctx.qblock(xd, blk, yd, b)
+
+
+@pytest.mark.parametrize("n,cin,mid,cout,h,w,stride,pad,add", [
+    (1, 64, 384, 64, 14, 14, 1, ((1, 1), (1, 1)), True),      # sixteen waves, one 16-pixel unit each
+    (1, 24, 72, 32, 11, 9, 1, ((1, 1), (1, 1)), False),       # a second chunk of eight channels, tiles that end outside
+    (2, 160, 128, 96, 9, 16, 2, ((0, 1), (0, 1)), False),     # three k-steps of expansion, odd halo
+    (90, 32, 192, 32, 14, 14, 1, ((1, 1), (1, 1)), True),     # more tiles than compute units: eight waves
+    (1, 16, 64, 16, 3, 2, 1, ((1, 1), (1, 1)), False)])       # an image of fewer pixels than a unit
+def test_blocks_whose_inner_codes_only_saturate(hip_ctx, monkeypatch, n, cin, mid, cout, h, w, stride, pad, add):
+    """Without a clamp tighter than the u8 range the inner requantisations have a path of their own."""
+    whole = pick_quant
+    monkeypatch.setitem(globals(), "pick_quant", lambda real, relu6_like=False: whole(real, False))
+    run_block(hip_ctx, n, cin, mid, cout, h, w, stride, pad, add, seed=cin + mid)
