@@ -20,7 +20,8 @@ void nnhip::describe_conv_kernel(const nncase_hip_ctx *ctx, const nncase_hip_wei
                                  char *buf, size_t cap) {
     if (w->kind == nncase_hip_weights::kDepthwise) {
         if (depthwise_uses_3x3(w, a)) snprintf(buf, cap, "dw3x3<S=%d>", a->stride_h);
-        else snprintf(buf, cap, "dw_generic<VEC=%d>", w->out_channels % 4 == 0 ? 4 : 1);
+        else if (depthwise_uses_5x5(w, a)) snprintf(buf, cap, "dw_window<K=5,S=%d>", a->stride_h);
+        else snprintf(buf, cap, "dw_generic<VEC=%d>", w->out_channels >= 4 ? 4 : 1);
         return;
     }
     if (w->d_smallc && a->dilation_h == 1 && a->dilation_w == 1 && !a->residual_dev && !w->d_post_lut && !a->dequantize_output &&

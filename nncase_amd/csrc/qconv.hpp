@@ -174,6 +174,7 @@ int igemm_load_mode(const nncase_hip_weights *w, const nncase_hip_conv2d_args_t 
 void nncase_hip_qblock_describe(const nncase_hip_qblock_t *b, const nncase_hip_qblock_args_t *a, char *buf, size_t cap);
 namespace nnhip {
 bool depthwise_uses_3x3(const nncase_hip_weights *w, const nncase_hip_conv2d_args_t *c);
+bool depthwise_uses_5x5(const nncase_hip_weights *w, const nncase_hip_conv2d_args_t *c);
 
 // Correctly rounded a / b from b and rb = RN(1 / b): one multiply and two fused
 // multiply-adds (Markstein's correction step: the residual a - b*q0 is exact in an

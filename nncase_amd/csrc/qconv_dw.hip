@@ -13,7 +13,11 @@
 // strip of output rows keeping the last three input rows unpacked in
 // registers, so each input byte is loaded from memory once per strip (plus a
 // two-row halo) and unpacked once.
-// dw_generic_kernel: any kernel size / stride / dilation / channel count.
+// dw_window_kernel: 5x5 windows, 4 channels x 4 output columns a thread as well.
+// dw_generic_kernel: any kernel size / stride / dilation, 4 channels a thread.
+// Channel counts that are no multiple of four: a pixel's last four channels overlap the four before them, which computes and
+// stores up to three codes twice, the same ones, and every access is a dword at any byte (a channel a thread was 187 us for 63
+// channels of 32 x 112 x 112 3x3, 64 channels take 16.6).  Fewer than four channels go one by one.
 #include "qconv.hpp"
 
 #include <algorithm>
@@ -24,6 +28,18 @@ namespace nnhip {
 constexpr int kDwThreads = 256;
 constexpr int kDwCols = 4;  // output columns per thread
 constexpr int kDwMaxRows = 8; // most output rows one thread walks down (3x3 kernel)
+
+// Four channels' codes, weights and terms, at any byte, any int16 and any int32.
+struct __attribute__((packed, aligned(1))) DwCodes {
+    uint32_t v;
+};
+struct __attribute__((packed, aligned(2))) DwTaps {
+    uint32_t x, y;
+};
+typedef int32_t dw_i32x4 __attribute__((ext_vector_type(4), aligned(4)));
+typedef float dw_f32x4 __attribute__((ext_vector_type(4), aligned(4)));
+__device__ __forceinline__ uint32_t dw_load(const uint8_t *p) { return reinterpret_cast<const DwCodes *>(p)->v; }
+__device__ __forceinline__ void dw_put(uint8_t *p, uint32_t v) { reinterpret_cast<DwCodes *>(p)->v = v; }
 
 struct DwArgs {
     const uint8_t *x;
@@ -52,16 +68,16 @@ __device__ __forceinline__ uint32_t select_u32(bool c, uint32_t yes, uint32_t no
 // Stores 4 adjacent channels of one output pixel; `o` is the element offset of the first.
 __device__ __forceinline__ void dw_store4(const DwArgs &a, uint32_t o, const int32_t (&v)[4]) {
     if (a.ep.out_mode == kOutU8) {
-        *reinterpret_cast<uint32_t *>(reinterpret_cast<uint8_t *>(a.y) + o) = requant4_u8_packed(v, a.ep);
+        dw_put(reinterpret_cast<uint8_t *>(a.y) + o, requant4_u8_packed(v, a.ep));
     } else if (a.ep.out_mode == kOutI32) {
-        *reinterpret_cast<int4 *>(reinterpret_cast<int32_t *>(a.y) + o) = int4{v[0], v[1], v[2], v[3]};
+        *reinterpret_cast<dw_i32x4 *>(reinterpret_cast<int32_t *>(a.y) + o) = dw_i32x4{v[0], v[1], v[2], v[3]};
     } else {
-        float4 f;
+        dw_f32x4 f;
         f.x = clamp_ref((float)v[0] * a.ep.mult, a.ep.lo, a.ep.hi);
         f.y = clamp_ref((float)v[1] * a.ep.mult, a.ep.lo, a.ep.hi);
         f.z = clamp_ref((float)v[2] * a.ep.mult, a.ep.lo, a.ep.hi);
         f.w = clamp_ref((float)v[3] * a.ep.mult, a.ep.lo, a.ep.hi);
-        *reinterpret_cast<float4 *>(reinterpret_cast<float *>(a.y) + o) = f;
+        *reinterpret_cast<dw_f32x4 *>(reinterpret_cast<float *>(a.y) + o) = f;
     }
 }
 
@@ -87,23 +103,23 @@ __device__ __forceinline__ void dw_store_row(const DwArgs &a, uint32_t o, const 
         for (int c = 0; c < kDwCols; c++) {
             const bool sel = row_stored && col_stored[c];
             const uint32_t off = select_u32(sel, o + (uint32_t)(c * a.channels), safe_off);
-            *reinterpret_cast<uint32_t *>(reinterpret_cast<uint8_t *>(a.y) + off) = select_u32(sel, q[c], safe_val);
+            dw_put(reinterpret_cast<uint8_t *>(a.y) + off, select_u32(sel, q[c], safe_val));
         }
     } else if (a.ep.out_mode == kOutI32) {
 #pragma unroll
         for (int c = 0; c < kDwCols; c++)
             if (row_stored && col_stored[c])
-                *reinterpret_cast<int4 *>(reinterpret_cast<int32_t *>(a.y) + o + (uint32_t)(c * a.channels)) =
-                    int4{(int32_t)v[c][0], (int32_t)v[c][1], (int32_t)v[c][2], (int32_t)v[c][3]};
+                *reinterpret_cast<dw_i32x4 *>(reinterpret_cast<int32_t *>(a.y) + o + (uint32_t)(c * a.channels)) =
+                    dw_i32x4{(int32_t)v[c][0], (int32_t)v[c][1], (int32_t)v[c][2], (int32_t)v[c][3]};
     } else {
 #pragma unroll
         for (int c = 0; c < kDwCols; c++) {
-            float4 f;
+            dw_f32x4 f;
             f.x = clamp_ref((float)v[c][0] * a.ep.mult, a.ep.lo, a.ep.hi);
             f.y = clamp_ref((float)v[c][1] * a.ep.mult, a.ep.lo, a.ep.hi);
             f.z = clamp_ref((float)v[c][2] * a.ep.mult, a.ep.lo, a.ep.hi);
             f.w = clamp_ref((float)v[c][3] * a.ep.mult, a.ep.lo, a.ep.hi);
-            if (row_stored && col_stored[c]) *reinterpret_cast<float4 *>(reinterpret_cast<float *>(a.y) + o + (uint32_t)(c * a.channels)) = f;
+            if (row_stored && col_stored[c]) *reinterpret_cast<dw_f32x4 *>(reinterpret_cast<float *>(a.y) + o + (uint32_t)(c * a.channels)) = f;
         }
     }
 }
@@ -147,7 +163,7 @@ template <int S, bool FP, bool FF, bool MG = false> __global__ __launch_bounds__
     const int img = (int)q;
 
     const uint32_t zx_splat = a.zx_splat;
-    const int c0 = cq * 4;
+    const int c0 = min(cq * 4, a.channels - 4);
     const int ox0 = strip * kDwCols;
     const int oy0 = rchunk * a.rows;
     const int ix0 = ox0 * S - a.pad_w;
@@ -158,7 +174,7 @@ template <int S, bool FP, bool FF, bool MG = false> __global__ __launch_bounds__
     acc_t ct[4];
 #pragma unroll
     for (int tap = 0; tap < 9; tap++) {
-        const uint2 raw = *reinterpret_cast<const uint2 *>(a.w + (uint32_t)(tap * a.channels + c0));
+        const DwTaps raw = *reinterpret_cast<const DwTaps *>(a.w + (uint32_t)(tap * a.channels + c0));
         if constexpr (FP) {
             wf[tap][0] = (float)(int16_t)(raw.x & 0xffffu);
             wf[tap][1] = (float)((int32_t)raw.x >> 16);
@@ -170,8 +186,8 @@ template <int S, bool FP, bool FF, bool MG = false> __global__ __launch_bounds__
         }
     }
     {
-        const int4 b = *reinterpret_cast<const int4 *>(a.bias + c0);
-        const int4 s = *reinterpret_cast<const int4 *>(a.wsum + c0);
+        const dw_i32x4 b = *reinterpret_cast<const dw_i32x4 *>(a.bias + c0);
+        const dw_i32x4 s = *reinterpret_cast<const dw_i32x4 *>(a.wsum + c0);
         constexpr int32_t start = MG ? kMagicBias : 0;
         ct[0] = (acc_t)(b.x - a.zx * s.x + start);
         ct[1] = (acc_t)(b.y - a.zx * s.y + start);
@@ -202,7 +218,7 @@ template <int S, bool FP, bool FF, bool MG = false> __global__ __launch_bounds__
         row_ok = (unsigned)next_iy < (unsigned)a.in_h;
         const uint32_t row_off = in_base + (uint32_t)min(max(next_iy, 0), a.in_h - 1) * in_row;
 #pragma unroll
-        for (int col = 0; col < NCOL; col++) raw[col] = *reinterpret_cast<const uint32_t *>(a.x + (row_off + col_off[col]));
+        for (int col = 0; col < NCOL; col++) raw[col] = dw_load(a.x + (row_off + col_off[col]));
         next_iy++;
     };
     auto unpack_row = [&](int buf, const uint32_t (&raw)[NCOL], bool row_ok) {
@@ -301,12 +317,88 @@ template <int S, bool FP, bool FF, bool MG = false> __global__ __launch_bounds__
     }
 }
 
+// Windows of K x K taps, four channels by four columns a thread.  A row of the input under them is asked for whole, all K before the
+// first is used, and taken apart once for its four outputs of every channel; it is not kept for the next output row (80 registers of 5x5,
+// which halve the waves).  Bound by the multiply-adds, v_mad_i32_i16 at a quarter of a wave per clock (25 of 33 instructions an output):
+// 64 channels of 32 x 112 x 112 5x5 132 us with a thread per four channels and pixel, 43 so.  (With the rows kept as they were loaded 51,
+// with room for four waves on a SIMD 43, and stride 2, 152 channels of 16 x 80 x 80, 19.3 instead of 12.5: both spill.)
+template <int K, int S> __global__ __launch_bounds__(kDwThreads, 3) void dw_window_kernel(const DwArgs a) {
+    constexpr int NCOL = (kDwCols - 1) * S + K;
+    const uint32_t nblk = gridDim.x, per = nblk >> 3, rem = nblk & 7u; // (as in dw3x3_kernel: a contiguous run for every XCD)
+    const uint32_t xcd = blockIdx.x & 7u, slot = blockIdx.x >> 3;
+    const uint32_t gid = (xcd * per + min(xcd, rem) + slot) * kDwThreads + threadIdx.x;
+    if (gid >= (uint32_t)a.total) return;
+    uint32_t t = gid, q = fastdiv(t, a.d_cq);
+    const int c0 = min((int)(t - q * a.d_cq.div) * 4, a.channels - 4);
+    t = q, q = fastdiv(t, a.d_strips);
+    const int ox0 = (int)(t - q * a.d_strips.div) * kDwCols;
+    t = q, q = fastdiv(t, a.d_rows);
+    const int oy0 = (int)(t - q * a.d_rows.div) * a.rows, img = (int)q;
+
+    uint32_t w01[K * K], w23[K * K]; // (w - zw) of channels (0,1) and (2,3) as int16 pairs, per tap
+#pragma unroll
+    for (int tap = 0; tap < K * K; tap++) {
+        const DwTaps raw = *reinterpret_cast<const DwTaps *>(a.w + (uint32_t)(tap * a.channels + c0));
+        w01[tap] = raw.x, w23[tap] = raw.y;
+    }
+    const dw_i32x4 b = *reinterpret_cast<const dw_i32x4 *>(a.bias + c0), ws = *reinterpret_cast<const dw_i32x4 *>(a.wsum + c0);
+    int32_t ct[4];
+#pragma unroll
+    for (int c = 0; c < 4; c++) ct[c] = b[c] - a.zx * ws[c];
+    const uint32_t in_row = (uint32_t)(a.in_w * a.channels);
+    const uint32_t in_base = (uint32_t)img * (uint32_t)a.in_h * in_row + (uint32_t)c0;
+    const int ix0 = ox0 * S - a.pad_w;
+    bool col_ok[NCOL]; // (a tap outside the image reads the nearest pixel inside it and is replaced by the zero point)
+    uint32_t col_off[NCOL];
+#pragma unroll
+    for (int col = 0; col < NCOL; col++) {
+        col_ok[col] = (unsigned)(ix0 + col) < (unsigned)a.in_w;
+        col_off[col] = (uint32_t)(min(max(ix0 + col, 0), a.in_w - 1) * a.channels);
+    }
+    for (int oy = oy0; oy < min(oy0 + a.rows, a.out_h); oy++) {
+        uint32_t raw[K][NCOL];
+#pragma unroll
+        for (int ky = 0; ky < K; ky++) {
+            const uint32_t row = in_base + (uint32_t)min(max(oy * S - a.pad_h + ky, 0), a.in_h - 1) * in_row;
+#pragma unroll
+            for (int col = 0; col < NCOL; col++) raw[ky][col] = dw_load(a.x + (row + col_off[col]));
+        }
+        int32_t acc[kDwCols][4];
+#pragma unroll
+        for (int o = 0; o < kDwCols; o++)
+#pragma unroll
+            for (int c = 0; c < 4; c++) acc[o][c] = ct[c];
+#pragma unroll
+        for (int ky = 0; ky < K; ky++) {
+            const bool row_ok = (unsigned)(oy * S - a.pad_h + ky) < (unsigned)a.in_h;
+#pragma unroll
+            for (int col = 0; col < NCOL; col++) {
+                const uint32_t d = select_u32(row_ok && col_ok[col], raw[ky][col], a.zx_splat);
+                const uint32_t x01 = __builtin_amdgcn_perm(0u, d, 0x0c010c00u), x23 = __builtin_amdgcn_perm(0u, d, 0x0c030c02u);
+#pragma unroll
+                for (int o = 0; o < kDwCols; o++) {
+                    const int kx = col - o * S;
+                    if (kx < 0 || kx >= K) continue;
+                    acc[o][0] = mad16_lo(x01, w01[ky * K + kx], acc[o][0]);
+                    acc[o][1] = mad16_hi(x01, w01[ky * K + kx], acc[o][1]);
+                    acc[o][2] = mad16_lo(x23, w23[ky * K + kx], acc[o][2]);
+                    acc[o][3] = mad16_hi(x23, w23[ky * K + kx], acc[o][3]);
+                }
+            }
+        }
+        const uint32_t at = (((uint32_t)img * (uint32_t)a.out_h + (uint32_t)oy) * (uint32_t)a.out_w + (uint32_t)ox0) * (uint32_t)a.channels + (uint32_t)c0;
+#pragma unroll
+        for (int o = 0; o < kDwCols; o++)
+            if (ox0 + o < a.out_w) dw_store4(a, at + (uint32_t)(o * a.channels), acc[o]);
+    }
+}
+
 template <int VEC> __global__ __launch_bounds__(kDwThreads) void dw_generic_kernel(const DwArgs a) {
     const long long gid = (long long)blockIdx.x * kDwThreads + threadIdx.x;
     if (gid >= a.total) return;
     uint32_t t = (uint32_t)gid;
     uint32_t q = fastdiv(t, a.d_cq);
-    const int c0 = (int)(t - q * a.d_cq.div) * VEC;
+    const int c0 = min((int)(t - q * a.d_cq.div) * VEC, a.channels - VEC);
     t = q;
     q = fastdiv(t, a.d_ow);
     const int ox = (int)(t - q * a.d_ow.div);
@@ -327,7 +419,7 @@ template <int VEC> __global__ __launch_bounds__(kDwThreads) void dw_generic_kern
             const int16_t *wt = a.w + (size_t)(ky * a.kw + kx) * a.channels + c0;
             if (VEC == 4) {
                 uint32_t d = a.zx_splat;
-                if (ok) d = *reinterpret_cast<const uint32_t *>(ximg + ((size_t)iy * a.in_w + ix) * a.channels);
+                if (ok) d = dw_load(ximg + ((size_t)iy * a.in_w + ix) * a.channels);
 #pragma unroll
                 for (int c = 0; c < VEC; c++) acc[c] += __mul24((int)((d >> (8 * c)) & 0xff), (int)wt[c]);
             } else {
@@ -376,10 +468,13 @@ int prepack_depthwise(nncase_hip_ctx *ctx, nncase_hip_weights *w, const uint8_t 
     return 0;
 }
 
-bool depthwise_uses_3x3(const nncase_hip_weights *w, const nncase_hip_conv2d_args_t *c) {
-    return w->out_channels % 4 == 0 && w->kernel_h == 3 && w->kernel_w == 3 && c->dilation_h == 1 && c->dilation_w == 1 &&
-           c->stride_h == c->stride_w && (c->stride_h == 1 || c->stride_h == 2);
+// Windows of k x k taps at strides of 1 and 2, undilated, over four channels and more: the kernels that share a row between columns.
+static bool shares_columns(const nncase_hip_weights *w, const nncase_hip_conv2d_args_t *c, int k) {
+    return w->out_channels >= 4 && w->kernel_h == k && w->kernel_w == k && c->dilation_h == 1 && c->dilation_w == 1 && c->stride_h == c->stride_w &&
+           (c->stride_h == 1 || c->stride_h == 2);
 }
+bool depthwise_uses_3x3(const nncase_hip_weights *w, const nncase_hip_conv2d_args_t *c) { return shares_columns(w, c, 3); }
+bool depthwise_uses_5x5(const nncase_hip_weights *w, const nncase_hip_conv2d_args_t *c) { return shares_columns(w, c, 5); }
 
 int launch_qconv_depthwise(nncase_hip_ctx *ctx, const uint8_t *x, const nncase_hip_weights *w, void *y,
                            const nncase_hip_conv2d_args_t *c, int out_h, int out_w) {
@@ -419,11 +514,10 @@ int launch_qconv_depthwise(nncase_hip_ctx *ctx, const uint8_t *x, const nncase_h
         if (rc) return rc;
     }
 
-    const bool vec4 = (ch % 4 == 0) && ((reinterpret_cast<uintptr_t>(x) & 3u) == 0) &&
-                      ((reinterpret_cast<uintptr_t>(y) & 15u) == 0);
+    const bool vec4 = ch >= 4 && ((reinterpret_cast<uintptr_t>(x) & 3u) == 0) && ((reinterpret_cast<uintptr_t>(y) & 15u) == 0);
     const bool k3 = vec4 && depthwise_uses_3x3(w, c);
     if (k3) {
-        a.cq = ch / 4;
+        a.cq = ceil_div(ch, 4);
         a.strips = ceil_div(out_w, kDwCols);
         // Rows per thread.  Long strips amortise the two-row halo and the per-thread set-up;
         // short ones give more waves.  While every SIMD gets at least a few waves, the waves are
@@ -477,8 +571,27 @@ int launch_qconv_depthwise(nncase_hip_ctx *ctx, const uint8_t *x, const nncase_h
         NNHIP_LAUNCH_CHECK(ctx, "dw3x3_kernel");
         return 0;
     }
+    if (vec4 && depthwise_uses_5x5(w, c)) {
+        a.cq = ceil_div(ch, 4);
+        a.strips = ceil_div(out_w, kDwCols);
+        // (a thread's weights are as much to fetch as an output row: long strips while they leave six waves to a SIMD)
+        const auto waves = [&](int rows) { return ((long long)c->batch * ceil_div(out_h, rows) * a.strips * a.cq + 63) / 64; };
+        a.rows = 8;
+        while (a.rows > 1 && waves(a.rows) < 6ll * 4 * ctx->compute_units) a.rows /= 2;
+        a.row_chunks = ceil_div(out_h, a.rows);
+        a.d_cq = make_fastdiv((uint32_t)a.cq);
+        a.d_strips = make_fastdiv((uint32_t)a.strips);
+        a.d_rows = make_fastdiv((uint32_t)a.row_chunks);
+        a.total = (long long)c->batch * a.row_chunks * a.strips * a.cq;
+        NNHIP_REQUIRE(ctx, a.total < ((long long)1 << 31), -EINVAL, "qconv2d(depthwise): too many work items");
+        const dim3 g((unsigned)((a.total + kDwThreads - 1) / kDwThreads)), t(kDwThreads);
+        if (c->stride_h == 1) hipLaunchKernelGGL((dw_window_kernel<5, 1>), g, t, 0, ctx->stream, a);
+        else hipLaunchKernelGGL((dw_window_kernel<5, 2>), g, t, 0, ctx->stream, a);
+        NNHIP_LAUNCH_CHECK(ctx, "dw_window_kernel");
+        return 0;
+    }
     const int vec = vec4 ? 4 : 1;
-    a.cq = ch / vec;
+    a.cq = ceil_div(ch, vec);
     a.d_cq = make_fastdiv((uint32_t)a.cq);
     a.d_ow = make_fastdiv((uint32_t)out_w);
     a.d_oh = make_fastdiv((uint32_t)out_h);

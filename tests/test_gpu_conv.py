@@ -920,6 +920,23 @@ def test_input_tiles_of_odd_groups_and_extreme_zero_points(hip_ctx, n, c, h, w, 
     run_case(hip_ctx, n, c, h, w, oc, k, k, (s, s), ((k // 2, k // 2), (k // 2, k // 2)), (1, 1), groups, seed=c + oc, zx=zx, zw=zw, modes=("u8",))
 
 
+@pytest.mark.parametrize("c", [3, 4, 5, 6, 7, 63, 130])
+@pytest.mark.parametrize("k,stride,hw,pad,dil", [
+    (3, 1, (9, 14), ((1, 1), (1, 1)), 1), (3, 2, (17, 11), ((0, 1), (1, 0)), 1), (5, 1, (12, 7), ((2, 2), (2, 2)), 1),
+    (5, 2, (21, 22), ((2, 2), (1, 2)), 1), (5, 1, (5, 5), ((0, 0), (0, 0)), 1), (7, 1, (9, 10), ((3, 3), (3, 3)), 1), (3, 1, (9, 9), ((2, 2), (2, 2)), 2)])
+def test_depthwise_channels_in_fours_that_overlap(hip_ctx, c, k, stride, hw, pad, dil):
+    """Channel counts that are no multiple of four (the last four overlap the ones before, at any byte), windows of 5x5 with their own
+    kernel, others with the general one, three channels one by one; every kind of result."""
+    run_case(hip_ctx, 3, c, *hw, c, k, k, (stride, stride), pad, (dil, dil), c, seed=c * 31 + k, clamp=None)
+
+
+@pytest.mark.parametrize("n,c,hw,k,stride", [(40, 61, 56, 3, 1), (40, 62, 57, 3, 2), (30, 66, 41, 5, 1), (30, 68, 57, 5, 2)])
+def test_depthwise_strips_of_odd_channel_counts(hip_ctx, n, c, hw, k, stride):
+    """Strips of several output rows, the last of them cut off by the image."""
+    p = k // 2
+    run_case(hip_ctx, n, c, hw, hw + 1, c, k, k, (stride, stride), ((p, p), (p, p)), (1, 1), c, seed=c, zx=255, zw=0, modes=("u8",))
+
+
 @pytest.mark.parametrize("m,k,n", [(16500, 516, 300), (16641, 1020, 258), (33000, 532, 257)])
 def test_matmul_of_rows_of_whole_dwords_in_256_channel_blocks(hip_ctx, m, k, n):
     """Rows that are no multiple of 16 bytes, moved straight to LDS in 256 x 256 blocks: last k-steps that end inside a piece, partial
