@@ -1,4 +1,4 @@
-// u8/u8 convolution over a window, with the input of a two-dimensional tile of output pixels in LDS.
+// u8/u8 convolution over a window to codes or float32, with the input of a two-dimensional tile of output pixels in LDS.
 //
 // The implicit-GEMM kernels fetch, re-bias and sum an activation once per tap of the window: nine times for 3x3, a hundred
 // instructions of a wave per k-step against eight products, and an instruction of a wave that is alone on its SIMD takes eight
@@ -19,6 +19,8 @@
 //   * a launch of few blocks splits each one's k-steps between groups of waves, which meet once: up to four k-steps of every group are on
 //     their way when the first product starts, where the ring of qconv_wide_kernel goes through a barrier for each.  In a chain, us there /
 //     here: 128 -> 128 3x3 of 1600 pixels 5.3 / 4.0, 256 -> 256 of 400 6.8 / 4.7, 512 -> 512 of 400 11.0 / 7.9.
+//   * float32 results leave the same way, four pieces for sixteen channels (116 layers of 8 to 640 channels 1.38 times as quick in the
+//     mean as by the ring; 441 -> 29 3x3 stride 2 of 2601 pixels 13.0 / 6.1, 80 -> 12 5x5 of 54 675 16.0 / 9.4); int32 stays there.
 // Arithmetic, weight packing and the bytes of the result are those of qconv_igemm.hpp.
 #include "qconv_tile.hpp"
 
@@ -43,7 +45,7 @@ TilePlan plan_tile(const IgemmArgs &a, int pix, int tb, int threads, int nchunks
     t.d_nchunks = make_fastdiv((uint32_t)nchunks), t.d_rest = make_fastdiv((uint32_t)std::max(1, a.ksteps - 1));
     t.tile_off = (tb * 16 + groups * pix + (a.ksteps + 2 * groups) * 4) * 4 + 256 + parts;
     t.apart = threads / t.pieces, t.dc = t.apart % t.hc, t.dr = t.apart / t.hc;
-    p.lds = t.tile_off + std::max((size_t)t.hr * t.row_pitch, (size_t)pix * (tb * 16 + 16));
+    p.lds = t.tile_off + std::max((size_t)t.hr * t.row_pitch, (size_t)pix * (tb * 16 * (a.ep.out_mode == kOutU8 ? 1 : 4) + 16));
     return p;
 }
 
@@ -120,9 +122,10 @@ TileShape choose_tile(const nncase_hip_ctx *ctx, const IgemmArgs &a, bool ragged
 const char *tile_kernel_block(const nncase_hip_ctx *ctx, const nncase_hip_weights *w, const nncase_hip_conv2d_args_t *c, int out_h, int out_w) {
     static const char *const names[] = {"128x32", "64x32", "32x64", "128x128", "64x128", "32x32,KG=2", "32x32,KG=4", "16x32,KG=4", "32x64,KG=2",
                                         "32x64,KG=4", "16x64,KG=4", nullptr};
-    if (c->out_dtype != NNCASE_HIP_DT_U8 || c->dequantize_output) return nullptr;
+    if (c->dequantize_output || c->out_dtype == NNCASE_HIP_DT_I32) return nullptr;
     IgemmArgs a;
     memset(&a, 0, sizeof(a));
+    a.ep.out_mode = c->out_dtype == NNCASE_HIP_DT_U8 ? kOutU8 : kOutF32;
     a.m = (int)std::min<int64_t>((int64_t)c->batch * out_h * out_w, 1 << 30);
     a.d_ohow = make_fastdiv((uint32_t)(out_h * out_w)), a.d_ow = make_fastdiv((uint32_t)out_w);
     a.kh = w->kernel_h, a.kw = w->kernel_w, a.stride_h = c->stride_h, a.stride_w = c->stride_w, a.dil_h = c->dilation_h, a.dil_w = c->dilation_w;
@@ -133,7 +136,7 @@ const char *tile_kernel_block(const nncase_hip_ctx *ctx, const nncase_hip_weight
 
 TilePlan plan_qconv_tile(const nncase_hip_ctx *ctx, const IgemmArgs &a, bool ragged, int tiles, int nchunks) {
     TilePlan plan;
-    const TileShape shape = a.ep.out_mode == kOutU8 && !a.deq ? choose_tile(ctx, a, ragged, tiles, nchunks, &plan) : kTileNone;
+    const TileShape shape = !a.deq && a.ep.out_mode != kOutI32 ? choose_tile(ctx, a, ragged, tiles, nchunks, &plan) : kTileNone;
     plan.shape = shape;
     plan.t.ragged = ragged;
     return plan;

@@ -45,15 +45,26 @@ TilePlan plan_qconv_tile(const nncase_hip_ctx *ctx, const IgemmArgs &a, bool rag
 int launch_qconv_tile(nncase_hip_ctx *ctx, const IgemmArgs &a, const TilePlan &plan, int nchunks);
 int launch_tile_ragged(nncase_hip_ctx *ctx, const IgemmArgs &a, const TilePlan &plan, int nchunks); // (qconv_tile_ragged.hip)
 
+// A launch's results: codes; codes whose requantisation is the one-instruction form without a clamp of its own (Epilogue::fast and ::full);
+// float32.
+enum TileOut { kTileCodes, kTileFastCodes, kTileFloats };
+
 // What a launch's last stage takes of the arguments, in one trip: fetched ahead, the values would be spilled while the reduction runs,
 // and a request of the first stage would wait behind them.
-template <bool FAST> __device__ __forceinline__ IgemmArgs gather_store_args() {
+template <TileOut OUT> __device__ __forceinline__ IgemmArgs gather_store_args() {
     auto p = (const __attribute__((address_space(4))) IgemmArgs *)__builtin_amdgcn_kernarg_segment_ptr();
     asm volatile("" : "+s"(p));
     const IgemmArgs &a = *(const IgemmArgs *)p;
     IgemmArgs l; // (what is not assigned here is not used)
+    if constexpr (OUT == kTileFloats) {
+        l.ep.mult = a.ep.mult, l.ep.lo = a.ep.lo, l.ep.hi = a.ep.hi;
+        l.y = a.y, l.n = a.n, l.ldy = a.ldy, l.y_coff = a.y_coff, l.zwp = a.zwp, l.m = a.m, l.d_ohow.div = a.d_ohow.div, l.d_ow.div = a.d_ow.div;
+        asm volatile("" ::"s"(l.ep.mult), "s"(l.ep.lo), "s"(l.ep.hi), "s"(l.y), "s"(l.n), "s"(l.ldy), "s"(l.y_coff), "s"(l.zwp), "s"(l.m),
+                     "s"(l.d_ohow.div), "s"(l.d_ow.div));
+        return l;
+    }
     l.ep.c1 = a.ep.c1, l.ep.c2 = a.ep.c2;
-    if constexpr (!FAST) {
+    if constexpr (OUT == kTileCodes) {
         l.ep.mult = a.ep.mult, l.ep.sy = a.ep.sy, l.ep.rsy = a.ep.rsy, l.ep.zy = a.ep.zy, l.ep.qlo = a.ep.qlo, l.ep.qhi = a.ep.qhi;
         l.ep.fast = a.ep.fast, l.ep.full = a.ep.full;
         asm volatile("" ::"s"(l.ep.mult), "s"(l.ep.sy), "s"(l.ep.rsy), "s"(l.ep.zy), "s"(l.ep.qlo), "s"(l.ep.qhi), "s"(l.ep.fast), "s"(l.ep.full));
@@ -68,10 +79,9 @@ template <bool FAST> __device__ __forceinline__ IgemmArgs gather_store_args() {
     return l;
 }
 
-// FAST: the requantisation is the one-instruction form without a clamp of its own (Epilogue::fast and ::full).
 // KG > 1: KG groups of WM x WN waves share the reduction, every KG-th k-step each, and add their sums up at the end.
 // RAGGED: channels that are no multiple of 16, at any byte (qconv_igemm.hip packs the weights such that what else a piece holds adds nothing).
-template <int T, int RG, int WM, int WN, int KG, bool FAST, bool RAGGED>
+template <int T, int RG, int WM, int WN, int KG, TileOut OUT, bool RAGGED>
 __global__ __launch_bounds__(WM * WN * KG * 64, 4) void qconv_tile_kernel(const IgemmArgs a, const TileArgs t) {
     constexpr int THREADS = WM * WN * KG * 64, PIX = WM * RG * 16, TB = T * WN;
     constexpr int D = 4;                                             // k-steps of weights in flight
@@ -288,7 +298,7 @@ __global__ __launch_bounds__(WM * WN * KG * 64, 4) void qconv_tile_kernel(const 
         }
         keep(fa, i0);
     }
-    const IgemmArgs late = gather_store_args<FAST>();
+    const IgemmArgs late = gather_store_args<OUT>();
     __syncthreads();
 
     // ---- the reduction ----
@@ -348,22 +358,24 @@ __global__ __launch_bounds__(WM * WN * KG * 64, 4) void qconv_tile_kernel(const 
 
     // ---- epilogue ----
     // whole pixel rows: TB threads per pixel, 16 channels each.  Their bytes of the residual are asked for before the sums meet.
-    constexpr int PPT = THREADS / TB < PIX ? THREADS / TB : PIX, PASSES = PIX / PPT; // pixels of a pass
+    // (floats: four pieces for every sixteen channels)
+    constexpr int ES = OUT == kTileFloats ? 4 : 1, PIECES = TB * ES;
+    constexpr int PPT = THREADS / PIECES < PIX ? THREADS / PIECES : PIX, PASSES = PIX / PPT; // pixels of a pass
     static_assert(PIX % PPT == 0, "whole passes");
     const int oh_img = (int)late.d_ohow.div, ow = (int)late.d_ow.div;
-    const int cb = (tid % TB) * 16, ch = ch_base + cb;
-    const bool whole = ch + 16 <= late.n, wide_y = ((late.ldy | late.y_coff) & 3) == 0;
+    const int cb = (tid % PIECES) * (16 / ES), ch = ch_base + cb;
+    const bool whole = ch + 16 / ES <= late.n, wide_y = OUT == kTileFloats || ((late.ldy | late.y_coff) & 3) == 0;
     int px[PASSES]; // pixel index of the tensor, late.m where there is none
     u32x4 rv[PASSES];
 #pragma unroll
     for (int it = 0; it < PASSES; it++) {
-        const int p = it * PPT + tid / TB;
+        const int p = it * PPT + tid / PIECES;
         const int ty = tile_div(p, t.d_tw);
         const int oy = oy0 + ty, ox = ox0 + p - __mul24(ty, t.tw);
         const int at = __mul24(oy, ow) + ox;
         px[it] = p < PIX && ty < t.th && ox < ow && at < oh_img && ch < late.n ? (int)img * oh_img + at : late.m;
     }
-    if (late.rep.res) {
+    if (OUT != kTileFloats && late.rep.res) {
         const bool wide_r = ((late.ldr | late.r_coff) & 3) == 0;
 #pragma unroll
         for (int it = 0; it < PASSES; it++) {
@@ -394,7 +406,7 @@ __global__ __launch_bounds__(WM * WN * KG * 64, 4) void qconv_tile_kernel(const 
         });
     }
     __syncthreads(); // the sums are there, and every wave is through with the tile: its place takes the result
-    constexpr int kOutPitch = TB * 16 + 16;
+    constexpr int kOutPitch = TB * 16 * ES + 16;
     auto finish = [&](auto first_c) __attribute__((always_inline)) { // the EACH units from there on
         constexpr int first = decltype(first_c)::value, count = KG == 1 ? UNITS : (UNITS - first < EACH ? UNITS - first : EACH);
         int32_t owed[RG];
@@ -423,8 +435,16 @@ __global__ __launch_bounds__(WM * WN * KG * 64, 4) void qconv_tile_kernel(const 
             int32_t v[4];
 #pragma unroll
             for (int r = 0; r < 4; r++) v[r] = acc[rg][nt][r] + owed[rg];
-            packed[u] = FAST ? requant4_u8_packed_direct(v, late.ep) : requant4_u8_packed(v, late.ep);
+            if constexpr (OUT == kTileFloats) {
+                u32x4 o;
+#pragma unroll
+                for (int r = 0; r < 4; r++) o[r] = __float_as_uint(clamp_ref((float)v[r] * late.ep.mult, late.ep.lo, late.ep.hi));
+                *reinterpret_cast<u32x4 *>(tile + ((wm * RG + rg) * 16 + j) * kOutPitch + (ch0 + nt * 4) * 4) = o;
+            } else {
+                packed[u] = OUT == kTileFastCodes ? requant4_u8_packed_direct(v, late.ep) : requant4_u8_packed(v, late.ep);
+            }
         }
+        if constexpr (OUT == kTileFloats) return;
         if (late.lut) { // (every byte is asked for before the first is used)
             uint32_t b[count][4];
 #pragma unroll
@@ -450,7 +470,18 @@ __global__ __launch_bounds__(WM * WN * KG * 64, 4) void qconv_tile_kernel(const 
 #pragma unroll
     for (int it = 0; it < PASSES; it++) {
         if (px[it] >= late.m) continue;
-        u32x4 v = *reinterpret_cast<const u32x4 *>(tile + (it * PPT + tid / TB) * kOutPitch + cb);
+        u32x4 v = *reinterpret_cast<const u32x4 *>(tile + (it * PPT + tid / PIECES) * kOutPitch + cb * ES);
+        if constexpr (OUT == kTileFloats) {
+            uint32_t *const yo = reinterpret_cast<uint32_t *>(late.y) + (size_t)px[it] * late.ldy + late.y_coff + ch;
+            if (whole) {
+                *reinterpret_cast<u32x4_a4 *>(yo) = u32x4_a4{v[0], v[1], v[2], v[3]};
+            } else {
+#pragma unroll
+                for (int b = 0; b < 4; b++)
+                    if (ch + b < late.n) yo[b] = v[b];
+            }
+            continue;
+        }
         if (late.rep.res) {
 #pragma unroll
             for (int d = 0; d < 4; d++) v[d] = residual4_packed(v[d], rv[it][d], late.rep);
@@ -469,9 +500,9 @@ __global__ __launch_bounds__(WM * WN * KG * 64, 4) void qconv_tile_kernel(const 
     }
 }
 
-template <int T, int RG, int WM, int WN, int KG, bool FAST, bool RAGGED> int launch_tile_f(nncase_hip_ctx *ctx, const IgemmArgs &args, const TilePlan &plan, int nchunks) {
-    if (plan.lds > 65536) NNHIP_HIP(ctx, (raise_dynamic_lds<qconv_tile_kernel<T, RG, WM, WN, KG, FAST, RAGGED>>(ctx->device, 160 * 1024)));
-    hipLaunchKernelGGL((qconv_tile_kernel<T, RG, WM, WN, KG, FAST, RAGGED>), dim3(ceil_div(args.num_mtiles, 8) * 8 * nchunks), dim3(WM * WN * KG * 64), plan.lds, ctx->stream, args,
+template <int T, int RG, int WM, int WN, int KG, TileOut OUT, bool RAGGED> int launch_tile_f(nncase_hip_ctx *ctx, const IgemmArgs &args, const TilePlan &plan, int nchunks) {
+    if (plan.lds > 65536) NNHIP_HIP(ctx, (raise_dynamic_lds<qconv_tile_kernel<T, RG, WM, WN, KG, OUT, RAGGED>>(ctx->device, 160 * 1024)));
+    hipLaunchKernelGGL((qconv_tile_kernel<T, RG, WM, WN, KG, OUT, RAGGED>), dim3(ceil_div(args.num_mtiles, 8) * 8 * nchunks), dim3(WM * WN * KG * 64), plan.lds, ctx->stream, args,
                        plan.t);
     NNHIP_LAUNCH_CHECK(ctx, "qconv_tile_kernel");
     return 0;
@@ -479,7 +510,9 @@ template <int T, int RG, int WM, int WN, int KG, bool FAST, bool RAGGED> int lau
 template <bool RAGGED, int T, int RG, int WM, int WN, int KG = 1> int launch_tile_t(nncase_hip_ctx *ctx, const IgemmArgs &a, const TilePlan &plan, int nchunks) {
     IgemmArgs args = a;
     args.num_mtiles = plan.tiles;
-    return a.ep.fast && a.ep.full ? launch_tile_f<T, RG, WM, WN, KG, true, RAGGED>(ctx, args, plan, nchunks) : launch_tile_f<T, RG, WM, WN, KG, false, RAGGED>(ctx, args, plan, nchunks);
+    if (a.ep.out_mode != kOutU8) return launch_tile_f<T, RG, WM, WN, KG, kTileFloats, RAGGED>(ctx, args, plan, nchunks);
+    return a.ep.fast && a.ep.full ? launch_tile_f<T, RG, WM, WN, KG, kTileFastCodes, RAGGED>(ctx, args, plan, nchunks)
+                                  : launch_tile_f<T, RG, WM, WN, KG, kTileCodes, RAGGED>(ctx, args, plan, nchunks);
 }
 
 template <bool RAGGED> int launch_tile_shape(nncase_hip_ctx *ctx, const IgemmArgs &a, const TilePlan &plan, int nchunks) {

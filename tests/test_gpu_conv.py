@@ -920,6 +920,17 @@ def test_input_tiles_of_odd_groups_and_extreme_zero_points(hip_ctx, n, c, h, w, 
     run_case(hip_ctx, n, c, h, w, oc, k, k, (s, s), ((k // 2, k // 2), (k // 2, k // 2)), (1, 1), groups, seed=c + oc, zx=zx, zw=zw, modes=("u8",))
 
 
+@pytest.mark.parametrize("n,c,h,w,oc,k,s", [
+    (1, 64, 19, 23, 100, 3, 1), (2, 128, 40, 40, 126, 3, 1), (4, 128, 40, 41, 128, 3, 1), (1, 32, 40, 40, 30, 3, 1), (2, 128, 80, 80, 32, 3, 1),
+    (2, 128, 112, 110, 32, 3, 1), (3, 64, 64, 67, 60, 3, 1), (2, 64, 100, 97, 31, 3, 1), (8, 32, 100, 131, 30, 3, 1), (12, 128, 56, 64, 130, 3, 2),
+    (6, 96, 90, 91, 100, 3, 1),                                                                     # every block, whole channels
+    (1, 5, 9, 7, 40, 5, 1), (3, 97, 41, 40, 60, 3, 1), (3, 90, 77, 75, 203, 3, 2), (3, 111, 92, 91, 125, 3, 1), (2, 33, 13, 14, 3, 3, 1)])
+def test_windows_over_an_input_tile_with_float_results(hip_ctx, n, c, h, w, oc, k, s):
+    """float32 results of the window kernel: rows of whole pieces, the last of them cut off by the channels; int32 beside them."""
+    p = k // 2
+    run_case(hip_ctx, n, c, h, w, oc, k, k, (s, s), ((p, p), (p, p)), (1, 1), 1, seed=c + oc, zx=203, zw=135, modes=("i32", "f32"))
+
+
 @pytest.mark.parametrize("c", [3, 4, 5, 6, 7, 63, 130])
 @pytest.mark.parametrize("k,stride,hw,pad,dil", [
     (3, 1, (9, 14), ((1, 1), (1, 1)), 1), (3, 2, (17, 11), ((0, 1), (1, 0)), 1), (5, 1, (12, 7), ((2, 2), (2, 2)), 1),
