@@ -731,8 +731,9 @@ NNCASE_HIP_API int nncase_hip_function_capture(nncase_hip_function_t *fn);
 /* Per-operator device time: every operator is enqueued `iterations` times
  * back to back between two HIP events recorded on the context's stream and
  * the mean duration in milliseconds is written to avg_ms[index] (the array
- * holds nncase_hip_function_size entries; of operators that share a launch the
- * first has its time and the others 0).  Blocks until done.  The HIP
+ * holds nncase_hip_function_size entries; of max pools that share a launch the
+ * first has its time and the others 0, a convolution that shares one when the
+ * function runs is timed by itself).  Blocks until done.  The HIP
  * counterpart of the reference's per-op profiler
  * (src/Native/include/nncase/runtime/stackvm/op_profile.h:41-76). */
 NNCASE_HIP_API int nncase_hip_function_profile(nncase_hip_function_t *fn, int32_t iterations, float *avg_ms);

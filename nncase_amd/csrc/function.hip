@@ -227,14 +227,15 @@ static int run_joined_convs(nncase_hip_function *fn, size_t at, size_t *count) {
 }
 
 // Runs the operators from `at` on that run as one launch; *next is the first behind them.
-static int run_ops(nncase_hip_function *fn, size_t at, size_t *next) {
+static int run_ops(nncase_hip_function *fn, size_t at, size_t *next, bool join_convs = true) {
     MaxPoolChain chain;
     if (const size_t n = find_pool_chain(fn->ops, at, &chain)) {
         *next = at + n;
         return launch_maxpool_chain(fn->ctx, chain);
     }
     size_t joined = 0;
-    if (int rc = run_joined_convs(fn, at, &joined)) return rc;
+    if (join_convs)
+        if (int rc = run_joined_convs(fn, at, &joined)) return rc;
     *next = at + std::max<size_t>(joined, 1);
     return joined ? 0 : run_op(fn, fn->ops[at]);
 }
@@ -867,11 +868,11 @@ extern "C" int nncase_hip_function_profile(nncase_hip_function_t *fn, int32_t it
     NNHIP_HIP(ctx, hipEventCreate(&e1));
     int rc = 0;
     std::fill(avg_ms, avg_ms + fn->ops.size(), 0.f);
-    for (size_t i = 0, next = 0; i < fn->ops.size() && rc == 0; i = next) { // (operators that run as one launch: the first has its time)
-        rc = run_ops(fn, i, &next); // warm
+    for (size_t i = 0, next = 0; i < fn->ops.size() && rc == 0; i = next) { // (pools that run as one launch: the first has its time)
+        rc = run_ops(fn, i, &next, false); // warm
         if (rc) break;
         hipError_t e = hipEventRecord(e0, ctx->stream);
-        for (int it = 0; it < iterations && rc == 0; it++) rc = run_ops(fn, i, &next);
+        for (int it = 0; it < iterations && rc == 0; it++) rc = run_ops(fn, i, &next, false);
         if (e == hipSuccess) e = hipEventRecord(e1, ctx->stream);
         if (e == hipSuccess) e = hipEventSynchronize(e1);
         float ms = 0.f;

@@ -548,3 +548,17 @@ def test_operators_whose_buffers_meet_stay_apart(hip_ctx):
         fn.invoke()
         hip_ctx.sync()
         assert np.array_equal(out.download((m * n2,), np.uint8), want)
+
+
+def test_operators_that_may_share_a_launch_are_timed_by_themselves(hip_ctx):
+    rng = np.random.default_rng(5)
+    k1, n1, n2, hw = 384, 64, 384, 14
+    ws = [rng.integers(0, 256, s, dtype=np.uint8) for s in ((k1, 1, 3, 3), (n1, k1, 1, 1), (n2, n1, 1, 1))]
+    weights = [hip_ctx.prepack_conv2d(w, None, qp(128, 0.004), groups=k1 if i == 0 else 1, expected_pixels=hw * hw) for i, w in enumerate(ws)]
+    bufs = [hip_ctx.alloc(hw * hw * c).fill(0x40) for c in (k1, k1, n1, n2)]
+    fn = rt.Function(hip_ctx)
+    q = qp(120, 0.5)
+    fn.add_qconv2d(bufs[0], weights[0], bufs[1], rt.Conv2dArgs(1, hw, hw, 1, 1, 1, 1, 1, 1, 1, 1, q, q, FULL[0], FULL[1], rt.DT_U8))
+    for i in (1, 2):
+        fn.add_qconv2d(bufs[i], weights[i], bufs[i + 1], conv_args(1, hw, hw, q, q, FULL))
+    assert all(ms > 0 for ms in fn.profile(3))
