@@ -175,7 +175,8 @@ inline uint32_t make_tile_div(int d) { return ((1u << 20) + (uint32_t)d - 1) / (
 // and 2, whole_window_ksteps and more).  us, implicit GEMM / window kernel:
 //   * tiles that images do not fill by half stay, their surplus pixels are multiplied and dropped; with fewer than three waves per
 //     compute unit a sixth is too much (3388 pixels 256 -> 170 in two groups, 63 % full, 12.1 / 14.4)
-//   * with fewer than three waves per two compute units (stride 2: four per unit) the k-steps split over groups of waves win
+//   * with fewer than three waves per two compute units (stride 2: four per unit) the k-steps split over groups of waves win, in the
+//     ring and, quicker still, here (split_window_pays)
 //     (400 pixels 256 -> 256 7.1 / 7.5; 1600 pixels 128 -> 256 stride 2 5.8 / 6.8)
 //   * blocks of two waves have to leave room in LDS for four of a compute unit from 400 channels on (560 -> 32 3x3 of 40 344 pixels
 //     27.4 / 34.2, 512 -> 48 5x5 of 18 150 41.9 / 49.0; up to there three are enough: 256 -> 32 5x5 of 85 264 61.4 / 43.6), and for

@@ -1,27 +1,4 @@
-// u8/u8 convolution over a window to codes or float32, with the input of a two-dimensional tile of output pixels in LDS.
-//
-// The implicit-GEMM kernels fetch, re-bias and sum an activation once per tap of the window: nine times for 3x3, a hundred
-// instructions of a wave per k-step against eight products, and an instruction of a wave that is alone on its SIMD takes eight
-// to nine cycles.  Here a block brings the input under its tile of output pixels into LDS once (re-biased, the padding filled
-// with the zero point) and every tap is an LDS read at another offset; the sum of x over a window, which the weight zero
-// point multiplies, is the sum of per-pixel channel sums taken on the way in.  What is left of a k-step is RG + 1 LDS reads
-// (operands and where the next tap lies), T loads of packed weights straight into registers, four k-steps ahead, and the
-// products: no barrier, no staging.  A wave owns RG * 16 pixels x T * 16 channels; a block is WM x WN waves.
-//   * weights come from L2 through the vector L1 (64 bytes per clock): with 64 x 32 outputs per wave a k-step of four waves
-//     takes 8 KiB of them for 128 clocks of matrix work, so waves share pixels rather than channels where they can;
-//   * blocks start the reduction at different k-steps (integer sums do not care): otherwise all of them wait for the same
-//     weights to come from memory at the same time, step after step;
-//   * results leave through LDS as whole pixel rows, whose bytes of a residual are asked for before the sums meet;
-//   * what a block does before its first request and after its last product counts as much as the reduction: all arguments of the
-//     requests in one trip and those of the stores in another, a thread that keeps its piece of a pixel (two multiply-adds an address,
-//     short divisions), a channel's terms asked for first.  Start to end of a block, 6400 pixels 64 -> 64 3x3 with a residual 4.6 us ->
-//     3.7 (before the first request 0.6 -> 0.4, requests 0.5 -> 0.3, results 1.1 -> 0.5), 409 600 pixels 32 -> 32 21.8 -> 19.2 a launch.
-//   * a launch of few blocks splits each one's k-steps between groups of waves, which meet once: up to four k-steps of every group are on
-//     their way when the first product starts, where the ring of qconv_wide_kernel goes through a barrier for each.  In a chain, us there /
-//     here: 128 -> 128 3x3 of 1600 pixels 5.3 / 4.0, 256 -> 256 of 400 6.8 / 4.7, 512 -> 512 of 400 11.0 / 7.9.
-//   * float32 results leave the same way, four pieces for sixteen channels (116 layers of 8 to 640 channels 1.38 times as quick in the
-//     mean as by the ring; 441 -> 29 3x3 stride 2 of 2601 pixels 13.0 / 6.1, 80 -> 12 5x5 of 54 675 16.0 / 9.4); int32 stays there.
-// Arithmetic, weight packing and the bytes of the result are those of qconv_igemm.hpp.
+// Which launches the window kernel of qconv_tile.hpp takes, with which block, and the launches for channels that are multiples of 16.
 #include "qconv_tile.hpp"
 
 namespace nnhip {
